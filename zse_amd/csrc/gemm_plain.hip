@@ -1,12 +1,12 @@
-// Plain matrix product C[M,N] = A[M,K] * W[N,K]^T with float accumulation,
-// no matrix cores and no reduced precision: the 32-bit path's product and the
-// twin that the tuned bf16 kernels are checked against.  Weights are
-// [out, in] row-major as in the reference (orchestrator/kernels.py:1075-1126,
-// a 32x32 shared-memory tile per block).  The sum over K runs in a fixed
-// order for every output element, whatever M is, so a row's result does not
+// Plain matrix product C[M,N] = A[M,K] * W[N,K]^T with float accumulation and no reduced
+// precision: the 32-bit path's product and, in the bf16 library, the twin that the tuned
+// kernels are checked against.  Weights are [out, in] row-major as in the reference
+// (orchestrator/kernels.py:1075-1126, a 32x32 shared-memory tile per block).  The sum over K
+// runs in a fixed order for every output element, whatever M is, so a row's result does not
 // depend on which other rows are in the batch.
 #include "common.h"
 
+#if ZSE_ACT_BF16
 #define GP_BM 64
 #define GP_BN 64
 #define GP_BK 16
@@ -55,14 +55,188 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
   }
 }
 
+#else
+
+// The 32-bit product on the 32-bit matrix cores (16x16x4, float in, float out).
+//
+// A block owns 16 MF x 16 NF of C and its eight waves share K out: wave w takes the 32-wide
+// steps w, w + 8, .., every wave the whole tile, and their sums meet in LDS, (w, w + 4), then
+// (w, w + 2), then (w, w + 1).  So the order of a sum follows from K alone and the tile may
+// follow from M and N.  Operands come straight from memory: in a 16-wide piece of K the four
+// products take k = 4 (lane / 16) + e, e = 0..3, from both sides, so a lane's float4 of a row
+// is its operand of four products and a load takes 64-byte runs of sixteen rows.  A product is
+// 32 cycles long, a load of 16 bytes a lane 16: at 4 x 4 pieces the matrix cores are the bound,
+// below that L2 (a 2 x 2 tile reads twice the bytes per flop).
+//
+// Measured (us; before: 64 x 64 tiles of scalar multiply-adds through LDS, one block a tile):
+//   M = 303: 1024 x 4096 and 1024 x 1024 (average)  452 -> 42;  8192 x 1024  217 -> 87;
+//   1536 x 1024  191 -> 20;  M = 4: 32768 x 1024  207 -> 28.
+// The error against 64 bits is no larger than the scalar sum's (eight shorter sums added up).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define GF_WAVES 8
+
+// HOW: 2: K is a whole number of steps; 1: rows of whole 16-byte pieces; 0: every value is loaded
+// on its own.  The loads of the next H pieces of a wave's run are on their way while the current
+// ones are multiplied, so nothing may look at them before: with HOW = 1 the pieces behind K are
+// set to zero right before they are multiplied.
+template <int MF, int NF, int H, int AHEAD, int HOW>
+__global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __restrict__ A, int lda,
+                                                                 const float* __restrict__ W,
+                                                                 float* __restrict__ C, int ldc, int M, int N,
+                                                                 int K, int tiles_m, int tiles_n) {
+  __shared__ f32x4 part[GF_WAVES / 2][MF * NF][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  // the blocks that share a strip of W run on one XCD, one after the other (ids go round-robin over 8)
+  int id = blockIdx.x;
+  const int total = tiles_m * tiles_n;
+  if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
+  const int m0 = id % tiles_m * (16 * MF), n0 = id / tiles_m * (16 * NF);
+  const float* ap[MF];
+  const float* wp[NF];
+#pragma unroll
+  for (int i = 0; i < MF; i++) ap[i] = A + (size_t)min(m0 + 16 * i + r, M - 1) * lda;
+#pragma unroll
+  for (int j = 0; j < NF; j++) wp[j] = W + (size_t)min(n0 + 16 * j + r, N - 1) * K;
+  const int steps = (K + 31) / 32;
+
+  auto piece = [&](const float* row, int k) {
+    f32x4 v;
+    if (HOW == 2) {
+      v = *(const f32x4*)(row + k);
+    } else if (HOW == 1) {       // K is a multiple of 4: the piece lies inside or outside as a whole
+      v = *(const f32x4*)(row + min(k, K - 4));
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; e++) v[e] = k + e < K ? row[k + e] : 0.f;
+    }
+    return v;
+  };
+  // The wave's run, counted in units of H pieces of 16: two pieces make one of its 32-wide
+  // steps.  (A unit past the last reads inside the matrix again and is not multiplied: no load
+  // is under a condition.)
+  const int units = (steps - wave + GF_WAVES - 1) / GF_WAVES * (2 / H);
+  auto fetch = [&](int u, f32x4 (&af)[MF][H], f32x4 (&wf)[NF][H]) {
+    const int p = min(u, units - 1) * H;
+    const int k = (wave + p / 2 * GF_WAVES) * 32 + p % 2 * 16 + 4 * q;
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+#pragma unroll
+      for (int i = 0; i < MF; i++) af[i][h] = piece(ap[i], k + 16 * h);
+#pragma unroll
+      for (int j = 0; j < NF; j++) wf[j][h] = piece(wp[j], k + 16 * h);
+    }
+  };
+  f32x4 acc[MF][NF];
+#pragma unroll
+  for (int i = 0; i < MF; i++)
+#pragma unroll
+    for (int j = 0; j < NF; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // W is the first operand: a lane then holds columns 4 q + 0..3 of row r of C
+  auto multiply = [&](int u, f32x4 (&a)[MF][H], f32x4 (&w)[NF][H]) {
+    if (HOW == 1) {
+#pragma unroll
+      for (int h = 0; h < H; h++) {
+        const int p = u * H + h;
+        if ((wave + p / 2 * GF_WAVES) * 32 + p % 2 * 16 + 4 * q < K) continue;
+#pragma unroll
+        for (int i = 0; i < MF; i++) a[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < NF; j++) w[j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < H; h++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int i = 0; i < MF; i++)
+#pragma unroll
+          for (int j = 0; j < NF; j++)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][h][e], a[i][h][e], acc[i][j], 0, 0, 0);
+  };
+  // Unit u lies in register set u % AHEAD; the loads of the next AHEAD - 1 units are on their
+  // way.  (No branch lies between a load and its product inside the loop: the load would be
+  // sunk behind it.)
+  f32x4 a[AHEAD][MF][H], w[AHEAD][NF][H];
+  if (wave < steps) {
+#pragma unroll
+    for (int t = 0; t < AHEAD - 1; t++) fetch(t, a[t], w[t]);
+    int u = 0;
+    for (; u + AHEAD <= units; u += AHEAD) {
+#pragma unroll
+      for (int t = 0; t < AHEAD; t++) {
+        fetch(u + t + AHEAD - 1, a[(t + AHEAD - 1) % AHEAD], w[(t + AHEAD - 1) % AHEAD]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(u + t, a[t], w[t]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < AHEAD - 1; t++)
+      if (u + t < units) multiply(u + t, a[t], w[t]);
+  }
+#pragma unroll
+  for (int half = GF_WAVES / 2; half > 0; half /= 2) {
+    if (wave >= half && wave < 2 * half) {
+#pragma unroll
+      for (int i = 0; i < MF; i++)
+#pragma unroll
+        for (int j = 0; j < NF; j++) part[wave - half][i * NF + j][lane] = acc[i][j];
+    }
+    __syncthreads();
+    if (wave < half) {
+#pragma unroll
+      for (int i = 0; i < MF; i++)
+#pragma unroll
+        for (int j = 0; j < NF; j++) acc[i][j] += part[wave][i * NF + j][lane];
+    }
+    __syncthreads();
+  }
+  if (wave > 0) return;
+  const bool whole = ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
+#pragma unroll
+  for (int i = 0; i < MF; i++) {
+    const int m = m0 + 16 * i + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < NF; j++) {
+      const int n = n0 + 16 * j + 4 * q;
+      float* dst = C + (size_t)m * ldc + n;
+      if (whole && n + 4 <= N) *(f32x4*)dst = acc[i][j];
+      else
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          if (n + e < N) dst[e] = acc[i][j][e];
+    }
+  }
+}
+
+template <int MF, int NF, int H, int AHEAD>
+static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc, int M, int N, int K,
+                      hipStream_t s) {
+  const int tiles_m = (M + 16 * MF - 1) / (16 * MF), tiles_n = (N + 16 * NF - 1) / (16 * NF);
+  ZK_REQUIRE((long long)tiles_m * tiles_n < 2147483647LL, "zk_gemm_plain: too many tiles");
+  const bool vec = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+  const dim3 grid(tiles_m * tiles_n);
+  const int how = !vec ? 0 : K % 32 ? 1 : 2;
+  auto kernel = how == 2 ? gemm_f32_kernel<MF, NF, H, AHEAD, 2> : how == 1 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1> : gemm_f32_kernel<MF, NF, H, AHEAD, 0>;
+  kernel<<<grid, 64 * GF_WAVES, 0, s>>>(A, lda, W, C, ldc, M, N, K, tiles_m, tiles_n);
+  return zk_launch_status("zk_gemm_plain");
+}
+
+#endif  // ZSE_ACT_BF16
+
 extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
                              int M, int N, int K, void* stream) {
   ZK_REQUIRE(M >= 0 && N > 0 && K > 0, "zk_gemm_plain: bad sizes");
   ZK_REQUIRE(lda >= K && ldc >= N, "zk_gemm_plain: leading dimensions too small");
   if (M == 0) return 0;
-  dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
-  ZK_REQUIRE(grid.y <= 65535, "zk_gemm_plain: too many rows");
+  ZK_REQUIRE((M + 63) / 64 <= 65535, "zk_gemm_plain: too many rows");
   hipStream_t s = (hipStream_t)stream;
+#if ZSE_ACT_BF16
+  dim3 grid((N + GP_BN - 1) / GP_BN, (M + GP_BM - 1) / GP_BM);
   if (c_is_f32)
     gemm_plain_kernel<act_t, float><<<grid, 256, 0, s>>>((const act_t*)A, lda, (const act_t*)W,
                                                          (float*)C, ldc, M, N, K);
@@ -70,4 +244,17 @@ extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int
     gemm_plain_kernel<act_t, act_t><<<grid, 256, 0, s>>>((const act_t*)A, lda, (const act_t*)W,
                                                          (act_t*)C, ldc, M, N, K);
   return zk_launch_status("zk_gemm_plain");
+#else
+  // 64 x 64 where the CUs then work through four rounds of blocks or more (2048 x 8192 x 1024:
+  // 433 us against 459 with 32 x 32, but 303 x 8192 x 1024, 2.5 rounds: 83 against 77), 32 x 32
+  // otherwise; up to sixteen rows two strips of sixteen columns where every CU then has two
+  // blocks (4 x 32768 x 1024: 21.5 against 24.0 us), one where it has not (1 x 1024 x 4096: 10.8
+  // against 18.1).
+  auto blocks = [&](int mf, int nf) { return (long)((M + 16 * mf - 1) / (16 * mf)) * ((N + 16 * nf - 1) / (16 * nf)); };
+  const float *a = (const float*)A, *w = (const float*)W;
+  if (M > 16 && blocks(4, 4) >= 1024) return launch_f32<4, 4, 1, 3>(a, lda, w, (float*)C, ldc, M, N, K, s);
+  if (M > 16) return launch_f32<2, 2, 1, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+  if (blocks(1, 2) >= 512) return launch_f32<1, 2, 2, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+  return launch_f32<1, 1, 2, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+#endif
 }
