@@ -32,3 +32,57 @@ def test_product(rt, M, N, K, gap):
     for m in {0, M // 2, M - 1}:        # a row's bits do not depend on the rows beside it
         k.zk_gemm_plain(A.ptr + 4 * m * (K + gap), K + gap, W.ptr, one.ptr, N, 1, 1, N, K, rt.stream)
         assert np.array_equal(rt.download(one)[0], got[m, :N]), m
+
+
+# heads, key heads (one to seventeen heads a key head), sizes of keys and values, page, window, first keys kept
+@pytest.mark.parametrize("nh,nkv,hd,vd,bs,window,keep", [(4, 2, 64, 64, 16, 0, 0), (3, 1, 20, 36, 4, 7, 0), (17, 1, 128, 128, 16, 70, 3),
+                                                         (6, 6, 256, 256, 8, 0, 0), (10, 2, 132, 64, 32, 33, 0), (16, 1, 4, 4, 1, 0, 0)])
+def test_attention(rt, nh, nkv, hd, vd, bs, window, keep):
+    k = rt.kernels("float32")
+    rng = np.random.default_rng(nh * hd + bs)
+    reqs = [(60, 9), (0, 5), (200, 1), (63, 2), (1, 1)]            # tokens before, tokens: runs that share blocks
+    pages = sum(-(-(a + n) // bs) for a, n in reqs) + 1
+    kc, vc = (np.full((pages, nkv, bs, d), np.nan, np.float32) for d in (hd, vd))
+    table = np.full((len(reqs), max(-(-(a + n) // bs) for a, n in reqs)), -1, np.int32)
+    q, pos, own, want, seen_by = [], [], [], [], []
+    sinks, free = rng.normal(size=nh).astype(np.float32), list(rng.permutation(pages))
+    gates = rng.normal(size=(sum(n for _, n in reqs) + 1, nh)).astype(np.float32)
+    for r, (past, n) in enumerate(reqs):
+        ks, vs, qs = (rng.normal(size=(m, g, d)).astype(np.float32) for m, g, d in ((past + n, nkv, hd), (past + n, nkv, vd), (n, nh, hd)))
+        if r == 0:
+            vs[past + n - 1] = np.inf               # the last token's own value: no earlier token of its block sees it
+        for j in range(past + n):
+            if j % bs == 0:
+                table[r, j // bs] = free.pop()
+            kc[table[r, j // bs], :, j % bs], vc[table[r, j // bs], :, j % bs] = ks[j], vs[j]
+        for i in range(n):
+            p = past + i
+            sees = [j for j in range(p + 1) if not window or j > p - window or j < keep]
+            o = np.zeros((nh, vd))
+            for h in range(nh):
+                g = h // (nh // nkv)
+                s = 30 * np.tanh(ks[sees, g].astype(np.float64) @ qs[i, h].astype(np.float64) * 0.2 / 30)
+                w = np.exp(s - s.max())
+                with np.errstate(all="ignore"):
+                    o[h] = w @ vs[sees, g].astype(np.float64) / (w.sum() + np.exp(sinks[h] - s.max())) / (1 + np.exp(-gates[len(q), h]))
+            q.append(qs[i]), pos.append(p), own.append(r), want.append(o)
+        if r == 1:                                  # a padding row between two requests
+            q.append(np.zeros((nh, hd), np.float32)), pos.append(-1), own.append(0), want.append(np.zeros((nh, vd)))
+    T = len(q)
+    Q, KC, VC, TBL, G, S = (rt.upload(np.ascontiguousarray(x)) for x in (np.stack(q), kc, vc, table, gates, sinks))
+    POS, REQ, OUT = rt.upload(np.array(pos, np.int32)), rt.upload(np.array(own, np.int32)), rt.zeros((T, nh, vd), "float32")
+
+    def run(t, n):
+        k.zk_attention_plain_gated(Q.ptr + 4 * t * nh * hd, nh * hd, KC.ptr, VC.ptr, TBL.ptr, table.shape[1], REQ.ptr + 4 * t,
+                                   POS.ptr + 4 * t, OUT.ptr + 4 * t * nh * vd, n, nh, nkv, hd, vd, bs, 0.2, 30.0, window, 0, None, 0, S.ptr,
+                                   0, 0, 0, keep, G.ptr + 4 * t * nh, nh, rt.stream)
+        return rt.download(OUT)
+    got, want = run(0, T), np.stack(want)
+    fine = np.isfinite(want)
+    assert np.array_equal(fine, np.isfinite(got)) and not fine[8].all() and fine[:8].all()
+    # scores of up to about hd sums, weights by exp of them: hd + 200 roundings of 2^-24, eight times over
+    assert np.abs(got[fine] - want[fine]).max() < 8 * 2.0 ** -24 * (hd + 200)
+    rt.zero_(OUT)
+    for t in range(T):                              # each token alone: the same bits
+        alone = run(t, 1)
+    assert np.array_equal(alone[9:], got[9:]) and np.array_equal(alone[:8], got[:8])

@@ -20,6 +20,8 @@
 // contiguous K/V instead (:859-958) and never applies a window (:883).
 #include "common.h"
 
+#include <climits>
+
 #define AP_MAX_HD 256
 
 // MAXD: the most channels a head's queries, keys and values have (256, or 1024 for the wide rows
@@ -138,6 +140,259 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
   }
 }
 
+#if !ZSE_ACT_BF16
+// The 32-bit path's attention on the 32-bit matrix cores (16x16x4), for heads of whole 16-byte
+// pieces.  Sixteen rows, the query heads of one key head times as many neighbouring tokens of
+// one request as fit, share every key and value that is read.
+//
+// Scores are taken as keys x queries: lane l then holds, for the query l % 16, the keys
+// 16 f + 4 (l / 16) + e of a tile of 64 (f, e = 0..3), which is just what the second product,
+// values x weights, wants as its operand, so nothing is moved between lanes but the maxima and
+// sums over the four lanes of a query.  Both products take their sums in the order of the
+// registers (k = 4 (l / 16) + e of each piece of 16), keys and values come as 16 bytes a lane.
+//
+// The keys' tiles of 64, aligned to absolute positions, go round-robin over the block's waves
+// (tile j / 64 to wave j / 64 % WAVES); each keeps a running maximum and sum, and the waves'
+// sums are joined in their order.  So a row's sums are cut and ordered by its position alone,
+// however the step was cut, and rows that share a block do not touch each other: a key that a
+// row does not see has weight 0 there, and a tile with such a key and a value that is not
+// finite is taken value by value.
+//
+// Bound by the latency of the loads for few tokens and by the matrix cores for many.  Measured
+// (us; before: a wave per token and head whose lanes each walked a key's row):
+//   303 tokens, 8 heads of 128, contexts of 300 and three of 50 to 700: 852 -> 55.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int MAXD, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
+    const float* __restrict__ q, int q_stride, const float* __restrict__ kcache, const float* __restrict__ vcache,
+    const int* __restrict__ block_table, int max_blocks, const int* __restrict__ req_of_token,
+    const int* __restrict__ positions, float* __restrict__ out, int T, int nh, int nkv, int hd, int vd, int bs,
+    float scale, float softcap, int window, const float* __restrict__ v_freq, int v_interleaved,
+    const float* __restrict__ sinks, int chunk, int unit_sink, int keep, const float* __restrict__ gate, int gate_ld) {
+  constexpr int QC = MAXD / 16, VC = MAXD / 64;       // pieces of 16 channels of a query, of 64 of a value
+  __shared__ float s_acc[WAVES][16][MAXD];
+  __shared__ float s_m[WAVES][16], s_l[WAVES][16];
+  const int group = nh / nkv, chunks = (group + 15) / 16;
+  const int kvh = blockIdx.y / chunks, h0 = blockIdx.y % chunks * 16;       // first of the block's heads in the group
+  const int gh = min(16, group - h0), tb = max(1, 16 / group);              // heads, tokens of a block
+  const int t0 = blockIdx.x * tb, n_tok = min(tb, T - t0);
+  // Block z takes the z-th run of neighbouring tokens of one request; padding rows (position < 0) belong to none.
+  int first = 0, last = -1, seen = -1;
+  bool running = false;
+  for (int i = 0; i < n_tok; i++) {
+    const bool live = positions[t0 + i] >= 0;
+    const bool starts = live && (!running || req_of_token[t0 + i] != req_of_token[t0 + i - 1]);
+    if (starts && ++seen == (int)blockIdx.z) first = i;
+    if (live && seen == (int)blockIdx.z) last = i;
+    running = live;
+    if (!live && blockIdx.z == 0)
+      for (int x = threadIdx.x; x < gh * vd; x += 64 * WAVES)
+        out[((size_t)(t0 + i) * nh + (size_t)kvh * group + h0) * vd + x] = 0.f;
+  }
+  if (last < 0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, qd = lane >> 4;
+  const int rows = (last - first + 1) * gh;
+  auto lowest = [&](int pos) { return window > 0 ? max(pos - window + 1, 0) : chunk > 0 ? pos / chunk * chunk : 0; };
+  // the run's keys: from the lowest that a token of it sees to its highest position
+  int seg_lo = INT_MAX, seg_hi = -1;
+  for (int i = first; i <= last; i++) {
+    const int p = positions[t0 + i];
+    seg_lo = min(seg_lo, lowest(p));
+    seg_hi = max(seg_hi, p);
+  }
+  const int row = min(r, rows - 1);                  // rows past the last repeat it and are not stored
+  const int tok = t0 + first + row / gh, head = kvh * group + h0 + row % gh;
+  const int pos = positions[tok], lo = lowest(pos);
+  const int* table = block_table + (size_t)req_of_token[tok] * max_blocks;
+
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 qf[QC];
+#pragma unroll
+  for (int c = 0; c < QC; c++) {
+    const int d = 16 * c + 4 * qd;
+    qf[c] = d < hd ? *(const f32x4*)(q + (size_t)tok * q_stride + (size_t)head * hd + d) : zero;
+  }
+  float m = -INFINITY, l = 0.f;
+  f32x4 acc[VC][4];            // [c][e][i]: channel 64 c + 16 qd + 4 i + e of the lane's query
+#pragma unroll
+  for (int c = 0; c < VC; c++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) acc[c][e] = zero;
+
+  const int lo_tile = seg_lo / 64, kept_tiles = (keep + 63) / 64;
+  const int tile0 = keep > 0 ? 0 : lo_tile, tile1 = seg_hi / 64 + 1;
+  for (int tile = tile0 + (wave - tile0 % WAVES + WAVES) % WAVES; tile < tile1; tile += WAVES) {
+    if (tile >= kept_tiles && tile < lo_tile) continue;
+    const int j0 = tile * 64;
+    // the cache row of key 16 f + r; a key that no row of the run sees is never read (row -1)
+    int at[4];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      const int j = j0 + 16 * f + r;
+      at[f] = -1;
+      if (j <= seg_hi && (j >= seg_lo || j < keep)) {
+        const int page = table[j / bs];
+        if (page >= 0) at[f] = (page * nkv + kvh) * bs + j % bs;
+      }
+    }
+    f32x4 s[4];
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      s[f] = zero;
+      const float* kr = kcache + (size_t)max(at[f], 0) * hd;
+#pragma unroll
+      for (int c = 0; c < QC; c++) {
+        const int d = 16 * c + 4 * qd;
+        const f32x4 k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
+#pragma unroll
+        for (int e = 0; e < 4; e++) s[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], qf[c][e], s[f], 0, 0, 0);
+      }
+    }
+    float top = -INFINITY;
+    bool all = true;             // the lane's query sees all of the lane's keys
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int j = j0 + 16 * f + 4 * qd + e;
+        float x = s[f][e] * scale;
+        if (softcap > 0.f) x = softcap * tanhf(x / softcap);
+        const bool sees = (j >= lo || j < keep) && j <= pos;
+        all = all && sees;
+        s[f][e] = sees ? x : -INFINITY;
+        top = fmaxf(top, s[f][e]);
+      }
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float m_new = fmaxf(m, top);
+    const float corr = m == m_new ? 1.f : expf(m - m_new);
+    float sum = 0.f;
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int j = j0 + 16 * f + 4 * qd + e;
+        s[f][e] = (j >= lo || j < keep) && j <= pos ? expf(s[f][e] - m_new) : 0.f;
+        sum += s[f][e];
+      }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    l = l * corr + sum;
+    m = m_new;
+#pragma unroll
+    for (int c = 0; c < VC; c++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[c][e] *= corr;
+    const bool whole = __all(all);
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
+      int va[4];
+      bool fine = true;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        va[e] = __shfl(at[f], 4 * qd + e);
+#pragma unroll
+        for (int c = 0; c < VC; c++) {
+          const int d = 64 * c + 4 * r;
+          v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
+        }
+      }
+      if (!whole) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int c = 0; c < VC; c++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) fine = fine && fabsf(v[e][c][x]) < INFINITY;
+      }
+      if (__all(fine)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int c = 0; c < VC; c++)
+#pragma unroll
+            for (int x = 0; x < 4; x++)
+              acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
+      } else {
+        for (int kk = 0; kk < 16; kk++) {        // rare: each query takes the keys that it sees
+          const int j = j0 + 16 * f + kk, av = __shfl(at[f], kk);
+          float p = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const float x = __shfl(s[f][e], (kk >> 2) * 16 + r);
+            if (e == (kk & 3)) p = x;
+          }
+          if (av < 0 || !((j >= lo || j < keep) && j <= pos)) continue;
+#pragma unroll
+          for (int c = 0; c < VC; c++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              const int d = 64 * c + 16 * qd + 4 * i;
+              if (d >= vd) continue;
+#pragma unroll
+              for (int e = 0; e < 4; e++) acc[c][e][i] = fmaf(vcache[(size_t)av * vd + d + e], p, acc[c][e][i]);
+            }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < VC; c++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      *(f32x4*)&s_acc[wave][r][64 * c + 16 * qd + 4 * i] = f32x4{acc[c][0][i], acc[c][1][i], acc[c][2][i], acc[c][3][i]};
+  if (qd == 0) {
+    s_m[wave][r] = m;
+    s_l[wave][r] = l;
+  }
+  __syncthreads();
+  // a thread joins four channels of a row over the waves
+  for (int x = threadIdx.x; x < rows * (vd / 4); x += 64 * WAVES) {
+    const int rr = x / (vd / 4), d = x % (vd / 4) * 4;
+    const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
+    float top = -INFINITY, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) top = fmaxf(top, s_m[w][rr]);
+    f32x4 o = zero;
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) {
+      const float f = s_m[w][rr] == top ? 1.f : expf(s_m[w][rr] - top);
+      den += s_l[w][rr] * f;
+      o += *(const f32x4*)&s_acc[w][rr][d] * f;
+    }
+    if (sinks != nullptr || unit_sink) {
+      const float sk = sinks != nullptr ? sinks[h] : 0.f;
+      const float m_new = fmaxf(top, sk), corr = expf(top - m_new);
+      den = den * corr + expf(sk - m_new);
+      o *= corr;
+    }
+    float inv = 1.f / den;
+    if (gate != nullptr) inv *= 1.f / (1.f + expf(-gate[(size_t)t * gate_ld + h]));
+    o *= inv;
+    if (v_freq == nullptr) *(f32x4*)(out + ((size_t)t * nh + h) * vd + d) = o;
+    else *(f32x4*)&s_acc[0][rr][d] = o;          // the place that this thread alone has read
+  }
+  if (v_freq == nullptr) return;
+  // values were turned by their own positions when they were stored: the sum is turned back
+  // by the query's position, pair m by -pos * v_freq[m]
+  __syncthreads();
+  const int half = vd / 2;
+  for (int x = threadIdx.x; x < rows * half; x += 64 * WAVES) {
+    const int rr = x / half, m2 = x % half;
+    const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
+    float sn, cs, ra, rb;
+    sincosf(-(float)positions[t] * v_freq[m2], &sn, &cs);
+    const int ia = v_interleaved ? 2 * m2 : m2, ib = v_interleaved ? 2 * m2 + 1 : m2 + half;
+    rotate_pair(s_acc[0][rr][ia], s_acc[0][rr][ib], sn, cs, ra, rb);
+    out[((size_t)t * nh + h) * vd + ia] = ra;
+    out[((size_t)t * nh + h) * vd + ib] = rb;
+  }
+}
+#endif  // !ZSE_ACT_BF16
+
 // softcap <= 0: no cap; window <= 0: every earlier key is visible.  v_transposed: V is
 // cached as [page][kv head][hd][bs] instead of [page][kv head][bs][hd].
 // hd: the size of a head's queries and keys; vd: of its values (the output's too).  v_freq (may
@@ -166,6 +421,26 @@ extern "C" int zk_attention_plain_gated(const void* q, int q_stride, const void*
   ZK_REQUIRE(q_stride >= nh * hd, "zk_attention_plain: q row stride too small");
   ZK_REQUIRE(!v_in_k || (vd <= hd && !v_transposed), "zk_attention_plain: values inside keys are no wider than the keys");
   if (T == 0) return 0;
+#if !ZSE_ACT_BF16
+  // Heads of up to 256 channels in whole 16-byte pieces, keys and values in rows of their own:
+  // the matrix-core kernel.  Everything else (values inside keys, odd sizes) is taken key by key.
+  if (hd <= 256 && vd <= 256 && hd % 4 == 0 && vd % 4 == 0 && q_stride % 4 == 0 && !v_in_k && !v_transposed &&
+      ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)out) % 16 == 0 &&
+      (long long)nkv * ((nh / nkv + 15) / 16) <= 65535) {
+    const int group = nh / nkv, tb = group < 16 ? 16 / group : 1, most = hd > vd ? hd : vd;
+    const dim3 blocks((T + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
+#define ZK_ATTENTION_F32(D_, W_)                                                                                      \
+  attention_f32_kernel<D_, W_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                          \
+      (const float*)q, q_stride, (const float*)kcache, (const float*)vcache, block_table, max_blocks, req_of_token,   \
+      positions, (float*)out, T, nh, nkv, hd, vd, bs, scale, softcap, window, v_freq, v_interleaved, sinks, chunk,    \
+      unit_sink, keep, (const float*)gate, gate_ld)
+    if (most <= 64) ZK_ATTENTION_F32(64, 8);
+    else if (most <= 128) ZK_ATTENTION_F32(128, 8);
+    else ZK_ATTENTION_F32(256, 4);
+#undef ZK_ATTENTION_F32
+    return zk_launch_status("zk_attention_plain");
+  }
+#endif
   dim3 grid(T, nh);
   if (hd <= AP_MAX_HD && vd <= AP_MAX_HD)
     attention_plain_kernel<AP_MAX_HD><<<grid, 64, 0, (hipStream_t)stream>>>(
