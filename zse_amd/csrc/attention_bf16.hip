@@ -26,13 +26,13 @@
 // cut into ranges over several blocks, joined by attn_portion_join_kernel (few groups with long
 // contexts: a portion of a prompt behind thousands of tokens).
 //
-// Decoded tokens use a split variant: the keys are cut into chunks of 64 (or 32, as
-// the caller says) aligned to absolute positions, one wave per chunk writes (max, sum, O)
-// and a second kernel joins the chunks in order; the cut is the caller's choice and never
-// follows from the batch, so a request's result is the same whoever shares its step.  With
-// at most 16 heads a KV head the chunks run on 16x16x32 MFMAs (attn_decode_kernel):
-// a single query token fills only g of a tile's columns, and the narrower tile
-// halves both the accumulator registers and the wasted work, so two waves fit a SIMD.
+// Decoded tokens use a split variant: the keys are cut into chunks aligned to absolute positions,
+// each leaves (max, sum, O) and a second kernel joins the chunks in order; the cut never follows
+// from the batch, so a request's result is the same whoever shares its step.  With at most 16
+// heads a KV head a wave takes 32 keys on 16x16x32 MFMAs and a block of four waves leaves one
+// partial result (attn_decode_kernel): a single query token fills only g of a tile's columns,
+// and the narrower tile halves both the accumulator registers and the wasted work.  Otherwise a
+// wave takes 64 keys on 32x32x16 MFMAs and leaves a result of its own.
 //
 // A head's values may be half or twice as wide as its keys.  Where a window keeps the sequence's first
 // keys in sight, the tiles (or a decoded token's chunks) of those keys come first and are
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64) void attn_portion_join_kernel(AttnParams p, int
 
 // Joins the chunks of a decoded token's attention, in chunk order: a block per
 // (request, head), a thread per channel; the chunks' weights exp(m_c - m) are computed once.
-#define ATT_MAX_CHUNKS 1024
+#define ATT_MAX_CHUNKS 2048      // 262,144 keys in parts of 128
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ part_o,
                                                            const float* __restrict__ part_ml,
                                                            const int* __restrict__ q_start,
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   const int np = kept + c1 - c0 + 1;
   // the first partial results of the thread's channel are asked for now: they come in while
   // the weights are worked out (a part past the last is read from the last and not used)
-  constexpr int PF = 16;
+  constexpr int PF = 32;
   const int d0 = min((int)threadIdx.x, hd - 1);
   float pf[PF];
   {
@@ -277,17 +277,14 @@ static bool decode_on_narrow_tiles(int nh, int nkv, int hd) { return nh / nkv <=
 long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chunk) {
   if (nkv <= 0 || nh % nkv) return 0;
   const int chunk = decode_chunk == 32 ? 32 : ATT_CHUNK;
-  const long long span = decode_on_narrow_tiles(nh, nkv, hd) ? 4LL * chunk : ATT_CHUNK;
-  return span * ATT_MAX_CHUNKS;
+  return decode_on_narrow_tiles(nh, nkv, hd) ? 4LL * chunk * 1024 : ATT_CHUNK * 1024LL;
 }
 
 // Requests [0, r_prefill) hold portions of more than one token (max_q_len the longest);
 // requests [r_prefill, R) hold one token each and use the split variant over max_ctx keys.
-// decode_chunk: keys a wave of the split variant takes on the 16-wide tiles, 32 or 64 (0: 64).
-// It fixes where the sums over keys are cut, and so the bits of the result: a caller that wants
-// a request's result not to depend on the rest of the batch passes the same value in every
-// step.  32 gives twice the waves, each with one load from memory in its chain instead of
-// two: better for few requests with short contexts, worse for many.
+// decode_chunk: 32 or 64 (0: 64) sets the longest context that decoded tokens on the 16-wide tiles
+// take, 131,072 or 262,144 keys.  Their keys are cut after every 128 either way (blocks of 256 keys
+// were 3 to 20 % slower), so a request's result does not depend on it.
 // mask_chunk > 0: a row sees the keys of its own chunk of that many positions (counted from
 // position 0) instead of a window; sink: a key of score 0 without a value in every denominator;
 // wide_weights: the weights keep 16 bits of mantissa in the product with the values.
@@ -425,14 +422,10 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
     dim3 grid((nchunks + 3) / 4, nkv, n_dec);
     int rc = 0;
     int span = ATT_CHUNK;        // keys one partial result covers
-    p.chunk = ATT_CHUNK;
     if (decode_on_narrow_tiles(nh, nkv, hd)) {
-      if (decode_chunk == 32) {
-        p.chunk = ATT_CHUNK / 2;
-        grid.x = (2 * nchunks + 3) / 4;
-      }
-      // the block joins its four chunks: one partial result per 4 chunks of keys
-      span = 4 * p.chunk;
+      // a block joins its four waves: one partial result per ATT_DECODE_SPAN keys
+      span = ATT_DECODE_SPAN;
+      grid.x = (max_ctx + span - 1) / span;
       p.nchunks = grid.x;
       // a window covers at most ceil(window / span) + 1 blocks of span keys
       const int reach = mask_chunk > 0 ? mask_chunk : window;

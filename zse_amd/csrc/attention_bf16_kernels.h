@@ -5,6 +5,8 @@
 #pragma once
 #include "common.h"
 
+#include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #if ZSE_ACT_BF16
@@ -15,6 +17,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define ATT_CHUNK 64
+#define ATT_DECODE_SPAN 128    // keys of a partial result of a decoded token on 16-wide tiles
 #define ATT_MOST_RANGES 8      // ranges of keys a block of rows of a portion is cut into, at most
 
 struct AttnParams {
@@ -43,7 +46,7 @@ struct AttnParams {
   int r_begin;            // first request of this launch
   int nchunks;            // split: chunks the grid covers
   int from_window;        // decode: block 0 of a request is the one its window begins in
-  int chunk;              // decoded tokens on 16-wide tiles: keys a wave takes, 32 or 64
+  int chunk;              // portions with their keys in ranges: tiles of a range
   int mask_chunk;         // > 0: a row sees the keys of its own chunk of this many positions only (no window then)
   int keep;               // beside its window a row sees the first ``keep`` keys of its sequence
   int sink;               // 1: a key of score 0 without a value joins every row's denominator
@@ -744,189 +747,189 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
     }
 }
 
-// One wave per (request, KV head, chunk of 64 keys) for requests that bring one token.
-// Columns of every tile are the g query heads of the KV head (col = lane % 16), rows are
-// keys (first product) or channels (second product).
+// One wave per (request, KV head, 32 keys) for requests that bring one token; a block's four
+// waves take 128 neighbouring keys and leave one partial result.  Columns of every tile are
+// the g query heads of the KV head (col = lane % 16), rows are keys (first product) or channels
+// (second product).  Row 4 a + i of score tile t (a, i = 0..3) is key 8 a + 4 t + i of the 32, so
+// that a lane's eight weights belong to eight neighbouring keys, 8 kq + 0..7: its operand of the
+// second product, and 16 bytes of a channel of the transposed values.
+//
+// The time is the way from memory.  A wave has one tile only, so its chain holds one or two waits
+// for memory, and blocks are small, so that the CUs get even shares of requests of uneven
+// lengths.  Measured (us, with the joining launch, 8 heads over 4 of 256 channels) against blocks
+// of four waves with two tiles each one after the other and values in 8-byte pieces: 64 requests
+// of 200 to 3,840 keys 146 -> 105 (109 by the order of the blocks alone), of 4,096 keys 192 ->
+// 193 (5.6 TB/s), 23 of 130 to 2,000 35.7 -> 27.1, 8 of 4,000 31.6 -> 31.1, 1 of 4,000 13.3 ->
+// 11.8.  Eight waves of one tile each: 119, 202, 33.1, 32.9.
 template <int HD32, int VD16>
-__global__ __launch_bounds__(256, 2) void attn_decode_kernel(AttnParams p) {
+__global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
   constexpr int KS = HD32;       // 32-wide steps over head_dim
   constexpr int DT = VD16;       // 16-channel output tiles
+  constexpr int NW = 4, SPAN = ATT_DECODE_SPAN;      // waves and keys of a block
+  static_assert(SPAN == 32 * NW, "a wave takes 32 keys");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, kq = lane >> 4;
   const int r = p.r_begin + blockIdx.z;
   const int kvh = blockIdx.y;
+  // A request's blocks are counted from a place that differs from one (request, key head) to the
+  // next.  Blocks go to the 8 XCDs in turn, so with 8 or 16 of them a request block 0 of every
+  // request would run on the first XCD and the last one on the last: with requests of uneven
+  // lengths, whose last blocks have no keys, the first XCD then reads half as much again as the
+  // average (64 requests of 200 to 3,840 keys, 4 key heads of 256: 146 -> 109 us).
+  int block_x = (blockIdx.x + blockIdx.y + gridDim.y * blockIdx.z) % gridDim.x;
   // Where the window is much shorter than the longest context, the grid covers a window's
   // blocks only and counts them from the block the request's window begins in.
-  int block_x = blockIdx.x;
   // In front of them come the blocks of the kept first keys, which every request has.
-  const int kept_blocks = (p.keep + 4 * p.chunk - 1) / (4 * p.chunk);
+  const int kept_blocks = (p.keep + SPAN - 1) / SPAN;
   if (p.from_window && block_x >= kept_blocks)
-    block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / (4 * p.chunk), kept_blocks) - kept_blocks;
-  const int chunk = block_x * 4 + wave;
+    block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / SPAN, kept_blocks) - kept_blocks;
+  const int key0 = block_x * SPAN + 32 * wave;
   const int* table = p.block_table + (size_t)r * p.max_blocks;
   const int hd = p.hd, vd = p.vd, bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
-  // The pages of the chunk's (up to two) tiles are asked for before the request's length is
-  // known, beside it: where a key lies follows from the chunk alone.  A key past the context is
-  // masked below; a hole in the table reads page 0, which the caller keeps cleared, and the
-  // places of a request's last page behind its last token are cleared too (a masked value
-  // still meets a weight of 0 in the second product, and 0 x NaN is NaN).
-  int kpage[2][2], vpage[2][2];
+  // The pages of the wave's keys are asked for before the request's length is known, beside it:
+  // where a key lies follows from the block alone.  A key past the context is masked below; a
+  // hole in the table reads page 0, which the caller keeps cleared, and the places of a
+  // request's last page behind its last token are cleared too (a masked value still meets a
+  // weight of 0 in the second product, and 0 x NaN is NaN).
+  int kpage[2], vpage[2];
 #pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int k0 = chunk * p.chunk + 32 * i;
-#pragma unroll
-    for (int t = 0; t < 2; t++) {
-      kpage[i][t] = table[min((k0 + 16 * t + col) >> bsh, p.max_blocks - 1)];
-      vpage[i][t] = table[min((k0 + 16 * t + 4 * kq) >> bsh, p.max_blocks - 1)];
-    }
+  for (int t = 0; t < 2; t++) {
+    kpage[t] = table[min((key0 + 8 * (col >> 2) + 4 * t + (col & 3)) >> bsh, p.max_blocks - 1)];
+    vpage[t] = table[min((key0 + 8 * kq + 4 * t) >> bsh, p.max_blocks - 1)];
   }
   const int n = p.q_start[r + 1] - p.q_start[r];
   if (n <= 0) return;
   const int pos = p.ctx_len[r] - 1;
   const int row_lo = first_key(p, pos);
-  // a block whose four chunks all lie past the context or before the window ends here, all
-  // its waves alike: the grid is sized for the longest context the caller allows
-  const int first_chunk = block_x * 4;
-  if (first_chunk * p.chunk > pos ||
-      (first_chunk * p.chunk + 4 * p.chunk - 1 < row_lo && first_chunk * p.chunk >= p.keep)) return;
-  const int key_lo = chunk * p.chunk < p.keep ? chunk * p.chunk : max(row_lo, chunk * p.chunk);
-  const int key_hi = min(pos, chunk * p.chunk + p.chunk - 1);
-  const bool active = key_lo <= key_hi;          // a wave without keys still meets the others at the barrier
+  // a block whose keys all lie past the context or before the window ends here, all its waves
+  // alike: the grid is sized for the longest context the caller allows
+  if (block_x * SPAN > pos || (block_x * SPAN + SPAN - 1 < row_lo && block_x * SPAN >= p.keep)) return;
+  // a wave without keys still meets the others at the barrier
+  const bool active = key0 <= pos && (key0 + 31 >= row_lo || key0 < p.keep);
   const int g = p.nh / p.nkv;
   const bool col_ok = col < g;
   const int head = q_head_of(p, kvh, col_ok ? col : 0);
   const int trow = p.q_start[r];
 
-  // the query operand waits in LDS (one 16-byte piece per lane and step), not in registers
-  __shared__ bf16x8 sq[4][KS][64];
-  {
+  extern __shared__ __align__(16) unsigned char dec_lds[];
+  float* sm_o = (float*)(dec_lds + NW * KS * 64 * sizeof(bf16x8));      // [NW][g][vd]
+  constexpr int ML = KS * 64 * sizeof(bf16x8) / sizeof(float);            // a wave's maxima and sums lie where its
+  float* sm_ml = (float*)dec_lds;                                         // queries were: [NW] x [16][2], ML apart
+  float* so = sm_o + ((size_t)wave * g + col) * vd + 4 * kq;
+  float m_run = -INFINITY, l_run = 0.f;
+  if (active) {
+    // The query operand goes from memory straight to LDS, one 16-byte piece per lane and step.
+    // (Columns past the g heads repeat the first head; nothing of them is used.)
+    bf16x8(*sq)[64] = (bf16x8(*)[64])dec_lds + wave * KS;
     const __bf16* qr = p.q + (size_t)trow * p.q_stride + (size_t)head * hd + kq * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) {
-      bf16x8 t;
-      if (col_ok) t = *(const bf16x8*)(qr + ks * 32);
-      else
-#pragma unroll
-        for (int e = 0; e < 8; e++) t[e] = (__bf16)0.f;
-      sq[wave][ks][lane] = t;
-    }
-  }
-  f32x4 o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-
-#pragma unroll
-  for (int i = 0; i < 2; i++) {
-    const int key0 = chunk * p.chunk + 32 * i;
-    if (!active || 32 * i >= p.chunk || key0 > key_hi || key0 + 31 < key_lo) continue;
+    for (int ks = 0; ks < KS; ks++)
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(qr + ks * 32),
+                                       (__attribute__((address_space(3))) void*)sq[ks], 16, 0, 0);
     bf16x8 kf[2][KS];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
-      const int kk = key0 + 16 * t + col;
-      const int page = max(kpage[i][t], 0);
-      const __bf16* kr = p.kcache + ((((size_t)page * nkv + kvh) << bsh) + (kk & bmask)) * hd + kq * 8;
+      const int kk = key0 + 8 * (col >> 2) + 4 * t + (col & 3);
+      const __bf16* kr = p.kcache + ((((size_t)max(kpage[t], 0) * nkv + kvh) << bsh) + (kk & bmask)) * hd + kq * 8;
 #pragma unroll
       for (int ks = 0; ks < KS; ks++) kf[t][ks] = *(const bf16x8*)(kr + ks * 32);
     }
     bf16x8 vf[DT];
-    {
-      const int ka = key0 + 4 * kq, kb = key0 + 16 + 4 * kq;
-      const int pa = max(vpage[i][0], 0), pb = max(vpage[i][1], 0);
-      const __bf16* va_base = p.vcache + ((((size_t)pa * (nkv >> p.v_shift) + (kvh >> p.v_shift)) * vd) << bsh) + (ka & bmask);
-      const __bf16* vb_base = p.vcache + ((((size_t)pb * (nkv >> p.v_shift) + (kvh >> p.v_shift)) * vd) << bsh) + (kb & bmask);
+    const int vheads = nkv >> p.v_shift, vh = kvh >> p.v_shift;
+    const __bf16* va = p.vcache + ((((size_t)max(vpage[0], 0) * vheads + vh) * vd) << bsh) + ((key0 + 8 * kq) & bmask);
+    const __bf16* vb = p.vcache + ((((size_t)max(vpage[1], 0) * vheads + vh) * vd) << bsh);
+    auto load_v = [&]() {
+      if (bsh >= 3) {
 #pragma unroll
-      for (int dt = 0; dt < DT; dt++) {
-        const int d = dt * 16 + col;
-        const bf16x4 va = *(const bf16x4*)(va_base + ((size_t)d << bsh));
-        const bf16x4 vb = *(const bf16x4*)(vb_base + ((size_t)d << bsh));
+        for (int dt = 0; dt < DT; dt++) vf[dt] = *(const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh));
+      } else {         // pages of four keys
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          vf[dt][e] = va[e];
-          vf[dt][4 + e] = vb[e];
+        for (int dt = 0; dt < DT; dt++) {
+          const bf16x4 x = *(const bf16x4*)(va + ((size_t)(dt * 16 + col) << bsh)), y = *(const bf16x4*)(vb + ((size_t)(dt * 16 + col) << bsh));
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            vf[dt][e] = x[e];
+            vf[dt][4 + e] = y[e];
+          }
         }
       }
-    }
+    };
+    // Values of 256 channels are asked for after the score products have used up the keys: with
+    // both at once a wave has 199 registers, two waves a SIMD, and the CU less on its way.
+    constexpr bool LATE = DT > 8;
+    if (!LATE) load_v();
+    // the queries are in LDS (the compiler does not know that the reads below depend on them)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     f32x4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
       s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ks = 0; ks < KS; ks++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks], sq[wave][ks][lane], s[t], 0, 0, 0);
+      for (int ks = 0; ks < KS; ks++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks], sq[ks][lane], s[t], 0, 0, 0);
     }
-    float mt = -INFINITY;
+    if (LATE) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v();
+    }
 #pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int key = key0 + 16 * t + 4 * kq + i;
-        float v = score_log2(p, s[t][i]);
-        v = (col_ok && (key >= row_lo || key < p.keep) && key <= key_hi) ? v : -INFINITY;
-        s[t][i] = v;
-        mt = fmaxf(mt, v);
+        const int key = key0 + 8 * kq + 4 * t + i;
+        const float v = score_log2(p, s[t][i]);
+        s[t][i] = (col_ok && (key >= row_lo || key < p.keep) && key <= pos) ? v : -INFINITY;
+        m_run = fmaxf(m_run, s[t][i]);
       }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float m_new = fmaxf(m_run, mt);
-    const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
-    float rs = 0.f;
+    m_run = fmaxf(m_run, __shfl_xor(m_run, 16, 64));
+    m_run = fmaxf(m_run, __shfl_xor(m_run, 32, 64));
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;
     bf16x8 pb8;
 #pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const float pe = __builtin_amdgcn_exp2f(s[t][i] - m_use);
-        rs += pe;
-        pb8[4 * t + i] = (__bf16)pe;
-        s[t][i] = pe;
+        s[t][i] = __builtin_amdgcn_exp2f(s[t][i] - m_use);
+        l_run += s[t][i];
+        pb8[4 * t + i] = (__bf16)s[t][i];
       }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * corr + rs;
-    m_run = m_new;
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
+    bf16x8 rest8;          // (wide weights) what the rounding left
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rest8[4 * t + i] = (__bf16)(s[t][i] - (float)pb8[4 * t + i]);
+    // the results go to LDS as they come, so that they do not hold registers beside the values
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) {
-      o[dt] *= corr;
-      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb8, o[dt], 0, 0, 0);
+      f32x4 o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb8, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      if (p.wide_weights) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], rest8, o, 0, 0, 0);
+      if (col_ok) *(f32x4*)(so + dt * 16) = o;
     }
-    if (p.wide_weights) {
+  } else if (col_ok) {
 #pragma unroll
-      for (int t = 0; t < 2; t++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) pb8[4 * t + i] = (__bf16)(s[t][i] - (float)pb8[4 * t + i]);
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb8, o[dt], 0, 0, 0);
-    }
+    for (int dt = 0; dt < DT; dt++) *(f32x4*)(so + dt * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  // the block's four chunks are joined here, in chunk order: one partial result per 256 keys
-  extern __shared__ float dyn[];
-  float* sm_ml = dyn;                 // [4][16][2]
-  float* sm_o = dyn + 4 * 16 * 2;     // [4][g][vd]
-  if (col_ok) {
-    if (kq == 0) {
-      sm_ml[(wave * 16 + col) * 2] = m_run;
-      sm_ml[(wave * 16 + col) * 2 + 1] = l_run;
-    }
-    float* so = sm_o + ((size_t)wave * g + col) * vd;
-#pragma unroll
-    for (int dt = 0; dt < DT; dt++) *(f32x4*)(so + dt * 16 + 4 * kq) = o[dt];
+  // the block's waves are joined here, in the order of their keys
+  if (col_ok && kq == 0) {
+    sm_ml[wave * ML + col * 2] = m_run;
+    sm_ml[wave * ML + col * 2 + 1] = l_run;
   }
   __syncthreads();
-  for (int idx = threadIdx.x; idx < g * vd; idx += 256) {
+  for (int idx = threadIdx.x; idx < g * vd; idx += NW * 64) {
     const int c = idx / vd, d = idx - c * vd;
-    float mw[4], m = -INFINITY;
+    float mw[NW], m = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
-      mw[w] = sm_ml[(w * 16 + c) * 2];
+    for (int w = 0; w < NW; w++) {
+      mw[w] = sm_ml[w * ML + c * 2];
       m = fmaxf(m, mw[w]);
     }
     float acc = 0.f, l = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
+    for (int w = 0; w < NW; w++) {
       const float e = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - m);
       acc += e * sm_o[((size_t)w * g + c) * vd + d];
-      l += e * sm_ml[(w * 16 + c) * 2 + 1];
+      l += e * sm_ml[w * ML + c * 2 + 1];
     }
     const size_t slot = ((size_t)(r - p.r_begin) * p.nh + q_head_of(p, kvh, c)) * p.nchunks + block_x;
     p.part_o[slot * vd + d] = acc;
@@ -972,7 +975,14 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
     case ATT_RANGES: return launch_shared_one<HD16, VD16, 4, true>(p, grid, s);
     case ATT_DECODE:
       if constexpr (HD16 % 2 == 0) {
-        const size_t lds = (4 * 16 * 2 + (size_t)4 * (p.nh / p.nkv) * p.vd) * sizeof(float);
+        const size_t lds = (size_t)4 * (p.nh / p.nkv) * p.vd * sizeof(float) + (size_t)4 * (HD16 / 2) * 64 * sizeof(bf16x8);
+        static std::atomic<bool> prepared{false};
+        if (lds > 64 * 1024 && !prepared) {      // 16 heads a KV head with values of 256 channels: 96 KB
+          if (hipFuncSetAttribute((const void*)attn_decode_kernel<HD16 / 2, VD16>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  96 * 1024) != hipSuccess)
+            return zk_fail("zk_attention_bf16: the decode kernel's LDS was refused");
+          prepared = true;
+        }
         attn_decode_kernel<HD16 / 2, VD16><<<grid, 256, lds, s>>>(p);
         break;
       } else {
