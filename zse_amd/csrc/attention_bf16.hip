@@ -272,6 +272,20 @@ size_t zk_attention_bf16_portion_workspace(int max_rows, int nh, int nkv, int hd
 // chunks at a time inside a block) or on the 32-wide ones (one partial result a chunk).
 static bool decode_on_narrow_tiles(int nh, int nkv, int hd) { return nh / nkv <= 16 && hd % 32 == 0; }
 
+// Whether they go in blocks of 256 keys instead of 128.  By what a runner's limits fix alone (its
+// decode_chunk and the width of its block tables), never by a step's requests, because it says where
+// a request's sums are cut.  The blocks' queries and results have to fit in 64 KB of LDS.
+// Measured (us, blocks of 256 against 128, 8 heads over 4 of 256 channels unless said): 64 requests
+// of 8,192 keys 367 against 384, behind a window of 4,096 188 against 200; 8 of 8,192 54 against 56;
+// 16 of 8,192, 32 heads over 16 of 128: 198 against 210.  Below the line 128 is the better one: 64 of 200
+// to 2,000 keys 70 against 63, 23 of 130 to 2,000 33 against 27.  At 4,096 it depends: full contexts
+// are better off with 256 (a whole step of 64 requests 7.20 ms against 7.27), uneven ones with 128 (64 of 200 to
+// 3,840 keys 109 us against 103, 8 of 500 to 4,000 24 against 22); the line lets no full one wait.
+static bool decode_in_long_blocks(int nh, int nkv, int hd, int vd, int bs, int max_blocks, int decode_chunk) {
+  return decode_chunk != 32 && (long long)max_blocks * bs >= ATT_DECODE_LONG_FROM &&
+         decode_long_lds(nh / nkv, vd) + (size_t)hd / 32 * 4 * 64 * 16 <= 64 * 1024;
+}
+
 // The longest context the split variant takes for decoded tokens (the joining kernel keeps one
 // weight per partial result in LDS).  ``decode_chunk`` as in zk_attention_bf16.
 long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chunk) {
@@ -283,8 +297,8 @@ long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chun
 // Requests [0, r_prefill) hold portions of more than one token (max_q_len the longest);
 // requests [r_prefill, R) hold one token each and use the split variant over max_ctx keys.
 // decode_chunk: 32 or 64 (0: 64) sets the longest context that decoded tokens on the 16-wide tiles
-// take, 131,072 or 262,144 keys.  Their keys are cut after every 128 either way (blocks of 256 keys
-// were 3 to 20 % slower), so a request's result does not depend on it.
+// take, 131,072 or 262,144 keys.  Their keys are cut after every 128, or with 64 and a table of
+// ATT_DECODE_LONG_FROM keys a request or more after every 256: never by what shares the step.
 // mask_chunk > 0: a row sees the keys of its own chunk of that many positions (counted from
 // position 0) instead of a window; sink: a key of score 0 without a value in every denominator;
 // wide_weights: the weights keep 16 bits of mantissa in the product with the values.
@@ -423,8 +437,9 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
     int rc = 0;
     int span = ATT_CHUNK;        // keys one partial result covers
     if (decode_on_narrow_tiles(nh, nkv, hd)) {
-      // a block joins its four waves: one partial result per ATT_DECODE_SPAN keys
-      span = ATT_DECODE_SPAN;
+      // a block joins its four waves: one partial result per block of keys
+      const bool long_blocks = decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk);
+      span = long_blocks ? 4 * ATT_CHUNK : ATT_DECODE_SPAN;
       grid.x = (max_ctx + span - 1) / span;
       p.nchunks = grid.x;
       // a window covers at most ceil(window / span) + 1 blocks of span keys
@@ -435,7 +450,7 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
         grid.x = window_blocks;
       }
       p.part_ml = (float*)workspace + (size_t)n_dec * nh * p.nchunks * vd;
-      rc = launch_attn(ATT_DECODE, p, grid, s);
+      rc = launch_attn(long_blocks ? ATT_DECODE_LONG : ATT_DECODE, p, grid, s);
     } else {
       rc = launch_attn(ATT_DECODE_WIDE, p, grid, s);
     }

@@ -18,6 +18,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define ATT_CHUNK 64
 #define ATT_DECODE_SPAN 128    // keys of a partial result of a decoded token on 16-wide tiles
+#define ATT_DECODE_LONG_FROM 4096      // 256 instead where a request's table holds this many keys or more
 #define ATT_MOST_RANGES 8      // ranges of keys a block of rows of a portion is cut into, at most
 
 struct AttnParams {
@@ -747,6 +748,18 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
     }
 }
 
+// Which of a (request, key head)'s blocks a block is.  Blocks go to the 8 XCDs in turn, so with an even
+// number of them a request the first blocks of all requests would share a few XCDs and the last ones
+// the others: with requests of uneven lengths, whose last blocks have no keys, the first XCD then
+// reads half as much again as the average (64 requests of 200 to 3,840 keys, 4 key heads of 256:
+// 146 -> 109 us).  They are therefore counted from a place one further on for each (request, key
+// head).  An odd number (a window's 17 or 33 blocks) moves them on by itself, and a rotation would
+// undo that (64 requests of 200 to 8,000 keys behind a window of 4,096: 153 us without, 168 with).
+__device__ __forceinline__ int rotated_block(int blocks) {
+  const int turn = blocks % 2 ? 0 : blockIdx.y + gridDim.y * blockIdx.z;
+  return (blockIdx.x + turn) % blocks;
+}
+
 // One wave per (request, KV head, 32 keys) for requests that bring one token; a block's four
 // waves take 128 neighbouring keys and leave one partial result.  Columns of every tile are
 // the g query heads of the KV head (col = lane % 16), rows are keys (first product) or channels
@@ -771,12 +784,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
   const int col = lane & 15, kq = lane >> 4;
   const int r = p.r_begin + blockIdx.z;
   const int kvh = blockIdx.y;
-  // A request's blocks are counted from a place that differs from one (request, key head) to the
-  // next.  Blocks go to the 8 XCDs in turn, so with 8 or 16 of them a request block 0 of every
-  // request would run on the first XCD and the last one on the last: with requests of uneven
-  // lengths, whose last blocks have no keys, the first XCD then reads half as much again as the
-  // average (64 requests of 200 to 3,840 keys, 4 key heads of 256: 146 -> 109 us).
-  int block_x = (blockIdx.x + blockIdx.y + gridDim.y * blockIdx.z) % gridDim.x;
+  int block_x = rotated_block(gridDim.x);
   // Where the window is much shorter than the longest context, the grid covers a window's
   // blocks only and counts them from the block the request's window begins in.
   // In front of them come the blocks of the kept first keys, which every request has.
@@ -940,10 +948,208 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
   }
 }
 
+// One wave per (request, KV head, chunk of 64 keys) for requests that bring one token.
+// Columns of every tile are the g query heads of the KV head (col = lane % 16), rows are
+// keys (first product) or channels (second product).
+//
+// For callers whose limit is a long context (ATT_DECODE_LONG_FROM keys a request or more): blocks of
+// 256 keys leave half as many partial results as those of 128, whose writing and reading are what
+// is left to save once every CU has many blocks.  Figures at decode_in_long_blocks.
+template <int HD32, int VD16>
+__global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) {
+  constexpr int KS = HD32;       // 32-wide steps over head_dim
+  constexpr int DT = VD16;       // 16-channel output tiles
+  constexpr int CHUNK = ATT_CHUNK, SPAN = 4 * CHUNK;      // keys of a wave and of a block
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, kq = lane >> 4;
+  const int r = p.r_begin + blockIdx.z;
+  const int kvh = blockIdx.y;
+  // Where the window is much shorter than the longest context, the grid covers a window's
+  // blocks only and counts them from the block the request's window begins in.
+  int block_x = rotated_block(gridDim.x);
+  // In front of them come the blocks of the kept first keys, which every request has.
+  const int kept_blocks = (p.keep + SPAN - 1) / SPAN;
+  if (p.from_window && block_x >= kept_blocks)
+    block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / SPAN, kept_blocks) - kept_blocks;
+  const int chunk = block_x * 4 + wave;
+  const int* table = p.block_table + (size_t)r * p.max_blocks;
+  const int hd = p.hd, vd = p.vd, bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
+  // The pages of the chunk's (up to two) tiles are asked for before the request's length is
+  // known, beside it: where a key lies follows from the chunk alone.  A key past the context is
+  // masked below; a hole in the table reads page 0, which the caller keeps cleared, and the
+  // places of a request's last page behind its last token are cleared too (a masked value
+  // still meets a weight of 0 in the second product, and 0 x NaN is NaN).
+  int kpage[2][2], vpage[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int k0 = chunk * CHUNK + 32 * i;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      kpage[i][t] = table[min((k0 + 16 * t + col) >> bsh, p.max_blocks - 1)];
+      vpage[i][t] = table[min((k0 + 16 * t + 4 * kq) >> bsh, p.max_blocks - 1)];
+    }
+  }
+  const int n = p.q_start[r + 1] - p.q_start[r];
+  if (n <= 0) return;
+  const int pos = p.ctx_len[r] - 1;
+  const int row_lo = first_key(p, pos);
+  // a block whose four chunks all lie past the context or before the window ends here, all
+  // its waves alike: the grid is sized for the longest context the caller allows
+  const int first_chunk = block_x * 4;
+  if (first_chunk * CHUNK > pos ||
+      (first_chunk * CHUNK + SPAN - 1 < row_lo && first_chunk * CHUNK >= p.keep)) return;
+  const int key_lo = chunk * CHUNK < p.keep ? chunk * CHUNK : max(row_lo, chunk * CHUNK);
+  const int key_hi = min(pos, chunk * CHUNK + CHUNK - 1);
+  const bool active = key_lo <= key_hi;          // a wave without keys still meets the others at the barrier
+  const int g = p.nh / p.nkv;
+  const bool col_ok = col < g;
+  const int head = q_head_of(p, kvh, col_ok ? col : 0);
+  const int trow = p.q_start[r];
+
+  // the query operand waits in LDS (one 16-byte piece per lane and step), not in registers
+  __shared__ bf16x8 sq[4][KS][64];
+  {
+    const __bf16* qr = p.q + (size_t)trow * p.q_stride + (size_t)head * hd + kq * 8;
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      bf16x8 t;
+      if (col_ok) t = *(const bf16x8*)(qr + ks * 32);
+      else
+#pragma unroll
+        for (int e = 0; e < 8; e++) t[e] = (__bf16)0.f;
+      sq[wave][ks][lane] = t;
+    }
+  }
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int key0 = chunk * CHUNK + 32 * i;
+    if (!active || key0 > key_hi || key0 + 31 < key_lo) continue;
+    bf16x8 kf[2][KS];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int kk = key0 + 16 * t + col;
+      const int page = max(kpage[i][t], 0);
+      const __bf16* kr = p.kcache + ((((size_t)page * nkv + kvh) << bsh) + (kk & bmask)) * hd + kq * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) kf[t][ks] = *(const bf16x8*)(kr + ks * 32);
+    }
+    bf16x8 vf[DT];
+    {
+      const int ka = key0 + 4 * kq, kb = key0 + 16 + 4 * kq;
+      const int pa = max(vpage[i][0], 0), pb = max(vpage[i][1], 0);
+      const __bf16* va_base = p.vcache + ((((size_t)pa * (nkv >> p.v_shift) + (kvh >> p.v_shift)) * vd) << bsh) + (ka & bmask);
+      const __bf16* vb_base = p.vcache + ((((size_t)pb * (nkv >> p.v_shift) + (kvh >> p.v_shift)) * vd) << bsh) + (kb & bmask);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) {
+        const int d = dt * 16 + col;
+        const bf16x4 va = *(const bf16x4*)(va_base + ((size_t)d << bsh));
+        const bf16x4 vb = *(const bf16x4*)(vb_base + ((size_t)d << bsh));
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          vf[dt][e] = va[e];
+          vf[dt][4 + e] = vb[e];
+        }
+      }
+    }
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks], sq[wave][ks][lane], s[t], 0, 0, 0);
+    }
+    float mt = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int key = key0 + 16 * t + 4 * kq + i;
+        float v = score_log2(p, s[t][i]);
+        v = (col_ok && (key >= row_lo || key < p.keep) && key <= key_hi) ? v : -INFINITY;
+        s[t][i] = v;
+        mt = fmaxf(mt, v);
+      }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float m_new = fmaxf(m_run, mt);
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
+    float rs = 0.f;
+    bf16x8 pb8;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float pe = __builtin_amdgcn_exp2f(s[t][i] - m_use);
+        rs += pe;
+        pb8[4 * t + i] = (__bf16)pe;
+        s[t][i] = pe;
+      }
+    rs += __shfl_xor(rs, 16, 64);
+    rs += __shfl_xor(rs, 32, 64);
+    l_run = l_run * corr + rs;
+    m_run = m_new;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) {
+      o[dt] *= corr;
+      o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb8, o[dt], 0, 0, 0);
+    }
+    if (p.wide_weights) {
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) pb8[4 * t + i] = (__bf16)(s[t][i] - (float)pb8[4 * t + i]);
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb8, o[dt], 0, 0, 0);
+    }
+  }
+  // the block's four chunks are joined here, in chunk order: one partial result per 256 keys
+  extern __shared__ float dyn[];
+  float* sm_ml = dyn;                 // [4][16][2]
+  float* sm_o = dyn + 4 * 16 * 2;     // [4][g][vd]
+  if (col_ok) {
+    if (kq == 0) {
+      sm_ml[(wave * 16 + col) * 2] = m_run;
+      sm_ml[(wave * 16 + col) * 2 + 1] = l_run;
+    }
+    float* so = sm_o + ((size_t)wave * g + col) * vd;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) *(f32x4*)(so + dt * 16 + 4 * kq) = o[dt];
+  }
+  __syncthreads();
+  for (int idx = threadIdx.x; idx < g * vd; idx += 256) {
+    const int c = idx / vd, d = idx - c * vd;
+    float mw[4], m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      mw[w] = sm_ml[(w * 16 + c) * 2];
+      m = fmaxf(m, mw[w]);
+    }
+    float acc = 0.f, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const float e = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - m);
+      acc += e * sm_o[((size_t)w * g + c) * vd + d];
+      l += e * sm_ml[(w * 16 + c) * 2 + 1];
+    }
+    const size_t slot = ((size_t)(r - p.r_begin) * p.nh + q_head_of(p, kvh, c)) * p.nchunks + block_x;
+    p.part_o[slot * vd + d] = acc;
+    if (d == 0) {
+      p.part_ml[slot * 2] = m;
+      p.part_ml[slot * 2 + 1] = l;
+    }
+  }
+}
+
 // One pair of sizes.  what: 0 decoded tokens on 32-wide tiles, 1 pairs of groups a block, 2 a group a block,
 // 3 shared tiles with four waves, 4 with eight, 5 with four and the keys in ranges, 6 decoded tokens
-// on 16-wide tiles (keys in whole 32s).
-enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE };
+// on 16-wide tiles (keys in whole 32s), 7 the same in blocks of 256 keys.
+enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE, ATT_DECODE_LONG };
 
 template <int HD16, int VD16, int NW, bool SPLIT>
 static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
@@ -959,6 +1165,9 @@ static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
   attn_shared_kernel<HD16, VD16, NW, SPLIT><<<grid, NW * 64, lds, s>>>(p);
   return zk_launch_status("zk_attention_bf16 (shared tiles)");
 }
+
+// the maxima and sums, and the results, of the four waves of a block of 256 keys
+static inline size_t decode_long_lds(int g, int vd) { return (4 * 16 * 2 + (size_t)4 * g * vd) * sizeof(float); }
 
 template <int HD16, int VD16>
 static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s) {
@@ -984,6 +1193,13 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
           prepared = true;
         }
         attn_decode_kernel<HD16 / 2, VD16><<<grid, 256, lds, s>>>(p);
+        break;
+      } else {
+        return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
+      }
+    case ATT_DECODE_LONG:
+      if constexpr (HD16 % 2 == 0) {
+        attn_decode_long_kernel<HD16 / 2, VD16><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
         break;
       } else {
         return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");

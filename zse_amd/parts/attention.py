@@ -108,7 +108,7 @@ class PagedAttention(Part):
             raise ValueError(f"rotated values need an even value_dim, got {self.value_dim}")
         self.q_gain = self.k_gain = self.head_scale = self.value_freq = self.sinks = None
         self.q_row_gain = self.k_row_gain = None
-        self.decode_chunk = 64                     # keys a wave of the split decode attention takes
+        self.decode_chunk = 64                     # 32 or 64: how far the split decode attention reaches, and beside a wide table how its keys are cut
 
     def children(self):
         return [self.position] + ([self.conv] if self.conv is not None else [])
@@ -207,9 +207,9 @@ class PagedAttention(Part):
                     kernels.zk_attention_bf16_supports_values(s.num_heads, s.num_kv_heads, s.head_dim, self.value_dim, page_size))
 
     def prepare(self, kernels, dtype, max_seqs, max_model_len, page_size, max_batch_tokens=0) -> int:
-        """Workspace of the split attention of decoded tokens at the runner's limits, and the
-        number of keys a wave of it takes.  That number fixes where the sums over keys are cut:
-        it follows from the limits alone, never from a step's batch, so a request's result does
+        """Workspace of the split attention of decoded tokens at the runner's limits, and its
+        decode_chunk.  With the width of the block table it fixes where the sums over keys are cut:
+        both follow from the limits alone, never from a step's batch, so a request's result does
         not depend on who shares its step."""
         s = self.spec
         if not self.wants_v_transposed(kernels, dtype, page_size):

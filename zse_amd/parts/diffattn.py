@@ -39,7 +39,7 @@ class DifferentialAttention(Part):
             raise ValueError(f"temp_every must not be negative and a window positive, got {s.temp_every} and {s.window}")
         self.w_qkv = self.w_o = None
         self.lam = float(s.diff)
-        self.decode_chunk = 64                     # keys a wave of the split decode attention takes
+        self.decode_chunk = 64                     # 32 or 64: how far the split decode attention reaches, and beside a wide table how its keys are cut
 
     def wants_v_transposed(self, kernels, dtype: str, page_size: int) -> bool:
         """Whether the matrix-core kernel serves this layer (it reads V as [page][head][channel][slot])."""
@@ -48,8 +48,8 @@ class DifferentialAttention(Part):
                     kernels.zk_attention_bf16_supports(2 * s.num_heads, 2 * s.num_kv_heads, s.head_dim, page_size))
 
     def prepare(self, kernels, dtype, max_seqs, max_model_len, page_size, max_batch_tokens=0) -> int:
-        """Workspace of the split attention of decoded tokens at the runner's limits, and the number
-        of keys a wave of it takes (fixed by the limits, never by a step's batch)."""
+        """Workspace of the split attention of decoded tokens at the runner's limits, and its
+        decode_chunk (fixed by the limits, never by a step's batch)."""
         s = self.spec
         if not self.wants_v_transposed(kernels, dtype, page_size):
             return 0
