@@ -86,3 +86,39 @@ def test_attention(rt, nh, nkv, hd, vd, bs, window, keep):
     for t in range(T):                              # each token alone: the same bits
         alone = run(t, 1)
     assert np.array_equal(alone[9:], got[9:]) and np.array_equal(alone[:8], got[:8])
+
+
+# One request whose tokens share a block.  A value that is not finite lies in a piece of 16 keys of which
+# every row sees several more: at the last token's own place (hidden from the tokens before it), or at a place
+# that a window shows to the first tokens only.
+@pytest.mark.parametrize("nh,nkv,past,n,window,at", [(1, 1, 70, 9, 0, 78), (4, 2, 72, 8, 0, 79), (2, 2, 70, 9, 8, 66),
+                                                     (16, 1, 140, 1, 0, 3), (3, 1, 125, 5, 0, 127)])
+@pytest.mark.parametrize("what", [np.inf, -np.inf, np.nan])
+def test_a_value_changes_only_the_rows_that_see_it(rt, nh, nkv, past, n, window, at, what):
+    k = rt.kernels("float32")
+    rng = np.random.default_rng(past + at)
+    hd, vd, bs, ctx = 64, 128, 16, past + n
+    pages = -(-ctx // bs)
+    kc, vc = (rng.normal(size=(pages, nkv, bs, d)).astype(np.float32) for d in (hd, vd))
+    q = rng.normal(size=(n, nh, hd)).astype(np.float32)
+    bad = vc.copy()
+    bad[at // bs, :, at % bs, ::3] = what
+    Q, KC, TBL = rt.upload(q), rt.upload(kc), rt.upload(np.arange(pages, dtype=np.int32)[None])
+    POS, REQ, OUT = rt.upload(np.arange(past, ctx, dtype=np.int32)), rt.upload(np.zeros(n, np.int32)), rt.zeros((n, nh, vd), "float32")
+
+    def run(v, t, m):
+        V = rt.upload(v)
+        k.zk_attention_plain_gated(Q.ptr + 4 * t * nh * hd, nh * hd, KC.ptr, V.ptr, TBL.ptr, pages, REQ.ptr + 4 * t, POS.ptr + 4 * t,
+                                   OUT.ptr + 4 * t * nh * vd, m, nh, nkv, hd, vd, bs, 0.2, 0.0, window, 0, None, 0, None, 0, 0, 0, 0,
+                                   None, 0, rt.stream)
+        return rt.download(OUT)
+    fine, got = run(vc, 0, n), run(bad, 0, n)
+    for i in range(n):
+        sees = at <= past + i and not (window and at <= past + i - window)
+        clean = np.ones(vd, bool)
+        clean[::3] = not sees
+        assert np.array_equal(got[i][:, clean], fine[i][:, clean]), i       # the others' bits stay
+        assert np.isfinite(got[i][:, clean]).all() and not np.isfinite(got[i][:, ~clean]).any(), i
+    for t in range(n):                              # and each token alone has the bits that it has in company
+        alone = run(bad, t, 1)
+    assert np.array_equal(alone, got, equal_nan=True)
