@@ -122,3 +122,21 @@ def test_a_value_changes_only_the_rows_that_see_it(rt, nh, nkv, past, n, window,
     for t in range(n):                              # and each token alone has the bits that it has in company
         alone = run(bad, t, 1)
     assert np.array_equal(alone, got, equal_nan=True)
+
+
+def test_rows_of_the_cache_past_2_to_the_31(rt):
+    # the cache's row of a key (page, key head, place) has more than 31 bits; one page of it is filled and read
+    k = rt.kernels("float32")
+    nh, d, bs, page, n = 3, 4, 16, 1 << 27, 13
+    rng = np.random.default_rng(0)
+    kv = rng.normal(size=(bs, d)).astype(np.float32)
+    cache, small = rt.empty((page + 1, 1, bs, d), "float32"), rt.upload(kv)
+    rt.copy_h2d(cache.ptr + 4 * page * bs * d, kv)
+    Q, O = rt.upload(rng.normal(size=(n, nh, d)).astype(np.float32)), rt.empty((n, nh, d), "float32")
+    REQ, POS = rt.upload(np.zeros(n, np.int32)), rt.upload(np.arange(n, dtype=np.int32))
+
+    def run(c, at):
+        TBL = rt.upload(np.array([[at]], np.int32))
+        k.zk_attention_plain(Q.ptr, nh * d, c.ptr, c.ptr, TBL.ptr, 1, REQ.ptr, POS.ptr, O.ptr, n, nh, 1, d, bs, 0.5, 0.0, 0, 0, rt.stream)
+        return rt.download(O)
+    assert np.array_equal(run(cache, page), run(small, 0))

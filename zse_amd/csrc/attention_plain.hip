@@ -227,21 +227,21 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
     if (tile >= kept_tiles && tile < lo_tile) continue;
     const int j0 = tile * 64;
     // the cache row of key 16 f + r; a key that no row of the run sees is never read (row -1)
-    int at[4];
+    long long at[4];
 #pragma unroll
     for (int f = 0; f < 4; f++) {
       const int j = j0 + 16 * f + r;
       at[f] = -1;
       if (j <= seg_hi && (j >= seg_lo || j < keep)) {
         const int page = table[j / bs];
-        if (page >= 0) at[f] = (page * nkv + kvh) * bs + j % bs;
+        if (page >= 0) at[f] = ((long long)page * nkv + kvh) * bs + j % bs;
       }
     }
     f32x4 s[4];
 #pragma unroll
     for (int f = 0; f < 4; f++) {
       s[f] = zero;
-      const float* kr = kcache + (size_t)max(at[f], 0) * hd;
+      const float* kr = kcache + (size_t)max(at[f], 0LL) * hd;
 #pragma unroll
       for (int c = 0; c < QC; c++) {
         const int d = 16 * c + 4 * qd;
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
     for (int f = 0; f < 4; f++) {
       f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
-      int va[4];
+      long long va[4];
       bool fine = true;
 #pragma unroll
       for (int e = 0; e < 4; e++) {
@@ -327,7 +327,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
             acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
       if (odd) {
         for (int kk = 0; kk < 16; kk++) {        // rare: what was left out joins the queries that see it
-          const int j = j0 + 16 * f + kk, av = __shfl(at[f], kk);
+          const int j = j0 + 16 * f + kk;
+          const long long av = __shfl(at[f], kk);
           float p = 0.f;
 #pragma unroll
           for (int e = 0; e < 4; e++) {
