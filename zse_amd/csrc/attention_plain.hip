@@ -155,8 +155,8 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // (tile j / 64 to wave j / 64 % WAVES); each keeps a running maximum and sum, and the waves'
 // sums are joined in their order.  So a row's sums are cut and ordered by its position alone,
 // however the step was cut, and rows that share a block do not touch each other: a key that a
-// row does not see has weight 0 there, and in a tile with such a key a value that is not finite
-// stays out of the product and is added to the rows that see it, which are not finite from then on.
+// row does not see has weight 0 there, and a tile with such a key and a value that is not finite
+// is taken value by value, in the order in which the matrix cores take them.
 //
 // Bound by the latency of the loads for few tokens and by the matrix cores for many.  Measured
 // (us; before: a wave per token and head whose lanes each walked a key's row):
@@ -308,26 +308,18 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
             for (int x = 0; x < 4; x++) fine = fine && fabsf(v[e][c][x]) < INFINITY;
       }
-      const bool odd = !__all(fine);
-      if (odd) {
+      if (__all(fine)) {
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
           for (int c = 0; c < VC; c++)
 #pragma unroll
             for (int x = 0; x < 4; x++)
-              if (!(fabsf(v[e][c][x]) < INFINITY)) v[e][c][x] = 0.f;
-      }
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-#pragma unroll
-        for (int c = 0; c < VC; c++)
-#pragma unroll
-          for (int x = 0; x < 4; x++)
-            acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
-      if (odd) {
-        for (int kk = 0; kk < 16; kk++) {        // rare: what was left out joins the queries that see it
-          const int j = j0 + 16 * f + kk;
+              acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
+      } else {
+        // rare: each query takes the keys that it sees, in the products' order (0, 4, 8, 12, 1, 5, ..)
+        for (int n = 0; n < 16; n++) {
+          const int kk = n % 4 * 4 + n / 4, j = j0 + 16 * f + kk;
           const long long av = __shfl(at[f], kk);
           float p = 0.f;
 #pragma unroll
@@ -343,10 +335,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
               const int d = 64 * c + 16 * qd + 4 * i;
               if (d >= vd) continue;
 #pragma unroll
-              for (int e = 0; e < 4; e++) {
-                const float x = vcache[(size_t)av * vd + d + e];
-                if (!(fabsf(x) < INFINITY)) acc[c][e][i] = fmaf(x, p, acc[c][e][i]);
-              }
+              for (int e = 0; e < 4; e++) acc[c][e][i] = fmaf(vcache[(size_t)av * vd + d + e], p, acc[c][e][i]);
             }
         }
       }
