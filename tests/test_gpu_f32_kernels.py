@@ -140,3 +140,22 @@ def test_rows_of_the_cache_past_2_to_the_31(rt):
         k.zk_attention_plain(Q.ptr, nh * d, c.ptr, c.ptr, TBL.ptr, 1, REQ.ptr, POS.ptr, O.ptr, n, nh, 1, d, bs, 0.5, 0.0, 0, 0, rt.stream)
         return rt.download(O)
     assert np.array_equal(run(cache, page), run(small, 0))
+
+
+def test_more_tokens_than_one_launch_holds(rt):
+    # sixteen heads over one: a block a token, of 512 threads
+    k = rt.kernels("float32")
+    T, nh, d, bs = (1 << 23) + 1000, 16, 4, 8
+    rng = np.random.default_rng(0)
+    kc, vc = (rt.upload(rng.normal(size=(1, 1, bs, d)).astype(np.float32)) for _ in range(2))
+    TBL, REQ, POS = rt.upload(np.zeros((1, 1), np.int32)), rt.upload(np.zeros(T, np.int32)), rt.upload(np.arange(T, dtype=np.int32) % bs)
+    Q, O, few = rt.empty((T, nh, d), "float32"), rt.empty((T, nh, d), "float32"), rt.empty((512, nh, d), "float32")
+    k.zk_fill_normal(Q.ptr, 0, Q.numel, 5, 1, 0.0, 1.0, rt.stream)
+
+    def run(t, n, out):
+        k.zk_attention_plain(Q.ptr + 4 * t * nh * d, nh * d, kc.ptr, vc.ptr, TBL.ptr, 1, REQ.ptr + 4 * t, POS.ptr + 4 * t, out, n, nh, 1, d, bs,
+                             0.5, 0.0, 0, 0, rt.stream)
+    run(0, T, O.ptr)
+    for t in (0, (1 << 22) - 256, (1 << 23) - 256, T - 512):
+        run(t, 512, few.ptr)
+        assert np.array_equal(rt.download(O.rows(t, t + 512)), rt.download(few)), t

@@ -430,16 +430,22 @@ extern "C" int zk_attention_plain_gated(const void* q, int q_stride, const void*
       ((uintptr_t)q | (uintptr_t)kcache | (uintptr_t)vcache | (uintptr_t)out) % 16 == 0 &&
       (long long)nkv * ((nh / nkv + 15) / 16) <= 65535) {
     const int group = nh / nkv, tb = group < 16 ? 16 / group : 1, most = hd > vd ? hd : vd;
-    const dim3 blocks((T + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
+    // a launch of 2^32 threads or more would run its low 32 bits only: tokens are taken 2^22 blocks at a time
+    const int most_tokens = (1 << 22) * tb;
+    for (long long t = 0; t < T; t += most_tokens) {
+      const int n = T - t < most_tokens ? (int)(T - t) : most_tokens;
+      const dim3 blocks((n + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
 #define ZK_ATTENTION_F32(D_, W_)                                                                                      \
   attention_f32_kernel<D_, W_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                          \
-      (const float*)q, q_stride, (const float*)kcache, (const float*)vcache, block_table, max_blocks, req_of_token,   \
-      positions, (float*)out, T, nh, nkv, hd, vd, bs, scale, softcap, window, v_freq, v_interleaved, sinks, chunk,    \
-      unit_sink, keep, (const float*)gate, gate_ld)
-    if (most <= 64) ZK_ATTENTION_F32(64, 8);
-    else if (most <= 128) ZK_ATTENTION_F32(128, 8);
-    else ZK_ATTENTION_F32(256, 4);
+      (const float*)q + t * q_stride, q_stride, (const float*)kcache, (const float*)vcache, block_table,              \
+      max_blocks, req_of_token + t, positions + t, (float*)out + t * nh * vd, n, nh, nkv, hd, vd, bs, scale,  \
+      softcap, window, v_freq, v_interleaved, sinks, chunk, unit_sink, keep,                                          \
+      gate == nullptr ? nullptr : (const float*)gate + t * gate_ld, gate_ld)
+      if (most <= 64) ZK_ATTENTION_F32(64, 8);
+      else if (most <= 128) ZK_ATTENTION_F32(128, 8);
+      else ZK_ATTENTION_F32(256, 4);
 #undef ZK_ATTENTION_F32
+    }
     return zk_launch_status("zk_attention_plain");
   }
 #endif
