@@ -159,3 +159,20 @@ def test_more_tokens_than_one_launch_holds(rt):
     for t in (0, (1 << 22) - 256, (1 << 23) - 256, T - 512):
         run(t, 512, few.ptr)
         assert np.array_equal(rt.download(O.rows(t, t + 512)), rt.download(few)), t
+
+
+def test_more_blocks_of_columns_than_one_launch_holds(rt):
+    # a launch holds less than 2^32 threads: 2^28 columns and more leave in several
+    k = rt.kernels("float32")
+    M, N, K = 2, (1 << 28) + 2000, 4
+    W, C = rt.empty((N, K), "float32"), rt.empty((M, N), "float32")
+    k.zk_fill_normal(W.ptr, 0, W.numel, 5, 1, 0.0, 1.0, rt.stream)
+    a = np.random.default_rng(0).normal(size=(M, K)).astype(np.float32)
+    A = rt.upload(a)
+    k.zk_gemm_plain(A.ptr, K, W.ptr, C.ptr, N, 1, M, N, K, rt.stream)
+    few = rt.empty((M, 2048), "float32")
+    for n0 in (0, (1 << 27) - 1024, (1 << 28) - 1024, N - 2048):
+        k.zk_gemm_plain(A.ptr, K, W.ptr + 4 * K * n0, few.ptr, 2048, 1, M, 2048, K, rt.stream)
+        want = rt.download(few)
+        for m in range(M):
+            assert np.array_equal(rt.download(type(C)(C.ptr + 4 * (m * N + n0), (2048,), "float32")), want[m]), (n0, m)

@@ -6,6 +6,8 @@
 // depend on which other rows are in the batch.
 #include "common.h"
 
+#include <algorithm>
+
 #if ZSE_ACT_BF16
 #define GP_BM 64
 #define GP_BN 64
@@ -216,13 +218,16 @@ __global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __
 template <int MF, int NF, int H, int AHEAD>
 static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc, int M, int N, int K,
                       hipStream_t s) {
-  const int tiles_m = (M + 16 * MF - 1) / (16 * MF), tiles_n = (N + 16 * NF - 1) / (16 * NF);
-  ZK_REQUIRE((long long)tiles_m * tiles_n < 2147483647LL, "zk_gemm_plain: too many tiles");
+  const int tiles_m = (M + 16 * MF - 1) / (16 * MF);
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-  const dim3 grid(tiles_m * tiles_n);
   const int how = !vec ? 0 : K % 32 ? 1 : 2;
   auto kernel = how == 2 ? gemm_f32_kernel<MF, NF, H, AHEAD, 2> : how == 1 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1> : gemm_f32_kernel<MF, NF, H, AHEAD, 0>;
-  kernel<<<grid, 64 * GF_WAVES, 0, s>>>(A, lda, W, C, ldc, M, N, K, tiles_m, tiles_n);
+  // a launch of 2^32 threads or more would run its low 32 bits only: columns are taken 2^22 tiles at a time
+  const long long most = (long long)std::max((1 << 22) / tiles_m, 1) * (16 * NF);
+  for (long long n = 0; n < N; n += most) {
+    const int cols = (int)std::min(most, N - n), tiles_n = (cols + 16 * NF - 1) / (16 * NF);
+    kernel<<<dim3(tiles_m * tiles_n), 64 * GF_WAVES, 0, s>>>(A, lda, W + n * K, C + n, ldc, M, cols, K, tiles_m, tiles_n);
+  }
   return zk_launch_status("zk_gemm_plain");
 }
 
