@@ -161,9 +161,17 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // Bound by the latency of the loads for few tokens and by the matrix cores for many.  Measured
 // (us; before: a wave per token and head whose lanes each walked a key's row):
 //   303 tokens, 8 heads of 128, contexts of 300 and three of 50 to 700: 852 -> 55.
+//   One token, 8 heads over 2 of 128: 1 key 12.4 -> 9.5, 100 keys 57 -> 16, 4,000 keys 2,111 -> 144; 4 heads
+//   of 16: 6.9 -> 8.5, 26 -> 11, 884 -> 83; 8 over 4 of 256: 21.7 -> 22.7, 109 -> 27, 6,260 -> 458.  (Heads of up
+//   to 64 are slower than before below about ten keys, of 256 below three.)
+//
+// ASK: keys are asked for without a condition, and pieces of 16 that no row sees are passed over in the
+// first product too.  For key heads of 65 to 128 channels: one token with 1 key 14.5 -> 9.5 us, 16 tokens of 500
+// to 1,055 keys 53 -> 47, 1,500 tokens behind a window 102 -> 91.  Not for 64 channels with values of 128 (4,000
+// keys 125 -> 138) nor for smaller heads (80 -> 89); of 256 the loads in flight do not fit (446 -> 472).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int MAXD, int WAVES>
+template <int MAXD, int WAVES, bool ASK>
 __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ kcache, const float* __restrict__ vcache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ req_of_token,
@@ -171,6 +179,9 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
     float scale, float softcap, int window, const float* __restrict__ v_freq, int v_interleaved,
     const float* __restrict__ sinks, int chunk, int unit_sink, int keep, const float* __restrict__ gate, int gate_ld) {
   constexpr int QC = MAXD / 16, VC = MAXD / 64;       // pieces of 16 channels of a query, of 64 of a value
+  // A piece of 16 keys that no row of the run sees has weight 0 everywhere: its products are passed over
+  // where that was measured to pay (a branch keeps the next piece's loads from being asked for early).
+  constexpr bool PASS_VALUES = MAXD <= 128;
   __shared__ float s_acc[WAVES][16][MAXD];
   __shared__ float s_m[WAVES][16], s_l[WAVES][16];
   const int group = nh / nkv, chunks = (group + 15) / 16;
@@ -237,15 +248,23 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
         if (page >= 0) at[f] = ((long long)page * nkv + kvh) * bs + j % bs;
       }
     }
+    auto unseen = [&](int f) { return j0 + 16 * f > seg_hi || (j0 + 16 * f + 15 < seg_lo && j0 + 16 * f >= keep); };
     f32x4 s[4];
 #pragma unroll
     for (int f = 0; f < 4; f++) {
       s[f] = zero;
+      if (ASK && unseen(f)) continue;
       const float* kr = kcache + (size_t)max(at[f], 0LL) * hd;
 #pragma unroll
       for (int c = 0; c < QC; c++) {
         const int d = 16 * c + 4 * qd;
-        const f32x4 k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
+        f32x4 k4;
+        if (ASK) {
+          k4 = *(const f32x4*)(kr + min(d, hd - 4));
+          k4 = at[f] >= 0 && d < hd ? k4 : zero;
+        } else {
+          k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) s[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], qf[c][e], s[f], 0, 0, 0);
       }
@@ -288,6 +307,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
     const bool whole = __all(all);
 #pragma unroll
     for (int f = 0; f < 4; f++) {
+      if (PASS_VALUES && unseen(f)) continue;
       f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
       long long va[4];
       bool fine = true;
@@ -435,15 +455,16 @@ extern "C" int zk_attention_plain_gated(const void* q, int q_stride, const void*
     for (long long t = 0; t < T; t += most_tokens) {
       const int n = T - t < most_tokens ? (int)(T - t) : most_tokens;
       const dim3 blocks((n + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
-#define ZK_ATTENTION_F32(D_, W_)                                                                                      \
-  attention_f32_kernel<D_, W_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                          \
+#define ZK_ATTENTION_F32(D_, W_, A_)                                                                                  \
+  attention_f32_kernel<D_, W_, A_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                      \
       (const float*)q + t * q_stride, q_stride, (const float*)kcache, (const float*)vcache, block_table,              \
-      max_blocks, req_of_token + t, positions + t, (float*)out + t * nh * vd, n, nh, nkv, hd, vd, bs, scale,  \
+      max_blocks, req_of_token + t, positions + t, (float*)out + t * nh * vd, n, nh, nkv, hd, vd, bs, scale,          \
       softcap, window, v_freq, v_interleaved, sinks, chunk, unit_sink, keep,                                          \
       gate == nullptr ? nullptr : (const float*)gate + t * gate_ld, gate_ld)
-      if (most <= 64) ZK_ATTENTION_F32(64, 8);
-      else if (most <= 128) ZK_ATTENTION_F32(128, 8);
-      else ZK_ATTENTION_F32(256, 4);
+      if (most <= 64) ZK_ATTENTION_F32(64, 8, false);
+      else if (most <= 128 && hd > 64) ZK_ATTENTION_F32(128, 8, true);
+      else if (most <= 128) ZK_ATTENTION_F32(128, 8, false);
+      else ZK_ATTENTION_F32(256, 4, false);
 #undef ZK_ATTENTION_F32
     }
     return zk_launch_status("zk_attention_plain");
