@@ -34,6 +34,30 @@ def test_product(rt, M, N, K, gap):
         assert np.array_equal(rt.download(one)[0], got[m, :N]), m
 
 
+# Tiles of 64 x 64 (1,024 of them or more) with ragged last ones, and of the other sizes; K of fewer values than a
+# load takes, of one and two steps (one and two waves), around the steps of eight waves and odd; rows and
+# weights that begin at any float's address
+@pytest.mark.parametrize("M,N", [(129, 22000), (40, 70001), (17, 300), (16, 17000), (2, 50)])
+@pytest.mark.parametrize("K,gap,shift", [(1, 0, 0), (3, 1, 1), (4, 0, 0), (5, 0, 3), (31, 0, 0), (32, 4, 0), (36, 0, 1), (63, 1, 0), (64, 0, 2),
+                                         (65, 0, 0), (260, 4, 0), (544, 0, 1), (801, 2, 0)])
+def test_product_tiles_and_addresses(rt, M, N, K, gap, shift):
+    k = rt.kernels("float32")
+    rng = np.random.default_rng(M + K)
+    a, w = rng.normal(size=(M, K + gap)).astype(np.float32), rng.normal(size=(N, K)).astype(np.float32)
+    a[:, K:] = np.nan                                       # nothing between the rows is used
+    pad = lambda x: np.concatenate([np.full(shift, np.nan, np.float32), x.ravel(), np.full(4, np.nan, np.float32)])
+    A, W = rt.upload(pad(a)), rt.upload(pad(w))
+    C, one = rt.upload(np.full((M, N + 3), 7.0, np.float32)), rt.empty((1, N), "float32")
+    k.zk_gemm_plain(A.ptr + 4 * shift, K + gap, W.ptr + 4 * shift, C.ptr, N + 3, 1, M, N, K, rt.stream)
+    got = rt.download(C)
+    want = a[:, :K].astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(got[:, :N] - want).max() < 8 * 2.0 ** -24 * max(K, 8)        # as above
+    assert (got[:, N:] == 7.0).all()
+    for m in {0, M // 2, M - 1}:
+        k.zk_gemm_plain(A.ptr + 4 * (shift + m * (K + gap)), K + gap, W.ptr + 4 * shift, one.ptr, N, 1, 1, N, K, rt.stream)
+        assert np.array_equal(rt.download(one)[0], got[m, :N]), m
+
+
 # heads, key heads (one to seventeen heads a key head), sizes of keys and values, page, window, first keys kept
 @pytest.mark.parametrize("nh,nkv,hd,vd,bs,window,keep", [(4, 2, 64, 64, 16, 0, 0), (3, 1, 20, 36, 4, 7, 0), (17, 1, 128, 128, 16, 70, 3),
                                                          (6, 6, 256, 256, 8, 0, 0), (10, 2, 132, 64, 32, 33, 0), (16, 1, 4, 4, 1, 0, 0)])

@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
 
 // The 32-bit product on the 32-bit matrix cores (16x16x4, float in, float out).
 //
-// A block owns 16 MF x 16 NF of C and its eight waves share K out: wave w takes the 32-wide
+// A block owns 16 MF x 16 NF of C and its waves, eight of them, share K out: wave w takes the 32-wide
 // steps w, w + 8, .., every wave the whole tile, and their sums meet in LDS, (w, w + 4), then
 // (w, w + 2), then (w, w + 1).  So the order of a sum follows from K alone and the tile may
 // follow from M and N.  Operands come straight from memory: in a 16-wide piece of K the four
@@ -76,18 +76,21 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
 // The error against 64 bits is no larger than the scalar sum's (eight shorter sums added up).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-#define GF_WAVES 8
+typedef f32x4 f32x4_any __attribute__((aligned(4)));       // the loads take any float's address
 
-// HOW: 2: K is a whole number of steps; 1: rows of whole 16-byte pieces; 0: every value is loaded
-// on its own.  The loads of the next H pieces of a wave's run are on their way while the current
-// ones are multiplied, so nothing may look at them before: with HOW = 1 the pieces behind K are
-// set to zero right before they are multiplied.
-template <int MF, int NF, int H, int AHEAD, int HOW>
-__global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __restrict__ A, int lda,
-                                                                 const float* __restrict__ W,
-                                                                 float* __restrict__ C, int ldc, int M, int N,
-                                                                 int K, int tiles_m, int tiles_n) {
-  __shared__ f32x4 part[GF_WAVES / 2][MF * NF][64];
+// HOW: 3: K is a whole number of steps; 2: a multiple of four; 1: four or more; 0: fewer, every value is
+// loaded on its own.  The loads of the next H pieces of a wave's run are on their way while the
+// current ones are multiplied, so nothing may look at them before: with HOW = 1 and 2 what lies
+// behind K is set to zero right before it is multiplied.  (2048 x 5000 x 200: 84 us with 2, 99 with 1;
+// 2048 x 4096 x 1023: 253 with 1, 390 value by value.)
+// WAVES: 8, or 1 or 2 where K has no more steps (waves without a step would bring zeros, so the sum
+// is the same): 2048 x 5000 with K = 16 53 -> 21 us, with K = 64 52 -> 27; scalar multiply-adds took 25 and 44.
+template <int MF, int NF, int H, int AHEAD, int HOW, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(const float* __restrict__ A, int lda,
+                                                              const float* __restrict__ W,
+                                                              float* __restrict__ C, int ldc, int M, int N,
+                                                              int K, int tiles_m, int tiles_n) {
+  __shared__ f32x4 part[WAVES > 1 ? WAVES / 2 : 1][MF * NF][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, q = lane >> 4;
   // the blocks that share a strip of W run on one XCD, one after the other (ids go round-robin over 8)
@@ -105,10 +108,10 @@ __global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __
 
   auto piece = [&](const float* row, int k) {
     f32x4 v;
-    if (HOW == 2) {
-      v = *(const f32x4*)(row + k);
-    } else if (HOW == 1) {       // K is a multiple of 4: the piece lies inside or outside as a whole
-      v = *(const f32x4*)(row + min(k, K - 4));
+    if (HOW == 3) {
+      v = *(const f32x4_any*)(row + k);
+    } else if (HOW > 0) {       // the last four values where the piece reaches past them
+      v = *(const f32x4_any*)(row + min(k, K - 4));
     } else {
 #pragma unroll
       for (int e = 0; e < 4; e++) v[e] = k + e < K ? row[k + e] : 0.f;
@@ -118,10 +121,10 @@ __global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __
   // The wave's run, counted in units of H pieces of 16: two pieces make one of its 32-wide
   // steps.  (A unit past the last reads inside the matrix again and is not multiplied: no load
   // is under a condition.)
-  const int units = (steps - wave + GF_WAVES - 1) / GF_WAVES * (2 / H);
+  const int units = (steps - wave + WAVES - 1) / WAVES * (2 / H);
   auto fetch = [&](int u, f32x4 (&af)[MF][H], f32x4 (&wf)[NF][H]) {
     const int p = min(u, units - 1) * H;
-    const int k = (wave + p / 2 * GF_WAVES) * 32 + p % 2 * 16 + 4 * q;
+    const int k = (wave + p / 2 * WAVES) * 32 + p % 2 * 16 + 4 * q;
 #pragma unroll
     for (int h = 0; h < H; h++) {
 #pragma unroll
@@ -137,15 +140,22 @@ __global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __
     for (int j = 0; j < NF; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // W is the first operand: a lane then holds columns 4 q + 0..3 of row r of C
   auto multiply = [&](int u, f32x4 (&a)[MF][H], f32x4 (&w)[NF][H]) {
-    if (HOW == 1) {
+    if (HOW == 1 || HOW == 2) {
 #pragma unroll
       for (int h = 0; h < H; h++) {
         const int p = u * H + h;
-        if ((wave + p / 2 * GF_WAVES) * 32 + p % 2 * 16 + 4 * q < K) continue;
+        const int over = (wave + p / 2 * WAVES) * 32 + p % 2 * 16 + 4 * q + 4 - K;       // values of the piece behind K
+        if (over <= 0) continue;
+        auto cut = [&](f32x4& v) {         // what was loaded are the row's last four values
+          if (HOW == 2) v = f32x4{0.f, 0.f, 0.f, 0.f};       // all of them belong to the piece before
+          else
+            v = f32x4{over == 1 ? v[1] : over == 2 ? v[2] : over == 3 ? v[3] : 0.f,
+                      over == 1 ? v[2] : over == 2 ? v[3] : 0.f, over == 1 ? v[3] : 0.f, 0.f};
+        };
 #pragma unroll
-        for (int i = 0; i < MF; i++) a[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < MF; i++) cut(a[i][h]);
 #pragma unroll
-        for (int j = 0; j < NF; j++) w[j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NF; j++) cut(w[j][h]);
       }
     }
 #pragma unroll
@@ -180,7 +190,7 @@ __global__ __launch_bounds__(64 * GF_WAVES) void gemm_f32_kernel(const float* __
       if (u + t < units) multiply(u + t, a[t], w[t]);
   }
 #pragma unroll
-  for (int half = GF_WAVES / 2; half > 0; half /= 2) {
+  for (int half = WAVES / 2; half > 0; half /= 2) {
     if (wave >= half && wave < 2 * half) {
 #pragma unroll
       for (int i = 0; i < MF; i++)
@@ -219,14 +229,18 @@ template <int MF, int NF, int H, int AHEAD>
 static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc, int M, int N, int K,
                       hipStream_t s) {
   const int tiles_m = (M + 16 * MF - 1) / (16 * MF);
-  const bool vec = K % 4 == 0 && lda % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-  const int how = !vec ? 0 : K % 32 ? 1 : 2;
-  auto kernel = how == 2 ? gemm_f32_kernel<MF, NF, H, AHEAD, 2> : how == 1 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1> : gemm_f32_kernel<MF, NF, H, AHEAD, 0>;
+  auto kernel = K < 4     ? gemm_f32_kernel<MF, NF, H, AHEAD, 0, 1>
+                : K <= 32 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 1>
+                : K <= 64 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 2>
+                : K % 4   ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 8>
+                : K % 32  ? gemm_f32_kernel<MF, NF, H, AHEAD, 2, 8>
+                          : gemm_f32_kernel<MF, NF, H, AHEAD, 3, 8>;
+  const int waves = K <= 32 ? 1 : K <= 64 ? 2 : 8;
   // a launch of 2^32 threads or more would run its low 32 bits only: columns are taken 2^22 tiles at a time
   const long long most = (long long)std::max((1 << 22) / tiles_m, 1) * (16 * NF);
   for (long long n = 0; n < N; n += most) {
     const int cols = (int)std::min(most, N - n), tiles_n = (cols + 16 * NF - 1) / (16 * NF);
-    kernel<<<dim3(tiles_m * tiles_n), 64 * GF_WAVES, 0, s>>>(A, lda, W + n * K, C + n, ldc, M, cols, K, tiles_m, tiles_n);
+    kernel<<<dim3(tiles_m * tiles_n), 64 * waves, 0, s>>>(A, lda, W + n * K, C + n, ldc, M, cols, K, tiles_m, tiles_n);
   }
   return zk_launch_status("zk_gemm_plain");
 }
