@@ -748,16 +748,23 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
     }
 }
 
-// Which of a (request, key head)'s blocks a block is.  Blocks go to the 8 XCDs in turn, so with an even
-// number of them a request the first blocks of all requests would share a few XCDs and the last ones
-// the others: with requests of uneven lengths, whose last blocks have no keys, the first XCD then
-// reads half as much again as the average (64 requests of 200 to 3,840 keys, 4 key heads of 256:
-// 146 -> 109 us).  They are therefore counted from a place one further on for each (request, key
-// head).  An odd number (a window's 17 or 33 blocks) moves them on by itself, and a rotation would
-// undo that (64 requests of 200 to 8,000 keys behind a window of 4,096: 153 us without, 168 with).
+// Which of a (request, key head)'s blocks a block is.  Blocks go in turn to the 8 XCDs and there to the
+// shader engines, 32 in all, so with an even number of them a request the first blocks of all requests
+// would share a few and the last ones the others: with requests of uneven lengths, whose last blocks have
+// no keys, the first then read half as much again as the average.  They are therefore counted from
+// a place of their own.  From one request to the next it moves by 3, through all of them.  From one key
+// head to the next it moves by 8, so that the same keys of all heads, which lie side by side in their pages,
+// are read by one XCD, on its engines in turn.  (Moved by 1, in launches one after the other over the
+// caches of several layers, 64 full requests of 32 heads over 16 of 128 lost a fifth; a launch alone lost 2 %, with
+// the same reads, hits and first-level translation misses: which cache or table it is was not found.)
+// Measured (us, with the joining launch; from place 0, by 1 further for each head and request, as it is):
+// 64 requests of 682 to 8,192 keys, 8 heads over 4 of 256 277, 212, 205; 32 over 16 of 128 510, 450, 401, and
+// all of 8,192 keys 737, 901, 745; 64 of 200 to 3,840 keys, 8 over 4 of 256 146, 109, 107.
+// An odd number (a window's 17 or 33 blocks) moves them on by itself, and a rotation would undo that (64 requests
+// of 200 to 8,000 keys behind a window of 4,096: 153 us without, 168 with).
 __device__ __forceinline__ int rotated_block(int blocks) {
-  const int turn = blocks % 2 ? 0 : blockIdx.y + gridDim.y * blockIdx.z;
-  return (blockIdx.x + turn) % blocks;
+  if (blocks % 2) return blockIdx.x;
+  return (blockIdx.x + 8 * blockIdx.y + 3 * blockIdx.z) % blocks;
 }
 
 // One wave per (request, KV head, 32 keys) for requests that bring one token; a block's four
