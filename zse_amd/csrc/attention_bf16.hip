@@ -446,7 +446,8 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
     if (decode_on_narrow_tiles(nh, nkv, hd)) {
       // a block joins its four waves: one partial result per block of keys
       const bool long_blocks = decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk);
-      span = long_blocks ? 4 * ATT_CHUNK : ATT_DECODE_SPAN;
+      p.chunk = ATT_CHUNK;
+      span = long_blocks ? 4 * p.chunk : ATT_DECODE_SPAN;
       grid.x = (max_ctx + span - 1) / span;
       p.nchunks = grid.x;
       // a window covers at most ceil(window / span) + 1 blocks of span keys

@@ -47,7 +47,7 @@ struct AttnParams {
   int r_begin;            // first request of this launch
   int nchunks;            // split: chunks the grid covers
   int from_window;        // decode: block 0 of a request is the one its window begins in
-  int chunk;              // portions with their keys in ranges: tiles of a range
+  int chunk;              // portions with their keys in ranges: tiles of a range; decoded tokens in blocks of 256 keys: a wave's keys
   int mask_chunk;         // > 0: a row sees the keys of its own chunk of this many positions only (no window then)
   int keep;               // beside its window a row sees the first ``keep`` keys of its sequence
   int sink;               // 1: a key of score 0 without a value joins every row's denominator
@@ -966,7 +966,11 @@ template <int HD32, int VD16>
 __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) {
   constexpr int KS = HD32;       // 32-wide steps over head_dim
   constexpr int DT = VD16;       // 16-channel output tiles
-  constexpr int CHUNK = ATT_CHUNK, SPAN = 4 * CHUNK;      // keys of a wave and of a block
+  // Keys of a wave (64) and of a block.  A number of the launch: with a constant the compiler orders a
+  // wave's two tiles otherwise, which loses where the chip is full (us, 64 requests of 4,096 keys, 8 heads over 4
+  // of 256 187.2 against 186.1; 8 behind a window of 2,048, 16 over 4 of 128 15.7 against 15.3) and gains with few
+  // blocks (8 of 4,096 keys, 8 over 4 of 256 35.8 against 36.7).
+  const int wave_keys = p.chunk, span = 4 * wave_keys;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, kq = lane >> 4;
   const int r = p.r_begin + blockIdx.z;
@@ -975,9 +979,9 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
   // blocks only and counts them from the block the request's window begins in.
   int block_x = rotated_block(gridDim.x);
   // In front of them come the blocks of the kept first keys, which every request has.
-  const int kept_blocks = (p.keep + SPAN - 1) / SPAN;
+  const int kept_blocks = (p.keep + span - 1) / span;
   if (p.from_window && block_x >= kept_blocks)
-    block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / SPAN, kept_blocks) - kept_blocks;
+    block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / span, kept_blocks) - kept_blocks;
   const int chunk = block_x * 4 + wave;
   const int* table = p.block_table + (size_t)r * p.max_blocks;
   const int hd = p.hd, vd = p.vd, bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
@@ -989,7 +993,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
   int kpage[2][2], vpage[2][2];
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const int k0 = chunk * CHUNK + 32 * i;
+    const int k0 = chunk * wave_keys + 32 * i;
 #pragma unroll
     for (int t = 0; t < 2; t++) {
       kpage[i][t] = table[min((k0 + 16 * t + col) >> bsh, p.max_blocks - 1)];
@@ -1003,10 +1007,10 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
   // a block whose four chunks all lie past the context or before the window ends here, all
   // its waves alike: the grid is sized for the longest context the caller allows
   const int first_chunk = block_x * 4;
-  if (first_chunk * CHUNK > pos ||
-      (first_chunk * CHUNK + SPAN - 1 < row_lo && first_chunk * CHUNK >= p.keep)) return;
-  const int key_lo = chunk * CHUNK < p.keep ? chunk * CHUNK : max(row_lo, chunk * CHUNK);
-  const int key_hi = min(pos, chunk * CHUNK + CHUNK - 1);
+  if (first_chunk * wave_keys > pos ||
+      (first_chunk * wave_keys + span - 1 < row_lo && first_chunk * wave_keys >= p.keep)) return;
+  const int key_lo = chunk * wave_keys < p.keep ? chunk * wave_keys : max(row_lo, chunk * wave_keys);
+  const int key_hi = min(pos, chunk * wave_keys + wave_keys - 1);
   const bool active = key_lo <= key_hi;          // a wave without keys still meets the others at the barrier
   const int g = p.nh / p.nkv;
   const bool col_ok = col < g;
@@ -1034,8 +1038,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
 
 #pragma unroll
   for (int i = 0; i < 2; i++) {
-    const int key0 = chunk * CHUNK + 32 * i;
-    if (!active || key0 > key_hi || key0 + 31 < key_lo) continue;
+    const int key0 = chunk * wave_keys + 32 * i;
+    if (!active || 32 * i >= wave_keys || key0 > key_hi || key0 + 31 < key_lo) continue;
     bf16x8 kf[2][KS];
 #pragma unroll
     for (int t = 0; t < 2; t++) {
