@@ -14,7 +14,7 @@ def rt():
 
 
 # rows around 16 and 64 and many of them; columns around 16, 32 and 64; K below a step, around the
-# eight waves' steps of 32, odd (values loaded one by one) and with rows further apart than K
+# eight waves' steps of 32, odd and with rows further apart than K (in tiles of 16 and 32; of 64 below)
 @pytest.mark.parametrize("M,N,K,gap", [(1, 16, 4, 0), (3, 33, 31, 0), (16, 1000, 256, 4), (17, 64, 260, 0), (15, 16400, 64, 0),
                                        (63, 65, 1024, 0), (64, 64, 36, 8), (300, 4096, 1028, 0), (129, 8200, 100, 3), (5, 7, 1, 0)])
 def test_product(rt, M, N, K, gap):

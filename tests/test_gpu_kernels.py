@@ -449,12 +449,14 @@ def test_attention_over_pages(rt, kernel, case):
     q = np.concatenate(q_rows)
     Q, KC, VC = up(rt, q, dtype), up(rt, kc, dtype), up(rt, vc, dtype)
     TBL = rt.upload(table)
+    wide_blocks = max(max_blocks, 4096 // bs)
+    WIDE = rt.upload(np.pad(table, ((0, 0), (0, wide_blocks - max_blocks)), constant_values=-1))
     POS, REQ = rt.upload(np.array(tok_pos, np.int32)), rt.upload(np.array(tok_req, np.int32))
     qs = np.concatenate([[0], np.cumsum([n for _, n in reqs])]).astype(np.int32)
     QS, CL = rt.upload(qs), rt.upload(np.array(total, np.int32))
     tol = 2e-5 if dtype == "float32" else 0.02
     outs = []
-    # both cuts of the decoded tokens' keys; and every kernel for the portions: a group of rows a
+    # both cuts of the decoded tokens' keys (after 256 with 64 and a table of 4,096 keys or more, else after 128); and every kernel for the portions: a group of rows a
     # block (1), tiles shared by 4 or 8 groups (pages of 8 keys or more), shared tiles with the keys
     # in ranges and a join (5; long contexts, else as 4), the choice by size (0)
     turns = [(0, 0)]
@@ -471,7 +473,8 @@ def test_attention_over_pages(rt, kernel, case):
             ws_bytes += k.zk_attention_bf16_portion_workspace(max(1, n_multi) * (max(n for _, n in reqs) + 128), nh, nkv, hd)
             ws = rt.zeros((ws_bytes // 4 + 1,), "float32")
             try:
-                k.zk_attention_bf16(Q.ptr, nh * hd, KC.ptr, VC.ptr, TBL.ptr, max_blocks, QS.ptr, CL.ptr, OUT.ptr,
+                tbl, width = (WIDE, wide_blocks) if chunk == 64 else (TBL, max_blocks)
+                k.zk_attention_bf16(Q.ptr, nh * hd, KC.ptr, VC.ptr, tbl.ptr, width, QS.ptr, CL.ptr, OUT.ptr,
                                     R, n_multi, max(n for _, n in reqs), max_ctx, nh, nkv, hd, bs, scale,
                                     c["cap"], c["window"], chunk, ws.ptr, ws.nbytes, rt.stream)
             finally:
