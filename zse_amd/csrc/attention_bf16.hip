@@ -282,12 +282,13 @@ static bool decode_on_narrow_tiles(int nh, int nkv, int hd) { return nh / nkv <=
 // Whether they go in blocks of 256 keys instead of 128.  By what a runner's limits fix alone (its
 // decode_chunk and the width of its block tables), never by a step's requests, because it says where
 // a request's sums are cut.  The blocks' queries and results have to fit in 64 KB of LDS.
-// Measured (us, blocks of 256 against 128, 8 heads over 4 of 256 channels unless said): 64 requests
-// of 8,192 keys 367 against 384, behind a window of 4,096 188 against 200; 8 of 8,192 54 against 56;
-// 16 of 8,192, 32 heads over 16 of 128: 198 against 210.  Below the line 128 is the better one: 64 of 200
-// to 2,000 keys 70 against 63, 23 of 130 to 2,000 33 against 27.  At 4,096 it depends: full contexts
-// are better off with 256 (a whole step of 64 requests 7.20 ms against 7.27), uneven ones with 128 (64 of 200 to
-// 3,840 keys 109 us against 103, 8 of 500 to 4,000 24 against 22); the line lets no full one wait.
+// Measured (us with the joining launch, blocks of 256 against 128; 8 heads over 4 of 256 channels, A, or 32 over
+// 16 of 128, B).  Full contexts of many requests are better off with 256, which leaves half the partial
+// results: 64 of 8,192 keys A 357 and 385, B 743 and 810; 64 of 4,096 A 189 and 193, B 372 and 393; below the
+// line 64 of 3,072 A 142 and 145, B 283 and 295, of 2,048 A 99.5 and 99.2, B 191 and 197.  Few or uneven requests
+// are better off with 128: 1 of 4,096 A 15.1 and 12.1, 8 of 3,000 A 27.8 and 24.7, 8 of 500 to 4,000 24.9 and 21.8,
+// 64 of 200 to 3,840 110 and 104, of 200 to 3,000 94 and 85, of 200 to 2,000 65 and 62.  The line lies where the
+// loss of full launches by 128 (3 to 4 % under it, 4 to 9 % from 8,192 on) begins to outweigh the rest.
 static bool decode_in_long_blocks(int nh, int nkv, int hd, int vd, int bs, int max_blocks, int decode_chunk) {
   return decode_chunk != 32 && (long long)max_blocks * bs >= ATT_DECODE_LONG_FROM &&
          decode_long_lds(nh / nkv, vd) + (size_t)hd / 32 * 4 * 64 * 16 <= 64 * 1024;

@@ -1492,10 +1492,8 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
 #define ZK_TILE(W_, M_, N_)                                                                            \
   (gated ? (exact ? ZK_TILE_(W_, M_, N_, true, true) : ZK_TILE_(W_, M_, N_, true, false))             \
          : (exact ? ZK_TILE_(W_, M_, N_, false, true) : ZK_TILE_(W_, M_, N_, false, false)))
-  // 256 x 256 blocks of sixteen waves where there are tiles enough.  The tile product is bound
-  // by what the caches deliver to a CU (a 128 x 256 x 64 step moves 48 KB for 4.2 MFLOP; hits in L2
-  // give 33 TB/s over all CUs, the memory-side cache behind it 7.5); a
-  // 256 x 256 block moves a third fewer bytes per flop.  Measured against 128 x 256: 0.88 of its
+  // 256 x 256 blocks of sixteen waves where there are tiles enough.  A 128 x 256 x 64 step moves 48 KB
+  // into a CU for 4.2 MFLOP, a 256 x 256 block a third fewer bytes per flop.  Measured against 128 x 256: 0.88 of its
   // time with many rounds of tiles (4096 x 36864 x 4608 gated), 0.91 at 2048 x 9216 x 2304 gated
   // (2.25 rounds), 1.4 at 2048 x 4096 x 2304 (half a round: half of the CUs idle).  The rule:
   // time = (rounds, at least one, + 0.15) x time of a tile.
