@@ -200,3 +200,39 @@ def test_more_blocks_of_columns_than_one_launch_holds(rt):
         want = rt.download(few)
         for m in range(M):
             assert np.array_equal(rt.download(type(C)(C.ptr + 4 * (m * N + n0), (2048,), "float32")), want[m]), (n0, m)
+
+
+# Many short runs: blocks that take eight (four) runs at once, one with all its waves, and several rounds of runs, with
+# padding rows between; the same tokens a few at a time go a run a block
+@pytest.mark.parametrize("nh,nkv,hd,vd,window,keep,chunk,turned", [(8, 8, 64, 64, 0, 0, 0, 0), (9, 3, 20, 128, 70, 3, 0, 0), (16, 8, 128, 128, 0, 0, 96, 1),
+                                                                   (6, 6, 256, 64, 40, 0, 0, 0), (34, 17, 4, 8, 0, 0, 0, 1)])
+def test_many_short_runs(rt, nh, nkv, hd, vd, window, keep, chunk, turned):
+    k = rt.kernels("float32")
+    rng = np.random.default_rng(nh + hd)
+    bs, slots, own, pos = 16, 24, [], []
+    lens = [rng.integers(1, 64), 64, 65, 128, 129, 250, 300, 600]            # keys a run may reach, by regions of the step
+    while len(own) < 3000:
+        top, n = int(lens[len(own) * len(lens) // 3001]), int(rng.choice([1, 1, 2, 3, 5, 9, 20]))
+        first = int(rng.integers(0, max(top - n, 0) + 1))
+        own += [len(own) % slots] * n
+        pos += list(range(first, first + n))
+        if rng.random() < 0.1:
+            own.append(0), pos.append(-1)
+    T, per = len(own), 640 // bs
+    Q, KC, VC = (rt.upload(rng.normal(size=s).astype(np.float32)) for s in ((T, nh, hd), (slots * per, nkv, bs, hd), (slots * per, nkv, bs, vd)))
+    TBL, S = rt.upload(rng.permutation(slots * per).astype(np.int32).reshape(slots, per)), rt.upload(rng.normal(size=nh).astype(np.float32))
+    POS, REQ, F = rt.upload(np.array(pos, np.int32)), rt.upload(np.array(own, np.int32)), rt.upload(rng.random(vd // 2).astype(np.float32))
+    OUT = rt.upload(np.full((T, nh, vd), 7.0, np.float32))
+
+    def run(t, n):
+        k.zk_attention_plain_gated(Q.ptr + 4 * t * nh * hd, nh * hd, KC.ptr, VC.ptr, TBL.ptr, per, REQ.ptr + 4 * t, POS.ptr + 4 * t,
+                                   OUT.ptr + 4 * t * nh * vd, n, nh, nkv, hd, vd, bs, 0.2, 0.0, window, 0, F.ptr if turned else None, 0, S.ptr,
+                                   0, chunk, 0, keep, None, 0, rt.stream)
+    run(0, T)
+    together = rt.download(OUT)
+    rt.zero_(OUT)
+    for t in range(0, T, 61):
+        run(t, min(61, T - t))
+    alone = rt.download(OUT)
+    assert np.isfinite(together).all() and np.array_equal(together, alone)
+    assert (together[np.array(pos) < 0] == 0).all() and (np.abs(together[np.array(pos) >= 0]).max(axis=(1, 2)) > 0).all()

@@ -20,6 +20,7 @@
 // contiguous K/V instead (:859-958) and never applies a window (:883).
 #include "common.h"
 
+#include <algorithm>
 #include <climits>
 
 #define AP_MAX_HD 256
@@ -165,13 +166,26 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 //   of 16: 6.9 -> 8.5, 26 -> 11, 884 -> 83; 8 over 4 of 256: 21.7 -> 22.7, 109 -> 27, 6,260 -> 458.  (Heads of up
 //   to 64 are slower than before below about ten keys, of 256 below three.)
 //
+// PACK: launches of many short runs (a step of many requests with a few tokens each).  A run that has a block to itself
+// leaves most of its waves without a tile, and with one head a key head most blocks are without a run.  1,000 requests of
+// 3 tokens (us; key by key, a run a block, packed): 8 heads of 128 over 2 68, 174, 92; 8 of 64 41, 480, 67; 8 over 4
+// of 256 136, 484, 172.  1,500 tokens behind a window of 64, 8 of 64: 99, 159, 50.  Finding a block's runs side by side is
+// in these figures; alone it makes one token with 1 key 9.7 -> 8.7 (4 heads of 16), 300 tokens 22.1 -> 20.9 (8 over 2
+// of 128), but long contexts of heads up to 64 5 to 8 % slower (4,000 keys, 8 of 64: 79.7 -> 84.1; cause not found).
+//
 // ASK: keys are asked for without a condition, and pieces of 16 that no row sees are passed over in the
 // first product too.  For key heads of 65 to 128 channels: one token with 1 key 14.5 -> 9.5 us, 16 tokens of 500
 // to 1,055 keys 53 -> 47, 1,500 tokens behind a window 102 -> 91.  Not for 64 channels with values of 128 (4,000
 // keys 125 -> 138) nor for smaller heads (80 -> 89); of 256 the loads in flight do not fit (446 -> 472).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int MAXD, int WAVES, bool ASK>
+// The value of another lane of the row of 16: 0x110 + n: of the lane n before (none: what is there for it), 0x120 + n: in a circle
+template <int WHICH>
+__device__ __forceinline__ int row_lane(int v, int none) {
+  return __builtin_amdgcn_update_dpp(none, v, WHICH, 0xf, 0xf, false);
+}
+
+template <int MAXD, int WAVES, bool ASK, bool PACK>
 __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
     const float* __restrict__ q, int q_stride, const float* __restrict__ kcache, const float* __restrict__ vcache,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ req_of_token,
@@ -188,229 +202,269 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
   const int kvh = blockIdx.y / chunks, h0 = blockIdx.y % chunks * 16;       // first of the block's heads in the group
   const int gh = min(16, group - h0), tb = max(1, 16 / group);              // heads, tokens of a block
   const int t0 = blockIdx.x * tb, n_tok = min(tb, T - t0);
-  // Block z takes the z-th run of neighbouring tokens of one request; padding rows (position < 0) belong to none.
-  int first = 0, last = -1, seen = -1;
-  bool running = false;
-  for (int i = 0; i < n_tok; i++) {
-    const bool live = positions[t0 + i] >= 0;
-    const bool starts = live && (!running || req_of_token[t0 + i] != req_of_token[t0 + i - 1]);
-    if (starts && ++seen == (int)blockIdx.z) first = i;
-    if (live && seen == (int)blockIdx.z) last = i;
-    running = live;
-    if (!live && blockIdx.z == 0)
-      for (int x = threadIdx.x; x < gh * vd; x += 64 * WAVES)
-        out[((size_t)(t0 + i) * nh + (size_t)kvh * group + h0) * vd + x] = 0.f;
-  }
-  if (last < 0) return;
+  // Lane i of every row of 16 looks at the block's token i, so one wait finds all runs of neighbouring tokens of one
+  // request; padding rows (position < 0) belong to none.
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, qd = lane >> 4;
-  const int rows = (last - first + 1) * gh;
+  const int my_pos = positions[t0 + min(r, n_tok - 1)], my_req = req_of_token[t0 + min(r, n_tok - 1)];
+  const bool my_live = r < n_tok && my_pos >= 0;
+  const unsigned live = (unsigned)__ballot(my_live) & 0xffffu;
+  const int req_before = row_lane<0x111>(my_req, -1);          // of the lane before
+  unsigned starts = (unsigned)__ballot(my_live && (!(live << 1 >> r & 1) || my_req != req_before)) & 0xffffu;
+  if (blockIdx.z == 0 && live != (1u << n_tok) - 1)
+    for (int i = 0; i < n_tok; i++)
+      if (!(live >> i & 1))
+        for (int x = threadIdx.x; x < gh * vd; x += 64 * WAVES)
+          out[((size_t)(t0 + i) * nh + (size_t)kvh * group + h0) * vd + x] = 0.f;
+  // a run's keys, at its last lane: from the lowest that a token of it sees to its highest position
   auto lowest = [&](int pos) { return window > 0 ? max(pos - window + 1, 0) : chunk > 0 ? pos / chunk * chunk : 0; };
-  // the run's keys: from the lowest that a token of it sees to its highest position
-  int seg_lo = INT_MAX, seg_hi = -1;
-  for (int i = first; i <= last; i++) {
-    const int p = positions[t0 + i];
-    seg_lo = min(seg_lo, lowest(p));
-    seg_hi = max(seg_hi, p);
+  const int my_run = __popc(starts & ((2u << r) - 1));
+  int run_lo = my_live ? lowest(my_pos) : INT_MAX, run_hi = my_live ? my_pos : -1;
+  auto widen = [&](int run, int lo, int hi) {
+    run_lo = run == my_run ? min(run_lo, lo) : run_lo;
+    run_hi = run == my_run ? max(run_hi, hi) : run_hi;
+  };
+  widen(row_lane<0x111>(my_run, -1), row_lane<0x111>(run_lo, 0), row_lane<0x111>(run_hi, 0));
+  widen(row_lane<0x112>(my_run, -1), row_lane<0x112>(run_lo, 0), row_lane<0x112>(run_hi, 0));
+  widen(row_lane<0x114>(my_run, -1), row_lane<0x114>(run_lo, 0), row_lane<0x114>(run_hi, 0));
+  widen(row_lane<0x118>(my_run, -1), row_lane<0x118>(run_lo, 0), row_lane<0x118>(run_hi, 0));
+  // With PACK as many waves as the longest run has tiles take a run (a power of two), and a block takes as many runs
+  // at once as it has room for.  A tile's place in the join's order stays its number modulo WAVES.
+  int team = WAVES;
+  if (PACK) {
+    int most = my_live ? run_hi / 64 + 1 - (keep > 0 ? 0 : run_lo / 64) : 0;
+    most = max(most, row_lane<0x128>(most, 0));
+    most = max(most, row_lane<0x124>(most, 0));
+    most = max(most, row_lane<0x122>(most, 0));
+    most = __builtin_amdgcn_readfirstlane(max(most, row_lane<0x121>(most, 0)));
+    team = most <= 1 ? 1 : most <= 2 ? 2 : most <= 4 ? 4 : WAVES;
   }
-  const int row = min(r, rows - 1);                  // rows past the last repeat it and are not stored
-  const int tok = t0 + first + row / gh, head = kvh * group + h0 + row % gh;
-  const int pos = positions[tok], lo = lowest(pos);
-  const int* table = block_table + (size_t)req_of_token[tok] * max_blocks;
+  const int runs = __popc(starts);
+  for (int z0 = blockIdx.z * (WAVES / team); z0 < runs; z0 += gridDim.z * (WAVES / team)) {
+    const bool active = z0 + wave / team < runs;              // a wave without a run still meets the others at the barriers
+    unsigned from = starts;
+    for (int z = active ? z0 + wave / team : 0; z > 0; z--) from &= from - 1;
+    const int run_first = __builtin_ctz(from);
+    // the run ends before the next one, before a padding row or with the block's tokens
+    const int run_last = __builtin_ctz((from & (from - 1)) | (~live & (~0u << run_first)) | 1u << n_tok) - 1;
+    const int run_rows = (run_last - run_first + 1) * gh;
+    const int seg_lo = __builtin_amdgcn_readlane(run_lo, run_last), seg_hi = active ? __builtin_amdgcn_readlane(run_hi, run_last) : -1;
+    const int row = min(r, run_rows - 1);              // rows past the last repeat it and are not stored
+    const int tok = t0 + run_first + row / gh, head = kvh * group + h0 + row % gh;
+    const int pos = __shfl(my_pos, run_first + row / gh), lo = lowest(pos);
+    const int* table = block_table + (size_t)__builtin_amdgcn_readlane(my_req, run_first) * max_blocks;
+    // what the join alone needs waits in a vector register: the loop wants more scalar ones than there are
+    int join = run_first | (active ? run_rows : 0) << 8 | team << 16;
+    asm volatile("" : "+v"(join));
 
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 qf[QC];
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 qf[QC];
 #pragma unroll
-  for (int c = 0; c < QC; c++) {
-    const int d = 16 * c + 4 * qd;
-    qf[c] = d < hd ? *(const f32x4*)(q + (size_t)tok * q_stride + (size_t)head * hd + d) : zero;
-  }
-  float m = -INFINITY, l = 0.f;
-  f32x4 acc[VC][4];            // [c][e][i]: channel 64 c + 16 qd + 4 i + e of the lane's query
-#pragma unroll
-  for (int c = 0; c < VC; c++)
-#pragma unroll
-    for (int e = 0; e < 4; e++) acc[c][e] = zero;
-
-  const int lo_tile = seg_lo / 64, kept_tiles = (keep + 63) / 64;
-  const int tile0 = keep > 0 ? 0 : lo_tile, tile1 = seg_hi / 64 + 1;
-  for (int tile = tile0 + (wave - tile0 % WAVES + WAVES) % WAVES; tile < tile1; tile += WAVES) {
-    if (tile >= kept_tiles && tile < lo_tile) continue;
-    const int j0 = tile * 64;
-    // the cache row of key 16 f + r; a key that no row of the run sees is never read (row -1)
-    long long at[4];
-#pragma unroll
-    for (int f = 0; f < 4; f++) {
-      const int j = j0 + 16 * f + r;
-      at[f] = -1;
-      if (j <= seg_hi && (j >= seg_lo || j < keep)) {
-        const int page = table[j / bs];
-        if (page >= 0) at[f] = ((long long)page * nkv + kvh) * bs + j % bs;
-      }
+    for (int c = 0; c < QC; c++) {
+      const int d = 16 * c + 4 * qd;
+      qf[c] = d < hd ? *(const f32x4*)(q + (size_t)tok * q_stride + (size_t)head * hd + d) : zero;
     }
-    auto unseen = [&](int f) { return j0 + 16 * f > seg_hi || (j0 + 16 * f + 15 < seg_lo && j0 + 16 * f >= keep); };
-    f32x4 s[4];
-#pragma unroll
-    for (int f = 0; f < 4; f++) {
-      s[f] = zero;
-      if (ASK && unseen(f)) continue;
-      const float* kr = kcache + (size_t)max(at[f], 0LL) * hd;
-#pragma unroll
-      for (int c = 0; c < QC; c++) {
-        const int d = 16 * c + 4 * qd;
-        f32x4 k4;
-        if (ASK) {
-          k4 = *(const f32x4*)(kr + min(d, hd - 4));
-          k4 = at[f] >= 0 && d < hd ? k4 : zero;
-        } else {
-          k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) s[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], qf[c][e], s[f], 0, 0, 0);
-      }
-    }
-    float top = -INFINITY;
-    bool all = true;             // the lane's query sees all of the lane's keys
-#pragma unroll
-    for (int f = 0; f < 4; f++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int j = j0 + 16 * f + 4 * qd + e;
-        float x = s[f][e] * scale;
-        if (softcap > 0.f) x = softcap * tanhf(x / softcap);
-        const bool sees = (j >= lo || j < keep) && j <= pos;
-        all = all && sees;
-        s[f][e] = sees ? x : -INFINITY;
-        top = fmaxf(top, s[f][e]);
-      }
-    top = fmaxf(top, __shfl_xor(top, 16));
-    top = fmaxf(top, __shfl_xor(top, 32));
-    const float m_new = fmaxf(m, top);
-    const float corr = m == m_new ? 1.f : expf(m - m_new);
-    float sum = 0.f;
-#pragma unroll
-    for (int f = 0; f < 4; f++)
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const int j = j0 + 16 * f + 4 * qd + e;
-        s[f][e] = (j >= lo || j < keep) && j <= pos ? expf(s[f][e] - m_new) : 0.f;
-        sum += s[f][e];
-      }
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    l = l * corr + sum;
-    m = m_new;
+    float m = -INFINITY, l = 0.f;
+    f32x4 acc[VC][4];            // [c][e][i]: channel 64 c + 16 qd + 4 i + e of the lane's query
 #pragma unroll
     for (int c = 0; c < VC; c++)
 #pragma unroll
-      for (int e = 0; e < 4; e++) acc[c][e] *= corr;
-    const bool whole = __all(all);
+      for (int e = 0; e < 4; e++) acc[c][e] = zero;
+
+    const int lo_tile = seg_lo / 64, kept_tiles = (keep + 63) / 64;
+    const int tile0 = keep > 0 ? 0 : lo_tile, tile1 = (seg_hi + 64) / 64;
+    auto first_tile = [&](int members) { return tile0 + ((wave - tile0) & (members - 1)); };       // the wave's first tile
+    for (int tile = first_tile(team); tile < tile1; tile += WAVES) {
+      if (tile >= kept_tiles && tile < lo_tile) continue;
+      const int j0 = tile * 64;
+      // the cache row of key 16 f + r; a key that no row of the run sees is never read (row -1)
+      long long at[4];
 #pragma unroll
-    for (int f = 0; f < 4; f++) {
-      if (PASS_VALUES && unseen(f)) continue;
-      f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
-      long long va[4];
-      bool fine = true;
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        va[e] = __shfl(at[f], 4 * qd + e);
-#pragma unroll
-        for (int c = 0; c < VC; c++) {
-          const int d = 64 * c + 4 * r;
-          v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
+      for (int f = 0; f < 4; f++) {
+        const int j = j0 + 16 * f + r;
+        at[f] = -1;
+        if (j <= seg_hi && (j >= seg_lo || j < keep)) {
+          const int page = table[j / bs];
+          if (page >= 0) at[f] = ((long long)page * nkv + kvh) * bs + j % bs;
         }
       }
-      if (!whole) {
+      auto unseen = [&](int f) { return j0 + 16 * f > seg_hi || (j0 + 16 * f + 15 < seg_lo && j0 + 16 * f >= keep); };
+      f32x4 s[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++)
+      for (int f = 0; f < 4; f++) {
+        s[f] = zero;
+        if (ASK && unseen(f)) continue;
+        const float* kr = kcache + (size_t)max(at[f], 0LL) * hd;
 #pragma unroll
-          for (int c = 0; c < VC; c++)
-#pragma unroll
-            for (int x = 0; x < 4; x++) fine = fine && fabsf(v[e][c][x]) < INFINITY;
-      }
-      if (__all(fine)) {
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-#pragma unroll
-          for (int c = 0; c < VC; c++)
-#pragma unroll
-            for (int x = 0; x < 4; x++)
-              acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
-      } else {
-        // rare: each query takes the keys that it sees, in the products' order (0, 4, 8, 12, 1, 5, ..)
-        for (int n = 0; n < 16; n++) {
-          const int kk = n % 4 * 4 + n / 4, j = j0 + 16 * f + kk;
-          const long long av = __shfl(at[f], kk);
-          float p = 0.f;
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const float x = __shfl(s[f][e], (kk >> 2) * 16 + r);
-            if (e == (kk & 3)) p = x;
+        for (int c = 0; c < QC; c++) {
+          const int d = 16 * c + 4 * qd;
+          f32x4 k4;
+          if (ASK) {
+            k4 = *(const f32x4*)(kr + min(d, hd - 4));
+            k4 = at[f] >= 0 && d < hd ? k4 : zero;
+          } else {
+            k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
           }
-          if (av < 0 || !((j >= lo || j < keep) && j <= pos)) continue;
 #pragma unroll
-          for (int c = 0; c < VC; c++)
+          for (int e = 0; e < 4; e++) s[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], qf[c][e], s[f], 0, 0, 0);
+        }
+      }
+      float top = -INFINITY;
+      bool all = true;             // the lane's query sees all of the lane's keys
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const int d = 64 * c + 16 * qd + 4 * i;
-              if (d >= vd) continue;
+      for (int f = 0; f < 4; f++)
 #pragma unroll
-              for (int e = 0; e < 4; e++) acc[c][e][i] = fmaf(vcache[(size_t)av * vd + d + e], p, acc[c][e][i]);
+        for (int e = 0; e < 4; e++) {
+          const int j = j0 + 16 * f + 4 * qd + e;
+          float x = s[f][e] * scale;
+          if (softcap > 0.f) x = softcap * tanhf(x / softcap);
+          const bool sees = (j >= lo || j < keep) && j <= pos;
+          all = all && sees;
+          s[f][e] = sees ? x : -INFINITY;
+          top = fmaxf(top, s[f][e]);
+        }
+      top = fmaxf(top, __shfl_xor(top, 16));
+      top = fmaxf(top, __shfl_xor(top, 32));
+      const float m_new = fmaxf(m, top);
+      const float corr = m == m_new ? 1.f : expf(m - m_new);
+      float sum = 0.f;
+#pragma unroll
+      for (int f = 0; f < 4; f++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const int j = j0 + 16 * f + 4 * qd + e;
+          s[f][e] = (j >= lo || j < keep) && j <= pos ? expf(s[f][e] - m_new) : 0.f;
+          sum += s[f][e];
+        }
+      sum += __shfl_xor(sum, 16);
+      sum += __shfl_xor(sum, 32);
+      l = l * corr + sum;
+      m = m_new;
+#pragma unroll
+      for (int c = 0; c < VC; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[c][e] *= corr;
+      const bool whole = __all(all);
+#pragma unroll
+      for (int f = 0; f < 4; f++) {
+        if (PASS_VALUES && unseen(f)) continue;
+        f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
+        long long va[4];
+        bool fine = true;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          va[e] = __shfl(at[f], 4 * qd + e);
+#pragma unroll
+          for (int c = 0; c < VC; c++) {
+            const int d = 64 * c + 4 * r;
+            v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
+          }
+        }
+        if (!whole) {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int c = 0; c < VC; c++)
+#pragma unroll
+              for (int x = 0; x < 4; x++) fine = fine && fabsf(v[e][c][x]) < INFINITY;
+        }
+        if (__all(fine)) {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int c = 0; c < VC; c++)
+#pragma unroll
+              for (int x = 0; x < 4; x++)
+                acc[c][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[e][c][x], s[f][e], acc[c][x], 0, 0, 0);
+        } else {
+          // rare: each query takes the keys that it sees, in the products' order (0, 4, 8, 12, 1, 5, ..)
+          for (int n = 0; n < 16; n++) {
+            const int kk = n % 4 * 4 + n / 4, j = j0 + 16 * f + kk;
+            const long long av = __shfl(at[f], kk);
+            float p = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+              const float x = __shfl(s[f][e], (kk >> 2) * 16 + r);
+              if (e == (kk & 3)) p = x;
             }
+            if (av < 0 || !((j >= lo || j < keep) && j <= pos)) continue;
+#pragma unroll
+            for (int c = 0; c < VC; c++)
+#pragma unroll
+              for (int i = 0; i < 4; i++) {
+                const int d = 64 * c + 16 * qd + 4 * i;
+                if (d >= vd) continue;
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[c][e][i] = fmaf(vcache[(size_t)av * vd + d + e], p, acc[c][e][i]);
+              }
+          }
         }
       }
     }
-  }
+    join = __builtin_amdgcn_readfirstlane(join);
+    const int first = join & 255, rows = join >> 8 & 255, members = join >> 16;
+    if (first_tile(members) < tile1) {
 #pragma unroll
-  for (int c = 0; c < VC; c++)
+      for (int c = 0; c < VC; c++)
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-      *(f32x4*)&s_acc[wave][r][64 * c + 16 * qd + 4 * i] = f32x4{acc[c][0][i], acc[c][1][i], acc[c][2][i], acc[c][3][i]};
-  if (qd == 0) {
-    s_m[wave][r] = m;
-    s_l[wave][r] = l;
-  }
-  __syncthreads();
-  // a thread joins four channels of a row over the waves
-  for (int x = threadIdx.x; x < rows * (vd / 4); x += 64 * WAVES) {
-    const int rr = x / (vd / 4), d = x % (vd / 4) * 4;
-    const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
-    float top = -INFINITY, den = 0.f;
-#pragma unroll
-    for (int w = 0; w < WAVES; w++) top = fmaxf(top, s_m[w][rr]);
-    f32x4 o = zero;
-#pragma unroll
-    for (int w = 0; w < WAVES; w++) {
-      const float f = s_m[w][rr] == top ? 1.f : expf(s_m[w][rr] - top);
-      den += s_l[w][rr] * f;
-      o += *(const f32x4*)&s_acc[w][rr][d] * f;
+        for (int i = 0; i < 4; i++)
+          *(f32x4*)&s_acc[wave][r][64 * c + 16 * qd + 4 * i] = f32x4{acc[c][0][i], acc[c][1][i], acc[c][2][i], acc[c][3][i]};
+      if (qd == 0) {
+        s_m[wave][r] = m;
+        s_l[wave][r] = l;
+      }
     }
-    if (sinks != nullptr || unit_sink) {
-      const float sk = sinks != nullptr ? sinks[h] : 0.f;
-      const float m_new = fmaxf(top, sk), corr = expf(top - m_new);
-      den = den * corr + expf(sk - m_new);
-      o *= corr;
+    __syncthreads();
+    // a thread joins four channels of a row over the run's waves
+    const int wave0 = wave & -members;
+    for (int x = threadIdx.x & (64 * members - 1); x < rows * (vd / 4); x += 64 * members) {
+      const int rr = x / (vd / 4), d = x % (vd / 4) * 4;
+      const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
+      float part[WAVES], top = -INFINITY, den = 0.f;
+      auto holds = [&](int w) { return tile0 + ((w - tile0) & (WAVES - 1)) < tile1; };       // the w-th place in the order
+      auto at_wave = [&](int w) { return holds(w) ? wave0 + (w & (members - 1)) : wave0; };
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) {
+        part[w] = holds(w) ? s_m[at_wave(w)][rr] : -INFINITY;
+        top = fmaxf(top, part[w]);
+      }
+      f32x4 o = zero;
+#pragma unroll
+      for (int w = 0; w < WAVES; w++) {
+        const float f = part[w] == top ? 1.f : expf(part[w] - top);
+        den += holds(w) ? s_l[at_wave(w)][rr] * f : 0.f;
+        o += holds(w) ? *(const f32x4*)&s_acc[at_wave(w)][rr][d] * f : zero;
+      }
+      if (sinks != nullptr || unit_sink) {
+        const float sk = sinks != nullptr ? sinks[h] : 0.f;
+        const float m_new = fmaxf(top, sk), corr = expf(top - m_new);
+        den = den * corr + expf(sk - m_new);
+        o *= corr;
+      }
+      float inv = 1.f / den;
+      if (gate != nullptr) inv *= 1.f / (1.f + expf(-gate[(size_t)t * gate_ld + h]));
+      o *= inv;
+      if (v_freq == nullptr) *(f32x4*)(out + ((size_t)t * nh + h) * vd + d) = o;
+      else *(f32x4*)&s_acc[wave0][rr][d] = o;      // a place that no other thread reads
     }
-    float inv = 1.f / den;
-    if (gate != nullptr) inv *= 1.f / (1.f + expf(-gate[(size_t)t * gate_ld + h]));
-    o *= inv;
-    if (v_freq == nullptr) *(f32x4*)(out + ((size_t)t * nh + h) * vd + d) = o;
-    else *(f32x4*)&s_acc[0][rr][d] = o;          // the place that this thread alone has read
-  }
-  if (v_freq == nullptr) return;
-  // values were turned by their own positions when they were stored: the sum is turned back
-  // by the query's position, pair m by -pos * v_freq[m]
-  __syncthreads();
-  const int half = vd / 2;
-  for (int x = threadIdx.x; x < rows * half; x += 64 * WAVES) {
-    const int rr = x / half, m2 = x % half;
-    const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
-    float sn, cs, ra, rb;
-    sincosf(-(float)positions[t] * v_freq[m2], &sn, &cs);
-    const int ia = v_interleaved ? 2 * m2 : m2, ib = v_interleaved ? 2 * m2 + 1 : m2 + half;
-    rotate_pair(s_acc[0][rr][ia], s_acc[0][rr][ib], sn, cs, ra, rb);
-    out[((size_t)t * nh + h) * vd + ia] = ra;
-    out[((size_t)t * nh + h) * vd + ib] = rb;
+    if (v_freq != nullptr) {
+      // values were turned by their own positions when they were stored: the sum is turned back
+      // by the query's position, pair m by -pos * v_freq[m]
+      __syncthreads();
+      const int half = vd / 2;
+      for (int x = threadIdx.x & (64 * members - 1); x < rows * half; x += 64 * members) {
+        const int rr = x / half, m2 = x % half;
+        const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
+        float sn, cs, ra, rb;
+        sincosf(-(float)positions[t] * v_freq[m2], &sn, &cs);
+        const int ia = v_interleaved ? 2 * m2 : m2, ib = v_interleaved ? 2 * m2 + 1 : m2 + half;
+        rotate_pair(s_acc[wave0][rr][ia], s_acc[wave0][rr][ib], sn, cs, ra, rb);
+        out[((size_t)t * nh + h) * vd + ia] = ra;
+        out[((size_t)t * nh + h) * vd + ib] = rb;
+      }
+    }
+    if (!PACK) break;                // a block for every run that there can be
+    __syncthreads();                 // the next runs' results go where these were
   }
 }
 #endif  // !ZSE_ACT_BF16
@@ -454,17 +508,33 @@ extern "C" int zk_attention_plain_gated(const void* q, int q_stride, const void*
     const int most_tokens = (1 << 22) * tb;
     for (long long t = 0; t < T; t += most_tokens) {
       const int n = T - t < most_tokens ? (int)(T - t) : most_tokens;
-      const dim3 blocks((n + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
-#define ZK_ATTENTION_F32(D_, W_, A_)                                                                                  \
-  attention_f32_kernel<D_, W_, A_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                      \
+      // Where a run a block makes few rounds of blocks, a run has a block to itself; otherwise short runs share blocks,
+      // and few blocks are without a run.  From 1,024 blocks on where eight tokens or more share one (64 requests of 3
+      // tokens, 8 heads of 64: 20 -> 12 us), else from 4,096 on (1,500 tokens, 8 over 1 of 32: 1,500 blocks take 65 us
+      // and 75 packed; 16 requests of 20, 8 over 4 of 256: 1,280 take 28 and 36).
+      dim3 blocks((n + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
+      const long long columns = (long long)blocks.x * blocks.y;
+      const bool pack = columns * tb > (tb >= 8 && most <= 128 ? 1024 : 4096) && tb > 1;
+      if (pack) blocks.z = (unsigned)std::min<long long>(tb, (2048 + columns - 1) / columns);
+#define ZK_ATTENTION_F32(D_, W_, A_, P_)                                                                               \
+  attention_f32_kernel<D_, W_, A_, P_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                      \
       (const float*)q + t * q_stride, q_stride, (const float*)kcache, (const float*)vcache, block_table,              \
       max_blocks, req_of_token + t, positions + t, (float*)out + t * nh * vd, n, nh, nkv, hd, vd, bs, scale,          \
       softcap, window, v_freq, v_interleaved, sinks, chunk, unit_sink, keep,                                          \
       gate == nullptr ? nullptr : (const float*)gate + t * gate_ld, gate_ld)
-      if (most <= 64) ZK_ATTENTION_F32(64, 8, false);
-      else if (most <= 128 && hd > 64) ZK_ATTENTION_F32(128, 8, true);
-      else if (most <= 128) ZK_ATTENTION_F32(128, 8, false);
-      else ZK_ATTENTION_F32(256, 4, false);
+#define ZK_ATTENTION_F32_PACK(D_, W_, A_)                                                                             \
+  if (pack) ZK_ATTENTION_F32(D_, W_, A_, true);                                                                       \
+  else ZK_ATTENTION_F32(D_, W_, A_, false)
+      if (most <= 64) {
+        ZK_ATTENTION_F32_PACK(64, 8, false);
+      } else if (most <= 128 && hd > 64) {
+        ZK_ATTENTION_F32_PACK(128, 8, true);
+      } else if (most <= 128) {
+        ZK_ATTENTION_F32_PACK(128, 8, false);
+      } else {
+        ZK_ATTENTION_F32_PACK(256, 4, false);
+      }
+#undef ZK_ATTENTION_F32_PACK
 #undef ZK_ATTENTION_F32
     }
     return zk_launch_status("zk_attention_plain");
