@@ -169,9 +169,7 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // PACK: launches of many short runs (a step of many requests with a few tokens each).  A run that has a block to itself
 // leaves most of its waves without a tile, and with one head a key head most blocks are without a run.  1,000 requests of
 // 3 tokens (us; key by key, a run a block, packed): 8 heads of 128 over 2 68, 174, 92; 8 of 64 41, 480, 67; 8 over 4
-// of 256 136, 484, 172.  1,500 tokens behind a window of 64, 8 of 64: 99, 159, 50.  Finding a block's runs side by side is
-// in these figures; alone it makes one token with 1 key 9.7 -> 8.7 (4 heads of 16), 300 tokens 22.1 -> 20.9 (8 over 2
-// of 128), but long contexts of heads up to 64 5 to 8 % slower (4,000 keys, 8 of 64: 79.7 -> 84.1; cause not found).
+// of 256 136, 484, 172.  1,500 tokens behind a window of 64, 8 of 64: 99, 159, 50.
 //
 // ASK: keys are asked for without a condition, and pieces of 16 that no row sees are passed over in the
 // first product too.  For key heads of 65 to 128 channels: one token with 1 key 14.5 -> 9.5 us, 16 tokens of 500
@@ -402,8 +400,8 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
       }
     }
     join = __builtin_amdgcn_readfirstlane(join);
-    const int first = join & 255, rows = join >> 8 & 255, members = join >> 16;
-    if (first_tile(members) < tile1) {
+    const int first = join & 255, rows = join >> 8 & 255, members = PACK ? join >> 16 : WAVES;
+    if (!PACK || first_tile(members) < tile1) {
 #pragma unroll
       for (int c = 0; c < VC; c++)
 #pragma unroll
@@ -421,7 +419,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
       const int rr = x / (vd / 4), d = x % (vd / 4) * 4;
       const int t = t0 + first + rr / gh, h = kvh * group + h0 + rr % gh;
       float part[WAVES], top = -INFINITY, den = 0.f;
-      auto holds = [&](int w) { return tile0 + ((w - tile0) & (WAVES - 1)) < tile1; };       // the w-th place in the order
+      auto holds = [&](int w) { return !PACK || tile0 + ((w - tile0) & (WAVES - 1)) < tile1; };       // the w-th place in the order
       auto at_wave = [&](int w) { return holds(w) ? wave0 + (w & (members - 1)) : wave0; };
 #pragma unroll
       for (int w = 0; w < WAVES; w++) {
@@ -432,8 +430,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
       for (int w = 0; w < WAVES; w++) {
         const float f = part[w] == top ? 1.f : expf(part[w] - top);
-        den += holds(w) ? s_l[at_wave(w)][rr] * f : 0.f;
-        o += holds(w) ? *(const f32x4*)&s_acc[at_wave(w)][rr][d] * f : zero;
+        // (written out: the sums' bits are not to hang on what the compiler fuses in which form)
+        den = fmaf(holds(w) ? s_l[at_wave(w)][rr] : 0.f, f, den);
+        const f32x4 v = holds(w) ? *(const f32x4*)&s_acc[at_wave(w)][rr][d] : zero;
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = fmaf(v[e], f, o[e]);
       }
       if (sinks != nullptr || unit_sink) {
         const float sk = sinks != nullptr ? sinks[h] : 0.f;
@@ -510,11 +511,12 @@ extern "C" int zk_attention_plain_gated(const void* q, int q_stride, const void*
       const int n = T - t < most_tokens ? (int)(T - t) : most_tokens;
       // Where a run a block makes few rounds of blocks, a run has a block to itself; otherwise short runs share blocks,
       // and few blocks are without a run.  From 1,024 blocks on where eight tokens or more share one (64 requests of 3
-      // tokens, 8 heads of 64: 20 -> 12 us), else from 4,096 on (1,500 tokens, 8 over 1 of 32: 1,500 blocks take 65 us
-      // and 75 packed; 16 requests of 20, 8 over 4 of 256: 1,280 take 28 and 36).
+      // tokens, 8 heads of 64: 20 -> 12 us), from 2,048 on with more than 128 channels (16 requests of 20, 8 over 4 of 256:
+      // 1,280 blocks take 28 us and 36 packed, 256 of 3: 3,072 take 128 and 57), else from 4,096 on (1,500 tokens, 8 over
+      // 1 of 32: 1,500 blocks take 65 and 75).
       dim3 blocks((n + tb - 1) / tb, nkv * ((group + 15) / 16), tb);
       const long long columns = (long long)blocks.x * blocks.y;
-      const bool pack = columns * tb > (tb >= 8 && most <= 128 ? 1024 : 4096) && tb > 1;
+      const bool pack = columns * tb > (tb < 8 ? 4096 : most > 128 ? 2048 : 1024) && tb > 1;
       if (pack) blocks.z = (unsigned)std::min<long long>(tb, (2048 + columns - 1) / columns);
 #define ZK_ATTENTION_F32(D_, W_, A_, P_)                                                                               \
   attention_f32_kernel<D_, W_, A_, P_><<<blocks, 64 * W_, 0, (hipStream_t)stream>>>(                                      \
