@@ -9,8 +9,8 @@
 //    needed.  Partial sums of the waves meet in LDS.
 //  * mid (17 <= M <= 64, strip layout): four strips a block, two waves each, the activations
 //    of a k chunk shared through LDS, K split over blocks when N alone gives too few of them.
-//  * tile (M > 64, prefill): 256x256x64 (sixteen waves), 128x256x64 (eight) or 128x128x64 (four)
-//    block tiles staged through LDS, each wave a 64x64 corner built from 32x32x16 MFMAs.
+//  * tile (M > 64, prefill): weights in strip layout by the kernel of gemm_bf16_tiles.h, others by
+//    128x128x64 to 256x256x64 block tiles staged through registers and LDS.
 // Epilogues: plain store (bf16 or float), soft cap on float output (LM head), and
 // the gated activation act(gate) * up over a [2I, K] weight whose first I rows are
 // the gate (the feed-forward's first product; the [T, 2I] intermediate never
@@ -703,157 +703,6 @@ __global__ __launch_bounds__(64 * NWM * NWN, NWM * NWN <= 4 ? 2 : 1) void gemm_t
   tile_store<WMT, NWN, GATED>(acc, C, ldc, c_is_f32, M, N, m0, n0, wm, wn, lane, epi, cap);
 }
 
-// A tile product whose operands are copied from memory straight into LDS (global_load_lds, 16
-// bytes a lane): no registers hold a tile on its way and no LDS writes are issued, so a wave
-// has room for a second set of operand fragments, and LDS has room for GD_NS stages of 32 k
-// values each.  The block meets at a barrier once per stage, and the reads of a wave's operands
-// run one k step of 16 ahead of its products across that barrier: when the barrier of stage s
-// has shown that stage s + 1 is there, its first operands are read while the second half of
-// stage s is multiplied, so the matrix unit does not drain at a stage's end.  For weights in the
-// strip layout and K a whole number of 64; the sums and their order are those of
-// gemm_tile_kernel, and so are the partial sums of a split K and the results' way out.
-// Measured on 2B and 9B layer shapes of 2,048 and 4,096 rows against the 256 x 256 block of
-// sixteen waves that stages its tiles through registers: two stages of 64 k with one barrier
-// each and 16-byte pieces of sixteen different rows a quarter wave 1.05 of its time; the same
-// with 128-byte runs of a row 0.98; four stages of 32 k with the reads running ahead 0.96 (five
-// stages 0.97); eight waves of 128 x 64 each instead of sixteen of 64 x 64 0.94.
-//
-// Such a load puts lane l's 16 bytes at (destination + 16 l).  W: a strip's 1 KB for one k
-// step lies in LDS as it lies in memory, [k piece of 8][row 16][8 values]; an operand read
-// (row lane % 32, k piece lane / 32) takes whole 256-byte runs.  A: an instruction takes 16
-// rows x 32 k, four lanes a row (a 64-byte run of the row); lane c of a row fetches k piece
-// c ^ ((row / 4) % 4), so piece q of row R lies at place q ^ ((R / 4) % 4) of the row's 64
-// bytes and the sixteen rows a read takes at once lie in different banks.
-#define ZK_GLOBAL_AS __attribute__((address_space(1)))
-#define ZK_LDS_AS __attribute__((address_space(3)))
-#define GD_NS 4
-#define GD_BK 32
-template <int WMT, int NWM, int NWN, bool GATED>
-__global__ __launch_bounds__(64 * NWM * NWN, NWM * NWN <= 4 ? 2 : 1) void gemm_tile_direct_kernel(
-    const __bf16* __restrict__ A, int lda, const __bf16* __restrict__ W, void* __restrict__ C, int ldc,
-    int c_is_f32, int M, int N, int K_all, int epi, float cap, int tiles_m, int tiles_n, int w_strip,
-    f32x16* __restrict__ partials, int ksplit, int tile_base) {
-  constexpr int BM = 32 * WMT * NWM, BN = 64 * NWN, NW = NWM * NWN;
-  constexpr int LPA = BM / 16 / NW, LPB = BN / 16 / NW;     // row blocks of A, strips of W, a wave copies
-  static_assert(LPA * NW * 16 == BM && LPB * NW * 16 == BN, "the waves do not share the copies evenly");
-  constexpr int HALF = BM * GD_BK * 2, STAGE = (BM + BN) * GD_BK * 2;      // bytes of a stage's A part, of a stage
-  extern __shared__ __align__(16) unsigned char gt_lds[];
-  int tm, tn;
-  tile_of_block(blockIdx.x + tile_base, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM;
-  constexpr int NCOLS = GATED ? BN / 2 : BN;
-  const int n0 = tn * NCOLS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / NWN, wn = wave % NWN;
-  const int lr = lane & 31, lk = lane >> 5;
-  const int ktiles = K_all / GT_BK;
-  const int kt0 = (int)((long)blockIdx.y * ktiles / ksplit), kt1 = (int)((long)(blockIdx.y + 1) * ktiles / ksplit);
-  const int ns = 2 * (kt1 - kt0);                       // stages: an even number
-  // a wave copies the 16-row blocks wave, wave + NW, .. of A and the same strips of W
-  const __bf16* ga[LPA];
-  const __bf16* gw[LPB];
-  const int ksteps = K_all / 32;
-  const int strips = GATED ? 2 * N / 16 : N / 16;
-#pragma unroll
-  for (int c = 0; c < LPA; c++) {
-    const int a_row = (wave + c * NW) * 16 + (lane >> 2);
-    ga[c] = A + (size_t)min(m0 + a_row, M - 1) * lda + (size_t)kt0 * GT_BK + (((lane & 3) ^ ((a_row >> 2) & 3)) * 8);
-  }
-#pragma unroll
-  for (int c = 0; c < LPB; c++) {
-    const int blk = wave + c * NW;
-    int gs;
-    if (GATED) gs = blk < BN / 32 ? n0 / 16 + blk : N / 16 + n0 / 16 + (blk - BN / 32);
-    else gs = n0 / 16 + blk;
-    gs = min(gs, strips - 1);
-    gw[c] = W + ((size_t)gs * ksteps + 2 * kt0) * 512 + lane * 8;
-  }
-  auto issue = [&](int buf, int stage) {
-    stage = min(stage, ns - 1);      // past the end: the last stage again, into a buffer nobody reads
-    unsigned char* dst = gt_lds + buf * STAGE + wave * 1024;
-#pragma unroll
-    for (int c = 0; c < LPA; c++)
-      __builtin_amdgcn_global_load_lds((const ZK_GLOBAL_AS void*)(ga[c] + (size_t)stage * GD_BK), (ZK_LDS_AS void*)(dst + c * NW * 1024), 16, 0, 0);
-#pragma unroll
-    for (int c = 0; c < LPB; c++)
-      __builtin_amdgcn_global_load_lds((const ZK_GLOBAL_AS void*)(gw[c] + (size_t)stage * 512), (ZK_LDS_AS void*)(dst + HALF + c * NW * 1024), 16, 0, 0);
-  };
-  // where a lane reads its operand pieces of k step ks (0 or 1) of a stage
-  int a_at[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ks++) a_at[ks] = (wm * (32 * WMT) + lr) * 64 + (((ks * 2 + lk) ^ ((lr >> 2) & 3)) * 16);   // + i * 2048
-  const int w_row = GATED ? wn * 32 : wn * 64;                                    // + j * (GATED ? 128 : 32)
-  const int w_at = HALF + (w_row / 16 + (lr >> 4)) * 1024 + lk * 256 + (lr & 15) * 16;   // + ks * 512 + j * W_J
-  constexpr int W_J = GATED ? (BN / 32) * 1024 : 2048;
-  f32x16 acc[WMT][2];
-#pragma unroll
-  for (int i = 0; i < WMT; i++)
-#pragma unroll
-    for (int j = 0; j < 2; j++)
-#pragma unroll
-      for (int e = 0; e < 16; e++) acc[i][j][e] = 0.f;
-  bf16x8 fa[2][WMT], fb[2][2];
-  auto read = [&](int buf, int ks) {
-    const unsigned char* base = gt_lds + buf * STAGE;
-#pragma unroll
-    for (int i = 0; i < WMT; i++) fa[ks][i] = *(const bf16x8*)(base + a_at[ks] + i * 2048);
-#pragma unroll
-    for (int j = 0; j < 2; j++) fb[ks][j] = *(const bf16x8*)(base + w_at + ks * 512 + j * W_J);
-  };
-  auto products = [&](int ks) {
-    __builtin_amdgcn_sched_barrier(0x616);
-#pragma unroll
-    for (int i = 0; i < WMT; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks][j], fa[ks][i], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0x616);
-  };
-  // Stage s lives in buffer s % GD_NS.  In flight when a step begins: stages s + 1 .. s + GD_NS - 2
-  // (LPA + LPB loads a wave each); the wait is for the wave's own loads of stage s + 1, the barrier
-  // then says that every wave's are there and that every wave has read stage s - 1 (the products
-  // that use its operands were issued before the barrier, so the operands had arrived), whose
-  // buffer the next loads go to.
-  auto step = [&](int b, int s) {
-    read(b, 1);
-    products(0);
-    // (the barrier as text: before one it knows, the compiler waits for every load in flight)
-    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((LPA + LPB) * (GD_NS - 3)) : "memory");
-    issue((b + GD_NS - 1) % GD_NS, s + GD_NS - 1);
-    read((b + 1) % GD_NS, 0);
-    products(1);
-  };
-#pragma unroll
-  for (int b = 0; b < GD_NS - 1; b++) issue(b, b);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((LPA + LPB) * (GD_NS - 2)) : "memory");
-  read(0, 0);
-  for (int s = 0; s < ns; s += GD_NS) {
-#pragma unroll
-    for (int b = 0; b < GD_NS; b += 2) {
-      if (b > 0 && s + b >= ns) break;
-      step(b, s + b);
-      step(b + 1, s + b + 1);
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();                              // the buffers are free for the results' way out
-  if (ksplit > 1) {
-    f32x16* mine = partials + (((size_t)blockIdx.x * ksplit + blockIdx.y) * NW + wave) * (WMT * 2 * 64) + lane;
-#pragma unroll
-    for (int i = 0; i < WMT; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) mine[(i * 2 + j) * 64] = acc[i][j];
-    return;
-  }
-  if (!c_is_f32 && n0 + NCOLS <= N && ldc % 8 == 0 && (uintptr_t)C % 16 == 0) {
-    constexpr int WCOLS = GATED ? 32 : 64;
-    tile_store_staged<WMT, GATED>(acc, (__bf16*)C, ldc, M, m0 + wm * (32 * WMT), n0 + wn * WCOLS, lane, epi, cap,
-                                  (__bf16*)gt_lds + (size_t)wave * (32 * WMT) * (WCOLS + 8));
-    return;
-  }
-  tile_store<WMT, NWN, GATED>(acc, C, ldc, c_is_f32, M, N, m0, n0, wm, wn, lane, epi, cap);
-}
-
 // Second half of a tile product whose K was split over blocks: the ranges are added in order.
 // A thread takes four consecutive floats of a lane's accumulator pair (i, 0), (i, 1), so the
 // partial sums are read in 16-byte pieces, neighbours by neighbouring threads.
@@ -907,16 +756,14 @@ __global__ __launch_bounds__(256) void gemm_tile_join_kernel(
                                    wave / NWN, wave % NWN, lane, epi, cap);
 }
 
-template <int WMT, int NWM, int NWN, bool GATED, bool EXACT, bool DIRECT = false>
+template <int WMT, int NWM, int NWN, bool GATED, bool EXACT>
 static int launch_tile(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32, int M, int N,
                        int K, int epi, float cap, int w_strip, const GemmWorkspace& wsp, int ksplit,
                        int tail_split, hipStream_t s) {
   constexpr int BM = 32 * WMT * NWM, BN = 64 * NWN;
   constexpr int ncols = GATED ? BN / 2 : BN;
-  constexpr size_t lds_staged = (size_t)2 * (BM + BN) * GT_LD * sizeof(__bf16);
-  constexpr size_t lds = DIRECT && (size_t)GD_NS * (BM + BN) * GD_BK * 2 > lds_staged ? (size_t)GD_NS * (BM + BN) * GD_BK * 2 : lds_staged;
-  auto kernel = gemm_tile_kernel<WMT, NWM, NWN, GATED, EXACT>;
-  if constexpr (DIRECT) kernel = gemm_tile_direct_kernel<WMT, NWM, NWN, GATED>;
+  constexpr size_t lds = (size_t)2 * (BM + BN) * GT_LD * sizeof(__bf16);
+  const auto kernel = gemm_tile_kernel<WMT, NWM, NWN, GATED, EXACT>;
   static bool prepared = false;
   if (!prepared) {
     if (lds > 64 * 1024 &&
@@ -1154,6 +1001,20 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const __bf16* __restrict_
   if (strip_ok) mid_store<MT, GATED>(acc, C, ldc, c_is_f32, M, N, strip, lane, epi, cap, partials, nstrips);
 }
 
+// Four neighbouring results of a row, in one store where the address allows it.
+__device__ __forceinline__ void store_quad(void* __restrict__ C, int ldc, int c_is_f32, int m, int n, int N, const float (&v)[4]) {
+  if (!c_is_f32 && n + 4 <= N && ldc % 4 == 0 && (uintptr_t)C % 8 == 0) {
+    store4((__bf16*)C + (size_t)m * ldc + n, v);
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    if (n + i >= N) continue;
+    if (c_is_f32) ((float*)C)[(size_t)m * ldc + n + i] = v[i];
+    else ((__bf16*)C)[(size_t)m * ldc + n + i] = (__bf16)v[i];
+  }
+}
+
 // Second half of a mid product whose K was split over blocks: `ksplit`
 // ranges of one ([M, npad] floats) or, GATED, two planes each; a thread adds four neighbouring
 // columns of a row in the order of the ranges and applies the epilogue.  A reader that adds the
@@ -1174,17 +1035,13 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(const float* __restrict_
     x += *(const f32x4*)(at + (size_t)p * NS * plane);
     if (GATED) y += *(const f32x4*)(at + ((size_t)p * NS + 1) * plane);
   }
+  float v[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (n + i >= N) continue;
-    float v = x[i];
-    if (GATED) v = epi_gate(v, y[i], epi, cap);
-    else v = epi_unary(v, epi, cap);
-    if (c_is_f32) ((float*)C)[(size_t)m * ldc + n + i] = v;
-    else ((__bf16*)C)[(size_t)m * ldc + n + i] = (__bf16)v;
-  }
+  for (int i = 0; i < 4; i++) v[i] = GATED ? epi_gate(x[i], y[i], epi, cap) : epi_unary(x[i], epi, cap);
+  store_quad(C, ldc, c_is_f32, m, n, N, v);
 }
 
+#include "gemm_bf16_tiles.h"
 
 template <bool GATED>
 static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32, int M, int N,
@@ -1440,28 +1297,12 @@ static double tile_cost(TileChoice c, int M, int N, int K, bool gated, size_t ro
   return t > memory ? t : memory;
 }
 
-static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
-                         int M, int N, int K, int epi, float cap, int w_strip, const GemmWorkspace& wsp,
-                         int* parts, void* stream) {
-  ZK_REQUIRE(M >= 0 && N > 0 && K > 0, "zk_gemm_bf16: bad sizes");
-  ZK_REQUIRE(K % 8 == 0 && lda % 8 == 0, "zk_gemm_bf16: K and lda must be multiples of 8");
-  ZK_REQUIRE(lda >= K && ldc >= N, "zk_gemm_bf16: leading dimensions too small");
-  ZK_REQUIRE(epi >= 0 && epi <= EPI_GELU, "zk_gemm_bf16: unknown epilogue");
-  ZK_REQUIRE((epi != EPI_SOFTCAP && epi != EPI_CLAMPED) || cap > 0.f, "zk_gemm_bf16: soft cap or clamp limit must be positive");
-  ZK_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "zk_gemm_bf16: operands must be 16-byte aligned");
-  const bool gated = epi == EPI_GELU_TANH || epi == EPI_SILU || epi == EPI_RELU || epi == EPI_CLAMPED;
-  ZK_REQUIRE(!w_strip || (K % 32 == 0 && (!gated || N % 16 == 0)), "zk_gemm_bf16: strip layout needs K % 32 == 0 (and N % 16 == 0 when gated)");
-  if (parts) *parts = 0;
-  if (M == 0) return 0;
-  hipStream_t s = (hipStream_t)stream;
-  if (M > 16 && M <= 64 && w_strip) {
-    return gated ? launch_mid<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s)
-                 : launch_mid<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s);
-  }
-  if (M <= 64) {
-    return gated ? launch_skinny<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s)
-                 : launch_skinny<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s);
-  }
+// Tiles that pass through registers (weights row by row, or K not whole stages): which block, how
+// many ranges of K, of the last round's tiles.
+struct StagedCut {
+  int variant, ksplit, tail_split;      // 0: 128 x 128, 1: 64 x 128, 2: 128 x 256, 3: 256 x 256
+};
+static StagedCut staged_cut(int M, int N, int K, bool gated, size_t room) {
   // 128 x 128 blocks of four waves (two share a CU) or 128 x 256 blocks of eight (one a CU,
   // about 1.2 times the rate).  What counts is the CU with the most blocks; a lone small block
   // runs at about 0.8 of the rate of two.  The constants are measured (M = 512 and 2048 with
@@ -1487,11 +1328,6 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
   // a block; 64-row tiles make twice as many (they lose to a split of K where K allows one)
   const bool low = !wide && M > 64 && nb_small * ksplit <= 128;
   if (low) ksplit = ranges((long)((M + 63) / 64) * (nb_small / tiles_m));
-#define ZK_TILE_(W_, M_, N_, G_, E_) \
-  launch_tile<W_, M_, N_, G_, E_>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, ksplit, tail_split, s)
-#define ZK_TILE(W_, M_, N_)                                                                            \
-  (gated ? (exact ? ZK_TILE_(W_, M_, N_, true, true) : ZK_TILE_(W_, M_, N_, true, false))             \
-         : (exact ? ZK_TILE_(W_, M_, N_, false, true) : ZK_TILE_(W_, M_, N_, false, false)))
   // 256 x 256 blocks of sixteen waves where there are tiles enough.  A 128 x 256 x 64 step moves 48 KB
   // into a CU for 4.2 MFLOP, a 256 x 256 block a third fewer bytes per flop.  Measured against 128 x 256: 0.88 of its
   // time with many rounds of tiles (4096 x 36864 x 4608 gated), 0.91 at 2048 x 9216 x 2304 gated
@@ -1512,7 +1348,6 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
   // more than 3 % slower than the rules on the sweep, and 5 % faster in the sum).
   {
     const TileChoice rule{variant, ksplit};
-    const size_t room = (wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 64 == 0) ? wsp.split_bytes() : 0;
     const double rule_cost = tile_cost(rule, M, N, K, gated, room);
     TileChoice best = rule;
     double best_cost = rule_cost;
@@ -1526,28 +1361,89 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
     if (best_cost * 1.12 < rule_cost) { variant = best.v; ksplit = best.ks; }
   }
   int tail_split = 1;
-  {
-    const size_t room = (wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 64 == 0) ? wsp.split_bytes() : 0;
-    tile_cost(TileChoice{variant, ksplit}, M, N, K, gated, room, &tail_split);
+  tile_cost(TileChoice{variant, ksplit}, M, N, K, gated, room, &tail_split);
+  return StagedCut{variant, ksplit, tail_split};
+}
+
+// The bytes of partial sums for which the static array (strict) refuses a product of tiles that pass
+// through registers: 0, or more than the array holds.  As launch_tile has it.
+static size_t staged_sums(int M, int N, int K, bool gated, const GemmWorkspace& wsp) {
+  StagedCut c = staged_cut(M, N, K, gated, wsp.split_bytes());
+  static const int BM[4] = {128, 64, 128, 256}, BN[4] = {128, 128, 256, 256};
+  const int ncols = gated ? BN[c.variant] / 2 : BN[c.variant], round = c.variant <= 1 ? 512 : 256;
+  const int tiles = ((M + BM[c.variant] - 1) / BM[c.variant]) * ((N + ncols - 1) / ncols), tail = tiles % round;
+  const size_t tile = (size_t)BM[c.variant] * BN[c.variant] * sizeof(float);
+  while (c.ksplit > 1 && tile * tiles * c.ksplit > wsp.split_bytes()) c.ksplit--;
+  size_t need = c.ksplit > 1 ? tile * tiles * c.ksplit : 0;
+  if (c.ksplit <= 1 && c.tail_split > 1 && tail > 0 && tiles > round && tile * tail * c.tail_split <= wsp.split_bytes())
+    need = tile * tail * c.tail_split;
+  return need > wsp.bytes ? need : 0;
+}
+
+static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
+                         int M, int N, int K, int epi, float cap, int w_strip, const GemmWorkspace& wsp,
+                         int* parts, void* stream) {
+  ZK_REQUIRE(M >= 0 && N > 0 && K > 0, "zk_gemm_bf16: bad sizes");
+  ZK_REQUIRE(K % 8 == 0 && lda % 8 == 0, "zk_gemm_bf16: K and lda must be multiples of 8");
+  ZK_REQUIRE(lda >= K && ldc >= N, "zk_gemm_bf16: leading dimensions too small");
+  ZK_REQUIRE(epi >= 0 && epi <= EPI_GELU, "zk_gemm_bf16: unknown epilogue");
+  ZK_REQUIRE((epi != EPI_SOFTCAP && epi != EPI_CLAMPED) || cap > 0.f, "zk_gemm_bf16: soft cap or clamp limit must be positive");
+  ZK_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0), "zk_gemm_bf16: operands must be 16-byte aligned");
+  const bool gated = epi == EPI_GELU_TANH || epi == EPI_SILU || epi == EPI_RELU || epi == EPI_CLAMPED;
+  ZK_REQUIRE(!w_strip || (K % 32 == 0 && (!gated || N % 16 == 0)), "zk_gemm_bf16: strip layout needs K % 32 == 0 (and N % 16 == 0 when gated)");
+  if (parts) *parts = 0;
+  if (M == 0) return 0;
+  hipStream_t s = (hipStream_t)stream;
+  if (M > 16 && M <= 64 && w_strip) {
+    return gated ? launch_mid<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s)
+                 : launch_mid<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s);
   }
-  // The two wide blocks have a form that copies its operands straight into LDS (weights in the
-  // strip layout, K a whole number of tiles): 3 to 6 % less time from about 200 rows on, the
-  // same sums in the same order.  (The 128 x 128 and 64 x 128 blocks gained nothing from it
-  // where K is split and lost where it is short.)
-#define ZK_DIRECT(W_, M_, N_)                                                                                              \
-  (gated ? launch_tile<W_, M_, N_, true, true, true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, ksplit, tail_split, s) \
-         : launch_tile<W_, M_, N_, false, true, true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, ksplit, tail_split, s))
-  if (w_strip && K % GT_BK == 0 && N % 16 == 0) {
-    if (variant == 3) return ZK_DIRECT(4, 2, 4);
-    if (variant == 2) return ZK_DIRECT(2, 2, 4);
+  if (M <= 64) {
+    return gated ? launch_skinny<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s)
+                 : launch_skinny<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s);
   }
-#undef ZK_DIRECT
+  // more than 64 rows by weights in strips, K in whole stages (and offsets of a tile's rows that 31 bits hold)
+  if (w_strip && K % 64 == 0 && lda <= (1 << 22)) {
+    const bool aligned = wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 16 == 0;
+    const bool by_reader = parts != nullptr && joinable_by_reader(N, ldc, c_is_f32, epi);
+    TileCut cut = tile_cut(gated, by_reader, M, N, K, aligned ? wsp.split_bytes() : 0);
+    if (wsp.strict) {
+      // sums that the caller's array does not hold: another cut (what the array is refused for
+      // stays what it was before the tiles had other shapes)
+      if (const size_t need = staged_sums(M, N, K, gated, wsp)) return wsp.too_small(need);
+      if (max(tile_sums(gated, M, N, cut.ks), tail_sums(cut.shape, cut_tail(cut, gated, M, N), cut.tail_ks)) > wsp.bytes) cut = tile_cut(gated, by_reader, M, N, K, wsp.bytes);
+    }
+    const TileProduct p{A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap};
+    return launch_direct_shape(cut.shape, gated, p, cut.ks, cut.tail_ks, (float*)wsp.ptr, parts, s);
+  }
+  const bool exact = K % GT_BK == 0;
+  const size_t room = (wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 64 == 0) ? wsp.split_bytes() : 0;
+  const StagedCut cut = staged_cut(M, N, K, gated, room);
+  const int variant = cut.variant, ksplit = cut.ksplit, tail_split = cut.tail_split;
+#define ZK_TILE_(W_, M_, N_, G_, E_) \
+  launch_tile<W_, M_, N_, G_, E_>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, ksplit, tail_split, s)
+#define ZK_TILE(W_, M_, N_)                                                                            \
+  (gated ? (exact ? ZK_TILE_(W_, M_, N_, true, true) : ZK_TILE_(W_, M_, N_, true, false))             \
+         : (exact ? ZK_TILE_(W_, M_, N_, false, true) : ZK_TILE_(W_, M_, N_, false, false)))
   if (variant == 3) return gated ? ZK_TILE_(2, 4, 4, true, true) : ZK_TILE_(2, 4, 4, false, true);
   if (variant == 2) return ZK_TILE(2, 2, 4);
   if (variant == 1) return ZK_TILE(1, 2, 2);
   return ZK_TILE(2, 2, 2);
 #undef ZK_TILE
 #undef ZK_TILE_
+}
+
+// Which tile (its number in tile_shapes) and how many ranges of K, of the last round's tiles alone, a product
+// of more than 64 rows by weights in strips, K a multiple of 64, takes with the standard workspace
+// (``by_reader``: the caller passes ``parts``).  For tests that mean to reach each of them.
+extern "C" int zk_gemm_bf16_tile_cut(int gated, int by_reader, int M, int N, int K, int* shape, int* ks,
+                                     int* tail_ks) {
+  ZK_REQUIRE(M > 64 && N > 0 && K > 0 && K % 64 == 0, "zk_gemm_bf16_tile_cut: no tile product of this size");
+  const TileCut c = tile_cut(gated != 0, by_reader != 0, M, N, K, ZK_GEMM_WORKSPACE_BYTES);
+  *shape = c.shape;
+  *ks = c.ks;
+  *tail_ks = c.tail_ks;
+  return 0;
 }
 
 extern "C" int zk_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
