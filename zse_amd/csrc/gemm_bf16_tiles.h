@@ -70,8 +70,8 @@ __device__ __forceinline__ void interleave() {
 //
 // LDS: W's strips lie as in memory, 1 KB for 32 k: [k piece of 8][row 16][8 values]; an operand
 // read (row lane % 32, k piece lane / 32) takes whole 256-byte runs.  A: a copy takes 8 rows x
-// 64 k, eight lanes a row; lane c of a row fetches k piece c ^ (row % 8), so the eight rows that a
-// read takes at once lie in different banks.
+// 64 k, eight lanes a row; lane c of a row fetches k piece c ^ (row / 2 % 8), so that of the sixteen
+// rows that a read takes at once no two lie in the same banks.
 //
 // The products are taken as W tile x A tile^T: a lane holds, of row lane % 32 of a square, the
 // columns 8 b + 4 (lane / 32) + e.  GATED: the first TN / 2 squares of a wave are gate columns,
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
   for (int c = 0; c < LPA; c++) {
     const int piece = min(wave + c * NW, CA - 1), row = piece * 8 + (lane >> 3);
     la[c] = piece * 1024;
-    va[c] = (min(m0 + row, M - 1) - m0) * lda * 2 + (((lane & 7) ^ (row & 7)) * 16);
+    va[c] = (min(m0 + row, M - 1) - m0) * lda * 2 + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
   }
 #pragma unroll
   for (int c = 0; c < LPB; c++) {
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
   };
   int a_at[4];
 #pragma unroll
-  for (int q = 0; q < 4; q++) a_at[q] = (wm * (32 * TM) + lr) * 128 + (((q * 2 + lk) ^ (lr & 7)) * 16);
+  for (int q = 0; q < 4; q++) a_at[q] = (wm * (32 * TM) + lr) * 128 + (((q * 2 + lk) ^ ((lr >> 1) & 7)) * 16);
   const int w_at = WBASE + (wn * (GATED ? TN / 2 : TN) * 2 + (lr >> 4)) * 2048 + lk * 256 + (lr & 15) * 16;
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -176,7 +176,9 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
 #pragma unroll
   for (int t = 1 - NSB; t < 0; t++) {
     if (t + NSA - 1 >= 0) copy_a((t + NSA - 1) * SA, t + NSA - 1);
+    __builtin_amdgcn_sched_barrier(0);          // the wait below counts on this order
     copy_w((t + NSB - 1) * SB, t + NSB - 1);
+    __builtin_amdgcn_sched_barrier(0);
   }
   // (the barrier as text: before one it knows, the compiler waits for every load in flight)
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LEFT) : "memory");
