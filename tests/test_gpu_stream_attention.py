@@ -1,0 +1,98 @@
+"""Portions of heads of 128 and 256 channels whose tiles are copied ahead, without and with ranges of keys, against a
+plain implementation in 64 bits: last blocks of a few rows (waves with no rows among them), heads that do not fill
+a wave's 32 rows, pages of 16 to 64 keys, windows with kept first keys, scores whose maximum rises with every
+tile, and the choice by sizes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    from zse_amd.runtime.device import Runtime
+    return Runtime.get()
+
+
+def rounded(x):
+    from zse_amd.weights.safetensors import bf16_bits_to_f32, f32_to_bf16_bits
+    return bf16_bits_to_f32(f32_to_bf16_bits(np.ascontiguousarray(x, np.float32)))
+
+
+def up(rt, x):
+    from zse_amd.weights.safetensors import f32_to_bf16_bits
+    return rt.upload(f32_to_bf16_bits(np.ascontiguousarray(x, np.float32)), "bfloat16")
+
+
+def plain(q, k, v, before, scale, cap, window, keep):
+    """q [n, H, D] behind ``before`` keys of k [ctx, G, D], v [ctx, G, E]."""
+    n, H, _ = q.shape
+    pos, key = before + np.arange(n)[:, None], np.arange(len(k))[None]
+    ok = (key <= pos) & ((key > pos - window) | (key < keep) if window else True)
+    out = np.zeros((n, H, v.shape[2]))
+    for h in range(H):
+        g = h // (H // k.shape[1])
+        s = q[:, h] @ k[:, g].T * scale
+        s = np.where(ok, cap * np.tanh(s / cap) if cap else s, -np.inf)
+        w = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = w / w.sum(1, keepdims=True) @ v[:, g]
+    return out
+
+
+CASES = [
+    # heads, key heads, key and value channels, page, (cached, new) of each request, window, kept, cap, rising
+    (8, 4, 256, 256, 16, [(0, 64), (37, 300)], 0, 0, 50.0, False),
+    (2, 2, 256, 256, 16, [(0, 1500)], 0, 0, 50.0, False),                  # a last block of one wave with rows
+    (6, 2, 256, 256, 32, [(5, 97), (130, 333)], 130, 0, 0.0, False),       # 30 of a wave's 32 rows
+    (4, 2, 256, 256, 64, [(700, 161)], 300, 40, 20.0, False),
+    (4, 4, 256, 256, 16, [(0, 260)], 0, 0, 0.0, True),
+    (8, 2, 128, 128, 16, [(0, 33), (1, 31), (900, 129)], 0, 0, 0.0, False),
+    (10, 2, 128, 128, 32, [(64, 200)], 90, 7, 30.0, False),
+    (4, 1, 128, 128, 16, [(300, 520)], 0, 0, 0.0, True),
+    (16, 1, 128, 128, 64, [(3, 70)], 1, 0, 50.0, False),
+    (4, 2, 256, 128, 16, [(40, 150)], 0, 0, 50.0, False),
+    (4, 2, 128, 256, 32, [(40, 150)], 77, 33, 0.0, False),
+]
+
+
+@pytest.mark.parametrize("mode", [0, 4, 5])           # by the sizes, four groups a block, with ranges
+@pytest.mark.parametrize("case", CASES)
+def test_portions(rt, case, mode):
+    H, G, D, E, bs, reqs, window, keep, cap, rising = case
+    kern = rt.kernels("bfloat16")
+    rng = np.random.default_rng(D + E + len(reqs) + window)
+    R, ctx, fresh = len(reqs), [a + b for a, b in reqs], [b for _, b in reqs]
+    blocks = -(-max(ctx) // bs)
+    pages = 1 + R * blocks
+    table = (1 + rng.permutation(R * blocks)).astype(np.int32).reshape(R, blocks)
+    kc, vc = np.zeros((pages, G, bs, D), np.float32), np.zeros((pages, G, E, bs), np.float32)
+    q = rounded(rng.normal(size=(sum(fresh), H, D)))
+    starts = np.concatenate([[0], np.cumsum(fresh)]).astype(np.int32)
+    want = []
+    for r in range(R):
+        kk, vv = rng.normal(size=(ctx[r], G, D)), rounded(rng.normal(size=(ctx[r], G, E)))
+        mine = q[starts[r]:starts[r + 1]]
+        if rising:           # the n-th key agrees with every query the better the later it comes: about 60 maxima on the way
+            q[starts[r]:starts[r + 1], :, 0] = 4.0
+            kk[:, :, 0] = np.linspace(-40, 40, ctx[r])[:, None] * D ** 0.5 / 4
+        kk = rounded(kk)
+        for p in range(ctx[r]):
+            kc[table[r, p // bs], :, p % bs], vc[table[r, p // bs], :, :, p % bs] = kk[p], vv[p]
+        table[r, -(-ctx[r] // bs):] = -1
+        want.append(plain(mine.astype(np.float64), kk.astype(np.float64), vv.astype(np.float64), reqs[r][0], D ** -0.5, cap, window, keep))
+    want = np.concatenate(want)
+    out = rt.zeros((len(q), H * E), "bfloat16")
+    ws = rt.zeros((int(kern.zk_attention_bf16_portion_workspace(R * (max(fresh) + 128), H, G, E)) // 4 + 64,), "float32")
+    args = [up(rt, q.reshape(len(q), -1)), up(rt, kc), up(rt, vc), rt.upload(table, "int32"), rt.upload(starts, "int32"),
+            rt.upload(np.array(ctx, np.int32), "int32")]
+    before = kern.zk_attention_bf16_portion_kernel(mode)
+    try:
+        kern.zk_attention_bf16_sized(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, blocks, args[4].ptr, args[5].ptr,
+                                     out.ptr, R, R, max(fresh), max(ctx), H, G, D, bs, D ** -0.5, cap, window, 0, ws.ptr, ws.nbytes,
+                                     0, 0, 0, 0, E, keep, rt.stream)
+        got = rt.download_f32(out).reshape(want.shape)
+    finally:
+        kern.zk_attention_bf16_portion_kernel(before)
+    # weights and results rounded to 8 bits of mantissa; values of size 1, the largest about 4.5
+    assert np.abs(got - want).max() < 0.03, np.unravel_index(np.abs(got - want).argmax(), got.shape)
+    assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)

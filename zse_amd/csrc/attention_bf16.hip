@@ -233,6 +233,60 @@ static int portion_ranges(int max_q_len, int max_ctx, int window, int mask_chunk
   return best;
 }
 
+// Heads of 128 and 256 channels on attn_stream_kernel: a group a block (0), four groups a block (4) or the
+// latter with the keys in ranges of ``ranges`` tiles (5), by the least of three prices in microseconds.  A
+// block costs a start and a time a tile; blocks beyond one a CU (two for 128 channels) take their
+// share of the CUs' time, the last ones half of the shortest block's more; ranges add a block's partial
+// results and the joining launch.  The constants are fitted to launches of 300 to 4,000 rows behind up to
+// 4,096 keys, 2 to 16 key heads, one and three requests (us; group, four, ranges, taken): 8 heads over 4 of 256, 512 rows at 512
+// keys 25, 28, 23, ranges; behind 3,584 112, 145, 43, ranges; 4,000 rows 241, 142, 178, four; three
+// times 1,000 98, 45, -, four; 16 over 8, 3,000 rows 287, 117, 139, four; 32 over 16 of 128, 512 rows at 512 keys
+// 16, 22, 26, group; 2,048 rows 169, 70, 95, four.
+struct PortionPlan { int kind, ranges; };      // ranges: the best cut with ranges, taken or not (0: none)
+static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int tpw, int nkv, int r_prefill,
+                                int bound_tiles, int wide) {
+  const bool narrow = wide <= 128;
+  const int slots = narrow ? 512 : 256, per_block = 4 * tpw, row_blocks = (max_q_len + per_block - 1) / per_block;
+  const long copies = (long)nkv * r_prefill;
+  const double start_group = narrow ? 8.7 : 11.6, tile_group = narrow ? 0.64 : 0.77;
+  const double start_four = narrow ? 6.6 : 11.0, tile_four = narrow ? 0.83 : 1.06;
+  auto tiles_of = [&](int bi) {
+    const int lo = max_ctx - max_q_len + bi * per_block, hi = std::min(max_ctx, lo + per_block) - 1;
+    const int klo = mask_chunk > 0 ? lo - lo % mask_chunk : window > 0 ? std::max(0, lo - window + 1) : 0;
+    return std::min((keep + 31) / 32, klo / 32) + hi / 32 - klo / 32 + 1;
+  };
+  int longest = 0, shortest = 1 << 30;
+  double sum = 0;
+  for (int bi = 0; bi < row_blocks; bi++) {
+    const int t = tiles_of(bi);
+    longest = std::max(longest, t);
+    shortest = std::min(shortest, t);
+    sum += t;
+  }
+  auto price = [&](double blocks, double start, double per_tile, double tiles, int most, int least) {
+    const double alone = start + per_tile * most;
+    if (blocks <= slots) return alone;
+    return std::max(alone, (blocks * start + per_tile * tiles) / slots + 0.5 * (start + per_tile * least));
+  };
+  PortionPlan best{0, 0};
+  const double groups = (max_q_len + tpw - 1) / tpw;
+  double best_price = price(groups * copies, start_group, tile_group, sum * copies * groups / row_blocks, longest, shortest);
+  const double four = price((double)row_blocks * copies, start_four, tile_four, sum * copies, longest, shortest);
+  if (four < best_price) best = {4, 0}, best_price = four;
+  double best_ranges = 1e30;
+  static const int cands[] = {64, 48, 40, 32, 24, 16, 12, 10, 8, 6, 4};
+  for (int ct : cands) {
+    if (2 * ct > longest || (bound_tiles + ct - 1) / ct > ATT_MOST_RANGES) continue;
+    double blocks = 0;
+    for (int bi = 0; bi < row_blocks; bi++) blocks += (tiles_of(bi) + ct - 1) / ct;
+    blocks *= copies;
+    const double t = price(blocks, start_four, tile_four, sum * copies, ct, std::min(shortest, ct)) + blocks * wide * (0.035 / 256) + 4.0;
+    if (t < best_ranges) best.ranges = ct, best_ranges = t;
+  }
+  if (best_ranges < best_price) best.kind = 5;
+  return best;
+}
+
 // 0: the portion kernel is chosen by the sizes; 1: a group of rows a block; 4, 8: shared
 // tiles with that many waves a block; 5: shared tiles, four waves, the keys in ranges (as far as
 // the workspace allows).  For tests and measurements (process-wide).
@@ -380,8 +434,9 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
     // 8 heads of 256, 512 groups: 75 us against 111; 768 groups: a tie), with more the shared
     // tiles are (8 portions of 512 rows behind 7,680 tokens, 32 heads of 128: 1,630 -> 780 us;
     // 16 heads of 256: 1,560 -> 845 us; 8,192 rows of 8 heads of 256: 877 -> 463 us).
+    const bool stream = stream_takes(hd, vd, bs, wide_weights);
     int shared_waves = 0;
-    if (bs >= 8 && portion_kernel_mode != 1) {
+    if (bs >= 8 && portion_kernel_mode != 1 && !(stream && portion_kernel_mode == 0)) {
       if (portion_kernel_mode > 1) shared_waves = portion_kernel_mode;
       else if (single >= 4096 && wide <= 128) shared_waves = 8;
       else if (single >= 768) shared_waves = 4;
@@ -402,7 +457,13 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
       // (a chunk's rows see no more keys than a window of its size would show them)
       const int reach = mask_chunk > 0 ? mask_chunk : window;
       if (reach > 0) bound = std::min(bound, (reach + per_block + 31) / 32 + 1 + (keep + 31) / 32);
-      range_tiles = portion_ranges(max_q_len, max_ctx, window, mask_chunk, keep, per_block, nkv, r_prefill, bound);
+      if (stream) {
+        const PortionPlan plan = portion_plan(max_q_len, max_ctx, window, mask_chunk, keep, p.tpw, nkv, r_prefill, bound, wide);
+        if (portion_kernel_mode == 5 || plan.kind == 5) range_tiles = plan.ranges;
+        if (plan.kind) shared_waves = std::max(shared_waves, 4);           // also where the workspace does not hold the ranges
+      } else {
+        range_tiles = portion_ranges(max_q_len, max_ctx, window, mask_chunk, keep, per_block, nkv, r_prefill, bound);
+      }
       if (range_tiles) {
         most_ranges = (bound + range_tiles - 1) / range_tiles;
         if (R - r_prefill > 0) split_at = (zk_attention_bf16_workspace(R - r_prefill, nh, vd, max_ctx) + 255) / 256 * 256;

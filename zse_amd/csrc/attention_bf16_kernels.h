@@ -748,6 +748,384 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
     }
 }
 
+// The order of a quarter of a turn of attn_stream_kernel: a product, two LDS reads for the next
+// quarter, a few vector operations; in the second half no more reads, so that the last have arrived when
+// the next quarter begins.
+template <int MFMAS, int VALUS>
+__device__ __forceinline__ void stream_order() {
+#pragma unroll
+  for (int i = 0; i < MFMAS; i++) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+    if (i < MFMAS / 2) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, VALUS, 0);
+  }
+}
+
+// Long portions, heads of 128 and 256 channels: attn_shared_kernel's division of the work (four waves of
+// 32 rows, the same tiles of 32 keys, the same results) with the keys and values on their way
+// for several tiles, and three tiles in work at a time.
+//
+// What bounded the other: a turn asked for the next tile and waited for it at its end, so a tile
+// took a trip to memory (2.4 to 2.7 us at 256 channels, of which its products are 0.5), and a wave's scores,
+// weights and second product followed each other, one wave a SIMD.  Here tiles are copied into
+// LDS without passing through registers, keys up to four tiles ahead and values three; and a turn t multiplies tile
+// t + 1 by the queries and tile t - 1's weights by its values while the vector unit turns tile t's scores into
+// weights.  The page table is read 64 entries at a time into a register.
+//
+// LDS, a ring of four tiles each.  K: a key's row of HD channels; place p of 16 bytes of row r holds
+// piece p ^ (r % 16), so that sixteen rows read at once lie in different banks.  V: [16 keys][channel][the 16 keys' values], the two
+// pieces of a channel swapped where its number has bit 3, for the same reason; pages of 16 keys or more, so that a copy
+// is one run of such a page.
+// Row 8 j + 4 a + i of a score tile is key 16 (j / 2) + 8 a + 4 (j % 2) + i, so that a lane's eight weights of a
+// half tile belong to eight neighbouring keys: 16 bytes of a channel of the transposed values.
+//
+// A masked score is set to the score's least value before the turn and its weight to zero after it; only tiles at an edge
+// have any.  Tiles past the range are copied (from the table's last entries) and multiplied, never weighted.
+template <int HD16, int VD16, bool SPLIT, bool CAPPED>
+__global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_stream_kernel(AttnParams p) {
+  // (the host's pass knows no address spaces)
+#ifdef __HIP_DEVICE_COMPILE__
+  constexpr int HD = HD16 * 16, VD = VD16 * 16, DT = VD16 / 2, NW = 4, RING = 4;
+  constexpr int KT = 32 * HD * 2, VT = 32 * VD * 2;     // bytes of a tile
+  constexpr int KPI = 512 / HD;                         // keys of a copy (1 KB of K)
+  constexpr int KW = 8 / KPI, VW = VD / 64;             // copies of a tile a wave issues
+  static_assert(HD >= 128 && VD >= 128, "copies of at most four keys");
+  extern __shared__ __attribute__((aligned(16))) unsigned char stream_lds[];
+  unsigned char* const sV = stream_lds + RING * KT;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, lk = lane >> 5;
+  const int r = p.r_begin + blockIdx.z;
+  int block_x, kvh;
+  portion_block(block_x, kvh);
+  const int qs = p.q_start[r], n = p.q_start[r + 1] - qs;
+  if (n <= 0) return;
+  const int start = p.ctx_len[r] - n;
+  const int per_block = NW * p.tpw;
+  // the last rows of a portion see the most keys and go first
+  const int rows_x = SPLIT ? block_x / p.nchunks : block_x;
+  const int range = SPLIT ? block_x - rows_x * p.nchunks : 0;
+  const int bi = (n + per_block - 1) / per_block - 1 - rows_x;
+  if (bi < 0) return;
+  const int g = p.nh / p.nkv;
+  const int blk_lo = start + bi * per_block, blk_hi = start + min(n, (bi + 1) * per_block) - 1;
+  const KeyTiles ts(p, first_key(p, blk_lo), blk_hi);
+  int tile_0 = 0, tile_end = ts.count;
+  if (SPLIT) {
+    tile_0 = range * p.chunk;
+    if (tile_0 >= ts.count) return;                    // the block of rows has fewer ranges
+    tile_end = min(ts.count, tile_0 + p.chunk);
+  }
+  const int turns = tile_end - tile_0;
+  // the wave's rows
+  const int t0 = bi * per_block + wave * p.tpw;
+  const int ntok = max(0, min(p.tpw, n - t0));
+  const int tok = lr / g, hq = lr - tok * g;
+  const bool row_ok = tok < ntok;
+  const int trow = qs + (row_ok ? t0 + tok : 0);
+  const int pos = start + (row_ok ? t0 + tok : 0);
+  const int head = q_head_of(p, kvh, row_ok ? hq : 0);
+  // keys [all_lo, all_hi] are seen by every row of the wave.  (What becomes of rows that are not there does not matter; if
+  // they made every tile of their wave one to mask, a last block of a few rows, which has the most keys, took 1.5 times as
+  // long: 1,500 rows of 8 heads of 256, no ranges, 92 us against 62.)
+  const int row_lo = first_key(p, pos);
+  const int all_hi = ntok > 0 ? start + t0 : 0x7fffff00;
+  const int all_lo = ntok > 0 ? first_key(p, start + t0 + ntok - 1) : 0;
+  const int* table = p.block_table + (size_t)r * p.max_blocks;
+  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, last_entry = p.max_blocks - 1;
+
+  // bytes of a page, and what lies before the key head's part of it
+  const unsigned k_page = (unsigned)(nkv * HD * 2) << bsh, v_page = (unsigned)((nkv >> p.v_shift) * VD * 2) << bsh;
+  const unsigned char* const k_base = (const unsigned char*)p.kcache + ((size_t)kvh * HD * 2 << bsh);
+  const unsigned char* const v_base = (const unsigned char*)p.vcache + ((size_t)(kvh >> p.v_shift) * VD * 2 << bsh);
+  // the places of 64 pages, from entry ``first`` of the table on, one a lane; a tile lies in at most two (of 16 keys)
+  struct Pages { unsigned lo, hi; int first; };
+  auto cover = [&](Pages& e, int key0, const unsigned char* base, unsigned page_bytes) __attribute__((always_inline)) {
+    const int first = key0 >> bsh;
+    if ((unsigned)(first - e.first) > 60u) {
+      e.first = first;
+      const uint64_t at = (uint64_t)base + (uint64_t)(unsigned)max(table[min(first + lane, last_entry)], 0) * page_bytes;
+      e.lo = (unsigned)at;
+      e.hi = (unsigned)(at >> 32);
+      asm volatile("" : "+v"(e.lo), "+v"(e.hi));        // arrived here, so that no turn waits for loads
+    }
+  };
+  // Copies: K copy c = wave + 4 j is keys KPI c .. of the tile, V copy c 32 channels of the tile's first or last 16 keys.
+  // Per copy: its page counted from the tile's first, and a lane's place behind the page's begin (tiles begin at
+  // multiples of 32 keys: with pages of up to 32 keys the place does not depend on the tile, with larger ones a tile
+  // adds the same for all).
+  unsigned k_off[KW], v_off[VW];
+  int k_idx[KW], v_idx[VW];
+#pragma unroll
+  for (int j = 0; j < KW; j++) {
+    const int key = (wave + 4 * j) * KPI, row = key + lane / (64 / KPI);
+    k_idx[j] = key >> bsh;
+    k_off[j] = (unsigned)((row & bmask) * HD + ((lane % (64 / KPI)) ^ (row & 15)) * 8) * 2;
+  }
+#pragma unroll
+  for (int j = 0; j < VW; j++) {
+    const int copy = wave + 4 * j, half = copy / (VD / 32), d = copy % (VD / 32) * 32 + lane / 2;
+    const int key = 16 * half + 8 * ((lane & 1) ^ (d >> 3 & 1));
+    v_idx[j] = 16 * half >> bsh;
+    v_off[j] = (unsigned)((d << bsh) + (key & bmask)) * 2;
+  }
+  typedef const __attribute__((address_space(1))) void* from_t;
+  typedef __attribute__((address_space(3))) void* to_t;
+  auto place = [&](const Pages& e, int entry, unsigned off) __attribute__((always_inline)) {
+    const uint64_t page = (uint64_t)(unsigned)__builtin_amdgcn_readlane(e.hi, entry) << 32 | (unsigned)__builtin_amdgcn_readlane(e.lo, entry);
+    return (from_t)((const unsigned char*)page + off);
+  };
+  auto copy_k = [&](int slot, int key0, const Pages& e) __attribute__((always_inline)) {
+    const int first = (key0 >> bsh) - e.first;
+    const unsigned in_page = (unsigned)(key0 & bmask) * (HD * 2);
+#pragma unroll
+    for (int j = 0; j < KW; j++)
+      __builtin_amdgcn_global_load_lds(place(e, first + k_idx[j], k_off[j] + in_page),
+                                       (to_t)(stream_lds + slot * KT + (wave + 4 * j) * 1024), 16, 0, 0);
+  };
+  auto copy_v = [&](int slot, int key0, const Pages& e) __attribute__((always_inline)) {
+    const int first = (key0 >> bsh) - e.first;
+    const unsigned in_page = (unsigned)(key0 & bmask) * 2;
+#pragma unroll
+    for (int j = 0; j < VW; j++)
+      __builtin_amdgcn_global_load_lds(place(e, first + v_idx[j], v_off[j] + in_page),
+                                       (to_t)(sV + slot * VT + (wave + 4 * j) * 1024), 16, 0, 0);
+  };
+
+  // (a row that is not there reads another's queries; its scores are masked)
+  bf16x8 qf[HD16];
+  {
+    const __bf16* qr = p.q + (size_t)trow * p.q_stride + (size_t)head * HD + lk * 8;
+#pragma unroll
+    for (int ks = 0; ks < HD16; ks++) qf[ks] = *(const bf16x8*)(qr + ks * 16);
+  }
+  // the values of "tile -1", whose weights are zero, must not be NaN
+#pragma unroll
+  for (int i = 0; i < VT / 4096; i++) *(f32x4*)(sV + (RING - 1) * VT + (i * 256 + tid) * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
+  Pages ek{0, 0, -1000}, ev{0, 0, -1000};
+  auto key_of = [&](int t) { return ts.key_of(tile_0 + t); };
+  // the copies that turns -4 to -1 would issue (keys of tiles 0 to 3, values of 0 and 1; the waits count on their order)
+#pragma unroll 1
+  for (int t = -4; t < 0; t++) {
+    cover(ek, key_of(t + 4), k_base, k_page);
+    copy_k(t + 4, key_of(t + 4), ek);
+    if (t >= -2) {
+      cover(ev, key_of(t + 2), v_base, v_page);
+      copy_v(t + 2, key_of(t + 2), ev);
+    }
+  }
+  // a lane's weights of a half tile: two a register
+  union Weights { bf16x8 v[2]; int w[8]; };
+  Weights pb;
+#pragma unroll
+  for (int e = 0; e < 8; e++) pb.w[e] = 0;
+  f32x16 zero;
+#pragma unroll
+  for (int e = 0; e < 16; e++) zero[e] = 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)       // zeros, in 8 bytes of code instead of 128
+    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pb.v[0], pb.v[0], zero, 0, 0, 0);
+  float m_run = -INFINITY, l_run = 0.f;
+  // where a lane reads: its score row's key and the pieces of its half
+  const int key_row = 16 * (lr >> 4) + 8 * ((lr >> 2) & 1) + 4 * ((lr >> 3) & 1) + (lr & 3);
+  int k_at8[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ks++) k_at8[ks] = key_row * HD * 2 + (((ks * 2 + lk) ^ (key_row & 15)) * 16);
+  auto k_at = [&](int ks) { return k_at8[ks & 7] + (ks >> 3) * 256; };
+  const int v_at = lr * 32 + (lk ^ (lr >> 3 & 1)) * 16;
+  // A wait for all but the copies of the last two turns, and a meeting (as text: before a barrier it knows the
+  // compiler waits for every load in flight).  The copies of turn t go to the places that turn t - 1 read
+  // before its meeting.
+#define ZK_STREAM_MEET() asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * (KW + VW)) : "memory")
+  ZK_STREAM_MEET();
+  f32x16 s = zero;
+#pragma unroll
+  for (int ks = 0; ks < HD16; ks++)
+    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(stream_lds + k_at(ks)), qf[ks], s, 0, 0, 0);
+  ZK_STREAM_MEET();                             // every wave has read tile 0, whose place turn 0 writes to
+  // What the products so far are multiplied by once a larger maximum was met, right before the next ones
+  // (at the end of a turn the branch made the compiler copy all accumulators out and back): in the
+  // accumulation registers, where the products keep them.
+  float corr = 1.f;
+  auto rescale = [&]() __attribute__((always_inline)) {
+    if (__builtin_expect(__any(corr != 1.f), 0)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+          float x;
+          asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 0\n\tv_accvgpr_write_b32 %0, %1"
+                       : "+a"(o[dt][e]), "=&v"(x)
+                       : "v"(corr));
+        }
+    }
+  };
+  const float k = CAPPED ? p.k2 : p.k1, c2 = p.c2;
+  const float least = k > 0.f ? -INFINITY : k < 0.f ? INFINITY : 0.f;      // times k: the least score
+  // A turn goes in quarters: each multiplies the operands that the one before it has read, and turns a part of
+  // the scores.  The waves meet before the last quarter, which reads for the next turn's first.
+  constexpr int SB = HD16 / 4, PB = VD16 / 4;
+  bf16x8 kf[2][SB], vf[2][PB];
+  auto read = [&](int t, int b) __attribute__((always_inline)) {
+    const unsigned char* kb = stream_lds + ((t + 1) & 3) * KT;
+    const unsigned char* vb = sV + ((t + 3) & 3) * VT + v_at;
+#pragma unroll
+    for (int i = 0; i < SB; i++) kf[b & 1][i] = *(const bf16x8*)(kb + k_at(b * SB + i));
+#pragma unroll
+    for (int i = 0; i < PB; i++) {
+      const int x = b * PB + i;
+      vf[b & 1][i] = *(const bf16x8*)(vb + (x / DT) * VD * 32 + (x % DT) * 1024);
+    }
+  };
+  read(0, 0);
+  for (int t = 0; t < turns; t++) {
+    const int key0 = key_of(t);
+    const bool edge = key0 < all_lo || key0 + 31 > all_hi;
+    unsigned seen = 0xffffu;
+    if (edge) {
+      seen = 0;
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int key = key0 + 16 * (e >> 3) + 8 * lk + (e & 7);
+        const bool ok = row_ok && (key >= row_lo || key < p.keep) && key <= pos;
+        seen |= (unsigned)ok << e;
+        s[e] = ok ? s[e] : least;
+      }
+    }
+    cover(ek, key_of(t + 4), k_base, k_page);
+    cover(ev, key_of(t + 2), v_base, v_page);
+    rescale();
+    f32x16 next;
+    auto multiply = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < (SB > PB ? SB : PB); i++) {
+        if (i < SB) {
+          next = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[b & 1][i], qf[b * SB + i], b == 0 && i == 0 ? zero : next, 0, 0, 0);
+        }
+        if (i < PB) {
+          const int x = b * PB + i;
+          o[x % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[b & 1][i], pb.v[x / DT], o[x % DT], 0, 0, 0);
+        }
+      }
+    };
+    // Scores into weights.  Capped: c2 tanh = c2 - 2 c2 r with r = 1 / (2^(k2 dot) + 1), so the largest
+    // score has the least r.
+    float best = CAPPED ? INFINITY : -INFINITY;
+    auto scores = [&](int from) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = from; e < from + 8; e++) {
+        if (CAPPED) {
+          s[e] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(k * s[e]) + 1.f);
+          best = fminf(best, s[e]);
+        } else {
+          s[e] *= k;
+          best = fmaxf(best, s[e]);
+        }
+      }
+    };
+    float rs = 0.f, off;
+    Weights pn;
+    auto weights = [&](int from) __attribute__((always_inline)) {
+      bf16x8 w;
+#pragma unroll
+      for (int e = from; e < from + 8; e++) {
+        s[e] = __builtin_amdgcn_exp2f(CAPPED ? fmaf(s[e], -2.f * c2, off) : s[e] + off);
+        rs += s[e];
+        w[e - from] = (__bf16)s[e];
+      }
+      pn.v[from / 8] = w;
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    read(t, 1);
+    copy_k(t & 3, key_of(t + 4), ek);
+    scores(0);
+    stream_order<SB + PB, CAPPED ? 5 : 2>();
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    read(t, 2);
+    copy_v((t + 2) & 3, key_of(t + 2), ev);
+    scores(8);
+    stream_order<SB + PB, CAPPED ? 5 : 2>();
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(2);
+    read(t, 3);
+    {
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_int(best), __float_as_int(best), false, false);
+      const float a = __int_as_float(both[0]), b = __int_as_float(both[1]);
+      best = CAPPED ? fminf(a, b) : fmaxf(a, b);
+    }
+    const float mt = CAPPED ? fmaf(best, -2.f * c2, c2) : best;
+    const float m_new = mt > m_run + 8.f ? mt : m_run;      // the maximum is followed lazily
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;
+    corr = m_new > m_run && m_run > -INFINITY ? __builtin_amdgcn_exp2f(m_run - m_use) : 1.f;     // (nothing to correct yet)
+    off = CAPPED ? c2 - m_use : -m_use;
+    weights(0);
+    stream_order<SB + PB, 5>();
+    __builtin_amdgcn_sched_barrier(0);
+    ZK_STREAM_MEET();
+    multiply(3);
+    read(t + 1, 0);
+    weights(8);
+    stream_order<SB + PB, 4>();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+v"(rs), "+v"(pn.w[0]), "+v"(pn.w[1]), "+v"(pn.w[2]), "+v"(pn.w[3]), "+v"(pn.w[4]), "+v"(pn.w[5]),
+                 "+v"(pn.w[6]), "+v"(pn.w[7]));      // here, not on the way without an edge
+    if (edge) {
+      rs = 0.f;
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const bool ok = seen >> e & 1;
+        rs += ok ? s[e] : 0.f;
+        pn.w[e >> 1] = ok ? pn.w[e >> 1] : pn.w[e >> 1] & (e & 1 ? 0xffff : 0xffff0000);
+      }
+    }
+    {
+      const auto both = __builtin_amdgcn_permlane32_swap(__float_as_int(rs), __float_as_int(rs), false, false);
+      rs = __int_as_float(both[0]) + __int_as_float(both[1]);
+    }
+    l_run = l_run * corr + rs;
+    m_run = m_new;
+    pb = pn;
+    s = next;
+  }
+  rescale();
+  {
+    const unsigned char* vb = sV + ((turns + 3) & 3) * VT + v_at;
+#pragma unroll
+    for (int x = 0; x < 2 * DT; x++)
+      o[x % DT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(vb + (x / DT) * VD * 32 + (x % DT) * 1024),
+                                                          pb.v[x / DT], o[x % DT], 0, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no copy is on its way into LDS when the block ends
+#undef ZK_STREAM_MEET
+  if (SPLIT) {
+    // a wave's results of its range, as in attn_shared_kernel
+    const size_t slot = ((((size_t)blockIdx.z * p.nkv + kvh) * (gridDim.x / p.nchunks) + rows_x) * p.nchunks + range) * NW + wave;
+    p.part_ml[slot * 128 + lane] = lk == 0 ? m_run : l_run;
+    f32x4* po = (f32x4*)p.part_o + slot * (DT * 4 * 64) + lane;
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        po[(dt * 4 + j) * 64] = f32x4{o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]};
+    return;
+  }
+  if (!row_ok) return;
+  const float inv = row_factor(p, trow, head, l_run, m_run);
+  __bf16* orow = p.out + ((size_t)trow * p.nh + head) * VD;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      bf16x4 w;
+#pragma unroll
+      for (int i = 0; i < 4; i++) w[i] = (__bf16)(o[dt][4 * j + i] * inv);
+      *(bf16x4*)(orow + dt * 32 + 8 * j + 4 * lk) = w;
+    }
+#endif
+}
+
 // Which of a (request, key head)'s blocks a block is.  Blocks go in turn to the 8 XCDs and there to the
 // shader engines, 32 in all, so with an even number of them a request the first blocks of all requests
 // would share a few and the last ones the others: with requests of uneven lengths, whose last blocks have
@@ -1177,6 +1555,25 @@ static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
   return zk_launch_status("zk_attention_bf16 (shared tiles)");
 }
 
+// What attn_stream_kernel takes of the launches of four groups a block.
+static inline bool stream_takes(int hd, int vd, int bs, int wide_weights) {
+  return (hd == 128 || hd == 256) && (vd == 128 || vd == 256) && bs >= 16 && !wide_weights;
+}
+
+template <int HD16, int VD16, bool SPLIT>
+static int launch_stream(const AttnParams& p, dim3 grid, hipStream_t s) {
+  constexpr size_t lds = (size_t)4 * 32 * (HD16 + VD16) * 16 * sizeof(__bf16);
+  const auto kernel = p.softcap > 0.f ? attn_stream_kernel<HD16, VD16, SPLIT, true> : attn_stream_kernel<HD16, VD16, SPLIT, false>;
+  static std::atomic<bool> prepared[2];
+  if (lds > 64 * 1024 && !prepared[p.softcap > 0.f]) {
+    if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+      return zk_fail("zk_attention_bf16: the stream kernel's LDS was refused");
+    prepared[p.softcap > 0.f] = true;
+  }
+  kernel<<<grid, 256, lds, s>>>(p);
+  return zk_launch_status("zk_attention_bf16 (tiles copied ahead)");
+}
+
 // the maxima and sums, and the results, of the four waves of a block of 256 keys
 static inline size_t decode_long_lds(int g, int vd) { return (4 * 16 * 2 + (size_t)4 * g * vd) * sizeof(float); }
 
@@ -1188,11 +1585,17 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
     case ATT_DECODE_WIDE: attn_mfma_kernel<HD16, VD16, true, false><<<grid, 256, 0, s>>>(p); break;
     case ATT_PAIRS: attn_mfma_kernel<HD16, VD16, false, true><<<grid, 256, join, s>>>(p); break;
     case ATT_GROUPS: attn_mfma_kernel<HD16, VD16, false, false><<<grid, 256, join, s>>>(p); break;
-    case ATT_SHARED4: return launch_shared_one<HD16, VD16, 4, false>(p, grid, s);
+    case ATT_SHARED4:
+      if constexpr (HD16 >= 8 && VD16 >= 8)
+        if (stream_takes(p.hd, p.vd, p.bs, p.wide_weights)) return launch_stream<HD16, VD16, false>(p, grid, s);
+      return launch_shared_one<HD16, VD16, 4, false>(p, grid, s);
     case ATT_SHARED8:
       if constexpr (HD16 <= 8 && VD16 <= 8) return launch_shared_one<HD16, VD16, 8, false>(p, grid, s);
       else return zk_fail("zk_attention_bf16: eight waves a block take head sizes up to 128");
-    case ATT_RANGES: return launch_shared_one<HD16, VD16, 4, true>(p, grid, s);
+    case ATT_RANGES:
+      if constexpr (HD16 >= 8 && VD16 >= 8)
+        if (stream_takes(p.hd, p.vd, p.bs, p.wide_weights)) return launch_stream<HD16, VD16, true>(p, grid, s);
+      return launch_shared_one<HD16, VD16, 4, true>(p, grid, s);
     case ATT_DECODE:
       if constexpr (HD16 % 2 == 0) {
         const size_t lds = (size_t)4 * (p.nh / p.nkv) * p.vd * sizeof(float) + (size_t)4 * (HD16 / 2) * 64 * sizeof(bf16x8);
