@@ -58,6 +58,15 @@ def test_product_tiles_and_addresses(rt, M, N, K, gap, shift):
         assert np.array_equal(rt.download(one)[0], got[m, :N]), m
 
 
+# More than sixteen rows, K of 512 or more: sizes at which each of the tiles from 16 x 16 to 64 x 64 has the least price,
+# with ragged last rows and columns, K a whole number of steps, of fours, and odd
+@pytest.mark.parametrize("M,N,K", [(21, 102, 516), (22, 132, 513), (19, 2057, 516), (17, 2087, 513), (17, 4548, 516), (17, 4269, 513),
+                                   (33, 4419, 512), (33, 4185, 513), (17, 8279, 512), (17, 8988, 515), (33, 8266, 512), (33, 8332, 513),
+                                   (97, 6165, 516), (98, 6300, 513), (303, 1024, 4096)])
+def test_product_tiles_by_price(rt, M, N, K):
+    test_product(rt, M, N, K, 0)
+
+
 # heads, key heads (one to seventeen heads a key head), sizes of keys and values, page, window, first keys kept
 @pytest.mark.parametrize("nh,nkv,hd,vd,bs,window,keep", [(4, 2, 64, 64, 16, 0, 0), (3, 1, 20, 36, 4, 7, 0), (17, 1, 128, 128, 16, 70, 3),
                                                          (6, 6, 256, 256, 8, 0, 0), (10, 2, 132, 64, 32, 33, 0), (16, 1, 4, 4, 1, 0, 0)])

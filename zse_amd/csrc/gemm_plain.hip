@@ -7,6 +7,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cmath>
 
 #if ZSE_ACT_BF16
 #define GP_BM 64
@@ -72,7 +73,8 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
 //
 // Measured (us; before: 64 x 64 tiles of scalar multiply-adds through LDS, one block a tile):
 //   M = 303: 1024 x 4096 and 1024 x 1024 (average)  452 -> 42;  8192 x 1024  217 -> 87;
-//   1536 x 1024  191 -> 20;  M = 4: 32768 x 1024  207 -> 28.
+//   1536 x 1024  191 -> 20;  M = 4: 32768 x 1024  207 -> 28.  By f32_tile's choice: 1024 x 4096 61 -> 41, 1024 x 1024
+//   18.7 -> 14.2, 8192 x 1024 86 -> 80, 1536 x 1024 19.3 -> 18.9.
 // The error against 64 bits is no larger than the scalar sum's (eight shorter sums added up).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -225,16 +227,19 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(const float* __res
   }
 }
 
-template <int MF, int NF, int H, int AHEAD>
+// LONG: K of 512 or more only.
+template <int MF, int NF, int H, int AHEAD, bool LONG = false>
 static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc, int M, int N, int K,
                       hipStream_t s) {
   const int tiles_m = (M + 16 * MF - 1) / (16 * MF);
-  auto kernel = K < 4     ? gemm_f32_kernel<MF, NF, H, AHEAD, 0, 1>
-                : K <= 32 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 1>
-                : K <= 64 ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 2>
-                : K % 4   ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 8>
-                : K % 32  ? gemm_f32_kernel<MF, NF, H, AHEAD, 2, 8>
-                          : gemm_f32_kernel<MF, NF, H, AHEAD, 3, 8>;
+  auto kernel = K % 4    ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 8>
+                : K % 32 ? gemm_f32_kernel<MF, NF, H, AHEAD, 2, 8>
+                         : gemm_f32_kernel<MF, NF, H, AHEAD, 3, 8>;
+  if constexpr (!LONG) {
+    if (K < 4) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 0, 1>;
+    else if (K <= 32) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 1, 1>;
+    else if (K <= 64) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 1, 2>;
+  }
   const int waves = K <= 32 ? 1 : K <= 64 ? 2 : 8;
   // a launch of 2^32 threads or more would run its low 32 bits only: columns are taken 2^22 tiles at a time
   const long long most = (long long)std::max((1 << 22) / tiles_m, 1) * (16 * NF);
@@ -245,6 +250,34 @@ static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc
   return zk_launch_status("zk_gemm_plain");
 }
 
+// More than sixteen rows, K of 512 or more: the tile with the least price.  A launch takes as many rounds as the CU
+// with the most blocks has, whatever a block's registers would allow (303 x 1024 x 4096: 320 blocks of 32 x 32 61 us, 224 of
+// 48 x 32 41): a block alone already takes what its CU gets from its L2.  Microseconds, fitted to 17 to 2,048
+// rows by thirteen weights (512 to 18,432 columns, K of 1,024 to 9,216): a round's start, and for every 1,024 of K
+// one round's time and that of several.  The tile it names takes 1.009 times the best one's time in the mean and
+// 0.81 of that of 32 x 32 and 64 x 64 alone, 0.98 times the old rule's speed at the least.  The sums are the same bits.
+struct F32Tile { int mf, nf; double start, lone, several; };
+static const F32Tile f32_tiles[] = {
+    {1, 1, 0.88, 3.65, 3.47},
+    {1, 2, 1.39, 5.45, 5.16},
+    {2, 2, 0.74, 8.06, 7.45},
+    {3, 2, 2.54, 8.66, 8.68},
+    {2, 3, 2.71, 8.94, 8.55},
+    {3, 4, 0.00, 22.29, 21.65},
+    {4, 4, 2.23, 23.23, 22.63}};
+static int f32_tile(int M, int N, int K) {
+  int best = 0;
+  double best_time = 1e30;
+  const double t_mem = ((double)N * K + (double)M * K + (double)M * N) * 4e-6 / 5.0;
+  for (int i = 0; i < (int)(sizeof(f32_tiles) / sizeof(f32_tiles[0])); i++) {
+    const F32Tile& t = f32_tiles[i];
+    const long blocks = (long)((M + 16 * t.mf - 1) / (16 * t.mf)) * ((N + 16 * t.nf - 1) / (16 * t.nf)), rounds = (blocks + 255) / 256;
+    const double work = rounds * (t.start + (rounds == 1 ? t.lone : t.several) * K / 1024.0);
+    const double time = sqrt(sqrt(work * work * work * work + t_mem * t_mem * t_mem * t_mem));
+    if (time < best_time) best = i, best_time = time;
+  }
+  return best;
+}
 #endif  // ZSE_ACT_BF16
 
 extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
@@ -264,13 +297,24 @@ extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int
                                                          (act_t*)C, ldc, M, N, K);
   return zk_launch_status("zk_gemm_plain");
 #else
-  // 64 x 64 where the CUs then work through four rounds of blocks or more (2048 x 8192 x 1024:
+  // Few rows or a short K: 64 x 64 where the CUs then work through four rounds of blocks or more (2048 x 8192 x 1024:
   // 433 us against 459 with 32 x 32, but 303 x 8192 x 1024, 2.5 rounds: 83 against 77), 32 x 32
   // otherwise; up to sixteen rows two strips of sixteen columns where every CU then has two
   // blocks (4 x 32768 x 1024: 21.5 against 24.0 us), one where it has not (1 x 1024 x 4096: 10.8
   // against 18.1).
   auto blocks = [&](int mf, int nf) { return (long)((M + 16 * mf - 1) / (16 * mf)) * ((N + 16 * nf - 1) / (16 * nf)); };
   const float *a = (const float*)A, *w = (const float*)W;
+  if (M > 16 && K >= 512) {
+    switch (f32_tile(M, N, K)) {
+      case 0: return launch_f32<1, 1, 2, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 1: return launch_f32<1, 2, 2, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 2: return launch_f32<2, 2, 1, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 3: return launch_f32<3, 2, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 4: return launch_f32<2, 3, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 5: return launch_f32<3, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      default: return launch_f32<4, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+    }
+  }
   if (M > 16 && blocks(4, 4) >= 1024) return launch_f32<4, 4, 1, 3>(a, lda, w, (float*)C, ldc, M, N, K, s);
   if (M > 16) return launch_f32<2, 2, 1, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
   if (blocks(1, 2) >= 512) return launch_f32<1, 2, 2, 2>(a, lda, w, (float*)C, ldc, M, N, K, s);
