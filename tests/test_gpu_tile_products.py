@@ -22,6 +22,10 @@ CUTS = [
     (9, 1, 1, 0, 65, 32, 64), (9, 1, 1, 1, 65, 32, 64), (9, 4, 1, 0, 66, 32, 1024), (9, 4, 1, 1, 66, 32, 1024),
 ]
 
+# gated, 256 x 256 tiles in whole rounds and the columns behind them by another tile: that tile, rows, columns, K
+RESTS = [(1, 1545, 11664, 576), (2, 1538, 11360, 576), (3, 1031, 10912, 1536), (4, 1415, 12320, 576), (5, 675, 12368, 1024),
+         (7, 1415, 12944, 576), (8, 1057, 8368, 1024), (9, 642, 12336, 2112)]
+
 
 @pytest.fixture(scope="module")
 def rt():
@@ -31,7 +35,7 @@ def rt():
 
 def cut_of(gated, by_reader, M, N, K):
     from zse_amd.runtime import build
-    out = [C.c_int() for _ in range(3)]
+    out = [C.c_int() for _ in range(4)]
     assert C.CDLL(build.lib_path("kernels_bf16")).zk_gemm_bf16_tile_cut(gated, by_reader, M, N, K, *map(C.byref, out)) == 0
     return tuple(v.value for v in out)
 
@@ -60,7 +64,17 @@ def gelu_tanh(z):
 
 @pytest.mark.parametrize("shape,ks,tail,gated,M,N,K", CUTS)
 def test_every_cut(rt, shape, ks, tail, gated, M, N, K):
-    assert cut_of(gated, 0, M, N, K) == (shape, ks, tail)
+    assert cut_of(gated, 0, M, N, K) == (shape, ks, tail, -1)
+    check_product(rt, gated, M, N, K)
+
+
+@pytest.mark.parametrize("rest,M,N,K", RESTS)
+def test_columns_behind_the_whole_rounds(rt, rest, M, N, K):
+    assert cut_of(1, 0, M, N, K) == (0, 1, 1, rest)
+    check_product(rt, 1, M, N, K)
+
+
+def check_product(rt, gated, M, N, K):
     A, S, z = operands(rt, M, N * (1 + gated), K, seed=M + N)
     ws = workspace(rt)
     out = rt.upload(np.full((M + 2, N + 8), 0x4040, np.uint16), "bfloat16")

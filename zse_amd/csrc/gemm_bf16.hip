@@ -1414,7 +1414,7 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
       if (max(tile_sums(gated, M, N, cut.ks), tail_sums(cut.shape, cut_tail(cut, gated, M, N), cut.tail_ks)) > wsp.bytes) cut = tile_cut(gated, by_reader, M, N, K, wsp.bytes);
     }
     const TileProduct p{A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap};
-    return launch_direct_shape(cut.shape, gated, p, cut.ks, cut.tail_ks, (float*)wsp.ptr, parts, s);
+    return launch_cut(cut, gated, p, (float*)wsp.ptr, parts, s);
   }
   const bool exact = K % GT_BK == 0;
   const size_t room = (wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 64 == 0) ? wsp.split_bytes() : 0;
@@ -1435,14 +1435,15 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
 
 // Which tile (its number in tile_shapes) and how many ranges of K, of the last round's tiles alone, a product
 // of more than 64 rows by weights in strips, K a multiple of 64, takes with the standard workspace
-// (``by_reader``: the caller passes ``parts``).  For tests that mean to reach each of them.
+// (``by_reader``: the caller passes ``parts``), and which tile the columns behind the whole rounds take (-1: the same).  For tests that mean to reach each of them.
 extern "C" int zk_gemm_bf16_tile_cut(int gated, int by_reader, int M, int N, int K, int* shape, int* ks,
-                                     int* tail_ks) {
+                                     int* tail_ks, int* rest) {
   ZK_REQUIRE(M > 64 && N > 0 && K > 0 && K % 64 == 0, "zk_gemm_bf16_tile_cut: no tile product of this size");
   const TileCut c = tile_cut(gated != 0, by_reader != 0, M, N, K, ZK_GEMM_WORKSPACE_BYTES);
   *shape = c.shape;
   *ks = c.ks;
   *tail_ks = c.tail_ks;
+  *rest = c.rest;
   return 0;
 }
 

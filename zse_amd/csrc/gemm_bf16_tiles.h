@@ -7,9 +7,9 @@
 
 // How the tiles of a launch are dealt to blocks.  The first ``whole`` tiles in K ranges
 // ``ks``, the rest (a last round that would leave most CUs idle) in ``tail_ks`` ranges, all in
-// one grid.  ``gm``: rows of tiles of a group (tile_at).
+// one grid.  ``gm``: rows of tiles of a group (tile_at).  ``col0``: the launch's first column.
 struct TileGrid {
-  int tiles_m, tiles_n, gm, whole, ks, tail_ks;
+  int tiles_m, tiles_n, gm, whole, ks, tail_ks, col0;
 };
 
 // Blocks go round-robin over the 8 XCDs by their number; this gives each XCD a run of
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
   const int tile = place - range * part_tiles + (tail ? g.whole : 0);
   int tm, tn;
   tile_at(tile, g, tm, tn);
-  const int m0 = tm * BM, n0 = tn * OC;
+  const int m0 = tm * BM, n0 = g.col0 + tn * OC;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / NWN, wn = wave % NWN;
   const int lr = lane & 31, lk = lane >> 5;
@@ -379,7 +379,7 @@ static size_t tail_sums(int v, int tail, int ks) {
 }
 
 template <int TM, int TN, int NWM, int NWN, int NSA, int NSB, int MB, bool GATED>
-static int launch_direct(const TileProduct& p, int ks, int tail_ks, float* sums, int* parts, hipStream_t s) {
+static int launch_direct(const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, int* parts, hipStream_t s) {
   constexpr int BM = 32 * TM * NWM, BN = 32 * TN * NWN, OC = GATED ? BN / 2 : BN;
   constexpr size_t lds = (size_t)(NSA * BM + NSB * BN) * 128;
   static_assert(lds * MB <= 160 * 1024, "the blocks of a CU do not fit its LDS");
@@ -393,13 +393,14 @@ static int launch_direct(const TileProduct& p, int ks, int tail_ks, float* sums,
   }
   TileGrid g;
   g.tiles_m = (p.M + BM - 1) / BM;
-  g.tiles_n = (p.N + OC - 1) / OC;
+  g.tiles_n = (cols + OC - 1) / OC;
   ZK_REQUIRE((long long)g.tiles_m * g.tiles_n * max(ks, tail_ks) < 2147483647LL, "zk_gemm_bf16: too many tiles");
   g.gm = tile_group(g.tiles_m);
   const int tiles = g.tiles_m * g.tiles_n, tail = tail_ks > 1 ? tiles % (256 * MB) : 0;
   g.whole = tiles - tail;
   g.ks = ks;
   g.tail_ks = max(tail_ks, 1);
+  g.col0 = col0;
   kernel<<<g.whole * ks + tail * g.tail_ks, 64 * NWM * NWN, lds, s>>>(
       (const __bf16*)p.A, p.lda, (const __bf16*)p.W, p.C, p.ldc, p.c_is_f32, p.M, p.N, p.K, p.epi, p.cap, sums, g);
   if (ks > 1) {
@@ -418,10 +419,18 @@ static int launch_direct(const TileProduct& p, int ks, int tail_ks, float* sums,
   return zk_launch_status("zk_gemm_bf16 (tile)");
 }
 
-// How a product is cut.
+// How a product is cut.  ``rest``: the tile of the columns behind the whole rounds, a launch of their own
+// (-1: all columns by ``shape``).
 struct TileCut {
-  int shape, ks, tail_ks;
+  int shape, ks, tail_ks, rest;
 };
+
+// The columns that whole rounds of a shape's tiles take.
+static int whole_columns(int v, bool gated, int M, int N) {
+  const TileShape& t = tile_shapes[v];
+  const int oc = gated ? t.bn / 2 : t.bn, tiles_m = (M + t.bm - 1) / t.bm, slots = 256 * t.blocks;
+  return (int)((long)tiles_m * ((N + oc - 1) / oc) / slots * slots / tiles_m) * oc;
+}
 
 // The time of a cut in microseconds, and the cut with the least.  A CU works through its blocks one
 // after the other (or two at a time), each with a start and a time a step; the memory's time
@@ -433,24 +442,38 @@ struct TileCut {
 // registers, 128 x 256 and 256 x 256 copied in stages of 32 k, whole columns to an XCD): 0.82 of the
 // time in the geometric mean with joining launches, 0.77 where the reader joins; the most that was
 // lost is 4 to 7 % (448 to 1,024 rows by 4608 x 36864).
+//
+// A gated product by 256 x 256 tiles whose last round is not full may take the columns behind the whole
+// rounds by a smaller tile, in a launch of its own (5.5 us: it begins when the first has drained; 10.5 by
+// tiles of which two share a CU, 4.5 to 8 us slower there than their price).  The
+// ranges of a last round of such tiles write and read two planes of sums, which a joining launch adds up:
+// 2048 x (2 x 9216) x 2304 161 us with four ranges, 145 with 128 x 128 tiles for the last eighth; 1024 rows 98 -> 87.
+// 94 measured (rows, shape) of 150 to 4,096 rows that it takes: 0.97 of the time in the mean, 1.007 at the worst.
+// Not taken where it lost: products without a gate (3,600 x 4608 x 4096 126 -> 132 us), whole rounds of other
+// tiles (512 x (2 x 9216) x 2304 by 256 x 128 48.5 -> 55.8), short K (2,400 x (2 x 4096) x 1024 46.3 -> 47.9 at a price of 2 to 4).
 static double tile_time(const TileCut& c, bool gated, bool by_reader, int M, int N, int K) {
   const TileShape& t = tile_shapes[c.shape];
   const int oc = gated ? t.bn / 2 : t.bn;
   const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + oc - 1) / oc), slots = 256 * t.blocks;
-  auto rounds = [&](long blocks, double steps) {
+  auto rounds = [](const TileShape& t, long blocks, double steps) {
     const double one = t.start + steps * t.step, full = t.blocks == 2 ? t.start + steps * t.step_two : one;
-    const long rest = blocks % slots;
+    const long slots = 256 * t.blocks, rest = blocks % slots;
     return (double)(blocks / slots) * full + (rest == 0 ? 0.0 : rest <= 256 ? one : full);
   };
   const double steps = K / 32.0, mb = 1e-6, rows_out = (double)M * N;
   const double sums = c.ks > 1 ? (gated ? 2.0 : 1.0) * c.ks * rows_out * 4.0 * mb : 0.0;
   double t_blocks;
-  if (c.tail_ks > 1) {
+  if (c.rest >= 0) {
+    const TileShape& u = tile_shapes[c.rest];
+    const int ou = gated ? u.bn / 2 : u.bn, cols = whole_columns(c.shape, gated, M, N);
+    t_blocks = rounds(t, (long)((M + t.bm - 1) / t.bm) * (cols / oc), steps) + (u.blocks == 2 ? 10.5 : 5.5) +
+               rounds(u, (long)((M + u.bm - 1) / u.bm) * ((N - cols + ou - 1) / ou), steps);
+  } else if (c.tail_ks > 1) {
     const long tail = tiles % slots;
-    t_blocks = rounds(tiles - tail, steps) + rounds(tail * c.tail_ks, steps / c.tail_ks) + 3.5 +
+    t_blocks = rounds(t, tiles - tail, steps) + rounds(t, tail * c.tail_ks, steps / c.tail_ks) + 3.5 +
                (double)tail * c.tail_ks * t.bm * t.bn * 4.0 * mb / 5.0;
   } else {
-    t_blocks = rounds(tiles * c.ks, steps / c.ks);
+    t_blocks = rounds(t, tiles * c.ks, steps / c.ks);
   }
   const double t_mem = ((double)(gated ? 2 : 1) * N * K * 2.0 * mb + (double)M * K * 2.0 * mb + rows_out * 2.0 * mb + sums) / 4.15;
   double time = 1.65 + cbrt(t_blocks * t_blocks * t_blocks + t_mem * t_mem * t_mem);
@@ -467,7 +490,7 @@ static int cut_tail(const TileCut& c, bool gated, int M, int N) {
 
 static TileCut tile_cut(bool gated, bool by_reader, int M, int N, int K, size_t room) {
   static const int splits[] = {2, 3, 4, 5, 6, 8};
-  TileCut best{0, 1, 1};
+  TileCut best{0, 1, 1, -1};
   double best_time = 1e30;
   auto price = [&](const TileCut& c) {
     const double t = tile_time(c, gated, by_reader, M, N, K);
@@ -478,27 +501,37 @@ static TileCut tile_cut(bool gated, bool by_reader, int M, int N, int K, size_t 
     if (t.bm > 64 && 2L * t.bm > 3L * M) continue;
     const int oc = gated ? t.bn / 2 : t.bn;
     const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + oc - 1) / oc), slots = 256 * t.blocks, tail = tiles % slots;
-    price(TileCut{v, 1, 1});
+    price(TileCut{v, 1, 1, -1});
     // ranges of at least 256 k, no more blocks than about a round and a half; a last round no more
     // than half full, cut to one round at the most
     for (int ks : splits)
-      if (5 * tiles * ks <= 8 * slots && K / ks >= 256 && tile_sums(gated, M, N, ks) <= room) price(TileCut{v, ks, 1});
+      if (5 * tiles * ks <= 8 * slots && K / ks >= 256 && tile_sums(gated, M, N, ks) <= room) price(TileCut{v, ks, 1, -1});
     if (tiles > slots && tail > 0 && 2 * tail <= slots)
       for (int ks : {2, 4, 8})
-        if (10 * tail * ks <= 11 * slots && K / ks >= 256 && tail_sums(v, (int)tail, ks) <= room) price(TileCut{v, 1, ks});
+        if (10 * tail * ks <= 11 * slots && K / ks >= 256 && tail_sums(v, (int)tail, ks) <= room) price(TileCut{v, 1, ks, -1});
+    if (gated && v == 0 && tiles > slots && tail > 0 && whole_columns(v, gated, M, N) > 0)
+      for (int u = 0; u < tile_shape_count; u++)
+        if (u != v) price(TileCut{v, 1, 1, u});
   }
   return best;
 }
 
-static int launch_direct_shape(int v, bool gated, const TileProduct& p, int ks, int tail_ks, float* sums, int* parts,
-                               hipStream_t s) {
+static int launch_columns(int v, bool gated, const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, int* parts,
+                          hipStream_t s) {
   switch (v) {
 #define ZK_SHAPE(V, TM, TN, NWM, NWN, NSA, NSB, MB, START, STEP, STEP2)                                                       \
   case V:                                                                                           \
-    return gated ? launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, true>(p, ks, tail_ks, sums, parts, s)    \
-                 : launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, false>(p, ks, tail_ks, sums, parts, s);
+    return gated ? launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, true>(p, col0, cols, ks, tail_ks, sums, parts, s)    \
+                 : launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, false>(p, col0, cols, ks, tail_ks, sums, parts, s);
     ZK_TILE_SHAPES(ZK_SHAPE)
 #undef ZK_SHAPE
   }
   return zk_fail("zk_gemm_bf16: no such tile");
+}
+
+static int launch_cut(const TileCut& c, bool gated, const TileProduct& p, float* sums, int* parts, hipStream_t s) {
+  if (c.rest < 0) return launch_columns(c.shape, gated, p, 0, p.N, c.ks, c.tail_ks, sums, parts, s);
+  const int cols = whole_columns(c.shape, gated, p.M, p.N);
+  if (int rc = launch_columns(c.shape, gated, p, 0, cols, 1, 1, sums, parts, s)) return rc;
+  return launch_columns(c.rest, gated, p, cols, p.N - cols, 1, 1, sums, parts, s);
 }
