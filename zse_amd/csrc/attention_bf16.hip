@@ -19,12 +19,13 @@
 // the same permutation.  V is therefore cached transposed, [page][kv head][hd][bs],
 // so that four consecutive keys of a channel are one 8-byte load.
 //
-// Portions have three kernels, chosen by the launch's sizes (zk_attention_bf16): a group of 32
+// Portions have these kernels, chosen by the launch's sizes and a price (portion_plan): a group of 32
 // rows a block, its four waves sharing out the keys (attn_mfma_kernel: few groups); four or
 // eight consecutive groups a block with every tile of keys and values fetched once into LDS for
 // all of them (attn_shared_kernel: many groups); and the latter with the keys of a block of rows
 // cut into ranges over several blocks, joined by attn_portion_join_kernel (few groups with long
-// contexts: a portion of a prompt behind thousands of tokens).
+// contexts: a portion of a prompt behind thousands of tokens).  Heads of 128 and 256 channels with
+// pages of 16 or more take attn_stream_kernel in place of the shared tiles, in ranges or not.
 //
 // Decoded tokens use a split variant: the keys are cut into chunks aligned to absolute positions,
 // each leaves (max, sum, O) and a second kernel joins the chunks in order; the cut never follows
