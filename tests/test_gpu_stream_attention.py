@@ -96,3 +96,35 @@ def test_portions(rt, case, mode):
     # weights and results rounded to 8 bits of mantissa; values of size 1, the largest about 4.5
     assert np.abs(got - want).max() < 0.03, np.unravel_index(np.abs(got - want).argmax(), got.shape)
     assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("mode", [0, 4, 5])
+def test_pages_of_4_gib(rt, mode):
+    """A page's bytes and the places in it are more than 32 bits can count: the bits of a cache of small pages."""
+    kern = rt.kernels("bfloat16")
+    H, G, D, n, big, small = 8, 2, 256, 288, 1 << 22, 32
+    rng = np.random.default_rng(4)
+    q, k, v = up(rt, rng.normal(size=(n, H * D))), rng.normal(size=(G, n, D)), rng.normal(size=(G, D, n))
+    starts, ctx, out = rt.upload(np.array([0, n], np.int32)), rt.upload(np.array([n], np.int32)), rt.zeros((n, H * D), "bfloat16")
+    ws = rt.zeros((int(kern.zk_attention_bf16_portion_workspace(n + 128, H, G, D)) // 4 + 64,), "float32")
+
+    def run(kc, vc, table, bs):
+        table, n_pages = rt.upload(np.array([table], np.int32)), len(table)
+        before = kern.zk_attention_bf16_portion_kernel(mode)
+        try:
+            kern.zk_attention_bf16_sized(q.ptr, H * D, kc.ptr, vc.ptr, table.ptr, n_pages, starts.ptr, ctx.ptr, out.ptr, 1, 1, n, n, H, G, D,
+                                         bs, D ** -0.5, 50.0, 0, 0, ws.ptr, ws.nbytes, 0, 0, 0, 0, D, 0, rt.stream)
+            return rt.download(out)
+        finally:
+            kern.zk_attention_bf16_portion_kernel(before)
+
+    from zse_amd.weights.safetensors import f32_to_bf16_bits
+    bits = lambda x: f32_to_bf16_bits(np.ascontiguousarray(x, np.float32))
+    want = run(up(rt, k.reshape(G, n // small, small, D).swapaxes(0, 1)), up(rt, v.reshape(G, D, n // small, small).transpose(2, 0, 1, 3)),
+               list(range(n // small)), small)
+    kc, vc = rt.empty((2, G, big, D), "bfloat16"), rt.empty((2, G, D, big), "bfloat16")       # 16 GiB; page 1 is the request's
+    for g in range(G):
+        rt.copy_h2d(kc.ptr + 2 * (G + g) * big * D, bits(k[g]))
+        for d in range(D):
+            rt.copy_h2d(vc.ptr + 2 * ((G + g) * D + d) * big, bits(v[g, d]))
+    assert np.array_equal(run(kc, vc, [1], big), want)

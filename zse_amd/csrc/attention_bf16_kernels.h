@@ -833,13 +833,13 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
   const int* table = p.block_table + (size_t)r * p.max_blocks;
   const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, last_entry = p.max_blocks - 1;
 
-  // bytes of a page, and what lies before the key head's part of it
-  const unsigned k_page = (unsigned)(nkv * HD * 2) << bsh, v_page = (unsigned)((nkv >> p.v_shift) * VD * 2) << bsh;
+  // bytes of a page (4 GiB and more among them), and what lies before the key head's part of it
+  const size_t k_page = (size_t)nkv * HD * 2 << bsh, v_page = (size_t)(nkv >> p.v_shift) * VD * 2 << bsh;
   const unsigned char* const k_base = (const unsigned char*)p.kcache + ((size_t)kvh * HD * 2 << bsh);
   const unsigned char* const v_base = (const unsigned char*)p.vcache + ((size_t)(kvh >> p.v_shift) * VD * 2 << bsh);
   // the places of 64 pages, from entry ``first`` of the table on, one a lane; a tile lies in at most two (of 16 keys)
   struct Pages { unsigned lo, hi; int first; };
-  auto cover = [&](Pages& e, int key0, const unsigned char* base, unsigned page_bytes) __attribute__((always_inline)) {
+  auto cover = [&](Pages& e, int key0, const unsigned char* base, size_t page_bytes) __attribute__((always_inline)) {
     const int first = key0 >> bsh;
     if ((unsigned)(first - e.first) > 60u) {
       e.first = first;
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
   // Copies: K copy c = wave + 4 j is keys KPI c .. of the tile, V copy c 32 channels of the tile's first or last 16 keys.
   // Per copy: its page counted from the tile's first, and a lane's place behind the page's begin (tiles begin at
   // multiples of 32 keys: with pages of up to 32 keys the place does not depend on the tile, with larger ones a tile
-  // adds the same for all).
+  // adds the same for all).  A head's part of a page is at most 4 GiB (stream_takes), so 32 bits hold a place in it.
   unsigned k_off[KW], v_off[VW];
   int k_idx[KW], v_idx[VW];
 #pragma unroll
@@ -1557,7 +1557,7 @@ static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
 
 // What attn_stream_kernel takes of the launches of four groups a block.
 static inline bool stream_takes(int hd, int vd, int bs, int wide_weights) {
-  return (hd == 128 || hd == 256) && (vd == 128 || vd == 256) && bs >= 16 && !wide_weights;
+  return (hd == 128 || hd == 256) && (vd == 128 || vd == 256) && bs >= 16 && bs <= (1 << 23) && !wide_weights;
 }
 
 template <int HD16, int VD16, bool SPLIT>
