@@ -128,3 +128,33 @@ def test_pages_of_4_gib(rt, mode):
         for d in range(D):
             rt.copy_h2d(vc.ptr + 2 * ((G + g) * D + d) * big, bits(v[g, d]))
     assert np.array_equal(run(kc, vc, [1], big), want)
+
+
+@pytest.mark.parametrize("mode", [0, 4, 5])
+@pytest.mark.parametrize("D,E,before,n", [(256, 256, 0, 40), (128, 128, 0, 296), (256, 256, 200, 121), (128, 256, 1000, 70), (256, 128, 0, 705)])
+def test_table_entries_behind_the_last_page(rt, mode, D, E, before, n):
+    """The page after a request's last one is another's and holds NaN; the last tile of keys reaches into it."""
+    kern = rt.kernels("bfloat16")
+    H, G, bs, ctx = 4, 2, 16, before + n
+    used = -(-ctx // bs)
+    assert used % 2 == 1
+    rng = np.random.default_rng(n)
+    q, k, v = (rounded(rng.normal(size=s)) for s in ((n, H, D), (ctx, G, D), (ctx, G, E)))
+    kc, vc = np.full((used + 2, bs, G, D), np.nan, np.float32), np.full((used + 2, bs, G, E), np.nan, np.float32)
+    kc[:used], vc[:used] = 0, 0
+    kc[:used].reshape(-1, G, D)[:ctx], vc[:used].reshape(-1, G, E)[:ctx] = k, v
+    table = np.concatenate([np.arange(used + 1), np.full(7, used + 1)]).astype(np.int32)
+    out = rt.zeros((n, H * E), "bfloat16")
+    ws = rt.zeros((int(kern.zk_attention_bf16_portion_workspace(n + 128, H, G, E)) // 4 + 64,), "float32")
+    args = [up(rt, q.reshape(n, -1)), up(rt, kc.swapaxes(1, 2)), up(rt, vc.transpose(0, 2, 3, 1)), rt.upload(table, "int32"),
+            rt.upload(np.array([0, n], np.int32), "int32"), rt.upload(np.array([ctx], np.int32), "int32")]
+    mode_before = kern.zk_attention_bf16_portion_kernel(mode)
+    try:
+        kern.zk_attention_bf16_sized(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, len(table), args[4].ptr, args[5].ptr, out.ptr,
+                                     1, 1, n, ctx, H, G, D, bs, D ** -0.5, 0.0, 0, 0, ws.ptr, ws.nbytes, 0, 0, 0, 0, E, 0, rt.stream)
+        got = rt.download_f32(out).reshape(n, H, E)
+    finally:
+        kern.zk_attention_bf16_portion_kernel(mode_before)
+    want = plain(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), before, D ** -0.5, 0.0, 0, 0)
+    assert np.isfinite(got).all()
+    assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)

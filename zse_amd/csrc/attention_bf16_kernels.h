@@ -780,7 +780,8 @@ __device__ __forceinline__ void stream_order() {
 // half tile belong to eight neighbouring keys: 16 bytes of a channel of the transposed values.
 //
 // A masked score is set to the score's least value before the turn and its weight to zero after it; only tiles at an edge
-// have any.  Tiles past the range are copied (from the table's last entries) and multiplied, never weighted.
+// have any.  Tiles past the range are copied and multiplied, never weighted.  Keys past the block's last page are copied from
+// that page: whatever the table holds behind it is neither followed nor multiplied by a weight of 0.
 template <int HD16, int VD16, bool SPLIT, bool CAPPED>
 __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_stream_kernel(AttnParams p) {
   // (the host's pass knows no address spaces)
@@ -831,7 +832,7 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
   const int all_hi = ntok > 0 ? start + t0 : 0x7fffff00;
   const int all_lo = ntok > 0 ? first_key(p, start + t0 + ntok - 1) : 0;
   const int* table = p.block_table + (size_t)r * p.max_blocks;
-  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, last_entry = p.max_blocks - 1;
+  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, last_entry = min(p.max_blocks - 1, blk_hi >> bsh);
 
   // bytes of a page (4 GiB and more among them), and what lies before the key head's part of it
   const size_t k_page = (size_t)nkv * HD * 2 << bsh, v_page = (size_t)(nkv >> p.v_shift) * VD * 2 << bsh;
