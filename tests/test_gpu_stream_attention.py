@@ -158,3 +158,29 @@ def test_table_entries_behind_the_last_page(rt, mode, D, E, before, n):
     want = plain(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), before, D ** -0.5, 0.0, 0, 0)
     assert np.isfinite(got).all()
     assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("H,G,D,rows,ctx", [(8, 4, 256, 512, 4096), (32, 16, 128, 512, 4096)])
+def test_ranges_without_room_for_them(rt, H, G, D, rows, ctx):
+    """Where the workspace does not hold the ranges' results, the better of the forms that need none runs: here the one of a
+    group of rows a block, whose bits are not those of four groups."""
+    kern = rt.kernels("bfloat16")
+    rng, bs = np.random.default_rng(D), 16
+    pages = ctx // bs
+    args = [up(rt, rng.normal(size=s)) for s in ((rows, H * D), (pages, G, bs, D), (pages, G, D, bs))]
+    args += [rt.upload(np.array(x, np.int32), "int32") for x in ([list(range(pages))], [0, rows], [ctx])]
+    ws = rt.zeros((int(kern.zk_attention_bf16_portion_workspace(rows + 128, H, G, D)) // 4 + 64,), "float32")
+
+    def run(mode, ws_bytes):
+        out = rt.zeros((rows, H * D), "bfloat16")
+        before = kern.zk_attention_bf16_portion_kernel(mode)
+        try:
+            kern.zk_attention_bf16(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, pages, args[4].ptr, args[5].ptr, out.ptr, 1, 1,
+                                   rows, ctx, H, G, D, bs, D ** -0.5, 50.0, 0, 0, ws.ptr, ws_bytes, rt.stream)
+            return rt.download(out)
+        finally:
+            kern.zk_attention_bf16_portion_kernel(before)
+    group, four, ranges = run(1, 0), run(4, 0), run(5, ws.nbytes)
+    assert not np.array_equal(group, four) and not np.array_equal(group, ranges)
+    assert np.array_equal(run(0, ws.nbytes), ranges)
+    assert np.array_equal(run(0, 0), group) and np.array_equal(run(0, 4096), group)

@@ -1,0 +1,34 @@
+"""Which kernel a launch of portions takes (host code: no GPU needed)."""
+import ctypes as C
+
+import pytest
+
+
+def form_of(room, R, rows, ctx, H, G, D, E=0, bs=16, window=0, chunk=0, keep=0, wide_weights=0):
+    """(groups of rows a block, or 5 for four with the keys in ranges; tiles of a range; by attn_stream_kernel)"""
+    from zse_amd.runtime import build
+    lib = C.CDLL(build.ensure("kernels_bf16"))
+    ranges, stream = C.c_int(-1), C.c_int(-1)
+    form = lib.zk_attention_bf16_portion_form(R, rows, ctx, H, G, D, E or D, bs, window, chunk, keep, wide_weights, C.c_size_t(room),
+                                              C.byref(ranges), C.byref(stream))
+    return form, ranges.value, stream.value
+
+
+# requests, rows, context, heads, key heads, channels; the form without ranges
+CASES = [((1, 512, 4096, 8, 4, 256), 1), ((1, 512, 4096, 32, 16, 128), 1), ((1, 1024, 2048, 8, 4, 256), 1),
+         ((2, 1024, 3000, 8, 4, 256), 4), ((1, 2048, 2048, 16, 8, 256), 4)]
+
+
+@pytest.mark.parametrize("case,whole", CASES)
+def test_without_room_for_ranges_the_better_form_that_needs_none(case, whole):
+    form, tiles, stream = form_of(1 << 30, *case)
+    assert (form, stream) == (5, 1) and tiles > 0
+    assert form_of(0, *case)[0] in ((1, 2) if whole == 1 else (4,))
+    assert form_of(4096, *case) == form_of(0, *case)
+
+
+def test_pages_whose_places_32_bits_do_not_hold():
+    assert form_of(0, 1, 4000, 4000, 8, 4, 256, bs=1 << 23)[2] == 1
+    assert form_of(0, 1, 4000, 4000, 8, 4, 256, bs=1 << 24)[2] == 0
+    assert form_of(0, 1, 4000, 4000, 8, 4, 256, bs=8)[2] == 0
+    assert form_of(0, 1, 4000, 4000, 8, 4, 256, wide_weights=1)[2] == 0

@@ -243,7 +243,7 @@ static int portion_ranges(int max_q_len, int max_ctx, int window, int mask_chunk
 // keys 25, 28, 23, ranges; behind 3,584 112, 145, 43, ranges; 4,000 rows 241, 142, 178, four; three
 // times 1,000 98, 45, -, four; 16 over 8, 3,000 rows 287, 117, 139, four; 32 over 16 of 128, 512 rows at 512 keys
 // 16, 22, 26, group; 2,048 rows 169, 70, 95, four.
-struct PortionPlan { int kind, ranges; };      // ranges: the best cut with ranges, taken or not (0: none)
+struct PortionPlan { int kind, ranges, whole; };      // ranges: the best cut with ranges, taken or not (0: none); whole: the better kind without
 static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int tpw, int nkv, int r_prefill,
                                 int bound_tiles, int wide) {
   const bool narrow = wide <= 128;
@@ -269,11 +269,11 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
     if (blocks <= slots) return alone;
     return std::max(alone, (blocks * start + per_tile * tiles) / slots + 0.5 * (start + per_tile * least));
   };
-  PortionPlan best{0, 0};
+  PortionPlan best{0, 0, 0};
   const double groups = (max_q_len + tpw - 1) / tpw;
   double best_price = price(groups * copies, start_group, tile_group, sum * copies * groups / row_blocks, longest, shortest);
   const double four = price((double)row_blocks * copies, start_four, tile_four, sum * copies, longest, shortest);
-  if (four < best_price) best = {4, 0}, best_price = four;
+  if (four < best_price) best = {4, 0, 4}, best_price = four;
   double best_ranges = 1e30;
   static const int cands[] = {64, 48, 40, 32, 24, 16, 12, 10, 8, 6, 4};
   for (int ct : cands) {
@@ -293,12 +293,79 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
 // the workspace allows).  For tests and measurements (process-wide).
 static int portion_kernel_mode = 0;
 
+// How a launch of portions runs: which kernel, and with ranges the tiles of one and the most that a
+// block of rows has.  ``room``: bytes of workspace for the ranges' partial results.
+struct PortionForm {
+  AttnWhat what;
+  int range_tiles, most_ranges;
+};
+static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, int nh, int nkv, int hd, int vd, int bs, int window,
+                                int mask_chunk, int keep, int wide_weights, size_t room) {
+  const int tpw = 32 / (nh / nkv), per_block = 4 * tpw, wide = std::max(hd, vd), groups = (max_q_len + tpw - 1) / tpw;
+  const bool stream = stream_takes(hd, vd, bs, wide_weights);
+  // one block a group; two groups a block when that lets every block run at once (256 CUs,
+  // one block each) where single groups would need a second round
+  const long long single = (long long)groups * nkv * r_prefill, paired = (long long)((groups + 1) / 2) * nkv * r_prefill;
+  // Many groups: tiles shared by the four or eight groups of a block, where that still gives
+  // every CU a block (four) or two (eight; head sizes up to 128, whose registers let two
+  // waves share a SIMD).  Measured at 8 to 32 heads of 128 and 256 with 512 to 8,192 rows:
+  // with fewer than about 768 groups the kernel of one group a block is faster (2,048 rows of
+  // 8 heads of 256, 512 groups: 75 us against 111; 768 groups: a tie), with more the shared
+  // tiles are (8 portions of 512 rows behind 7,680 tokens, 32 heads of 128: 1,630 -> 780 us;
+  // 16 heads of 256: 1,560 -> 845 us; 8,192 rows of 8 heads of 256: 877 -> 463 us).
+  int shared_waves = 0;
+  if (bs >= 8 && portion_kernel_mode != 1 && !(stream && portion_kernel_mode == 0)) {
+    if (portion_kernel_mode > 1) shared_waves = portion_kernel_mode == 8 ? 8 : 4;
+    else if (single >= 4096 && wide <= 128) shared_waves = 8;
+    else if (single >= 768) shared_waves = 4;
+    if (shared_waves == 8 && wide > 128) shared_waves = 4;       // no room for two waves a SIMD
+  }
+  // Few blocks of rows with many keys each (a portion of a few hundred rows behind thousands of
+  // tokens): four groups a block and the keys in ranges, where the workspace behind the decoded
+  // tokens' part holds the ranges' partial results.  512 rows behind 3,584 tokens, 8 heads of
+  // 256: 111 -> 52 us; behind 7,680: 209 -> 79 us; 16 heads of 256: 118 -> 76 us; 32 heads of
+  // 128: 100 -> 73 us.  A whole prompt from its first token, 8 heads of 256: 2,048 rows 74 -> 62
+  // us, 1,024 rows the same time either way (its blocks of rows are many and short already).
+  if (bs >= 8 && (portion_kernel_mode == 5 || (portion_kernel_mode == 0 && !shared_waves))) {
+    // no block of rows has more tiles than this, whatever its request's length
+    int bound = (max_ctx + 31) / 32, range_tiles;
+    // (a chunk's rows see no more keys than a window of its size would show them)
+    const int reach = mask_chunk > 0 ? mask_chunk : window;
+    if (reach > 0) bound = std::min(bound, (reach + per_block + 31) / 32 + 1 + (keep + 31) / 32);
+    if (stream) {
+      const PortionPlan plan = portion_plan(max_q_len, max_ctx, window, mask_chunk, keep, tpw, nkv, r_prefill, bound, wide);
+      range_tiles = portion_kernel_mode == 5 || plan.kind == 5 ? plan.ranges : 0;
+      shared_waves = std::max(shared_waves, plan.whole);       // without ranges, also where the workspace does not hold them
+    } else {
+      range_tiles = portion_ranges(max_q_len, max_ctx, window, mask_chunk, keep, per_block, nkv, r_prefill, bound);
+    }
+    if (range_tiles) {
+      const int most_ranges = (bound + range_tiles - 1) / range_tiles;
+      const long row_blocks = (long)r_prefill * ((max_q_len + per_block - 1) / per_block);
+      if (portion_split_bytes(row_blocks, nkv, vd, most_ranges) <= room) return {ATT_RANGES, range_tiles, most_ranges};
+    }
+  }
+  if (shared_waves) return {shared_waves == 8 ? ATT_SHARED8 : ATT_SHARED4, 0, 0};
+  return {single > 256 && paired <= 256 ? ATT_PAIRS : ATT_GROUPS, 0, 0};
+}
+
 extern "C" {
 
 int zk_attention_bf16_portion_kernel(int mode) {
   const int before = portion_kernel_mode;
   if (mode == 0 || mode == 1 || mode == 4 || mode == 5 || mode == 8) portion_kernel_mode = mode;
   return before;
+}
+
+// Which form a launch of ``r_prefill`` portions takes with ``room`` bytes of workspace behind the decoded tokens' part: 1, 2, 4 or 8
+// groups of rows a block, or 5, four with the keys in ranges of *range_tiles tiles.  *stream: by attn_stream_kernel.  For tests that mean
+// to reach each of them.
+int zk_attention_bf16_portion_form(int r_prefill, int max_q_len, int max_ctx, int nh, int nkv, int hd, int vd, int bs, int window,
+                                   int mask_chunk, int keep, int wide_weights, size_t room, int* range_tiles, int* stream) {
+  const PortionForm f = portion_form(r_prefill, max_q_len, max_ctx, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights, room);
+  *range_tiles = f.range_tiles;
+  *stream = (f.what == ATT_SHARED4 || f.what == ATT_RANGES) && stream_takes(hd, vd, bs, wide_weights);
+  return f.what == ATT_RANGES ? 5 : f.what == ATT_SHARED8 ? 8 : f.what == ATT_SHARED4 ? 4 : f.what == ATT_PAIRS ? 2 : 1;
 }
 
 // 1 if the matrix-core kernel takes these sizes, else 0 (the caller then uses the plain kernel).
@@ -420,64 +487,20 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
   p.k1 = scale * log2e;
   p.k2 = softcap > 0.f ? 2.f * scale / softcap * log2e : 0.f;
   p.c2 = softcap * log2e;
-  const int g = nh / nkv, wide = std::max(hd, vd);
+  const int g = nh / nkv;
   if (r_prefill > 0) {
     p.tpw = 32 / g; p.r_begin = 0; p.nchunks = 1; p.part_o = nullptr; p.part_ml = nullptr;
     const int groups = (max_q_len + p.tpw - 1) / p.tpw;
-    // one block a group; two groups a block when that lets every block run at once (256 CUs,
-    // one block each) where single groups would need a second round
-    const long long single = (long long)groups * nkv * r_prefill, paired = (long long)((groups + 1) / 2) * nkv * r_prefill;
-    int rc;
-    // Many groups: tiles shared by the four or eight groups of a block, where that still gives
-    // every CU a block (four) or two (eight; head sizes up to 128, whose registers let two
-    // waves share a SIMD).  Measured at 8 to 32 heads of 128 and 256 with 512 to 8,192 rows:
-    // with fewer than about 768 groups the kernel of one group a block is faster (2,048 rows of
-    // 8 heads of 256, 512 groups: 75 us against 111; 768 groups: a tie), with more the shared
-    // tiles are (8 portions of 512 rows behind 7,680 tokens, 32 heads of 128: 1,630 -> 780 us;
-    // 16 heads of 256: 1,560 -> 845 us; 8,192 rows of 8 heads of 256: 877 -> 463 us).
-    const bool stream = stream_takes(hd, vd, bs, wide_weights);
-    int shared_waves = 0;
-    if (bs >= 8 && portion_kernel_mode != 1 && !(stream && portion_kernel_mode == 0)) {
-      if (portion_kernel_mode > 1) shared_waves = portion_kernel_mode;
-      else if (single >= 4096 && wide <= 128) shared_waves = 8;
-      else if (single >= 768) shared_waves = 4;
-      if (shared_waves == 8 && wide > 128) shared_waves = 4;       // no room for two waves a SIMD
-    }
-    // Few blocks of rows with many keys each (a portion of a few hundred rows behind thousands of
-    // tokens): four groups a block and the keys in ranges, where the workspace behind the decoded
-    // tokens' part holds the ranges' partial results.  512 rows behind 3,584 tokens, 8 heads of
-    // 256: 111 -> 52 us; behind 7,680: 209 -> 79 us; 16 heads of 256: 118 -> 76 us; 32 heads of
-    // 128: 100 -> 73 us.  A whole prompt from its first token, 8 heads of 256: 2,048 rows 74 -> 62
-    // us, 1,024 rows the same time either way (its blocks of rows are many and short already).
-    int range_tiles = 0, most_ranges = 0;
     size_t split_at = 0;
-    if (bs >= 8 && (portion_kernel_mode == 5 || (portion_kernel_mode == 0 && !shared_waves))) {
-      const int per_block = 4 * p.tpw;
-      // no block of rows has more tiles than this, whatever its request's length
-      int bound = (max_ctx + 31) / 32;
-      // (a chunk's rows see no more keys than a window of its size would show them)
-      const int reach = mask_chunk > 0 ? mask_chunk : window;
-      if (reach > 0) bound = std::min(bound, (reach + per_block + 31) / 32 + 1 + (keep + 31) / 32);
-      if (stream) {
-        const PortionPlan plan = portion_plan(max_q_len, max_ctx, window, mask_chunk, keep, p.tpw, nkv, r_prefill, bound, wide);
-        if (portion_kernel_mode == 5 || plan.kind == 5) range_tiles = plan.ranges;
-        if (plan.kind) shared_waves = std::max(shared_waves, 4);           // also where the workspace does not hold the ranges
-      } else {
-        range_tiles = portion_ranges(max_q_len, max_ctx, window, mask_chunk, keep, per_block, nkv, r_prefill, bound);
-      }
-      if (range_tiles) {
-        most_ranges = (bound + range_tiles - 1) / range_tiles;
-        if (R - r_prefill > 0) split_at = (zk_attention_bf16_workspace(R - r_prefill, nh, vd, max_ctx) + 255) / 256 * 256;
-        const size_t need = portion_split_bytes((long)r_prefill * ((max_q_len + per_block - 1) / per_block), nkv, vd,
-                                                most_ranges);
-        if (workspace == nullptr || (uintptr_t)workspace % 16 != 0 || split_at + need > workspace_bytes)
-          range_tiles = 0;
-      }
-    }
-    if (range_tiles) {
-      const int per_block = 4 * p.tpw;
+    if (R - r_prefill > 0) split_at = (zk_attention_bf16_workspace(R - r_prefill, nh, vd, max_ctx) + 255) / 256 * 256;
+    const bool usable = workspace != nullptr && (uintptr_t)workspace % 16 == 0 && split_at < workspace_bytes;
+    const PortionForm form = portion_form(r_prefill, max_q_len, max_ctx, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights,
+                                          usable ? workspace_bytes - split_at : 0);
+    int rc;
+    if (form.what == ATT_RANGES) {
+      const int per_block = 4 * p.tpw, most_ranges = form.most_ranges;
       AttnParams ps = p;
-      ps.chunk = range_tiles;
+      ps.chunk = form.range_tiles;
       ps.nchunks = most_ranges;
       const int row_blocks = (max_q_len + per_block - 1) / per_block;
       const size_t slots = (size_t)r_prefill * nkv * row_blocks * most_ranges * 4;
@@ -489,12 +512,10 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
       if (rc) return rc;
       attn_portion_join_kernel<<<dim3(row_blocks * 4 * dts, nkv, r_prefill), 64, 0, s>>>(ps, per_block, row_blocks, dts);
       rc = zk_launch_status("zk_attention_bf16 (join of the portions' ranges)");
-    } else if (shared_waves) {
-      if (shared_waves == 5) shared_waves = 4;
-      dim3 grid((groups + shared_waves - 1) / shared_waves, nkv, r_prefill);
-      rc = launch_attn(shared_waves == 4 ? ATT_SHARED4 : ATT_SHARED8, p, grid, s);
-    } else if (single > 256 && paired <= 256) rc = launch_attn(ATT_PAIRS, p, dim3((groups + 1) / 2, nkv, r_prefill), s);
-    else rc = launch_attn(ATT_GROUPS, p, dim3(groups, nkv, r_prefill), s);
+    } else {
+      const int a_block = form.what == ATT_SHARED8 ? 8 : form.what == ATT_SHARED4 ? 4 : form.what == ATT_PAIRS ? 2 : 1;
+      rc = launch_attn(form.what, p, dim3((groups + a_block - 1) / a_block, nkv, r_prefill), s);
+    }
     if (rc) return rc;
   }
   const int n_dec = R - r_prefill;
