@@ -16,7 +16,7 @@ def form_of(room, R, rows, ctx, H, G, D, E=0, bs=16, window=0, chunk=0, keep=0, 
 
 # requests, rows, context, heads, key heads, channels; the form without ranges
 CASES = [((1, 512, 4096, 8, 4, 256), 1), ((1, 512, 4096, 32, 16, 128), 1), ((1, 1024, 2048, 8, 4, 256), 1),
-         ((2, 1024, 3000, 8, 4, 256), 4), ((1, 2048, 2048, 16, 8, 256), 4)]
+         ((2, 1024, 3000, 8, 4, 256), 4), ((1, 3000, 4096, 8, 4, 256), 4)]
 
 
 @pytest.mark.parametrize("case,whole", CASES)
@@ -32,3 +32,11 @@ def test_pages_whose_places_32_bits_do_not_hold():
     assert form_of(0, 1, 4000, 4000, 8, 4, 256, bs=1 << 24)[2] == 0
     assert form_of(0, 1, 4000, 4000, 8, 4, 256, bs=8)[2] == 0
     assert form_of(0, 1, 4000, 4000, 8, 4, 256, wide_weights=1)[2] == 0
+
+
+@pytest.mark.parametrize("case,form", [((1, 2048, 2048, 32, 16, 128), 4), ((1, 2048, 2048, 32, 8, 128), 4), ((1, 2048, 2048, 16, 8, 256), 4),
+                                       ((1, 104, 104, 8, 8, 128), 1), ((2, 116, 116, 8, 8, 128), 1)])
+def test_launches_that_a_form_with_fewer_blocks_runs_faster(case, form):
+    """Two ranges a block of rows lie on halves of the chip that have unlike work, and a block of four groups that has rows for
+    one is slower than a group a block (94 us against 70, 80 against 61, 98 against 81, 12.4 against 10.5 twice)."""
+    assert form_of(1 << 30, *case)[0] == form

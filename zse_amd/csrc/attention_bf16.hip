@@ -238,19 +238,25 @@ static int portion_ranges(int max_q_len, int max_ctx, int window, int mask_chunk
 // latter with the keys in ranges of ``ranges`` tiles (5), by the least of three prices in microseconds.  A
 // block costs a start and a time a tile; blocks beyond one a CU (two for 128 channels) take their
 // share of the CUs' time, the last ones half of the shortest block's more; ranges add a block's partial
-// results and the joining launch.  The constants are fitted to launches of 300 to 4,000 rows behind up to
-// 4,096 keys, 2 to 16 key heads, one and three requests (us; group, four, ranges, taken): 8 heads over 4 of 256, 512 rows at 512
-// keys 25, 28, 23, ranges; behind 3,584 112, 145, 43, ranges; 4,000 rows 241, 142, 178, four; three
-// times 1,000 98, 45, -, four; 16 over 8, 3,000 rows 287, 117, 139, four; 32 over 16 of 128, 512 rows at 512 keys
-// 16, 22, 26, group; 2,048 rows 169, 70, 95, four.
+// results, the blocks that find nothing to do and the joining launch.  A block of rows' ranges are neighbours in
+// the grid, and blocks go round to the XCDs and their shader engines by number: where 2, 4 or 8 divides the most ranges of a
+// block of rows, the first ranges share one half, quarter or eighth of the chip and the last, short or not there,
+// another, so each such class is priced on its part (2,048 rows from their first token, 32 heads over 16 of 128: ranges of 32 tiles,
+// two a block of rows, 94 us, of 24, three, 82; four groups a block 70).
+// The constants are fitted to launches of 40 to 4,096 rows behind up to 8,000 keys, 2 to 16 key heads, one to eight
+// requests: over 390 of them the form that is named takes 1.016 times the best one's time in the mean, 1.32 at the
+// most (us; group, four, ranges, taken): 8 heads over 4 of 256, 512 rows at 512
+// keys 25, 28, 23, ranges; behind 3,584 112, 143, 42, ranges; 4,096 rows 238, 135, 129, ranges; 16 over 8, 2,048 rows 149, 81, 84,
+// four; 32 over 16 of 128, 512 rows at 512 keys 16, 21, 25, group; 2,048 rows 168, 70, 82, four.
 struct PortionPlan { int kind, ranges, whole; };      // ranges: the best cut with ranges, taken or not (0: none); whole: the better kind without
 static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int tpw, int nkv, int r_prefill,
                                 int bound_tiles, int wide) {
   const bool narrow = wide <= 128;
   const int slots = narrow ? 512 : 256, per_block = 4 * tpw, row_blocks = (max_q_len + per_block - 1) / per_block;
   const long copies = (long)nkv * r_prefill;
-  const double start_group = narrow ? 8.7 : 11.6, tile_group = narrow ? 0.64 : 0.77;
-  const double start_four = narrow ? 6.6 : 11.0, tile_four = narrow ? 0.83 : 1.06;
+  const double start_group = narrow ? 8.7 : 12.0, tile_group = narrow ? 0.64 : 0.77;
+  const double start_four = narrow ? 5.5 : 9.5, start_range = narrow ? 6.6 : 11.0, tile_four = narrow ? 0.83 : 1.06;
+  const double edges = (narrow ? 1.0 : 0.4) * std::min(max_q_len, per_block) / 32;       // tiles whose scores are masked
   auto tiles_of = [&](int bi) {
     const int lo = max_ctx - max_q_len + bi * per_block, hi = std::min(max_ctx, lo + per_block) - 1;
     const int klo = mask_chunk > 0 ? lo - lo % mask_chunk : window > 0 ? std::max(0, lo - window + 1) : 0;
@@ -264,24 +270,32 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
     shortest = std::min(shortest, t);
     sum += t;
   }
-  auto price = [&](double blocks, double start, double per_tile, double tiles, int most, int least) {
+  auto price = [&](int slots, double blocks, double start, double per_tile, double tiles, int most, int least) {
     const double alone = start + per_tile * most;
     if (blocks <= slots) return alone;
     return std::max(alone, (blocks * start + per_tile * tiles) / slots + 0.5 * (start + per_tile * least));
   };
   PortionPlan best{0, 0, 0};
   const double groups = (max_q_len + tpw - 1) / tpw;
-  double best_price = price(groups * copies, start_group, tile_group, sum * copies * groups / row_blocks, longest, shortest);
-  const double four = price((double)row_blocks * copies, start_four, tile_four, sum * copies, longest, shortest);
+  double best_price = price(slots, groups * copies, start_group, tile_group, sum * copies * groups / row_blocks, longest, shortest);
+  const double four = edges + price(slots, (double)row_blocks * copies, start_four, tile_four, sum * copies, longest, shortest);
   if (four < best_price) best = {4, 0, 4}, best_price = four;
   double best_ranges = 1e30;
   static const int cands[] = {64, 48, 40, 32, 24, 16, 12, 10, 8, 6, 4};
   for (int ct : cands) {
-    if (2 * ct > longest || (bound_tiles + ct - 1) / ct > ATT_MOST_RANGES) continue;
-    double blocks = 0;
-    for (int bi = 0; bi < row_blocks; bi++) blocks += (tiles_of(bi) + ct - 1) / ct;
-    blocks *= copies;
-    const double t = price(blocks, start_four, tile_four, sum * copies, ct, std::min(shortest, ct)) + blocks * wide * (0.035 / 256) + 4.0;
+    const int most_ranges = (bound_tiles + ct - 1) / ct, classes = most_ranges & -most_ranges;
+    if (2 * ct > longest || most_ranges > ATT_MOST_RANGES) continue;
+    double blocks[ATT_MOST_RANGES] = {}, tiles[ATT_MOST_RANGES] = {}, t = 0, all = 0;
+    for (int bi = 0; bi < row_blocks; bi++)
+      for (int i = 0, left = tiles_of(bi); left > 0; i++, left -= ct) {
+        blocks[i % classes] += copies;
+        tiles[i % classes] += (double)std::min(left, ct) * copies;
+      }
+    for (int i = 0; i < classes; i++) {
+      t = std::max(t, price(slots / classes, blocks[i], start_range, tile_four, tiles[i], ct, std::min(shortest, ct)));
+      all += blocks[i];
+    }
+    t += all * wide * (0.035 / 256) + ((double)row_blocks * copies * most_ranges - all) * 0.005 + 4.0;
     if (t < best_ranges) best.ranges = ct, best_ranges = t;
   }
   if (best_ranges < best_price) best.kind = 5;
