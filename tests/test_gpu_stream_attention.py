@@ -184,3 +184,47 @@ def test_ranges_without_room_for_them(rt, H, G, D, rows, ctx):
     assert not np.array_equal(group, four) and not np.array_equal(group, ranges)
     assert np.array_equal(run(0, ws.nbytes), ranges)
     assert np.array_equal(run(0, 0), group) and np.array_equal(run(0, 4096), group)
+
+
+def test_portions_are_cut_by_their_own_context(rt):
+    """Fresh rows beside a decoded request of 3,840 keys: with their own context given, the bits that they have alone."""
+    kern = rt.kernels("bfloat16")
+    H, G, D, rows, far, bs = 16, 8, 128, 300, 3840, 16
+    rng, blocks = np.random.default_rng(7), far // bs
+    args = [up(rt, rng.normal(size=s)) for s in ((rows + 1, H * D), (blocks + 19, G, bs, D), (blocks + 19, G, D, bs))]
+    table = np.full((2, blocks), -1)
+    table[0, :19], table[1] = np.arange(19), 19 + np.arange(blocks)
+    args += [rt.upload(np.array(x, np.int32), "int32") for x in (table, [0, rows, rows + 1], [rows, far])]
+    n_ws = kern.zk_attention_bf16_portion_workspace(rows + 128, H, G, D) + kern.zk_attention_bf16_workspace(1, H, D, far) + 1024
+    ws = rt.zeros((int(n_ws) // 4,), "float32")
+
+    def run(R, max_ctx, portion_ctx):
+        out = rt.zeros((rows + 1, H * D), "bfloat16")
+        kern.zk_attention_bf16_step(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, blocks, args[4].ptr, args[5].ptr, out.ptr, R, 1,
+                                    rows, max_ctx, H, G, D, bs, D ** -0.5, 50.0, 0, 0, ws.ptr, ws.nbytes, 0, 0, 0, 0, D, 0, None, None, 0,
+                                    portion_ctx, rt.stream)
+        return rt.download(out)
+    alone, beside, unknown = run(1, rows, 0), run(2, far, rows), run(2, far, 0)
+    assert np.array_equal(beside[:rows], alone[:rows])
+    assert not np.array_equal(unknown[:rows], alone[:rows])         # ranges, by a context that is not theirs
+    assert np.array_equal(beside[rows:], unknown[rows:]) and beside[rows:].any()
+
+
+def test_the_runner_tells_portions_contexts_from_decoded_ones(rt, monkeypatch, tmp_path):
+    from conftest import TINY
+    from gpu_util import make_runner
+    from zse_amd.engine.runner import StepEntry, StepRunner
+    from zse_amd.weights import write_random_model
+    name = sorted(TINY)[0]
+    write_random_model(str(tmp_path), TINY[name][0], seed=1, dtype="bfloat16")
+    runner = make_runner(str(tmp_path), "bfloat16", page_size=16, cache_tokens=2048, max_seqs=3, max_batch_tokens=700, max_model_len=1024)
+    seen, forward = [], StepRunner._forward
+    monkeypatch.setattr(StepRunner, "_forward", lambda self, ctx, *a, **k: (seen.append((ctx.n_multi, ctx.max_ctx, ctx.portion_ctx)),
+                                                                           forward(self, ctx, *a, **k))[1])
+    for r in "abc":
+        runner.add(r)
+    runner.step([StepEntry("a", [1] * 600, [])])
+    runner.step([StepEntry("a", [2], [0]), StepEntry("b", [3] * 40, [39])])
+    runner.step([StepEntry("a", [2], [0]), StepEntry("b", [3] * 300, [0]), StepEntry("c", [3] * 5, [0])])
+    runner.step([StepEntry("a", [2], [0]), StepEntry("b", [3], [0])])
+    assert seen == [(1, 768, 768), (1, 768, 256), (2, 768, 512), (0, 768, 0)]

@@ -4,13 +4,13 @@ import ctypes as C
 import pytest
 
 
-def form_of(room, R, rows, ctx, H, G, D, E=0, bs=16, window=0, chunk=0, keep=0, wide_weights=0):
+def form_of(room, R, rows, ctx, H, G, D, E=0, bs=16, window=0, chunk=0, keep=0, wide_weights=0, not_theirs=0):
     """(groups of rows a block, or 5 for four with the keys in ranges; tiles of a range; by attn_stream_kernel)"""
     from zse_amd.runtime import build
     lib = C.CDLL(build.ensure("kernels_bf16"))
     ranges, stream = C.c_int(-1), C.c_int(-1)
-    form = lib.zk_attention_bf16_portion_form(R, rows, ctx, H, G, D, E or D, bs, window, chunk, keep, wide_weights, C.c_size_t(room),
-                                              C.byref(ranges), C.byref(stream))
+    form = lib.zk_attention_bf16_portion_form(R, rows, ctx, not_theirs, H, G, D, E or D, bs, window, chunk, keep, wide_weights,
+                                              C.c_size_t(room), C.byref(ranges), C.byref(stream))
     return form, ranges.value, stream.value
 
 
@@ -40,3 +40,10 @@ def test_launches_that_a_form_with_fewer_blocks_runs_faster(case, form):
     """Two ranges a block of rows lie on halves of the chip that have unlike work, and a block of four groups that has rows for
     one is slower than a group a block (94 us against 70, 80 against 61, 98 against 81, 12.4 against 10.5 twice)."""
     assert form_of(1 << 30, *case)[0] == form
+
+
+@pytest.mark.parametrize("R,rows,H,G,D", [(8, 128, 32, 16, 128), (4, 512, 16, 4, 128), (1, 2048, 16, 4, 128), (1, 1024, 32, 16, 128)])
+def test_many_groups_beside_a_long_decoded_context(R, rows, H, G, D):
+    """A context that may be a decoded request's does not cut the keys of many groups into ranges."""
+    assert form_of(1 << 30, R, rows, 8192, H, G, D)[0] == 5
+    assert form_of(1 << 30, R, rows, 8192, H, G, D, not_theirs=1)[0] == 4

@@ -308,13 +308,14 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
 static int portion_kernel_mode = 0;
 
 // How a launch of portions runs: which kernel, and with ranges the tiles of one and the most that a
-// block of rows has.  ``room``: bytes of workspace for the ranges' partial results.
+// block of rows has.  ``max_ctx``: the portions' longest context, or (not_theirs) that of all requests of the step, decoded ones
+// among them.  ``room``: bytes of workspace for the ranges' partial results.
 struct PortionForm {
   AttnWhat what;
   int range_tiles, most_ranges;
 };
-static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, int nh, int nkv, int hd, int vd, int bs, int window,
-                                int mask_chunk, int keep, int wide_weights, size_t room) {
+static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, bool not_theirs, int nh, int nkv, int hd, int vd, int bs,
+                                int window, int mask_chunk, int keep, int wide_weights, size_t room) {
   const int tpw = 32 / (nh / nkv), per_block = 4 * tpw, wide = std::max(hd, vd), groups = (max_q_len + tpw - 1) / tpw;
   const bool stream = stream_takes(hd, vd, bs, wide_weights);
   // one block a group; two groups a block when that lets every block run at once (256 CUs,
@@ -349,6 +350,9 @@ static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, int n
     if (stream) {
       const PortionPlan plan = portion_plan(max_q_len, max_ctx, window, mask_chunk, keep, tpw, nkv, r_prefill, bound, wide);
       range_tiles = portion_kernel_mode == 5 || plan.kind == 5 ? plan.ranges : 0;
+      // Many groups priced by a context that may be another's: no ranges (8 times 128 fresh rows beside 3,840 keys, 32 heads over 16
+      // of 128: 26 us, 13 without; 3,584 rows beside 8,192, 16 over 4: 176 and 91).  Few groups do gain from them where the context is theirs.
+      if (not_theirs && single >= 768 && portion_kernel_mode == 0) range_tiles = 0;
       shared_waves = std::max(shared_waves, plan.whole);       // without ranges, also where the workspace does not hold them
     } else {
       range_tiles = portion_ranges(max_q_len, max_ctx, window, mask_chunk, keep, per_block, nkv, r_prefill, bound);
@@ -374,9 +378,9 @@ int zk_attention_bf16_portion_kernel(int mode) {
 // Which form a launch of ``r_prefill`` portions takes with ``room`` bytes of workspace behind the decoded tokens' part: 1, 2, 4 or 8
 // groups of rows a block, or 5, four with the keys in ranges of *range_tiles tiles.  *stream: by attn_stream_kernel.  For tests that mean
 // to reach each of them.
-int zk_attention_bf16_portion_form(int r_prefill, int max_q_len, int max_ctx, int nh, int nkv, int hd, int vd, int bs, int window,
-                                   int mask_chunk, int keep, int wide_weights, size_t room, int* range_tiles, int* stream) {
-  const PortionForm f = portion_form(r_prefill, max_q_len, max_ctx, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights, room);
+int zk_attention_bf16_portion_form(int r_prefill, int max_q_len, int max_ctx, int not_theirs, int nh, int nkv, int hd, int vd, int bs,
+                                   int window, int mask_chunk, int keep, int wide_weights, size_t room, int* range_tiles, int* stream) {
+  const PortionForm f = portion_form(r_prefill, max_q_len, max_ctx, not_theirs, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights, room);
   *range_tiles = f.range_tiles;
   *stream = (f.what == ATT_SHARED4 || f.what == ATT_RANGES) && stream_takes(hd, vd, bs, wide_weights);
   return f.what == ATT_RANGES ? 5 : f.what == ATT_SHARED8 ? 8 : f.what == ATT_SHARED4 ? 4 : f.what == ATT_PAIRS ? 2 : 1;
@@ -453,13 +457,15 @@ long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chun
 // beside its window; the caller keeps their pages.
 // sinks (may be null; not together with ``sink``): float [nh], exp(sinks[h]) joins head h's denominators.
 // gate (may be null): bf16, row t's nh numbers at gate + t * gate_ld; head h's output times sigmoid of the h-th.
-int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, const void* vcache_t,
+// portion_ctx: the longest context among the portions, whose kernel it chooses (0: not known, max_ctx stands for it).
+int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, const void* vcache_t,
                            const int* block_table, int max_blocks, const int* q_start, const int* ctx_len,
                            void* out, int R, int r_prefill, int max_q_len, int max_ctx, int nh, int nkv,
                            int hd, int bs, float scale, float softcap, int window, int decode_chunk,
                            void* workspace, size_t workspace_bytes, int mask_chunk, int sink, int wide_weights,
                            int v_shift, int vd, int keep, const float* sinks, const void* gate, int gate_ld,
-                           void* stream) {
+                           int portion_ctx, void* stream) {
+  ZK_REQUIRE(portion_ctx >= 0, "zk_attention_bf16: bad context of the portions");
   ZK_REQUIRE(!sink || sinks == nullptr, "zk_attention_bf16: a unit sink or learned sinks, not both");
   ZK_REQUIRE(gate == nullptr || gate_ld >= nh, "zk_attention_bf16: gate rows hold a number per head");
   ZK_REQUIRE(keep >= 0 && (keep == 0 || window > 0), "zk_attention_bf16: first keys are kept beside a window");
@@ -508,8 +514,8 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
     size_t split_at = 0;
     if (R - r_prefill > 0) split_at = (zk_attention_bf16_workspace(R - r_prefill, nh, vd, max_ctx) + 255) / 256 * 256;
     const bool usable = workspace != nullptr && (uintptr_t)workspace % 16 == 0 && split_at < workspace_bytes;
-    const PortionForm form = portion_form(r_prefill, max_q_len, max_ctx, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights,
-                                          usable ? workspace_bytes - split_at : 0);
+    const PortionForm form = portion_form(r_prefill, max_q_len, portion_ctx ? portion_ctx : max_ctx, !portion_ctx && R > r_prefill, nh, nkv,
+                                          hd, vd, bs, window, mask_chunk, keep, wide_weights, usable ? workspace_bytes - split_at : 0);
     int rc;
     if (form.what == ATT_RANGES) {
       const int per_block = 4 * p.tpw, most_ranges = form.most_ranges;
@@ -570,6 +576,19 @@ int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, con
   return 0;
 }
 
+int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, const void* vcache_t,
+                           const int* block_table, int max_blocks, const int* q_start, const int* ctx_len,
+                           void* out, int R, int r_prefill, int max_q_len, int max_ctx, int nh, int nkv,
+                           int hd, int bs, float scale, float softcap, int window, int decode_chunk,
+                           void* workspace, size_t workspace_bytes, int mask_chunk, int sink, int wide_weights,
+                           int v_shift, int vd, int keep, const float* sinks, const void* gate, int gate_ld,
+                           void* stream) {
+  return zk_attention_bf16_step(q, q_stride, kcache, vcache_t, block_table, max_blocks, q_start, ctx_len, out, R,
+                                r_prefill, max_q_len, max_ctx, nh, nkv, hd, bs, scale, softcap, window, decode_chunk,
+                                workspace, workspace_bytes, mask_chunk, sink, wide_weights, v_shift, vd, keep, sinks, gate,
+                                gate_ld, 0, stream);
+}
+
 int zk_attention_bf16_sized(const void* q, int q_stride, const void* kcache, const void* vcache_t,
                            const int* block_table, int max_blocks, const int* q_start, const int* ctx_len,
                            void* out, int R, int r_prefill, int max_q_len, int max_ctx, int nh, int nkv,
@@ -620,6 +639,10 @@ extern "C" int zk_steplist_register(const char* name, int nargs, void* fn);
 static const int zk_attention_bf16_masked_entered = zk_steplist_register(
     "zk_attention_bf16_masked", zk_packed::Call<zk_attention_bf16_masked>::nargs,
     (void*)zk_packed::Call<zk_attention_bf16_masked>::call);
+
+static const int zk_attention_bf16_step_entered = zk_steplist_register(
+    "zk_attention_bf16_step", zk_packed::Call<zk_attention_bf16_step>::nargs,
+    (void*)zk_packed::Call<zk_attention_bf16_step>::call);
 
 static const int zk_attention_bf16_gated_entered = zk_steplist_register(
     "zk_attention_bf16_gated", zk_packed::Call<zk_attention_bf16_gated>::nargs,

@@ -116,6 +116,7 @@ class StepContext:
         self.groups: List[GroupView] = []
         self.max_q_len = 0
         self.max_ctx = 0
+        self.portion_ctx = 0         # the longest context among requests [0, n_multi) (0: not known)
         self.n_multi = 0             # requests [0, n_multi) of the batch bring more than one token
         self.entries: List[Tuple[object, int, int, int]] = []   # (req, slot, start, n) on the host
         self.state = None            # Tensor uint8-as-float32 words [max_seqs, slot_words] or None
@@ -376,7 +377,7 @@ class StepRunner:
         t = 0
         host_entries = []
         first_token = [0] * R
-        max_q = max_ctx = 0
+        max_q = max_ctx = portion_ctx = 0
         for r, i in enumerate(order):
             e = entries[i]
             n = len(e.tokens)
@@ -401,12 +402,14 @@ class StepRunner:
             first_token[i] = t
             host_entries.append((e.req, m.slot(e.req), start, n))
             max_q, max_ctx = max(max_q, n), max(max_ctx, start + n)
+            if n > 1:
+                portion_ctx = max(portion_ctx, start + n)
             t += n
-        # The two maxima only size the attention kernels' grids (a block past a request's own
-        # rows or keys ends at once); rounded up, steps of many lengths share one launch list.
+        # The maxima only size the attention kernels' grids and choose the portions' kernel (a block past a
+        # request's own rows or keys ends at once); rounded up, steps of many lengths share one launch list.
         if max_q > 1:
             max_q = -(-max_q // 32) * 32
-        max_ctx = min(-(-max_ctx // 256) * 256, max(self.max_model_len, max_ctx))
+        max_ctx, portion_ctx = (min(-(-c // 256) * 256, max(self.max_model_len, c)) for c in (max_ctx, portion_ctx))
         n_rows = 0
         for i, e in enumerate(entries):
             for w in e.want:
@@ -427,9 +430,9 @@ class StepRunner:
         slot_of_req[R:] = 0
         for g in range(G):
             tables[g][R:] = -1
-        return off, cur, T, R, n_rows, host_entries, max_q, max_ctx, n_multi
+        return off, cur, T, R, n_rows, host_entries, max_q, max_ctx, portion_ctx, n_multi
 
-    def _context(self, off, T_pad, R_pad, host_entries, max_q, max_ctx, n_multi) -> StepContext:
+    def _context(self, off, T_pad, R_pad, host_entries, max_q, max_ctx, portion_ctx, n_multi) -> StepContext:
         ctx = StepContext(self)
         base = self.meta_dev.ptr
         p = lambda name: base + off[name] * 4
@@ -440,7 +443,7 @@ class StepRunner:
         ctx.groups = [GroupView(p(f"table{g}"), self.max_blocks, p(f"slot_map{g}"), self.page_size)
                       for g in range(len(self.manager.groups))]
         ctx.entries = host_entries
-        ctx.max_q_len, ctx.max_ctx, ctx.n_multi = max_q, max_ctx, n_multi
+        ctx.max_q_len, ctx.max_ctx, ctx.portion_ctx, ctx.n_multi = max_q, max_ctx, portion_ctx, n_multi
         ctx.state, ctx.slot_bytes = self.state, self.slot_bytes
         ctx.embedding_state = self.embedding_state
         return ctx
@@ -514,7 +517,7 @@ class StepRunner:
         attention kernels' grids; a block past a request's keys ends at once, but a grid of
         mostly such blocks still costs time.)"""
         R = len(entries)
-        off, words, T, _, n_rows, host_entries, _, longest, _ = self._pack(entries, bucket, bucket, feed)
+        off, words, T, _, n_rows, host_entries, _, longest, _, _ = self._pack(entries, bucket, bucket, feed)
         grain = 1024
         while grain * 8 < self.max_model_len:
             grain *= 2
@@ -540,7 +543,7 @@ class StepRunner:
             self.rt.graph_launch(graph)
             self.graph_runs += 1
             return result()
-        ctx = self._context(off, bucket, bucket, host_entries, 1, covered, 0)
+        ctx = self._context(off, bucket, bucket, host_entries, 1, covered, 0, 0)
         self.arena.reset()
         warm = bucket if mode == "logits" else (bucket, mode)
         if warm not in self.graphs:             # first time: eager, lets the arena grow
@@ -680,21 +683,21 @@ class StepRunner:
         if bucket:
             out = self._graph_step(entries, bucket, tokens_from, pick, feed)
         else:
-            off, words, T, R, n_rows, host_entries, max_q, max_ctx, n_multi = self._pack(entries, T, R, feed)
+            off, words, T, R, n_rows, host_entries, max_q, max_ctx, portion_ctx, n_multi = self._pack(entries, T, R, feed)
             picks = self._pick_buffers(n_rows) if pick and n_rows else None
             if picks is None:
                 self._ensure_logits(n_rows)
             self.rt.copy_h2d_async(self.meta_dev.ptr, self.meta_host.ptr, words * 4)
             self.rt.record(self.meta_copied)
             self._feed(off, tokens_from, R, feed is None)
-            ctx = self._context(off, T, R, host_entries, max_q, max_ctx, n_multi)
+            ctx = self._context(off, T, R, host_entries, max_q, max_ctx, portion_ctx, n_multi)
             self.arena.reset()
             if picks is not None:
-                self._forward(ctx, n_rows, None, (T, R, n_rows, n_multi, max_q, max_ctx, "pick", picks[0].ptr), pick=picks)
+                self._forward(ctx, n_rows, None, (T, R, n_rows, n_multi, max_q, max_ctx, portion_ctx, "pick", picks[0].ptr), pick=picks)
                 out = self.pick_ids.rows(0, n_rows)
             else:
                 out = self.logits.rows(0, n_rows)
-                self._forward(ctx, n_rows, out, (T, R, n_rows, n_multi, max_q, max_ctx, out.ptr))
+                self._forward(ctx, n_rows, out, (T, R, n_rows, n_multi, max_q, max_ctx, portion_ctx, out.ptr))
                 if pick:
                     out = self._argmax_of(out, n_rows)
         for e in entries:
