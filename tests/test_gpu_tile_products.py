@@ -127,7 +127,7 @@ def test_every_way_out(rt, epi, K, M, N, extra, f32):
     assert (got[M:] == 3.0).all() and (got[:, N:] == 3.0).all()
 
 
-def test_the_static_array_takes_another_cut_where_its_sums_do_not_fit(rt):
+def test_the_static_array_where_its_sums_do_not_fit(rt):
     """535 x 2304 x 9216: ranges of K whose sums are more than the array's 16 MiB."""
     M, N, K = 535, 2304, 9216
     assert cut_of(0, 0, M, N, K)[1] * M * N * 4 > 16 << 20
@@ -140,3 +140,50 @@ def test_the_static_array_takes_another_cut_where_its_sums_do_not_fit(rt):
     assert dll.zk_gemm_bf16_static(A.ptr, K, S.ptr, out.ptr, N, 0, M, N, K, 0, 0.0, 1, rt.stream) == 0
     got = rt.download_f32(out)
     assert (np.abs(got - want) <= np.abs(want) * 2.0 ** -8 + 1e-4).all()
+
+
+STATIC = [
+    # rows, columns, K, gated: ranges of K, of the last round's tiles, whose sums are more than the static array's 16 MiB
+    (535, 2304, 9216, 0), (526, 4099, 4608, 0), (412, 3072, 4608, 1), (583, 2304, 4608, 1), (184, 2304, 18432, 1),
+    (2179, 4096, 3072, 0), (583, 8208, 3072, 1), (3604, 2304, 3072, 1), (2863, 3072, 3072, 0),
+]
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("M,N,K,gated", STATIC)
+def test_the_static_array_gives_the_bits_of_the_workspace_also_where_the_sums_do_not_fit(rt, M, N, K, gated, f32):
+    from zse_amd.runtime import build
+    shape, ks, tail_ks, _ = cut_of(gated, 0, M, N, K)
+    assert ks > 1 or tail_ks > 1
+    if ks > 1:
+        assert ks * (1 + gated) * M * -(-N // 16) * 16 * 4 > 16 << 20
+    kern, epi, ld = rt.kernels("bfloat16"), 3 if gated else 0, N + 5
+    A, S = rt.empty((M, K), "bfloat16"), rt.empty((-(-N * (1 + gated) // 16) * 16, K), "bfloat16")
+    for t, seed in ((A, 1), (S, 2)):
+        kern.zk_fill_normal(t.ptr, 1, t.numel, seed, 1, 0.0, K ** -0.25, rt.stream)
+    dll = C.CDLL(build.lib_path("kernels_bf16"))
+    VP, I, F = C.c_void_p, C.c_int, C.c_float
+    dll.zk_gemm_bf16_static.argtypes = [VP, I, VP, VP, I, I, I, I, I, I, F, I, VP]
+    got, want = (rt.upload(np.full((M, ld), 3.0, np.float32) if f32 else np.full((M, ld), 0x4040, np.uint16), "float32" if f32 else "bfloat16")
+                 for _ in range(2))
+    ws = workspace(rt)
+    kern.zk_gemm_bf16(A.ptr, K, S.ptr, want.ptr, ld, f32, M, N, K, epi, 0.0, 1, ws.ptr, ws.nbytes, None, rt.stream)
+    assert dll.zk_gemm_bf16_static(A.ptr, K, S.ptr, got.ptr, ld, f32, M, N, K, epi, 0.0, 1, rt.stream) == 0
+    got, want = rt.download(got), rt.download(want)
+    assert (want[:, :N] != 0).any() and (want[:, N:] == (3.0 if f32 else 0x4040)).all()
+    assert np.array_equal(got, want)
+
+
+def test_what_the_static_array_refuses_of_weights_in_strips(rt):
+    """The shapes that it refused of them before they had tiles of their own: those of weights that lie row by row."""
+    from zse_amd.runtime import build
+    M, N, K = 1024, 1024, 65536
+    A, S, out = rt.zeros((M, K), "bfloat16"), rt.zeros((N, K), "bfloat16"), rt.zeros((M, N), "bfloat16")
+    dll = C.CDLL(build.lib_path("kernels_bf16"))
+    VP, I, F = C.c_void_p, C.c_int, C.c_float
+    dll.zk_gemm_bf16_static.argtypes = [VP, I, VP, VP, I, I, I, I, I, I, F, I, VP]
+    dll.zk_last_error.restype = C.c_char_p
+    for strip in (0, 1):
+        assert dll.zk_gemm_bf16_static(A.ptr, K, S.ptr, out.ptr, N, 0, M, N, K, 0, 0.0, strip, rt.stream) != 0
+        assert b"static scratch array holds 16777216" in dll.zk_last_error()
+    rt.sync()

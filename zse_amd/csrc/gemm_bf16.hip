@@ -1406,15 +1406,12 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
   if (w_strip && K % 64 == 0 && lda <= (1 << 22)) {
     const bool aligned = wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 16 == 0;
     const bool by_reader = parts != nullptr && joinable_by_reader(N, ldc, c_is_f32, epi);
-    TileCut cut = tile_cut(gated, by_reader, M, N, K, aligned ? wsp.split_bytes() : 0);
-    if (wsp.strict) {
-      // sums that the caller's array does not hold: another cut (what the array is refused for
-      // stays what it was before the tiles had other shapes)
+    const TileCut cut = tile_cut(gated, by_reader, M, N, K, aligned ? wsp.split_bytes() : 0);
+    // (what the static array is refused for stays what it was before the tiles had other shapes)
+    if (wsp.strict)
       if (const size_t need = staged_sums(M, N, K, gated, wsp)) return wsp.too_small(need);
-      if (max(tile_sums(gated, M, N, cut.ks), tail_sums(cut.shape, cut_tail(cut, gated, M, N), cut.tail_ks)) > wsp.bytes) cut = tile_cut(gated, by_reader, M, N, K, wsp.bytes);
-    }
     const TileProduct p{A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap};
-    return launch_cut(cut, gated, p, (float*)wsp.ptr, parts, s);
+    return launch_cut(cut, gated, p, (float*)wsp.ptr, wsp.bytes, parts, s);
   }
   const bool exact = K % GT_BK == 0;
   const size_t room = (wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 64 == 0) ? wsp.split_bytes() : 0;

@@ -19,9 +19,8 @@
 //    32768 columns: 64 x 32768 floats, twice that with a gate, are the array's 16 MiB);
 //    products of more rows that split K fit while (tiles) x (ranges of K) x (4 bytes a tile
 //    element) stays within the array, the tiles being those of weights that lie row by row.
-//  * One exception to the same split: more than 64 rows by weights in strip layout, K a multiple of 64, where
-//    the standard workspace allows ranges whose sums the array does not hold.  Such a product
-//    is cut as the array's size allows, and its sums are added in another order.
+//  * More than 64 rows by weights in strip layout, K a multiple of 64: where the array does not hold the sums
+//    of the standard workspace's ranges, the product is made a few tiles at a time, with the same ranges.
 //  * Every call on a GPU shares that GPU's array, which keeps the last call's contents.
 //    Nothing in it has to start at zero (each plane of partial sums is written in full before
 //    it is read, within one call), so calls need no clearing between them; but two calls

@@ -6,10 +6,11 @@
 #define ZK_LDS_AS __attribute__((address_space(3)))
 
 // How the tiles of a launch are dealt to blocks.  The first ``whole`` tiles in K ranges
-// ``ks``, the rest (a last round that would leave most CUs idle) in ``tail_ks`` ranges, all in
-// one grid.  ``gm``: rows of tiles of a group (tile_at).  ``col0``: the launch's first column.
+// ``ks``, and ``tail`` tiles from the ``from``-th on (a last round that would leave most CUs idle) in
+// ``tail_ks`` ranges, all in one grid.  ``gm``: rows of tiles of a group (tile_at).  ``col0``, ``cols``: the
+// launch's columns.
 struct TileGrid {
-  int tiles_m, tiles_n, gm, whole, ks, tail_ks, col0;
+  int tiles_m, tiles_n, gm, whole, ks, from, tail, tail_ks, col0, cols;
 };
 
 // Blocks go round-robin over the 8 XCDs by their number; this gives each XCD a run of
@@ -95,11 +96,10 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
   extern __shared__ __align__(16) unsigned char gd_lds[];
   const int first = g.whole * g.ks;
   const bool tail = (int)blockIdx.x >= first;
-  const int tiles = g.tiles_m * g.tiles_n;
-  const int ks = tail ? g.tail_ks : g.ks, part_tiles = tail ? tiles - g.whole : g.whole;
+  const int ks = tail ? g.tail_ks : g.ks, part_tiles = tail ? g.tail : g.whole;
   const int place = tail ? xcd_run(blockIdx.x - first, part_tiles * ks) : xcd_run(blockIdx.x, first);
   const int range = place / part_tiles;
-  const int tile = place - range * part_tiles + (tail ? g.whole : 0);
+  const int tile = place - range * part_tiles + (tail ? g.from : 0);
   int tm, tn;
   tile_at(tile, g, tm, tn);
   const int m0 = tm * BM, n0 = g.col0 + tn * OC;
@@ -220,12 +220,12 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
   __syncthreads();                              // the buffers are free for the results' way out
   const int wc = wn * (GATED ? TN / 2 : TN) * 32;        // the wave's first column in the tile
   if (ks > 1) {
-    // The range's partial sums in planes (range, gate or up).  Every tile split: planes of [M, N
-    // rounded up to 16]; the tail alone: of [tail tile, BM, OC].
-    const int npad = (N + 15) / 16 * 16, ld = tail ? OC : npad;
-    const size_t plane = tail ? (size_t)(tiles - g.whole) * BM * OC : (size_t)M * npad;
+    // The range's partial sums in planes (range, gate or up).  Every tile split: planes of [M, the launch's
+    // columns rounded up to 16]; the tail alone: of [tail tile, BM, OC].
+    const int npad = (g.cols + 15) / 16 * 16, ld = tail ? OC : npad;
+    const size_t plane = tail ? (size_t)g.tail * BM * OC : (size_t)M * npad;
     float* mine = partials + (size_t)range * NG * plane +
-                  (tail ? (size_t)(tile - g.whole) * BM * OC : (size_t)m0 * npad + n0);
+                  (tail ? (size_t)(tile - g.from) * BM * OC : (size_t)m0 * npad + n0 - g.col0);
 #pragma unroll
     for (int i = 0; i < TM; i++) {
       const int row = wm * 32 * TM + i * 32 + lr;
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(64 * NWM * NWN, MB) void gemm_tile_direct_kernel(
         const int gate = GATED && j >= TN / 2 ? 1 : 0, col = wc + (j - gate * (TN / 2)) * 32 + 4 * lk;
 #pragma unroll
         for (int b = 0; b < 4; b++)
-          if (tail || n0 + col + 8 * b < npad)
+          if (tail || n0 - g.col0 + col + 8 * b < npad)
             *(f32x4*)(mine + gate * plane + (size_t)row * ld + col + 8 * b) =
                 f32x4{acc[i][j][4 * b], acc[i][j][4 * b + 1], acc[i][j][4 * b + 2], acc[i][j][4 * b + 3]};
       }
@@ -319,10 +319,10 @@ __global__ __launch_bounds__(256) void gemm_tail_join_kernel(const float* __rest
   const int idx = blockIdx.x * 256 + threadIdx.x, t = idx / quads, in = idx - t * quads;
   const int row = in / (OC / 4), col = in % (OC / 4) * 4;
   int tm, tn;
-  tile_at(g.whole + t, g, tm, tn);
+  tile_at(g.from + t, g, tm, tn);
   const int m = tm * BM + row, n = tn * OC + col;
   if (m >= M || n >= N) return;
-  const size_t plane = (size_t)(g.tiles_m * g.tiles_n - g.whole) * BM * OC;
+  const size_t plane = (size_t)g.tail * BM * OC;
   const float* at = partials + (size_t)t * BM * OC + (size_t)row * OC + col;
   f32x4 x = *(const f32x4*)at, y = x;
   if (GATED) y = *(const f32x4*)(at + plane);
@@ -384,8 +384,9 @@ static size_t tail_sums(int v, int tail, int ks) {
   return ks > 1 ? (size_t)ks * tail * tile_shapes[v].bm * tile_shapes[v].bn * sizeof(float) : 0;
 }
 
+// ``room``: the bytes that the last round's partial sums may take; where they take more, its tiles go a few at a time.
 template <int TM, int TN, int NWM, int NWN, int NSA, int NSB, int MB, bool GATED>
-static int launch_direct(const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, int* parts, hipStream_t s) {
+static int launch_direct(const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, size_t room, int* parts, hipStream_t s) {
   constexpr int BM = 32 * TM * NWM, BN = 32 * TN * NWN, OC = GATED ? BN / 2 : BN;
   constexpr size_t lds = (size_t)(NSA * BM + NSB * BN) * 128;
   static_assert(lds * MB <= 160 * 1024, "the blocks of a CU do not fit its LDS");
@@ -403,24 +404,31 @@ static int launch_direct(const TileProduct& p, int col0, int cols, int ks, int t
   ZK_REQUIRE((long long)g.tiles_m * g.tiles_n * max(ks, tail_ks) < 2147483647LL, "zk_gemm_bf16: too many tiles");
   g.gm = tile_group(g.tiles_m);
   const int tiles = g.tiles_m * g.tiles_n, tail = tail_ks > 1 ? tiles % (256 * MB) : 0;
-  g.whole = tiles - tail;
+  const int most = (int)min((size_t)tail, max(room / ((size_t)tail_ks * BM * BN * sizeof(float)), (size_t)1));
+  g.whole = g.from = tiles - tail;
   g.ks = ks;
   g.tail_ks = max(tail_ks, 1);
   g.col0 = col0;
-  kernel<<<g.whole * ks + tail * g.tail_ks, 64 * NWM * NWN, lds, s>>>(
-      (const __bf16*)p.A, p.lda, (const __bf16*)p.W, p.C, p.ldc, p.c_is_f32, p.M, p.N, p.K, p.epi, p.cap, sums, g);
+  g.cols = cols;
+  do {
+    g.tail = min(most, tiles - g.from);
+    kernel<<<g.whole * ks + g.tail * g.tail_ks, 64 * NWM * NWN, lds, s>>>(
+        (const __bf16*)p.A, p.lda, (const __bf16*)p.W, p.C, p.ldc, p.c_is_f32, p.M, p.N, p.K, p.epi, p.cap, sums, g);
+    if (g.tail > 0)
+      gemm_tail_join_kernel<GATED><<<g.tail * (BM * OC / 1024), 256, 0, s>>>(sums, p.C, p.ldc, p.c_is_f32, p.M, p.N, p.epi, p.cap,
+                                                                             g, BM, OC);
+    g.whole = 0;
+    g.from += g.tail;
+  } while (g.from < tiles);
   if (ks > 1) {
     if (parts && joinable_by_reader(p.N, p.ldc, p.c_is_f32, p.epi)) {
       *parts = ks;
     } else {
-      const int npad = (p.N + 15) / 16 * 16;
+      const int npad = (cols + 15) / 16 * 16;
       const size_t quads = (size_t)p.M * (npad / 4);
-      gemm_join_kernel<GATED><<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(sums, ks, p.C, p.ldc, p.c_is_f32, p.M, p.N, npad,
-                                                                            p.epi, p.cap);
+      gemm_join_kernel<GATED><<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(sums, ks, (char*)p.C + (size_t)col0 * (p.c_is_f32 ? 4 : 2), p.ldc,
+                                                                            p.c_is_f32, p.M, cols, npad, p.epi, p.cap);
     }
-  } else if (tail > 0) {
-    gemm_tail_join_kernel<GATED><<<tail * (BM * OC / 1024), 256, 0, s>>>(sums, p.C, p.ldc, p.c_is_f32, p.M, p.N, p.epi, p.cap, g,
-                                                                         BM, OC);
   }
   return zk_launch_status("zk_gemm_bf16 (tile)");
 }
@@ -487,13 +495,6 @@ static double tile_time(const TileCut& c, bool gated, bool by_reader, int M, int
   return time;
 }
 
-// Tiles of a cut's last round.
-static int cut_tail(const TileCut& c, bool gated, int M, int N) {
-  const TileShape& t = tile_shapes[c.shape];
-  const int oc = gated ? t.bn / 2 : t.bn;
-  return (int)((long)((M + t.bm - 1) / t.bm) * ((N + oc - 1) / oc) % (256 * t.blocks));
-}
-
 static TileCut tile_cut(bool gated, bool by_reader, int M, int N, int K, size_t room) {
   static const int splits[] = {2, 3, 4, 5, 6, 8};
   TileCut best{0, 1, 1, -1};
@@ -522,22 +523,34 @@ static TileCut tile_cut(bool gated, bool by_reader, int M, int N, int K, size_t 
   return best;
 }
 
-static int launch_columns(int v, bool gated, const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, int* parts,
-                          hipStream_t s) {
+static int launch_columns(int v, bool gated, const TileProduct& p, int col0, int cols, int ks, int tail_ks, float* sums, size_t room,
+                          int* parts, hipStream_t s) {
   switch (v) {
 #define ZK_SHAPE(V, TM, TN, NWM, NWN, NSA, NSB, MB, START, STEP, STEP2)                                                       \
   case V:                                                                                           \
-    return gated ? launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, true>(p, col0, cols, ks, tail_ks, sums, parts, s)    \
-                 : launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, false>(p, col0, cols, ks, tail_ks, sums, parts, s);
+    return gated ? launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, true>(p, col0, cols, ks, tail_ks, sums, room, parts, s)    \
+                 : launch_direct<TM, TN, NWM, NWN, NSA, NSB, MB, false>(p, col0, cols, ks, tail_ks, sums, room, parts, s);
     ZK_TILE_SHAPES(ZK_SHAPE)
 #undef ZK_SHAPE
   }
   return zk_fail("zk_gemm_bf16: no such tile");
 }
 
-static int launch_cut(const TileCut& c, bool gated, const TileProduct& p, float* sums, int* parts, hipStream_t s) {
-  if (c.rest < 0) return launch_columns(c.shape, gated, p, 0, p.N, c.ks, c.tail_ks, sums, parts, s);
-  const int cols = whole_columns(c.shape, gated, p.M, p.N);
-  if (int rc = launch_columns(c.shape, gated, p, 0, cols, 1, 1, sums, parts, s)) return rc;
-  return launch_columns(c.rest, gated, p, cols, p.N - cols, 1, 1, sums, parts, s);
+// ``room``: the bytes at ``sums``.  A cut whose partial sums take more is made some columns (or some of the last round's
+// tiles) at a time: the ranges of K, and the order in which an element's sums are added, are those of the whole
+// product, and so are the bits.
+static int launch_cut(const TileCut& c, bool gated, const TileProduct& p, float* sums, size_t room, int* parts, hipStream_t s) {
+  if (c.rest >= 0) {
+    const int cols = whole_columns(c.shape, gated, p.M, p.N);
+    if (int rc = launch_columns(c.shape, gated, p, 0, cols, 1, 1, sums, room, parts, s)) return rc;
+    return launch_columns(c.rest, gated, p, cols, p.N - cols, 1, 1, sums, room, parts, s);
+  }
+  if (tile_sums(gated, p.M, p.N, c.ks) <= room) return launch_columns(c.shape, gated, p, 0, p.N, c.ks, c.tail_ks, sums, room, parts, s);
+  const int oc = gated ? tile_shapes[c.shape].bn / 2 : tile_shapes[c.shape].bn;
+  const int cols = (int)(room / tile_sums(gated, p.M, oc, c.ks)) * oc;
+  // (of 64 cuts whose sums for one tile's columns are more than the static array's 16 MiB, all are refused before)
+  ZK_REQUIRE(cols > 0, "zk_gemm_bf16: no room for the partial sums of one tile's columns");
+  for (int n = 0; n < p.N; n += cols)
+    if (int rc = launch_columns(c.shape, gated, p, n, min(cols, p.N - n), c.ks, 1, sums, room, nullptr, s)) return rc;
+  return 0;
 }
