@@ -5,6 +5,8 @@ tile, and the choice by sizes."""
 import numpy as np
 import pytest
 
+from test_portion_forms import form_of
+
 pytestmark = pytest.mark.gpu
 
 
@@ -52,6 +54,8 @@ CASES = [
     (16, 1, 128, 128, 64, [(3, 70)], 1, 0, 50.0, False),
     (4, 2, 256, 128, 16, [(40, 150)], 0, 0, 50.0, False),
     (4, 2, 128, 256, 32, [(40, 150)], 77, 33, 0.0, False),
+    (4, 2, 256, 128, 16, [(231, 190)], 0, 0, 50.0, False),                # uneven heads in ranges
+    (4, 2, 128, 256, 32, [(700, 150)], 300, 33, 0.0, False),
 ]
 
 
@@ -87,6 +91,11 @@ def test_portions(rt, case, mode):
             rt.upload(np.array(ctx, np.int32), "int32")]
     before = kern.zk_attention_bf16_portion_kernel(mode)
     try:
+        form, tiles, stream = form_of(ws.nbytes, R, max(fresh), max(ctx), H, G, D, E, bs, window, 0, keep)
+        if mode:
+            # the longest block's tiles: ranges of at least four, two of them or more
+            reach = min(max(ctx), window + 4 * (32 // (H // G)) - 1 if window else max(ctx))
+            assert stream and form == (5 if mode == 5 and reach >= 8 * 32 else 4) and (form != 5 or tiles >= 4)
         kern.zk_attention_bf16_sized(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, blocks, args[4].ptr, args[5].ptr,
                                      out.ptr, R, R, max(fresh), max(ctx), H, G, D, bs, D ** -0.5, cap, window, 0, ws.ptr, ws.nbytes,
                                      0, 0, 0, 0, E, keep, rt.stream)
@@ -228,3 +237,35 @@ def test_the_runner_tells_portions_contexts_from_decoded_ones(rt, monkeypatch, t
     runner.step([StepEntry("a", [2], [0]), StepEntry("b", [3] * 300, [0]), StepEntry("c", [3] * 5, [0])])
     runner.step([StepEntry("a", [2], [0]), StepEntry("b", [3], [0])])
     assert seen == [(1, 768, 768), (1, 768, 256), (2, 768, 512), (0, 768, 0)]
+
+
+@pytest.mark.parametrize("mode", [0, 4, 5])
+@pytest.mark.parametrize("H,G,D,E,shift,before,n", [(8, 4, 128, 128, 1, 100, 300), (8, 8, 256, 256, 2, 0, 333), (16, 4, 128, 256, 1, 37, 290)])
+def test_key_heads_that_share_a_value_head(rt, mode, H, G, D, E, shift, before, n):
+    """2^shift maps of keys over one value head: key head (v << shift) + m serves map m of v's query heads."""
+    kern = rt.kernels("bfloat16")
+    bs, ctx, V, maps = 16, before + n, G >> shift, 1 << shift
+    pages, g = -(-ctx // bs), H // G
+    rng = np.random.default_rng(n)
+    q, k, v = (rounded(rng.normal(size=s)) for s in ((n, H, D), (ctx, G, D), (ctx, V, E)))
+    kc, vc = np.zeros((pages * bs, G, D), np.float32), np.zeros((pages * bs, V, E), np.float32)
+    kc[:ctx], vc[:ctx] = k, v
+    args = [up(rt, q.reshape(n, -1)), up(rt, kc.reshape(pages, bs, G, D).swapaxes(1, 2)), up(rt, vc.reshape(pages, bs, V, E).transpose(0, 2, 3, 1))]
+    args += [rt.upload(np.array(x, np.int32), "int32") for x in ([list(range(pages))], [0, n], [ctx])]
+    out = rt.zeros((n, H * E), "bfloat16")
+    ws = rt.zeros((int(kern.zk_attention_bf16_portion_workspace(n + 128, H, G, E)) // 4 + 64,), "float32")
+    mode_before = kern.zk_attention_bf16_portion_kernel(mode)
+    try:
+        assert mode == 0 or form_of(ws.nbytes, 1, n, ctx, H, G, D, E)[::2] == (mode, 1)
+        kern.zk_attention_bf16_sized(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, pages, args[4].ptr, args[5].ptr, out.ptr,
+                                     1, 1, n, ctx, H, G, D, bs, D ** -0.5, 30.0, 0, 0, ws.ptr, ws.nbytes, 0, 0, 0, shift, E, 0, rt.stream)
+        got = rt.download_f32(out).reshape(n, H, E)
+    finally:
+        kern.zk_attention_bf16_portion_kernel(mode_before)
+    want = np.zeros((n, H, E))
+    for h in range(H):
+        vh, m = (h >> shift) // g, h & (maps - 1)
+        want[:, h] = plain(q[:, h:h + 1].astype(np.float64), k[:, (vh << shift) + m][:, None].astype(np.float64),
+                           v[:, vh][:, None].astype(np.float64), before, D ** -0.5, 30.0, 0, 0)[:, 0]
+    assert np.abs(got - want).max() < 0.03
+    assert np.linalg.norm(got - want) < 4e-3 * np.linalg.norm(want)
