@@ -321,13 +321,14 @@ static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, bool 
   // one block a group; two groups a block when that lets every block run at once (256 CUs,
   // one block each) where single groups would need a second round
   const long long single = (long long)groups * nkv * r_prefill, paired = (long long)((groups + 1) / 2) * nkv * r_prefill;
-  // Many groups: tiles shared by the four or eight groups of a block, where that still gives
+  // Heads of up to 64 channels, pages of 8 keys and wide weights (the others are priced below).  Many groups: tiles
+  // shared by the four or eight groups of a block, where that still gives
   // every CU a block (four) or two (eight; head sizes up to 128, whose registers let two
-  // waves share a SIMD).  Measured at 8 to 32 heads of 128 and 256 with 512 to 8,192 rows:
-  // with fewer than about 768 groups the kernel of one group a block is faster (2,048 rows of
-  // 8 heads of 256, 512 groups: 75 us against 111; 768 groups: a tie), with more the shared
-  // tiles are (8 portions of 512 rows behind 7,680 tokens, 32 heads of 128: 1,630 -> 780 us;
-  // 16 heads of 256: 1,560 -> 845 us; 8,192 rows of 8 heads of 256: 877 -> 463 us).
+  // waves share a SIMD).  Measured with pages of 8 (us, a group a block and four): 8 heads over 4 of 256, 2,048 rows (512
+  // groups) 75 and 112, 3,072 rows (768) 158 and 164, 8,192 rows 878 and 457; 32 over 16 of 128, 512 rows (512) 16 and 25, 1,024
+  // rows (1,024) 55 and 44, 4,096 rows 577 and 246 (eight: 223).  The lines are those of these heads; for heads of 64 they
+  // lie too low: 32 over 8, 1,024 rows (1,024 groups) 27 and 35, 2,048 rows (2,048) 68 and 63, 4,096 rows (4,096) 219 and 159
+  // (eight: 178); 16 over 16, 3,072 rows (1,536) 72 and 93.
   int shared_waves = 0;
   if (bs >= 8 && portion_kernel_mode != 1 && !(stream && portion_kernel_mode == 0)) {
     if (portion_kernel_mode > 1) shared_waves = portion_kernel_mode == 8 ? 8 : 4;
@@ -337,10 +338,9 @@ static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, bool 
   }
   // Few blocks of rows with many keys each (a portion of a few hundred rows behind thousands of
   // tokens): four groups a block and the keys in ranges, where the workspace behind the decoded
-  // tokens' part holds the ranges' partial results.  512 rows behind 3,584 tokens, 8 heads of
-  // 256: 111 -> 52 us; behind 7,680: 209 -> 79 us; 16 heads of 256: 118 -> 76 us; 32 heads of
-  // 128: 100 -> 73 us.  A whole prompt from its first token, 8 heads of 256: 2,048 rows 74 -> 62
-  // us, 1,024 rows the same time either way (its blocks of rows are many and short already).
+  // tokens' part holds the ranges' partial results.  By attn_stream_kernel: portion_plan.  The others, with pages of 8 (us, a
+  // group a block and ranges): 512 rows behind 3,584 tokens, 8 heads over 4 of 256, 110 and 53, behind 7,680 211 and 80; 32
+  // over 16 of 128 92 and 78, 190 and 148; 2,048 rows of 8 heads of 256 from their first token 75 and 61, 1,024 rows 37 and 39.
   if (bs >= 8 && (portion_kernel_mode == 5 || (portion_kernel_mode == 0 && !shared_waves))) {
     // no block of rows has more tiles than this, whatever its request's length
     int bound = (max_ctx + 31) / 32, range_tiles;

@@ -1298,7 +1298,8 @@ static double tile_cost(TileChoice c, int M, int N, int K, bool gated, size_t ro
 }
 
 // Tiles that pass through registers (weights row by row, or K not whole stages): which block, how
-// many ranges of K, of the last round's tiles.
+// many ranges of K, of the last round's tiles.  (The figures are from before weights in strips had tiles of
+// their own: layer shapes, whose weights are in strips, no longer come here.)
 struct StagedCut {
   int variant, ksplit, tail_split;      // 0: 128 x 128, 1: 64 x 128, 2: 128 x 256, 3: 256 x 256
 };

@@ -68,9 +68,9 @@ __device__ __forceinline__ void interleave() {
 // half a line costs as much as a whole one.  Stages of 32 k, whose copies of A are 64-byte
 // pieces of a row, ran at 0.29 us a step of 128 x 128 x 32 whether one or two blocks shared the CU; with the 128-byte
 // pieces of 64 k 2048 x 4096 x 2304 takes 36.9 us instead of 41.5 (tiles of 128 x 256) and 535 x 2304 x 9216 in four
-// ranges 32.9 instead of 41.4.  Many full rounds of 256 x 256 tiles reach 1.2 to 1.3 PFLOP/s
-// (4096 x 4096 x 16384 in 425 us; the library product of that process 367, where it is not clear that more is to be had at
-// the clock that power allows).
+// ranges 32.9 instead of 41.4.  Many full rounds of 256 x 256 tiles reach 1.2 to 1.35 PFLOP/s
+// (4096 x 4096 x 16384 in 412 us; the library product 367 to 425 from one process to the next).  In the two whole rounds of
+// 2048 x (2 x 9216) x 2304 a CU's matrix units are busy for 0.75 of its cycles, at 1.6 GHz of 2.4.
 //
 // LDS: W's strips lie as in memory, 1 KB for 32 k: [k piece of 8][row 16][8 values]; an operand
 // read (row lane % 32, k piece lane / 32) takes whole 256-byte runs.  A: a copy takes 8 rows x
