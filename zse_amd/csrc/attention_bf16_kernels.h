@@ -834,17 +834,17 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
   const int* table = p.block_table + (size_t)r * p.max_blocks;
   const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, last_entry = min(p.max_blocks - 1, blk_hi >> bsh);
 
-  // bytes of a page (4 GiB and more among them), and what lies before the key head's part of it
-  const size_t k_page = (size_t)nkv * HD * 2 << bsh, v_page = (size_t)(nkv >> p.v_shift) * VD * 2 << bsh;
+  // bytes of a page's key (a page may have 4 GiB and more), and what lies before the key head's part of a page
+  const unsigned k_bytes = nkv * HD * 2, v_bytes = (nkv >> p.v_shift) * VD * 2;
   const unsigned char* const k_base = (const unsigned char*)p.kcache + ((size_t)kvh * HD * 2 << bsh);
   const unsigned char* const v_base = (const unsigned char*)p.vcache + ((size_t)(kvh >> p.v_shift) * VD * 2 << bsh);
   // the places of 64 pages, from entry ``first`` of the table on, one a lane; a tile lies in at most two (of 16 keys)
   struct Pages { unsigned lo, hi; int first; };
-  auto cover = [&](Pages& e, int key0, const unsigned char* base, size_t page_bytes) __attribute__((always_inline)) {
+  auto cover = [&](Pages& e, int key0, const unsigned char* base, unsigned key_bytes) __attribute__((always_inline)) {
     const int first = key0 >> bsh;
     if ((unsigned)(first - e.first) > 60u) {
       e.first = first;
-      const uint64_t at = (uint64_t)base + (uint64_t)(unsigned)max(table[min(first + lane, last_entry)], 0) * page_bytes;
+      const uint64_t at = (uint64_t)base + ((uint64_t)(unsigned)max(table[min(first + lane, last_entry)], 0) * key_bytes << bsh);
       e.lo = (unsigned)at;
       e.hi = (unsigned)(at >> 32);
       asm volatile("" : "+v"(e.lo), "+v"(e.hi));        // arrived here, so that no turn waits for loads
@@ -907,10 +907,10 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
   // the copies that turns -4 to -1 would issue (keys of tiles 0 to 3, values of 0 and 1; the waits count on their order)
 #pragma unroll 1
   for (int t = -4; t < 0; t++) {
-    cover(ek, key_of(t + 4), k_base, k_page);
+    cover(ek, key_of(t + 4), k_base, k_bytes);
     copy_k(t + 4, key_of(t + 4), ek);
     if (t >= -2) {
-      cover(ev, key_of(t + 2), v_base, v_page);
+      cover(ev, key_of(t + 2), v_base, v_bytes);
       copy_v(t + 2, key_of(t + 2), ev);
     }
   }
@@ -993,8 +993,8 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8) ? 2 : 1) void attn_st
         s[e] = ok ? s[e] : least;
       }
     }
-    cover(ek, key_of(t + 4), k_base, k_page);
-    cover(ev, key_of(t + 2), v_base, v_page);
+    cover(ek, key_of(t + 4), k_base, k_bytes);
+    cover(ev, key_of(t + 2), v_base, v_bytes);
     rescale();
     f32x16 next;
     auto multiply = [&](int b) __attribute__((always_inline)) {
