@@ -38,33 +38,73 @@ __device__ __forceinline__ void rotate_pair(float a, float b, float sn, float cs
   rb = __fmaf_rn(b, cs, __fmul_rn(a, sn));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = ZSE_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, ZSE_WAVE);
+// Reductions over a wave and a block.  A lane's partner is fetched by a lane permutation of the vector unit (a few
+// cycles; through the local memory, as __shfl_xor goes, about a hundred), in the order 32, 16, 8, 4, 2, 1: the sum is
+// the same bits in every lane.  Kernels of a few rows are a chain of such steps (us, through the local memory and so: a
+// step of one decoded token, 2B shapes, 1,786 and 1,722, of eight 2,423 and 2,355; a model of six layers of width 1,024 234 and 222).
+// Lane l's partner l ^ 32 or l ^ 16: the pair's two values, in some order.
+__device__ __forceinline__ void wave_pair32(float v, float& a, float& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  a = __uint_as_float(p[0]);
+  b = __uint_as_float(p[1]);
+#endif
+}
+__device__ __forceinline__ void wave_pair16(float v, float& a, float& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  a = __uint_as_float(p[0]);
+  b = __uint_as_float(p[1]);
+#endif
+}
+// The value of a lane of the same 16: rotated by 8 or 4 (the partner l ^ 8, and l ^ 4 where lanes 8 apart agree), or
+// permuted inside groups of four.
+#define ZSE_DPP_ROR8 0x128
+#define ZSE_DPP_ROR4 0x124
+#define ZSE_DPP_XOR2 0x4E
+#define ZSE_DPP_XOR1 0xB1
+template <int CTRL>
+__device__ __forceinline__ float wave_dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float wave_sum16(float v) {      // over the 16 lanes of a row
+  v += wave_dpp<ZSE_DPP_ROR8>(v);
+  v += wave_dpp<ZSE_DPP_ROR4>(v);
+  v += wave_dpp<ZSE_DPP_XOR2>(v);
+  v += wave_dpp<ZSE_DPP_XOR1>(v);
   return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  float a = 0.f, b = 0.f;
+  wave_pair32(v, a, b);
+  wave_pair16(a + b, a, b);
+  return wave_sum16(a + b);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = ZSE_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, ZSE_WAVE));
-  return v;
+  float a = 0.f, b = 0.f;
+  wave_pair32(v, a, b);
+  wave_pair16(fmaxf(a, b), a, b);
+  v = fmaxf(a, b);
+  v = fmaxf(v, wave_dpp<ZSE_DPP_ROR8>(v));
+  v = fmaxf(v, wave_dpp<ZSE_DPP_ROR4>(v));
+  v = fmaxf(v, wave_dpp<ZSE_DPP_XOR2>(v));
+  return fmaxf(v, wave_dpp<ZSE_DPP_XOR1>(v));
 }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.
-// ``scratch`` holds at least 17 floats of LDS.
-__device__ __forceinline__ float block_sum(float v, float* scratch) {
+// Sum over a block of up to 1024 threads; every thread gets the result (each wave adds the waves' sums up for
+// itself).  ``scratch`` holds at least 16 floats of LDS that nothing else of the block is reading or writing;
+// block_sum may be called again with the same ones.
+__device__ __forceinline__ float block_sum_once(float v, float* scratch) {
   const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE;
   const int nw = (blockDim.x + ZSE_WAVE - 1) / ZSE_WAVE;
   v = wave_sum(v);
-  __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  if (wave == 0) {
-    float t = lane < nw ? scratch[lane] : 0.f;
-    t = wave_sum(t);
-    if (lane == 0) scratch[16] = t;
-  }
+  return wave_sum16((lane & 15) < nw ? scratch[lane & 15] : 0.f);
+}
+__device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
-  return scratch[16];
+  return block_sum_once(v, scratch);
 }
 
 // ---- host side ----

@@ -145,7 +145,7 @@ __global__ __launch_bounds__(256) void rmsnorm_fast_kernel(const TIn* __restrict
                                                            const float* __restrict__ w,
                                                            act_t* __restrict__ out, float eps,
                                                            int unit_offset, int H) {
-  __shared__ float red[17];
+  __shared__ float red[2][16];
   const int r = blockIdx.x;
   const TIn* xr = x + (size_t)(rows ? rows[r] : r) * H;
   float v[NF_MAXV][4];
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void rmsnorm_fast_kernel(const TIn* __restrict
       for (int e = 0; e < 4; e++) ss += v[j][e] * v[j][e];
     }
   }
-  ss = block_sum(ss, red);
+  ss = block_sum_once(ss, red[0]);
   const float rs = rsqrtf(ss / (float)H + eps);
   act_t* o = out + (size_t)r * H;
 #pragma unroll
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void norm_add_norm_fast_kernel(
     const void* __restrict__ sub, int parts, const float* __restrict__ w_post, float eps_post, int uo_post,
     float* __restrict__ h, const float* __restrict__ w_next, float eps_next, int uo_next,
     act_t* __restrict__ out, int H) {
-  __shared__ float red[17];
+  __shared__ float red[2][16];
   const int r = blockIdx.x;
   const act_t* s = (const act_t*)sub + (size_t)r * H;
   const float* sf = (const float*)sub + (size_t)r * H;      // parts > 0: planes of [rows, H] partial sums
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(256) void norm_add_norm_fast_kernel(
   }
   float rs = 1.f;
   if (w_post) {
-    ss = block_sum(ss, red);
+    ss = block_sum_once(ss, red[0]);
     rs = rsqrtf(ss / (float)H + eps_post);
   }
   float ss2 = 0.f;
@@ -301,7 +301,7 @@ __global__ __launch_bounds__(256) void norm_add_norm_fast_kernel(
     }
   }
   if (!w_next) return;
-  ss2 = block_sum(ss2, red);
+  ss2 = block_sum_once(ss2, red[1]);
   const float rs2 = rsqrtf(ss2 / (float)H + eps_next);
   act_t* o = out + (size_t)r * H;
 #pragma unroll
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(1024) void norm_add_norm_wide_kernel(
     const void* __restrict__ sub, int parts, const float* __restrict__ w_post, float eps_post, int uo_post,
     float* __restrict__ h, const float* __restrict__ w_next, float eps_next, int uo_next,
     act_t* __restrict__ out, int H) {
-  __shared__ float red[17];
+  __shared__ float red[2][16];
   const int r = blockIdx.x;
   const act_t* s = (const act_t*)sub + (size_t)r * H;
   const float* sf = (const float*)sub + (size_t)r * H;
@@ -389,7 +389,7 @@ __global__ __launch_bounds__(1024) void norm_add_norm_wide_kernel(
     }
   float rs = 1.f;
   if (w_post) {
-    ss = block_sum(ss, red);
+    ss = block_sum_once(ss, red[0]);
     rs = rsqrtf(ss / (float)H + eps_post);
   }
   float ss2 = 0.f;
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(1024) void norm_add_norm_wide_kernel(
     }
   }
   if (!w_next) return;
-  ss2 = block_sum(ss2, red);
+  ss2 = block_sum_once(ss2, red[1]);
   const float rs2 = rsqrtf(ss2 / (float)H + eps_next);
   act_t* o = out + (size_t)r * H;
 #pragma unroll
