@@ -285,3 +285,35 @@ def test_head_norms_rotations_and_the_store(dev, inter):
     d_v = up(rt, want_v.reshape(T, nkv * E).astype(np.float32))
     k.zk_rotate_heads(d_v.ptr, i32(rt, pos).ptr, up(rt, vf).ptr, T, nkv, E, inter, -1.0, rt.stream)
     assert np.abs(rt.download(d_v).reshape(T, nkv, E) - v).max() < 1e-5
+
+
+MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17]       # rows of 72 requests
+
+
+def test_matrix_memory_of_many_requests(dev):
+    """The chunks of a step side by side, over more requests than a wave adds up at once."""
+    rt, k = dev
+    rng = np.random.default_rng(5)
+    H, D, E, R, T = 2, 12, 20, len(MANY), sum(MANY)
+    rows = rng.normal(size=(T, 2 * H * (D + E))).astype(np.float32)
+    gates = rng.normal(size=(T, 2 * H)).astype(np.float32)
+    bi, bf, g = up(rt, rng.normal(size=H).astype(np.float32)), up(rt, (rng.normal(size=H) + 2).astype(np.float32)), up(rt, np.ones(H * E, np.float32))
+    words, q_start = k.zk_mlstm_state_bytes(H, D, E) // 4, np.concatenate([[0], np.cumsum(MANY)])
+    req = np.repeat(np.arange(R), MANY)
+    d_rows, d_g, d_q, d_s = up(rt, rows), up(rt, gates), i32(rt, q_start), i32(rt, range(R))
+    got = []
+    for side_by_side in (True, False):
+        state, d_o = rt.zeros((R, words), "float32"), rt.zeros((T, H * E), "float32")
+        if side_by_side:
+            floats = k.zk_mlstm_scan_floats(T, R, H, D, E, max(MANY))
+            work, o_raw = rt.zeros((floats,), "float32"), rt.zeros((T, H * E), "float32")
+            k.zk_mlstm_scan(d_rows.ptr, rows.shape[1], d_g.ptr, bi.ptr, bf.ptr, state.ptr, words, 0, d_q.ptr, d_s.ptr,
+                            o_raw.ptr, work.ptr, floats, T, R, H, D, E, 5.0, max(MANY), rt.stream)
+            k.zk_mlstm_finish(o_raw.ptr, d_rows.ptr, rows.shape[1], g.ptr, None, state.ptr, words, 0, i32(rt, req).ptr, d_q.ptr,
+                              d_s.ptr, d_o.ptr, T, H, D, E, 1e-6, rt.stream)
+        else:
+            k.zk_mlstm(d_rows.ptr, rows.shape[1], d_g.ptr, bi.ptr, bf.ptr, g.ptr, state.ptr, words, 0, d_q.ptr, d_s.ptr, d_o.ptr, R,
+                       H, D, E, 5.0, 1e-6, rt.stream)
+        got.append((rt.download(d_o), rt.download(state)))
+    for a, b in zip(*got):
+        assert np.abs(a - b).max() < 1e-4 * max(1.0, np.abs(b).max())

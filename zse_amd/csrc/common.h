@@ -91,6 +91,34 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(v, wave_dpp<ZSE_DPP_XOR1>(v));
 }
 
+// Running sums and maxima over a wave's lanes (each lane's own value included): rows of 16 lanes by shifts, then a row's
+// last lane handed to the next row, then lane 31 to the upper half.  ``none``: what a lane without a neighbour joins.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int wave_shifted(int v, int none) {
+  return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+#define ZSE_WAVE_SCAN(v, join, cast, back, none)                        \
+  v = join(v, cast(wave_shifted<0x111, 0xf>(back(v), back(none))));     \
+  v = join(v, cast(wave_shifted<0x112, 0xf>(back(v), back(none))));     \
+  v = join(v, cast(wave_shifted<0x114, 0xf>(back(v), back(none))));     \
+  v = join(v, cast(wave_shifted<0x118, 0xf>(back(v), back(none))));     \
+  v = join(v, cast(wave_shifted<0x142, 0xa>(back(v), back(none))));     \
+  v = join(v, cast(wave_shifted<0x143, 0xc>(back(v), back(none))));
+__device__ __forceinline__ int wave_add(int a, int b) { return a + b; }
+__device__ __forceinline__ float wave_add(float a, float b) { return a + b; }
+__device__ __forceinline__ int wave_running_sum(int v) {
+  ZSE_WAVE_SCAN(v, wave_add, int, int, 0)
+  return v;
+}
+__device__ __forceinline__ float wave_running_sum(float v) {
+  ZSE_WAVE_SCAN(v, wave_add, __int_as_float, __float_as_int, 0.f)
+  return v;
+}
+__device__ __forceinline__ float wave_running_max(float v) {
+  ZSE_WAVE_SCAN(v, fmaxf, __int_as_float, __float_as_int, -INFINITY)
+  return v;
+}
+
 // Sum over a block of up to 1024 threads; every thread gets the result (each wave adds the waves' sums up for
 // itself).  ``scratch`` holds at least 16 floats of LDS that nothing else of the block is reading or writing;
 // block_sum may be called again with the same ones.
@@ -105,6 +133,34 @@ __device__ __forceinline__ float block_sum_once(float v, float* scratch) {
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   __syncthreads();
   return block_sum_once(v, scratch);
+}
+
+// Requests are rows [q_start[r], q_start[r + 1]) of a step, cut into pieces of ``len`` rows that are numbered
+// through all requests.  Where piece x lies: its request, that request's rows and the piece's first row among
+// them; false behind the last piece.  All lanes of a wave call it and get the same; 64 requests are added
+// up at a time (one request after the other costs a wait for memory each).
+struct Piece {
+  int r, t0, n, first;
+};
+__device__ __forceinline__ bool find_piece(const int* __restrict__ q_start, int R, int len, int x, Piece& at) {
+  const int lane = threadIdx.x & (ZSE_WAVE - 1);
+  int acc = 0;
+  for (int r0 = 0; r0 < R; r0 += ZSE_WAVE) {
+    const int t0 = q_start[min(r0 + lane, R)], n = q_start[min(r0 + lane + 1, R)] - t0;
+    const int end = acc + wave_running_sum((n + len - 1) / len);          // pieces up to this request's last
+    const unsigned long long later = __ballot(end > x);
+    if (later) {
+      const int i = __ffsll(later) - 1;
+      const int before = i ? __builtin_amdgcn_readlane(end, i - 1) : acc;
+      at.r = r0 + i;
+      at.t0 = __builtin_amdgcn_readlane(t0, i);
+      at.n = __builtin_amdgcn_readlane(n, i);
+      at.first = (x - before) * len;
+      return true;
+    }
+    acc = __builtin_amdgcn_readlane(end, ZSE_WAVE - 1);
+  }
+  return false;
 }
 
 // ---- host side ----

@@ -15,6 +15,8 @@
 #include "common.h"
 #include "packed_call.h"
 
+#include <type_traits>
+
 extern "C" int zk_steplist_register(const char* name, int nargs, void* fn);
 #define ZK_ENTER(fn) \
   static const int fn##_entered = zk_steplist_register(#fn, zk_packed::Call<fn>::nargs, (void*)zk_packed::Call<fn>::call);
@@ -410,297 +412,425 @@ __global__ __launch_bounds__(64) void mlstm_finish_kernel(
 //          M = max(m0, A),  S0' = exp(m0 - M) S0 + exp(A - M) U,  m0' = F + M;   S0, n0, m0 of every chunk are kept
 //   output (every chunk at once):   the read-out of the chunk kernel from the kept S0, n0, m0
 //
-// Chunks are numbered through the step's requests (request r has ceil(n_r / L) of them); a block
-// finds its request by walking q_start.  U is stored where the scan then leaves S0 of that chunk.
-__device__ __forceinline__ bool mlstm_find_chunk(const int* __restrict__ q_start, int R, int L, int x, int& r, int& c0,
-                                                 int& Lc) {
-  int acc = 0;
-  for (r = 0; r < R; r++) {
-    const int t0 = q_start[r], n = q_start[r + 1] - t0;
-    const int nc = (n + L - 1) / L;
-    if (x < acc + nc) {
-      c0 = t0 + (x - acc) * L;
-      Lc = min(L, t0 + n - c0);
-      return true;
-    }
-    acc += nc;
-  }
-  return false;
-}
+// Chunks are numbered through the step's requests (request r has ceil(n_r / L) of them).  U is stored where
+// the scan then leaves S0 of that chunk.
+//
+// The products run on the 32-bit matrix cores (16x16x4), whose operands take q, k and P from the
+// local memory and S0, v and U straight from and to memory: a wave owns 32 value channels and goes through
+// all rows, so each of their elements is fetched once, on its way while the scores are made.  What is
+// left is the chain of loads, scores, read-out of one block a head and chunk.  Multiply-adds out of
+// the local memory, a block a head, chunk and 32 value channels, the chunks of a request after each other in the scan
+// with a wait for memory at each, took (us; 700 tokens and 8 single ones, 16 heads of 64 key and 128 value channels)
+// local 17.7, scan 15.1, output 58.0; so 12.0, 13.0 and 19.5 (of which
+// the 32-bit matrix cores of the CUs that have a full chunk are busy for 8).
+#define MLSTM_EB 128             // value channels a block: 32 for each of its four waves
+typedef float mlstm_f4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ mlstm_f4 mlstm_mfma(float a, float b, mlstm_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// Loads a chunk's k (and q) rows and its slice of v into the local memory, zero beyond Lc.
-template <int L, bool WITH_Q>
-__device__ __forceinline__ void mlstm_load_chunk(const act_t* __restrict__ qkvz, int ld, int c0, int Lc, int hd, int e0, int H,
-                                                 int D, int E, float q_scale, float* Qs, float* Ks, float* Vs) {
-  const int tid = threadIdx.x, DP = D + 1;
-  const bool vec8 = D % 8 == 0 && ld % 8 == 0 && (uintptr_t)qkvz % 16 == 0;
-  if (vec8) {
-    const int D8 = D / 8;
-    for (int i = tid; i < L * D8; i += MLSTM_THREADS) {
-      const int j = i / D8, d = (i % D8) * 8;
-      float q[8] = {}, k[8] = {};
-      if (j < Lc) {
-        const act_t* row = qkvz + (size_t)(c0 + j) * ld;
-        if (WITH_Q) load8(row + (size_t)hd * D + d, q);
-        load8(row + (size_t)(H + hd) * D + d, k);
-      }
-#pragma unroll
-      for (int x = 0; x < 8; x++) {
-        if (WITH_Q) Qs[j * DP + d + x] = q[x] * q_scale;
-        Ks[j * DP + d + x] = k[x];
-      }
+// Key channels in the local memory: whole groups of 16, the rest zero, and four more that spread the rows over
+// the banks (and keep them 16-byte pieces).
+__host__ __device__ __forceinline__ int mlstm_pitch(int D) { return (D + 15) / 16 * 16 + 4; }
+
+// Rows [0, L) of a chunk's q (part 0, times ``scale``) or k (part 1) as floats, zero beyond Lc and D.
+template <int L>
+__device__ __forceinline__ void mlstm_stage(const act_t* __restrict__ qkvz, int ld, int c0, int Lc, int hd, int part, int H, int D,
+                                            float scale, float* dst) {
+  const int P = mlstm_pitch(D), first = (part * H + hd) * D;
+  if (D % 8 == 0 && ld % 8 == 0 && (uintptr_t)qkvz % 16 == 0) {      // eight channels a load
+    const int groups = (P - 4) / 8;
+    for (int i = threadIdx.x; i < L * groups; i += MLSTM_THREADS) {
+      const int j = i / groups, d = (i % groups) * 8;
+      float v[8] = {};
+      if (j < Lc && d < D) load8(qkvz + (size_t)(c0 + j) * ld + first + d, v);
+      *(float4*)(dst + j * P + d) = make_float4(v[0] * scale, v[1] * scale, v[2] * scale, v[3] * scale);
+      *(float4*)(dst + j * P + d + 4) = make_float4(v[4] * scale, v[5] * scale, v[6] * scale, v[7] * scale);
     }
   } else {
-    for (int i = tid; i < L * D; i += MLSTM_THREADS) {
-      const int j = i / D, d = i % D;
-      float q = 0.f, k = 0.f;
-      if (j < Lc) {
-        const act_t* row = qkvz + (size_t)(c0 + j) * ld;
-        if (WITH_Q) q = to_f32(row[(size_t)hd * D + d]) * q_scale;
-        k = to_f32(row[(size_t)(H + hd) * D + d]);
-      }
-      if (WITH_Q) Qs[j * DP + d] = q;
-      Ks[j * DP + d] = k;
+    for (int i = threadIdx.x; i < L * (P - 4); i += MLSTM_THREADS) {
+      const int j = i / (P - 4), d = i % (P - 4);
+      dst[j * P + d] = j < Lc && d < D ? to_f32(qkvz[(size_t)(c0 + j) * ld + first + d]) * scale : 0.f;
     }
-  }
-  for (int i = tid; i < L * MLSTM_EC; i += MLSTM_THREADS) {
-    const int j = i / MLSTM_EC, e = e0 + i % MLSTM_EC;
-    Vs[i] = (j < Lc && e < E) ? to_f32(qkvz[(size_t)(c0 + j) * ld + (size_t)2 * H * D + (size_t)hd * E + e]) : 0.f;
   }
 }
 
-template <int L>
+// The gates of the chunk's token j (lane j of a wave): asked for here ...
+struct MlstmGate {
+  float i, f, bias_i, bias_f;
+};
+__device__ __forceinline__ MlstmGate mlstm_gate_load(const float* __restrict__ gates, const float* __restrict__ bias_i,
+                                                     const float* __restrict__ bias_f, int c0, int Lc, int hd, int H, int j) {
+  const float* g = gates + (size_t)(c0 + min(j, Lc - 1)) * 2 * H + hd;
+  return {g[0], g[H], bias_i[hd], bias_f[hd]};
+}
+// ... and worked out here: a_j (-inf beyond Lc) and the running sum F_j.
+__device__ __forceinline__ void mlstm_gates(const MlstmGate& g, int Lc, float cap, int j, float& a, float& F) {
+  const float gi = cap * tanhf((g.i + g.bias_i) / cap);
+  const float f = log_sigmoid(cap * tanhf((g.f + g.bias_f) / cap));
+  F = wave_running_sum(j < Lc ? f : 0.f);
+  a = j < Lc ? gi - F : -INFINITY;
+}
+
+// Channels e and e + 1 of a row of E (zero from E on and where the row is not there); PAIRS: rows in whole pairs
+template <bool PAIRS, typename T>
+__device__ __forceinline__ void mlstm_pair(const T* __restrict__ row, int e, int E, bool there, float (&v)[2]) {
+  if constexpr (PAIRS) {
+    typedef T t2 __attribute__((ext_vector_type(2)));
+    const t2 x = *(const t2*)(row + min(e, E - 2));
+    v[0] = there && e < E ? to_f32(x[0]) : 0.f;
+    v[1] = there && e < E ? to_f32(x[1]) : 0.f;
+  } else {
+    const float x = to_f32(row[min(e, E - 1)]), y = to_f32(row[min(e + 1, E - 1)]);
+    v[0] = there && e < E ? x : 0.f;
+    v[1] = there && e + 1 < E ? y : 0.f;
+  }
+}
+template <bool PAIRS>
+__device__ __forceinline__ void mlstm_put(float* __restrict__ row, int e, int E, float x, float y) {
+  if constexpr (PAIRS) {
+    if (e < E) *(float2*)(row + e) = make_float2(x, y);
+  } else {
+    if (e < E) row[e] = x;
+    if (e + 1 < E) row[e + 1] = y;
+  }
+}
+
+// Tiles of 16 tokens that a chunk of L uses: one, or all of them.
+#define MLSTM_TILES(L, Lc, f)                           \
+  do {                                                  \
+    if ((Lc) <= 16) f(std::integral_constant<int, 1>{}); \
+    else f(std::integral_constant<int, (L) / 16>{});    \
+  } while (0)
+
+template <int L, bool PAIRS>
 __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_local_kernel(
     const act_t* __restrict__ qkvz, int ld, const float* __restrict__ gates, const float* __restrict__ bias_i,
     const float* __restrict__ bias_f, const int* __restrict__ q_start, float* __restrict__ Uw, float* __restrict__ uw,
     float* __restrict__ af, int R, int H, int D, int E, float cap) {
-  constexpr int EC = MLSTM_EC;
-  extern __shared__ float lds[];
-  const int x = blockIdx.x, hd = blockIdx.y, e0 = blockIdx.z * EC, tid = threadIdx.x;
-  int r, c0, Lc;
-  if (!mlstm_find_chunk(q_start, R, L, x, r, c0, Lc)) return;
-  const int DP = D + 1;
-  float* Ks = lds;                       // [L][DP]
-  float* Vs = Ks + (size_t)L * DP;       // [L][EC]
-  float* ga = Vs + (size_t)L * EC;
-  float* gF = ga + L;
-  float* gw = gF + L;
-  mlstm_load_chunk<L, false>(qkvz, ld, c0, Lc, hd, e0, H, D, E, 0.f, nullptr, Ks, Vs);
-  if (tid < ZSE_WAVE) {
-    const int j = tid;
-    float F = 0.f, gi = 0.f;
-    if (j < Lc) {
-      const size_t t = c0 + j;
-      gi = cap * tanhf((gates[t * 2 * H + hd] + bias_i[hd]) / cap);
-      F = log_sigmoid(cap * tanhf((gates[t * 2 * H + H + hd] + bias_f[hd]) / cap));
-    }
-#pragma unroll
-    for (int o = 1; o < ZSE_WAVE; o <<= 1) {
-      const float up = __shfl_up(F, o, ZSE_WAVE);
-      if (j >= o) F += up;
-    }
-    const float a = j < Lc ? gi - F : -INFINITY;
-    const float A = wave_max(a);
-    if (j < L) gw[j] = j < Lc ? expf(a - A) : 0.f;
-    if (j == Lc - 1 && blockIdx.z == 0) {
-      af[((size_t)x * H + hd) * 2] = A;
-      af[((size_t)x * H + hd) * 2 + 1] = F;
-    }
-  }
-  __syncthreads();
-  for (int i = tid; i < L * EC; i += MLSTM_THREADS) Vs[i] *= gw[i / EC];
-  if (blockIdx.z == 0)
-    for (int d = tid; d < D; d += MLSTM_THREADS) {
-      float acc = 0.f;
-      for (int s2 = 0; s2 < Lc; s2++) acc = fmaf(gw[s2], Ks[s2 * DP + d], acc);
-      uw[((size_t)x * H + hd) * D + d] = acc;
-    }
-  __syncthreads();
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int x = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, kq = lane >> 4;
+  Piece at_chunk;
+  if (!find_piece(q_start, R, L, x, at_chunk)) return;
+  const int c0 = at_chunk.t0 + at_chunk.first, Lc = min(L, at_chunk.n - at_chunk.first);
+  const int P = mlstm_pitch(D);
+  float* Ks = lds;                       // [L][P]
+  float* gw = Ks + (size_t)L * P;        // exp(a_s - A)
+  const int e0 = blockIdx.z * MLSTM_EB + wave * 32 + 2 * lr;
+  const act_t* v0 = qkvz + (size_t)c0 * ld + (size_t)2 * H * D + (size_t)hd * E;
   float* U = Uw + ((size_t)x * H + hd) * D * E;
-  const int ec = (tid % 16) * 2, dg = (tid / 16) * 4;
-  for (int db = 0; db < D; db += 64) {
-    float acc[4][2] = {};
-    const int d = db + dg;
-    for (int s2 = 0; s2 < Lc; s2++) {
-      const float v0 = Vs[s2 * EC + ec], v1 = Vs[s2 * EC + ec + 1];
+  auto run = [&](auto tiles) {
+    constexpr int KS = decltype(tiles)::value;
+    MlstmGate gate;
+    if (wave == 0) gate = mlstm_gate_load(gates, bias_i, bias_f, c0, Lc, hd, H, lane);
+    mlstm_stage<16 * KS>(qkvz, ld, c0, Lc, hd, 1, H, D, 1.f, Ks);
+    float v[KS][4][2];                   // token 16 g + 4 kq + i, channels e0 and e0 + 1
 #pragma unroll
-      for (int a = 0; a < 4; a++) {
-        const float k = d + a < D ? Ks[s2 * DP + d + a] : 0.f;
-        acc[a][0] = fmaf(k, v0, acc[a][0]);
-        acc[a][1] = fmaf(k, v1, acc[a][1]);
+    for (int g = 0; g < KS; g++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = 16 * g + 4 * kq + i;
+        mlstm_pair<PAIRS>(v0 + (size_t)min(row, Lc - 1) * ld, e0, E, row < Lc, v[g][i]);
+      }
+    if (wave == 0) {
+      float a, F;
+      mlstm_gates(gate, Lc, cap, lane, a, F);
+      const float A = wave_max(a);
+      if (lane < L) gw[lane] = lane < Lc ? expf(a - A) : 0.f;
+      if (lane == Lc - 1 && blockIdx.z == 0) {
+        af[((size_t)x * H + hd) * 2] = A;
+        af[((size_t)x * H + hd) * 2 + 1] = F;
       }
     }
+    __syncthreads();
 #pragma unroll
-    for (int a = 0; a < 4; a++)
-      if (d + a < D) {
-        if (e0 + ec < E) U[(size_t)(d + a) * E + e0 + ec] = acc[a][0];
-        if (e0 + ec + 1 < E) U[(size_t)(d + a) * E + e0 + ec + 1] = acc[a][1];
+    for (int g = 0; g < KS; g++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) v[g][i][c] *= gw[16 * g + 4 * kq + i];
+    for (int d0 = 0; d0 < D; d0 += 16) {
+      float k[KS][4];
+#pragma unroll
+      for (int g = 0; g < KS; g++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) k[g][i] = Ks[(16 * g + 4 * kq + i) * P + d0 + lr];
+      mlstm_f4 acc[2] = {};
+#pragma unroll
+      for (int g = 0; g < KS; g++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int c = 0; c < 2; c++) acc[c] = mlstm_mfma(k[g][i], v[g][i][c], acc[c]);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int d = d0 + 4 * kq + i;
+        if (d < D) mlstm_put<PAIRS>(U + (size_t)d * E, e0, E, acc[0][i], acc[1][i]);
       }
-  }
+    }
+    if (blockIdx.z == 0)                 // u: four threads a channel
+      for (int d0 = 0; d0 < D; d0 += MLSTM_THREADS / 4) {
+        const int d = d0 + tid / 4;
+        float acc = 0.f;
+        if (d < D) {
+#pragma unroll
+          for (int s2 = 0; s2 < 4 * KS; s2++) acc = fmaf(gw[4 * s2 + tid % 4], Ks[(4 * s2 + tid % 4) * P + d], acc);
+        }
+        acc += wave_dpp<ZSE_DPP_XOR1>(acc);
+        acc += wave_dpp<ZSE_DPP_XOR2>(acc);
+        if (d < D && tid % 4 == 0) uw[((size_t)x * H + hd) * D + d] = acc;
+      }
+  };
+  MLSTM_TILES(L, Lc, run);
 }
 
-// One thread per element of a head's state (S, then n, then one more thread that keeps m).
+// MLSTM_ELEMS elements of a head's state a thread (S, then n, then one more that writes down every chunk's m; the
+// state's own m, which all threads read, is renewed by the output kernel).  Eight chunks' U are
+// asked for at once: a store of S0 into the place of a U would otherwise hold back the next load.
+#define MLSTM_ELEMS 4
 __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_scan_kernel(
     float* __restrict__ state, int slot_words, int offset_words, const int* __restrict__ q_start,
     const int* __restrict__ slot_of_req, float* __restrict__ Uw, float* __restrict__ uw, const float* __restrict__ af,
     float* __restrict__ mprev, int L, int H, int D, int E) {
-  const int r = blockIdx.x, hd = blockIdx.y;
-  const int idx = blockIdx.z * MLSTM_THREADS + threadIdx.x;
-  const int DE = D * E;
-  if (idx > DE + D) return;
+  constexpr int AHEAD = 8, NE = MLSTM_ELEMS;
+  const int r = blockIdx.x, hd = blockIdx.y, lane = threadIdx.x & (ZSE_WAVE - 1);
+  const int idx0 = blockIdx.z * (MLSTM_THREADS * NE) + threadIdx.x;      // and every MLSTM_THREADS further on
+  const int DE = D * E, slot = slot_of_req[r];
   const int t0 = q_start[r], n = q_start[r + 1] - t0;
-  if (n <= 0) return;
-  int first = 0;
-  for (int r2 = 0; r2 < r; r2++) first += (q_start[r2 + 1] - q_start[r2] + L - 1) / L;
-  const int nc = (n + L - 1) / L;
-  float* st = state + (size_t)slot_of_req[r] * slot_words + offset_words + (size_t)hd * ((size_t)DE + D + 1);
-  float m = st[DE + D];
-  float val = idx < DE + D ? st[idx] : 0.f;
-  for (int ci = 0; ci < nc; ci++) {
-    const size_t at = (size_t)(first + ci) * H + hd;
-    const float A = af[at * 2], F = af[at * 2 + 1];
-    const float M = fmaxf(m, A);
-    if (idx < DE + D) {
-      float* p = idx < DE ? Uw + at * DE + idx : uw + at * D + (idx - DE);
-      const float U = *p;
-      *p = val;                                   // the state this chunk starts from
-      val = fmaf(expf(m - M), val, expf(A - M) * U);
-    } else {
-      mprev[at] = m;
-    }
-    m = F + M;
+  int first = 0;                         // chunks of the requests in front of r
+  for (int r0 = 0; r0 < r; r0 += ZSE_WAVE) {
+    const int q = min(r0 + lane, r - 1);
+    const int c = r0 + lane < r ? (q_start[q + 1] - q_start[q] + L - 1) / L : 0;
+    first += __builtin_amdgcn_readlane(wave_running_sum(c), ZSE_WAVE - 1);
   }
-  st[idx] = idx < DE + D ? val : m;
+  if (n <= 0 || idx0 > DE + D) return;
+  const int nc = (n + L - 1) / L;
+  float* st = state + (size_t)slot * slot_words + offset_words + (size_t)hd * ((size_t)DE + D + 1);
+  float m = st[DE + D];
+  float val[NE];
+  float* p0[NE];                         // the element of chunk 0's U or u, and how far on the next chunk's is
+  size_t step[NE];
+#pragma unroll
+  for (int k = 0; k < NE; k++) {
+    const int idx = min(idx0 + k * MLSTM_THREADS, DE + D - 1);      // (past the last: the last again, not stored)
+    val[k] = st[idx];
+    p0[k] = idx < DE ? Uw + ((size_t)first * H + hd) * DE + idx : uw + ((size_t)first * H + hd) * D + (idx - DE);
+    step[k] = (size_t)H * (idx < DE ? DE : D);
+  }
+  auto mine = [&](int k) { return idx0 + k * MLSTM_THREADS < DE + D; };
+  const bool keeps_m = (DE + D - idx0) % MLSTM_THREADS == 0 && DE + D - idx0 < NE * MLSTM_THREADS;
+  const float* g0 = af + ((size_t)first * H + hd) * 2;
+  for (int c0 = 0; c0 < nc; c0 += AHEAD) {
+    float U[AHEAD][NE], A[AHEAD], F[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) {
+      const int ci = min(c0 + i, nc - 1);
+#pragma unroll
+      for (int k = 0; k < NE; k++) U[i][k] = p0[k][ci * step[k]];
+      A[i] = g0[(size_t)ci * H * 2];
+      F[i] = g0[(size_t)ci * H * 2 + 1];
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) {
+      const int ci = c0 + i;
+      if (ci < nc) {
+        const float M = fmaxf(m, A[i]), keep = expf(m - M), add = expf(A[i] - M);
+#pragma unroll
+        for (int k = 0; k < NE; k++)
+          if (mine(k)) {
+            p0[k][ci * step[k]] = val[k];                        // the state this chunk starts from
+            val[k] = fmaf(keep, val[k], add * U[i][k]);
+          }
+        if (keeps_m) mprev[(size_t)(first + ci) * H + hd] = m;
+        m = F[i] + M;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NE; k++)
+    if (mine(k)) st[idx0 + k * MLSTM_THREADS] = val[k];
 }
 
-template <int L>
+template <int L, bool PAIRS>
 __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_output_kernel(
     const act_t* __restrict__ qkvz, int ld, const float* __restrict__ gates, const float* __restrict__ bias_i,
     const float* __restrict__ bias_f, const int* __restrict__ q_start, const float* __restrict__ Sw,
-    const float* __restrict__ nw, const float* __restrict__ mprev, float* __restrict__ o_raw, int R, int H, int D, int E,
-    float cap, float q_scale) {
-  constexpr int EC = MLSTM_EC;
-  constexpr int TP = L / 16;
-  extern __shared__ float lds[];
-  const int x = blockIdx.x, hd = blockIdx.y, e0 = blockIdx.z * EC, tid = threadIdx.x;
-  int r, c0, Lc;
-  if (!mlstm_find_chunk(q_start, R, L, x, r, c0, Lc)) return;
-  const int DP = D + 1, LP = L + 1;
-  float* Ss = lds;
-  float* ns = Ss + (size_t)D * EC;
-  float* Qs = ns + D;
-  float* Ks = Qs + (size_t)L * DP;
-  float* Vs = Ks + (size_t)L * DP;
-  float* Ps = Vs + (size_t)L * EC;
-  float* ga = Ps + (size_t)L * LP;
+    const float* __restrict__ nw, const float* __restrict__ mprev, float* __restrict__ o_raw, float* __restrict__ state,
+    int slot_words, int offset_words, const int* __restrict__ slot_of_req, int R, int H, int D, int E, float cap, float q_scale) {
+  constexpr int LP = L + 4;
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  const int x = blockIdx.x, hd = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 15, kq = lane >> 4;
+  Piece at_chunk;
+  if (!find_piece(q_start, R, L, x, at_chunk)) return;
+  const int c0 = at_chunk.t0 + at_chunk.first, Lc = min(L, at_chunk.n - at_chunk.first);
+  const int P = mlstm_pitch(D);
+  float* Qs = lds;                       // [L][P]
+  float* Ks = Qs + (size_t)L * P;        // [L][P]
+  float* Ps = Ks + (size_t)L * P;        // [L][LP]
+  float* ns = Ps + (size_t)L * LP;       // [P]
+  float* ga = ns + P;
   float* gM = ga + L;
   float* gF = gM + L;
-  float* gden = gF + L;
+  float* gden = gF + L;                  // n . q, then the denominators
   const size_t at = (size_t)x * H + hd;
+  const int e0 = blockIdx.z * MLSTM_EB + wave * 32 + 2 * lr;
   const float* S0 = Sw + at * D * E;
-  for (int i = tid; i < D * EC; i += MLSTM_THREADS) {
-    const int d = i / EC, e = e0 + i % EC;
-    Ss[i] = e < E ? S0[(size_t)d * E + e] : 0.f;
-  }
-  for (int d = tid; d < D; d += MLSTM_THREADS) ns[d] = nw[at * D + d];
-  const float m_prev = mprev[at];
-  mlstm_load_chunk<L, true>(qkvz, ld, c0, Lc, hd, e0, H, D, E, q_scale, Qs, Ks, Vs);
-  if (tid < ZSE_WAVE) {
-    const int j = tid;
-    float F = 0.f, gi = 0.f;
-    if (j < Lc) {
-      const size_t t = c0 + j;
-      gi = cap * tanhf((gates[t * 2 * H + hd] + bias_i[hd]) / cap);
-      F = log_sigmoid(cap * tanhf((gates[t * 2 * H + H + hd] + bias_f[hd]) / cap));
+  const act_t* v0 = qkvz + (size_t)c0 * ld + (size_t)2 * H * D + (size_t)hd * E;
+  auto run = [&](auto tiles) {
+    constexpr int RT = decltype(tiles)::value;             // tiles of 16 tokens
+    MlstmGate gate;
+    if (wave == 0) gate = mlstm_gate_load(gates, bias_i, bias_f, c0, Lc, hd, H, lane);
+    const float m_prev = mprev[at];
+    mlstm_stage<16 * RT>(qkvz, ld, c0, Lc, hd, 0, H, D, q_scale, Qs);
+    mlstm_stage<16 * RT>(qkvz, ld, c0, Lc, hd, 1, H, D, 1.f, Ks);
+    for (int d = tid; d < P; d += MLSTM_THREADS) ns[d] = d < D ? nw[at * D + d] : 0.f;
+    // S0 of 64 key channels and v of the chunk's tokens, on their way from now on
+    float sv[4][4][2], v[RT][4][2];
+    auto fetch_s = [&](int d0) {
+#pragma unroll
+      for (int g = 0; g < 4; g++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int d = d0 + 16 * g + 4 * kq + i;
+          mlstm_pair<PAIRS>(S0 + (size_t)min(d, D - 1) * E, e0, E, d < D, sv[g][i]);
+        }
+    };
+    fetch_s(0);
+#pragma unroll
+    for (int g = 0; g < RT; g++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = 16 * g + 4 * kq + i;
+        mlstm_pair<PAIRS>(v0 + (size_t)min(row, Lc - 1) * ld, e0, E, row < Lc, v[g][i]);
+      }
+    if (wave == 0) {
+      float a, F;
+      mlstm_gates(gate, Lc, cap, lane, a, F);
+      const float M = fmaxf(wave_running_max(a), m_prev);
+      if (lane < L) {
+        ga[lane] = a;
+        gM[lane] = M;
+        gF[lane] = F;
+      }
+      if (at_chunk.first + Lc == at_chunk.n && lane == Lc - 1 && blockIdx.z == 0)      // the request's last chunk
+        state[(size_t)slot_of_req[at_chunk.r] * slot_words + offset_words + (size_t)hd * ((size_t)D * E + D + 1) + (size_t)D * E + D] =
+            F + M;
+    }
+    __syncthreads();
+    // P and the denominators: a wave takes every fourth tile of rows, and the tiles of columns up to the diagonal
+    const int KS = (P - 4) / 16;           // groups of 16 key channels
+#pragma unroll
+    for (int a0 = 0; a0 < (RT + 3) / 4; a0++) {
+      const int a = wave + 4 * a0;
+      if (a >= RT) break;
+      mlstm_f4 acc[RT];
+#pragma unroll
+      for (int b = 0; b < RT; b++) acc[b] = mlstm_f4{0.f, 0.f, 0.f, 0.f};
+      float nq = 0.f;                      // n . q of row lr, the lane's channels
+      for (int g = 0; g < KS; g++) {
+        const float4 q = *(const float4*)(Qs + (16 * a + lr) * P + 16 * g + 4 * kq), n = *(const float4*)(ns + 16 * g + 4 * kq);
+        const float qe[4] = {q.x, q.y, q.z, q.w};
+        float ke[RT][4];
+#pragma unroll
+        for (int b = 0; b < RT; b++) {
+          const float4 k = *(const float4*)(Ks + (16 * b + lr) * P + 16 * g + 4 * kq);
+          ke[b][0] = k.x, ke[b][1] = k.y, ke[b][2] = k.z, ke[b][3] = k.w;
+        }
+        nq = fmaf(q.w, n.w, fmaf(q.z, n.z, fmaf(q.y, n.y, fmaf(q.x, n.x, nq))));
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int b = 0; b < RT; b++) acc[b] = mlstm_mfma(qe[i], ke[b][i], acc[b]);
+      }
+      float ps[4] = {};
+#pragma unroll
+      for (int b = 0; b < RT; b++) {
+        const float as = ga[16 * b + lr];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const int j = 16 * a + 4 * kq + i, s2 = 16 * b + lr;
+          const float p = (s2 <= j && j < Lc) ? acc[b][i] * expf(as - gM[j]) : 0.f;
+          Ps[j * LP + s2] = p;
+          ps[i] += p;
+        }
+      }
+      float x0 = 0.f, x1 = 0.f;
+      wave_pair32(nq, x0, x1);
+      wave_pair16(x0 + x1, x0, x1);
+      if (kq == 0) gden[16 * a + lr] = x0 + x1;
+#pragma unroll
+      for (int i = 0; i < 4; i++) ps[i] = wave_sum16(ps[i]);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");      // the wave reads what its other lanes wrote
+      __builtin_amdgcn_wave_barrier();
+      if (lr < 4) {                        // lane (lr, kq): row 4 kq + lr
+        const int j = 16 * a + 4 * kq + lr;
+        const float p = lr == 0 ? ps[0] : lr == 1 ? ps[1] : lr == 2 ? ps[2] : ps[3];
+        const float den = fmaf(gden[j], expf(m_prev - gM[j]), p);
+        gden[j] = 1.0f / (fmaxf(fabsf(den), expf(-(gF[j] + gM[j]))) + 1e-6f);
+      }
+    }
+    __syncthreads();
+    mlstm_f4 acc[RT][2];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) acc[a][c] = mlstm_f4{0.f, 0.f, 0.f, 0.f};
+    for (int d0 = 0; d0 < D; d0 += 64) {
+      if (d0) fetch_s(d0);
+      const int most = P - 20;             // a group past the last one reads the last again, against zeros
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        float qe[RT][4];
+#pragma unroll
+        for (int a = 0; a < RT; a++) {
+          const float4 q = *(const float4*)(Qs + (16 * a + lr) * P + min(d0 + 16 * g, most) + 4 * kq);
+          qe[a][0] = q.x, qe[a][1] = q.y, qe[a][2] = q.z, qe[a][3] = q.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int a = 0; a < RT; a++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) acc[a][c] = mlstm_mfma(qe[a][i], sv[g][i][c], acc[a][c]);
+      }
     }
 #pragma unroll
-    for (int o = 1; o < ZSE_WAVE; o <<= 1) {
-      const float up = __shfl_up(F, o, ZSE_WAVE);
-      if (j >= o) F += up;
-    }
-    const float a = j < Lc ? gi - F : -INFINITY;
-    float M = a;
+    for (int a = 0; a < RT; a++)
 #pragma unroll
-    for (int o = 1; o < ZSE_WAVE; o <<= 1) {
-      const float up = __shfl_up(M, o, ZSE_WAVE);
-      if (j >= o) M = fmaxf(M, up);
-    }
-    if (j < L) {
-      ga[j] = a;
-      gM[j] = fmaxf(M, m_prev);
-      gF[j] = F;
-    }
-  }
-  __syncthreads();
-  {
-    const int pj = tid / 16, ps = tid % 16;
-    float acc[TP][TP] = {};
-    for (int d = 0; d < D; d++) {
-      float q[TP], k[TP];
+      for (int i = 0; i < 4; i++) {
+        const float g = expf(m_prev - gM[16 * a + 4 * kq + i]);
 #pragma unroll
-      for (int y = 0; y < TP; y++) {
-        q[y] = Qs[(pj + 16 * y) * DP + d];
-        k[y] = Ks[(ps + 16 * y) * DP + d];
+        for (int c = 0; c < 2; c++) acc[a][c][i] *= g;
       }
 #pragma unroll
-      for (int a = 0; a < TP; a++)
+    for (int g = 0; g < RT; g++) {
+      float pe[RT][4];
 #pragma unroll
-        for (int b = 0; b < TP; b++) acc[a][b] = fmaf(q[a], k[b], acc[a][b]);
-    }
-#pragma unroll
-    for (int a = 0; a < TP; a++)
-#pragma unroll
-      for (int b = 0; b < TP; b++) {
-        const int j = pj + 16 * a, s2 = ps + 16 * b;
-        Ps[j * LP + s2] = (s2 <= j && j < Lc) ? acc[a][b] * expf(ga[s2] - gM[j]) : 0.f;
+      for (int a = g; a < RT; a++) {
+        const float4 p = *(const float4*)(Ps + (16 * a + lr) * LP + 16 * g + 4 * kq);
+        pe[a][0] = p.x, pe[a][1] = p.y, pe[a][2] = p.z, pe[a][3] = p.w;
       }
-  }
-  __syncthreads();
-  if (tid < L) {
-    const int j = tid;
-    float nq = 0.f;
-    for (int d = 0; d < D; d++) nq = fmaf(ns[d], Qs[j * DP + d], nq);
-    nq *= expf(m_prev - gM[j]);
-    for (int s2 = 0; s2 <= j; s2++) nq += Ps[j * LP + s2];
-    gden[j] = fmaxf(fabsf(nq), expf(-(gF[j] + gM[j]))) + 1e-6f;
-  }
-  const int ec = (tid % 16) * 2, rg = tid / 16;
-  float acc[TP][2] = {};
-  for (int d = 0; d < D; d++) {
-    const float s0 = Ss[d * EC + ec], s1 = Ss[d * EC + ec + 1];
 #pragma unroll
-    for (int a = 0; a < TP; a++) {
-      const float q = Qs[(rg + 16 * a) * DP + d];
-      acc[a][0] = fmaf(q, s0, acc[a][0]);
-      acc[a][1] = fmaf(q, s1, acc[a][1]);
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int a = g; a < RT; a++)
+#pragma unroll
+          for (int c = 0; c < 2; c++) acc[a][c] = mlstm_mfma(pe[a][i], v[g][i][c], acc[a][c]);
     }
-  }
 #pragma unroll
-  for (int a = 0; a < TP; a++) {
-    const float g = expf(m_prev - gM[rg + 16 * a]);
-    acc[a][0] *= g;
-    acc[a][1] *= g;
-  }
-  for (int s2 = 0; s2 < Lc; s2++) {
-    const float v0 = Vs[s2 * EC + ec], v1 = Vs[s2 * EC + ec + 1];
+    for (int a = 0; a < RT; a++)
 #pragma unroll
-    for (int a = 0; a < TP; a++) {
-      const float p = Ps[(rg + 16 * a) * LP + s2];
-      acc[a][0] = fmaf(p, v0, acc[a][0]);
-      acc[a][1] = fmaf(p, v1, acc[a][1]);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int a = 0; a < TP; a++) {
-    const int j = rg + 16 * a;
-    if (j < Lc) {
-      float* o = o_raw + ((size_t)(c0 + j) * H + hd) * E;
-      if (e0 + ec < E) o[e0 + ec] = acc[a][0] / gden[j];
-      if (e0 + ec + 1 < E) o[e0 + ec + 1] = acc[a][1] / gden[j];
-    }
-  }
+      for (int i = 0; i < 4; i++) {
+        const int j = 16 * a + 4 * kq + i;
+        if (j < Lc) {
+          const float inv = gden[j];
+          mlstm_put<PAIRS>(o_raw + ((size_t)(c0 + j) * H + hd) * E, e0, E, acc[a][0][i] * inv, acc[a][1][i] * inv);
+        }
+      }
+  };
+  MLSTM_TILES(L, Lc, run);
 }
+
+static size_t mlstm_local_lds(int L, int D) { return ((size_t)L * mlstm_pitch(D) + L) * 4; }
+static size_t mlstm_output_lds(int L, int D) { return ((size_t)2 * L * mlstm_pitch(D) + (size_t)L * (L + 4) + mlstm_pitch(D) + 4 * L) * 4; }
 
 static size_t mlstm_chunk_lds(int L, int D) {
   return ((size_t)D * MLSTM_EC + D + (size_t)2 * L * (D + 1) + (size_t)L * MLSTM_EC + (size_t)L * (L + 1) + 5 * L + 8) * 4;
@@ -806,7 +936,7 @@ int zk_mlstm_chunked(const void* qkvz, int ld, const float* gates, const float* 
 
 static int mlstm_scan_len(int max_q_len, int D) {
   int L = max_q_len <= 16 ? 16 : max_q_len <= 32 ? 32 : 64;
-  while (L > 16 && mlstm_chunk_lds(L, D) > 150 * 1024) L /= 2;
+  while (L > 16 && mlstm_output_lds(L, D) > 150 * 1024) L /= 2;
   return L;
 }
 
@@ -817,7 +947,7 @@ extern "C" size_t zk_mlstm_scan_floats(int T, int R, int H, int D, int E, int ma
   return chunks * H * ((size_t)D * E + D + 3);
 }
 
-template <int L>
+template <int L, bool PAIRS>
 static int mlstm_scan_launch(const void* qkvz, int ld, const float* gates, const float* bias_i, const float* bias_f,
                              float* state, int slot_words, int offset_words, const int* q_start, const int* slot_of_req,
                              float* o_raw, float* work, int chunks, int R, int H, int D, int E, float cap, hipStream_t s) {
@@ -825,27 +955,26 @@ static int mlstm_scan_launch(const void* qkvz, int ld, const float* gates, const
   float* uw = Uw + (size_t)chunks * H * D * E;
   float* af = uw + (size_t)chunks * H * D;
   float* mprev = af + (size_t)chunks * H * 2;
-  const int zs = (E + MLSTM_EC - 1) / MLSTM_EC;
-  const size_t lds_local = ((size_t)L * (D + 1) + (size_t)L * MLSTM_EC + 3 * L + 8) * 4;
-  const size_t lds_out = mlstm_chunk_lds(L, D);
+  const int zs = (E + MLSTM_EB - 1) / MLSTM_EB;
+  const size_t lds_local = mlstm_local_lds(L, D), lds_out = mlstm_output_lds(L, D);
   static size_t raised_local = 0, raised_out = 0;
   if (lds_local > 48 * 1024 && lds_local > raised_local) {
-    hipFuncSetAttribute((const void*)mlstm_local_kernel<L>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_local);
+    hipFuncSetAttribute((const void*)mlstm_local_kernel<L, PAIRS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_local);
     raised_local = lds_local;
   }
   if (lds_out > 48 * 1024 && lds_out > raised_out) {
-    hipFuncSetAttribute((const void*)mlstm_output_kernel<L>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_out);
+    hipFuncSetAttribute((const void*)mlstm_output_kernel<L, PAIRS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_out);
     raised_out = lds_out;
   }
-  mlstm_local_kernel<L><<<dim3(chunks, H, zs), MLSTM_THREADS, lds_local, s>>>((const act_t*)qkvz, ld, gates, bias_i, bias_f,
-                                                                              q_start, Uw, uw, af, R, H, D, E, cap);
+  mlstm_local_kernel<L, PAIRS><<<dim3(chunks, H, zs), MLSTM_THREADS, lds_local, s>>>(
+      (const act_t*)qkvz, ld, gates, bias_i, bias_f, q_start, Uw, uw, af, R, H, D, E, cap);
   if (int rc = zk_launch_status("zk_mlstm_scan (local)")) return rc;
-  mlstm_scan_kernel<<<dim3(R, H, (D * E + D + 1 + MLSTM_THREADS - 1) / MLSTM_THREADS), MLSTM_THREADS, 0, s>>>(
+  mlstm_scan_kernel<<<dim3(R, H, (D * E + D + MLSTM_THREADS * MLSTM_ELEMS) / (MLSTM_THREADS * MLSTM_ELEMS)), MLSTM_THREADS, 0, s>>>(
       state, slot_words, offset_words, q_start, slot_of_req, Uw, uw, af, mprev, L, H, D, E);
   if (int rc = zk_launch_status("zk_mlstm_scan (scan)")) return rc;
-  mlstm_output_kernel<L><<<dim3(chunks, H, zs), MLSTM_THREADS, lds_out, s>>>((const act_t*)qkvz, ld, gates, bias_i, bias_f,
-                                                                             q_start, Uw, uw, mprev, o_raw, R, H, D, E, cap,
-                                                                             1.0f / sqrtf((float)D));
+  mlstm_output_kernel<L, PAIRS><<<dim3(chunks, H, zs), MLSTM_THREADS, lds_out, s>>>(
+      (const act_t*)qkvz, ld, gates, bias_i, bias_f, q_start, Uw, uw, mprev, o_raw, state, slot_words, offset_words, slot_of_req, R, H,
+      D, E, cap, 1.0f / sqrtf((float)D));
   return zk_launch_status("zk_mlstm_scan (output)");
 }
 
@@ -868,9 +997,14 @@ int zk_mlstm_scan(const void* qkvz, int ld, const float* gates, const float* bia
   const int L = mlstm_scan_len(max_q_len, D);
   const int chunks = (T + L - 1) / L + R;
   hipStream_t s = (hipStream_t)stream;
-#define ZK_SCAN_(L_) \
-  mlstm_scan_launch<L_>(qkvz, ld, gates, bias_i, bias_f, state, slot_words, offset_words, q_start, slot_of_req, o_raw, work, \
-                        chunks, R, H, D, E, cap, s)
+  // two value channels an access, where every row of them begins on a pair
+  const bool pairs = E % 2 == 0 && ld % 2 == 0 && (uintptr_t)qkvz % (2 * sizeof(act_t)) == 0 && (uintptr_t)work % 8 == 0 &&
+                     (uintptr_t)o_raw % 8 == 0;
+#define ZK_SCAN_(L_)                                                                                                          \
+  (pairs ? mlstm_scan_launch<L_, true>(qkvz, ld, gates, bias_i, bias_f, state, slot_words, offset_words, q_start, slot_of_req, \
+                                       o_raw, work, chunks, R, H, D, E, cap, s)                                               \
+         : mlstm_scan_launch<L_, false>(qkvz, ld, gates, bias_i, bias_f, state, slot_words, offset_words, q_start, slot_of_req, \
+                                        o_raw, work, chunks, R, H, D, E, cap, s))
   return L == 64 ? ZK_SCAN_(64) : L == 32 ? ZK_SCAN_(32) : ZK_SCAN_(16);
 #undef ZK_SCAN_
 }
