@@ -287,6 +287,31 @@ def test_head_norms_rotations_and_the_store(dev, inter):
     assert np.abs(rt.download(d_v).reshape(T, nkv, E) - v).max() < 1e-5
 
 
+@pytest.mark.parametrize("S,W,parts", [(4, 4, 0), (2, 1020, 2), (4, 1024, 0), (4, 1028, 0), (2, 2048, 1), (4, 4096, 3), (4, 4100, 0)])
+def test_streams_of_whole_pieces(dev, S, W, parts):
+    """Two and four streams of rows in 16-byte pieces: one, two and four of them a thread, a last thread
+    without any, and a width (4,100) that the kernel for rows held in registers leaves to the other."""
+    rt, k = dev
+    rng = np.random.default_rng(W + S)
+    T = 3
+    xs = rng.normal(size=(T, S, W)).astype(np.float32)
+    planes = rng.normal(size=(max(parts, 1), T, W)).astype(np.float32)
+    mix, out, win = (rng.normal(size=s).astype(np.float32) for s in ((S, S), (S,), (S,)))
+    g, b = rng.normal(1, 0.2, W).astype(np.float32), rng.normal(0, 0.2, W).astype(np.float32)
+    d_xs, d_o = up(rt, xs), rt.empty((T, W), "float32")
+    k.zk_streams_step(d_xs.ptr, S, up(rt, planes).ptr, parts, up(rt, mix).ptr, up(rt, out).ptr, up(rt, win).ptr, up(rt, g).ptr,
+                      up(rt, b).ptr, 1e-5, None, d_o.ptr, T, T, W, rt.stream)
+    want_xs = P.streams_write(xs, mix, out, planes.astype(np.float64).sum(0), np.float64)
+    want = P.layer_norm(P.streams_read(want_xs, win, np.float64), g, b, 1e-5, np.float64)
+    assert np.abs(rt.download(d_xs) - want_xs).max() < 2e-5
+    assert np.abs(rt.download(d_o) - want).max() < 3e-5
+    d_p = rt.empty((2, W), "float32")
+    k.zk_streams_step(d_xs.ptr, S, None, 0, None, None, None, up(rt, g).ptr, None, 1e-5, i32(rt, [2, 0]).ptr, d_p.ptr, 2, T, W,
+                      rt.stream)
+    want = P.layer_norm(want_xs.sum(axis=1)[[2, 0]], g, np.zeros(W), 1e-5, np.float64)
+    assert np.abs(rt.download(d_p) - want).max() < 3e-5
+
+
 MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17]       # rows of 72 requests
 
 
