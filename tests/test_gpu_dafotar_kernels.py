@@ -315,6 +315,28 @@ def test_streams_of_whole_pieces(dev, S, W, parts):
 MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17]       # rows of 72 requests
 
 
+def test_short_convolution_of_many_requests(dev):
+    """More requests than a wave adds up at once, of no, one and several runs of rows; padding behind the last."""
+    rt, k = dev
+    rng = np.random.default_rng(3)
+    C, taps, R, T = 16, 4, len(MANY), sum(MANY)
+    w = rng.normal(0, 0.7, (C, taps)).astype(np.float32)
+    x = rng.normal(size=(T + 3, C)).astype(np.float32)
+    state = rt.zeros((R, (taps - 1) * C), "float32")
+    out = up(rt, np.full((T + 3, C), 7.0, np.float32))
+    q_start = np.concatenate([[0], np.cumsum(MANY)])
+    k.zk_conv_rows(up(rt, x).ptr, C, None, up(rt, w).ptr, None, state.ptr, (taps - 1) * C, 0, i32(rt, q_start).ptr,
+                   i32(rt, range(R)).ptr, out.ptr, C, T + 3, R, max(MANY), C, taps, 1, 0, rt.stream)
+    got, st = rt.download(out), rt.download(state).reshape(R, taps - 1, C)
+    for r in range(R):
+        rows = x[q_start[r]:q_start[r + 1]].astype(np.float64)
+        back = np.concatenate([np.zeros((taps - 1, C)), rows])
+        want = rows + sum(w[:, j] * back[j:j + len(rows)] for j in range(taps))
+        assert not len(rows) or np.abs(got[q_start[r]:q_start[r + 1]] - want).max() < 3e-5, r
+        assert np.array_equal(st[r], back[::-1][:taps - 1].astype(np.float32)), r
+    assert not got[T:].any()
+
+
 def test_matrix_memory_of_many_requests(dev):
     """The chunks of a step side by side, over more requests than a wave adds up at once."""
     rt, k = dev

@@ -11,6 +11,10 @@
 // once a run.  Runs are counted from the request's first token of the step: only the first of
 // them reads the state (span >= taps - 1), and its threads renew it, each its own columns, after
 // they have read them.  One launch serves every kind of step.
+//
+// Few bytes (5.8 MB at 708 rows of 2,048): the time is the launch and one trip to memory, so a run's rows are
+// all asked for before the first is used, and blocks are narrow until the chip is full.  (Row after row in
+// blocks of 256 threads, a grid of the longest portion's runs for every request: 9.1 us; so 7.4.)
 #include "common.h"
 #include "packed_call.h"
 
@@ -21,21 +25,23 @@ extern "C" int zk_steplist_register(const char* name, int nargs, void* fn);
 #define CONV_SPAN 8
 #define CONV_MOST_TAPS (CONV_SPAN + 1)
 
+// V channels of a row as they lie in memory, and their values
+template <int V>
+struct ConvRaw {
+  act_t v[V] __attribute__((aligned(sizeof(act_t) * V > 16 ? 16 : sizeof(act_t) * V)));
+};
+template <int V>
+__device__ __forceinline__ ConvRaw<V> conv_raw(const act_t* p) {
+  return *(const ConvRaw<V>*)p;
+}
+template <int V>
+__device__ __forceinline__ void conv_values(const ConvRaw<V>& r, float (&v)[V]) {
+#pragma unroll
+  for (int e = 0; e < V; e++) v[e] = to_f32(r.v[e]);
+}
 template <int V>
 __device__ __forceinline__ void conv_get(const act_t* p, float (&v)[V]) {
-  if constexpr (V == 8) {
-#if ZSE_ACT_BF16
-    typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-    const b8 q = *(const b8*)p;
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (float)q[e];
-#else
-    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-#endif
-  } else {
-    v[0] = to_f32(p[0]);
-  }
+  conv_values<V>(conv_raw<V>(p), v);
 }
 template <int V>
 __device__ __forceinline__ void conv_put(act_t* p, const float (&v)[V]) {
@@ -81,25 +87,33 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
                                                         int slot_words, int offset_words, const int* __restrict__ q_start,
                                                         const int* __restrict__ slot_of_req, act_t* __restrict__ out,
                                                         int ld_out, int T, int R, int C, int taps_given, int residual,
-                                                        int act) {
+                                                        int act, int one_run) {
   constexpr int MOST = TAPS ? TAPS : CONV_MOST_TAPS, BACK = MOST > 1 ? MOST - 1 : 1;
   const int taps = TAPS ? TAPS : taps_given;
-  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * V;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V;
+  Piece run;
+  bool found;
+  if (one_run) {                         // no request has more than one run: block x is request x's
+    run.r = blockIdx.x;
+    found = run.r < R;
+    run.t0 = q_start[run.r];
+    run.n = found ? q_start[run.r + 1] - run.t0 : 0;
+    run.first = 0;
+    if (found && run.n <= 0) return;
+  } else {
+    found = find_piece(q_start, R, CONV_SPAN, blockIdx.x, run);      // (all lanes of a wave call it)
+  }
   if (c >= C) return;
-  const int r = blockIdx.z, first = blockIdx.y * CONV_SPAN;
-  const int t0 = q_start[r];
-  if (r == R) {                          // rows behind the last request: padding of a captured step
-    if (first == 0) {
+  if (!found) {                          // the grid's last: padding of a captured step, behind the last request
+    if (blockIdx.x == gridDim.x - 1) {
       float zero[V];
 #pragma unroll
       for (int e = 0; e < V; e++) zero[e] = 0.f;
-      for (int t = t0; t < T; t++) conv_put<V>(out + (size_t)t * ld_out + c, zero);
+      for (int t = q_start[R]; t < T; t++) conv_put<V>(out + (size_t)t * ld_out + c, zero);
     }
     return;
   }
-  const int n = q_start[r + 1] - t0;
-  if (first >= n) return;
-  const int last = min(n, first + CONV_SPAN);
+  const int t0 = run.t0, n = run.n, first = run.first, last = min(n, first + CONV_SPAN);
   float ib[V], b0[V], wt[MOST][V];
 #pragma unroll
   for (int e = 0; e < V; e++) {
@@ -113,7 +127,11 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
 #pragma unroll
     for (int e = 0; e < V; e++) v[e] += ib[e];
   };
-  float* st = taps > 1 ? state + (size_t)slot_of_req[r] * slot_words + offset_words + c : nullptr;
+  // the run's rows as they lie in memory (a row past the last: the last again)
+  ConvRaw<V> rows[CONV_SPAN];
+#pragma unroll
+  for (int i = 0; i < CONV_SPAN; i++) rows[i] = conv_raw<V>(x + (size_t)(t0 + min(first + i, last - 1)) * ld_in + c);
+  float* st = taps > 1 ? state + (size_t)slot_of_req[run.r] * slot_words + offset_words + c : nullptr;
   // back[b]: the row b + 1 places before the current token
   float back[BACK][V];
 #pragma unroll
@@ -144,11 +162,16 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
         conv_put_state<V>(st + (size_t)a * C, v);
       }
   }
-  for (int i = first; i < last; i++) {
-    float cur[V], acc[V];
-    input(i, cur);
 #pragma unroll
-    for (int e = 0; e < V; e++) acc[e] = b0[e];
+  for (int i = 0; i < CONV_SPAN; i++) {
+    if (first + i >= last) break;
+    float cur[V], acc[V];
+    conv_values<V>(rows[i], cur);
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+      cur[e] += ib[e];
+      acc[e] = b0[e];
+    }
 #pragma unroll
     for (int b = BACK - 1; b >= 0; b--)
       if (b < taps - 1) {
@@ -173,7 +196,7 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
       if (residual) acc[e] = cur[e] + acc[e];
       if (act == 1) acc[e] = acc[e] / (1.0f + expf(-acc[e]));      // silu
     }
-    conv_put<V>(out + (size_t)(t0 + i) * ld_out + c, acc);
+    conv_put<V>(out + (size_t)(t0 + first + i) * ld_out + c, acc);
 #pragma unroll
     for (int b = BACK - 1; b > 0; b--)
 #pragma unroll
@@ -207,16 +230,18 @@ int zk_conv_rows(const void* x, int ld_in, const float* in_bias, const float* w,
   auto aligned = [](const void* p, size_t n) { return (uintptr_t)p % n == 0; };
   const bool vec = C % 8 == 0 && ld_in % 8 == 0 && ld_out % 8 == 0 && aligned(x, 16) && aligned(out, 16) &&
                    (taps == 1 || (aligned(state, 16) && slot_words % 4 == 0 && offset_words % 4 == 0));
-  const int runs = max_q_len > 0 ? (max_q_len + CONV_SPAN - 1) / CONV_SPAN : 1;
-  ZK_REQUIRE(runs <= 65535, "zk_conv_rows: too many tokens");
+  ZK_REQUIRE(max_q_len <= 65535 * CONV_SPAN, "zk_conv_rows: too many tokens");
+  // the step's runs, at most (full ones and every request's last), and one block more for the padding behind the last request
+  const int one_run = max_q_len <= CONV_SPAN, runs = (one_run ? R : T / CONV_SPAN + R) + 1;
   const int per = vec ? 8 : 1, columns = (C + per - 1) / per;
   // few runs: narrow blocks, so that they spread over the compute units
-  const int threads = (long long)((columns + 255) / 256) * runs * R >= 512 ? 256 : 64;
-  dim3 grid((columns + threads - 1) / threads, runs, R + 1);
+  const int threads = (long long)((columns + 255) / 256) * runs >= 512 ? 256 : 64;
+  ZK_REQUIRE((columns + threads - 1) / threads <= 65535, "zk_conv_rows: too many channels");
+  dim3 grid(runs, (columns + threads - 1) / threads);
 #define LAUNCH(V, N)                                                                                                  \
   conv_rows_kernel<V, N><<<grid, threads, 0, (hipStream_t)stream>>>((const act_t*)x, ld_in, in_bias, w, bias, state,  \
                                                                     slot_words, offset_words, q_start, slot_of_req,   \
-                                                                    (act_t*)out, ld_out, T, R, C, taps, residual, act)
+                                                                    (act_t*)out, ld_out, T, R, C, taps, residual, act, one_run)
   if (vec) {
     if (taps == 2) LAUNCH(8, 2);
     else if (taps == 3) LAUNCH(8, 3);
