@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8 && !PAIR) ? 2 : 1) voi
     }
 #pragma unroll
     for (int e = 0; e < 16; e++) mt = fmaxf(mt, s[e]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = wave_max32(mt);
     const float m_new = mt > m_run + 8.f ? mt : m_run;      // the reference follows the maximum lazily
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const bool moved = m_new > m_run;
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256, (HD16 <= 8 && VD16 <= 8 && !PAIR) ? 2 : 1) voi
       s[e] = pe;
       rs += pe;
     }
-    rs += __shfl_xor(rs, 32, 64);
+    rs = wave_add32(rs);
     l_run = l_run * corr + rs;
     m_run = m_new;
     bf16x8 pb[2];
@@ -642,7 +642,7 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
     }
 #pragma unroll
     for (int e = 0; e < 16; e++) mt = fmaxf(mt, s[e]);
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = wave_max32(mt);
     const float m_new = mt > m_run + 8.f ? mt : m_run;      // the maximum is followed lazily
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const bool moved = m_new > m_run;
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(NW * 64, (HD16 <= 8 && VD16 <= 8 && NW <= 4) ? 2 : 
       s[e] = pe;
       rs += pe;
     }
-    rs += __shfl_xor(rs, 32, 64);
+    rs = wave_add32(rs);
     l_run = l_run * corr + rs;
     m_run = m_new;
     bf16x8 pb[2];
@@ -1179,7 +1179,8 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
     block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / SPAN, kept_blocks) - kept_blocks;
   const int key0 = block_x * SPAN + 32 * wave;
   const int* table = p.block_table + (size_t)r * p.max_blocks;
-  const int hd = p.hd, vd = p.vd, bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
+  constexpr int hd = HD32 * 32, vd = VD16 * 16;
+  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
   // The pages of the wave's keys are asked for before the request's length is known, beside it:
   // where a key lies follows from the block alone.  A key past the context is masked below; a
   // hole in the table reads page 0, which the caller keeps cleared, and the places of a
@@ -1249,7 +1250,8 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
       }
     };
     // Values of 256 channels are asked for after the score products have used up the keys: with
-    // both at once a wave has 199 registers, two waves a SIMD, and the CU less on its way.
+    // both at once a wave has 199 registers, two waves a SIMD, and the CU less on its way (also where blocks are few: 8 requests of
+    // 500 keys 11.1 us with the join, beside the keys 12.0; 4 of 3,000 17.1 and 17.8).
     constexpr bool LATE = DT > 8;
     if (!LATE) load_v();
     // the queries are in LDS (the compiler does not know that the reads below depend on them)
@@ -1274,8 +1276,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
         s[t][i] = (col_ok && (key >= row_lo || key < p.keep) && key <= pos) ? v : -INFINITY;
         m_run = fmaxf(m_run, s[t][i]);
       }
-    m_run = fmaxf(m_run, __shfl_xor(m_run, 16, 64));
-    m_run = fmaxf(m_run, __shfl_xor(m_run, 32, 64));
+    m_run = wave_max16_32(m_run);
     const float m_use = m_run == -INFINITY ? 0.f : m_run;
     bf16x8 pb8;
 #pragma unroll
@@ -1286,8 +1287,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
         l_run += s[t][i];
         pb8[4 * t + i] = (__bf16)s[t][i];
       }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = wave_add16_32(l_run);
     bf16x8 rest8;          // (wide weights) what the rounding left
 #pragma unroll
     for (int t = 0; t < 2; t++)
@@ -1363,7 +1363,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
     block_x += max(first_key(p, max(p.ctx_len[r] - 1, 0)) / span, kept_blocks) - kept_blocks;
   const int chunk = block_x * 4 + wave;
   const int* table = p.block_table + (size_t)r * p.max_blocks;
-  const int hd = p.hd, vd = p.vd, bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
+  constexpr int hd = HD32 * 32, vd = VD16 * 16;
+  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv;
   // The pages of the chunk's (up to two) tiles are asked for before the request's length is
   // known, beside it: where a key lies follows from the chunk alone.  A key past the context is
   // masked below; a hole in the table reads page 0, which the caller keeps cleared, and the
@@ -1464,8 +1465,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
         s[t][i] = v;
         mt = fmaxf(mt, v);
       }
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    mt = wave_max16_32(mt);
     const float m_new = fmaxf(m_run, mt);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float corr = __builtin_amdgcn_exp2f(m_run - m_use);
@@ -1480,8 +1480,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
         pb8[4 * t + i] = (__bf16)pe;
         s[t][i] = pe;
       }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
+    rs = wave_add16_32(rs);
     l_run = l_run * corr + rs;
     m_run = m_new;
 #pragma unroll

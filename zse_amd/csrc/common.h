@@ -91,6 +91,28 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(v, wave_dpp<ZSE_DPP_XOR1>(v));
 }
 
+// Sums and maxima over a lane and its partners 16, 32 or both away (in that order).
+__device__ __forceinline__ float wave_add32(float v) {
+  float a = 0.f, b = 0.f;
+  wave_pair32(v, a, b);
+  return a + b;
+}
+__device__ __forceinline__ float wave_max32(float v) {
+  float a = 0.f, b = 0.f;
+  wave_pair32(v, a, b);
+  return fmaxf(a, b);
+}
+__device__ __forceinline__ float wave_add16_32(float v) {
+  float a = 0.f, b = 0.f;
+  wave_pair16(v, a, b);
+  return wave_add32(a + b);
+}
+__device__ __forceinline__ float wave_max16_32(float v) {
+  float a = 0.f, b = 0.f;
+  wave_pair16(v, a, b);
+  return wave_max32(fmaxf(a, b));
+}
+
 // Running sums and maxima over a wave's lanes (each lane's own value included): rows of 16 lanes by shifts, then a row's
 // last lane handed to the next row, then lane 31 to the upper half.  ``none``: what a lane without a neighbour joins.
 template <int CTRL, int ROWS>
