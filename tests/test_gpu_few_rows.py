@@ -1,4 +1,7 @@
-"""Decoded tokens' attention over few and many parts: the same bits where the sums are the same."""
+"""Products of up to 16 rows whose addresses go by whole groups of steps, or K in ranges over few long strips, and decoded
+tokens' attention in its forms for few and for many blocks: against 64-bit arithmetic, and the same bits where the sums are the same."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -9,6 +12,79 @@ def dev():
     from zse_amd.runtime.device import Runtime
     rt = Runtime.get()
     return rt, rt.kernels("bfloat16")
+
+
+# one group; not whole (288); a last strip that is not full; few long strips in ranges (two, four, five of them), few short ones
+# and 224 that nearly fill the chip (no ranges); more strips than compute units in ranges
+@pytest.mark.parametrize("N,K,ranges", [(48, 256, 0), (64, 288, 0), (1000, 1024, 0), (2048, 8192, 2), (1024, 4096, 4), (2304, 9216, 5),
+                                        (2048, 2048, 0), (3584, 4096, 0), (4608, 4096, 4)])
+@pytest.mark.parametrize("gated", [0, 1])
+def test_products(N, K, ranges, gated):
+    from zse_amd.weights.safetensors import bf16_bits_to_f32, f32_to_bf16_bits
+    rt, k = dev()
+    if gated and N * K > 1 << 22 or gated and N % 16:
+        pytest.skip("the gated product has no ranges and takes whole strips")
+    rng = np.random.default_rng(N + K)
+    bits = lambda *shape: f32_to_bf16_bits(rng.normal(size=shape).astype(np.float32) * K ** -0.25)
+    a, w = bits(16, K), bits(N * (1 + gated), K)
+    A, W = rt.upload(a, "bfloat16"), rt.upload(w, "bfloat16")
+    S = rt.empty((-(-w.shape[0] // 16) * 16, K), "bfloat16")
+    k.zk_strip_layout(W.ptr, S.ptr, *w.shape, rt.stream)
+    ws = rt.zeros((k.zk_gemm_bf16_workspace() // 4,), "float32")
+    want = bf16_bits_to_f32(a).astype(np.float64) @ bf16_bits_to_f32(w).astype(np.float64).T
+    if gated:
+        want = np.maximum(want[:, :N], 0) * want[:, N:]
+    rows = {}
+    for M in (1, 7, 16):
+        for ldc in (N, N + 8):
+            C = rt.upload(np.full((M + 1, ldc), 0x4040, np.uint16), "bfloat16")
+            k.zk_gemm_bf16(A.ptr, K, S.ptr, C.ptr, ldc, 0, M, N, K, 5 if gated else 0, 0.0, 1, ws.ptr, ws.nbytes, None, rt.stream)
+            got = rt.download_f32(C)
+            # a result rounded to 8 bits of mantissa; K float additions of products of size K^-0.5
+            assert (np.abs(got[:M, :N] - want[:M]) <= np.abs(want[:M]) * 2.0 ** -8 + 1e-4 * (1 + 3 * gated)).all(), (M, ldc)
+            assert (got[M:] == 3.0).all() and (got[:, N:] == 3.0).all()
+            rows.setdefault("whole", got[0, :N])
+            assert np.array_equal(got[0, :N], rows["whole"])       # a row does not know of the others
+        if gated:
+            continue
+        parts = ctypes.c_int(0)
+        C = rt.zeros((M, N), "bfloat16")
+        k.zk_gemm_bf16(A.ptr, K, S.ptr, C.ptr, N, 0, M, N, K, 0, 0.0, 1, ws.ptr, ws.nbytes, ctypes.byref(parts), rt.stream)
+        assert parts.value == ranges, (M, parts.value)
+        if ranges:
+            planes = rt.download(ws)[:ranges * M * N].reshape(ranges, M, N)
+            # float sums of K products of size K^-0.5, in another order
+            assert np.abs(planes.astype(np.float64).sum(0) - want[:M]).max() < 2e-5 * max(1.0, np.abs(want).max())
+            rows.setdefault("ranges", planes[:, 0])
+            assert np.array_equal(planes[:, 0], rows["ranges"])
+
+
+@pytest.mark.parametrize("nh,nkv,hd,K", [(4, 2, 64, 256), (2, 1, 256, 2304), (3, 1, 16, 512), (4, 0, 128, 1024)])
+@pytest.mark.parametrize("M", [1, 16])
+def test_the_rotating_product_gives_the_bits_of_product_and_rotation(M, nh, nkv, hd, K):
+    from zse_amd.weights.safetensors import f32_to_bf16_bits
+    rt, k = dev()
+    rng = np.random.default_rng(hd + K)
+    N, bs = (nh + 2 * nkv) * hd, 16
+    up = lambda x: rt.upload(f32_to_bf16_bits(np.ascontiguousarray(x, np.float32)), "bfloat16")
+    A, W, S = up(rng.normal(size=(M, K))), up(rng.normal(size=(N, K)) * K ** -0.5), rt.empty((N, K), "bfloat16")
+    k.zk_strip_layout(W.ptr, S.ptr, N, K, rt.stream)
+    pos = rt.upload(rng.integers(0, 8000, M).astype(np.int32))
+    slots = rt.upload((rng.permutation(2 * bs)[:M]).astype(np.int32))
+    freq = rt.upload((10000.0 ** (-np.arange(hd // 2) * 2 / hd)).astype(np.float32))
+    got = []
+    for fused in (True, False):
+        Q = rt.zeros((M, N), "bfloat16")
+        kc, vc = rt.zeros((2 * max(nkv, 1) * bs * hd,), "bfloat16"), rt.zeros((2 * max(nkv, 1) * bs * hd,), "bfloat16")
+        if fused:
+            k.zk_qkv_rope_bf16(A.ptr, K, S.ptr, Q.ptr, N, M, K, 1, pos.ptr, slots.ptr if nkv else None, freq.ptr, kc.ptr, vc.ptr, nh, nkv,
+                               hd, bs, 1, rt.stream)
+        else:
+            k.zk_gemm_bf16(A.ptr, K, S.ptr, Q.ptr, N, 0, M, N, K, 0, 0.0, 1, None, 0, None, rt.stream)
+            k.zk_rope_cache_write(Q.ptr, pos.ptr, slots.ptr if nkv else None, freq.ptr, hd, kc.ptr, vc.ptr, M, nh, nkv, hd, bs, 1, rt.stream)
+        got.append((rt.download_f32(Q)[:, :nh * hd], rt.download_f32(kc), rt.download_f32(vc)))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
 
 
 @pytest.mark.parametrize("nh,nkv,hd", [(8, 4, 256), (8, 2, 128), (16, 1, 64)])

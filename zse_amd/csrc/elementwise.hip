@@ -9,6 +9,8 @@
 // of K and V into pages :961-1012.
 #include "common.h"
 
+#include <type_traits>
+
 #include <algorithm>
 
 ZK_DEFINE_HOST_SIDE
@@ -350,29 +352,34 @@ __global__ __launch_bounds__(1024) void norm_add_norm_wide_kernel(
     }
   }
   if (parts > 0) {
-    // a plane past the last is read from the last and not added; the planes are added in order
-    for (int p0 = 1; p0 < parts; p0 += 8) {
-      float t[MAXV][8][4];
+    // eight planes a turn, or four where there are no more; a plane past the last is read from the last and not
+    // added; the planes are added in order
+    auto turn = [&](int p0, auto planes) {
+      constexpr int NP = decltype(planes)::value;
+      float t[MAXV][NP][4];
 #pragma unroll
       for (int j = 0; j < MAXV; j++) {
         const int i = threadIdx.x * 4 + j * 4096;
         if (i < H) {
 #pragma unroll
-          for (int q = 0; q < 8; q++) load4<float>(sf + (size_t)min(p0 + q, parts - 1) * plane + i, t[j][q]);
+          for (int q = 0; q < NP; q++) load4<float>(sf + (size_t)min(p0 + q, parts - 1) * plane + i, t[j][q]);
         }
       }
 #pragma unroll
       for (int j = 0; j < MAXV; j++) {
         if (threadIdx.x * 4 + j * 4096 < H) {
 #pragma unroll
-          for (int q = 0; q < 8; q++)
+          for (int q = 0; q < NP; q++)
             if (p0 + q < parts) {
 #pragma unroll
               for (int e = 0; e < 4; e++) v[j][e] += t[j][q][e];
             }
         }
       }
-    }
+    };
+    if (parts <= 5) turn(1, std::integral_constant<int, 4>{});
+    else
+      for (int p0 = 1; p0 < parts; p0 += 8) turn(p0, std::integral_constant<int, 8>{});
 #pragma unroll
     for (int j = 0; j < MAXV; j++)
       if (threadIdx.x * 4 + j * 4096 < H) {

@@ -22,6 +22,7 @@
 #include "common.h"
 #include "gemm_bf16_static.h"
 
+#include <algorithm>
 #include <mutex>
 
 // Where a product that splits K over blocks leaves its partial sums.  ``strict``: the split is
@@ -159,7 +160,12 @@ __device__ __forceinline__ void store4(__bf16* dst, const float (&x)[4]) {
 // alone: with loads under per-lane conditions it waits for every load before each group, and
 // the next group's loads, just issued, no longer overlap anything (down projection of 2304 x
 // 9216 at 8 rows: 14 us against 9).
-template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false>
+// WHOLE (EXACT, up to 16 rows, K in whole groups of 8 steps, every launch of a real model's sizes): a load's address is a scalar that
+// moves on from group to group, a lane's own offset that does not, and a constant.  Worked out for each load from its step (clamped, in 64
+// bits), the addresses of a group are a hundred instructions that a wave issues one every fourth cycle in
+// front of its loads (us, 8 rows: 4,096 columns of K 2,304 6.3 -> 5.5, 2,304 of 2,048
+// 5.0 -> 4.4, 2,304 of 9,216 13.3 -> 12.4; a step of 8 decoded tokens of the 2B shapes 2,319 -> 2,278).  The same sums.
+template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false, bool WHOLE = false>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __restrict__ A, int lda,
                                                           const __bf16* __restrict__ W,
                                                           void* __restrict__ C, int ldc, int c_is_f32,
@@ -167,6 +173,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
                                                           int w_strip, RopeStore rs,
                                                           float* __restrict__ partials = nullptr, int ksplit = 1) {
   static_assert(!ROPE || (MT == 1 && !GATED), "the rotating epilogue takes up to 16 rows");
+  static_assert(!WHOLE || (EXACT && MT == 1), "whole groups: strips, up to 16 rows");
   constexpr int NS = GATED ? 2 : 1;
   __shared__ f32x4 red[NW - 1][NS][MT][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -224,7 +231,35 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
   const int gy1 = SPLIT ? ((int)blockIdx.y + 1) * total_groups / ksplit : total_groups;
   const int gw0 = gy0 + uwave * (gy1 - gy0) / NW, gw1 = gy0 + (uwave + 1) * (gy1 - gy0) / NW;
   const int run_lo = gw0 * STEPS, run_n = (gw1 - gw0) * STEPS;      // the wave's run of steps
+  // WHOLE: the wave's run in each strip and in A (scalars), and where the lane reads in a step of them
+  const char* wrun[NS];
+  const char* arun = (const char*)A + (size_t)run_lo * 64;
+  unsigned wlane = lane * 16;
+  const unsigned alane = (unsigned)min(r, M - 1) * (unsigned)lda * 2 + kq * 16;
+  if (WHOLE) {
+    int first = strip0;
+    if (ROPE) {
+      first = (head * rs.hd + hpos) / 16;
+      const int row = head * rs.hd + hpos + (r < 8 ? r : rs.hd / 2 + r - 8);
+      wlane = (unsigned)(row / 16 - first) * (unsigned)ksteps * 1024 + (16 * kq + row % 16) * 16;
+    }
+    wrun[0] = (const char*)W + ((size_t)first * ksteps + run_lo) * 1024;
+    if (GATED) wrun[NS - 1] = (const char*)W + ((size_t)strip1 * ksteps + run_lo) * 1024;
+  }
   auto fetch = [&](int s0, bf16x8 (&wf)[NS][STEPS], bf16x8 (&af)[MT][STEPS]) {
+    if constexpr (WHOLE) {
+      const char* a = arun + (size_t)s0 * 64;
+#pragma unroll
+      for (int g = 0; g < NS; g++) {
+        // (a constant in an address reaches 4 KB)
+        const char *lo = wrun[g] + (size_t)s0 * 1024, *hi = lo + 4096;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) wf[g][s] = *(const bf16x8*)((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane);
+      }
+#pragma unroll
+      for (int s = 0; s < STEPS; s++) af[0][s] = *(const bf16x8*)(a + s * 64 + alane);
+      return;
+    }
     if (EXACT) {
       // A whole group of steps, counted from the start of the wave's run; only the last group
       // of K may hold fewer steps, and then the steps past K read K's last step again and count
@@ -272,15 +307,16 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
   } else if (s_begin < s_end) {
     fetch(s_begin, wf0, af0);
   }
-  // the angles of the lane's four pairs, worked out while the first loads are on their way
-  float sn[4], cs[4];
+  // the angles of the lane's four pairs, worked out by four waves while the first loads are on their way (all by
+  // the one that stores, they are 0.7 us that the others wait for)
+  __shared__ float2 turn[ROPE ? 4 : 1][64];
   int slot = -1;
-  if (ROPE && wave == 0) {
-    if (head >= rs.nh && rs.slot_map) slot = rs.slot_map[min(r, M - 1)];
-    if (head < rs.nh + rs.nkv) {
-      const float pos = (float)rs.positions[min(r, M - 1)];
-#pragma unroll
-      for (int i = 0; i < 4; i++) sincosf(pos * rs.inv_freq[hpos + 4 * (kq & 1) + i], &sn[i], &cs[i]);
+  if (ROPE) {
+    if (wave == 0 && head >= rs.nh && rs.slot_map) slot = rs.slot_map[min(r, M - 1)];
+    if (wave < 4 && head < rs.nh + rs.nkv) {
+      float sn, cs;
+      sincosf((float)rs.positions[min(r, M - 1)] * rs.inv_freq[hpos + 4 * (kq & 1) + wave], &sn, &cs);
+      turn[wave][lane] = make_float2(sn, cs);
     }
   }
   if (EXACT) {
@@ -361,7 +397,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
         const float y = __shfl_xor(x[i], 32);
         if (head < rs.nh + rs.nkv) {
           float ra, rb;
-          rotate_pair(first ? x[i] : y, first ? y : x[i], sn[i], cs[i], ra, rb);
+          const float2 t = turn[ROPE ? i : 0][lane];
+          rotate_pair(first ? x[i] : y, first ? y : x[i], t.x, t.y, ra, rb);
           x[i] = first ? ra : rb;
         }
       }
@@ -389,6 +426,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
       continue;
     }
     if (m >= M) continue;
+    if (WHOLE && !c_is_f32 && n0 + 16 <= N && (((uintptr_t)C | (unsigned)ldc * 2) & 7) == 0) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i] = GATED ? epi_gate(v[0][i], v[NS - 1][i], epi, cap) : epi_unary(v[0][i], epi, cap);
+      store4((__bf16*)C + (size_t)m * ldc + n0 + 4 * kq, x);
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int n = n0 + 4 * kq + i;
@@ -1111,34 +1155,55 @@ static int launch_skinny(const void* A, int lda, const void* W, void* C, int ldc
   // idle.  Splitting K into ks ranges makes ks times the blocks of 1/ks the length, and the time
   // of the fullest CU goes with ceil(strips ks / 256) / ks.  That pays where strips are more
   // than the CUs and spread unevenly (N = 4608 with K = 36864 at 8 rows: 87 -> 50 us with eight
-  // ranges); with fewer strips than CUs it was measured three times and lost each time (144
-  // strips, two and eight ranges: the product then goes as fast as memory gives to this pattern
-  // of reads whatever the number of CUs, and the shorter blocks only add their start-up).
+  // ranges), and where they are fewer and long (blocks of four waves; us, 1 and 8 rows, without the reader's
+  // half a microsecond and more: 144 strips of 9,216 in five ranges 10.3 -> 9.2 and 12.3 -> 9.8, 128 of 8,192 in two 9.3 -> 8.2 and
+  // 11.2 -> 8.4, 64 of 4,096 in four 4.1 -> 3.5 and 5.3 -> 3.7), not where they are short (128 of 2,048 in two 3.4 -> 3.5 and
+  // 3.9 -> 3.7) or nearly fill the chip (224 of 14,336 in eight 19.1 -> 19.2 and 20.1 -> 20.5).
   // Only where the reader adds up the partial sums itself (the norm kernel, through `parts`):
   // a joining launch would cost what the split gains.
   int ksplit = 1;
   float* partials = (float*)wsp.ptr;
   const size_t npad = (size_t)grid.x * 16;
-  if (!GATED && mt == 1 && w_strip && grid.x > 256 && parts != nullptr && partials != nullptr &&
+  bool few_long = false;
+  if (!GATED && mt == 1 && w_strip && parts != nullptr && partials != nullptr &&
       (uintptr_t)partials % 16 == 0 && joinable_by_reader(N, ldc, c_is_f32, epi)) {
     auto longest = [&](int ks) { return (double)(((long)grid.x * ks + 255) / 256) / ks; };
-    double best = longest(1);
-    for (int ks = 2; ks <= 8; ks *= 2) {
-      if (K / ks < 1024 || (size_t)ks * M * npad * sizeof(float) > wsp.split_bytes()) break;
-      if (longest(ks) < 0.97 * best && longest(ks) <= 0.85 * longest(1)) {
-        best = longest(ks);
-        ksplit = ks;
+    if (grid.x <= 256) {
+      // microseconds: the fullest CU at 25 KB, the chip at 6.1 MB, the reader's additions
+      const double kb = K * 0.032, chip = grid.x * kb / 6100;
+      auto price = [&](int ks) { return std::max(longest(ks) * kb / 25, chip) + (ks > 1 ? 0.5 + 0.05 * ks : 0.0); };
+      double best = price(1) - 1.5;
+      for (int ks = 2; ks <= 6 && K / ks >= 1024 && (size_t)ks * M * npad * sizeof(float) <= wsp.split_bytes(); ks++)
+        if (price(ks) < best) {
+          best = price(ks);
+          ksplit = ks;
+          few_long = true;
+        }
+    } else {
+      double best = longest(1);
+      for (int ks = 2; ks <= 8; ks *= 2) {
+        if (K / ks < 1024 || (size_t)ks * M * npad * sizeof(float) > wsp.split_bytes()) break;
+        if (longest(ks) < 0.97 * best && longest(ks) <= 0.85 * longest(1)) {
+          best = longest(ks);
+          ksplit = ks;
+        }
       }
     }
     if (ksplit > 1 && (size_t)ksplit * M * npad * sizeof(float) > wsp.bytes)
       return wsp.too_small((size_t)ksplit * M * npad * sizeof(float));
     grid.y = ksplit;
   }
+  // rows of A within reach of a lane's own offset
+  const bool whole = w_strip && mt == 1 && K % 256 == 0 && lda <= (1 << 26);
   // few strips: eight waves a strip keep enough loads in flight
-  const bool wide = (long)grid.x * ksplit < 512 && K / ksplit >= 2048 && mt <= 2;
+  const bool wide = !few_long && (long)grid.x * ksplit < 512 && K / ksplit >= 2048 && mt <= 2;
 #define ZK_SKINNY(MT_, NW_)                                                                           \
   do {                                                                                                \
-    if (w_strip)                                                                                      \
+    if (MT_ == 1 && whole)                                                                            \
+      gemm_skinny_kernel<1, GATED, NW_, false, true, false, true><<<grid, NW_ * 64, 0, s>>>(          \
+          (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
+          partials, 1);                                                                               \
+    else if (w_strip)                                                                                      \
       gemm_skinny_kernel<MT_, GATED, NW_, false, true><<<grid, NW_ * 64, 0, s>>>(                     \
           (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
           partials, 1);                                                                               \
@@ -1147,22 +1212,20 @@ static int launch_skinny(const void* A, int lda, const void* W, void* C, int ldc
           (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
           partials, 1);                                                                               \
   } while (0)
+#define ZK_SPLIT(NW_, WHOLE_)                                                                        \
+  gemm_skinny_kernel<1, false, NW_, false, true, true, WHOLE_><<<grid, NW_ * 64, 0, s>>>(             \
+      (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, partials, ksplit)
   if (ksplit > 1) {
     if constexpr (!GATED) {
-      if (wide)
-        gemm_skinny_kernel<1, false, 8, false, true, true><<<grid, 8 * 64, 0, s>>>(
-            (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{},
-            partials, ksplit);
-      else
-        gemm_skinny_kernel<1, false, 4, false, true, true><<<grid, 4 * 64, 0, s>>>(
-            (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{},
-            partials, ksplit);
+      if (wide) { if (whole) ZK_SPLIT(8, true); else ZK_SPLIT(8, false); }
+      else { if (whole) ZK_SPLIT(4, true); else ZK_SPLIT(4, false); }
     }
   } else if (mt == 1) { if (wide) ZK_SKINNY(1, 8); else ZK_SKINNY(1, 4); }
   else if (mt == 2) { if (wide) ZK_SKINNY(2, 8); else ZK_SKINNY(2, 4); }
   else if (mt == 3) ZK_SKINNY(3, 4);
   else ZK_SKINNY(4, 4);
 #undef ZK_SKINNY
+#undef ZK_SPLIT
   if (ksplit > 1) *parts = ksplit;
   return zk_launch_status("zk_gemm_bf16 (skinny)");
 }
@@ -1194,13 +1257,14 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
                v_transposed};
   dim3 grid(N / 16);
   hipStream_t s = (hipStream_t)stream;
-#define ZK_QKV(NW_, EX_)                                                                                  \
-  gemm_skinny_kernel<1, false, NW_, true, EX_><<<grid, NW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, Q, \
-                                                                         ldq, 0, M, N, K, EPI_NONE, 0.f, w_strip, rs)
+  const bool whole = w_strip && K % 256 == 0 && lda <= (1 << 26);
+#define ZK_QKV(NW_, EX_, WH_)                                                                                          \
+  gemm_skinny_kernel<1, false, NW_, true, EX_, false, WH_><<<grid, NW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, Q, \
+                                                                                    ldq, 0, M, N, K, EPI_NONE, 0.f, w_strip, rs)
   if (grid.x < 512 && K >= 2048) {
-    if (w_strip) ZK_QKV(8, true); else ZK_QKV(8, false);
+    if (whole) ZK_QKV(8, true, true); else if (w_strip) ZK_QKV(8, true, false); else ZK_QKV(8, false, false);
   } else {
-    if (w_strip) ZK_QKV(4, true); else ZK_QKV(4, false);
+    if (whole) ZK_QKV(4, true, true); else if (w_strip) ZK_QKV(4, true, false); else ZK_QKV(4, false, false);
   }
 #undef ZK_QKV
   return zk_launch_status("zk_qkv_rope_bf16");
