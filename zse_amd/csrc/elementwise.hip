@@ -478,6 +478,24 @@ struct QkvSource {
     for (int p = 1; p < sums; p++) x += planes[p * plane + i];
     return to_f32(from_f32<act_t>(x));
   }
+  // two neighbouring values of an even place
+  __device__ __forceinline__ void at2(size_t i, float v[2]) const {
+    typedef act_t a2 __attribute__((ext_vector_type(2)));
+    if (sums <= 0) {
+      const a2 x = *(const a2*)(rows + i);
+      v[0] = to_f32(x[0]);
+      v[1] = to_f32(x[1]);
+      return;
+    }
+    float2 x = *(const float2*)(planes + i);
+    for (int p = 1; p < sums; p++) {
+      const float2 y = *(const float2*)(planes + p * plane + i);
+      x.x += y.x;
+      x.y += y.y;
+    }
+    v[0] = to_f32(from_f32<act_t>(x.x));
+    v[1] = to_f32(from_f32<act_t>(x.y));
+  }
   __device__ __forceinline__ void at4(size_t i, float v[4]) const {
     if (sums <= 0) {
       load4<act_t>(rows + i, v);
@@ -549,29 +567,52 @@ __global__ void rope_cache_write_kernel(act_t* __restrict__ qkv, QkvSource from,
 
 // The same for the usual case (rotation over the whole head, head_dim a multiple of 8 and at
 // most 512): one block a token, the sines and cosines of the token's angles computed once for
-// all heads, four values a load.
+// all heads, four values a load.  What a thread reads first is asked for before the angles are worked out, and the
+// eight slots beside its own at once (one after the other, as a comparison that ends early reads them, they were up
+// to eight waits for memory).  MANY: so many tokens that the kernel is bound by its accesses, not by its waits: the values
+// are asked for when they are stored, four channels a thread, else before the angles, two.  us, 8 heads and 2 x 4 of 256: 535
+// tokens 5.7 -> 5.4, 1,000 6.6 -> 6.1 (MANY 6.8), 2,048 10.9 -> 9.2 (not MANY 9.8); 32 and 2 x 16 of 128, 2,048 15.1 -> 13.7 (16.7).
 #define ROPE_MAX_HALF 256
+template <bool MANY>
 __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
     act_t* __restrict__ qkv, QkvSource from, const int* __restrict__ positions, const int* __restrict__ slot_map,
     const float* __restrict__ inv_freq, act_t* __restrict__ kcache, act_t* __restrict__ vcache, int nh,
     int nkv, int hd, int bs, int v_transposed) {
   __shared__ float s_sin[ROPE_MAX_HALF], s_cos[ROPE_MAX_HALF];
-  const int t = blockIdx.x, tid = threadIdx.x;
-  const int half = hd / 2;
+  constexpr int FIRST = 2;
+  const int t = blockIdx.x, tid = threadIdx.x, tl = t - t % 8;
+  const int half = hd / 2, ppr = half / 4, items = (nh + nkv) * ppr;
+  const size_t width = (size_t)(nh + 2 * nkv) * hd, row_at = (size_t)t * width;
   const float pos = (float)positions[t];
   const int slot = slot_map ? slot_map[t] : -1;
+  const int beside = slot_map ? slot_map[min(tl + (tid & 7), (int)gridDim.x - 1)] : -1;
+  // q and k heads: pieces of four pairs (i, i + half)
+  float a[FIRST][4], b[FIRST][4];
+#pragma unroll
+  for (int j = 0; j < FIRST; j++) {
+    const int it = min(tid + j * 256, items - 1);
+    const size_t at = row_at + (size_t)(it / ppr) * hd + (it % ppr) * 4;
+    from.at4(at, a[j]);
+    from.at4(at + half, b[j]);
+  }
+  // v of the eight tokens tl .. tl + 7: the block's eighth of the channels, two a thread, from the last thread down (the first ones have more
+  // of q and k), if the slots turn out to be eight in a row
+  const bool eight = v_transposed && bs % 8 == 0 && tl + 7 < (int)gridDim.x;
+  const int pairs = nkv * hd / 2, mine = (pairs + 7) / 8, first = (t - tl) * mine, last = min(first + mine, pairs);
+  const size_t v_at = (size_t)tl * width + (size_t)(nh + nkv) * hd;
+  float v8[8][2];
+  const bool have_v = !MANY && eight && first + 255 - tid < last;
+  if (have_v) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) from.at2(v_at + (size_t)e * width + (first + 255 - tid) * 2, v8[e]);
+  }
   for (int i = tid; i < half; i += 256) sincosf(pos * inv_freq[i], &s_sin[i], &s_cos[i]);
   __syncthreads();
-  const size_t width = (size_t)(nh + 2 * nkv) * hd, row_at = (size_t)t * width;
   act_t* row = qkv + row_at;
   const size_t page = slot >= 0 ? slot / bs : 0, off = slot >= 0 ? slot % bs : 0;
-  // q and k heads: pieces of four pairs (i, i + half)
-  const int ppr = half / 4;
-  for (int it = tid; it < (nh + nkv) * ppr; it += 256) {
+  auto turn = [&](int it, const float (&a)[4], const float (&b)[4]) {
     const int head = it / ppr, i = (it % ppr) * 4;
-    float a[4], b[4], ra[4], rb[4];
-    from.at4(row_at + (size_t)head * hd + i, a);
-    from.at4(row_at + (size_t)head * hd + i + half, b);
+    float ra[4], rb[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       rotate_pair(a[e], b[e], s_sin[i + e], s_cos[i + e], ra[e], rb[e]);
@@ -584,32 +625,63 @@ __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
       store4(dst + i, ra);
       store4(dst + i + half, rb);
     }
+  };
+#pragma unroll
+  for (int j = 0; j < FIRST; j++)
+    if (tid + j * 256 < items) turn(tid + j * 256, a[j], b[j]);
+  for (int it = tid + FIRST * 256; it < items; it += 256) {
+    const size_t at = row_at + (size_t)(it / ppr) * hd + (it % ppr) * 4;
+    from.at4(at, a[0]);
+    from.at4(at + half, b[0]);
+    turn(it, a[0], b[0]);
   }
   // v heads.  Transposed cache: eight tokens in a row of the step whose slots are eight in a
   // row of one page (a prompt portion) go out together, 8 values of a channel per store, each
   // of the eight blocks an eighth of the channels; other tokens are written value by value.
-  if (v_transposed) {
-    const int tl = t - t % 8;
-    bool together = bs % 8 == 0 && tl + 7 < (int)gridDim.x && slot_map != nullptr;
-    int slot0 = -1;
-    if (together) {
-      slot0 = slot_map[tl];
-      together = slot0 >= 0 && slot0 % 8 == 0;
-      for (int e = 1; together && e < 8; e++) together = slot_map[tl + e] == slot0 + e;
-    }
-    if (together) {
-      // the eight tokens' blocks share the (kv head, channel) pairs among them, an eighth each
+  if (MANY && v_transposed && bs % 8 == 0 && tl + 7 < (int)gridDim.x) {
+    const int slot0 = __builtin_amdgcn_readfirstlane(beside);      // (lane 0 holds the first of the eight)
+    if (slot0 >= 0 && slot0 % 8 == 0 && __all(beside == slot0 + (tid & 7))) {
       typedef act_t av8 __attribute__((ext_vector_type(8)));
       const size_t page0 = slot0 / bs, off0 = slot0 % bs;
-      const size_t row0 = (size_t)tl * width;
-      const int items = nkv * hd, mine = (items + 7) / 8, first = (t - tl) * mine;
-      for (int it = first + tid; it < min(first + mine, items); it += 256) {
-        const int kvh = it / hd, d = it % hd;
-        const size_t src = row0 + (size_t)(nh + nkv + kvh) * hd + d;
-        av8 v;
+      const int pieces = nkv * hd / 4, share = (pieces + 7) / 8, begin = (t - tl) * share;
+      for (int it = begin + tid; it < min(begin + share, pieces); it += 256) {
+        const int kvh = it / (hd / 4), d = (it % (hd / 4)) * 4;
+        float v[8][4];
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] = from_f32<act_t>(from.at(src + (size_t)e * width));
-        *(av8*)(vcache + ((page0 * nkv + kvh) * (size_t)hd + d) * bs + off0) = v;
+        for (int e = 0; e < 8; e++) from.at4(v_at + (size_t)kvh * hd + d + (size_t)e * width, v[e]);
+        act_t* vt = vcache + ((page0 * nkv + kvh) * (size_t)hd + d) * bs + off0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          av8 x;
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = from_f32<act_t>(v[e][c]);
+          *(av8*)(vt + (size_t)c * bs) = x;
+        }
+      }
+      return;
+    }
+  }
+  if (!MANY && eight) {
+    const int slot0 = __builtin_amdgcn_readfirstlane(beside);      // (lane 0 holds the first of the eight)
+    if (slot0 >= 0 && slot0 % 8 == 0 && __all(beside == slot0 + (tid & 7))) {
+      typedef act_t av8 __attribute__((ext_vector_type(8)));
+      const size_t page0 = slot0 / bs, off0 = slot0 % bs;
+      auto put = [&](int it, const float (&v)[8][2]) {
+        const int kvh = it * 2 / hd, d = it * 2 % hd;
+        act_t* vt = vcache + ((page0 * nkv + kvh) * (size_t)hd + d) * bs + off0;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          av8 x;
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = from_f32<act_t>(v[e][c]);
+          *(av8*)(vt + (size_t)c * bs) = x;
+        }
+      };
+      if (have_v) put(first + 255 - tid, v8);
+      for (int it = first + 511 - tid; it < last; it += 256) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) from.at2(v_at + (size_t)e * width + it * 2, v8[e]);
+        put(it, v8);
       }
       return;
     }
@@ -876,12 +948,13 @@ int zk_rope_cache_write_sums(void* qkv, const float* planes, int sums, const int
   ZK_REQUIRE(sums == 0 || (planes != nullptr && (uintptr_t)planes % 16 == 0), "zk_rope_cache_write: partial sums must be 16-byte aligned");
   if (T == 0) return 0;
   const QkvSource from{(const act_t*)qkv, planes, sums, (size_t)T * (nh + 2 * nkv) * hd};
-  // a block a token pays off with many tokens (13.6 against 18.6 us at 2048 tokens of 8 + 2 x 4
-  // heads of 256); a handful of decoded tokens is quicker spread over a block per (token, head)
-  if (T >= 64 && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF) {
-    rope_cache_write_token_kernel<<<T, 256, 0, (hipStream_t)stream>>>((act_t*)qkv, from, positions, slot_map, inv_freq,
-                                                                     (act_t*)kcache, (act_t*)vcache, nh, nkv,
-                                                                     hd, bs, v_transposed);
+  // a block a token pays off with many values, few are quicker spread over a block per (token, head).  us, by heads and by tokens:
+  // 8 and 2 x 4 of 256, 64 tokens 3.2 and 4.3 (as three planes of sums 3.9 and 6.5), 200 4.4 and 4.4, 303 5.2 and 4.9; 8 and 2 x 2 of 128, 303
+  // 3.5 and 4.3, 535 4.5 and 4.6; 32 and 2 x 16 of 128, 100 4.8 and 5.7, 200 7.2 and 5.4.
+  if ((long long)T * (nh + 2 * nkv) * hd > 1 << 20 && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF) {
+    const auto kernel = T >= 1500 ? rope_cache_write_token_kernel<true> : rope_cache_write_token_kernel<false>;
+    kernel<<<T, 256, 0, (hipStream_t)stream>>>((act_t*)qkv, from, positions, slot_map, inv_freq, (act_t*)kcache, (act_t*)vcache, nh, nkv,
+                                               hd, bs, v_transposed);
     return zk_launch_status("zk_rope_cache_write");
   }
   dim3 grid(T, nh + 2 * nkv);
