@@ -128,3 +128,47 @@ def test_attention_of_few_and_many_blocks_and_with_a_window_that_shows_all(nh, n
 def test_rotation_and_store_of_many_tokens(dtype, T, nh, nkv, hd, bs, vt):
     from test_gpu_kernels import test_rope_and_cache_write
     test_rope_and_cache_write(dev()[0], dtype, T, nh, nkv, hd, hd, bs, vt)
+
+
+# heads, key heads, key and value channels, page, (cached, new) of each request, window, kept, cap, rising: one row; a block that is not
+# full; 5, 8 and 1 tokens a block; 32 keys and one more, a tile for each wave and one more; windows that begin inside a tile, with kept
+# keys; values of another width; maxima that rise
+SHORT = [(8, 4, 256, 256, 16, [(0, 2)], 0, 0, 50.0, False), (6, 2, 128, 128, 16, [(0, 33), (31, 5), (100, 29)], 0, 0, 0.0, False),
+         (16, 1, 256, 256, 32, [(60, 69)], 0, 0, 30.0, False), (8, 4, 256, 256, 64, [(3, 126), (0, 128)], 0, 0, 50.0, False),
+         (8, 2, 128, 128, 16, [(300, 150)], 97, 0, 0.0, False), (8, 4, 256, 256, 16, [(200, 40)], 50, 37, 50.0, False),
+         (4, 2, 256, 128, 16, [(10, 31)], 0, 0, 0.0, False), (4, 2, 128, 256, 16, [(0, 129)], 0, 0, 0.0, False),
+         (8, 8, 128, 128, 16, [(0, 290)], 0, 0, 0.0, True)]
+
+
+@pytest.mark.parametrize("case", SHORT)
+def test_portions_of_few_rows(case):
+    from test_gpu_stream_attention import test_portions
+    from test_portion_forms import form_of
+    H, G, D, E, bs, reqs, window, keep, cap, rising = case
+    assert form_of(1 << 28, len(reqs), max(b for _, b in reqs), max(a + b for a, b in reqs), H, G, D, E, bs, window, 0, keep)[2] == 2
+    test_portions(dev()[0], case, 0)
+
+
+@pytest.mark.parametrize("H,G,D,window", [(8, 4, 256, 0), (8, 2, 128, 40)])
+def test_nothing_outside_a_portions_keys_is_used(H, G, D, window):
+    """Keys and values behind the last key of a page, and in pages behind the last or in front of the window, are not numbers."""
+    from test_gpu_stream_attention import plain, rounded, up
+    rt, k = dev()
+    rng = np.random.default_rng(D)
+    bs, before, n = 16, 70, 23
+    ctx, blocks = before + n, 9
+    kc, vc = np.full((blocks + 1, G, bs, D), np.nan, np.float32), np.full((blocks + 1, G, D, bs), np.nan, np.float32)
+    q, kk, vv = (rounded(rng.normal(size=(m, h, D))) for m, h in ((n, H), (ctx, G), (ctx, G)))
+    first = max(0, before - window + 1) if window else 0
+    for p in range(first, ctx):
+        kc[1 + p // bs, :, p % bs], vc[1 + p // bs, :, :, p % bs] = kk[p], vv[p]
+    table = (1 + np.arange(blocks, dtype=np.int32)).reshape(1, -1)          # entries behind the last page lead to pages too
+    out = rt.zeros((n, H * D), "bfloat16")
+    ws = rt.zeros((1 << 20,), "float32")
+    args = [up(rt, q.reshape(n, -1)), up(rt, kc), up(rt, vc), rt.upload(table, "int32"), rt.upload(np.array([0, n], np.int32), "int32"),
+            rt.upload(np.array([ctx], np.int32), "int32")]
+    k.zk_attention_bf16(args[0].ptr, H * D, args[1].ptr, args[2].ptr, args[3].ptr, blocks, args[4].ptr, args[5].ptr, out.ptr, 1, 1, n, ctx, H,
+                        G, D, bs, D ** -0.5, 0.0, window, 0, ws.ptr, ws.nbytes, rt.stream)
+    got = rt.download_f32(out).reshape(n, H, D)
+    want = plain(q.astype(np.float64), kk.astype(np.float64), vv.astype(np.float64), before, D ** -0.5, 0.0, window, 0)
+    assert np.abs(got - want).max() < 0.03

@@ -25,7 +25,8 @@
 // all of them (attn_shared_kernel: many groups); and the latter with the keys of a block of rows
 // cut into ranges over several blocks, joined by attn_portion_join_kernel (few groups with long
 // contexts: a portion of a prompt behind thousands of tokens).  Heads of 128 and 256 channels with
-// pages of 16 or more take attn_stream_kernel in place of the shared tiles, in ranges or not.
+// pages of 16 or more take attn_stream_kernel in place of the shared tiles, in ranges or not, and attn_short_kernel, 16 rows a
+// block, where rows and keys are few.
 //
 // Decoded tokens use a split variant: the keys are cut into chunks aligned to absolute positions,
 // each leaves (max, sum, O) and a second kernel joins the chunks in order; the cut never follows
@@ -277,7 +278,8 @@ static int portion_ranges(int max_q_len, int max_ctx, int window, int mask_chunk
 // most (us; group, four, ranges, taken): 8 heads over 4 of 256, 512 rows at 512
 // keys 25, 28, 23, ranges; behind 3,584 112, 143, 42, ranges; 4,096 rows 238, 135, 129, ranges; 16 over 8, 2,048 rows 149, 81, 84,
 // four; 32 over 16 of 128, 512 rows at 512 keys 16, 21, 25, group; 2,048 rows 168, 70, 82, four.
-struct PortionPlan { int kind, ranges, whole; };      // ranges: the best cut with ranges, taken or not (0: none); whole: the better kind without
+// ranges: the best cut with ranges, taken or not (0: none); whole: the better kind without; price: of the kind
+struct PortionPlan { int kind, ranges, whole; double price; };
 static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int tpw, int nkv, int r_prefill,
                                 int bound_tiles, int wide) {
   const bool narrow = wide <= 128;
@@ -304,11 +306,11 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
     if (blocks <= slots) return alone;
     return std::max(alone, (blocks * start + per_tile * tiles) / slots + 0.5 * (start + per_tile * least));
   };
-  PortionPlan best{0, 0, 0};
+  PortionPlan best{0, 0, 0, 0};
   const double groups = (max_q_len + tpw - 1) / tpw;
   double best_price = price(slots, groups * copies, start_group, tile_group, sum * copies * groups / row_blocks, longest, shortest);
   const double four = edges + price(slots, (double)row_blocks * copies, start_four, tile_four, sum * copies, longest, shortest);
-  if (four < best_price) best = {4, 0, 4}, best_price = four;
+  if (four < best_price) best = {4, 0, 4, 0}, best_price = four;
   double best_ranges = 1e30;
   static const int cands[] = {64, 48, 40, 32, 24, 16, 12, 10, 8, 6, 4};
   for (int ct : cands) {
@@ -327,8 +329,26 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
     t += all * wide * (0.035 / 256) + ((double)row_blocks * copies * most_ranges - all) * 0.005 + 4.0;
     if (t < best_ranges) best.ranges = ct, best_ranges = t;
   }
-  if (best_ranges < best_price) best.kind = 5;
+  best.price = best_price;
+  if (best_ranges < best_price) best.kind = 5, best.price = best_ranges;
   return best;
+}
+
+// attn_short_kernel's price in microseconds: a start and a time for every tile that the longest block's waves take one after the other;
+// blocks beyond one a CU share its way to the L2.  Over 76 launches (7 to 1,024 rows, 8 to 32 heads, up to 2,000 keys in front, one to
+// five requests) it is 0.86 to 1.3 times what was measured up to one block a CU, and 0.93 to 1.9 times beyond, where what is close stays
+// with the others: 700 rows of 8 heads over 4 of 256, 352 blocks, 28.0 as they are and 30.9; 1,024 of 32 over 16 of 128 35.9 and 61.8.
+static double short_price(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int g, int nkv, int r_prefill, int wide) {
+  const int tokens = 16 / g, last = max_ctx - max_q_len + (max_q_len - 1) / tokens * tokens;      // the last block's first token
+  const int lo = mask_chunk > 0 ? last - last % mask_chunk : window > 0 ? std::max(0, last - window + 1) : 0;
+  const int tiles = std::min((keep + 31) / 32, lo / 32) + (max_ctx - 1) / 32 - lo / 32 + 1;
+  // (256 channels and more than four tiles a wave: the prices of both kinds are off by as much as they differ, 16 rows behind 500 keys
+  // 16.9 as they are and 17.6, 128 rows 20.8 and 19.1)
+  if (wide > 128 && tiles > 16) return 1e30;
+  const double blocks = (double)((max_q_len + tokens - 1) / tokens) * nkv * r_prefill;
+  const double alone = wide > 128 ? 3.6 + 2.8 * ((tiles + 3) / 4) : 3.2 + 1.8 * ((tiles + 3) / 4);
+  if (blocks <= 256) return alone;
+  return alone * (wide > 128 ? 1.3 * blocks / 256 : 1 + 0.45 * (blocks - 256) / 256);
 }
 
 // 0: the portion kernel is chosen by the sizes; 1: a group of rows a block; 4, 8: shared
@@ -378,6 +398,10 @@ static PortionForm portion_form(int r_prefill, int max_q_len, int max_ctx, bool 
     if (reach > 0) bound = std::min(bound, (reach + per_block + 31) / 32 + 1 + (keep + 31) / 32);
     if (stream) {
       const PortionPlan plan = portion_plan(max_q_len, max_ctx, window, mask_chunk, keep, tpw, nkv, r_prefill, bound, wide);
+      // few rows and keys: 16 rows a block, where that beats the best of the others, with room for it or not
+      if (portion_kernel_mode == 0 && nh / nkv <= 16 &&
+          short_price(max_q_len, max_ctx, window, mask_chunk, keep, nh / nkv, nkv, r_prefill, wide) < 0.92 * plan.price)
+        return {ATT_SHORT, 0, 0};
       range_tiles = portion_kernel_mode == 5 || plan.kind == 5 ? plan.ranges : 0;
       // Many groups priced by a context that may be another's: no ranges (8 times 128 fresh rows beside 3,840 keys, 32 heads over 16
       // of 128: 26 us, 13 without; 3,584 rows beside 8,192, 16 over 4: 176 and 91).  Few groups do gain from them where the context is theirs.
@@ -405,13 +429,13 @@ int zk_attention_bf16_portion_kernel(int mode) {
 }
 
 // Which form a launch of ``r_prefill`` portions takes with ``room`` bytes of workspace behind the decoded tokens' part: 1, 2, 4 or 8
-// groups of rows a block, or 5, four with the keys in ranges of *range_tiles tiles.  *stream: by attn_stream_kernel.  For tests that mean
-// to reach each of them.
+// groups of rows a block, or 5, four with the keys in ranges of *range_tiles tiles.  *stream: 1 by attn_stream_kernel, 2 by
+// attn_short_kernel (whose groups have 16 rows).  For tests that mean to reach each of them.
 int zk_attention_bf16_portion_form(int r_prefill, int max_q_len, int max_ctx, int not_theirs, int nh, int nkv, int hd, int vd, int bs,
                                    int window, int mask_chunk, int keep, int wide_weights, size_t room, int* range_tiles, int* stream) {
   const PortionForm f = portion_form(r_prefill, max_q_len, max_ctx, not_theirs, nh, nkv, hd, vd, bs, window, mask_chunk, keep, wide_weights, room);
   *range_tiles = f.range_tiles;
-  *stream = (f.what == ATT_SHARED4 || f.what == ATT_RANGES) && stream_takes(hd, vd, bs, wide_weights);
+  *stream = f.what == ATT_SHORT ? 2 : (f.what == ATT_SHARED4 || f.what == ATT_RANGES) && stream_takes(hd, vd, bs, wide_weights);
   return f.what == ATT_RANGES ? 5 : f.what == ATT_SHARED8 ? 8 : f.what == ATT_SHARED4 ? 4 : f.what == ATT_PAIRS ? 2 : 1;
 }
 
@@ -546,7 +570,10 @@ int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, cons
     const PortionForm form = portion_form(r_prefill, max_q_len, portion_ctx ? portion_ctx : max_ctx, !portion_ctx && R > r_prefill, nh, nkv,
                                           hd, vd, bs, window, mask_chunk, keep, wide_weights, usable ? workspace_bytes - split_at : 0);
     int rc;
-    if (form.what == ATT_RANGES) {
+    if (form.what == ATT_SHORT) {
+      const int tokens = 16 / g;
+      rc = launch_attn(ATT_SHORT, p, dim3((max_q_len + tokens - 1) / tokens, nkv, r_prefill), s);
+    } else if (form.what == ATT_RANGES) {
       const int per_block = 4 * p.tpw, most_ranges = form.most_ranges;
       AttnParams ps = p;
       ps.chunk = form.range_tiles;

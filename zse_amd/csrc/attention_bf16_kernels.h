@@ -19,6 +19,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define ATT_CHUNK 64
 #define ATT_DECODE_SPAN 128    // keys of a partial result of a decoded token on 16-wide tiles
 #define ATT_DECODE_LONG_FROM 4096      // 256 instead where a request's table holds this many keys or more
+#define ATT_SHORT_WAVES 4      // waves of a block of a portion of few rows
 #define ATT_MOST_RANGES 8      // ranges of keys a block of rows of a portion is cut into, at most
 
 struct AttnParams {
@@ -1334,6 +1335,153 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
   }
 }
 
+// Portions of few rows: 16 rows a block (16 / g tokens of one request times the g query heads of a KV head) on
+// 16x16x32 MFMAs, the block's waves take tiles of 32 keys in turn, each with a maximum, a sum and
+// results of its own, and are joined in LDS.  Rows are columns of every tile, as in the decode kernel, and
+// keys lie in it as there.
+//
+// What a launch of few rows waits for is one wave's chain: pages, keys, scores, weights, values, the join.  The kernel of 32 rows a
+// group walks 5,000 instructions of 32-wide tiles through it and twice the accumulators through
+// the join; half the rows a block also double the blocks.  us, that kernel, or tiles shared and joined where these are
+// faster, and this: 8 heads over 4 of 256, 7 rows 7.5 and 5.1, 37 11.5 and 5.4, 150 16.2 and 9.3, 512 23.2 and 16.6; 32 over 16 of 128, 37 8.7
+// and 4.5, 300 15.5 and 12.4; 16 over 4 of 128, 128 behind 500 keys 17.5 and 12.4.  At 512 rows eight waves a block: 16.1, 30.4 (32 over 16, four
+// 23.2), 15.4 (16 over 4, 13.7).
+template <int HD32, int VD16, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void attn_short_kernel(AttnParams p) {
+  constexpr int KS = HD32, DT = VD16, hd = HD32 * 32, vd = VD16 * 16, LD = vd + 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = lane & 15, kq = lane >> 4;
+  const int r = p.r_begin + blockIdx.z, kvh = blockIdx.y;
+  const int* table = p.block_table + (size_t)r * p.max_blocks;
+  const int qs = p.q_start[r], n = p.q_start[r + 1] - qs, ctx = p.ctx_len[r];
+  const int g = p.nh / p.nkv, tokens = 16 / g;
+  const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * tokens;      // the rows with the most keys first
+  if (t0 >= n) return;
+  const int start = ctx - n, ntok = min(tokens, n - t0);
+  const int tok = col / g, hq = col - tok * g;
+  const bool col_ok = tok < ntok;
+  const int pos = start + t0 + min(tok, ntok - 1), row_lo = first_key(p, pos);
+  const int head = q_head_of(p, kvh, hq), trow = qs + t0 + min(tok, ntok - 1);
+  const int key_lo = first_key(p, start + t0), key_hi = start + t0 + ntok - 1;
+  const KeyTiles tiles(p, key_lo, key_hi);
+  const int bsh = p.bs_shift, bmask = p.bs - 1, nkv = p.nkv, vheads = nkv >> p.v_shift, vh = kvh >> p.v_shift;
+
+  bf16x8 qf[KS];
+  const __bf16* qr = p.q + (size_t)trow * p.q_stride + (size_t)head * hd + kq * 8;
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) qf[ks] = *(const bf16x8*)(qr + ks * 32);
+  f32x4 o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  for (int i = wave; i < tiles.count; i += NW) {
+    const int key0 = tiles.key_of(i);
+    // (a key behind the block's last: that one's page, which is the request's own.  Asked for a tile ahead, the pages made a wave's
+    // registers too many: 512 rows, 8 heads over 4 of 256, 16.7 -> 17.4 us.)
+    int kpage[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) kpage[t] = table[min(key0 + 8 * (col >> 2) + 4 * t + (col & 3), key_hi) >> bsh];
+    const int vpage = table[min(key0 + 8 * kq, key_hi) >> bsh];
+    bf16x8 kf[2][KS], vf[DT];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      const int kk = key0 + 8 * (col >> 2) + 4 * t + (col & 3);
+      const __bf16* kr = p.kcache + ((((size_t)max(kpage[t], 0) * nkv + kvh) << bsh) + (kk & bmask)) * hd + kq * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) kf[t][ks] = *(const bf16x8*)(kr + ks * 32);
+    }
+    const __bf16* va = p.vcache + ((((size_t)max(vpage, 0) * vheads + vh) * vd) << bsh) + ((key0 + 8 * kq) & bmask);
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) vf[dt] = *(const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh));
+    f32x4 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ks++) s[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[t][ks], qf[ks], s[t], 0, 0, 0);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int key = key0 + 8 * kq + 4 * t + e;
+        const float v = score_log2(p, s[t][e]);
+        s[t][e] = (key >= row_lo || key < p.keep) && key <= pos ? v : -INFINITY;
+        top = fmaxf(top, s[t][e]);
+      }
+    top = fmaxf(m_run, wave_max16_32(top));
+    const float m_use = top == -INFINITY ? 0.f : top, corr = __builtin_amdgcn_exp2f(m_run - m_use);
+    m_run = top;
+    float sum = 0.f;
+    bf16x8 pb;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float w = __builtin_amdgcn_exp2f(s[t][e] - m_use);
+        sum += w;
+        pb[4 * t + e] = (__bf16)w;
+      }
+    l_run = l_run * corr + wave_add16_32(sum);
+    if (key0 + 31 > key_hi || key0 < key_lo) {
+      // values outside the block's keys may be anything, and a weight of 0 does not make them nothing
+      typedef unsigned u4 __attribute__((ext_vector_type(4)));
+      u4 keep;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const int key = key0 + 8 * kq + 2 * e;
+        auto in = [&](int k) { return k <= key_hi && (k >= key_lo || k < p.keep); };
+        keep[e] = (in(key) ? 0xffffu : 0u) | (in(key + 1) ? 0xffff0000u : 0u);
+      }
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) vf[dt] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u4, vf[dt]) & keep);
+    }
+    if (i != wave) {
+#pragma unroll
+      for (int dt = 0; dt < DT; dt++) o[dt] *= corr;
+    }
+#pragma unroll
+    for (int dt = 0; dt < DT; dt++) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb, o[dt], 0, 0, 0);
+  }
+  // the waves' results: rows of LD floats, then maxima and sums
+  extern __shared__ __align__(16) float short_lds[];
+  float* ml = short_lds + (size_t)NW * 16 * LD;
+  float* so = short_lds + ((size_t)wave * 16 + col) * LD + 4 * kq;
+#pragma unroll
+  for (int dt = 0; dt < DT; dt++) *(f32x4*)(so + dt * 16) = o[dt];
+  if (kq == 0) {
+    ml[(wave * 16 + col) * 2] = m_run;
+    ml[(wave * 16 + col) * 2 + 1] = l_run;
+  }
+  __syncthreads();
+  // every thread joins four channels of a row at a time
+  constexpr int PER_ROW = vd / 4;
+  for (int idx = threadIdx.x; idx < 16 * PER_ROW; idx += NW * 64) {
+    const int c = idx / PER_ROW, d = idx % PER_ROW * 4, ct = c / g;
+    if (ct >= ntok) break;
+    float mw[NW], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      mw[w] = ml[(w * 16 + c) * 2];
+      m = fmaxf(m, mw[w]);
+    }
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const float e = mw[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw[w] - m);
+      acc += e * *(const f32x4*)(short_lds + ((size_t)w * 16 + c) * LD + d);
+      l += e * ml[(w * 16 + c) * 2 + 1];
+    }
+    const int row = qs + t0 + ct, h = q_head_of(p, kvh, c - ct * g);
+    const float inv = row_factor(p, row, h, l, m);
+    bf16x4 x;
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[e] = (__bf16)(acc[e] * inv);
+    *(bf16x4*)(p.out + ((size_t)row * p.nh + h) * vd + d) = x;
+  }
+}
+
 // One wave per (request, KV head, chunk of 64 keys) for requests that bring one token.
 // Columns of every tile are the g query heads of the KV head (col = lane % 16), rows are
 // keys (first product) or channels (second product).
@@ -1538,7 +1686,7 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
 // One pair of sizes.  what: 0 decoded tokens on 32-wide tiles, 1 pairs of groups a block, 2 a group a block,
 // 3 shared tiles with four waves, 4 with eight, 5 with four and the keys in ranges, 6 decoded tokens
 // on 16-wide tiles (keys in whole 32s), 7 the same in blocks of 256 keys.
-enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE, ATT_DECODE_LONG };
+enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE, ATT_DECODE_LONG, ATT_SHORT };
 
 template <int HD16, int VD16, int NW, bool SPLIT>
 static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
@@ -1596,6 +1744,21 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
       if constexpr (HD16 >= 8 && VD16 >= 8)
         if (stream_takes(p.hd, p.vd, p.bs, p.wide_weights)) return launch_stream<HD16, VD16, true>(p, grid, s);
       return launch_shared_one<HD16, VD16, 4, true>(p, grid, s);
+    case ATT_SHORT:
+      if constexpr (HD16 % 2 == 0) {
+        constexpr size_t lds = ((size_t)ATT_SHORT_WAVES * 16 * (VD16 * 16 + 4) + ATT_SHORT_WAVES * 32) * sizeof(float);
+        static std::atomic<bool> prepared{false};
+        if (lds > 64 * 1024 && !prepared) {
+          if (hipFuncSetAttribute((const void*)attn_short_kernel<HD16 / 2, VD16, ATT_SHORT_WAVES>,
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return zk_fail("zk_attention_bf16: the LDS of the kernel of few rows was refused");
+          prepared = true;
+        }
+        attn_short_kernel<HD16 / 2, VD16, ATT_SHORT_WAVES><<<grid, ATT_SHORT_WAVES * 64, lds, s>>>(p);
+        break;
+      } else {
+        return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
+      }
     case ATT_DECODE:
       if constexpr (HD16 % 2 == 0) {
         const size_t lds = (size_t)4 * (p.nh / p.nkv) * p.vd * sizeof(float) + (size_t)4 * (HD16 / 2) * 64 * sizeof(bf16x8);
