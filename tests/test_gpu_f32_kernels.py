@@ -121,6 +121,14 @@ def test_attention(rt, nh, nkv, hd, vd, bs, window, keep):
     assert np.array_equal(alone[9:], got[9:]) and np.array_equal(alone[:8], got[:8])
 
 
+# Key heads of 65 to 128 channels, whose keys and values are asked for a piece of 16 ahead: ragged and full sizes of both,
+# pieces at both ends of a tile that no row sees, pages of fewer keys than a piece
+@pytest.mark.parametrize("nh,nkv,hd,vd,bs,window,keep", [(4, 2, 68, 4, 16, 0, 0), (8, 2, 128, 128, 16, 0, 0), (8, 8, 100, 64, 4, 20, 0),
+                                                         (2, 1, 128, 4, 16, 33, 17), (5, 1, 96, 100, 8, 0, 0)])
+def test_attention_a_piece_ahead(rt, nh, nkv, hd, vd, bs, window, keep):
+    test_attention(rt, nh, nkv, hd, vd, bs, window, keep)
+
+
 # One request whose tokens share a block.  A value that is not finite lies in a piece of 16 keys of which
 # every row sees several more: at the last token's own place (hidden from the tokens before it), or at a place
 # that a window shows to the first tokens only.

@@ -161,8 +161,8 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 //
 // Bound by the latency of the loads for few tokens and by the matrix cores for many.  Measured
 // (us; before: a wave per token and head whose lanes each walked a key's row):
-//   303 tokens, 8 heads of 128, contexts of 300 and three of 50 to 700: 852 -> 55.
-//   One token, 8 heads over 2 of 128: 1 key 12.4 -> 9.5, 100 keys 57 -> 16, 4,000 keys 2,111 -> 144; 4 heads
+//   303 tokens, 8 heads of 128, contexts of 300 and three of 50 to 700: 852 -> 38.
+//   One token, 8 heads over 2 of 128: 1 key 12.4 -> 10.2, 100 keys 57 -> 15, 4,000 keys 2,111 -> 132; 4 heads
 //   of 16: 6.9 -> 8.5, 26 -> 11, 884 -> 83; 8 over 4 of 256: 21.7 -> 22.7, 109 -> 27, 6,260 -> 458.  (Heads of up
 //   to 64 are slower than before below about ten keys, of 256 below three.)
 //
@@ -171,10 +171,14 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // 3 tokens (us; key by key, a run a block, packed): 8 heads of 128 over 2 68, 174, 92; 8 of 64 41, 480, 67; 8 over 4
 // of 256 136, 484, 172.  1,500 tokens behind a window of 64, 8 of 64: 99, 159, 50.
 //
-// ASK: keys are asked for without a condition, and pieces of 16 that no row sees are passed over in the
-// first product too.  For key heads of 65 to 128 channels: one token with 1 key 14.5 -> 9.5 us, 16 tokens of 500
-// to 1,055 keys 53 -> 47, 1,500 tokens behind a window 102 -> 91.  Not for 64 channels with values of 128 (4,000
-// keys 125 -> 138) nor for smaller heads (80 -> 89); of 256 the loads in flight do not fit (446 -> 472).
+// ASK: keys and values are asked for without a condition and a piece of 16 ahead of their products (the first values in
+// front of the weights), and pieces that no row sees are passed over in the first product too.  For key heads of 65 to
+// 128 channels, 8 heads over 2 of 128 (us; keys alone without a condition, and each piece at its turn; both ahead): 303 tokens,
+// 300 of them a prompt, 35.8 and 33.5; one token with 4,000 keys 141 and 132; 64 requests of 100 to 3,250 keys 142 and
+// 110; 1,000 requests of 3 tokens 493 and 381; 1,500 tokens 140 and 131, behind a window of 64 62 and 54; one token with
+// 1 key 9.9 and 10.2, 8 of 500 24.1 and 24.5 (the waits for pieces that are passed over, a few more instructions).  Not
+// for smaller key heads (8 over 4 of 64, 4,000 keys: 92 and 94; with values of 128 34 and 65: the registers
+// do not hold both); of 256 the loads in flight do not fit (446 -> 472).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // The value of another lane of the row of 16: 0x110 + n: of the lane n before (none: what is there for it), 0x120 + n: in a circle
@@ -287,26 +291,47 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
         }
       }
       auto unseen = [&](int f) { return j0 + 16 * f > seg_hi || (j0 + 16 * f + 15 < seg_lo && j0 + 16 * f >= keep); };
-      f32x4 s[4];
+      // ASK: a piece's keys and values are asked for a piece ahead, the first values in front of the weights.  They are
+      // held in front of the branches that pass over unseen pieces, behind which the compiler would move their loads.
+      f32x4 s[4], k_ahead[2][QC], v_ahead[2][4][VC];
+      bool has[2][4];              // the key of a value asked for is in the cache
+      auto ask_keys = [&](int f) {
+#pragma unroll
+        for (int c = 0; c < QC; c++)
+          k_ahead[f & 1][c] = *(const f32x4*)(kcache + (size_t)max(at[f], 0LL) * hd + min(16 * c + 4 * qd, hd - 4));
+      };
+      auto ask_values = [&](int f) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const long long va = __shfl(at[f], 4 * qd + e);
+          has[f & 1][e] = va >= 0;
+#pragma unroll
+          for (int c = 0; c < VC; c++)
+            v_ahead[f & 1][e][c] = *(const f32x4*)(vcache + (size_t)max(va, 0LL) * vd + min(64 * c + 4 * r, vd - 4));
+        }
+      };
+      if (ASK) ask_keys(0);
 #pragma unroll
       for (int f = 0; f < 4; f++) {
         s[f] = zero;
-        if (ASK && unseen(f)) continue;
+        if (ASK) {
+          if (f < 3) ask_keys(f + 1);
+#pragma unroll
+          for (int c = 0; c < QC; c++) asm volatile("" : "+v"(k_ahead[f & 1][c]));
+          if (unseen(f)) continue;
+        }
         const float* kr = kcache + (size_t)max(at[f], 0LL) * hd;
 #pragma unroll
         for (int c = 0; c < QC; c++) {
           const int d = 16 * c + 4 * qd;
           f32x4 k4;
-          if (ASK) {
-            k4 = *(const f32x4*)(kr + min(d, hd - 4));
-            k4 = at[f] >= 0 && d < hd ? k4 : zero;
-          } else {
-            k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
-          }
+          if (ASK) k4 = at[f] >= 0 && d < hd ? k_ahead[f & 1][c] : zero;
+          else k4 = at[f] >= 0 && d < hd ? *(const f32x4*)(kr + d) : zero;
 #pragma unroll
           for (int e = 0; e < 4; e++) s[f] = __builtin_amdgcn_mfma_f32_16x16x4f32(k4[e], qf[c][e], s[f], 0, 0, 0);
         }
       }
+      if (ASK) ask_values(0);
       float top = -INFINITY;
       bool all = true;             // the lane's query sees all of the lane's keys
 #pragma unroll
@@ -345,17 +370,25 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
       const bool whole = __all(all);
 #pragma unroll
       for (int f = 0; f < 4; f++) {
+        if (ASK) {
+          if (f < 3) ask_values(f + 1);
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+#pragma unroll
+            for (int c = 0; c < VC; c++) asm volatile("" : "+v"(v_ahead[f & 1][e][c]));
+        }
         if (PASS_VALUES && unseen(f)) continue;
         f32x4 v[4][VC];            // [key 16 f + 4 qd + e][c]: channels 64 c + 4 r ..
         long long va[4];
         bool fine = true;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          va[e] = __shfl(at[f], 4 * qd + e);
+          if (!ASK) va[e] = __shfl(at[f], 4 * qd + e);
 #pragma unroll
           for (int c = 0; c < VC; c++) {
             const int d = 64 * c + 4 * r;
-            v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
+            if (ASK) v[e][c] = has[f & 1][e] && d < vd ? v_ahead[f & 1][e][c] : zero;
+            else v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
           }
         }
         if (!whole) {
