@@ -176,7 +176,7 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // 128 channels, 8 heads over 2 of 128 (us; keys alone without a condition, and each piece at its turn; both ahead): 303 tokens,
 // 300 of them a prompt, 35.8 and 33.5; one token with 4,000 keys 141 and 132; 64 requests of 100 to 3,250 keys 142 and
 // 110; 1,000 requests of 3 tokens 493 and 381; 1,500 tokens 140 and 131, behind a window of 64 62 and 54; one token with
-// 1 key 9.9 and 10.2, 8 of 500 24.1 and 24.5 (the waits for pieces that are passed over, a few more instructions).  Not
+// 1 key 9.9 and 10.2, 8 of 500 24.1 and 24.5, 1,000 requests of 3 tokens with 3 keys 95 and 98 (the waits for pieces that are passed over, a few more instructions).  Not
 // for smaller key heads (8 over 4 of 64, 4,000 keys: 92 and 94; with values of 128 34 and 65: the registers
 // do not hold both); of 256 the loads in flight do not fit (446 -> 472).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
