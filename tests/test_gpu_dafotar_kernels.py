@@ -315,18 +315,23 @@ def test_streams_of_whole_pieces(dev, S, W, parts):
 MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17]       # rows of 72 requests
 
 
-def test_short_convolution_of_many_requests(dev):
+# Alike rows (a block a run and request), and one long portion among single rows (runs numbered through all requests, full
+# and one of a single row); channels in eights and one at a time
+@pytest.mark.parametrize("lens,by_piece", [(MANY, 0), ([0, 1, 393] + [1, 0, 2] * 24, 1)])
+@pytest.mark.parametrize("C,taps", [(16, 4), (264, 3), (13, 4)])
+def test_short_convolution_of_many_requests(dev, lens, by_piece, C, taps):
     """More requests than a wave adds up at once, of no, one and several runs of rows; padding behind the last."""
     rt, k = dev
     rng = np.random.default_rng(3)
-    C, taps, R, T = 16, 4, len(MANY), sum(MANY)
+    R, T = len(lens), sum(lens)
+    assert k._dll.zk_conv_rows_by_piece(T + 3, R, max(lens), C, 1 if C % 8 else 8) == by_piece
     w = rng.normal(0, 0.7, (C, taps)).astype(np.float32)
     x = rng.normal(size=(T + 3, C)).astype(np.float32)
     state = rt.zeros((R, (taps - 1) * C), "float32")
     out = up(rt, np.full((T + 3, C), 7.0, np.float32))
-    q_start = np.concatenate([[0], np.cumsum(MANY)])
+    q_start = np.concatenate([[0], np.cumsum(lens)])
     k.zk_conv_rows(up(rt, x).ptr, C, None, up(rt, w).ptr, None, state.ptr, (taps - 1) * C, 0, i32(rt, q_start).ptr,
-                   i32(rt, range(R)).ptr, out.ptr, C, T + 3, R, max(MANY), C, taps, 1, 0, rt.stream)
+                   i32(rt, range(R)).ptr, out.ptr, C, T + 3, R, max(lens), C, taps, 1, 0, rt.stream)
     got, st = rt.download(out), rt.download(state).reshape(R, taps - 1, C)
     for r in range(R):
         rows = x[q_start[r]:q_start[r + 1]].astype(np.float64)

@@ -12,9 +12,11 @@
 // them reads the state (span >= taps - 1), and its threads renew it, each its own columns, after
 // they have read them.  One launch serves every kind of step.
 //
-// Few bytes (5.8 MB at 708 rows of 2,048): the time is the launch and one trip to memory, so a run's rows are
-// all asked for before the first is used, and blocks are narrow until the chip is full.  (Row after row in
-// blocks of 256 threads, a grid of the longest portion's runs for every request: 9.1 us; so 7.4.)
+// A block works on one run.  As a rule block (y, z) is run y of request z; where more than half of many such blocks would
+// find no run, the runs are numbered through all requests and a block looks for its own (us, the one way and the other: 700
+// rows and 8 single ones of 2,048 channels 10.2 and 9.0, 2,000 and 500 single ones of 256 55.8 and 10.0; 2,048 rows of 2,048
+// 10.2 and 10.5, 1,000 requests of nine rows of 256 16.7 and 21.4).  A run's rows are read one after the other: all asked for
+// in front, also where a run is short, 2,048 rows of 2,048 take 12.9 and 8 single ones 3.6 in place of 3.4.
 #include "common.h"
 #include "packed_call.h"
 
@@ -25,23 +27,21 @@ extern "C" int zk_steplist_register(const char* name, int nargs, void* fn);
 #define CONV_SPAN 8
 #define CONV_MOST_TAPS (CONV_SPAN + 1)
 
-// V channels of a row as they lie in memory, and their values
-template <int V>
-struct ConvRaw {
-  act_t v[V] __attribute__((aligned(sizeof(act_t) * V > 16 ? 16 : sizeof(act_t) * V)));
-};
-template <int V>
-__device__ __forceinline__ ConvRaw<V> conv_raw(const act_t* p) {
-  return *(const ConvRaw<V>*)p;
-}
-template <int V>
-__device__ __forceinline__ void conv_values(const ConvRaw<V>& r, float (&v)[V]) {
-#pragma unroll
-  for (int e = 0; e < V; e++) v[e] = to_f32(r.v[e]);
-}
 template <int V>
 __device__ __forceinline__ void conv_get(const act_t* p, float (&v)[V]) {
-  conv_values<V>(conv_raw<V>(p), v);
+  if constexpr (V == 8) {
+#if ZSE_ACT_BF16
+    typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+    const b8 q = *(const b8*)p;
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = (float)q[e];
+#else
+    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+#endif
+  } else {
+    v[0] = to_f32(p[0]);
+  }
 }
 template <int V>
 __device__ __forceinline__ void conv_put(act_t* p, const float (&v)[V]) {
@@ -79,41 +79,47 @@ __device__ __forceinline__ void conv_put_state(float* p, const float (&v)[V]) {
   }
 }
 
-// TAPS: the number of taps where the launch knows it at compile time, 0: ``taps`` (up to 9)
-template <int V, int TAPS>
+// TAPS: the number of taps where the launch knows it at compile time, 0: ``taps`` (up to 9).  PIECES: runs are numbered through all
+// requests, ``columns`` blocks next to each other for each
+template <int V, int TAPS, bool PIECES>
 __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict__ x, int ld_in,
                                                         const float* __restrict__ in_bias, const float* __restrict__ w,
                                                         const float* __restrict__ bias, float* __restrict__ state,
                                                         int slot_words, int offset_words, const int* __restrict__ q_start,
                                                         const int* __restrict__ slot_of_req, act_t* __restrict__ out,
                                                         int ld_out, int T, int R, int C, int taps_given, int residual,
-                                                        int act, int one_run) {
+                                                        int act, int columns) {
   constexpr int MOST = TAPS ? TAPS : CONV_MOST_TAPS, BACK = MOST > 1 ? MOST - 1 : 1;
   const int taps = TAPS ? TAPS : taps_given;
-  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * V;
-  Piece run;
-  bool found;
-  if (one_run) {                         // no request has more than one run: block x is request x's
-    run.r = blockIdx.x;
-    found = run.r < R;
-    run.t0 = q_start[run.r];
-    run.n = found ? q_start[run.r + 1] - run.t0 : 0;
-    run.first = 0;
-    if (found && run.n <= 0) return;
-  } else {
-    found = find_piece(q_start, R, CONV_SPAN, blockIdx.x, run);      // (all lanes of a wave call it)
-  }
-  if (c >= C) return;
-  if (!found) {                          // the grid's last: padding of a captured step, behind the last request
-    if (blockIdx.x == gridDim.x - 1) {
-      float zero[V];
+  const int c = ((PIECES ? blockIdx.x % columns : blockIdx.x) * blockDim.x + threadIdx.x) * V;
+  auto padding = [&](int from) {         // rows behind the last request: padding of a captured step
+    float zero[V];
 #pragma unroll
-      for (int e = 0; e < V; e++) zero[e] = 0.f;
-      for (int t = q_start[R]; t < T; t++) conv_put<V>(out + (size_t)t * ld_out + c, zero);
+    for (int e = 0; e < V; e++) zero[e] = 0.f;
+    for (int t = from; t < T; t++) conv_put<V>(out + (size_t)t * ld_out + c, zero);
+  };
+  int r, t0, n, first;
+  if constexpr (PIECES) {
+    Piece run;
+    const bool found = find_piece(q_start, R, CONV_SPAN, blockIdx.x / columns, run);      // (all lanes of a wave call it)
+    if (c >= C) return;
+    if (!found) {
+      if (blockIdx.x + columns >= gridDim.x) padding(q_start[R]);
+      return;
     }
-    return;
+    r = run.r, t0 = run.t0, n = run.n, first = run.first;
+  } else {
+    if (c >= C) return;
+    r = blockIdx.z, first = blockIdx.y * CONV_SPAN;
+    t0 = q_start[r];
+    if (r == R) {
+      if (first == 0) padding(t0);
+      return;
+    }
+    n = q_start[r + 1] - t0;
+    if (first >= n) return;
   }
-  const int t0 = run.t0, n = run.n, first = run.first, last = min(n, first + CONV_SPAN);
+  const int last = min(n, first + CONV_SPAN);
   float ib[V], b0[V], wt[MOST][V];
 #pragma unroll
   for (int e = 0; e < V; e++) {
@@ -127,11 +133,7 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
 #pragma unroll
     for (int e = 0; e < V; e++) v[e] += ib[e];
   };
-  // the run's rows as they lie in memory (a row past the last: the last again)
-  ConvRaw<V> rows[CONV_SPAN];
-#pragma unroll
-  for (int i = 0; i < CONV_SPAN; i++) rows[i] = conv_raw<V>(x + (size_t)(t0 + min(first + i, last - 1)) * ld_in + c);
-  float* st = taps > 1 ? state + (size_t)slot_of_req[run.r] * slot_words + offset_words + c : nullptr;
+  float* st = taps > 1 ? state + (size_t)slot_of_req[r] * slot_words + offset_words + c : nullptr;
   // back[b]: the row b + 1 places before the current token
   float back[BACK][V];
 #pragma unroll
@@ -162,16 +164,11 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
         conv_put_state<V>(st + (size_t)a * C, v);
       }
   }
-#pragma unroll
-  for (int i = 0; i < CONV_SPAN; i++) {
-    if (first + i >= last) break;
+  for (int i = first; i < last; i++) {
     float cur[V], acc[V];
-    conv_values<V>(rows[i], cur);
+    input(i, cur);
 #pragma unroll
-    for (int e = 0; e < V; e++) {
-      cur[e] += ib[e];
-      acc[e] = b0[e];
-    }
+    for (int e = 0; e < V; e++) acc[e] = b0[e];
 #pragma unroll
     for (int b = BACK - 1; b >= 0; b--)
       if (b < taps - 1) {
@@ -196,7 +193,7 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
       if (residual) acc[e] = cur[e] + acc[e];
       if (act == 1) acc[e] = acc[e] / (1.0f + expf(-acc[e]));      // silu
     }
-    conv_put<V>(out + (size_t)(t0 + first + i) * ld_out + c, acc);
+    conv_put<V>(out + (size_t)(t0 + i) * ld_out + c, acc);
 #pragma unroll
     for (int b = BACK - 1; b > 0; b--)
 #pragma unroll
@@ -206,7 +203,36 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
   }
 }
 
+// How a step's runs are laid out: ``columns`` blocks of ``threads`` for each of ``runs`` runs, of every request or of them all.
+struct ConvGrid {
+  int threads, columns, runs, by_piece;
+};
+static ConvGrid conv_grid(int T, int R, int max_q_len, int holders) {      // holders: threads that hold a row between them
+  // few runs: narrow blocks, so that they spread over the compute units
+  auto threads_of = [&](long long runs) { return (holders + 255) / 256 * runs >= 512 ? 256 : 64; };
+  const int most = max_q_len > 0 ? (max_q_len + CONV_SPAN - 1) / CONV_SPAN : 1;
+  ConvGrid g{threads_of((long long)most * R), 0, most, 0};
+  g.columns = (holders + g.threads - 1) / g.threads;
+  // The step's runs, at most (full ones and every request's last), and one for the padding behind the last request.  Finding
+  // a run costs 0.2 us, and 0.2 more for every 64 requests: few blocks, or blocks that mostly have a run, do not bring that
+  // back.  Over 397 uneven steps this choice takes 0.95 of the time of a block a run and request throughout.
+  const long long runs = (long long)T / CONV_SPAN + R + 1, blocks = (long long)most * (R + 1);
+  if (most > 1 && g.columns * blocks >= 700 && 2 * runs < blocks && g.columns * runs < 1 << 22) {
+    g.threads = threads_of(runs);
+    g.columns = (holders + g.threads - 1) / g.threads;
+    g.runs = (int)runs;
+    g.by_piece = 1;
+  }
+  return g;
+}
+
 extern "C" {
+
+// 1 if a step's runs are numbered through all its requests (``per``: channels a thread holds, 8 or 1).  For tests that mean
+// to reach both ways.
+int zk_conv_rows_by_piece(int T, int R, int max_q_len, int C, int per) {
+  return conv_grid(T, R, max_q_len, (C + per - 1) / per).by_piece;
+}
 
 // The most taps zk_conv_rows takes.
 int zk_conv_rows_most_taps() { return CONV_MOST_TAPS; }
@@ -231,17 +257,18 @@ int zk_conv_rows(const void* x, int ld_in, const float* in_bias, const float* w,
   const bool vec = C % 8 == 0 && ld_in % 8 == 0 && ld_out % 8 == 0 && aligned(x, 16) && aligned(out, 16) &&
                    (taps == 1 || (aligned(state, 16) && slot_words % 4 == 0 && offset_words % 4 == 0));
   ZK_REQUIRE(max_q_len <= 65535 * CONV_SPAN, "zk_conv_rows: too many tokens");
-  // the step's runs, at most (full ones and every request's last), and one block more for the padding behind the last request
-  const int one_run = max_q_len <= CONV_SPAN, runs = (one_run ? R : T / CONV_SPAN + R) + 1;
-  const int per = vec ? 8 : 1, columns = (C + per - 1) / per;
-  // few runs: narrow blocks, so that they spread over the compute units
-  const int threads = (long long)((columns + 255) / 256) * runs >= 512 ? 256 : 64;
-  ZK_REQUIRE((columns + threads - 1) / threads <= 65535, "zk_conv_rows: too many channels");
-  dim3 grid(runs, (columns + threads - 1) / threads);
-#define LAUNCH(V, N)                                                                                                  \
-  conv_rows_kernel<V, N><<<grid, threads, 0, (hipStream_t)stream>>>((const act_t*)x, ld_in, in_bias, w, bias, state,  \
-                                                                    slot_words, offset_words, q_start, slot_of_req,   \
-                                                                    (act_t*)out, ld_out, T, R, C, taps, residual, act, one_run)
+  const int per = vec ? 8 : 1;
+  const ConvGrid g = conv_grid(T, R, max_q_len, (C + per - 1) / per);
+  const dim3 grid = g.by_piece ? dim3((unsigned)(g.columns * g.runs)) : dim3(g.columns, g.runs, R + 1);
+#define LAUNCH_(V, N, PIECES)                                                                                         \
+  conv_rows_kernel<V, N, PIECES><<<grid, g.threads, 0, (hipStream_t)stream>>>(                                        \
+      (const act_t*)x, ld_in, in_bias, w, bias, state, slot_words, offset_words, q_start, slot_of_req, (act_t*)out, ld_out, T, R, C, \
+      taps, residual, act, g.columns)
+#define LAUNCH(V, N)                              \
+  do {                                            \
+    if (g.by_piece) LAUNCH_(V, N, true);          \
+    else LAUNCH_(V, N, false);                    \
+  } while (0)
   if (vec) {
     if (taps == 2) LAUNCH(8, 2);
     else if (taps == 3) LAUNCH(8, 3);
@@ -251,6 +278,7 @@ int zk_conv_rows(const void* x, int ld_in, const float* in_bias, const float* w,
     LAUNCH(1, 0);
   }
 #undef LAUNCH
+#undef LAUNCH_
   return zk_launch_status("zk_conv_rows");
 }
 
