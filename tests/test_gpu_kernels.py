@@ -752,7 +752,7 @@ def test_gated_activation_and_softcap(rt, dtype):
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("T", [27, 75])          # a block per (token, head); from 64 tokens a block per token
+@pytest.mark.parametrize("T", [27, 75])          # a block per (token, head): few tokens, or more than a wave of slots
 @pytest.mark.parametrize("nh,nkv,hd,rot,bs,vt", [(4, 2, 16, 16, 4, 0), (6, 1, 32, 32, 8, 1), (8, 4, 256, 256, 16, 1),
                                                 (3, 3, 64, 32, 16, 0), (2, 2, 48, 0, 4, 1)])
 def test_rope_and_cache_write(rt, dtype, T, nh, nkv, hd, rot, bs, vt):
@@ -858,12 +858,17 @@ def test_qkv_product_that_rotates_and_stores(rt, M, K, nh, nkv, hd, bs, vt, stri
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("T,nh,nkv,hd,bs,vt,rot", [(5, 3, 1, 48, 8, 1, 48), (40, 8, 4, 64, 16, 1, 64), (64, 2, 2, 256, 16, 1, 256),
-                                                 (100, 4, 2, 32, 8, 0, 32), (23, 2, 1, 64, 4, 0, 32), (72, 3, 3, 16, 8, 1, 16)])
+                                                 (100, 4, 2, 32, 8, 0, 32), (23, 2, 1, 64, 4, 0, 32), (72, 3, 3, 16, 8, 1, 16),
+                                                 # a block a token: more and fewer of them than the chip takes at once, value channels
+                                                 # that a block goes through in several turns, pages of fewer than eight, rows
+                                                 (305, 8, 4, 256, 16, 1, 256), (2051, 4, 2, 32, 8, 1, 32), (107, 2, 20, 256, 8, 1, 256),
+                                                 (2052, 4, 2, 32, 4, 1, 32), (520, 3, 2, 96, 16, 0, 96)])
 def test_rotation_that_adds_up_partial_sums_itself(rt, dtype, T, nh, nkv, hd, bs, vt, rot):
     """The rows of [q | k | v] as three planes of float partial sums, added up by the kernel that
     rotates and stores: the same bits, in q and in the cache, as from the rows added up in order and
     rounded to the storage type beforehand.  Eight tokens in a row land in eight slots in a row of
-    one page (the transposed store of whole groups) and one token is stored nowhere."""
+    one page (the transposed store of whole groups) and one token is stored nowhere.  More than a hundred tokens: all in blocks of a
+    token, and every other group of eight lands so."""
     k = rt.kernels(dtype)
     rng = np.random.default_rng(T * 10 + hd)
     width = (nh + 2 * nkv) * hd
@@ -875,6 +880,11 @@ def test_rotation_that_adds_up_partial_sums_itself(rt, dtype, T, nh, nkv, hd, bs
     slots = rng.permutation(free)[:T].astype(np.int32)
     if T >= 16 and bs >= 8:
         slots[8:16] = 2 * bs + np.arange(8)
+    if T > 100:
+        assert k._dll.zk_rope_by_token(T, nh, nkv, hd, rot, vt)
+        for t in range(32, T // 8 * 8 if bs >= 8 else 0, 16):      # slots of pages behind the scattered ones
+            slots[t:t + 8] = pages * bs + (t - 32) // 2 + np.arange(8)
+        pages += (T // 2 + bs - 1) // bs + 1
     slots[min(3, T - 1)] = -1
     pos = rng.integers(0, 5000, T).astype(np.int32)
     inv = (1.0 / 10000.0 ** (2.0 * np.arange(rot // 2) / rot)).astype(np.float32)

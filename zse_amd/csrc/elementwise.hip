@@ -567,27 +567,34 @@ __global__ void rope_cache_write_kernel(act_t* __restrict__ qkv, QkvSource from,
 
 // The same for the usual case (rotation over the whole head, head_dim a multiple of 8 and at
 // most 512): one block a token, the sines and cosines of the token's angles computed once for
-// all heads, four values a load.  What a thread reads first is asked for before the angles are worked out, and the
-// eight slots beside its own at once (one after the other, as a comparison that ends early reads them, they were up
-// to eight waits for memory).  MANY: so many tokens that the kernel is bound by its accesses, not by its waits: the values
-// are asked for when they are stored, four channels a thread, else before the angles, two.  us, 8 heads and 2 x 4 of 256: 535
-// tokens 5.7 -> 5.4, 1,000 6.6 -> 6.1 (MANY 6.8), 2,048 10.9 -> 9.2 (not MANY 9.8); 32 and 2 x 16 of 128, 2,048 15.1 -> 13.7 (16.7).
+// all heads, four values a load.  Three forms, by where the values go and by the number of tokens:
+// ROPE_ROWS, values in rows: everything is read when it is written (asked for in front of the angles, as below, 3.3 us became
+// 3.5 at 64 tokens of 8 and 2 x 2 heads of 64, 13.9 became 16.0 at 8,192).
+// ROPE_FEW, values transposed: what a thread reads first is asked for before the angles are worked out, two channels of the
+// values too, and the eight slots beside its own at once (one after the other, as a comparison that ends early reads them,
+// they were up to eight waits for memory).
+// ROPE_MANY, values transposed, more blocks than the chip takes at once (eight a compute unit): bound by its accesses, not by
+// its waits; the values are asked for when they are stored, four channels a thread.
+// us, FEW and MANY: 8 heads and 2 x 4 of 256, 800 tokens 5.7 and 6.6, 1,500 8.1 and 9.0, 2,048 9.9 and 9.3; 8 and 2 x 2 of 128,
+// 1,500 6.1 and 7.1, 2,048 7.9 and 7.7.
 #define ROPE_MAX_HALF 256
-template <bool MANY>
+enum { ROPE_ROWS, ROPE_FEW, ROPE_MANY };
+template <int FORM>
 __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
     act_t* __restrict__ qkv, QkvSource from, const int* __restrict__ positions, const int* __restrict__ slot_map,
     const float* __restrict__ inv_freq, act_t* __restrict__ kcache, act_t* __restrict__ vcache, int nh,
-    int nkv, int hd, int bs, int v_transposed) {
+    int nkv, int hd, int bs) {
   __shared__ float s_sin[ROPE_MAX_HALF], s_cos[ROPE_MAX_HALF];
-  constexpr int FIRST = 2;
+  constexpr bool MANY = FORM == ROPE_MANY, ROWS = FORM == ROPE_ROWS;
+  constexpr int FIRST = ROWS ? 0 : 2;
   const int t = blockIdx.x, tid = threadIdx.x, tl = t - t % 8;
   const int half = hd / 2, ppr = half / 4, items = (nh + nkv) * ppr;
   const size_t width = (size_t)(nh + 2 * nkv) * hd, row_at = (size_t)t * width;
   const float pos = (float)positions[t];
   const int slot = slot_map ? slot_map[t] : -1;
-  const int beside = slot_map ? slot_map[min(tl + (tid & 7), (int)gridDim.x - 1)] : -1;
+  const int beside = !ROWS && slot_map ? slot_map[min(tl + (tid & 7), (int)gridDim.x - 1)] : -1;
   // q and k heads: pieces of four pairs (i, i + half)
-  float a[FIRST][4], b[FIRST][4];
+  float a[FIRST + 1][4], b[FIRST + 1][4];
 #pragma unroll
   for (int j = 0; j < FIRST; j++) {
     const int it = min(tid + j * 256, items - 1);
@@ -597,7 +604,7 @@ __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
   }
   // v of the eight tokens tl .. tl + 7: the block's eighth of the channels, two a thread, from the last thread down (the first ones have more
   // of q and k), if the slots turn out to be eight in a row
-  const bool eight = v_transposed && bs % 8 == 0 && tl + 7 < (int)gridDim.x;
+  const bool eight = !ROWS && bs % 8 == 0 && tl + 7 < (int)gridDim.x;
   const int pairs = nkv * hd / 2, mine = (pairs + 7) / 8, first = (t - tl) * mine, last = min(first + mine, pairs);
   const size_t v_at = (size_t)tl * width + (size_t)(nh + nkv) * hd;
   float v8[8][2];
@@ -638,7 +645,7 @@ __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
   // v heads.  Transposed cache: eight tokens in a row of the step whose slots are eight in a
   // row of one page (a prompt portion) go out together, 8 values of a channel per store, each
   // of the eight blocks an eighth of the channels; other tokens are written value by value.
-  if (MANY && v_transposed && bs % 8 == 0 && tl + 7 < (int)gridDim.x) {
+  if (MANY && eight) {
     const int slot0 = __builtin_amdgcn_readfirstlane(beside);      // (lane 0 holds the first of the eight)
     if (slot0 >= 0 && slot0 % 8 == 0 && __all(beside == slot0 + (tid & 7))) {
       typedef act_t av8 __attribute__((ext_vector_type(8)));
@@ -661,7 +668,7 @@ __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
       return;
     }
   }
-  if (!MANY && eight) {
+  if (!MANY && !ROWS && eight) {
     const int slot0 = __builtin_amdgcn_readfirstlane(beside);      // (lane 0 holds the first of the eight)
     if (slot0 >= 0 && slot0 % 8 == 0 && __all(beside == slot0 + (tid & 7))) {
       typedef act_t av8 __attribute__((ext_vector_type(8)));
@@ -691,7 +698,7 @@ __global__ __launch_bounds__(256) void rope_cache_write_token_kernel(
     const int kvh = it / (hd / 4), d = (it % (hd / 4)) * 4;
     float v[4];
     from.at4(row_at + (size_t)(nh + nkv + kvh) * hd + d, v);
-    if (v_transposed) {
+    if (!ROWS) {
       act_t* vt = vcache + ((page * nkv + kvh) * (size_t)hd + d) * bs + off;
 #pragma unroll
       for (int e = 0; e < 4; e++) vt[(size_t)e * bs] = from_f32<act_t>(v[e]);
@@ -935,6 +942,22 @@ int zk_softcap(float* z, size_t n, float cap, void* stream) {
   return zk_launch_status("zk_softcap");
 }
 
+// A block a token, or a block per (token, head), which is quicker while these are few: its time goes with the number of its
+// blocks, and a block's with the size of a head (0.24 ns up to 64 channels, 0.33 for 128, 0.5 for 256), so the line is drawn by
+// blocks times channels and 64 more.  us, per head and by token: values transposed, 16 heads and 2 x 4 of 16, 400 tokens 4.6 and 4.3,
+// 2,048 13.9 and 7.2; 64 and 2 x 8 of 64, 100 4.4 and 4.9, 200 6.4 and 4.9; 8 and 2 x 4 of 256, 200 4.5 and 4.7, 400 6.4
+// and 5.1; as three planes of sums 64 and 2 x 8 of 64, 100 5.0 and 7.5, 200 8.1 and 7.9.  Values in rows (their kernel waits less):
+// 16 and 2 x 4 of 16, 200 3.6 and 3.3; 8 and 2 x 4 of 256, 200 4.0 and 4.1, 400 4.9 and 4.4.
+static bool rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed) {
+  const long long weight = (long long)T * (nh + 2 * nkv) * (std::max(hd, 64) + 64);
+  return weight > (v_transposed ? 5 << 18 : 1 << 19) && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF;
+}
+
+// 1 if the rotation of these rows goes by blocks of a token.  For tests that mean to reach both kernels.
+int zk_rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed) {
+  return rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed);
+}
+
 // sums > 0: the rows are not in qkv yet but come as that many planes of [T, (nh + 2 nkv) hd] float
 // partial sums (a product that split K and left the adding up to its reader, see QkvSource).
 int zk_rope_cache_write_sums(void* qkv, const float* planes, int sums, const int* positions, const int* slot_map,
@@ -948,13 +971,11 @@ int zk_rope_cache_write_sums(void* qkv, const float* planes, int sums, const int
   ZK_REQUIRE(sums == 0 || (planes != nullptr && (uintptr_t)planes % 16 == 0), "zk_rope_cache_write: partial sums must be 16-byte aligned");
   if (T == 0) return 0;
   const QkvSource from{(const act_t*)qkv, planes, sums, (size_t)T * (nh + 2 * nkv) * hd};
-  // a block a token pays off with many values, few are quicker spread over a block per (token, head).  us, by heads and by tokens:
-  // 8 and 2 x 4 of 256, 64 tokens 3.2 and 4.3 (as three planes of sums 3.9 and 6.5), 200 4.4 and 4.4, 303 5.2 and 4.9; 8 and 2 x 2 of 128, 303
-  // 3.5 and 4.3, 535 4.5 and 4.6; 32 and 2 x 16 of 128, 100 4.8 and 5.7, 200 7.2 and 5.4.
-  if ((long long)T * (nh + 2 * nkv) * hd > 1 << 20 && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF) {
-    const auto kernel = T >= 1500 ? rope_cache_write_token_kernel<true> : rope_cache_write_token_kernel<false>;
+  if (rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed)) {
+    const auto kernel = !v_transposed ? rope_cache_write_token_kernel<ROPE_ROWS>
+                        : T >= 8 * 256 ? rope_cache_write_token_kernel<ROPE_MANY> : rope_cache_write_token_kernel<ROPE_FEW>;
     kernel<<<T, 256, 0, (hipStream_t)stream>>>((act_t*)qkv, from, positions, slot_map, inv_freq, (act_t*)kcache, (act_t*)vcache, nh, nkv,
-                                               hd, bs, v_transposed);
+                                               hd, bs);
     return zk_launch_status("zk_rope_cache_write");
   }
   dim3 grid(T, nh + 2 * nkv);
