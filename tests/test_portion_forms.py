@@ -47,3 +47,16 @@ def test_many_groups_beside_a_long_decoded_context(R, rows, H, G, D):
     """A context that may be a decoded request's does not cut the keys of many groups into ranges."""
     assert form_of(1 << 30, R, rows, 8192, H, G, D)[0] == 5
     assert form_of(1 << 30, R, rows, 8192, H, G, D, not_theirs=1)[0] == 4
+
+
+# requests, rows, context, heads, key heads, channels, chunk: the beginning of a chunk among the rows, at their end, in front of them, in front
+# of the last one
+@pytest.mark.parametrize("case,short", [((1, 512, 8448, 8, 4, 256, 8192), 0), ((1, 256, 8208, 32, 16, 128, 8192), 0),
+                                        ((1, 256, 8192, 32, 16, 128, 8192), 0), ((1, 64, 8193, 8, 2, 128, 8192), 0),
+                                        ((3, 64, 8200, 16, 4, 128, 8192), 0), ((1, 256, 8448, 8, 4, 256, 8192), 1),
+                                        ((1, 64, 8256, 32, 16, 128, 8192), 1), ((1, 64, 100, 32, 16, 128, 64), 1),
+                                        ((1, 512, 8448, 8, 4, 256, 128), 1)])
+def test_a_chunk_that_begins_among_the_rows(case, short):
+    """The rows in front of it see the whole chunk before: their block has the most keys, not the last one."""
+    R, rows, ctx, H, G, D, chunk = case
+    assert (form_of(1 << 30, R, rows, ctx, H, G, D, chunk=chunk)[2] == 2) == bool(short)

@@ -339,9 +339,18 @@ static PortionPlan portion_plan(int max_q_len, int max_ctx, int window, int mask
 // five requests) it is 0.86 to 1.3 times what was measured up to one block a CU, and 0.93 to 1.9 times beyond, where what is close stays
 // with the others: 700 rows of 8 heads over 4 of 256, 352 blocks, 28.0 as they are and 30.9; 1,024 of 32 over 16 of 128 35.9 and 61.8.
 static double short_price(int max_q_len, int max_ctx, int window, int mask_chunk, int keep, int g, int nkv, int r_prefill, int wide) {
-  const int tokens = 16 / g, last = max_ctx - max_q_len + (max_q_len - 1) / tokens * tokens;      // the last block's first token
-  const int lo = mask_chunk > 0 ? last - last % mask_chunk : window > 0 ? std::max(0, last - window + 1) : 0;
-  const int tiles = std::min((keep + 31) / 32, lo / 32) + (max_ctx - 1) / 32 - lo / 32 + 1;
+  const int tokens = 16 / g, start = max_ctx - max_q_len, last = start + (max_q_len - 1) / tokens * tokens;
+  auto tiles_of = [&](int first) {      // of the block whose first token that is
+    const int lo = mask_chunk > 0 ? first - first % mask_chunk : window > 0 ? std::max(0, first - window + 1) : 0;
+    return std::min((keep + 31) / 32, lo / 32) + (std::min(max_ctx, first + tokens) - 1) / 32 - lo / 32 + 1;
+  };
+  int tiles = tiles_of(last);
+  // Behind a chunk's beginning the rows see few keys again: where one lies among the rows, the block in front of it has the most (512
+  // rows of 8 heads over 4 of 256 that end 256 behind a chunk of 8,192: 8 tiles in the last block, 257 in the longest)
+  if (mask_chunk > 0) {
+    const int begins = last - last % mask_chunk;
+    if (begins > start) tiles = std::max(tiles, tiles_of(start + (begins - 1 - start) / tokens * tokens));
+  }
   // (256 channels and more than four tiles a wave: the prices of both kinds are off by as much as they differ, 16 rows behind 500 keys
   // 16.9 as they are and 17.6, 128 rows 20.8 and 19.1)
   if (wide > 128 && tiles > 16) return 1e30;
