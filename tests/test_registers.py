@@ -1,0 +1,38 @@
+"""Kernels that keep what they work on in registers: that the compiler did so, in both libraries."""
+import re
+import shutil
+import subprocess
+
+import pytest
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.fixture(scope="module", params=["kernels_bf16", "kernels_f32"])
+def scratch(request, tmp_path_factory):
+    """Bytes of scratch memory a lane of every kernel of a library, by its symbol."""
+    from zse_amd.runtime import build
+    if shutil.which(READELF) is None or shutil.which(OBJDUMP) is None:
+        pytest.skip("no llvm-readelf or llvm-objdump")
+    if not build.is_current(request.param):
+        build.build(request.param)
+    folder = tmp_path_factory.mktemp("code")
+    shutil.copy(build.lib_path(request.param), folder / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, stdout=subprocess.DEVNULL)
+    out = {}
+    for obj in sorted(folder.glob("*gfx950")):
+        notes = subprocess.run([READELF, "--notes", str(obj)], check=True, capture_output=True, text=True).stdout
+        for part in notes.split("  - .agpr_count:")[1:]:
+            out[re.search(r"\.name:\s+(\w+)", part)[1]] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", part)[1])
+    return out
+
+
+# a kernel, the number of its forms, those of them that may go through scratch memory
+@pytest.mark.parametrize("kernel,forms,but", [("streams_row_kernel", 7, "ILi4ELi4ELi1024E"), ("conv_rows_kernel", 10, None),
+                                              ("rope_cache_write_token_kernel", 3, None), ("mlstm_output_kernel", 6, None),
+                                              ("mlstm_local_kernel", 6, None)])
+def test_no_scratch_memory(scratch, kernel, forms, but):
+    found = {s: n for s, n in scratch.items() if kernel in s}
+    assert len(found) == forms
+    assert {s: n for s, n in found.items() if n and not (but and but in s)} == {}

@@ -34,11 +34,14 @@ __global__ void replicate_kernel(const float* __restrict__ src, float* __restric
 }
 
 // S streams of rows that are whole 16-byte pieces, NV of them a thread (4 NV threads >= W): a thread's part of all
-// streams is asked for at once and stays in its registers, so that the row is one trip to memory and
-// two sums.  The kernel below, which goes over the row pass by pass and keeps the read in the local memory, took (us; 708 rows of
-// four streams of 2,048, 52 MB) 19.7, this one 11.2.
-template <int S, int NV>
-__global__ __launch_bounds__(1024) void streams_row_kernel(
+// streams is asked for at once and kept, so that the row is one trip to memory and two sums.  The kernel below, which goes over
+// the row pass by pass and keeps the read in the local memory, took (us; 708 rows of four streams of 2,048, 52 MB)
+// 14.7, this one 8.0; of 4,096 28.3 and 17.8.
+// MOST: threads of a block, at most, which is what bounds its registers.  All forms are within 128 but four pieces of four
+// streams: 156 in blocks of 256 (held to 128, 72 of them go through scratch memory: 23.3); in blocks of 1,024 (up to 64 rows of
+// more than 8,192 channels) they do, and it still takes 20.1 in place of 22.7 (64 rows of 16,384).
+template <int S, int NV, int MOST>
+__global__ __launch_bounds__(MOST) void streams_row_kernel(
     float* __restrict__ xs, const void* __restrict__ y, int y_parts, size_t y_plane, const float* __restrict__ w_mix,
     const float* __restrict__ w_out, const float* __restrict__ w_in, const float* __restrict__ norm_w,
     const float* __restrict__ norm_b, float eps, const int* __restrict__ rows, act_t* __restrict__ out, int W) {
@@ -361,11 +364,14 @@ int zk_streams_step(float* xs, int S, const void* y, int y_parts, const float* w
   const bool pieces = vec && aligned(norm_w, 16) && aligned(norm_b, 16) && aligned(out, sizeof(act_t) * 4) &&
                       aligned(y, y_parts > 0 ? 16 : sizeof(act_t) * 4);
   if (pieces && (S == 2 || S == 4) && nv <= 4) {
-#define ZK_ROW(S_, NV_)                                                                                                       \
-  streams_row_kernel<S_, NV_><<<n_rows, threads, 0, (hipStream_t)stream>>>(xs, y, y_parts, (size_t)T * W, w_mix, w_out, w_in, \
-                                                                          norm_w, norm_b, eps, rows, (act_t*)out, W)
-    if (S == 2) { if (nv == 1) ZK_ROW(2, 1); else if (nv == 2) ZK_ROW(2, 2); else ZK_ROW(2, 4); }
-    else { if (nv == 1) ZK_ROW(4, 1); else if (nv == 2) ZK_ROW(4, 2); else ZK_ROW(4, 4); }
+#define ZK_ROW(S_, NV_, MOST_)                                                      \
+  streams_row_kernel<S_, NV_, MOST_><<<n_rows, threads, 0, (hipStream_t)stream>>>(  \
+      xs, y, y_parts, (size_t)T * W, w_mix, w_out, w_in, norm_w, norm_b, eps, rows, (act_t*)out, W)
+    if (S == 2) { if (nv == 1) ZK_ROW(2, 1, 1024); else if (nv == 2) ZK_ROW(2, 2, 1024); else ZK_ROW(2, 4, 1024); }
+    else if (nv == 1) ZK_ROW(4, 1, 1024);
+    else if (nv == 2) ZK_ROW(4, 2, 1024);
+    else if (threads == 256) ZK_ROW(4, 4, 256);
+    else ZK_ROW(4, 4, 1024);
 #undef ZK_ROW
     return zk_launch_status("zk_streams_step");
   }
