@@ -15,3 +15,5 @@ register_kernels("toy_decay", os.path.join(HERE, "toy_decay.hip"),
 # query and key heads scaled to unit length between product and rotation (test_gpu_parts.py)
 register_kernels("toy_head_norm", os.path.join(HERE, "toy_head_norm.hip"),
                  {"zk_toy_head_norm": [_VP, _I, _I, _I, _I, _VP]})
+# sums over waves and blocks of any size (test_gpu_wave_sums.py)
+register_kernels("toy_sums", os.path.join(HERE, "toy_sums.hip"), {"zk_toy_sums": [_VP, _VP, _I, _I, _VP]}, dtypes=("float32",))

@@ -164,9 +164,9 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
       ml[1] = at[1];
     }
     const bool mine = lane < np;
-    const float m = wave_max(mine ? ml[0] : -INFINITY);
+    const float m = wave_max_whole(mine ? ml[0] : -INFINITY);
     const float w = __builtin_amdgcn_exp2f(ml[0] - m);
-    const float l = wave_sum(mine ? ml[1] * w : 0.f);
+    const float l = wave_sum_whole(mine ? ml[1] * w : 0.f);
     const float inv = gate_factor(gate, gate_ld, row, head) / (l + sink_weight(sinks, sink, head, m));
     auto weight = [&](int c) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), c)); };
     if ((int)threadIdx.x < hd) {

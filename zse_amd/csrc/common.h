@@ -42,6 +42,9 @@ __device__ __forceinline__ void rotate_pair(float a, float b, float sn, float cs
 // cycles; through the local memory, as __shfl_xor goes, about a hundred), in the order 32, 16, 8, 4, 2, 1: the sum is
 // the same bits in every lane.  Kernels of a few rows are a chain of such steps (us, through the local memory and so: a
 // step of one decoded token, 2B shapes, 1,786 and 1,722, of eight 2,423 and 2,355; a model of six layers of width 1,024 234 and 222).
+//
+// The permutations do not fetch from lanes that are not there: everything down to the running sums, but for wave_sum, wave_max
+// and block_sum, is for waves whose 64 lanes are all active (blocks of whole waves, outside of conditions on lanes).
 // Lane l's partner l ^ 32 or l ^ 16: the pair's two values, in some order.
 __device__ __forceinline__ void wave_pair32(float v, float& a, float& b) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -74,13 +77,13 @@ __device__ __forceinline__ float wave_sum16(float v) {      // over the 16 lanes
   v += wave_dpp<ZSE_DPP_XOR1>(v);
   return v;
 }
-__device__ __forceinline__ float wave_sum(float v) {
+__device__ __forceinline__ float wave_sum_whole(float v) {
   float a = 0.f, b = 0.f;
   wave_pair32(v, a, b);
   wave_pair16(a + b, a, b);
   return wave_sum16(a + b);
 }
-__device__ __forceinline__ float wave_max(float v) {
+__device__ __forceinline__ float wave_max_whole(float v) {
   float a = 0.f, b = 0.f;
   wave_pair32(v, a, b);
   wave_pair16(fmaxf(a, b), a, b);
@@ -89,6 +92,21 @@ __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, wave_dpp<ZSE_DPP_ROR4>(v));
   v = fmaxf(v, wave_dpp<ZSE_DPP_XOR2>(v));
   return fmaxf(v, wave_dpp<ZSE_DPP_XOR1>(v));
+}
+// The same over the lanes that are active: in a wave that lacks some, one after the other.
+__device__ __forceinline__ bool wave_is_whole() { return __ballot(1) == ~0ull; }
+__device__ __forceinline__ float wave_lane(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
+__device__ __forceinline__ float wave_sum(float v) {
+  if (wave_is_whole()) return wave_sum_whole(v);
+  float t = 0.f;
+  for (unsigned long long left = __ballot(1); left; left &= left - 1) t += wave_lane(v, __ffsll(left) - 1);
+  return t;
+}
+__device__ __forceinline__ float wave_max(float v) {
+  if (wave_is_whole()) return wave_max_whole(v);
+  float t = -INFINITY;
+  for (unsigned long long left = __ballot(1); left; left &= left - 1) t = fmaxf(t, wave_lane(v, __ffsll(left) - 1));
+  return t;
 }
 
 // Sums and maxima over a lane and its partners 16, 32 or both away (in that order).
@@ -143,18 +161,25 @@ __device__ __forceinline__ float wave_running_max(float v) {
 
 // Sum over a block of up to 1024 threads; every thread gets the result (each wave adds the waves' sums up for
 // itself).  ``scratch`` holds at least 16 floats of LDS that nothing else of the block is reading or writing;
-// block_sum may be called again with the same ones.
+// block_sum may be called again with the same ones.  block_sum_once: blocks of whole waves.
 __device__ __forceinline__ float block_sum_once(float v, float* scratch) {
-  const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE;
-  const int nw = (blockDim.x + ZSE_WAVE - 1) / ZSE_WAVE;
-  v = wave_sum(v);
+  const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE, nw = blockDim.x / ZSE_WAVE;
+  v = wave_sum_whole(v);
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
   return wave_sum16((lane & 15) < nw ? scratch[lane & 15] : 0.f);
 }
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
+  const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE;
+  const int nw = (blockDim.x + ZSE_WAVE - 1) / ZSE_WAVE;
   __syncthreads();
-  return block_sum_once(v, scratch);
+  v = wave_sum(v);
+  if (lane == 0) scratch[wave] = v;
+  __syncthreads();
+  if (blockDim.x % ZSE_WAVE == 0) return wave_sum16((lane & 15) < nw ? scratch[lane & 15] : 0.f);
+  v = 0.f;                               // a last wave that is not whole: all waves add up alike
+  for (int w = 0; w < nw; w++) v += scratch[w];
+  return v;
 }
 
 // Requests are rows [q_start[r], q_start[r + 1]) of a step, cut into pieces of ``len`` rows that are numbered
