@@ -31,8 +31,10 @@ def scratch(request, tmp_path_factory):
 # a kernel, the number of its forms, those of them that may go through scratch memory
 @pytest.mark.parametrize("kernel,forms,but", [("streams_row_kernel", 7, "ILi4ELi4ELi1024E"), ("conv_rows_kernel", 10, None),
                                               ("rope_cache_write_token_kernel", 3, None), ("mlstm_output_kernel", 6, None),
-                                              ("mlstm_local_kernel", 6, None)])
+                                              ("mlstm_local_kernel", 6, None), ("attention_f32_kernel", 8, None)])
 def test_no_scratch_memory(scratch, kernel, forms, but):
     found = {s: n for s, n in scratch.items() if kernel in s}
+    if not found and kernel == "attention_f32_kernel":
+        pytest.skip("in the 32-bit library only")
     assert len(found) == forms
     assert {s: n for s, n in found.items() if n and not (but and but in s)} == {}

@@ -162,7 +162,7 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // Bound by the latency of the loads for few tokens and by the matrix cores for many.  Measured
 // (us; before: a wave per token and head whose lanes each walked a key's row):
 //   303 tokens, 8 heads of 128, contexts of 300 and three of 50 to 700: 852 -> 38.
-//   One token, 8 heads over 2 of 128: 1 key 12.4 -> 10.2, 100 keys 57 -> 15, 4,000 keys 2,111 -> 132; 4 heads
+//   One token, 8 heads over 2 of 128: 1 key 12.4 -> 9.3, 100 keys 57 -> 15, 4,000 keys 2,111 -> 130; 4 heads
 //   of 16: 6.9 -> 8.5, 26 -> 11, 884 -> 83; 8 over 4 of 256: 21.7 -> 22.7, 109 -> 27, 6,260 -> 458.  (Heads of up
 //   to 64 are slower than before below about ten keys, of 256 below three.)
 //
@@ -174,9 +174,10 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
 // ASK: keys and values are asked for without a condition and a piece of 16 ahead of their products (the first values in
 // front of the weights), and pieces that no row sees are passed over in the first product too.  For key heads of 65 to
 // 128 channels, 8 heads over 2 of 128 (us; keys alone without a condition, and each piece at its turn; both ahead): 303 tokens,
-// 300 of them a prompt, 35.8 and 33.5; one token with 4,000 keys 141 and 132; 64 requests of 100 to 3,250 keys 142 and
-// 110; 1,000 requests of 3 tokens 493 and 381; 1,500 tokens 140 and 131, behind a window of 64 62 and 54; one token with
-// 1 key 9.9 and 10.2, 8 of 500 24.1 and 24.5, 1,000 requests of 3 tokens with 3 keys 95 and 98 (the waits for pieces that are passed over, a few more instructions).  Not
+// 300 of them a prompt, 34.9 and 32.5; one token with 4,000 keys 140 and 130; 64 requests of 100 to 3,250 keys 138 and
+// 108; 1,000 requests of 3 tokens 498 and 381, with 3 keys 93 and 95; 1,500 tokens 137 and 130, behind a window of 64 61 and 53;
+// one token with 1 key 9.4 and 9.3, with 300 or 500 keys, a tile for each wave, 19.5 and 19.9, 23.1 and 23.4 (the keys of pieces behind the
+// last are waited for: not asked for under a condition, which costs 303 tokens 26 us).  Not
 // for smaller key heads (8 over 4 of 64, 4,000 keys: 92 and 94; with values of 128 34 and 65: the registers
 // do not hold both); of 256 the loads in flight do not fit (446 -> 472).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
       // ASK: a piece's keys and values are asked for a piece ahead, the first values in front of the weights.  They are
       // held in front of the branches that pass over unseen pieces, behind which the compiler would move their loads.
       f32x4 s[4], k_ahead[2][QC], v_ahead[2][4][VC];
-      bool has[2][4];              // the key of a value asked for is in the cache
+      bool has[2][4];              // the key of a value asked for is in the cache (with PACK found out again: the registers do not hold it)
       auto ask_keys = [&](int f) {
 #pragma unroll
         for (int c = 0; c < QC; c++)
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const long long va = __shfl(at[f], 4 * qd + e);
-          has[f & 1][e] = va >= 0;
+          if (!PACK) has[f & 1][e] = va >= 0;
 #pragma unroll
           for (int c = 0; c < VC; c++)
             v_ahead[f & 1][e][c] = *(const f32x4*)(vcache + (size_t)max(va, 0LL) * vd + min(64 * c + 4 * r, vd - 4));
@@ -371,6 +372,7 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
       for (int f = 0; f < 4; f++) {
         if (ASK) {
+          if (f && j0 + 16 * f > seg_hi) break;      // (no wait for a piece behind the last key)
           if (f < 3) ask_values(f + 1);
 #pragma unroll
           for (int e = 0; e < 4; e++)
@@ -384,10 +386,11 @@ __global__ __launch_bounds__(64 * WAVES) void attention_f32_kernel(
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           if (!ASK) va[e] = __shfl(at[f], 4 * qd + e);
+          const bool there = !ASK ? false : PACK ? __shfl((int)(at[f] >> 32), 4 * qd + e) >= 0 : has[f & 1][e];
 #pragma unroll
           for (int c = 0; c < VC; c++) {
             const int d = 64 * c + 4 * r;
-            if (ASK) v[e][c] = has[f & 1][e] && d < vd ? v_ahead[f & 1][e][c] : zero;
+            if (ASK) v[e][c] = there && d < vd ? v_ahead[f & 1][e][c] : zero;
             else v[e][c] = va[e] >= 0 && d < vd ? *(const f32x4*)(vcache + (size_t)va[e] * vd + d) : zero;
           }
         }
