@@ -29,3 +29,13 @@ def test_rotation_by_token(name, T, nh, nkv, hd, transposed, by_token):
     lib = library(name)
     assert lib.zk_rope_by_token(T, nh, nkv, hd, hd, transposed) == by_token
     assert lib.zk_rope_by_token(T, nh, nkv, hd, hd // 2, transposed) == 0      # a part of the head turned: per head
+
+
+@pytest.mark.parametrize("D,tokens", [(64, 64), (128, 64), (192, 64), (200, 32), (224, 32), (256, 32)])
+def test_chunks_of_the_matrix_memory(D, tokens):
+    """Chunks of 64 tokens of heads of 256 key channels took 64 us, of 32 52 (600 tokens, four heads of 40 value channels)."""
+    floats = library().zk_mlstm_scan_floats
+    floats.restype = C.c_size_t
+    chunks = lambda L: (600 + L - 1) // L + 2
+    assert floats(600, 2, 4, D, 40, 500) == chunks(tokens) * 4 * (D * 40 + D + 3)
+    assert floats(600, 2, 4, D, 40, 30) == chunks(32) * 4 * (D * 40 + D + 3)

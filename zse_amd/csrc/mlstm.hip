@@ -715,7 +715,7 @@ __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_output_kernel(
             F + M;
     }
     __syncthreads();
-    // P and the denominators: a wave takes every fourth tile of rows, and the tiles of columns up to the diagonal
+    // P and the denominators: a wave takes every fourth tile of rows, all tiles of columns (zeros behind the diagonal)
     const int KS = (P - 4) / 16;           // groups of 16 key channels
 #pragma unroll
     for (int a0 = 0; a0 < (RT + 3) / 4; a0++) {
@@ -934,9 +934,13 @@ int zk_mlstm_chunked(const void* qkvz, int ld, const float* gates, const float* 
 
 }  // extern "C"
 
+// Tokens a chunk: few enough that the output kernel's block leaves a quarter of the local memory (us, three launches; chunks of 64 and of
+// 32: one request of 600, four heads of 40 value channels, 256 key channels 63.9 and 52.2, 224 60.0 and 49.6, 192 51.9 and
+// 43.1; eight heads of 256 value channels 75.6 and 73.2, 70.0 and 68.1, 61.5 and 59.5; 2,048 tokens, four heads of 256, 93.4 and
+// 97.2, 85.7 and 91.8, 74.4 and 81.3).
 static int mlstm_scan_len(int max_q_len, int D) {
   int L = max_q_len <= 16 ? 16 : max_q_len <= 32 ? 32 : 64;
-  while (L > 16 && mlstm_output_lds(L, D) > 150 * 1024) L /= 2;
+  while (L > 16 && mlstm_output_lds(L, D) > 120 * 1024) L /= 2;
   return L;
 }
 
@@ -982,7 +986,7 @@ extern "C" {
 
 // zk_mlstm_chunked's work with the chunks of a step side by side (three launches); for steps
 // whose portions are several chunks long.  work: zk_mlstm_scan_floats(...) floats of scratch.
-// zk_mlstm_finish (with nm_new null: the scan stores n and m itself) must follow.
+// zk_mlstm_finish (with nm_new null: n is stored by the scan, m by the output kernel) must follow.
 int zk_mlstm_scan(const void* qkvz, int ld, const float* gates, const float* bias_i, const float* bias_f, float* state,
                   int slot_words, int offset_words, const int* q_start, const int* slot_of_req, float* o_raw, float* work,
                   size_t work_floats, int T, int R, int H, int D, int E, float cap, int max_q_len, void* stream) {
