@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 from plain import dafotar_plain as P
+from zse_amd.weights.safetensors import bf16_bits_to_f32, f32_to_bf16_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -27,8 +28,13 @@ def _operands():
 
 
 def up(rt, a, dtype=None):
-    _alive.append(rt.upload(np.ascontiguousarray(a), dtype))
+    a = np.ascontiguousarray(a)
+    _alive.append(rt.upload(f32_to_bf16_bits(a) if dtype == "bfloat16" else a, dtype))
     return _alive[-1]
+
+
+def bf16(a):
+    return bf16_bits_to_f32(f32_to_bf16_bits(np.ascontiguousarray(a, np.float32)))
 
 
 def i32(rt, a):
@@ -155,14 +161,28 @@ def test_matrix_memory_cut_into_steps(dev, H, D, E):
         assert not rt.download(state)[0].any()
 
 
+# (heads of more than 128 value channels are several blocks side by side, the last one with waves of which some lanes or none have
+# channels; an odd number of channels is read and written one at a time)
 @pytest.mark.parametrize("side_by_side", [False, True])
-@pytest.mark.parametrize("H,D,E", [(1, 8, 8), (3, 12, 20), (2, 64, 128), (1, 128, 48), (1, 256, 40)])
+@pytest.mark.parametrize("H,D,E", [(1, 8, 8), (3, 12, 20), (2, 64, 128), (1, 128, 48), (1, 256, 40), (2, 72, 256), (1, 20, 130),
+                                   (3, 7, 21), (1, 33, 161)])
 def test_matrix_memory_in_chunks(dev, H, D, E, side_by_side):
     """The chunked form of the recurrence with its finishing kernel: two requests side by side,
     portions of 1 to 150 tokens (chunks of 16, 32 and 64; full, partial and single-token ones),
     continuing from the state the portion before left.  ``side_by_side``: the three launches that
     run a step's chunks at once, instead of the kernel that walks them."""
     rt, k = dev
+    matrix_memory_in_chunks(rt, k, "float32", H, D, E, side_by_side)
+
+
+@pytest.mark.parametrize("side_by_side", [False, True])
+@pytest.mark.parametrize("H,D,E", [(2, 64, 128), (1, 72, 160), (3, 7, 21)])
+def test_matrix_memory_in_chunks_of_16_bits(dev, H, D, E, side_by_side):
+    """The same with q, k, v and the gate as bfloat16 rows; the state and all sums stay floats."""
+    matrix_memory_in_chunks(dev[0], dev[0].kernels("bfloat16"), "bfloat16", H, D, E, side_by_side)
+
+
+def matrix_memory_in_chunks(rt, k, dtype, H, D, E, side_by_side):
     rng = np.random.default_rng(D + E)
     W = 16
     mx = {"heads": H, "dim": D, "vdim": E, "gate_cap": 5.0}
@@ -174,9 +194,17 @@ def test_matrix_memory_in_chunks(dev, H, D, E, side_by_side):
     wts = {n: a.astype(np.float32) for n, a in wts.items()}
     lens = {0: 236, 1: 97}
     hs = {r: rng.normal(size=(n, W)).astype(np.float32) for r, n in lens.items()}
-    want = {r: P.mlstm(h, wts, "", mx, 1e-6, np.float64) for r, h in hs.items()}
     proj = {r: np.concatenate([h @ wts[n].T for n in ("q", "k", "v", "g")], axis=1).astype(np.float32) for r, h in hs.items()}
     gate = {r: np.concatenate([h @ wts["i"].T, h @ wts["f"].T], axis=1).astype(np.float32) for r, h in hs.items()}
+    if dtype == "bfloat16":
+        # the plain recurrence on the rows as the kernels see them: its projections pick them out of the row
+        proj = {r: bf16(p) for r, p in proj.items()}
+        width, at = 2 * H * (D + E) + 2 * H, 0
+        hs = {r: np.concatenate([proj[r], gate[r]], axis=1) for r in hs}
+        for n, rows in (("q", H * D), ("k", H * D), ("v", H * E), ("g", H * E), ("i", H), ("f", H)):
+            wts[n] = np.eye(rows, width, at, dtype=np.float32)
+            at += rows
+    want = {r: P.mlstm(h, wts, "", mx, 1e-6, np.float64) for r, h in hs.items()}
     cuts = {0: [150, 1, 17, 64, 4], 1: [30, 33, 1, 2, 31]}
     words = 4 + k.zk_mlstm_state_bytes(H, D, E) // 4
     state = rt.zeros((3, words), "float32")
@@ -189,10 +217,10 @@ def test_matrix_memory_in_chunks(dev, H, D, E, side_by_side):
         T = n0 + n1
         rows = np.concatenate([proj[0][at[0]:at[0] + n0], proj[1][at[1]:at[1] + n1]])
         gts = np.concatenate([gate[0][at[0]:at[0] + n0], gate[1][at[1]:at[1] + n1]])
-        d_rows, d_g = up(rt, rows), up(rt, gts)
+        d_rows, d_g = up(rt, rows, dtype), up(rt, gts)
         q_start, req = i32(rt, [0, n0, T]), i32(rt, [0] * n0 + [1] * n1)
         d_slots = i32(rt, slots)
-        o_raw, nm, d_o = rt.zeros((T, H * E), "float32"), rt.zeros((2, H * (D + 1)), "float32"), rt.empty((T, H * E), "float32")
+        o_raw, nm, d_o = rt.zeros((T, H * E), "float32"), rt.zeros((2, H * (D + 1)), "float32"), rt.empty((T, H * E), dtype)
         if side_by_side:
             floats = k.zk_mlstm_scan_floats(T, 2, H, D, E, max(n0, n1))
             work = rt.zeros((floats,), "float32")
@@ -203,19 +231,21 @@ def test_matrix_memory_in_chunks(dev, H, D, E, side_by_side):
                                o_raw.ptr, nm.ptr, 2, H, D, E, 5.0, max(n0, n1), rt.stream)
         k.zk_mlstm_finish(o_raw.ptr, d_rows.ptr, rows.shape[1], g.ptr, None if side_by_side else nm.ptr, state.ptr, words, 4,
                           req.ptr, q_start.ptr, d_slots.ptr, d_o.ptr, T, H, D, E, 1e-6, rt.stream)
-        o = rt.download(d_o)
+        o = rt.download_f32(d_o)
         got[0].append(o[:n0])
         got[1].append(o[n0:])
         at[0] += n0
         at[1] += n1
     for r in (0, 1):
-        err = np.abs(np.concatenate(got[r]) - want[r]).max()
+        # (bfloat16: and half a unit of its last place for the rounding of the result)
+        rounding = 2.0 ** -8 * np.abs(want[r]) if dtype == "bfloat16" else 0.0
+        err = (np.abs(np.concatenate(got[r]) - want[r]) - rounding).max()
         assert err < 5e-5 * max(1.0, np.abs(want[r]).max()), (r, err)
     # and the state it leaves is the one the token-by-token kernel leaves
     seq = rt.zeros((3, words), "float32")
     for r in (0, 1):
-        d_o = rt.empty((lens[r], H * E), "float32")
-        k.zk_mlstm(up(rt, proj[r]).ptr, proj[r].shape[1], up(rt, gate[r]).ptr, bi.ptr, bf.ptr, g.ptr, seq.ptr, words, 4,
+        d_o = rt.empty((lens[r], H * E), dtype)
+        k.zk_mlstm(up(rt, proj[r], dtype).ptr, proj[r].shape[1], up(rt, gate[r]).ptr, bi.ptr, bf.ptr, g.ptr, seq.ptr, words, 4,
                    i32(rt, [0, lens[r]]).ptr, i32(rt, [slots[r]]).ptr, d_o.ptr, 1, H, D, E, 5.0, 1e-6, rt.stream)
     a, b = rt.download(state), rt.download(seq)
     assert np.abs(a - b).max() < 1e-4 * max(1.0, np.abs(b).max())
@@ -310,6 +340,30 @@ def test_streams_of_whole_pieces(dev, S, W, parts):
                       rt.stream)
     want = P.layer_norm(want_xs.sum(axis=1)[[2, 0]], g, np.zeros(W), 1e-5, np.float64)
     assert np.abs(rt.download(d_p) - want).max() < 3e-5
+
+
+# (up to 64 rows in blocks of 1,024 threads, more in blocks of 256)
+@pytest.mark.parametrize("T,S,W,parts", [(3, 4, 4, 0), (64, 4, 2048, 2), (3, 2, 4100, 0), (2, 4, 8192, 0), (2, 4, 16384, 3), (2, 2, 16380, 1),
+                                         (65, 2, 1020, 0), (65, 4, 1024, 3), (65, 4, 2048, 0), (65, 2, 4096, 2), (65, 4, 3076, 0)])
+def test_streams_of_whole_pieces_in_16_bits(dev, T, S, W, parts):
+    """What is written to the streams and read from them as bfloat16 rows, the streams themselves floats.  Partial sums are
+    sixty-fourths below 8, whose sums are exact: they round to the same bfloat16 in every order."""
+    rt, k = dev[0], dev[0].kernels("bfloat16")
+    rng = np.random.default_rng(W + S)
+    xs = rng.normal(size=(T, S, W)).astype(np.float32)
+    y = rng.integers(-500, 501, (max(parts, 1), T, W)).astype(np.float32) / 64
+    mix, out, win = (rng.normal(size=s).astype(np.float32) for s in ((S, S), (S,), (S,)))
+    g, b = rng.normal(1, 0.2, W).astype(np.float32), rng.normal(0, 0.2, W).astype(np.float32)
+    d_xs, d_o = up(rt, xs), rt.empty((T, W), "bfloat16")
+    d_y = up(rt, y) if parts else up(rt, y[0], "bfloat16")
+    k.zk_streams_step(d_xs.ptr, S, d_y.ptr, parts, up(rt, mix).ptr, up(rt, out).ptr, up(rt, win).ptr, up(rt, g).ptr, up(rt, b).ptr,
+                      1e-5, None, d_o.ptr, T, T, W, rt.stream)
+    want_xs = P.streams_write(xs, mix, out, bf16(y.sum(0)), np.float64)
+    # S + 1 products, each added up with one rounding
+    most = P.streams_write(np.abs(xs), np.abs(mix), np.abs(out), np.abs(y.sum(0)), np.float64)
+    assert (np.abs(rt.download(d_xs) - want_xs) <= (S + 2) * 2.0 ** -24 * most).all()
+    want = P.layer_norm(P.streams_read(want_xs, win, np.float64), g, b, 1e-5, np.float64)
+    assert (np.abs(rt.download_f32(d_o) - want) - 2.0 ** -8 * np.abs(want)).max() < 3e-5
 
 
 MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17]       # rows of 72 requests
