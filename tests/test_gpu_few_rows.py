@@ -89,15 +89,18 @@ def test_the_rotating_product_gives_the_bits_of_product_and_rotation(M, nh, nkv,
 
 @pytest.mark.parametrize("nh,nkv,hd", [(8, 4, 256), (8, 2, 128), (16, 1, 64)])
 def test_attention_of_few_and_many_blocks_and_with_a_window_that_shows_all(nh, nkv, hd):
-    """Requests of one to 78 parts of 128 keys: alone, among so many that the chip is full,
-    and behind a window as long as the longest context, whose parts are counted from the request's length: the same bits."""
+    """Requests of one to 78 parts of 128 keys (32 of which the join asks for at once, and those up to 64 eight at a time): alone,
+    among so many that the chip is full, and behind a window as long as the longest context, whose parts are counted from the request's
+    length: the same bits, those of 64-bit sums but for the rounding of weights and results."""
+    from test_gpu_stream_attention import plain, rounded
     from zse_amd.weights.safetensors import f32_to_bf16_bits
     rt, k = dev()
     rng = np.random.default_rng(hd)
     up = lambda x: rt.upload(f32_to_bf16_bits(np.ascontiguousarray(x, np.float32)), "bfloat16")
-    bs, lens = 16, [1, 128, 129, 1000, 1030, 2049, 4100, 9900]
+    bs, lens = 16, [1, 128, 129, 1000, 1030, 2049, 4100, 9900, 5200, 8192]
     ends = np.cumsum([0] + [-(-n // bs) for n in lens])
-    kc, vc = up(rng.normal(size=(ends[-1], nkv, bs, hd))), up(rng.normal(size=(ends[-1], nkv, hd, bs)))
+    keys, values = rng.normal(size=(ends[-1], nkv, bs, hd)), rng.normal(size=(ends[-1], nkv, hd, bs))
+    kc, vc = up(keys), up(values)
     q = rng.normal(size=(len(lens), nh, hd)).astype(np.float32)
 
     def run(copies, window, chunk):
@@ -116,6 +119,12 @@ def test_attention_of_few_and_many_blocks_and_with_a_window_that_shows_all(nh, n
         return rt.download_f32(out).reshape(copies, len(lens), nh * hd)
     want = run(1, 0, 32)[0]
     assert np.isfinite(want).all() and want.any(axis=1).all()
+    for i, n in enumerate(lens):
+        kk = rounded(keys[ends[i]:ends[i + 1]]).transpose(0, 2, 1, 3).reshape(-1, nkv, hd)[:n].astype(np.float64)
+        vv = rounded(values[ends[i]:ends[i + 1]]).transpose(0, 3, 1, 2).reshape(-1, nkv, hd)[:n].astype(np.float64)
+        o, size = (plain(rounded(q[i:i + 1]).astype(np.float64), kk, v, n - 1, hd ** -0.5, 50.0, 0, 0) for v in (vv, np.abs(vv)))
+        # weights rounded to 8 bits of mantissa (not in their sum), and the result's own rounding
+        assert (np.abs(want[i].reshape(o.shape) - o) <= 2.0 ** -8 * (size + np.abs(o))).all(), n
     for copies, window in ((1, 9983), (12, 0), (12, 9900)):
         got = run(copies, window, 32)
         assert all(np.array_equal(x, want) for x in got), (copies, window)

@@ -174,7 +174,14 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
 #pragma unroll
       for (int q = 0; q < PF; q++)
         if (q < np) acc += pf[q] * weight(q);
-      for (int c = PF; c < np; c++) acc += po0[(size_t)part_of(c) * hd] * weight(c);
+      for (int c = PF; c < np; c += 8) {      // eight asked for at a time, added up in part order
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = po0[(size_t)part_of(min(c + q, np - 1)) * hd];
+#pragma unroll
+        for (int q = 0; q < 8; q++)
+          if (c + q < np) acc += v[q] * weight(c + q);
+      }
       orow[threadIdx.x] = (__bf16)(acc * inv);
     }
     return;
