@@ -60,3 +60,15 @@ def test_a_chunk_that_begins_among_the_rows(case, short):
     """The rows in front of it see the whole chunk before: their block has the most keys, not the last one."""
     R, rows, ctx, H, G, D, chunk = case
     assert (form_of(1 << 30, R, rows, ctx, H, G, D, chunk=chunk)[2] == 2) == bool(short)
+
+
+# requests, rows, context, heads, key heads, channels, window: many requests whose keys several blocks fetch, with long contexts and short
+# ones, and one block for all rows of a request
+@pytest.mark.parametrize("case,short", [((16, 16, 1516, 32, 16, 128, 0), 0), ((16, 16, 416, 32, 8, 128, 0), 0), ((8, 33, 233, 32, 16, 128, 0), 0),
+                                        ((8, 17, 417, 64, 8, 128, 300), 0), ((16, 16, 76, 32, 8, 128, 0), 1),
+                                        ((12, 37, 137, 8, 4, 256, 0), 1), ((64, 4, 404, 32, 8, 128, 0), 1), ((1, 150, 650, 32, 16, 128, 0), 1)])
+def test_few_rows_of_many_requests(case, short):
+    """Memory bounds them where blocks of 16 rows fetch a request's keys several times: 16 of 16 rows behind 1,500 keys, 32 heads over
+    16 of 128, took 60.6 us in place of 48.2."""
+    R, rows, ctx, H, G, D, window = case
+    assert (form_of(1 << 30, R, rows, ctx, H, G, D, window=window)[2] == 2) == bool(short)

@@ -364,7 +364,12 @@ static double short_price(int max_q_len, int max_ctx, int window, int mask_chunk
   const double blocks = (double)((max_q_len + tokens - 1) / tokens) * nkv * r_prefill;
   const double alone = wide > 128 ? 3.6 + 2.8 * ((tiles + 3) / 4) : 3.2 + 1.8 * ((tiles + 3) / 4);
   if (blocks <= 256) return alone;
-  return alone * (wide > 128 ? 1.3 * blocks / 256 : 1 + 0.45 * (blocks - 256) / 256);
+  // Blocks of one request and key head lie on up to eight XCDs, each of which fetches their keys and values: 7 TB/s, which many requests of
+  // few rows reach (32 heads over 16 of 128, 16 requests of 16 rows behind 1,500 keys, 48.2 as they are and 60.6; 32 over 8, 16 of 16
+  // behind 400 18.8 and 21.5)
+  const double price = alone * (wide > 128 ? 1.3 * blocks / 256 : 1 + 0.45 * (blocks - 256) / 256), each = (max_q_len + tokens - 1) / tokens;
+  const double mb = std::min(each, 8.0) * nkv * r_prefill * tiles * 32 * wide * 4 / 1e6;
+  return each < 2 ? price : std::max(price, 2 + mb / 7);
 }
 
 // 0: the portion kernel is chosen by the sizes; 1: a group of rows a block; 4, 8: shared
