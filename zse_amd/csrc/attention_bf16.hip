@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
   }
   float m = -INFINITY;
   for (int c = threadIdx.x; c < np; c += 256) m = fmaxf(m, part_ml[(base + part_of(c)) * 2]);
-  m = wave_max(m);
+  m = wave_max_whole(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
@@ -200,7 +200,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
     wgt[c] = w;
     l += part_ml[at + 1] * w;
   }
-  l = block_sum(l, red);
+  l = block_sum_whole(l, red);
   const float inv = gate_factor(gate, gate_ld, row, head) / (l + sink_weight(sinks, sink, head, m));
   if ((int)threadIdx.x < hd) {
     float acc = 0.f;

@@ -72,10 +72,10 @@ __global__ __launch_bounds__(64) void attention_plain_kernel(
       s = dot * scale;
       if (softcap > 0.f) s = softcap * tanhf(s / softcap);
     }
-    const float m_new = fmaxf(m, wave_max(s));
+    const float m_new = fmaxf(m, wave_max_whole(s));
     const float p = valid ? expf(s - m_new) : 0.f;
     const float corr = expf(m - m_new);  // m = -inf on the first tile: exp(-inf) = 0
-    l = l * corr + wave_sum(p);
+    l = l * corr + wave_sum_whole(p);
     m = m_new;
     __syncthreads();
     sp[lane] = p;

@@ -44,7 +44,9 @@ __device__ __forceinline__ void rotate_pair(float a, float b, float sn, float cs
 // step of one decoded token, 2B shapes, 1,786 and 1,722, of eight 2,423 and 2,355; a model of six layers of width 1,024 234 and 222).
 //
 // The permutations do not fetch from lanes that are not there: everything down to the running sums, but for wave_sum, wave_max
-// and block_sum, is for waves whose 64 lanes are all active (blocks of whole waves, outside of conditions on lanes).
+// and block_sum, is for waves whose 64 lanes are all active (blocks of whole waves, outside of conditions on lanes), as this tree's
+// kernels call them: the look at the lanes costs a recurrence that adds up twice a token 2 % (six layers of width 1,024 in 32
+// bits, 253 tokens, 3,346 and 3,427 us a step).
 // Lane l's partner l ^ 32 or l ^ 16: the pair's two values, in some order.
 __device__ __forceinline__ void wave_pair32(float v, float& a, float& b) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -160,14 +162,18 @@ __device__ __forceinline__ float wave_running_max(float v) {
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the result (each wave adds the waves' sums up for
-// itself).  ``scratch`` holds at least 16 floats of LDS that nothing else of the block is reading or writing;
-// block_sum may be called again with the same ones.  block_sum_once: blocks of whole waves.
+// itself).  ``scratch`` holds at least 16 floats of LDS; block_sum and block_sum_whole may be called again with the same ones,
+// block_sum_once with such that nothing else of the block is reading or writing.  The latter two: blocks of whole waves.
 __device__ __forceinline__ float block_sum_once(float v, float* scratch) {
   const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE, nw = blockDim.x / ZSE_WAVE;
   v = wave_sum_whole(v);
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
   return wave_sum16((lane & 15) < nw ? scratch[lane & 15] : 0.f);
+}
+__device__ __forceinline__ float block_sum_whole(float v, float* scratch) {
+  __syncthreads();
+  return block_sum_once(v, scratch);
 }
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
   const int lane = threadIdx.x & (ZSE_WAVE - 1), wave = threadIdx.x / ZSE_WAVE;

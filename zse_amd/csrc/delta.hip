@@ -261,7 +261,7 @@ __global__ __launch_bounds__(PRE > 1 ? 256 : 1024) void delta_rule_kernel(
     for (int tt = wave; tt < n; tt += nw) {        // unit RMS over the head's read-out, gain, gate
       float ss = 0.f;
       for (int c = lane; c < E; c += 64) ss = fmaf(ov[tt * COLS + c], ov[tt * COLS + c], ss);
-      ss = wave_sum(ss);
+      ss = wave_sum_whole(ss);
       const float inv = 1.0f / sqrtf(ss / (float)E + eps);
       const act_t* zr = z + (size_t)(c0 + tt) * ldz + (size_t)h * E;
       act_t* orow = out + ((size_t)(c0 + tt) * H + h) * E;
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64) void delta_finish_kernel(const float* __restric
   }
   float ss = 0.f;
   for (int c = lane; c < E; c += 64) ss = fmaf(rr[c], rr[c], ss);
-  ss = wave_sum(ss);
+  ss = wave_sum_whole(ss);
   const float inv = 1.0f / sqrtf(ss / (float)E + eps);
   const act_t* zr = z + (size_t)t * ldz + (size_t)h * E;
   for (int c = lane; c < E; c += 64) {

@@ -100,10 +100,10 @@ __global__ __launch_bounds__(64) void diff_attention_plain_kernel(
     __syncthreads();
 #pragma unroll
     for (int mp = 0; mp < 2; mp++) {
-      const float m_new = fmaxf(m[mp], wave_max(s[mp]));
+      const float m_new = fmaxf(m[mp], wave_max_whole(s[mp]));
       const float p = valid ? expf(s[mp] - m_new) : 0.f;
       corr[mp] = expf(m[mp] - m_new);
-      l[mp] = l[mp] * corr[mp] + wave_sum(p);
+      l[mp] = l[mp] * corr[mp] + wave_sum_whole(p);
       m[mp] = m_new;
       sp[mp][lane] = p;
     }
@@ -137,7 +137,7 @@ __global__ __launch_bounds__(64) void diff_attention_plain_kernel(
     res[c] = d < E ? acc[0][c] * inv0 - lambda * (acc[1][c] * inv1) : 0.f;
     ss = fmaf(res[c], res[c], ss);
   }
-  ss = wave_sum(ss);
+  ss = wave_sum_whole(ss);
   const float norm = (1.0f - diff) / sqrtf(ss / (float)E + eps);
 #pragma unroll
   for (int c = 0; c < DA_MAX / 64; c++) {
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64) void diff_join_kernel(const act_t* __restrict__
     res[c] = d < E ? to_f32(a1[d]) - lambda * to_f32(a2[d]) : 0.f;
     ss = fmaf(res[c], res[c], ss);
   }
-  ss = wave_sum(ss);
+  ss = wave_sum_whole(ss);
   const float norm = (1.0f - diff) / sqrtf(ss / (float)E + eps);
 #pragma unroll
   for (int c = 0; c < DA_MAX / 64; c++) {

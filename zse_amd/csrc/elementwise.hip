@@ -56,7 +56,7 @@ __global__ void rmsnorm_kernel(const TIn* __restrict__ x, const int* __restrict_
     float v = to_f32(xr[i]);
     ss += v * v;
   }
-  ss = block_sum(ss, red);
+  ss = block_sum_whole(ss, red);
   const float rs = rsqrtf(ss / (float)H + eps);
   act_t* o = out + (size_t)r * H;
   for (int i = threadIdx.x; i < H; i += blockDim.x)
@@ -91,7 +91,7 @@ __global__ void norm_add_norm_kernel(const void* __restrict__ sub, int parts, co
       float v = sub_value(sub, parts, plane, row + i);
       ss += v * v;
     }
-    ss = block_sum(ss, red);
+    ss = block_sum_whole(ss, red);
     rs = rsqrtf(ss / (float)H + eps_post);
   }
   float ss2 = 0.f;
@@ -104,7 +104,7 @@ __global__ void norm_add_norm_kernel(const void* __restrict__ sub, int parts, co
     ss2 += v * v;
   }
   if (!w_next) return;
-  ss2 = block_sum(ss2, red);
+  ss2 = block_sum_whole(ss2, red);
   const float rs2 = rsqrtf(ss2 / (float)H + eps_next);
   act_t* o = out + (size_t)r * H;
   for (int i = threadIdx.x; i < H; i += blockDim.x)  // each thread re-reads what it wrote

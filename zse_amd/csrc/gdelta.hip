@@ -227,7 +227,7 @@ __global__ __launch_bounds__(1024) void gdelta_kernel(const act_t* __restrict__ 
     for (int tt = wave; tt < n; tt += nw) {        // unit RMS over the head's read-out, gain, gate
       float ss = 0.f;
       for (int c = lane; c < D; c += 64) ss = fmaf(ov[tt * COLS + c], ov[tt * COLS + c], ss);
-      ss = wave_sum(ss);
+      ss = wave_sum_whole(ss);
       const float inv = 1.0f / sqrtf(ss / (float)D + eps);
       const act_t* gr = g + (size_t)(c0 + tt) * ldg + (size_t)h * D;
       act_t* orow = out + ((size_t)(c0 + tt) * H + h) * D;
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(64) void gdelta_finish_kernel(const float* __restri
   }
   float ss = 0.f;
   for (int c = lane; c < D; c += 64) ss = fmaf(rr[c], rr[c], ss);
-  ss = wave_sum(ss);
+  ss = wave_sum_whole(ss);
   const float inv = 1.0f / sqrtf(ss / (float)D + eps);
   const act_t* gr = g + (size_t)t * ldg + (size_t)h * D;
   for (int c = lane; c < D; c += 64)
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(1024) void gdelta_token_kernel(const act_t* __restr
     ws[e] = decay[at];
     as[e] = rate[at];
   }
-  const float norm = sqrtf(block_sum(kk * kk, red) + 1e-6f);      // its barriers also make us, rs, ws, as visible
+  const float norm = sqrtf(block_sum_whole(kk * kk, red) + 1e-6f);      // its barriers also make us, rs, ws, as visible
   const float inv = 1.0f / norm;
   float dot = 0.f;
 #pragma unroll
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(1024) void gdelta_token_kernel(const act_t* __restr
   o = 0.f;
   if (p == 0)
     for (int q = 0; q < P; q++) o += part[q * D + e];
-  const float ms = block_sum(p == 0 ? o * o : 0.f, red) / (float)D;
+  const float ms = block_sum_whole(p == 0 ? o * o : 0.f, red) / (float)D;
   if (p == 0)
     orow[e] = from_f32<act_t>(o * (1.0f / sqrtf(ms + eps)) * gain[(size_t)h * D + e] *
                               gd_sigmoid(to_f32(g[(size_t)t * ldg + (size_t)h * D + e])));
@@ -393,7 +393,7 @@ __global__ __launch_bounds__(512) void gdelta_chunk_kernel(const act_t* __restri
         const float x = to_f32(rkv[(size_t)(t0 + t) * ld + k_off + (size_t)h * D + d]);
         ss = fmaf(x, x, ss);
       }
-    ss = wave_sum(ss);
+    ss = wave_sum_whole(ss);
     if (lane == 0) kn[t] = sqrtf(ss + 1e-6f);
   }
   // the four scaled rows: a thread PER tokens of a channel; tokens past the portion's end change nothing (decay 1, rows 0)

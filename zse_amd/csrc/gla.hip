@@ -192,7 +192,7 @@ __global__ __launch_bounds__(1024) void gla_kernel(
     for (int tt = wave; tt < n; tt += nw) {        // unit RMS over the head's read-out, gain, gate
       float ss = 0.f;
       for (int c = lane; c < E; c += 64) ss = fmaf(ov[tt * COLS + c], ov[tt * COLS + c], ss);
-      ss = wave_sum(ss);
+      ss = wave_sum_whole(ss);
       const float inv = 1.0f / sqrtf(ss / (float)E + eps);
       const act_t* gr = g + (size_t)(c0 + tt) * ldg + (size_t)h * E;
       act_t* orow = out + ((size_t)(c0 + tt) * H + h) * E;
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64) void gla_finish_kernel(const float* __restrict_
   }
   float ss = 0.f;
   for (int c = lane; c < E; c += 64) ss = fmaf(rr[c], rr[c], ss);
-  ss = wave_sum(ss);
+  ss = wave_sum_whole(ss);
   const float inv = 1.0f / sqrtf(ss / (float)E + eps);
   const act_t* gr = g + (size_t)t * ldg + (size_t)h * E;
   for (int c = lane; c < E; c += 64) {

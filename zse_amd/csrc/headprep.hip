@@ -57,7 +57,7 @@ __global__ __launch_bounds__(64) void head_prep_kernel(
   }
   const float* gain = kind == 0 ? q_gain : kind == 1 ? k_gain : nullptr;
   if (gain != nullptr) {
-    sum = wave_sum(sum);
+    sum = wave_sum_whole(sum);
     const float inv = 1.0f / sqrtf(sum / (float)size + eps);
     const float c = (kind == 0 && head_scale) ? head_scale[head] : 1.f;
     for (int d = lane; d < size; d += 64) buf[d] = buf[d] * inv * gain[d] * c;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(64) void head_prep_kernel(
     // queries and keys divided by their root mean square over the head, after the rotation, no gain
     float ss = 0.f;
     for (int d = lane; d < size; d += 64) ss = fmaf(buf[d], buf[d], ss);
-    ss = wave_sum(ss);
+    ss = wave_sum_whole(ss);
     const float inv = 1.0f / sqrtf(ss / (float)size + eps);
     for (int d = lane; d < size; d += 64) buf[d] *= inv;
   }
@@ -202,8 +202,8 @@ __global__ __launch_bounds__(1024) void row_prep_kernel(
     if (i < nq) sq = fmaf(x, x, sq);
     else sk = fmaf(x, x, sk);
   }
-  sq = block_sum(sq, red);
-  sk = block_sum(sk, red);
+  sq = block_sum_whole(sq, red);
+  sk = block_sum_whole(sk, red);
   const int slot = slot_map ? slot_map[t] : -1;
   const size_t page = slot >= 0 ? slot / bs : 0, off = slot >= 0 ? slot % bs : 0;
   if (slot >= 0) {

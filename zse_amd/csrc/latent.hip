@@ -51,7 +51,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(
     const float x = to_f32(src[i]);
     ss = fmaf(x, x, ss);
   }
-  ss = block_sum(ss, red);
+  ss = block_sum_whole(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)C + eps);
   for (int i = tid; i < C; i += 256) dst[i] = from_f32<act_t>(to_f32(src[i]) * inv * gain[i]);
   for (int m = tid; m < half; m += 256) {
@@ -418,9 +418,9 @@ __global__ __launch_bounds__(256) void latent_join_kernel(const float* __restric
     const float ms = s < splits ? pr[(size_t)s * (CP + 2)] : -INFINITY;
     const float ls = s < splits ? pr[(size_t)s * (CP + 2) + 1] : 0.f;
     const float sk = sinks ? sinks[row % H] : -INFINITY;
-    const float M = fmaxf(wave_max(ms), sk);
+    const float M = fmaxf(wave_max_whole(ms), sk);
     const float w = ms > -INFINITY ? __expf(ms - M) : 0.f;
-    const float den = wave_sum(ls * w) + (sinks ? __expf(sk - M) : 0.f);
+    const float den = wave_sum_whole(ls * w) + (sinks ? __expf(sk - M) : 0.f);
     wgt[s] = w;
     if (s == 0) inv_den = 1.f / den;
   }

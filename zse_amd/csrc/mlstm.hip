@@ -104,14 +104,14 @@ __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_kernel(
       n[d] = v;
       nq = fmaf(v, sq[d], nq);
     }
-    nq = block_sum(nq, red);              // syncs: part[] is complete after it
+    nq = block_sum_whole(nq, red);              // syncs: part[] is complete after it
     const float den = fmaxf(fabsf(nq), expf(-m)) + 1e-6f;
     float o = 0.f;
     if (tid < E) {
       for (int s2 = 0; s2 < slices; s2++) o += part[s2 * E + tid];
       o = o / den;
     }
-    const float ms = block_sum(tid < E ? o * o : 0.f, red) / (float)E;
+    const float ms = block_sum_whole(tid < E ? o * o : 0.f, red) / (float)E;
     if (tid < E) {
       const size_t col = (size_t)hd * E + tid;
       const float z = to_f32(row[(size_t)2 * H * D + (size_t)H * E + col]);
@@ -386,7 +386,7 @@ __global__ __launch_bounds__(64) void mlstm_finish_kernel(
   const float* o = o_raw + ((size_t)t * H + hd) * E;
   float ss = 0.f;
   for (int e = lane; e < E; e += 64) ss = fmaf(o[e], o[e], ss);
-  const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)E + eps);
+  const float inv = 1.0f / sqrtf(wave_sum_whole(ss) / (float)E + eps);
   const act_t* z = qkvz + (size_t)t * ld + (size_t)2 * H * D + (size_t)H * E + (size_t)hd * E;
   for (int e = lane; e < E; e += 64) {
     const float y = o[e] * inv * norm_w[(size_t)hd * E + e] * (1.0f / (1.0f + expf(-to_f32(z[e]))));
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(MLSTM_THREADS) void mlstm_local_kernel(
     if (wave == 0) {
       float a, F;
       mlstm_gates(gate, Lc, cap, lane, a, F);
-      const float A = wave_max(a);
+      const float A = wave_max_whole(a);
       if (lane < L) gw[lane] = lane < Lc ? expf(a - A) : 0.f;
       if (lane == Lc - 1 && blockIdx.z == 0) {
         af[((size_t)x * H + hd) * 2] = A;

@@ -60,7 +60,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       s[i] = e < E ? logits[(size_t)t * ld + e] : -INFINITY;
       mx = fmaxf(mx, s[i]);
     }
-    mx = wave_max(mx);
+    mx = wave_max_whole(mx);
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < MOE_MAX_EXPERTS / 64; i++) {
@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
       s[i] = e < E ? expf(s[i] - mx) : 0.f;
       sum += s[i];
     }
-    sum = wave_sum(sum);
+    sum = wave_sum_whole(sum);
 #pragma unroll
     for (int i = 0; i < MOE_MAX_EXPERTS / 64; i++) s[i] = (lane + 64 * i) < E ? s[i] / sum : -1.f;
   } else {
@@ -125,10 +125,10 @@ __global__ __launch_bounds__(64) void moe_route_groups_kernel(const float* __res
   if (softmax) {
     mx = -INFINITY;
     for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
-    mx = wave_max(mx);
+    mx = wave_max_whole(mx);
     sum = 0.f;
     for (int e = lane; e < E; e += 64) sum += expf(z[e] - mx);
-    sum = wave_sum(sum);
+    sum = wave_sum_whole(sum);
   }
   for (int e = lane; e < E; e += 64) {
     const float s = softmax ? expf(z[e] - mx) / sum : 1.0f / (1.0f + expf(-z[e]));

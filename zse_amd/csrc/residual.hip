@@ -38,7 +38,7 @@ __global__ void sum_norm_kernel(float* __restrict__ h, const void* __restrict__ 
     ss = fmaf(v, v, ss);
   }
   if (!w_next) return;
-  ss = block_sum(ss, red);
+  ss = block_sum_whole(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)W + eps);
   for (int i = threadIdx.x; i < W; i += blockDim.x)      // each thread re-reads what it wrote
     out[row + i] = from_f32<act_t>(hr[i] * inv * (unit_offset ? 1.0f + w_next[i] : w_next[i]));
@@ -66,13 +66,13 @@ __global__ void sum_layer_norm_kernel(float* __restrict__ h, const void* __restr
     s += v;
   }
   if (!w_next) return;
-  const float mean = block_sum(s, red) / (float)W;
+  const float mean = block_sum_whole(s, red) / (float)W;
   float ss = 0.f;
   for (int i = threadIdx.x; i < W; i += blockDim.x) {      // each thread re-reads what it wrote
     const float d = hr[i] - mean;
     ss = fmaf(d, d, ss);
   }
-  ss = block_sum(ss, red);
+  ss = block_sum_whole(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)W + eps);
   for (int i = threadIdx.x; i < W; i += blockDim.x)
     out[row + i] = from_f32<act_t>((hr[i] - mean) * inv * w_next[i] + (c_next ? c_next[i] : 0.f));
@@ -101,7 +101,7 @@ __global__ void sum_norm_pair_kernel(float* __restrict__ h, const void* __restri
     ss = fmaf(v, v, ss);
   }
   if (!w1 && !w2) return;
-  ss = block_sum(ss, red);
+  ss = block_sum_whole(ss, red);
   const float inv = 1.0f / sqrtf(ss / (float)W + eps);
   for (int i = threadIdx.x; i < W; i += blockDim.x) {      // each thread re-reads what it wrote
     const float x = hr[i] * inv;

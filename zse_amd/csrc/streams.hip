@@ -232,13 +232,13 @@ __global__ __launch_bounds__(1024) void streams_step_kernel(
     }
   }
   if (out == nullptr) return;
-  const float mean = block_sum(sum, scratch) / (float)W;
+  const float mean = block_sum_whole(sum, scratch) / (float)W;
   float dev = 0.f;
   for (int c = tid; c < W; c += nt) {
     const float d = u_row[c] - mean;
     dev = fmaf(d, d, dev);
   }
-  const float var = block_sum(dev, scratch) / (float)W;
+  const float var = block_sum_whole(dev, scratch) / (float)W;
   const float inv = 1.0f / sqrtf(var + eps);
   act_t* o = out + (size_t)b * W;
   for (int c = tid; c < W; c += nt) o[c] = from_f32<act_t>(fmaf((u_row[c] - mean) * inv, norm_w[c], norm_b ? norm_b[c] : 0.f));

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(1024) void sublayer_step_kernel(float* __restrict__
       for (int e = 0; e < V; e++) ss = fmaf(v[e], v[e], ss);
       put_floats<V>(row + c, v);
     }
-    inv_y = 1.0f / sqrtf(block_sum(ss, red) / (float)W + y_eps);
+    inv_y = 1.0f / sqrtf(block_sum_whole(ss, red) / (float)W + y_eps);
   }
   float sum = 0.f;
   for (int c = tid * V; c < W; c += nt * V) {
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(1024) void sublayer_step_kernel(float* __restrict__
     }
   }
   if (out == nullptr) return;
-  const float mean = block_sum(sum, red) / (float)W;
+  const float mean = block_sum_whole(sum, red) / (float)W;
   float dev = 0.f;
   for (int c = tid * V; c < W; c += nt * V) {
     float x[V];
@@ -155,7 +155,7 @@ __global__ __launch_bounds__(1024) void sublayer_step_kernel(float* __restrict__
       dev = fmaf(d, d, dev);
     }
   }
-  const float inv = 1.0f / sqrtf(block_sum(dev, red) / (float)W + eps);
+  const float inv = 1.0f / sqrtf(block_sum_whole(dev, red) / (float)W + eps);
   const bool conv = cv.w != nullptr;
   const bool padding = conv && cv.positions[t] < 0;          // a padding row of a captured step
   float* st = (conv && !padding && cv.taps > 1)
@@ -337,13 +337,13 @@ __global__ __launch_bounds__(1024) void norm_stream_kernel(float* __restrict__ h
   float* hr = h + (size_t)blockIdx.x * W;
   float sum = 0.f;
   for (int c = threadIdx.x; c < W; c += blockDim.x) sum += hr[c];
-  const float mean = block_sum(sum, red) / (float)W;
+  const float mean = block_sum_whole(sum, red) / (float)W;
   float dev = 0.f;
   for (int c = threadIdx.x; c < W; c += blockDim.x) {
     const float d = hr[c] - mean;
     dev = fmaf(d, d, dev);
   }
-  const float inv = 1.0f / sqrtf(block_sum(dev, red) / (float)W + eps);
+  const float inv = 1.0f / sqrtf(block_sum_whole(dev, red) / (float)W + eps);
   for (int c = threadIdx.x; c < W; c += blockDim.x) hr[c] = fmaf((hr[c] - mean) * inv, w[c], b ? b[c] : 0.f);
 }
 
