@@ -370,11 +370,15 @@ MANY = [(7 * r) % 23 if r % 5 else 0 for r in range(66)] + [40, 0, 1, 9, 8, 17] 
 
 
 # Alike rows (a block a run and request), and one long portion among single rows (runs numbered through all requests, full
-# and one of a single row); channels in eights and one at a time
-@pytest.mark.parametrize("lens,by_piece", [(MANY, 0), ([0, 1, 393] + [1, 0, 2] * 24, 1)])
-@pytest.mark.parametrize("C,taps", [(16, 4), (264, 3), (13, 4)])
+# and one of a single row); channels in eights and one at a time, rows asked for in front and (more than 2^21 values) one after the other
+LONG = [0, 1, 393] + [1, 0, 2] * 24
+
+
+@pytest.mark.parametrize("lens,by_piece,C,taps", [(lens, by_piece, C, taps) for lens, by_piece in ((MANY, 0), (LONG, 1))
+                                                  for C, taps in ((16, 4), (264, 3), (13, 4), (16, 2))] +
+                         [(LONG, 1, 6152, 4), ([211, 214], 0, 6152, 4)])
 def test_short_convolution_of_many_requests(dev, lens, by_piece, C, taps):
-    """More requests than a wave adds up at once, of no, one and several runs of rows; padding behind the last."""
+    """Mostly more requests than a wave adds up at once, of no, one and several runs of rows; padding behind the last."""
     rt, k = dev
     rng = np.random.default_rng(3)
     R, T = len(lens), sum(lens)

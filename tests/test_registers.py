@@ -29,7 +29,7 @@ def scratch(request, tmp_path_factory):
 
 
 # a kernel, the number of its forms, those of them that may go through scratch memory
-@pytest.mark.parametrize("kernel,forms,but", [("streams_row_kernel", 7, "ILi4ELi4ELi1024E"), ("conv_rows_kernel", 10, None),
+@pytest.mark.parametrize("kernel,forms,but", [("streams_row_kernel", 7, "ILi4ELi4ELi1024E"), ("conv_rows_kernel", 16, None),
                                               ("rope_cache_write_token_kernel", 3, None), ("mlstm_output_kernel", 6, None),
                                               ("mlstm_local_kernel", 6, None), ("attention_f32_kernel", 8, None)])
 def test_no_scratch_memory(scratch, kernel, forms, but):

@@ -15,8 +15,12 @@
 // A block works on one run.  As a rule block (y, z) is run y of request z; where more than half of many such blocks would
 // find no run, the runs are numbered through all requests and a block looks for its own (us, the one way and the other: 700
 // rows and 8 single ones of 2,048 channels 10.2 and 9.0, 2,000 and 500 single ones of 256 55.8 and 10.0; 2,048 rows of 2,048
-// 10.2 and 10.5, 1,000 requests of nine rows of 256 16.7 and 21.4).  A run's rows are read one after the other: all asked for
-// in front, also where a run is short, 2,048 rows of 2,048 take 12.9 and 8 single ones 3.6 in place of 3.4.
+// 10.2 and 10.5, 1,000 requests of nine rows of 256 16.7 and 21.4).
+//
+// Up to 2 million values the time is the launch and a chain of waits, so a run's rows are all asked for before the first is used (us,
+// one after the other and so, taps of 4: 8 rows of 2,048 channels 5.4 and 4.6, 700 and 8 single ones 6.5 and 5.6, 60 requests of 20 rows
+// of 1,024 6.3 and 5.6); with more values, or of rows that are nearly alone, one after the other (2,048 rows of 2,048, in 32 bits, 9.3 and 10.1, 200 single
+// rows of 8,192 12.6 and 15.4, one 2.9 and 2.9).
 #include "common.h"
 #include "packed_call.h"
 
@@ -27,21 +31,23 @@ extern "C" int zk_steplist_register(const char* name, int nargs, void* fn);
 #define CONV_SPAN 8
 #define CONV_MOST_TAPS (CONV_SPAN + 1)
 
+// V channels of a row as they lie in memory, and their values
+template <int V>
+struct ConvRaw {
+  act_t v[V] __attribute__((aligned(sizeof(act_t) * V > 16 ? 16 : sizeof(act_t) * V)));
+};
+template <int V>
+__device__ __forceinline__ ConvRaw<V> conv_raw(const act_t* p) {
+  return *(const ConvRaw<V>*)p;
+}
+template <int V>
+__device__ __forceinline__ void conv_values(const ConvRaw<V>& r, float (&v)[V]) {
+#pragma unroll
+  for (int e = 0; e < V; e++) v[e] = to_f32(r.v[e]);
+}
 template <int V>
 __device__ __forceinline__ void conv_get(const act_t* p, float (&v)[V]) {
-  if constexpr (V == 8) {
-#if ZSE_ACT_BF16
-    typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-    const b8 q = *(const b8*)p;
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (float)q[e];
-#else
-    const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-#endif
-  } else {
-    v[0] = to_f32(p[0]);
-  }
+  conv_values<V>(conv_raw<V>(p), v);
 }
 template <int V>
 __device__ __forceinline__ void conv_put(act_t* p, const float (&v)[V]) {
@@ -80,8 +86,8 @@ __device__ __forceinline__ void conv_put_state(float* p, const float (&v)[V]) {
 }
 
 // TAPS: the number of taps where the launch knows it at compile time, 0: ``taps`` (up to 9).  PIECES: runs are numbered through all
-// requests, ``columns`` blocks next to each other for each
-template <int V, int TAPS, bool PIECES>
+// requests, ``columns`` blocks next to each other for each.  AHEAD: a run's rows are all asked for before the first is used
+template <int V, int TAPS, bool PIECES, bool AHEAD>
 __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict__ x, int ld_in,
                                                         const float* __restrict__ in_bias, const float* __restrict__ w,
                                                         const float* __restrict__ bias, float* __restrict__ state,
@@ -133,6 +139,11 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
 #pragma unroll
     for (int e = 0; e < V; e++) v[e] += ib[e];
   };
+  ConvRaw<V> rows[AHEAD ? CONV_SPAN : 1];      // (a row past the last: the last again)
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int i = 0; i < CONV_SPAN; i++) rows[i] = conv_raw<V>(x + (size_t)(t0 + min(first + i, last - 1)) * ld_in + c);
+  }
   float* st = taps > 1 ? state + (size_t)slot_of_req[r] * slot_words + offset_words + c : nullptr;
   // back[b]: the row b + 1 places before the current token
   float back[BACK][V];
@@ -164,42 +175,55 @@ __global__ __launch_bounds__(256) void conv_rows_kernel(const act_t* __restrict_
         conv_put_state<V>(st + (size_t)a * C, v);
       }
   }
-  for (int i = first; i < last; i++) {
-    float cur[V], acc[V];
-    input(i, cur);
+  constexpr int TURN = AHEAD ? CONV_SPAN : 1;
+  for (int turn = first; turn < last; turn += TURN) {
 #pragma unroll
-    for (int e = 0; e < V; e++) acc[e] = b0[e];
+    for (int k = 0; k < TURN; k++) {
+      const int i = turn + k;
+      if (i >= last) break;
+      float cur[V];
+      if constexpr (AHEAD) {
+        conv_values<V>(rows[k], cur);
 #pragma unroll
-    for (int b = BACK - 1; b >= 0; b--)
-      if (b < taps - 1) {
-#pragma unroll
-        for (int e = 0; e < V; e++) {
-          float wj = 0.f;
-          if (TAPS) {
-            wj = wt[MOST - 2 - b < 0 ? 0 : MOST - 2 - b][e];
-          } else {
-#pragma unroll
-            for (int j = 0; j < MOST; j++) wj = j == taps - 2 - b ? wt[j][e] : wj;
-          }
-          acc[e] = fmaf(wj, back[b][e], acc[e]);
-        }
+        for (int e = 0; e < V; e++) cur[e] += ib[e];
+      } else {
+        input(i, cur);
       }
+      float acc[V];
 #pragma unroll
-    for (int e = 0; e < V; e++) {
-      float wj = wt[0][e];
+      for (int e = 0; e < V; e++) acc[e] = b0[e];
 #pragma unroll
-      for (int j = 0; j < MOST; j++) wj = j == taps - 1 ? wt[j][e] : wj;
-      acc[e] = fmaf(wj, cur[e], acc[e]);
-      if (residual) acc[e] = cur[e] + acc[e];
-      if (act == 1) acc[e] = acc[e] / (1.0f + expf(-acc[e]));      // silu
+      for (int b = BACK - 1; b >= 0; b--)
+        if (b < taps - 1) {
+#pragma unroll
+          for (int e = 0; e < V; e++) {
+            float wj = 0.f;
+            if (TAPS) {
+              wj = wt[MOST - 2 - b < 0 ? 0 : MOST - 2 - b][e];
+            } else {
+#pragma unroll
+              for (int j = 0; j < MOST; j++) wj = j == taps - 2 - b ? wt[j][e] : wj;
+            }
+            acc[e] = fmaf(wj, back[b][e], acc[e]);
+          }
+        }
+#pragma unroll
+      for (int e = 0; e < V; e++) {
+        float wj = wt[0][e];
+#pragma unroll
+        for (int j = 0; j < MOST; j++) wj = j == taps - 1 ? wt[j][e] : wj;
+        acc[e] = fmaf(wj, cur[e], acc[e]);
+        if (residual) acc[e] = cur[e] + acc[e];
+        if (act == 1) acc[e] = acc[e] / (1.0f + expf(-acc[e]));      // silu
+      }
+      conv_put<V>(out + (size_t)(t0 + i) * ld_out + c, acc);
+#pragma unroll
+      for (int b = BACK - 1; b > 0; b--)
+#pragma unroll
+        for (int e = 0; e < V; e++) back[b][e] = back[b - 1][e];
+#pragma unroll
+      for (int e = 0; e < V; e++) back[0][e] = cur[e];
     }
-    conv_put<V>(out + (size_t)(t0 + i) * ld_out + c, acc);
-#pragma unroll
-    for (int b = BACK - 1; b > 0; b--)
-#pragma unroll
-      for (int e = 0; e < V; e++) back[b][e] = back[b - 1][e];
-#pragma unroll
-    for (int e = 0; e < V; e++) back[0][e] = cur[e];
   }
 }
 
@@ -260,23 +284,26 @@ int zk_conv_rows(const void* x, int ld_in, const float* in_bias, const float* w,
   const int per = vec ? 8 : 1;
   const ConvGrid g = conv_grid(T, R, max_q_len, (C + per - 1) / per);
   const dim3 grid = g.by_piece ? dim3((unsigned)(g.columns * g.runs)) : dim3(g.columns, g.runs, R + 1);
-#define LAUNCH_(V, N, PIECES)                                                                                         \
-  conv_rows_kernel<V, N, PIECES><<<grid, g.threads, 0, (hipStream_t)stream>>>(                                        \
+  const bool ahead = max_q_len >= 4 && (long long)T * C <= 1 << 21;      // (see the top)
+#define LAUNCH_(V, N, PIECES, AHEAD)                                                                                  \
+  conv_rows_kernel<V, N, PIECES, AHEAD><<<grid, g.threads, 0, (hipStream_t)stream>>>(                                 \
       (const act_t*)x, ld_in, in_bias, w, bias, state, slot_words, offset_words, q_start, slot_of_req, (act_t*)out, ld_out, T, R, C, \
       taps, residual, act, g.columns)
-#define LAUNCH(V, N)                              \
-  do {                                            \
-    if (g.by_piece) LAUNCH_(V, N, true);          \
-    else LAUNCH_(V, N, false);                    \
+#define LAUNCH(V, N, AHEAD)                              \
+  do {                                                   \
+    if (g.by_piece) LAUNCH_(V, N, true, AHEAD);          \
+    else LAUNCH_(V, N, false, AHEAD);                    \
   } while (0)
+#define LAUNCH_AHEAD(N) do { if (ahead) LAUNCH(8, N, true); else LAUNCH(8, N, false); } while (0)
   if (vec) {
-    if (taps == 2) LAUNCH(8, 2);
-    else if (taps == 3) LAUNCH(8, 3);
-    else if (taps == 4) LAUNCH(8, 4);
-    else LAUNCH(8, 0);
+    if (taps == 2) LAUNCH_AHEAD(2);
+    else if (taps == 3) LAUNCH_AHEAD(3);
+    else if (taps == 4) LAUNCH_AHEAD(4);
+    else LAUNCH(8, 0, false);
   } else {
-    LAUNCH(1, 0);
+    LAUNCH(1, 0, false);
   }
+#undef LAUNCH_AHEAD
 #undef LAUNCH
 #undef LAUNCH_
   return zk_launch_status("zk_conv_rows");
