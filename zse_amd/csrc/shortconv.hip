@@ -17,10 +17,10 @@
 // rows and 8 single ones of 2,048 channels 10.2 and 9.0, 2,000 and 500 single ones of 256 55.8 and 10.0; 2,048 rows of 2,048
 // 10.2 and 10.5, 1,000 requests of nine rows of 256 16.7 and 21.4).
 //
-// Up to 2 million values the time is the launch and a chain of waits, so a run's rows are all asked for before the first is used (us,
-// one after the other and so, taps of 4: 8 rows of 2,048 channels 5.4 and 4.6, 700 and 8 single ones 6.5 and 5.6, 60 requests of 20 rows
-// of 1,024 6.3 and 5.6); with more values, or of rows that are nearly alone, one after the other (2,048 rows of 2,048, in 32 bits, 9.3 and 10.1, 200 single
-// rows of 8,192 12.6 and 15.4, one 2.9 and 2.9).
+// Up to 2 million values (3 of 16 bits) the time is the launch and a chain of waits, so a run's rows are all asked for before the
+// first is used (us, one after the other and so, taps of 4: 8 rows of 2,048 channels 5.4 and 4.6, 700 and 8 single ones 6.5 and
+// 5.6, 60 requests of 20 rows of 1,024 6.3 and 5.6; in 16 bits 700 and 8 of 4,096 6.9 and 6.3); with more values, or of rows that
+// are nearly alone, one after the other (2,048 rows of 2,048 in 32 bits 9.3 and 10.1, 200 single rows of 8,192 12.6 and 15.4).
 #include "common.h"
 #include "packed_call.h"
 
@@ -284,7 +284,7 @@ int zk_conv_rows(const void* x, int ld_in, const float* in_bias, const float* w,
   const int per = vec ? 8 : 1;
   const ConvGrid g = conv_grid(T, R, max_q_len, (C + per - 1) / per);
   const dim3 grid = g.by_piece ? dim3((unsigned)(g.columns * g.runs)) : dim3(g.columns, g.runs, R + 1);
-  const bool ahead = max_q_len >= 4 && (long long)T * C <= 1 << 21;      // (see the top)
+  const bool ahead = max_q_len >= 4 && (long long)T * C <= (ZSE_ACT_BF16 ? 3 << 20 : 2 << 20);      // (see the top)
 #define LAUNCH_(V, N, PIECES, AHEAD)                                                                                  \
   conv_rows_kernel<V, N, PIECES, AHEAD><<<grid, g.threads, 0, (hipStream_t)stream>>>(                                 \
       (const act_t*)x, ld_in, in_bias, w, bias, state, slot_words, offset_words, q_start, slot_of_req, (act_t*)out, ld_out, T, R, C, \
