@@ -136,7 +136,7 @@ def test_attention_of_few_and_many_blocks_and_with_a_window_that_shows_all(nh, n
                                                (2100, 2, 1, 128, 16, 0)])
 def test_rotation_and_store_of_many_tokens(dtype, T, nh, nkv, hd, bs, vt):
     from test_gpu_kernels import test_rope_and_cache_write
-    assert dev()[1]._dll.zk_rope_by_token(T, nh, nkv, hd, hd, vt)
+    assert dev()[1]._dll.zk_rope_by_token(T, nh, nkv, hd, hd, vt, 0)
     test_rope_and_cache_write(dev()[0], dtype, T, nh, nkv, hd, hd, bs, vt)
 
 

@@ -861,8 +861,8 @@ def test_qkv_product_that_rotates_and_stores(rt, M, K, nh, nkv, hd, bs, vt, stri
                                                  (100, 4, 2, 32, 8, 0, 32), (23, 2, 1, 64, 4, 0, 32), (72, 3, 3, 16, 8, 1, 16),
                                                  # a block a token: more and fewer of them than the chip takes at once, value channels
                                                  # that a block goes through in several turns, pages of fewer than eight, rows
-                                                 (305, 8, 4, 256, 16, 1, 256), (2051, 4, 2, 32, 8, 1, 32), (107, 2, 20, 256, 8, 1, 256),
-                                                 (2052, 4, 2, 32, 4, 1, 32), (520, 3, 2, 96, 16, 0, 96)])
+                                                 (921, 8, 4, 256, 16, 1, 256), (2051, 8, 2, 32, 8, 1, 32), (427, 2, 20, 256, 8, 1, 256),
+                                                 (2052, 8, 2, 32, 4, 1, 32), (584, 3, 2, 96, 16, 0, 96)])
 def test_rotation_that_adds_up_partial_sums_itself(rt, dtype, T, nh, nkv, hd, bs, vt, rot):
     """The rows of [q | k | v] as three planes of float partial sums, added up by the kernel that
     rotates and stores: the same bits, in q and in the cache, as from the rows added up in order and
@@ -881,7 +881,7 @@ def test_rotation_that_adds_up_partial_sums_itself(rt, dtype, T, nh, nkv, hd, bs
     if T >= 16 and bs >= 8:
         slots[8:16] = 2 * bs + np.arange(8)
     if T > 100:
-        assert k._dll.zk_rope_by_token(T, nh, nkv, hd, rot, vt)
+        assert k._dll.zk_rope_by_token(T, nh, nkv, hd, rot, vt, 3)
         for t in range(32, T // 8 * 8 if bs >= 8 else 0, 16):      # slots of pages behind the scattered ones
             slots[t:t + 8] = pages * bs + (t - 32) // 2 + np.arange(8)
         pages += (T // 2 + bs - 1) // bs + 1

@@ -18,17 +18,21 @@ def test_runs_of_the_short_convolution(T, R, longest, channels, by_piece):
     assert library().zk_conv_rows_by_piece(T, R, longest, channels, 8) == by_piece
 
 
-# tokens, heads, key heads, channels of a head, values transposed: few blocks per (token, head) stay such blocks, whatever the size of a head
-@pytest.mark.parametrize("T,nh,nkv,hd,transposed,by_token", [
-    (64, 8, 4, 256, 1, 0), (200, 8, 4, 256, 1, 0), (400, 8, 4, 256, 1, 1), (100, 32, 16, 128, 1, 0), (200, 32, 16, 128, 1, 1),
-    (400, 8, 2, 64, 1, 0), (200, 64, 8, 64, 1, 1), (400, 64, 8, 32, 1, 1), (800, 16, 4, 16, 1, 1), (2048, 16, 4, 16, 1, 1),
-    (64, 8, 4, 256, 0, 0), (400, 8, 4, 256, 0, 1), (400, 16, 4, 16, 0, 1), (2048, 4, 2, 16, 0, 1), (1500, 6, 1, 32, 0, 1)])
-@pytest.mark.parametrize("name", ["kernels_bf16", "kernels_f32"])
-def test_rotation_by_token(name, T, nh, nkv, hd, transposed, by_token):
-    """2,048 tokens of 16 heads and 2 x 4 of 16 channels took 13.9 us per (token, head) and 7.2 by token, in rows of 32 bits 14.0 and 4.5."""
-    lib = library(name)
-    assert lib.zk_rope_by_token(T, nh, nkv, hd, hd, transposed) == by_token
-    assert lib.zk_rope_by_token(T, nh, nkv, hd, hd // 2, transposed) == 0      # a part of the head turned: per head
+# tokens, heads, key heads, channels of a head, values transposed, planes of partial sums; by token in 16 and in 32 bits
+@pytest.mark.parametrize("T,nh,nkv,hd,transposed,sums,by_token", [
+    (64, 8, 4, 256, 1, 0, (0, 0)), (140, 8, 4, 256, 1, 0, (0, 0)), (200, 8, 4, 256, 1, 0, (0, 1)), (400, 8, 4, 256, 1, 0, (1, 1)),
+    (100, 32, 16, 128, 1, 0, (0, 1)), (200, 32, 16, 128, 1, 0, (1, 1)), (200, 16, 4, 64, 1, 0, (0, 0)), (400, 16, 4, 64, 1, 0, (1, 1)),
+    (400, 8, 2, 64, 1, 0, (0, 0)), (200, 64, 8, 64, 1, 0, (1, 1)), (400, 64, 8, 32, 1, 0, (1, 1)), (2048, 16, 4, 16, 1, 0, (1, 1)),
+    (400, 8, 4, 256, 1, 3, (0, 0)), (1200, 8, 4, 256, 1, 3, (1, 1)), (140, 64, 8, 64, 1, 3, (0, 0)), (400, 64, 8, 64, 1, 3, (1, 1)),
+    (64, 32, 16, 128, 0, 0, (0, 0)), (200, 32, 16, 128, 0, 0, (1, 1)), (140, 8, 4, 256, 0, 0, (0, 0)), (400, 8, 4, 256, 0, 3, (1, 1)),
+    (100, 16, 4, 16, 0, 0, (0, 0)), (400, 16, 4, 16, 0, 0, (1, 1)), (2048, 4, 2, 16, 0, 0, (1, 1))])
+def test_rotation_by_token(T, nh, nkv, hd, transposed, sums, by_token):
+    """64 tokens of 32 heads and 2 x 16 of 128 with values in rows take 3.5 us per (token, head) and 4.6 by token, 2,048 of 16 and
+    2 x 4 of 16, transposed, 13.9 and 7.2."""
+    for name, want in zip(("kernels_bf16", "kernels_f32"), by_token):
+        lib = library(name)
+        assert lib.zk_rope_by_token(T, nh, nkv, hd, hd, transposed, sums) == want, name
+        assert lib.zk_rope_by_token(T, nh, nkv, hd, hd // 2, transposed, sums) == 0      # a part of the head turned: per head
 
 
 @pytest.mark.parametrize("D,tokens", [(64, 64), (128, 64), (192, 64), (200, 32), (224, 32), (256, 32)])

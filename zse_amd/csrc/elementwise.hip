@@ -943,19 +943,23 @@ int zk_softcap(float* z, size_t n, float cap, void* stream) {
 }
 
 // A block a token, or a block per (token, head), which is quicker while these are few: its time goes with the number of its
-// blocks, and a block's with the size of a head (0.24 ns up to 64 channels, 0.33 for 128, 0.5 for 256), so the line is drawn by
-// blocks times channels and 64 more.  us, per head and by token: values transposed, 16 heads and 2 x 4 of 16, 400 tokens 4.6 and 4.3,
-// 2,048 13.9 and 7.2; 64 and 2 x 8 of 64, 100 4.4 and 4.9, 200 6.4 and 4.9; 8 and 2 x 4 of 256, 200 4.5 and 4.7, 400 6.4
-// and 5.1; as three planes of sums 64 and 2 x 8 of 64, 100 5.0 and 7.5, 200 8.1 and 7.9.  Values in rows (their kernel waits less):
-// 16 and 2 x 4 of 16, 200 3.6 and 3.3; 8 and 2 x 4 of 256, 200 4.0 and 4.1, 400 4.9 and 4.4.
-static bool rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed) {
-  const long long weight = (long long)T * (nh + 2 * nkv) * (std::max(hd, 64) + 64);
-  return weight > (v_transposed ? 5 << 18 : 1 << 19) && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF;
+// blocks, and a block's with the size of a head; a token's block waits for one turn after the other of 2,048 channels of q and k,
+// and adds planes of partial sums up for eight tokens' values by itself.  Both were measured for 15 kinds of heads, 8 to 2,048 tokens, in 16
+// and 32 bits; the line loses 0.1 % of the better's time on average (one by blocks times channels 1.3 %, at most 58).  us, per head and by
+// token: values transposed, 16 heads and 2 x 4 of 64, 200 tokens 3.8 and 4.2, 400 5.0 and 4.5; 8 and 2 x 4 of 256, 200 4.6 and 4.6, 400
+// 6.4 and 5.0, in 32 bits 200 5.6 and 4.6; as three planes of sums 560 10.4 and 11.6.  Values in rows: 32 and 2 x 16 of 128, 64 3.5 and 4.6,
+// 140 4.8 and 4.8; 16 and 2 x 4 of 16, 200 3.5 and 3.3.
+static bool rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed, int sums) {
+  const double blocks = T * (nh + 2.0 * nkv) * 1e-3, turns = (double)(((long long)(nh + nkv) * hd + 2047) / 2048);
+  const bool few = !v_transposed ? blocks * (0.25 + 0.0008 * hd) <= 0.2 + turns
+                   : sums > 0    ? blocks * (0.15 + 0.0004 * hd) <= 2.4 + 0.6 * turns
+                                 : blocks * (0.25 + 0.002 * hd) * (ZSE_ACT_BF16 ? 1.0 : 1.5) <= 2.4 + 0.45 * turns;
+  return !few && rotary_dim == hd && hd % 8 == 0 && hd / 2 <= ROPE_MAX_HALF;
 }
 
 // 1 if the rotation of these rows goes by blocks of a token.  For tests that mean to reach both kernels.
-int zk_rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed) {
-  return rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed);
+int zk_rope_by_token(int T, int nh, int nkv, int hd, int rotary_dim, int v_transposed, int sums) {
+  return rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed, sums);
 }
 
 // sums > 0: the rows are not in qkv yet but come as that many planes of [T, (nh + 2 nkv) hd] float
@@ -971,7 +975,7 @@ int zk_rope_cache_write_sums(void* qkv, const float* planes, int sums, const int
   ZK_REQUIRE(sums == 0 || (planes != nullptr && (uintptr_t)planes % 16 == 0), "zk_rope_cache_write: partial sums must be 16-byte aligned");
   if (T == 0) return 0;
   const QkvSource from{(const act_t*)qkv, planes, sums, (size_t)T * (nh + 2 * nkv) * hd};
-  if (rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed)) {
+  if (rope_by_token(T, nh, nkv, hd, rotary_dim, v_transposed, sums)) {
     const auto kernel = !v_transposed ? rope_cache_write_token_kernel<ROPE_ROWS>
                         : T >= 8 * 256 ? rope_cache_write_token_kernel<ROPE_MANY> : rope_cache_write_token_kernel<ROPE_FEW>;
     kernel<<<T, 256, 0, (hipStream_t)stream>>>((act_t*)qkv, from, positions, slot_map, inv_freq, (act_t*)kcache, (act_t*)vcache, nh, nkv,
