@@ -1744,8 +1744,8 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
       if constexpr (HD16 >= 8 && VD16 >= 8)
         if (stream_takes(p.hd, p.vd, p.bs, p.wide_weights)) return launch_stream<HD16, VD16, true>(p, grid, s);
       return launch_shared_one<HD16, VD16, 4, true>(p, grid, s);
-    case ATT_SHORT:          // (chosen for the sizes that attn_stream_kernel takes)
-      if constexpr (HD16 >= 8 && VD16 >= 8) {
+    case ATT_SHORT:
+      if constexpr (HD16 % 2 == 0) {
         constexpr size_t lds = ((size_t)ATT_SHORT_WAVES * 16 * (VD16 * 16 + 4) + ATT_SHORT_WAVES * 32) * sizeof(float);
         static std::atomic<bool> prepared{false};
         if (lds > 64 * 1024 && !prepared) {
@@ -1757,7 +1757,7 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
         attn_short_kernel<HD16 / 2, VD16, ATT_SHORT_WAVES><<<grid, ATT_SHORT_WAVES * 64, lds, s>>>(p);
         break;
       } else {
-        return zk_fail("zk_attention_bf16: the kernel of few rows takes heads of 128 and 256 channels");
+        return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
       }
     case ATT_DECODE:
       if constexpr (HD16 % 2 == 0) {
