@@ -1237,7 +1237,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
     auto load_v = [&]() {
       if (bsh >= 3) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) vf[dt] = *(const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh));
+        for (int dt = 0; dt < DT; dt++) vf[dt] = load_once((const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh)));
       } else {         // pages of four keys
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) {
@@ -1586,8 +1586,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) {
         const int d = dt * 16 + col;
-        const bf16x4 va = *(const bf16x4*)(va_base + ((size_t)d << bsh));
-        const bf16x4 vb = *(const bf16x4*)(vb_base + ((size_t)d << bsh));
+        const bf16x4 va = load_once((const bf16x4*)(va_base + ((size_t)d << bsh)));
+        const bf16x4 vb = load_once((const bf16x4*)(vb_base + ((size_t)d << bsh)));
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           vf[dt][e] = va[e];

@@ -30,6 +30,17 @@ __device__ __forceinline__ float from_f32<float>(float x) { return x; }
 template <>
 __device__ __forceinline__ __bf16 from_f32<__bf16>(float x) { return (__bf16)x; }
 
+// A load of 8 or 16 bytes that one block reads once in a launch (a weight, a cached value), marked non-temporal: the
+// caches do not make room for it.  A streaming read reaches 6.5 to 6.8 TB/s so, 6.0 to 6.1 without (blocks of 4 or 8 waves, 100 MB to 1.6 GB);
+// a step of 8 decoded tokens of 27B shapes 10,830 -> 9,760 us, of 8 and 1 of 2B shapes 2,228 -> 2,160 and 1,655 -> 1,595.  Only for
+// whole 128-byte lines a load (weights in strips, transposed values): where a wave asks for a line's halves one after the other (rows of
+// cached keys), the second half comes from further away again (64 requests of 200 to 3,840 keys with the keys so too: 4,880 -> 5,010 us).
+template <typename T>
+__device__ __forceinline__ T load_once(const T* p) {
+  typedef unsigned words __attribute__((ext_vector_type(sizeof(T) / 4)));
+  return __builtin_bit_cast(T, __builtin_nontemporal_load((const words*)p));
+}
+
 // One rotation of a pair by an angle, written so that every kernel that rotates rounds alike
 // (a token's values must not depend on how many tokens the step holds or on which kernel took
 // it): a product rounded, then one fused multiply-add.

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
         // (a constant in an address reaches 4 KB)
         const char *lo = wrun[g] + (size_t)s0 * 1024, *hi = lo + 4096;
 #pragma unroll
-        for (int s = 0; s < STEPS; s++) wf[g][s] = *(const bf16x8*)((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane);
+        for (int s = 0; s < STEPS; s++) wf[g][s] = load_once((const bf16x8*)((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane));
       }
 #pragma unroll
       for (int s = 0; s < STEPS; s++) af[0][s] = *(const bf16x8*)(a + s * 64 + alane);
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) af[mt][s] = *(const bf16x8*)(ap[mt] + step * 32);
 #pragma unroll
-        for (int g = 0; g < NS; g++) wf[g][s] = *(const bf16x8*)(wp[g] + (size_t)step * wstep);
+        for (int g = 0; g < NS; g++) wf[g][s] = load_once((const bf16x8*)(wp[g] + (size_t)step * wstep));
       }
       if (run_lo + run_n > total_steps) {
 #pragma unroll
@@ -972,7 +972,7 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const __bf16* __restrict_
     for (int s = 0; s < WSTEPS; s++)
 #pragma unroll
       for (int g = 0; g < NS; g++)
-        wf[g][s] = *(const bf16x8*)(wp[g] + (size_t)min(s0 + khalf * WSTEPS + s, s_end - 1) * 512);
+        wf[g][s] = load_once((const bf16x8*)(wp[g] + (size_t)min(s0 + khalf * WSTEPS + s, s_end - 1) * 512));
   };
   auto multiply = [&](int buf, const bf16x8 (&wf)[NS][WSTEPS]) {
 #pragma unroll
