@@ -127,6 +127,13 @@ __device__ __forceinline__ bf16x8 zero8() {
   return z;
 }
 
+// Whether the weights are read past the caches: the caller says that no step finds there what the last one read (w_strip 3).
+static bool reads_once(int w_strip) { return (w_strip & 2) != 0; }
+template <bool ONCE>
+__device__ __forceinline__ bf16x8 load_weights(const void* p) {
+  return ONCE ? load_once((const bf16x8*)p) : *(const bf16x8*)p;
+}
+
 // ------------------------------------------------------------------ skinny
 // What the q|k|v product of decoded tokens does with its results instead of storing them all:
 // q and k heads are rotated (pairs (i, i + hd/2), angle position * inv_freq[i]), q goes to C,
@@ -165,7 +172,8 @@ __device__ __forceinline__ void store4(__bf16* dst, const float (&x)[4]) {
 // bits), the addresses of a group are a hundred instructions that a wave issues one every fourth cycle in
 // front of its loads (us, 8 rows: 4,096 columns of K 2,304 6.3 -> 5.5, 2,304 of 2,048
 // 5.0 -> 4.4, 2,304 of 9,216 13.3 -> 12.4; a step of 8 decoded tokens of the 2B shapes 2,319 -> 2,278).  The same sums.
-template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false, bool WHOLE = false>
+// ONCE (WHOLE): weights by loads that leave no trace in the caches (reads_once).
+template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false, bool WHOLE = false, bool ONCE = false>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __restrict__ A, int lda,
                                                           const __bf16* __restrict__ W,
                                                           void* __restrict__ C, int ldc, int c_is_f32,
@@ -254,7 +262,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
         // (a constant in an address reaches 4 KB)
         const char *lo = wrun[g] + (size_t)s0 * 1024, *hi = lo + 4096;
 #pragma unroll
-        for (int s = 0; s < STEPS; s++) wf[g][s] = load_once((const bf16x8*)((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane));
+        for (int s = 0; s < STEPS; s++) wf[g][s] = load_weights<ONCE>((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane);
       }
 #pragma unroll
       for (int s = 0; s < STEPS; s++) af[0][s] = *(const bf16x8*)(a + s * 64 + alane);
@@ -270,7 +278,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) af[mt][s] = *(const bf16x8*)(ap[mt] + step * 32);
 #pragma unroll
-        for (int g = 0; g < NS; g++) wf[g][s] = load_once((const bf16x8*)(wp[g] + (size_t)step * wstep));
+        for (int g = 0; g < NS; g++) wf[g][s] = *(const bf16x8*)(wp[g] + (size_t)step * wstep);
       }
       if (run_lo + run_n > total_steps) {
 #pragma unroll
@@ -861,89 +869,88 @@ static bool joinable_by_reader(int N, int ldc, int c_is_f32, int epi) {
   return N % 16 == 0 && ldc == N && !c_is_f32 && epi == EPI_NONE;
 }
 
-// ------------------------------------------------------------------ mid (16 < M <= 64)
-// With more than one column tile the activations weigh more than the weights on the way
-// from L2 to the CUs when every 16-row strip fetches them again (64 rows of A per 16 rows
-// of W).  Here a block owns four strips, a pair of waves each, all walk K together, and the
-// activations of the current 256-wide k chunk wait in LDS for all of them: 64 rows of A per
-// 64 rows of W.  Weights come straight from global memory in strip layout, the loads of the
-// next two chunks are in flight while the current one is multiplied.
+// ------------------------------------------------------------------ mid (up to 64 rows)
+// A block owns SPB strips (gated: strips of gate and up), KW waves each; all walk K together in chunks of CH 32-wide steps, of which a
+// wave multiplies CH / KW, and the activations of a chunk wait in LDS for all of them.  Weights come straight from global memory in
+// strip layout, the loads of the next two chunks are in flight while the current one is multiplied.
 //
-// Few column blocks (N of a few thousand) cannot fill 256 CUs, so blockIdx.y splits K into
+// Why through LDS: straight from memory every wave asks for 16 rows' half lines of 64 bytes a step, which a CU fetches at 13 to 20 bytes
+// a cycle, so from some ten rows on the activations and not the weights set the time (9,216 gated columns of K 2,304 at 24 and 64 rows 20 to 21 and
+// 33 us, through LDS 16.1 and 18.9).
+//
+// Which split (the launcher's tables): what counts is the most strips a CU gets, so SPB follows from the number of strips; KW then gives
+// the block eight to sixteen waves, because a chunk's chain (reads from LDS, products) takes as long as a load and more waves a SIMD
+// fill its waits.  Four waves of a strip and not two of eight strips' four places, one of them idle: 9,216 gated columns of K 2,304 at 24 and
+// 64 rows 18.9 -> 16.1 and 22.4 -> 18.9 us; 4,096 of 1,024, which were 64 blocks and a join, 10.0 -> 6.1 and 12.4 -> 7.6; 8,192 of 2,048 18.8 ->
+// 13.2 and 21.5 -> 15.0.
+//
+// Few column blocks of a plain product (N of a few thousand) cannot fill 256 CUs, so blockIdx.y splits K into
 // `ksplit` ranges.  Then each block leaves its partial sums in the workspace and a second,
 // small kernel adds them in the order of the ranges and applies the epilogue.  (One kernel
 // with a ticket per column block, the last block adding up, was measured three times slower:
 // the device-wide fences it needs write back and invalidate the L2 of every XCD.)
-#define GM_STEPS 8
-#define GM_LD (GM_STEPS * 32 + 16)
 
-// A lane's results of one strip: rows n = 16 * strip + 4 * kq + i of W, column m = 16 * mt + r of A.
-template <int MT, bool GATED>
-__device__ __forceinline__ void mid_store(const f32x4 (&acc)[GATED ? 2 : 1][MT], void* __restrict__ C, int ldc,
+// A lane's results of one strip and 16 rows: columns n = 16 * strip + 4 * kq + i, row m of A.
+template <bool GATED>
+__device__ __forceinline__ void mid_store(const f32x4& v, const f32x4& up, int m, void* __restrict__ C, int ldc,
                                           int c_is_f32, int M, int N, int strip, int lane, int epi, float cap,
                                           float* __restrict__ picks, int nstrips) {
-  const int r = lane & 15, kq = lane >> 4;
+  const int kq = lane >> 4;
+  if (!GATED && epi == EPI_PICK) {
+    const float x[4] = {v[0], v[1], v[2], v[3]};
+    const Pick p = pick_of_strip(x, strip * 16 + 4 * kq, N, cap);
+    if (kq == 0 && m < M) ((Pick*)picks)[(size_t)m * nstrips + strip] = p;
+    return;
+  }
+  if (m >= M) return;
+  float x[4];
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++) {
-    const int m = mt * 16 + r;
-    if (!GATED && epi == EPI_PICK) {
-      const float x[4] = {acc[0][mt][0], acc[0][mt][1], acc[0][mt][2], acc[0][mt][3]};
-      const Pick p = pick_of_strip(x, strip * 16 + 4 * kq, N, cap);
-      if (kq == 0 && m < M) ((Pick*)picks)[(size_t)m * nstrips + strip] = p;
-      continue;
-    }
-    if (m >= M) continue;
+  for (int i = 0; i < 4; i++) x[i] = GATED ? epi_gate(v[i], up[i], epi, cap) : epi_unary(v[i], epi, cap);
+  const int n = strip * 16 + 4 * kq;
+  if (!c_is_f32 && n + 4 <= N && (((uintptr_t)C | (unsigned)ldc * 2) & 7) == 0) {
+    store4((__bf16*)C + (size_t)m * ldc + n, x);
+    return;
+  }
+  if (c_is_f32 && n + 4 <= N && (((uintptr_t)C | (unsigned)ldc * 4) & 15) == 0) {
+    *(f32x4*)((float*)C + (size_t)m * ldc + n) = f32x4{x[0], x[1], x[2], x[3]};
+    return;
+  }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int n = strip * 16 + 4 * kq + i;
-      if (n >= N) continue;
-      float x = acc[0][mt][i];
-      if (GATED) x = epi_gate(x, acc[GATED ? 1 : 0][mt][i], epi, cap);
-      else x = epi_unary(x, epi, cap);
-      if (c_is_f32) ((float*)C)[(size_t)m * ldc + n] = x;
-      else ((__bf16*)C)[(size_t)m * ldc + n] = (__bf16)x;
-    }
+  for (int i = 0; i < 4; i++) {
+    if (n + i >= N) continue;
+    if (c_is_f32) ((float*)C)[(size_t)m * ldc + n + i] = x[i];
+    else ((__bf16*)C)[(size_t)m * ldc + n + i] = (__bf16)x[i];
   }
 }
 
-// Eight waves a block, two for each of its four strips: waves 0..3 take the first half of a
-// chunk's steps, waves 4..7 the second, and the second wave's sums reach the first through LDS
-// at the end.  A wave holds three chunks' weights in registers (one being multiplied, two on
-// their way) and the activations have three buffers in LDS: a chunk's products take less time
-// than a load (at 64 rows with a gate about 1.2 us against 2 us), so with one chunk on its way
-// every chunk waited for its loads, and where the column blocks are too few for a second block
-// on the CU (N = 9216 with a gate: 144 blocks) nothing filled the wait.  Against four waves with
-// one chunk ahead: 5 to 17 % less time at 24 to 64 rows on the layer shapes of the 2B, 9B and
-// 27B models (2B down at 64 rows 15.4 -> 13.1 us, 9B down at 32 rows 25.0 -> 21.2 us); two waves
-// a strip alone, without the second chunk ahead, gave 0 to 3 %.
-template <int MT, bool GATED>
-__global__ __launch_bounds__(512) void gemm_mid_kernel(const __bf16* __restrict__ A, int lda,
-                                                        const __bf16* __restrict__ W,
-                                                        void* __restrict__ C, int ldc, int c_is_f32,
-                                                        int M, int N, int K, int epi, float cap,
-                                                        float* __restrict__ partials, int ksplit, int spb) {
+template <int MT, bool GATED, int SPB, int KW, int CH, bool ONCE>
+__global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* __restrict__ A, int lda,
+                                                                 const __bf16* __restrict__ W,
+                                                                 void* __restrict__ C, int ldc, int c_is_f32,
+                                                                 int M, int N, int K, int epi, float cap,
+                                                                 float* __restrict__ partials, int ksplit) {
   constexpr int NS = GATED ? 2 : 1;
-  constexpr int WSTEPS = GM_STEPS / 2;                  // steps of a chunk a wave multiplies
-  __shared__ __bf16 sA[3][MT * 16][GM_LD];
-  const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) & 3, khalf = tid >> 8;
+  constexpr int T = SPB * KW * 64, WSTEPS = CH / KW;     // threads; steps of a chunk a wave multiplies
+  constexpr int LD = CH * 32 + 16, PPR = CH * 4;         // a row of a chunk in LDS, its 16-byte pieces
+  constexpr int PIECES = MT * 16 * PPR, APT = (PIECES + T - 1) / T;
+  static_assert(CH % KW == 0, "whole steps a wave");
+  // three chunks of activations, and after the loop the waves' sums
+  constexpr size_t ACTS = (size_t)3 * MT * 16 * LD * sizeof(__bf16), SUMS = (size_t)SPB * KW * NS * MT * 64 * sizeof(f32x4);
+  __shared__ __align__(16) unsigned char lds[ACTS > SUMS ? ACTS : SUMS];
+  __bf16(*sA)[MT * 16][LD] = (__bf16(*)[MT * 16][LD])lds;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int place = wave % SPB, kpart = wave / SPB;
   const int r = lane & 15, kq = lane >> 4;
   const int ksteps = K / 32;
   const int s_begin = (int)((long)blockIdx.y * ksteps / ksplit);
   const int s_end = (int)((long)(blockIdx.y + 1) * ksteps / ksplit);
   const int nstrips = (N + 15) / 16;
-  // spb strips a block (3 where that spreads the strips more evenly over the CUs).  The waves of
-  // the fourth place then do the first place's work over again and store nothing: their loads
-  // hit what the first place's waves have just fetched, and a branch around loads would make
-  // the compiler wait for every load in flight.
-  const int strip = blockIdx.x * spb + (wave < spb ? wave : 0);
-  const bool strip_ok = wave < spb && strip < nstrips;
-  const int strip_read = strip < nstrips ? strip : 0;
+  const int strip = blockIdx.x * SPB + place;
+  const bool strip_ok = strip < nstrips;
+  const int strip_read = min(strip, nstrips - 1);
   const __bf16* wp[NS];
   wp[0] = W + (size_t)strip_read * ksteps * 512 + lane * 8;
   if (GATED) wp[NS - 1] = W + ((size_t)(N / 16) + strip_read) * ksteps * 512 + lane * 8;
-  // A pieces of a chunk: MT*16 rows x 32 pieces of 16 bytes, 16 rows a pass of the 512 threads
-  constexpr int APT = MT * 16 * 32 / 512;
-  const int a_piece = tid & 31, a_row0 = tid >> 5;
   f32x4 acc[NS][MT];
 #pragma unroll
   for (int g = 0; g < NS; g++)
@@ -952,34 +959,37 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const __bf16* __restrict_
 
   // Every load is issued, none under a condition: a step past the range reads the range's last
   // step again, a row past M row M - 1; activations outside are set to zero afterwards, which
-  // makes the product nothing whatever the weights.
+  // makes the product nothing whatever the weights.  (A thread past the pieces takes the last one, as its owner does.)
   auto fetch_a = [&](int s0, bf16x8 (&ra)[APT]) {
 #pragma unroll
     for (int j = 0; j < APT; j++) {
-      const int row = a_row0 + 16 * j;
-      const bool in = row < M && s0 + a_piece / 4 < s_end;
-      const int step = min(s0 + a_piece / 4, s_end - 1);
-      const bf16x8 v = *(const bf16x8*)(A + (size_t)min(row, M - 1) * lda + step * 32 + (a_piece % 4) * 8);
+      const int q = min(tid + T * j, PIECES - 1), row = q / PPR, piece = q % PPR;
+      const bool in = row < M && s0 + piece / 4 < s_end;
+      const int step = min(s0 + piece / 4, s_end - 1);
+      const bf16x8 v = *(const bf16x8*)(A + (size_t)min(row, M - 1) * lda + step * 32 + (piece % 4) * 8);
       ra[j] = in ? v : zero8();
     }
   };
   auto stash_a = [&](int buf, const bf16x8 (&ra)[APT]) {
 #pragma unroll
-    for (int j = 0; j < APT; j++) *(bf16x8*)(&sA[buf][a_row0 + 16 * j][a_piece * 8]) = ra[j];
+    for (int j = 0; j < APT; j++) {
+      const int q = min(tid + T * j, PIECES - 1);
+      *(bf16x8*)(&sA[buf][q / PPR][(q % PPR) * 8]) = ra[j];
+    }
   };
   auto fetch_w = [&](int s0, bf16x8 (&wf)[NS][WSTEPS]) {
 #pragma unroll
     for (int s = 0; s < WSTEPS; s++)
 #pragma unroll
       for (int g = 0; g < NS; g++)
-        wf[g][s] = load_once((const bf16x8*)(wp[g] + (size_t)min(s0 + khalf * WSTEPS + s, s_end - 1) * 512));
+        wf[g][s] = load_weights<ONCE>(wp[g] + (size_t)min(s0 + kpart * WSTEPS + s, s_end - 1) * 512);
   };
   auto multiply = [&](int buf, const bf16x8 (&wf)[NS][WSTEPS]) {
 #pragma unroll
     for (int s = 0; s < WSTEPS; s++)
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
-        const bf16x8 af = *(const bf16x8*)(&sA[buf][mt * 16 + r][(khalf * WSTEPS + s) * 32 + kq * 8]);
+        const bf16x8 af = *(const bf16x8*)(&sA[buf][mt * 16 + r][(kpart * WSTEPS + s) * 32 + kq * 8]);
 #pragma unroll
         for (int g = 0; g < NS; g++)
           acc[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af, acc[g][mt], 0, 0, 0);
@@ -992,57 +1002,59 @@ __global__ __launch_bounds__(512) void gemm_mid_kernel(const __bf16* __restrict_
   bf16x8 ra0[APT], ra1[APT], w0[NS][WSTEPS], w1[NS][WSTEPS], w2[NS][WSTEPS];
   fetch_a(s_begin, ra0);
   fetch_w(s_begin, w0);
-  fetch_a(s_begin + GM_STEPS, ra1);
-  fetch_w(s_begin + GM_STEPS, w1);
+  fetch_a(s_begin + CH, ra1);
+  fetch_w(s_begin + CH, w1);
   stash_a(0, ra0);
   __syncthreads();
-#define ZK_MID8_TURN(BUF, WCUR, WNEXT2, RA_NEXT2, RA_NEXT1)   \
-  fetch_a(s0 + 2 * GM_STEPS, RA_NEXT2);                       \
-  fetch_w(s0 + 2 * GM_STEPS, WNEXT2);                         \
+#define ZK_MID_TURN(BUF, WCUR, WNEXT2, RA_NEXT2, RA_NEXT1)    \
+  fetch_a(s0 + 2 * CH, RA_NEXT2);                             \
+  fetch_w(s0 + 2 * CH, WNEXT2);                               \
   multiply(BUF, WCUR);                                        \
-  s0 += GM_STEPS;                                             \
+  s0 += CH;                                                   \
   if (s0 >= s_end) break;                                     \
   stash_a((BUF + 1) % 3, RA_NEXT1);                           \
   __syncthreads();
   for (int s0 = s_begin;;) {
-    ZK_MID8_TURN(0, w0, w2, ra0, ra1)
-    ZK_MID8_TURN(1, w1, w0, ra1, ra0)
-    ZK_MID8_TURN(2, w2, w1, ra0, ra1)
-    ZK_MID8_TURN(0, w0, w2, ra1, ra0)
-    ZK_MID8_TURN(1, w1, w0, ra0, ra1)
-    ZK_MID8_TURN(2, w2, w1, ra1, ra0)
+    ZK_MID_TURN(0, w0, w2, ra0, ra1)
+    ZK_MID_TURN(1, w1, w0, ra1, ra0)
+    ZK_MID_TURN(2, w2, w1, ra0, ra1)
+    ZK_MID_TURN(0, w0, w2, ra1, ra0)
+    ZK_MID_TURN(1, w1, w0, ra0, ra1)
+    ZK_MID_TURN(2, w2, w1, ra1, ra0)
   }
-#undef ZK_MID8_TURN
-  // the second wave of each strip hands its sums over (the activation buffers are free once
-  // every wave has left the loop); first half + second half, in that order
+#undef ZK_MID_TURN
+  // The waves of a strip lay their sums down (the activation buffers are free once every wave has left the
+  // loop) and share the rows out among themselves: sixteen rows a wave, the sums in the order of the chunk's parts.
   __syncthreads();
-  static_assert(sizeof(sA) >= (size_t)4 * NS * MT * 64 * sizeof(f32x4), "no room to hand the sums over");
-  f32x4* hand = (f32x4*)&sA[0][0][0] + ((size_t)wave * NS * MT) * 64 + lane;
-  if (khalf == 1) {
-#pragma unroll
-    for (int g = 0; g < NS; g++)
-#pragma unroll
-      for (int mt = 0; mt < MT; mt++) hand[(g * MT + mt) * 64] = acc[g][mt];
-  }
-  __syncthreads();
-  if (khalf == 1) return;
+  f32x4* sums = (f32x4*)lds + ((size_t)place * KW * NS * MT) * 64 + lane;
 #pragma unroll
   for (int g = 0; g < NS; g++)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[g][mt] += hand[(g * MT + mt) * 64];
-  if (ksplit > 1) {
-    // the range's partial sums: plane (range, g) of [M, npad] floats
-    if (!strip_ok) return;
-    const size_t npad = (size_t)nstrips * 16;
-    float* planes = partials + (size_t)blockIdx.y * NS * M * npad + strip * 16 + 4 * kq;
+    for (int mt = 0; mt < MT; mt++) sums[((kpart * NS + g) * MT + mt) * 64] = acc[g][mt];
+  __syncthreads();
+  if (!strip_ok) return;
+  const size_t npad = (size_t)nstrips * 16;
 #pragma unroll
-    for (int g = 0; g < NS; g++)
+  for (int mt0 = 0; mt0 < MT; mt0 += KW) {
+    const int mt = mt0 + kpart, m = mt * 16 + r;
+    if (mt >= MT) break;
+    f32x4 v[NS];
 #pragma unroll
-      for (int mt = 0; mt < MT; mt++)
-        if (mt * 16 + r < M) *(f32x4*)(planes + ((size_t)g * M + mt * 16 + r) * npad) = acc[g][mt];
-    return;
+    for (int g = 0; g < NS; g++) {
+      v[g] = sums[(g * MT + mt) * 64];
+#pragma unroll
+      for (int k = 1; k < KW; k++) v[g] += sums[((k * NS + g) * MT + mt) * 64];
+    }
+    if (ksplit > 1) {
+      // the range's partial sums: plane (range, g) of [M, npad] floats
+      float* planes = partials + (size_t)blockIdx.y * NS * M * npad + strip * 16 + 4 * kq;
+#pragma unroll
+      for (int g = 0; g < NS; g++)
+        if (m < M) *(f32x4*)(planes + ((size_t)g * M + m) * npad) = v[g];
+      continue;
+    }
+    mid_store<GATED>(v[0], v[NS - 1], m, C, ldc, c_is_f32, M, N, strip, lane, epi, cap, partials, nstrips);
   }
-  if (strip_ok) mid_store<MT, GATED>(acc, C, ldc, c_is_f32, M, N, strip, lane, epi, cap, partials, nstrips);
 }
 
 // Four neighbouring results of a row, in one store where the address allows it.
@@ -1087,52 +1099,117 @@ __global__ __launch_bounds__(256) void gemm_join_kernel(const float* __restrict_
 
 #include "gemm_bf16_tiles.h"
 
+// How a product of up to 64 rows by weights in strips is cut: strips a block, waves a strip, steps a chunk, ranges of K.
+struct MidCut {
+  int spb, kw, ch, ksplit;
+};
+
+// Ranges of K for blocks of ``ch`` steps a chunk: until every CU has a block, a range no shorter than a chunk; two
+// blocks a CU where ranges stay long (16 chunks of 8 steps or more: the blocks of a CU then cover each
+// other's waits).  More ranges than that cost more in partial sums than they gain.  The
+// longest range sets the time, so of the splits with that longest range the one with the
+// fewest ranges is taken (8 chunks: 4 ranges of 2 instead of 7 of 1 or 2; measured at the
+// shapes of the 2B, 9B and 27B layers with 24 to 64 rows).
+static int mid_ranges(int cblocks, int ksteps, int ch) {
+  const int chunks = max(1, ksteps / ch);
+  int ks = max(1, min(256 / cblocks, chunks));
+  if (ch == 8 && chunks / max(1, 512 / cblocks) >= 16) ks = max(1, min(512 / cblocks, chunks));
+  const int longest = (chunks + ks - 1) / ks;
+  return (chunks + longest - 1) / longest;
+}
+
+// The cut follows from the shape alone, and for up to 16 rows not from their number either: a request's bits do not depend on how
+// many share its step.
+static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
+  const int nstrips = (N + 15) / 16, ksteps = K / 32;
+  if (gated) {
+    // Few long strips (a lone block would fetch 0.8 MB and more): in ranges, with a join (2,048 columns of K 8,192 at 24 and 64 rows 20.1 and 22.0 us, whole
+    // 22.2 and 30.8; 512 of 4,096 at 64 14.4 and 16.5, at 24 not: 11.9 and 11.5).  Else whole, as many strips a block as give the fullest CU the
+    // least, of equals the more: 256 strips one a block, 512 two, 576 three, 896 four, 2,304 three.
+    if (split_ok && M > 16 && nstrips <= 192 && (64.0 + 2 * M) * K > 780e3) return {4, 2, 8, mid_ranges((nstrips + 3) / 4, ksteps, 8)};
+    int spb = 1;
+    auto most = [&](int b) { return (long)(((nstrips + b - 1) / b + 255) / 256) * b; };
+    for (int b = 2; b <= 4; b++)
+      if (most(b) <= most(spb)) spb = b;
+    if (nstrips <= 256) spb = 1;
+    return spb == 1 ? MidCut{1, 8, 8, 1} : spb == 2 ? MidCut{2, 4, 8, 1} : spb == 3 ? MidCut{3, 4, 4, 1} : MidCut{4, 2, 4, 1};
+  }
+  // Thousands of strips (a head): two strips a block up to 16 rows, eight beyond, where the activations weigh more
+  // (256,000 columns of K 2,304, four strips and eight, 24 rows 195 and 192 us, 48 228 and 214, 64 253 and 224); where those would be one block a
+  // CU, four with sixteen waves (32,768 of 2,048, eight and four: 24 rows 32.0 and 24.7, 64 36.1 and 27.3).
+  if (M <= 16 && nstrips >= 1024) return {2, 8, 16, 1};
+  if (nstrips >= 4096) return {8, 1, 4, 1};
+  if (nstrips >= 1024) return {4, 4, 4, 1};
+  if (M <= 16) return {3, 4, 8, mid_ranges((nstrips + 2) / 3, ksteps, 8)};
+  const int cblocks = (nstrips + 3) / 4;
+  if (!split_ok) return {4, 2, 8, 1};
+  const int ks = mid_ranges(cblocks, ksteps, 8);
+  // ranges of less than 24 steps: chunks of four and twice the waves (us, 24 and 64 rows: 4,096 columns of K 2,304 6.2 -> 5.9 and
+  // 7.7 -> 7.4, 2,304 of 2,048 5.2 -> 4.6 and 6.7 -> 6.1)
+  if (ks > 1 && ksteps / ks < 24) return {4, 4, 4, mid_ranges(cblocks, ksteps, 4)};
+  return {4, 2, 8, ks};
+}
+
+// Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us, straight
+// and so, 1, 8 and 16 rows.  Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3, 33.1, 33.4;
+// not 8,192 of 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.  Heads: 256,000 of 2,304
+// 170, 186, 249 and 174, 179, 206; not 32,768 of 1,024 12.2, 13.1, 15.8 and 14.1, 14.5, 15.1.  Long ones with the partial sums left to the reader:
+// 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of 36,864 53, 54, 69 and 53, 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1,
+// 9.3, 9.5.
+static bool mid_for_few(bool gated, int N, int K, bool by_reader) {
+  const int nstrips = (N + 15) / 16;
+  if (gated) return nstrips > 512 && nstrips <= 1024;
+  return (nstrips >= 1024 && K >= 2048) || (by_reader && K >= 8192 && nstrips > 192);
+}
+
 template <bool GATED>
 static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32, int M, int N,
-                      int K, int epi, float cap, const GemmWorkspace& wsp, int* parts, hipStream_t s) {
+                      int K, int epi, float cap, int w_strip, const GemmWorkspace& wsp, int* parts, hipStream_t s) {
   const int mt = (M + 15) / 16;
-  const int npad = (N + 15) / 16 * 16;
-  const int nstrips = (N + 15) / 16;
-  // Strips a block: four, or three where the blocks of four fill the CUs unevenly and K is not
-  // split anyway (N = 9216 with a gate is 576 strips: 144 blocks of four leave 112 CUs idle, 192
-  // blocks of three give every busy CU a quarter less to read: 28.0 -> 24.6 us at 64 rows;
-  // 2304 strips: three rounds of blocks either way, 157 -> 146 us).  What counts is the most
-  // strips a CU gets, rounds of 256 blocks times the strips of a block.
-  int spb = 4;
-  {
-    auto most = [&](int b) { return (long)(((nstrips + b - 1) / b + 255) / 256) * b; };
-    if ((nstrips + 3) / 4 > 128 && most(3) * 10 <= most(4) * 9) spb = 3;
-  }
-  const int cblocks = (nstrips + spb - 1) / spb;
-  // Split K until every CU has a block, a range no shorter than a chunk of GM_STEPS steps; two
-  // blocks a CU where ranges stay long (16 chunks or more: the blocks of a CU then cover each
-  // other's waits).  More ranges than that cost more in partial sums than they gain.  The
-  // longest range sets the time, so of the splits with that longest range the one with the
-  // fewest ranges is taken (8 chunks: 4 ranges of 2 instead of 7 of 1 or 2; measured at the
-  // shapes of the 2B, 9B and 27B layers with 24 to 64 rows).
-  const int chunks = max(1, K / 32 / GM_STEPS);
-  int ksplit = max(1, min(256 / cblocks, chunks));
-  if (chunks / max(1, 512 / cblocks) >= 16) ksplit = max(1, min(512 / cblocks, chunks));
-  {
-    const int longest = (chunks + ksplit - 1) / ksplit;
-    ksplit = (chunks + longest - 1) / longest;
-  }
-  const size_t per_range = (size_t)(GATED ? 2 : 1) * M * npad * sizeof(float);
+  const int nstrips = (N + 15) / 16, npad = nstrips * 16;
   void* ws = wsp.ptr;
-  if (ws == nullptr || (uintptr_t)ws % 16 != 0 || epi == EPI_PICK) ksplit = 1;      // picks are taken from whole sums
-  while (ksplit > 1 && ksplit * per_range > wsp.split_bytes()) ksplit--;
-  if (ksplit > 1 && ksplit * per_range > wsp.bytes) return wsp.too_small(ksplit * per_range);
+  // picks are taken from whole sums; up to 16 rows only a reader that adds up the partial sums itself is worth a split
+  const bool by_reader = parts != nullptr && joinable_by_reader(N, ldc, c_is_f32, epi);
+  const bool split_ok = ws != nullptr && (uintptr_t)ws % 16 == 0 && epi != EPI_PICK && (M > 16 || by_reader);
+  MidCut cut = mid_cut(GATED, M, N, K, split_ok);
+  const size_t per_range = (size_t)(GATED ? 2 : 1) * M * npad * sizeof(float);
+  while (cut.ksplit > 1 && cut.ksplit * per_range > wsp.split_bytes()) cut.ksplit--;
+  if (cut.ksplit > 1 && cut.ksplit * per_range > wsp.bytes) return wsp.too_small(cut.ksplit * per_range);
+  const int ksplit = cut.ksplit;
   float* partials = (float*)ws;
-  dim3 grid(cblocks, ksplit);
-#define ZK_MID(MT_)                                                                                   \
-  gemm_mid_kernel<MT_, GATED><<<grid, 512, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, \
-                                                   M, N, K, epi, cap, partials, ksplit, spb)
-  if (mt == 2) { ZK_MID(2); }
-  else if (mt == 3) { ZK_MID(3); }
-  else { ZK_MID(4); }
+  dim3 grid((nstrips + cut.spb - 1) / cut.spb, ksplit);
+#define ZK_MID_(MT_, SPB_, KW_, CH_, ONCE_)                                                             \
+  gemm_mid_kernel<MT_, GATED, SPB_, KW_, CH_, ONCE_><<<grid, SPB_ * KW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, C, ldc, \
+                                                                                     c_is_f32, M, N, K, epi, cap, partials, ksplit)
+#define ZK_MID(MT_, SPB_, KW_, CH_)                                                      \
+  do {                                                                                   \
+    if (reads_once(w_strip)) ZK_MID_(MT_, SPB_, KW_, CH_, true);                         \
+    else ZK_MID_(MT_, SPB_, KW_, CH_, false);                                            \
+  } while (0)
+#define ZK_MID_ROWS(SPB_, KW_, CH_)                   \
+  do {                                                \
+    if (mt == 1) ZK_MID(1, SPB_, KW_, CH_);           \
+    else if (mt == 2) ZK_MID(2, SPB_, KW_, CH_);      \
+    else if (mt == 3) ZK_MID(3, SPB_, KW_, CH_);      \
+    else ZK_MID(4, SPB_, KW_, CH_);                   \
+  } while (0)
+  if (cut.spb == 4 && cut.ch == 8) ZK_MID_ROWS(4, 2, 8);
+  else if constexpr (GATED) {
+    if (cut.spb == 1) ZK_MID_ROWS(1, 8, 8);
+    else if (cut.spb == 2) ZK_MID_ROWS(2, 4, 8);
+    else if (cut.spb == 3) ZK_MID_ROWS(3, 4, 4);
+    else ZK_MID_ROWS(4, 2, 4);
+  } else {
+    if (cut.spb == 8) ZK_MID_ROWS(8, 1, 4);
+    else if (cut.spb == 2) ZK_MID(1, 2, 8, 16);
+    else if (cut.spb == 3) ZK_MID(1, 3, 4, 8);
+    else ZK_MID_ROWS(4, 4, 4);
+  }
+#undef ZK_MID_ROWS
 #undef ZK_MID
+#undef ZK_MID_
   if (ksplit > 1) {
-    if (parts && joinable_by_reader(N, ldc, c_is_f32, epi)) {
+    if (by_reader) {
       *parts = ksplit;
       return zk_launch_status("zk_gemm_bf16 (mid)");
     }
@@ -1197,9 +1274,14 @@ static int launch_skinny(const void* A, int lda, const void* W, void* C, int ldc
   const bool whole = w_strip && mt == 1 && K % 256 == 0 && lda <= (1 << 26);
   // few strips: eight waves a strip keep enough loads in flight
   const bool wide = !few_long && (long)grid.x * ksplit < 512 && K / ksplit >= 2048 && mt <= 2;
+  const bool once = reads_once(w_strip);
 #define ZK_SKINNY(MT_, NW_)                                                                           \
   do {                                                                                                \
-    if (MT_ == 1 && whole)                                                                            \
+    if (MT_ == 1 && whole && once)                                                                    \
+      gemm_skinny_kernel<1, GATED, NW_, false, true, false, true, true><<<grid, NW_ * 64, 0, s>>>(    \
+          (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
+          partials, 1);                                                                               \
+    else if (MT_ == 1 && whole)                                                                       \
       gemm_skinny_kernel<1, GATED, NW_, false, true, false, true><<<grid, NW_ * 64, 0, s>>>(          \
           (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
           partials, 1);                                                                               \
@@ -1212,13 +1294,13 @@ static int launch_skinny(const void* A, int lda, const void* W, void* C, int ldc
           (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, \
           partials, 1);                                                                               \
   } while (0)
-#define ZK_SPLIT(NW_, WHOLE_)                                                                        \
-  gemm_skinny_kernel<1, false, NW_, false, true, true, WHOLE_><<<grid, NW_ * 64, 0, s>>>(             \
+#define ZK_SPLIT(NW_, WHOLE_, ONCE_)                                                                        \
+  gemm_skinny_kernel<1, false, NW_, false, true, true, WHOLE_, ONCE_><<<grid, NW_ * 64, 0, s>>>(             \
       (const __bf16*)A, lda, (const __bf16*)W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, RopeStore{}, partials, ksplit)
   if (ksplit > 1) {
     if constexpr (!GATED) {
-      if (wide) { if (whole) ZK_SPLIT(8, true); else ZK_SPLIT(8, false); }
-      else { if (whole) ZK_SPLIT(4, true); else ZK_SPLIT(4, false); }
+      if (wide) { if (whole && once) ZK_SPLIT(8, true, true); else if (whole) ZK_SPLIT(8, true, false); else ZK_SPLIT(8, false, false); }
+      else { if (whole && once) ZK_SPLIT(4, true, true); else if (whole) ZK_SPLIT(4, true, false); else ZK_SPLIT(4, false, false); }
     }
   } else if (mt == 1) { if (wide) ZK_SKINNY(1, 8); else ZK_SKINNY(1, 4); }
   else if (mt == 2) { if (wide) ZK_SKINNY(2, 8); else ZK_SKINNY(2, 4); }
@@ -1258,13 +1340,16 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
   dim3 grid(N / 16);
   hipStream_t s = (hipStream_t)stream;
   const bool whole = w_strip && K % 256 == 0 && lda <= (1 << 26);
-#define ZK_QKV(NW_, EX_, WH_)                                                                                          \
-  gemm_skinny_kernel<1, false, NW_, true, EX_, false, WH_><<<grid, NW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, Q, \
+  const bool once = reads_once(w_strip);
+#define ZK_QKV(NW_, EX_, WH_, ONCE_)                                                                                          \
+  gemm_skinny_kernel<1, false, NW_, true, EX_, false, WH_, ONCE_><<<grid, NW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, Q, \
                                                                                     ldq, 0, M, N, K, EPI_NONE, 0.f, w_strip, rs)
   if (grid.x < 512 && K >= 2048) {
-    if (whole) ZK_QKV(8, true, true); else if (w_strip) ZK_QKV(8, true, false); else ZK_QKV(8, false, false);
+    if (whole && once) ZK_QKV(8, true, true, true); else if (whole) ZK_QKV(8, true, true, false);
+    else if (w_strip) ZK_QKV(8, true, false, false); else ZK_QKV(8, false, false, false);
   } else {
-    if (whole) ZK_QKV(4, true, true); else if (w_strip) ZK_QKV(4, true, false); else ZK_QKV(4, false, false);
+    if (whole && once) ZK_QKV(4, true, true, true); else if (whole) ZK_QKV(4, true, true, false);
+    else if (w_strip) ZK_QKV(4, true, false, false); else ZK_QKV(4, false, false, false);
   }
 #undef ZK_QKV
   return zk_launch_status("zk_qkv_rope_bf16");
@@ -1300,7 +1385,8 @@ extern "C" int zk_strip_layout(const void* src, void* dst, int N, int K, void* s
 
 // epi: 0 none, 1 soft cap (cap > 0), 2 gelu_tanh gate, 3 silu gate, 5 relu gate, 6 clamped gate (cap: its limit).  For the gated
 // epilogues W is [2N, K] (gate rows, then up rows) and C is [M, N].
-// w_strip: W is in strip layout (zk_strip_layout), which needs K % 32 == 0 and, for the
+// w_strip: not 0: W is in strip layout (zk_strip_layout); 3: and belongs to a model too large for the memory side's cache, so that products of up to
+// 64 rows read it past the caches (the same bits either way).  Strip layout needs K % 32 == 0 and, for the
 // gated epilogues, N % 16 == 0.
 // The workspace may be null; then K is never split over blocks.  It serves one launch at a time.
 // parts (may be null): a caller whose next kernel can add partial sums up itself passes a place
@@ -1459,9 +1545,9 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
   if (parts) *parts = 0;
   if (M == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  if (M > 16 && M <= 64 && w_strip) {
-    return gated ? launch_mid<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s)
-                 : launch_mid<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, wsp, parts, s);
+  if (w_strip && M <= 64 && (M > 16 || mid_for_few(gated, N, K, parts != nullptr && joinable_by_reader(N, ldc, c_is_f32, epi)))) {
+    return gated ? launch_mid<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s)
+                 : launch_mid<false>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s);
   }
   if (M <= 64) {
     return gated ? launch_skinny<true>(A, lda, W, C, ldc, c_is_f32, M, N, K, epi, cap, w_strip, wsp, parts, s)

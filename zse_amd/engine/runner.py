@@ -96,6 +96,9 @@ class Arena:
         return self.rt.empty(((nbytes + 3) // 4,), F32)
 
 
+MEMORY_SIDE_CACHE = 256 << 20       # bytes
+
+
 class StepContext:
     """What parts see of a step."""
 
@@ -109,6 +112,7 @@ class StepContext:
         self.arena = runner.arena
         self.workspace = runner.workspace
         self.gemm_workspace = runner.gemm_workspace
+        self.weights_read_once = runner.weights_read_once
         self.T = 0
         self.R = 0
         self.tokens = self.positions = self.req_of_token = self.q_start = self.ctx_len = 0
@@ -260,6 +264,8 @@ class StepRunner:
             raise RuntimeError(f"the kernels' workspace for {self.max_seqs} requests of up to "
                                f"{self.max_model_len} tokens needs {need} bytes and cannot be "
                                f"allocated: {e}") from None
+        # a model larger than the cache on the memory's side leaves nothing of a step's weights there for the next step
+        self.weights_read_once = getattr(model, "weight_bytes", 0) > MEMORY_SIDE_CACHE
         self.gemm_workspace = None
         if self.dtype == BF16 and self.k.has("zk_gemm_bf16_workspace"):
             self.gemm_workspace = rt.zeros((self.k.zk_gemm_bf16_workspace() // 4,), F32)

@@ -20,7 +20,7 @@ import numpy as np
 from ..config.plan import ShortConvSpec
 from ..runtime.device import BF16, ITEMSIZE, Tensor
 from .base import ROLE_GAIN, PagedKV, Part, TensorReq, build_part, register_part
-from .ops import linear, tuned_gemm
+from .ops import linear, strip_flag, tuned_gemm
 
 
 class PagedAttention(Part):
@@ -335,7 +335,7 @@ class PagedAttention(Part):
             # few decoded tokens: the product rotates and stores its own results
             qkv = ctx.alloc((T, width))
             k.zk_qkv_rope_bf16(x.ptr, s.hidden_size, self.w_qkv.ptr, qkv.ptr, width, T, s.hidden_size,
-                               1 if self.w_qkv.layout == "strip" else 0, ctx.positions,
+                               strip_flag(ctx, self.w_qkv), ctx.positions,
                                None if self.shared_kv else g.slot_map, tables[0].ptr, cache.k.ptr,
                                cache.v.ptr, nh, n_store, hd, g.page_size, 1 if cache.v_transposed else 0,
                                ctx.stream)

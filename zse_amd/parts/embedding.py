@@ -15,7 +15,7 @@ import numpy as np
 
 from ..runtime.device import BF16, F32, Tensor
 from .base import Part, TensorReq, build_part, register_part
-from .ops import linear, tuned_gemm
+from .ops import linear, strip_flag, tuned_gemm
 
 
 class Embedding(Part):
@@ -125,7 +125,7 @@ class LMHead(Part):
         ``forward`` followed by the argmax kernel gives."""
         s = self.spec
         ctx.k.zk_head_pick_bf16(x.ptr, s.hidden_size, self.weight.ptr, x.shape[0], s.vocab_size, s.hidden_size,
-                                float(s.softcap) if s.softcap else 0.0, 1 if self.weight.layout == "strip" else 0,
+                                float(s.softcap) if s.softcap else 0.0, strip_flag(ctx, self.weight),
                                 scratch.ptr, scratch.nbytes, ids.ptr, ctx.stream)
         return ids
 

@@ -16,6 +16,14 @@ def tuned_gemm(ctx, K: int) -> bool:
     return ctx.dtype == BF16 and ctx.tuned and ctx.k.has("zk_gemm_bf16") and K % 8 == 0
 
 
+def strip_flag(ctx, w: Tensor) -> int:
+    """How a matrix-core product of few rows reads ``w``: 0 row by row, 1 in strips, 3 in strips and past the caches
+    (``ctx.weights_read_once``: a step finds nothing there of what the last one read)."""
+    if w.layout != "strip":
+        return 0
+    return 3 if getattr(ctx, "weights_read_once", False) else 1
+
+
 def linear(ctx, x: Tensor, w: Tensor, out: Tensor, epilogue=None, cap: float = 0.0, last_of=None,
            sums_ok: bool = False, lda: int = 0, ldc: int = 0) -> Tensor:
     """out[M, N] = x[M, K] @ w[N, K]^T with float accumulation.
@@ -71,7 +79,7 @@ def linear(ctx, x: Tensor, w: Tensor, out: Tensor, epilogue=None, cap: float = 0
         welcome = sums_ok or (last_of is not None and getattr(ctx, "sums_welcome", None) is last_of)
         parts = ctypes.c_int(0) if (welcome and ws is not None) else None
         k.zk_gemm_bf16(x.ptr, lda, w.ptr, out.ptr, ldc, out_f32, M, N, K, EPILOGUES[epilogue], float(cap),
-                       1 if strip else 0, ws.ptr if ws is not None else None,
+                       strip_flag(ctx, w), ws.ptr if ws is not None else None,
                        ws.nbytes if ws is not None else 0, ctypes.byref(parts) if parts is not None else None,
                        ctx.stream)
         if parts is not None and parts.value > 0:
