@@ -24,6 +24,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 // Where a product that splits K over blocks leaves its partial sums.  ``strict``: the split is
 // chosen as for the standard workspace (so that the bits do not depend on who brought the
@@ -134,6 +135,134 @@ __device__ __forceinline__ bf16x8 load_weights(const void* p) {
   return ONCE ? load_once((const bf16x8*)p) : *(const bf16x8*)p;
 }
 
+// ------------------------------------------------------------------ the norm in front of a product of one row
+// h_out = h + post(sub) and the row next(h_out), as zk_norm_add_norm makes them, to the bit: sub as activations or ``parts`` planes of
+// float sums.  Every block of the product works the row out for itself, while its first weights are on their way, and the first
+// block stores h_out (elsewhere than h, which the others are still reading).
+//
+// What it saves is a launch that waits for memory twice and that everything behind it waits for; what it costs is the row's planes read
+// by every CU from its L2, which is why it is for one row only (5 planes of 2,304 sums are 55 KB a block).  A step of one decoded token,
+// us: six layers of width 1,024 204 -> 184, the 2B shapes 1,565 -> 1,514.
+struct RowNorm {
+  const void* sub;
+  const float* w_post;
+  const float* h;
+  float* h_out;
+  const float* w_next;
+  float eps_post, eps_next;
+  int parts, uo_post, uo_next, H;
+};
+
+// h + x g, rounded in between: as the norm's kernels, where the post norm may be missing, round.
+__device__ __forceinline__ float row_joined(float h, float x, float g) {
+#pragma clang fp contract(off)
+  const float y = x * g;
+  return h + y;
+}
+
+__device__ __forceinline__ f32x4 load4_act(const __bf16* p) {
+  const bf16x4 x = *(const bf16x4*)p;
+  return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
+}
+
+// The sums run as in norm_add_norm_wide_kernel (WIDE, H >= 2,048: 16 waves, a vector of four a thread) or norm_add_norm_fast_kernel (4
+// waves, up to two vectors a thread), whose waves this block's NW waves take in turn, SLOTS each.  H a multiple of 256.  PL: 0, or as many planes asked for (parts <= PL).
+// Two halves, because loads come back in the order in which they were asked for: what the row is made of first, then (by the caller) the first
+// weights, then the sums, which wait for the former alone.  All that forks is fixed at compile time: with branches on the planes and the width the compiler
+// waits for every load and keeps rows in scratch memory (4,096 columns of K 2,304 8.0 and 9.1 us in a trace of a step).
+template <int NW, int SLOTS, bool WIDE, int PL>
+struct RowInWork {
+  static_assert(WIDE ? NW * SLOTS <= 16 || SLOTS <= 2 : NW == 4 && SLOTS <= 2, "every wave of the kernels above has a place");
+  f32x4 v[SLOTS], t[SLOTS][PL > 1 ? PL - 1 : 1], hv[SLOTS], gp[SLOTS], gn[SLOTS];
+
+  // Slot s of this wave: place (wave + s NW) of the wide kernel, or vector s of the narrow one's wave.  Below H for whole waves or not at all.
+  static __device__ __forceinline__ int at(int s) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return WIDE ? (wave + s * NW) * 256 + lane * 4 : wave * 256 + lane * 4 + s * 1024;
+  }
+  static __device__ __forceinline__ bool in(const RowNorm& p, int s) { return __builtin_amdgcn_readfirstlane(at(s)) < p.H; }
+
+  __device__ __forceinline__ void ask(const RowNorm& p) {
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++) {
+      if (!in(p, s)) continue;
+      const int i = at(s);
+      if constexpr (PL == 0) {
+        v[s] = load4_act((const __bf16*)p.sub + i);
+      } else {
+        const float* sf = (const float*)p.sub + i;
+        v[s] = *(const f32x4*)sf;
+#pragma unroll
+        for (int q = 1; q < PL; q++) t[s][q - 1] = *(const f32x4*)(sf + (size_t)min(q, p.parts - 1) * p.H);
+      }
+      hv[s] = *(const f32x4*)(p.h + i);
+      gp[s] = *(const f32x4*)(p.w_post + i);
+      gn[s] = *(const f32x4*)(p.w_next + i);
+    }
+  }
+
+  // the sum of squares as the kernels above have it: a thread's own in order, a wave's by permutations, the waves' in LDS
+  __device__ __forceinline__ float total(const RowNorm& p, float* scratch) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float ss = 0.f;
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++) {
+      if (WIDE) ss = 0.f;
+      if (in(p, s)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) ss += v[s][e] * v[s][e];
+      }
+      if (WIDE) {
+        const float w = wave_sum_whole(ss);
+        if (lane == 0 && in(p, s)) scratch[wave + s * NW] = w;
+      }
+    }
+    if (!WIDE) {
+      const float w = wave_sum_whole(ss);
+      if (lane == 0) scratch[wave] = w;
+    }
+    __syncthreads();
+    // (places without values would add nothing)
+    return wave_sum16((lane & 15) < (WIDE ? p.H / 256 : 4) ? scratch[lane & 15] : 0.f);
+  }
+
+  // ``row``: H values in LDS, red: 32 floats there; every thread of the block, which may read the row afterwards
+  __device__ __forceinline__ void make(const RowNorm& p, __bf16* __restrict__ row, float* __restrict__ red, bool store_h) {
+    if constexpr (PL > 0) {
+#pragma unroll
+      for (int s = 0; s < SLOTS; s++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+#pragma unroll
+          for (int q = 1; q < PL; q++) v[s][e] = q < p.parts ? v[s][e] + t[s][q - 1][e] : v[s][e];
+          v[s][e] = (float)(__bf16)v[s][e];
+        }
+    }
+    const float rs = rsqrtf(total(p, red) / (float)p.H + p.eps_post);
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        v[s][e] = row_joined(hv[s][e], v[s][e] * rs, p.uo_post ? 1.f + gp[s][e] : gp[s][e]);
+      }
+    const float rs2 = rsqrtf(total(p, red + 16) / (float)p.H + p.eps_next);
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++) {
+      if (!in(p, s)) continue;
+      bf16x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; e++) y[e] = (__bf16)(v[s][e] * rs2 * (p.uo_next ? 1.f + gn[s][e] : gn[s][e]));
+      *(bf16x4*)(row + at(s)) = y;
+      if (store_h) *(f32x4*)(p.h_out + at(s)) = v[s];
+    }
+    __syncthreads();
+  }
+};
+// The kernels' template argument: none, or slots + 8 WIDE + 16 PL.
+constexpr int row_norm_mode(int slots, bool wide, int pl) { return slots + 8 * wide + 16 * pl; }
+template <int NW, int MODE>
+using RowOf = RowInWork<MODE ? NW : 4, MODE ? MODE % 8 : 1, MODE ? MODE / 8 % 2 != 0 : false, MODE / 16>;
+
 // ------------------------------------------------------------------ skinny
 // What the q|k|v product of decoded tokens does with its results instead of storing them all:
 // q and k heads are rotated (pairs (i, i + hd/2), angle position * inv_freq[i]), q goes to C,
@@ -160,6 +289,7 @@ __device__ __forceinline__ void store4(__bf16* dst, const float (&x)[4]) {
 // meet in lanes 32 apart; the results are finished as RopeStore says.  Every result is rounded
 // to 16 bits before it is rotated, as the separate product and rotation kernels do, so a
 // token's keys are the same bits whichever way it came.
+// NORM (one row): the kernel makes the row it multiplies itself (RowInWork), so that a step of one token has no launch between two products.
 // EXACT (weights in strip layout, so K is a whole number of 32-wide steps): no load is under a
 // condition.  A step past the wave's run reads the run's last step again and its weights are
 // set to zero afterwards; a row past M reads row M - 1 (its results are never stored).  Only so
@@ -173,13 +303,17 @@ __device__ __forceinline__ void store4(__bf16* dst, const float (&x)[4]) {
 // front of its loads (us, 8 rows: 4,096 columns of K 2,304 6.3 -> 5.5, 2,304 of 2,048
 // 5.0 -> 4.4, 2,304 of 9,216 13.3 -> 12.4; a step of 8 decoded tokens of the 2B shapes 2,319 -> 2,278).  The same sums.
 // ONCE (WHOLE): weights by loads that leave no trace in the caches (reads_once).
-template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false, bool WHOLE = false, bool ONCE = false>
+template <int MT, bool GATED, int NW, bool ROPE = false, bool EXACT = false, bool SPLIT = false, bool WHOLE = false, bool ONCE = false, int NORM = 0>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __restrict__ A, int lda,
                                                           const __bf16* __restrict__ W,
                                                           void* __restrict__ C, int ldc, int c_is_f32,
                                                           int M, int N, int K, int epi, float cap,
                                                           int w_strip, RopeStore rs,
-                                                          float* __restrict__ partials = nullptr, int ksplit = 1) {
+                                                          float* __restrict__ partials = nullptr, int ksplit = 1,
+                                                          RowNorm norm = RowNorm{}) {
+  static_assert(!NORM || (WHOLE && !SPLIT), "a row made here is multiplied whole");
+  __shared__ __align__(16) __bf16 own_row[NORM ? 4096 : 8];
+  __shared__ float own_sums[NORM ? 32 : 1];
   static_assert(!ROPE || (MT == 1 && !GATED), "the rotating epilogue takes up to 16 rows");
   static_assert(!WHOLE || (EXACT && MT == 1), "whole groups: strips, up to 16 rows");
   constexpr int NS = GATED ? 2 : 1;
@@ -264,8 +398,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
 #pragma unroll
         for (int s = 0; s < STEPS; s++) wf[g][s] = load_weights<ONCE>((s < 4 ? lo + s * 1024 : hi + (s - 4) * 1024) + wlane);
       }
+      if (!NORM) {
 #pragma unroll
-      for (int s = 0; s < STEPS; s++) af[0][s] = *(const bf16x8*)(a + s * 64 + alane);
+        for (int s = 0; s < STEPS; s++) af[0][s] = *(const bf16x8*)(a + s * 64 + alane);
+      }
       return;
     }
     if (EXACT) {
@@ -300,6 +436,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
       for (int g = 0; g < NS; g++) wf[g][s] = in ? *(const bf16x8*)(wp[g] + (size_t)(s0 + s) * wstep) : zero8();
     }
   };
+  int at_step = run_lo;        // (NORM) the step of A that the next product takes
   auto multiply = [&](const bf16x8 (&wf)[NS][STEPS], const bf16x8 (&af)[MT][STEPS]) {
 #pragma unroll
     for (int s = 0; s < STEPS; s++)
@@ -307,9 +444,16 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
       for (int g = 0; g < NS; g++)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++)
-          acc[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af[mt][s], acc[g][mt], 0, 0, 0);
+          acc[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[g][s], NORM ? *(const bf16x8*)(own_row + (at_step + s) * 32 + kq * 8) : af[mt][s], acc[g][mt], 0, 0, 0);
+    if (NORM != 0) at_step += STEPS;
   };
   bf16x8 wf0[NS][STEPS], af0[MT][STEPS], wf1[NS][STEPS], af1[MT][STEPS];
+  RowOf<NW, NORM> own;
+  if constexpr (NORM != 0) {
+    own.ask(norm);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if (EXACT) {
     if (gw0 < gw1) fetch(0, wf0, af0);
   } else if (s_begin < s_end) {
@@ -326,6 +470,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
       sincosf((float)rs.positions[min(r, M - 1)] * rs.inv_freq[hpos + 4 * (kq & 1) + wave], &sn, &cs);
       turn[wave][lane] = make_float2(sn, cs);
     }
+  }
+  if constexpr (NORM != 0) {
+    __builtin_amdgcn_sched_barrier(0);
+    own.make(norm, own_row, own_sums, blockIdx.x == 0);
   }
   if (EXACT) {
     // The wave's run is a whole number of groups [gw0, gw1).  In the loop every product follows
@@ -1057,6 +1205,68 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   }
 }
 
+// The gated product of the kernel above for one row that it makes itself (RowInWork): the same sums, but the row lies in LDS whole, so the waves
+// never meet in the loop, and six chunks' weights are on their way.
+template <int SPB, int KW, int CH, bool ONCE, int NORM>
+__global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf16* __restrict__ W, __bf16* __restrict__ C, int N, int K,
+                                                                      int epi, RowNorm norm) {
+  constexpr int NW = SPB * KW, WSTEPS = CH / KW, DEPTH = 6;
+  __shared__ __align__(16) __bf16 row[4096 + CH * 32];
+  __shared__ float red[32];
+  __shared__ f32x4 sums[NW][2][64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int place = wave % SPB, kpart = wave / SPB, kq = lane >> 4;
+  const int ksteps = K / 32, nstrips = N / 16;
+  const int strip = blockIdx.x * SPB + place, strip_read = min(strip, nstrips - 1);
+  const __bf16* wp[2] = {W + (size_t)strip_read * ksteps * 512 + lane * 8, W + (size_t)(nstrips + strip_read) * ksteps * 512 + lane * 8};
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  bf16x8 w[DEPTH][2][WSTEPS];
+  // (steps past the end read the last one again; the row is zero there)
+  auto fetch = [&](int s0, bf16x8 (&wf)[2][WSTEPS]) {
+#pragma unroll
+    for (int s = 0; s < WSTEPS; s++)
+#pragma unroll
+      for (int g = 0; g < 2; g++) wf[g][s] = load_weights<ONCE>(wp[g] + (size_t)min(s0 + kpart * WSTEPS + s, ksteps - 1) * 512);
+  };
+  auto multiply = [&](int s0, const bf16x8 (&wf)[2][WSTEPS]) {
+#pragma unroll
+    for (int s = 0; s < WSTEPS; s++) {
+      const bf16x8 af = *(const bf16x8*)(row + (s0 + kpart * WSTEPS + s) * 32 + kq * 8);
+#pragma unroll
+      for (int g = 0; g < 2; g++) acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af, acc[g], 0, 0, 0);
+    }
+  };
+  RowOf<NW, NORM> own;
+  own.ask(norm);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int d = 0; d < DEPTH - 1; d++) fetch(d * CH, w[d]);
+  __builtin_amdgcn_sched_barrier(0);
+  for (int i = K + tid * 8; i < K + CH * 32; i += NW * 64 * 8) *(bf16x8*)(row + i) = zero8();
+  own.make(norm, row, red, blockIdx.x == 0);
+  for (int s0 = 0; s0 < ksteps;) {
+#pragma unroll
+    for (int d = 0; d < DEPTH; d++) {
+      fetch(s0 + (DEPTH - 1) * CH, w[(d + DEPTH - 1) % DEPTH]);
+      multiply(s0, w[d]);
+      s0 += CH;
+      if (s0 >= ksteps) break;
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 2; g++) sums[place * KW + kpart][g][lane] = acc[g];
+  __syncthreads();
+  if (kpart > 0 || strip >= nstrips) return;
+  f32x4 v[2];
+#pragma unroll
+  for (int g = 0; g < 2; g++) {
+    v[g] = sums[place * KW][g][lane];
+#pragma unroll
+    for (int k = 1; k < KW; k++) v[g] += sums[place * KW + k][g][lane];
+  }
+  mid_store<true>(v[0], v[1], lane & 15, C, N, 0, 1, N, strip, lane, epi, 0.f, nullptr, nstrips);
+}
+
 // Four neighbouring results of a row, in one store where the address allows it.
 __device__ __forceinline__ void store_quad(void* __restrict__ C, int ldc, int c_is_f32, int m, int n, int N, const float (&v)[4]) {
   if (!c_is_f32 && n + 4 <= N && ldc % 4 == 0 && (uintptr_t)C % 8 == 0) {
@@ -1353,6 +1563,100 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
   }
 #undef ZK_QKV
   return zk_launch_status("zk_qkv_rope_bf16");
+}
+
+// The two products behind a norm, for one row that the product makes itself: what zk_norm_add_norm (sub, up to 6 planes, w_post, h, w_next) followed by zk_qkv_rope_bf16, or by zk_gemm_bf16 with a gated epilogue, gives, to the bit.  h_out: the new stream,
+// elsewhere than h.  sub must not lie where the product writes.  Weights in strips, K a multiple of 256 up to 4,096.
+static int row_norm_of(RowNorm& p, const void* sub, int sub_parts, const float* w_post, float eps_post, int uo_post, const float* h, float* h_out,
+                       const float* w_next, float eps_next, int uo_next, int K) {
+  ZK_REQUIRE(K > 0 && K % 256 == 0 && K <= 4096, "zk_norm product: K must be a multiple of 256 up to 4096");
+  ZK_REQUIRE(sub_parts >= 0 && sub_parts <= 6, "zk_norm product: up to 6 planes of partial sums");
+  ZK_REQUIRE(sub && h && h_out && w_post && w_next && h != h_out, "zk_norm product: sub, h, another h_out, w_post and w_next are needed");
+  ZK_REQUIRE((((uintptr_t)sub | (uintptr_t)h | (uintptr_t)h_out | (uintptr_t)w_next | (uintptr_t)w_post) & 15) == 0,
+             "zk_norm product: operands must be 16-byte aligned");
+  p = RowNorm{sub, w_post, h, h_out, w_next, eps_post, eps_next, sub_parts, uo_post, uo_next, K};
+  return 0;
+}
+
+// N: the gated product's columns (0: the rotating product)
+extern "C" int zk_norm_product_supports(int N, int K, int sub_parts) {
+  return K > 0 && K % 256 == 0 && K <= 4096 && sub_parts <= 6 && (N == 0 || K >= 2048 || !mid_for_few(true, N, K, false));
+}
+
+#define ZK_NORM_MODES(NW_, SLOTS_, WIDE_)                                                          \
+  do {                                                                                             \
+    if (reads_once(w_strip)) {                                                                     \
+      if (sub_parts == 0) ZK_LAUNCH(NW_, true, row_norm_mode(SLOTS_, WIDE_, 0));                   \
+      else if (sub_parts <= 4) ZK_LAUNCH(NW_, true, row_norm_mode(SLOTS_, WIDE_, 4));              \
+      else ZK_LAUNCH(NW_, true, row_norm_mode(SLOTS_, WIDE_, 6));                                  \
+    } else {                                                                                       \
+      if (sub_parts == 0) ZK_LAUNCH(NW_, false, row_norm_mode(SLOTS_, WIDE_, 0));                  \
+      else if (sub_parts <= 4) ZK_LAUNCH(NW_, false, row_norm_mode(SLOTS_, WIDE_, 4));             \
+      else ZK_LAUNCH(NW_, false, row_norm_mode(SLOTS_, WIDE_, 6));                                 \
+    }                                                                                              \
+  } while (0)
+
+extern "C" int zk_norm_qkv_rope_bf16(const void* sub, int sub_parts, const float* w_post, float eps_post, int uo_post, const float* h,
+                                     void* h_out, const float* w_next, float eps_next, int uo_next, const void* W, void* Q, int ldq,
+                                     int K, int w_strip, const int* positions, const int* slot_map, const float* inv_freq, void* kcache,
+                                     void* vcache, int nh, int nkv, int hd, int bs, int v_transposed, void* stream) {
+  RowNorm p;
+  if (int rc = row_norm_of(p, sub, sub_parts, w_post, eps_post, uo_post, h, (float*)h_out, w_next, eps_next, uo_next, K)) return rc;
+  ZK_REQUIRE(w_strip, "zk_norm_qkv_rope_bf16: weights in strips");
+  ZK_REQUIRE(nh > 0 && nkv >= 0 && hd > 0 && hd % 16 == 0, "zk_norm_qkv_rope_bf16: head_dim must be a multiple of 16");
+  ZK_REQUIRE(ldq >= nh * hd && ldq % 4 == 0, "zk_norm_qkv_rope_bf16: ldq too small or not a multiple of 4");
+  ZK_REQUIRE(positions && inv_freq, "zk_norm_qkv_rope_bf16: positions and inv_freq are needed");
+  ZK_REQUIRE(nkv == 0 || (slot_map && kcache && vcache && bs > 0), "zk_norm_qkv_rope_bf16: the cache is needed");
+  ZK_REQUIRE((uintptr_t)W % 16 == 0 && (uintptr_t)Q % 8 == 0, "zk_norm_qkv_rope_bf16: operands must be 16-byte aligned");
+  const int N = (nh + 2 * nkv) * hd;
+  RopeStore rs{positions, nkv ? slot_map : nullptr, inv_freq, (__bf16*)kcache, (__bf16*)vcache, nh, nkv, hd, bs, v_transposed};
+  dim3 grid(N / 16);
+  hipStream_t s = (hipStream_t)stream;
+#define ZK_LAUNCH(NW_, ONCE_, MODE_)                                                                                           \
+  gemm_skinny_kernel<1, false, NW_, true, true, false, true, ONCE_, MODE_><<<grid, NW_ * 64, 0, s>>>(                           \
+      nullptr, K, (const __bf16*)W, Q, ldq, 0, 1, N, K, EPI_NONE, 0.f, w_strip, rs, nullptr, 1, p)
+  // as zk_qkv_rope_bf16: eight waves for few long strips, else four
+  if (grid.x < 512 && K >= 2048) ZK_NORM_MODES(8, 2, true);
+  else if (K >= 2048) ZK_NORM_MODES(4, 4, true);
+  else if (K > 1024) ZK_NORM_MODES(4, 2, false);
+  else ZK_NORM_MODES(4, 1, false);
+#undef ZK_LAUNCH
+  return zk_launch_status("zk_norm_qkv_rope_bf16");
+}
+
+extern "C" int zk_norm_gated_bf16(const void* sub, int sub_parts, const float* w_post, float eps_post, int uo_post, const float* h,
+                                  void* h_out, const float* w_next, float eps_next, int uo_next, const void* W, void* C, int N, int K,
+                                  int epi, int w_strip, void* stream) {
+  RowNorm p;
+  if (int rc = row_norm_of(p, sub, sub_parts, w_post, eps_post, uo_post, h, (float*)h_out, w_next, eps_next, uo_next, K)) return rc;
+  ZK_REQUIRE(w_strip && N > 0 && N % 16 == 0, "zk_norm_gated_bf16: weights in strips, N a multiple of 16");
+  ZK_REQUIRE(epi == EPI_GELU_TANH || epi == EPI_SILU || epi == EPI_RELU, "zk_norm_gated_bf16: not a gated epilogue without a limit");
+  ZK_REQUIRE((uintptr_t)W % 16 == 0 && (uintptr_t)C % 16 == 0, "zk_norm_gated_bf16: operands must be 16-byte aligned");
+  hipStream_t s = (hipStream_t)stream;
+  if (mid_for_few(true, N, K, false)) {
+    // as launch_mid for up to 16 rows: 513 to 1,024 strips, three or four a block
+    const MidCut cut = mid_cut(true, 1, N, K, false);
+    dim3 grid((N / 16 + cut.spb - 1) / cut.spb);
+    ZK_REQUIRE(K >= 2048 && (cut.spb == 3 || cut.spb == 4), "zk_norm_gated_bf16: no kernel for so many strips of this length");
+#define ZK_LAUNCH(NW_, ONCE_, MODE_)                                                                                                     \
+  gemm_mid_norm_kernel<NW_ == 12 ? 3 : 4, NW_ == 12 ? 4 : 2, 4, ONCE_, MODE_><<<grid, NW_ * 64, 0, s>>>((const __bf16*)W, (__bf16*)C, N, K, epi, p)
+    if (cut.spb == 4) ZK_NORM_MODES(8, 2, true);
+    else if (K > 3072) ZK_NORM_MODES(12, 2, true);
+    else ZK_NORM_MODES(12, 1, true);
+#undef ZK_LAUNCH
+    return zk_launch_status("zk_norm_gated_bf16 (mid)");
+  }
+  // as launch_skinny
+  dim3 grid(N / 16);
+#define ZK_LAUNCH(NW_, ONCE_, MODE_)                                                                                  \
+  gemm_skinny_kernel<1, true, NW_, false, true, false, true, ONCE_, MODE_><<<grid, NW_ * 64, 0, s>>>(                  \
+      nullptr, K, (const __bf16*)W, C, N, 0, 1, N, K, epi, 0.f, w_strip, RopeStore{}, nullptr, 1, p)
+  if ((long)grid.x < 512 && K >= 2048) ZK_NORM_MODES(8, 2, true);
+  else if (K >= 2048) ZK_NORM_MODES(4, 4, true);
+  else if (K > 1024) ZK_NORM_MODES(4, 2, false);
+  else ZK_NORM_MODES(4, 1, false);
+#undef ZK_LAUNCH
+  return zk_launch_status("zk_norm_gated_bf16 (skinny)");
 }
 
 // Strip layout of a [N, K] weight matrix, K % 32 == 0: rows in strips of 16 (the last strip

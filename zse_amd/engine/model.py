@@ -157,6 +157,8 @@ class Model:
         # (gathered a second time: a launch like any other, which a captured or written-down step repeats)
         first = self.embedding.forward(ctx) if again else None
         ctx.lent = {key: ctx.alloc((T, channels)) for key, channels in self.lent.items()}
+        # a second row for the stream of a single token: its products may make their own norms (see PendingNorm)
+        ctx.spare_stream = ctx.alloc((1, H), h.dtype) if T == 1 else None
         x = None
         base = ctx.arena.mark()
         cache_for = lambda i: caches[i] if caches[i].shared else caches[order[i].cache_of if order[i].cache_of is not None else i]
@@ -167,6 +169,7 @@ class Model:
             nxt = self.blocks[order[i + 1].layer] if i + 1 < len(order) else None
             if nxt is not None and getattr(order[i + 1], "add_embedding", False):
                 nxt = None           # the stream changes between the two entries: the next one norms it itself
+            ctx.next_block = nxt
             if getattr(call, "add_embedding", False):
                 x = self._add_embedding(ctx, h, first, blk, handoff[(i + 1) % 2])
             if hasattr(blk, "entry_norm"):

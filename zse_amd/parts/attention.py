@@ -20,7 +20,7 @@ import numpy as np
 from ..config.plan import ShortConvSpec
 from ..runtime.device import BF16, ITEMSIZE, Tensor
 from .base import ROLE_GAIN, PagedKV, Part, TensorReq, build_part, register_part
-from .ops import linear, strip_flag, tuned_gemm
+from .ops import PendingNorm, linear, strip_flag, tuned_gemm
 
 
 class PagedAttention(Part):
@@ -319,6 +319,15 @@ class PagedAttention(Part):
                 k.zk_add_bias(y.ptr, self.o_bias.ptr, T, s.hidden_size, ctx.stream)
         return y
 
+    def takes_pending_norm(self, ctx, size: int, planes: int) -> bool:
+        """Whether the product of one row that rotates and stores its results serves this mixer (and then makes its own norm)."""
+        s, tables = self.spec, self.position.rotary_tables()
+        return bool(not self.general and type(self).forward is PagedAttention.forward and size == s.hidden_size and
+                    type(self).between_product_and_rotation is PagedAttention.between_product_and_rotation and
+                    tables is not None and tuned_gemm(ctx, s.hidden_size) and self.w_qkv.layout == "strip" and
+                    ctx.k.zk_qkv_rope_bf16_supports(1, s.hidden_size, s.head_dim, tables[1]) and
+                    ctx.k.zk_norm_product_supports(0, size, planes))
+
     def forward(self, ctx, x: Tensor, cache) -> Tensor:
         if self.general:
             return self._forward_general(ctx, x, cache)
@@ -330,7 +339,13 @@ class PagedAttention(Part):
         g = ctx.group(cache.group)
         tables = self.position.rotary_tables()
         hooked = type(self).between_product_and_rotation is not PagedAttention.between_product_and_rotation
-        if (not hooked and tables is not None and tuned_gemm(ctx, s.hidden_size) and k.has("zk_qkv_rope_bf16")
+        if isinstance(x, PendingNorm):
+            qkv = ctx.alloc((T, width))
+            k.zk_norm_qkv_rope_bf16(*x.args(), self.w_qkv.ptr, qkv.ptr, width, s.hidden_size, strip_flag(ctx, self.w_qkv), ctx.positions,
+                                    None if self.shared_kv else g.slot_map, tables[0].ptr, cache.k.ptr, cache.v.ptr, nh, n_store, hd,
+                                    g.page_size, 1 if cache.v_transposed else 0, ctx.stream)
+            x.done()
+        elif (not hooked and tables is not None and tuned_gemm(ctx, s.hidden_size) and k.has("zk_qkv_rope_bf16")
                 and k.zk_qkv_rope_bf16_supports(T, s.hidden_size, hd, tables[1])):
             # few decoded tokens: the product rotates and stores its own results
             qkv = ctx.alloc((T, width))

@@ -13,6 +13,7 @@ from ..runtime.device import Tensor
 from ..config.plan import NoNormSpec
 from .base import Part, build_part, register_part
 from .norm import LayerNorm, NoNorm, RMSNorm
+from .ops import PendingNorm
 
 ARRANGEMENTS = {"sandwich": ("pre_mixer", "post_mixer", "pre_ffn", "post_ffn"),
                 "prenorm": ("pre_mixer", "pre_ffn"),
@@ -65,6 +66,15 @@ class Block(Part):
         return out
 
     @staticmethod
+    def _pending(ctx, sub: Tensor, post, h: Tensor, nxt, reader):
+        """The join as a row that ``reader``'s first product makes itself, where it does that; else None."""
+        if (isinstance(nxt, RMSNorm) and isinstance(post, RMSNorm) and hasattr(reader, "takes_pending_norm") and
+                PendingNorm.possible(ctx, h, sub) and
+                reader.takes_pending_norm(ctx, h.shape[1], sub.shape[0] if sub.layout == "parts" else 0)):
+            return PendingNorm(ctx, sub, post, h, nxt)
+        return None
+
+    @staticmethod
     def _joins_sums(post) -> bool:
         return post is None or isinstance(post, RMSNorm)
 
@@ -88,10 +98,18 @@ class Block(Part):
         if self.ffn is None:
             ctx.sums_welcome = None
             return self._join(ctx, a, n.get("post_mixer"), h, next_norm, x_out)
-        x = self._join(ctx, a, n.get("post_mixer"), h, n["pre_ffn"])
+        x = self._pending(ctx, a, n.get("post_mixer"), h, n["pre_ffn"], self.ffn)
+        if x is None:
+            x = self._join(ctx, a, n.get("post_mixer"), h, n["pre_ffn"])
         ctx.sums_welcome = self.ffn if self._joins_sums(n.get("post_ffn")) else None
         m = self.ffn.forward(ctx, x)
         ctx.sums_welcome = None
+        following = getattr(ctx, "next_block", None)
+        if m.layout == "parts" and next_norm is not None and isinstance(following, Block):
+            # (partial sums outlive this block's own memory)
+            x = self._pending(ctx, m, n.get("post_ffn"), h, next_norm, following.mixer)
+            if x is not None:
+                return x
         return self._join(ctx, m, n.get("post_ffn"), h, next_norm, x_out)
 
 

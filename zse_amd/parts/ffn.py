@@ -12,7 +12,7 @@ from typing import List
 
 from ..runtime.device import BF16, F32, I32, Tensor
 from .base import ROLE_GAIN, Part, TensorReq, build_part, register_part
-from .ops import linear, tuned_gemm
+from .ops import EPILOGUES, PendingNorm, linear, strip_flag, tuned_gemm
 
 ACTIVATION_CODES = {"gelu_tanh": 0, "silu": 1, "relu": 2}
 CLAMPED = "clamped_swiglu"     # g = min(gate, limit), u = clamp(up, +-limit): g sigmoid(1.702 g) (u + 1)
@@ -44,12 +44,25 @@ class GatedMLP(Part):
         self.w_down = (weights.matrix([s.names["down"]], strip=True) if strip and strip(s.intermediate_size)
                        else weights.matrix([s.names["down"]]))
 
+    def takes_pending_norm(self, ctx, size: int, planes: int) -> bool:
+        """Whether the first product makes its own norm for one row."""
+        s = self.spec
+        return bool(type(self).forward is GatedMLP.forward and size == s.hidden_size and s.activation != CLAMPED and
+                    tuned_gemm(ctx, s.hidden_size) and self.w_gu.layout == "strip" and s.intermediate_size % 16 == 0 and
+                    ctx.k.zk_norm_product_supports(s.intermediate_size, size, planes))
+
     def forward(self, ctx, x: Tensor, out: Tensor = None) -> Tensor:
         """``out``: where the result goes (activations or float32 [T, hidden]); the product that
         ends the layer then never hands partial sums back."""
         s = self.spec
         T, I = x.shape[0], s.intermediate_size
         last = None if out is not None else self
+        if isinstance(x, PendingNorm):
+            a = ctx.alloc((T, I))
+            ctx.k.zk_norm_gated_bf16(*x.args(), self.w_gu.ptr, a.ptr, I, s.hidden_size, EPILOGUES[s.activation],
+                                     strip_flag(ctx, self.w_gu), ctx.stream)
+            x.done()
+            return linear(ctx, a, self.w_down, out if out is not None else ctx.alloc((T, s.hidden_size)), last_of=last)
         if s.activation == CLAMPED and tuned_gemm(ctx, s.hidden_size):
             # the activation in the product's epilogue, on the float sums
             a = linear(ctx, x, self.w_gu, ctx.alloc((T, I)), epilogue=CLAMPED, cap=float(s.limit))

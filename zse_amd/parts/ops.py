@@ -24,6 +24,34 @@ def strip_flag(ctx, w: Tensor) -> int:
     return 3 if getattr(ctx, "weights_read_once", False) else 1
 
 
+class PendingNorm:
+    """One row that is not made yet: next(h + post(sub)).  The product that reads it makes it itself and stores the
+    new stream beside the old one, and a step of one token has a launch less between two products.  A block hands it only to a
+    part whose ``takes_pending_norm(ctx, size, planes)`` says yes; the part launches one product with ``args`` and then calls ``done``.
+    ``sub`` lies where nothing that runs before that product, nor the product itself, writes."""
+
+    def __init__(self, ctx, sub: Tensor, post, h: Tensor, nxt):
+        self.sub, self.post, self.h, self.nxt, self.spare = sub, post, h, nxt, ctx.spare_stream
+        self.shape, self.dtype, self.layout = h.shape, ctx.dtype, "pending"
+
+    @staticmethod
+    def possible(ctx, h: Tensor, sub: Tensor) -> bool:
+        return (h.shape[0] == 1 and ctx.dtype == BF16 and ctx.tuned and getattr(ctx, "spare_stream", None) is not None and
+                ctx.k.has("zk_norm_gated_bf16") and (sub.layout == "parts" or (sub.layout == "rows" and sub.dtype == BF16)))
+
+    def args(self):
+        """The leading arguments of the products that take one."""
+        post, nxt = self.post, self.nxt
+        return (self.sub.ptr, self.sub.shape[0] if self.sub.layout == "parts" else 0, post.weight.ptr,
+                float(post.spec.eps), int(post.spec.unit_offset), self.h.ptr,
+                self.spare.ptr, nxt.weight.ptr, float(nxt.spec.eps), int(nxt.spec.unit_offset))
+
+    def done(self) -> None:
+        """The stream lies in the spare row from here on, and the old row is the spare one."""
+        self.h.ptr, self.spare.ptr = self.spare.ptr, self.h.ptr
+        self.h.owner, self.spare.owner = self.spare.owner, self.h.owner
+
+
 def linear(ctx, x: Tensor, w: Tensor, out: Tensor, epilogue=None, cap: float = 0.0, last_of=None,
            sums_ok: bool = False, lda: int = 0, ldc: int = 0) -> Tensor:
     """out[M, N] = x[M, K] @ w[N, K]^T with float accumulation.

@@ -245,6 +245,9 @@ BF16_KERNEL_SIGNATURES = {
     "zk_strip_layout": [_VP, _VP, _I, _I, _VP],
     "zk_head_pick_bf16": [_VP, _I, _VP, _I, _I, _I, _F, _I, _VP, _SZ, _VP, _VP],
     "zk_probe_mfma_bf16": [_I, _VP, C.POINTER(C.c_double), _VP],
+    "zk_norm_qkv_rope_bf16": [_VP, _I, _VP, _F, _I, _VP, _VP, _VP, _F, _I, _VP, _VP, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I,
+                              _I, _VP],
+    "zk_norm_gated_bf16": [_VP, _I, _VP, _F, _I, _VP, _VP, _VP, _F, _I, _VP, _VP, _I, _I, _I, _I, _VP],
     "zk_qkv_rope_bf16": [_VP, _I, _VP, _VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "zk_attention_bf16": [_VP, _I, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I,
                           _F, _F, _I, _I, _VP, _SZ, _VP],
@@ -376,6 +379,9 @@ class KernelLibrary:
             self._dll.zk_qkv_rope_bf16_supports.restype = C.c_int
             self._dll.zk_qkv_rope_bf16_supports.argtypes = [_I, _I, _I, _I]
             self.zk_qkv_rope_bf16_supports = self._dll.zk_qkv_rope_bf16_supports
+            self._dll.zk_norm_product_supports.restype = C.c_int
+            self._dll.zk_norm_product_supports.argtypes = [_I, _I, _I]
+            self.zk_norm_product_supports = self._dll.zk_norm_product_supports
             self._dll.zk_head_pick_bf16_workspace.restype = C.c_size_t
             self._dll.zk_head_pick_bf16_workspace.argtypes = [_I, _I]
             self.zk_head_pick_bf16_workspace = self._dll.zk_head_pick_bf16_workspace
