@@ -318,14 +318,15 @@ __global__ __launch_bounds__(256) void norm_add_norm_fast_kernel(
   }
 }
 
-// The same for the few rows of a decode step (up to 64 rows of 2,048 to 8,192 values): 1,024
+// The same for rows of 2,048 to 8,192 values of which there are few, or which fill the threads: 1,024
 // threads a row instead of 256, so a thread holds one or two vectors (4 x 1024 x MAXV >= H) and can
 // ask for all planes of partial sums at once, eight a turn.  With so few rows the kernel's time is
 // its trips to memory and its two block sums, not its bytes: 8 rows of 4,608 values that come as
 // eight planes (27B shapes) 2.9 us less a launch, a decode step at batch 8 of 2B shapes 2.46 -> 2.42
-// ms, of 9B shapes (14 layers) 2.47 -> 2.40 ms, 2B shapes at batch 32 4.51 -> 4.40 ms; with 2,048
-// rows it loses (the 2B prefill 12.43 -> 12.75 ms), so more than 64 rows stay with the kernel
-// above.  The sums of the planes are the same bits; the two row sums are added up in another
+// ms, of 9B shapes (14 layers) 2.47 -> 2.40 ms, 2B shapes at batch 32 4.51 -> 4.40 ms.  us, 256 threads and 1,024, rows as activations: of
+// 2,304 values 65 rows 3.6 and 3.0, 256 4.4 and 3.9, 512 5.4 and 5.3, 768 6.1 and 7.2, 2,048 12.4 and 16.6 (9 waves of 16 have values);
+// of 3,584 (14 of 16) 441 to 512 7.3 and 6.6, 768 8.3 and 8.8, 1,024 12.1 and 10.5, 2,048 26.9 and 21.8; of 4,608 512 8.5 and 8.5, 2,048 39.3 and 34.1; of 2,048
+// 256 3.5 and 3.5, 384 4.4 and 4.6.  The sums of the planes are the same bits; the two row sums are added up in another
 // order than by 256 threads, so which of the two kernels serves a launch depends on the rows and
 // the width alone, never on whether planes come.
 template <int MAXV>
@@ -892,8 +893,8 @@ int zk_norm_add_norm(const void* sub, int sub_parts, const float* w_post, float 
   ZK_REQUIRE(T >= 0 && H > 0 && sub_parts >= 0, "zk_norm_add_norm: bad sizes");
   ZK_REQUIRE(w_next == nullptr || out != nullptr, "zk_norm_add_norm: next norm without output");
   if (T == 0) return 0;
-  if (ZSE_ACT_BF16 && T <= 64 && H % 4 == 0 && H >= 2048 && H <= 8192) {
-    // few rows of at least 2,048 values (see the kernel): a decode step's norms.  The 32-bit
+  if (ZSE_ACT_BF16 && H % 4 == 0 && H >= 2048 && H <= 8192 && (T <= 256 || (H > 2048 && T <= 512) || (H > 2560 && T >= 1024))) {
+    // few rows of at least 2,048 values, and many that fill the threads (see the kernel).  The 32-bit
     // library keeps to one kernel whatever the rows, so that its results stay the same bits
     // however a request's tokens are cut into steps.
     hipStream_t st = (hipStream_t)stream;
