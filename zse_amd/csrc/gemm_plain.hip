@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
 // Measured (us; before: 64 x 64 tiles of scalar multiply-adds through LDS, one block a tile):
 //   M = 303: 1024 x 4096 and 1024 x 1024 (average)  452 -> 42;  8192 x 1024  217 -> 87;
 //   1536 x 1024  191 -> 20;  M = 4: 32768 x 1024  207 -> 28.  By f32_tile's choice: 1024 x 4096 61 -> 41, 1024 x 1024
-//   18.7 -> 14.2, 8192 x 1024 86 -> 80, 1536 x 1024 19.3 -> 18.9.
+//   18.7 -> 14.2, 8192 x 1024 86 -> 67, 1536 x 1024 19.3 -> 17.2.
 // The error against 64 bits is no larger than the scalar sum's (eight shorter sums added up).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -253,9 +253,11 @@ static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc
 // More than sixteen rows, K of 512 or more: the tile with the least price.  A launch takes as many rounds as the CU
 // with the most blocks has, whatever a block's registers would allow (303 x 1024 x 4096: 320 blocks of 32 x 32 61 us, 224 of
 // 48 x 32 41): a block alone already takes what its CU gets from its L2.  Microseconds, fitted to 17 to 2,048
-// rows by thirteen weights (512 to 18,432 columns, K of 1,024 to 9,216): a round's start, and for every 1,024 of K
+// rows by thirteen weights (512 to 18,432 columns, K of 1,024 to 9,216; the last two to 64 to 303 rows, K of 1,024 and 4,096): a round's start, and for every 1,024 of K
 // one round's time and that of several.  The tile it names takes 1.009 times the best one's time in the mean and
-// 0.81 of that of 32 x 32 and 64 x 64 alone, 0.98 times the old rule's speed at the least.  The sums are the same bits.
+// 0.81 of that of 32 x 32 and 64 x 64 alone, 0.98 times the old rule's speed at the least.  The last two fill rounds that the others leave
+// half empty (us, without and with them: 303 x 8192 x 1024, 640 blocks of 64 x 64 or 512 of 80 x 64, 77.6 and 66.9; 150 rows 45 and 36;
+// 64 x 8192 x 1024, 256 blocks of 64 x 32, 20.8 and 18.3; 303 x 1536 x 1024 19.6 and 17.2).  The sums are the same bits.
 struct F32Tile { int mf, nf; double start, lone, several; };
 static const F32Tile f32_tiles[] = {
     {1, 1, 0.88, 3.65, 3.47},
@@ -264,7 +266,9 @@ static const F32Tile f32_tiles[] = {
     {3, 2, 2.54, 8.66, 8.68},
     {2, 3, 2.71, 8.94, 8.55},
     {3, 4, 0.00, 22.29, 21.65},
-    {4, 4, 2.23, 23.23, 22.63}};
+    {4, 4, 2.23, 23.23, 22.63},
+    {4, 2, -1.5, 16.1, 16.9},
+    {5, 4, 0.0, 32.7, 32.0}};
 static int f32_tile(int M, int N, int K) {
   int best = 0;
   double best_time = 1e30;
@@ -312,7 +316,9 @@ extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int
       case 3: return launch_f32<3, 2, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
       case 4: return launch_f32<2, 3, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
       case 5: return launch_f32<3, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
-      default: return launch_f32<4, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 6: return launch_f32<4, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 7: return launch_f32<4, 2, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      default: return launch_f32<5, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
     }
   }
   if (M > 16 && blocks(4, 4) >= 1024) return launch_f32<4, 4, 1, 3>(a, lda, w, (float*)C, ldc, M, N, K, s);
