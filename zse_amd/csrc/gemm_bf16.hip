@@ -283,6 +283,41 @@ __device__ __forceinline__ void store4(__bf16* dst, const float (&x)[4]) {
   *(bf16x4*)dst = o;
 }
 
+// A lane's results 4 kq + i of a strip of 16, row m: lanes 0..31 hold places hpos + 4 kq + i of the
+// head's first half, lanes 32..63 their partners in the second.  sn, cs: of the lane's four angles.  All 64 lanes call it.
+__device__ __forceinline__ void rope_store(const RopeStore& rs, const f32x4& v, int m, int M, int lane, int head, int hpos, int slot,
+                                           const float (&sn)[4], const float (&cs)[4], __bf16* __restrict__ C, int ldc) {
+  const int kq = lane >> 4;
+  const bool first = kq < 2;
+  const int half = rs.hd / 2, at = hpos + 4 * (kq & 1) + (first ? 0 : half);
+  float x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    x[i] = (float)(__bf16)v[i];
+    const float y = __shfl_xor(x[i], 32);
+    if (head < rs.nh + rs.nkv) {
+      float ra, rb;
+      rotate_pair(first ? x[i] : y, first ? y : x[i], sn[i], cs[i], ra, rb);
+      x[i] = first ? ra : rb;
+    }
+  }
+  if (m >= M) return;
+  if (head < rs.nh) {
+    store4(C + (size_t)m * ldc + (size_t)head * rs.hd + at, x);
+    return;
+  }
+  if (slot < 0) return;
+  const int kvh = (head - rs.nh) % rs.nkv;
+  const size_t page = slot / rs.bs, off = slot % rs.bs;
+  if (head < rs.nh + rs.nkv || !rs.v_transposed) {
+    store4((head < rs.nh + rs.nkv ? rs.kcache : rs.vcache) + ((page * rs.nkv + kvh) * rs.bs + off) * rs.hd + at, x);
+  } else {
+    __bf16* vt = rs.vcache + (page * rs.nkv + kvh) * (size_t)rs.hd * rs.bs + off;
+#pragma unroll
+    for (int i = 0; i < 4; i++) vt[(size_t)(at + i) * rs.bs] = (__bf16)x[i];
+  }
+}
+
 // GATED: the block also streams the strip of "up" rows I + n and stores act(g)*u.
 // ROPE (M <= 16): W is [(nh + 2 nkv) hd, K]; the block's 16 weight rows are eight places of a
 // head's first half and their partners in the rotation, hd/2 rows further on, so that partners
@@ -542,37 +577,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
       continue;
     }
     if (ROPE) {
-      // results 4 kq + i of the block's 16: lanes 0..31 hold places hpos + 4 kq + i of the
-      // head's first half, lanes 32..63 their partners in the second
-      const bool first = kq < 2;
-      const int half = rs.hd / 2, at = hpos + 4 * (kq & 1) + (first ? 0 : half);
-      float x[4];
+      float sn[4], cs[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        x[i] = (float)(__bf16)v[0][i];
-        const float y = __shfl_xor(x[i], 32);
-        if (head < rs.nh + rs.nkv) {
-          float ra, rb;
-          const float2 t = turn[ROPE ? i : 0][lane];
-          rotate_pair(first ? x[i] : y, first ? y : x[i], t.x, t.y, ra, rb);
-          x[i] = first ? ra : rb;
-        }
+        const float2 t = turn[ROPE ? i : 0][lane];
+        sn[i] = t.x;
+        cs[i] = t.y;
       }
-      if (m >= M) continue;
-      if (head < rs.nh) {
-        store4((__bf16*)C + (size_t)m * ldc + (size_t)head * rs.hd + at, x);
-        continue;
-      }
-      if (slot < 0) continue;
-      const int kvh = (head - rs.nh) % rs.nkv;
-      const size_t page = slot / rs.bs, off = slot % rs.bs;
-      if (head < rs.nh + rs.nkv || !rs.v_transposed) {
-        store4((head < rs.nh + rs.nkv ? rs.kcache : rs.vcache) + ((page * rs.nkv + kvh) * rs.bs + off) * rs.hd + at, x);
-      } else {
-        __bf16* vt = rs.vcache + (page * rs.nkv + kvh) * (size_t)rs.hd * rs.bs + off;
-#pragma unroll
-        for (int i = 0; i < 4; i++) vt[(size_t)(at + i) * rs.bs] = (__bf16)x[i];
-      }
+      rope_store(rs, v[0], m, M, lane, head, hpos, slot, sn, cs, (__bf16*)C, ldc);
       continue;
     }
     if (!GATED && epi == EPI_PICK) {
@@ -1071,12 +1083,13 @@ __device__ __forceinline__ void mid_store(const f32x4& v, const f32x4& up, int m
   }
 }
 
-template <int MT, bool GATED, int SPB, int KW, int CH, bool ONCE>
+template <int MT, bool GATED, int SPB, int KW, int CH, bool ONCE, bool ROPE = false>
 __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* __restrict__ A, int lda,
                                                                  const __bf16* __restrict__ W,
                                                                  void* __restrict__ C, int ldc, int c_is_f32,
                                                                  int M, int N, int K, int epi, float cap,
-                                                                 float* __restrict__ partials, int ksplit) {
+                                                                 float* __restrict__ partials, int ksplit, RopeStore rs = RopeStore{}) {
+  static_assert(!ROPE || (!GATED && KW >= MT), "a wave finishes sixteen rows");
   constexpr int NS = GATED ? 2 : 1;
   constexpr int T = SPB * KW * 64, WSTEPS = CH / KW;     // threads; steps of a chunk a wave multiplies
   constexpr int LD = CH * 32 + 16, PPR = CH * 4;         // a row of a chunk in LDS, its 16-byte pieces
@@ -1099,6 +1112,16 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   const __bf16* wp[NS];
   wp[0] = W + (size_t)strip_read * ksteps * 512 + lane * 8;
   if (GATED) wp[NS - 1] = W + ((size_t)(N / 16) + strip_read) * ksteps * 512 + lane * 8;
+  // (ROPE) the strip's rows are eight places of a head's first half and their partners, as in the kernel above
+  int head = 0, hpos = 0, slot = -1;
+  float sn[4], cs[4];
+  if (ROPE) {
+    const int per_head = rs.hd / 16;
+    head = strip_read / per_head;
+    hpos = (strip_read % per_head) * 8;
+    const int row = head * rs.hd + hpos + (r < 8 ? r : rs.hd / 2 + r - 8);
+    wp[0] = W + (size_t)(row / 16) * ksteps * 512 + (16 * kq + row % 16) * 8;
+  }
   f32x4 acc[NS][MT];
 #pragma unroll
   for (int g = 0; g < NS; g++)
@@ -1152,6 +1175,18 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   fetch_w(s_begin, w0);
   fetch_a(s_begin + CH, ra1);
   fetch_w(s_begin + CH, w1);
+  if constexpr (ROPE) {
+    // the angles of the rows that the wave will finish, while the first loads are on their way
+    const int m = min(kpart * 16 + r, M - 1);
+    if (kpart < MT) {
+      if (head >= rs.nh && rs.slot_map) slot = rs.slot_map[m];
+      if (head < rs.nh + rs.nkv) {
+        const float pos = (float)rs.positions[m];
+#pragma unroll
+        for (int i = 0; i < 4; i++) sincosf(pos * rs.inv_freq[hpos + 4 * (kq & 1) + i], &sn[i], &cs[i]);
+      }
+    }
+  }
   stash_a(0, ra0);
   __syncthreads();
 #define ZK_MID_TURN(BUF, WCUR, WNEXT2, RA_NEXT2, RA_NEXT1)    \
@@ -1192,6 +1227,10 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
       v[g] = sums[(g * MT + mt) * 64];
 #pragma unroll
       for (int k = 1; k < KW; k++) v[g] += sums[((k * NS + g) * MT + mt) * 64];
+    }
+    if constexpr (ROPE) {
+      rope_store(rs, v[0], m, M, lane, head, hpos, slot, sn, cs, (__bf16*)C, ldc);
+      continue;
     }
     if (ksplit > 1) {
       // the range's partial sums: plane (range, g) of [M, npad] floats
@@ -1563,6 +1602,44 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
   }
 #undef ZK_QKV
   return zk_launch_status("zk_qkv_rope_bf16");
+}
+
+// The same for 17 to 64 rows (weights in strips): a strip of a head's places and their partners a block, or two, K whole.  Against the product
+// with K in ranges and the rotation that adds them up it is a launch less (us, 24, 40 and 64 rows, two launches and this: 4,096 columns of K
+// 2,304 11.3, 12.5, 13.8 and 9.8, 11.2, 12.4; 8,192 of 3,584 16.7, 18.0, 20.3 and 14.3, 16.1, 18.9; 1,536 of 1,024 9.8, 10.4, 11.8 and 5.8, 6.7, 7.3).  Rounds
+// to 16 bits in front of the rotation, as those do.
+extern "C" int zk_qkv_rope_rows_bf16_supports(int M, int K, int hd, int rotary_dim) {
+  return M > 16 && M <= 64 && K > 0 && K % 32 == 0 && hd % 16 == 0 && rotary_dim == hd;
+}
+
+extern "C" int zk_qkv_rope_rows_bf16(const void* A, int lda, const void* W, void* Q, int ldq, int M, int K, int w_strip,
+                                     const int* positions, const int* slot_map, const float* inv_freq, void* kcache, void* vcache, int nh,
+                                     int nkv, int hd, int bs, int v_transposed, void* stream) {
+  ZK_REQUIRE(M > 16 && M <= 64 && K > 0 && K % 32 == 0 && lda % 8 == 0 && lda >= K && w_strip,
+             "zk_qkv_rope_rows_bf16: 17 to 64 rows, weights in strips, lda a multiple of 8");
+  ZK_REQUIRE(nh > 0 && nkv >= 0 && hd > 0 && hd % 16 == 0, "zk_qkv_rope_rows_bf16: head_dim must be a multiple of 16");
+  ZK_REQUIRE(ldq >= nh * hd && ldq % 4 == 0, "zk_qkv_rope_rows_bf16: ldq too small or not a multiple of 4");
+  ZK_REQUIRE(positions && inv_freq, "zk_qkv_rope_rows_bf16: positions and inv_freq are needed");
+  ZK_REQUIRE(nkv == 0 || (slot_map && kcache && vcache && bs > 0), "zk_qkv_rope_rows_bf16: the cache is needed");
+  ZK_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) && ((uintptr_t)Q % 8 == 0),
+             "zk_qkv_rope_rows_bf16: operands must be 16-byte aligned");
+  const int N = (nh + 2 * nkv) * hd, mt = (M + 15) / 16;
+  RopeStore rs{positions, nkv ? slot_map : nullptr, inv_freq, (__bf16*)kcache, (__bf16*)vcache, nh, nkv, hd, bs, v_transposed};
+  hipStream_t s = (hipStream_t)stream;
+#define ZK_ROPE_(MT_, SPB_, ONCE_)                                                                                        \
+  gemm_mid_kernel<MT_, false, SPB_, 8, 8, ONCE_, true><<<(N / 16 + SPB_ - 1) / SPB_, SPB_ * 512, 0, s>>>(                  \
+      (const __bf16*)A, lda, (const __bf16*)W, Q, ldq, 0, M, N, K, EPI_NONE, 0.f, nullptr, 1, rs)
+#define ZK_ROPE(SPB_, ONCE_)                      \
+  do {                                            \
+    if (mt == 2) ZK_ROPE_(2, SPB_, ONCE_);        \
+    else if (mt == 3) ZK_ROPE_(3, SPB_, ONCE_);   \
+    else ZK_ROPE_(4, SPB_, ONCE_);                \
+  } while (0)
+  if (N / 16 <= 256) { if (reads_once(w_strip)) ZK_ROPE(1, true); else ZK_ROPE(1, false); }
+  else { if (reads_once(w_strip)) ZK_ROPE(2, true); else ZK_ROPE(2, false); }
+#undef ZK_ROPE
+#undef ZK_ROPE_
+  return zk_launch_status("zk_qkv_rope_rows_bf16");
 }
 
 // The two products behind a norm, for one row that the product makes itself: what zk_norm_add_norm (sub, up to 6 planes, w_post, h, w_next) followed by zk_qkv_rope_bf16, or by zk_gemm_bf16 with a gated epilogue, gives, to the bit.  h_out: the new stream,

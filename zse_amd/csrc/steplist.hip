@@ -52,6 +52,9 @@ int zk_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc, int c_
 int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, int ldq, int M, int K, int w_strip,
                      const int* positions, const int* slot_map, const float* inv_freq, void* kcache, void* vcache,
                      int nh, int nkv, int hd, int bs, int v_transposed, void* stream);
+int zk_qkv_rope_rows_bf16(const void* A, int lda, const void* W, void* Q, int ldq, int M, int K, int w_strip,
+                          const int* positions, const int* slot_map, const float* inv_freq, void* kcache, void* vcache,
+                          int nh, int nkv, int hd, int bs, int v_transposed, void* stream);
 int zk_norm_qkv_rope_bf16(const void* sub, int sub_parts, const float* w_post, float eps_post, int uo_post, const float* h, void* h_out,
                           const float* w_next, float eps_next, int uo_next, const void* W, void* Q, int ldq, int K, int w_strip,
                           const int* positions, const int* slot_map, const float* inv_freq, void* kcache, void* vcache, int nh,
@@ -139,6 +142,7 @@ const int entered_at_load = []() {
 #if ZSE_ACT_BF16
   OWN(zk_gemm_bf16);
   OWN(zk_qkv_rope_bf16);
+  OWN(zk_qkv_rope_rows_bf16);
   OWN(zk_norm_qkv_rope_bf16);
   OWN(zk_norm_gated_bf16);
   OWN(zk_attention_bf16);

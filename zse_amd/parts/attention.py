@@ -319,6 +319,17 @@ class PagedAttention(Part):
                 k.zk_add_bias(y.ptr, self.o_bias.ptr, T, s.hidden_size, ctx.stream)
         return y
 
+    def _rotating_product(self, ctx, T: int, rotary_dim: int):
+        """The product that rotates and stores its own results, where there is one for so many rows."""
+        s, k = self.spec, ctx.k
+        if not (tuned_gemm(ctx, s.hidden_size) and k.has("zk_qkv_rope_bf16")):
+            return None
+        if k.zk_qkv_rope_bf16_supports(T, s.hidden_size, s.head_dim, rotary_dim):
+            return k.zk_qkv_rope_bf16
+        if self.w_qkv.layout == "strip" and k.zk_qkv_rope_rows_bf16_supports(T, s.hidden_size, s.head_dim, rotary_dim):
+            return k.zk_qkv_rope_rows_bf16
+        return None
+
     def takes_pending_norm(self, ctx, size: int, planes: int) -> bool:
         """Whether the product of one row that rotates and stores its results serves this mixer (and then makes its own norm)."""
         s, tables = self.spec, self.position.rotary_tables()
@@ -345,15 +356,13 @@ class PagedAttention(Part):
                                     None if self.shared_kv else g.slot_map, tables[0].ptr, cache.k.ptr, cache.v.ptr, nh, n_store, hd,
                                     g.page_size, 1 if cache.v_transposed else 0, ctx.stream)
             x.done()
-        elif (not hooked and tables is not None and tuned_gemm(ctx, s.hidden_size) and k.has("zk_qkv_rope_bf16")
-                and k.zk_qkv_rope_bf16_supports(T, s.hidden_size, hd, tables[1])):
-            # few decoded tokens: the product rotates and stores its own results
+        elif not hooked and tables is not None and self._rotating_product(ctx, T, tables[1]) is not None:
+            # few tokens: the product rotates and stores its own results
             qkv = ctx.alloc((T, width))
-            k.zk_qkv_rope_bf16(x.ptr, s.hidden_size, self.w_qkv.ptr, qkv.ptr, width, T, s.hidden_size,
-                               strip_flag(ctx, self.w_qkv), ctx.positions,
-                               None if self.shared_kv else g.slot_map, tables[0].ptr, cache.k.ptr,
-                               cache.v.ptr, nh, n_store, hd, g.page_size, 1 if cache.v_transposed else 0,
-                               ctx.stream)
+            self._rotating_product(ctx, T, tables[1])(
+                x.ptr, s.hidden_size, self.w_qkv.ptr, qkv.ptr, width, T, s.hidden_size, strip_flag(ctx, self.w_qkv), ctx.positions,
+                None if self.shared_kv else g.slot_map, tables[0].ptr, cache.k.ptr, cache.v.ptr, nh, n_store, hd, g.page_size,
+                1 if cache.v_transposed else 0, ctx.stream)
         else:
             # a product that splits K may leave the adding up of its partial sums to the kernel
             # that rotates and stores, unless something has to look at the rows in between

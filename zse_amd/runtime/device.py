@@ -249,6 +249,7 @@ BF16_KERNEL_SIGNATURES = {
                               _I, _VP],
     "zk_norm_gated_bf16": [_VP, _I, _VP, _F, _I, _VP, _VP, _VP, _F, _I, _VP, _VP, _I, _I, _I, _I, _VP],
     "zk_qkv_rope_bf16": [_VP, _I, _VP, _VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP],
+    "zk_qkv_rope_rows_bf16": [_VP, _I, _VP, _VP, _I, _I, _I, _I, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _VP],
     "zk_attention_bf16": [_VP, _I, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I,
                           _F, _F, _I, _I, _VP, _SZ, _VP],
     "zk_attention_bf16_masked": [_VP, _I, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I,
@@ -379,6 +380,9 @@ class KernelLibrary:
             self._dll.zk_qkv_rope_bf16_supports.restype = C.c_int
             self._dll.zk_qkv_rope_bf16_supports.argtypes = [_I, _I, _I, _I]
             self.zk_qkv_rope_bf16_supports = self._dll.zk_qkv_rope_bf16_supports
+            self._dll.zk_qkv_rope_rows_bf16_supports.restype = C.c_int
+            self._dll.zk_qkv_rope_rows_bf16_supports.argtypes = [_I, _I, _I, _I]
+            self.zk_qkv_rope_rows_bf16_supports = self._dll.zk_qkv_rope_rows_bf16_supports
             self._dll.zk_norm_product_supports.restype = C.c_int
             self._dll.zk_norm_product_supports.argtypes = [_I, _I, _I]
             self.zk_norm_product_supports = self._dll.zk_norm_product_supports
