@@ -7,8 +7,8 @@
 //    16x16x32 MFMAs straight from global memory: a lane's 16-byte load is exactly its MFMA
 //    operand (row = lane % 16, eight k values at 8 * (lane / 16)), so no LDS staging is
 //    needed.  Partial sums of the waves meet in LDS.
-//  * mid (17 <= M <= 64, strip layout): four strips a block, two waves each, the activations
-//    of a k chunk shared through LDS, K split over blocks when N alone gives too few of them.
+//  * mid (17 <= M <= 64, strip layout, and some shapes of fewer rows): one to eight strips a block, one to eight waves
+//    each, the activations of a k chunk shared through LDS, K split over blocks when N alone gives too few of them.
 //  * tile (M > 64, prefill): weights in strip layout by the kernel of gemm_bf16_tiles.h, others by
 //    128x128x64 to 256x256x64 block tiles staged through registers and LDS.
 // Epilogues: plain store (bf16 or float), soft cap on float output (LM head), and
@@ -168,7 +168,7 @@ __device__ __forceinline__ f32x4 load4_act(const __bf16* p) {
 // The sums run as in norm_add_norm_wide_kernel (WIDE, H >= 2,048: 16 waves, a vector of four a thread) or norm_add_norm_fast_kernel (4
 // waves, up to two vectors a thread), whose waves this block's NW waves take in turn, SLOTS each.  H a multiple of 256.  PL: 0, or as many planes asked for (parts <= PL).
 // Two halves, because loads come back in the order in which they were asked for: what the row is made of first, then (by the caller) the first
-// weights, then the sums, which wait for the former alone.  All that forks is fixed at compile time: with branches on the planes and the width the compiler
+// weights, then the sums, which wait for the former alone (weights first: a step of the 2B shapes 1,550 us, so 1,514).  All that forks is fixed at compile time: with branches on the planes and the width the compiler
 // waits for every load and keeps rows in scratch memory (4,096 columns of K 2,304 8.0 and 9.1 us in a trace of a step).
 template <int NW, int SLOTS, bool WIDE, int PL>
 struct RowInWork {
