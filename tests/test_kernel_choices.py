@@ -43,3 +43,24 @@ def test_chunks_of_the_matrix_memory(D, tokens):
     chunks = lambda L: (600 + L - 1) // L + 2
     assert floats(600, 2, 4, D, 40, 500) == chunks(tokens) * 4 * (D * 40 + D + 3)
     assert floats(600, 2, 4, D, 40, 30) == chunks(32) * 4 * (D * 40 + D + 3)
+
+
+# up to 16 rows with three strips a block, 17 to 64 rows in long and short ranges, gated in ranges
+@pytest.mark.parametrize("epi,M,N,K", [(0, 1, 3584, 14336), (0, 16, 4608, 36864), (0, 8, 3200, 8192), (0, 17, 2304, 9216), (0, 64, 2304, 2048),
+                                       (2, 64, 512, 8192)])
+def test_ranges_of_k_need_a_workspace(epi, M, N, K):
+    """Ranges of K leave their partial sums in the workspace by 16-byte stores: none, a misaligned one or one too small for two of them leave K whole."""
+    cut, mid_cut = (C.c_int * 4)(), library().zk_gemm_bf16_mid_cut
+    mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
+
+    def ranges(ws, room, by_reader=1):
+        assert mid_cut(epi, by_reader, M, N, K, ws, room, cut) == 1
+        return cut[3]
+
+    plane = (2 if epi else 1) * M * -(-N // 16) * 16 * 4
+    assert ranges(4096, 320 << 20) > 1
+    assert ranges(4096, 2 * plane) == 2
+    for ws, room in ((None, 320 << 20), (None, 0), (4096 + 4, 320 << 20), (4096 + 8, 320 << 20), (4096, 2 * plane - 1), (4096, 0)):
+        assert ranges(ws, room) == 1, (ws, room)
+    if M > 16:
+        assert ranges(4096, 320 << 20, 0) > 1 and ranges(None, 320 << 20, 0) == 1

@@ -1389,7 +1389,7 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
   if (M <= 16 && nstrips >= 1024) return {2, 8, 16, 1};
   if (nstrips >= 4096) return {8, 1, 4, 1};
   if (nstrips >= 1024) return {4, 4, 4, 1};
-  if (M <= 16) return {3, 4, 8, mid_ranges((nstrips + 2) / 3, ksteps, 8)};
+  if (M <= 16) return {3, 4, 8, split_ok ? mid_ranges((nstrips + 2) / 3, ksteps, 8) : 1};
   const int cblocks = (nstrips + 3) / 4;
   if (!split_ok) return {4, 2, 8, 1};
   const int ks = mid_ranges(cblocks, ksteps, 8);
@@ -1411,21 +1411,28 @@ static bool mid_for_few(bool gated, int N, int K, bool by_reader) {
   return (nstrips >= 1024 && K >= 2048) || (by_reader && K >= 8192 && nstrips > 192);
 }
 
+// Bytes of the partial sums of one range.
+static size_t mid_range_bytes(bool gated, int M, int N) { return (size_t)(gated ? 2 : 1) * M * ((N + 15) / 16 * 16) * sizeof(float); }
+
+// The cut of a launch: ranges of K only where there is a workspace that 16-byte stores reach and that holds them.  Picks are taken
+// from whole sums; up to 16 rows only a reader that adds up the partial sums itself is worth a split.
+static MidCut mid_cut_of_launch(bool gated, bool by_reader, int M, int N, int K, int epi, const GemmWorkspace& wsp) {
+  const bool split_ok = wsp.ptr != nullptr && (uintptr_t)wsp.ptr % 16 == 0 && epi != EPI_PICK && (M > 16 || by_reader);
+  MidCut cut = mid_cut(gated, M, N, K, split_ok);
+  while (cut.ksplit > 1 && cut.ksplit * mid_range_bytes(gated, M, N) > wsp.split_bytes()) cut.ksplit--;
+  return cut;
+}
+
 template <bool GATED>
 static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32, int M, int N,
                       int K, int epi, float cap, int w_strip, const GemmWorkspace& wsp, int* parts, hipStream_t s) {
   const int mt = (M + 15) / 16;
   const int nstrips = (N + 15) / 16, npad = nstrips * 16;
-  void* ws = wsp.ptr;
-  // picks are taken from whole sums; up to 16 rows only a reader that adds up the partial sums itself is worth a split
   const bool by_reader = parts != nullptr && joinable_by_reader(N, ldc, c_is_f32, epi);
-  const bool split_ok = ws != nullptr && (uintptr_t)ws % 16 == 0 && epi != EPI_PICK && (M > 16 || by_reader);
-  MidCut cut = mid_cut(GATED, M, N, K, split_ok);
-  const size_t per_range = (size_t)(GATED ? 2 : 1) * M * npad * sizeof(float);
-  while (cut.ksplit > 1 && cut.ksplit * per_range > wsp.split_bytes()) cut.ksplit--;
-  if (cut.ksplit > 1 && cut.ksplit * per_range > wsp.bytes) return wsp.too_small(cut.ksplit * per_range);
+  const MidCut cut = mid_cut_of_launch(GATED, by_reader, M, N, K, epi, wsp);
+  if (cut.ksplit > 1 && cut.ksplit * mid_range_bytes(GATED, M, N) > wsp.bytes) return wsp.too_small(cut.ksplit * mid_range_bytes(GATED, M, N));
   const int ksplit = cut.ksplit;
-  float* partials = (float*)ws;
+  float* partials = (float*)wsp.ptr;
   dim3 grid((nstrips + cut.spb - 1) / cut.spb, ksplit);
 #define ZK_MID_(MT_, SPB_, KW_, CH_, ONCE_)                                                             \
   gemm_mid_kernel<MT_, GATED, SPB_, KW_, CH_, ONCE_><<<grid, SPB_ * KW_ * 64, 0, s>>>((const __bf16*)A, lda, (const __bf16*)W, C, ldc, \
@@ -1974,6 +1981,19 @@ extern "C" int zk_gemm_bf16_tile_cut(int gated, int by_reader, int M, int N, int
   *tail_ks = c.tail_ks;
   *rest = c.rest;
   return 0;
+}
+
+// Whether a product of up to 64 rows by weights in strips takes the blocks of gemm_mid_kernel with this workspace, and how it is cut:
+// strips a block, waves a strip, steps a chunk, ranges of K.  ``epi`` and ``by_reader`` as above.  For tests.
+extern "C" int zk_gemm_bf16_mid_cut(int epi, int by_reader, int M, int N, int K, const void* ws, size_t ws_bytes, int* cut) {
+  const bool gated = epi == EPI_GELU_TANH || epi == EPI_SILU || epi == EPI_RELU || epi == EPI_CLAMPED;
+  if (M < 1 || M > 64 || (M <= 16 && !mid_for_few(gated, N, K, by_reader != 0))) return 0;
+  const MidCut c = mid_cut_of_launch(gated, by_reader != 0, M, N, K, epi, GemmWorkspace{const_cast<void*>(ws), ws_bytes, false});
+  cut[0] = c.spb;
+  cut[1] = c.kw;
+  cut[2] = c.ch;
+  cut[3] = c.ksplit;
+  return 1;
 }
 
 extern "C" int zk_gemm_bf16(const void* A, int lda, const void* W, void* C, int ldc, int c_is_f32,
