@@ -105,8 +105,7 @@ class Block(Part):
         m = self.ffn.forward(ctx, x)
         ctx.sums_welcome = None
         following = getattr(ctx, "next_block", None)
-        if m.layout == "parts" and next_norm is not None and getattr(type(following), "forward", None) is Block.forward:
-            # (partial sums outlive this block's own memory)
+        if next_norm is not None and getattr(type(following), "forward", None) is Block.forward and PendingNorm.outlasts_block(ctx, m):
             x = self._pending(ctx, m, n.get("post_ffn"), h, next_norm, following.mixer)
             if x is not None:
                 return x

@@ -39,6 +39,13 @@ class PendingNorm:
         return (h.shape[0] == 1 and ctx.dtype == BF16 and ctx.tuned and getattr(ctx, "spare_stream", None) is not None and
                 ctx.k.has("zk_norm_gated_bf16") and (sub.layout == "parts" or (sub.layout == "rows" and sub.dtype == BF16)))
 
+    @staticmethod
+    def outlasts_block(ctx, sub: Tensor) -> bool:
+        """Whether ``sub`` may wait for the next block's first product: partial sums in the products' workspace, not what lies in the
+        step's own memory, which that block hands out again (to the rows that the very product writes, while others of its blocks read)."""
+        ws = getattr(ctx, "gemm_workspace", None)
+        return sub.layout == "parts" and ws is not None and sub.ptr == ws.ptr
+
     def args(self):
         """The leading arguments of the products that take one."""
         post, nxt = self.post, self.nxt
