@@ -86,3 +86,15 @@ def test_no_norm_waits_for_a_block_of_its_own_kind():
     own.__dict__.update(block(in_workspace).__dict__)
     assert not isinstance(after(in_workspace, own), PendingNorm)
     assert not isinstance(after(in_workspace, None), PendingNorm)
+
+
+@pytest.mark.parametrize("off,waits", [(0, True), (8, False), (16, True)])
+def test_rows_that_16_byte_loads_do_not_reach(off, waits):
+    """The products that make their own norm read 16 bytes at a time; a mixer's row elsewhere goes through the norm's kernel."""
+    seen = []
+    b = block(lambda ctx, x: (seen.append(x), ctx.alloc((1, H)))[1])
+    b.ffn.takes_pending_norm = lambda ctx, size, planes: True
+    b.mixer.forward = lambda ctx, x, cache: Tensor(8192 + off, (1, H), BF16)
+    ctx = context(None)
+    b.forward(ctx, Tensor(1 << 22, (1, H), F32), None, x_in=ctx.alloc((1, H)), next_norm=norm(), x_out=Tensor(1 << 23, (1, H), BF16))
+    assert isinstance(seen[0], PendingNorm) == waits

@@ -37,7 +37,8 @@ class PendingNorm:
     @staticmethod
     def possible(ctx, h: Tensor, sub: Tensor) -> bool:
         return (h.shape[0] == 1 and ctx.dtype == BF16 and ctx.tuned and getattr(ctx, "spare_stream", None) is not None and
-                ctx.k.has("zk_norm_gated_bf16") and (sub.layout == "parts" or (sub.layout == "rows" and sub.dtype == BF16)))
+                ctx.k.has("zk_norm_gated_bf16") and (sub.layout == "parts" or (sub.layout == "rows" and sub.dtype == BF16)) and
+                sub.ptr % 16 == 0 and h.ptr % 16 == 0)       # (the norm's own kernel takes rows from 8-byte addresses too)
 
     @staticmethod
     def outlasts_block(ctx, sub: Tensor) -> bool:
