@@ -64,3 +64,26 @@ def test_ranges_of_k_need_a_workspace(epi, M, N, K):
         assert ranges(ws, room) == 1, (ws, room)
     if M > 16:
         assert ranges(4096, 320 << 20, 0) > 1 and ranges(None, 320 << 20, 0) == 1
+
+
+# query heads, key heads, channels of a key and a value, page, pages of a table, values shared by 2^shift key heads; whether they go past the caches
+@pytest.mark.parametrize("nh,nkv,hd,vd,bs,table,shift,past", [
+    (8, 4, 256, 256, 16, 64, 0, 1), (8, 4, 256, 256, 32, 32, 0, 1), (8, 4, 256, 256, 64, 16, 0, 0), (8, 4, 256, 256, 16, 512, 0, 1),
+    (8, 4, 256, 256, 32, 256, 0, 0), (32, 16, 128, 128, 4, 2048, 0, 1), (32, 16, 128, 128, 128, 64, 0, 0), (16, 8, 64, 128, 16, 64, 1, 0)])
+def test_values_past_the_caches(nh, nkv, hd, vd, bs, table, shift, past):
+    """Where loads past the caches take a line by halves they lose: 64 requests of 4,000 keys, pages of 64 206 and 239 us, of 128 231 and 279; values of two
+    key heads 113 and 128."""
+    choice = library().zk_attention_bf16_values_past_caches
+    assert choice(1, nh, nkv, hd, vd, bs, table, 64, shift) == past
+    assert choice(0, nh, nkv, hd, vd, bs, table, 64, shift) == 0
+
+
+def test_steps_that_pass_through_more_than_the_cache():
+    from types import SimpleNamespace as S
+    from zse_amd.parts.ops import values_once
+    own, step = S(shared=False, lent=False), lambda **kw: S(**{**dict(weights_read_once=False, R=8, max_ctx=1000, cache_token_bytes=24576), **kw})
+    assert values_once(step(), own) == 0                                  # 8 x 1,000 x 24 KB: 197 MB
+    assert values_once(step(max_ctx=1500), own) == 1
+    assert values_once(step(weights_read_once=True), own) == 1
+    for other in (S(shared=True, lent=False), S(shared=False, lent=True)):      # the same values are read again within the step
+        assert values_once(step(weights_read_once=True), other) == 0

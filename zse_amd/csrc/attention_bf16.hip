@@ -508,6 +508,20 @@ static bool decode_in_long_blocks(int nh, int nkv, int hd, int vd, int bs, int m
          decode_long_lds(nh / nkv, vd) + (size_t)hd / 32 * 4 * 64 * 16 <= 64 * 1024;
 }
 
+// Whether decoded tokens' values go past the caches (common.h's load_once) where the caller says that nothing reads them again before
+// they have left those anyway: only where a wave's loads take whole lines of a channel's page and one block alone reads them.  Pages of up to
+// 32 keys (a wave of the long blocks: 16), no value head under several key heads.  us, 64 requests of 4,000 keys, plain loads and these, 8
+// heads over 4 of 256 channels, pages of 8, 16, 32, 64, 128 keys: 201, 198, 198, 206, 231 and 189, 188, 185, 239, 279; 32 over 16 of 128: 393,
+// 392, 388, 397, 400 and 370, 365, 359, 441, 532; 1 request of 8,000 in long blocks, 8 over 4 of 256, pages of 16, 32, 64: 18.4, 17.5, 21.7 and 17.7, 17.9,
+// 22.9; 16 of 64 over 8 whose pairs share values of 128, 64 of 4,000, pages of 16: 113 and 128.
+static bool values_past_caches(int once, int bs, int v_shift, bool long_blocks) {
+  return once && v_shift == 0 && bs <= (long_blocks ? 16 : 32);
+}
+
+extern "C" int zk_attention_bf16_values_past_caches(int once, int nh, int nkv, int hd, int vd, int bs, int max_blocks, int decode_chunk, int v_shift) {
+  return decode_on_narrow_tiles(nh, nkv, hd) && values_past_caches(once, bs, v_shift, decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk));
+}
+
 // The longest context the split variant takes for decoded tokens (the joining kernel keeps one
 // weight per partial result in LDS).  ``decode_chunk`` as in zk_attention_bf16.
 long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chunk) {
@@ -532,13 +546,14 @@ long long zk_attention_bf16_max_context(int nh, int nkv, int hd, int decode_chun
 // sinks (may be null; not together with ``sink``): float [nh], exp(sinks[h]) joins head h's denominators.
 // gate (may be null): bf16, row t's nh numbers at gate + t * gate_ld; head h's output times sigmoid of the h-th.
 // portion_ctx: the longest context among the portions, whose kernel it chooses (0: not known, max_ctx stands for it).
-int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, const void* vcache_t,
+// once: no later launch finds a value that this one reads in the memory side's cache (see values_past_caches; the same bits either way).
+int zk_attention_bf16_once(const void* q, int q_stride, const void* kcache, const void* vcache_t,
                            const int* block_table, int max_blocks, const int* q_start, const int* ctx_len,
                            void* out, int R, int r_prefill, int max_q_len, int max_ctx, int nh, int nkv,
                            int hd, int bs, float scale, float softcap, int window, int decode_chunk,
                            void* workspace, size_t workspace_bytes, int mask_chunk, int sink, int wide_weights,
                            int v_shift, int vd, int keep, const float* sinks, const void* gate, int gate_ld,
-                           int portion_ctx, void* stream) {
+                           int portion_ctx, int once, void* stream) {
   ZK_REQUIRE(portion_ctx >= 0, "zk_attention_bf16: bad context of the portions");
   ZK_REQUIRE(!sink || sinks == nullptr, "zk_attention_bf16: a unit sink or learned sinks, not both");
   ZK_REQUIRE(gate == nullptr || gate_ld >= nh, "zk_attention_bf16: gate rows hold a number per head");
@@ -572,7 +587,7 @@ int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, cons
   p.q_start = q_start; p.ctx_len = ctx_len; p.out = (__bf16*)out;
   p.nh = nh; p.nkv = nkv; p.hd = hd; p.vd = vd; p.bs = bs; p.keep = keep;
   p.scale = scale; p.softcap = softcap; p.window = window;
-  p.from_window = 0;
+  p.from_window = 0; p.once = 0;
   p.mask_chunk = mask_chunk; p.sink = sink ? 1 : 0; p.wide_weights = wide_weights ? 1 : 0;
   p.sinks = sinks; p.gate = (const __bf16*)gate; p.gate_ld = gate_ld;
   p.bs_shift = 0;
@@ -627,6 +642,7 @@ int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, cons
     if (decode_on_narrow_tiles(nh, nkv, hd)) {
       // a block joins its four waves: one partial result per block of keys
       const bool long_blocks = decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk);
+      p.once = values_past_caches(once, bs, v_shift, long_blocks) ? 1 : 0;
       p.chunk = ATT_CHUNK;
       span = long_blocks ? 4 * p.chunk : ATT_DECODE_SPAN;
       grid.x = (max_ctx + span - 1) / span;
@@ -651,6 +667,19 @@ int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, cons
     return zk_launch_status("zk_attention_bf16 (combine)");
   }
   return 0;
+}
+
+int zk_attention_bf16_step(const void* q, int q_stride, const void* kcache, const void* vcache_t,
+                           const int* block_table, int max_blocks, const int* q_start, const int* ctx_len,
+                           void* out, int R, int r_prefill, int max_q_len, int max_ctx, int nh, int nkv,
+                           int hd, int bs, float scale, float softcap, int window, int decode_chunk,
+                           void* workspace, size_t workspace_bytes, int mask_chunk, int sink, int wide_weights,
+                           int v_shift, int vd, int keep, const float* sinks, const void* gate, int gate_ld,
+                           int portion_ctx, void* stream) {
+  return zk_attention_bf16_once(q, q_stride, kcache, vcache_t, block_table, max_blocks, q_start, ctx_len, out, R,
+                                r_prefill, max_q_len, max_ctx, nh, nkv, hd, bs, scale, softcap, window, decode_chunk,
+                                workspace, workspace_bytes, mask_chunk, sink, wide_weights, v_shift, vd, keep, sinks, gate,
+                                gate_ld, portion_ctx, 0, stream);
 }
 
 int zk_attention_bf16_gated(const void* q, int q_stride, const void* kcache, const void* vcache_t,
@@ -720,6 +749,10 @@ static const int zk_attention_bf16_masked_entered = zk_steplist_register(
 static const int zk_attention_bf16_step_entered = zk_steplist_register(
     "zk_attention_bf16_step", zk_packed::Call<zk_attention_bf16_step>::nargs,
     (void*)zk_packed::Call<zk_attention_bf16_step>::call);
+
+static const int zk_attention_bf16_once_entered = zk_steplist_register(
+    "zk_attention_bf16_once", zk_packed::Call<zk_attention_bf16_once>::nargs,
+    (void*)zk_packed::Call<zk_attention_bf16_once>::call);
 
 static const int zk_attention_bf16_gated_entered = zk_steplist_register(
     "zk_attention_bf16_gated", zk_packed::Call<zk_attention_bf16_gated>::nargs,

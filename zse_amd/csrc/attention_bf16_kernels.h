@@ -55,6 +55,7 @@ struct AttnParams {
   const float* sinks;     // [nh] (may be null): exp(sinks[h]) joins head h's denominator, with no key and no value
   const __bf16* gate;     // (may be null) row t's numbers per head at gate + t * gate_ld; head h's output is
   int gate_ld;            // multiplied by the sigmoid of the h-th
+  int once;               // decoded tokens: values by loads that leave no trace in the caches (values_past_caches)
   int wide_weights;       // 1: a weight meets the values as two bf16 numbers, its rounded value and what the
                           // rounding left (16 bits of mantissa instead of 8; one more product a tile)
 };
@@ -1161,7 +1162,7 @@ __device__ __forceinline__ int rotated_block(int blocks) {
 // of 200 to 3,840 keys 146 -> 105 (109 by the order of the blocks alone), of 4,096 keys 192 ->
 // 193 (5.6 TB/s), 23 of 130 to 2,000 35.7 -> 27.1, 8 of 4,000 31.6 -> 31.1, 1 of 4,000 13.3 ->
 // 11.8.  Eight waves of one tile each: 119, 202, 33.1, 32.9.
-template <int HD32, int VD16>
+template <int HD32, int VD16, bool ONCE>
 __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
   constexpr int KS = HD32;       // 32-wide steps over head_dim
   constexpr int DT = VD16;       // 16-channel output tiles
@@ -1237,7 +1238,7 @@ __global__ __launch_bounds__(256, 4) void attn_decode_kernel(AttnParams p) {
     auto load_v = [&]() {
       if (bsh >= 3) {
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) vf[dt] = load_once((const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh)));
+        for (int dt = 0; dt < DT; dt++) vf[dt] = load_maybe_once<ONCE>((const bf16x8*)(va + ((size_t)(dt * 16 + col) << bsh)));
       } else {         // pages of four keys
 #pragma unroll
         for (int dt = 0; dt < DT; dt++) {
@@ -1489,7 +1490,7 @@ __global__ __launch_bounds__(NW * 64, 2) void attn_short_kernel(AttnParams p) {
 // For callers whose limit is a long context (ATT_DECODE_LONG_FROM keys a request or more): blocks of
 // 256 keys leave half as many partial results as those of 128, whose writing and reading are what
 // is left to save once every CU has many blocks.  Figures at decode_in_long_blocks.
-template <int HD32, int VD16>
+template <int HD32, int VD16, bool ONCE>
 __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) {
   constexpr int KS = HD32;       // 32-wide steps over head_dim
   constexpr int DT = VD16;       // 16-channel output tiles
@@ -1586,8 +1587,8 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
 #pragma unroll
       for (int dt = 0; dt < DT; dt++) {
         const int d = dt * 16 + col;
-        const bf16x4 va = load_once((const bf16x4*)(va_base + ((size_t)d << bsh)));
-        const bf16x4 vb = load_once((const bf16x4*)(vb_base + ((size_t)d << bsh)));
+        const bf16x4 va = load_maybe_once<ONCE>((const bf16x4*)(va_base + ((size_t)d << bsh)));
+        const bf16x4 vb = load_maybe_once<ONCE>((const bf16x4*)(vb_base + ((size_t)d << bsh)));
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           vf[dt][e] = va[e];
@@ -1764,19 +1765,23 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
         const size_t lds = (size_t)4 * (p.nh / p.nkv) * p.vd * sizeof(float) + (size_t)4 * (HD16 / 2) * 64 * sizeof(bf16x8);
         static std::atomic<bool> prepared{false};
         if (lds > 64 * 1024 && !prepared) {      // 16 heads a KV head with values of 256 channels: 96 KB
-          if (hipFuncSetAttribute((const void*)attn_decode_kernel<HD16 / 2, VD16>, hipFuncAttributeMaxDynamicSharedMemorySize,
+          if (hipFuncSetAttribute((const void*)attn_decode_kernel<HD16 / 2, VD16, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  96 * 1024) != hipSuccess ||
+              hipFuncSetAttribute((const void*)attn_decode_kernel<HD16 / 2, VD16, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   96 * 1024) != hipSuccess)
             return zk_fail("zk_attention_bf16: the decode kernel's LDS was refused");
           prepared = true;
         }
-        attn_decode_kernel<HD16 / 2, VD16><<<grid, 256, lds, s>>>(p);
+        if (p.once) attn_decode_kernel<HD16 / 2, VD16, true><<<grid, 256, lds, s>>>(p);
+        else attn_decode_kernel<HD16 / 2, VD16, false><<<grid, 256, lds, s>>>(p);
         break;
       } else {
         return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
       }
     case ATT_DECODE_LONG:
       if constexpr (HD16 % 2 == 0) {
-        attn_decode_long_kernel<HD16 / 2, VD16><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
+        if (p.once) attn_decode_long_kernel<HD16 / 2, VD16, true><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
+        else attn_decode_long_kernel<HD16 / 2, VD16, false><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
         break;
       } else {
         return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");

@@ -42,6 +42,12 @@ __device__ __forceinline__ T load_once(const T* p) {
   return __builtin_bit_cast(T, __builtin_nontemporal_load((const words*)p));
 }
 
+template <bool ONCE, typename T>
+__device__ __forceinline__ T load_maybe_once(const T* p) {
+  if constexpr (ONCE) return load_once(p);
+  else return *p;
+}
+
 // One rotation of a pair by an angle, written so that every kernel that rotates rounds alike
 // (a token's values must not depend on how many tokens the step holds or on which kernel took
 // it): a product rounded, then one fused multiply-add.

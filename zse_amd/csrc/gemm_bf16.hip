@@ -132,7 +132,7 @@ __device__ __forceinline__ bf16x8 zero8() {
 static bool reads_once(int w_strip) { return (w_strip & 2) != 0; }
 template <bool ONCE>
 __device__ __forceinline__ bf16x8 load_weights(const void* p) {
-  return ONCE ? load_once((const bf16x8*)p) : *(const bf16x8*)p;
+  return load_maybe_once<ONCE>((const bf16x8*)p);
 }
 
 // ------------------------------------------------------------------ the norm in front of a product of one row

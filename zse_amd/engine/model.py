@@ -21,6 +21,7 @@ class CallCache:
     state_offset: int = 0            # byte offset inside a request's state slot
     state_bytes: int = 0
     shared: bool = False             # k, v and group are another entry's (this entry stores none)
+    lent: bool = False               # other entries read this entry's k and v
     extra: Dict[str, tuple] = field(default_factory=dict)   # states of the layer's other parts: key -> (offset, bytes)
 
 

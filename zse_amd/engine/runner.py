@@ -29,6 +29,7 @@ import numpy as np
 from ..cache.manager import CacheManager, GroupInfo, group_needs
 from ..cache.pages import OutOfPages
 from ..parts.base import PagedKV, StateNeed
+from ..parts.ops import MEMORY_SIDE_CACHE
 from ..runtime.device import BF16, F32, I32, ITEMSIZE, Runtime, Tensor, canonical_dtype
 from .model import CallCache, Model
 
@@ -96,9 +97,6 @@ class Arena:
         return self.rt.empty(((nbytes + 3) // 4,), F32)
 
 
-MEMORY_SIDE_CACHE = 256 << 20       # bytes
-
-
 class StepContext:
     """What parts see of a step."""
 
@@ -113,6 +111,7 @@ class StepContext:
         self.workspace = runner.workspace
         self.gemm_workspace = runner.gemm_workspace
         self.weights_read_once = runner.weights_read_once
+        self.cache_token_bytes = runner.cache_token_bytes
         self.T = 0
         self.R = 0
         self.tokens = self.positions = self.req_of_token = self.q_start = self.ctx_len = 0
@@ -216,7 +215,7 @@ class StepRunner:
                 # beside whatever state of its own it keeps
                 own = self.caches[call.cache_of]
                 cc.need, cc.group, cc.k, cc.v, cc.v_transposed = own.need, own.group, own.k, own.v, own.v_transposed
-                cc.shared = True
+                cc.shared = own.lent = True
             # what the layer's other parts keep per request (a convolution's last rows, say)
             block = model.blocks[call.layer]
             for key, nbytes in (block.state_needs() if hasattr(block, "state_needs") else []):
@@ -266,6 +265,9 @@ class StepRunner:
                                f"allocated: {e}") from None
         # a model larger than the cache on the memory's side leaves nothing of a step's weights there for the next step
         self.weights_read_once = getattr(model, "weight_bytes", 0) > MEMORY_SIDE_CACHE
+        # what a token of one request has in all layers' pages
+        self.cache_token_bytes = sum((c.k.nbytes + (0 if c.v is c.k else c.v.nbytes)) // (c.k.shape[0] * self.page_size)
+                                     for c in self.caches if c.k is not None and not c.shared)
         self.gemm_workspace = None
         if self.dtype == BF16 and self.k.has("zk_gemm_bf16_workspace"):
             self.gemm_workspace = rt.zeros((self.k.zk_gemm_bf16_workspace() // 4,), F32)

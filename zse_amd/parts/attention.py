@@ -20,7 +20,7 @@ import numpy as np
 from ..config.plan import ShortConvSpec
 from ..runtime.device import BF16, ITEMSIZE, Tensor
 from .base import ROLE_GAIN, PagedKV, Part, TensorReq, build_part, register_part
-from .ops import PendingNorm, linear, strip_flag, tuned_gemm
+from .ops import PendingNorm, linear, strip_flag, tuned_gemm, values_once
 
 
 class PagedAttention(Part):
@@ -295,12 +295,12 @@ class PagedAttention(Part):
         win = int(s.window) if s.window else 0
         head_gate = rows.ptr + heads_width * ITEMSIZE[ctx.dtype] if self.head_gate_name else None
         if cache.v_transposed and ctx.tuned:
-            k.zk_attention_bf16_step(qkv.ptr, width, cache.k.ptr, cache.v.ptr, g.block_table, g.max_blocks,
+            k.zk_attention_bf16_once(qkv.ptr, width, cache.k.ptr, cache.v.ptr, g.block_table, g.max_blocks,
                                      ctx.q_start, ctx.ctx_len, o.ptr, ctx.R, ctx.n_multi, ctx.max_q_len,
                                      ctx.max_ctx, nh, nkv, hd, g.page_size, s.scale, cap, win,
                                      self.decode_chunk, ctx.workspace.ptr, ctx.workspace.nbytes, self.chunk,
                                      1 if self.unit_sink else 0, 1 if self.wide_weights else 0, 0, vd, self.keep,
-                                     ptr(self.sinks), head_gate, row_width, getattr(ctx, "portion_ctx", 0), ctx.stream)
+                                     ptr(self.sinks), head_gate, row_width, getattr(ctx, "portion_ctx", 0), values_once(ctx, cache), ctx.stream)
             if vfreq is not None:
                 k.zk_rotate_heads(o.ptr, ctx.positions, vfreq, T, nh, vd, inter, -1.0, ctx.stream)
         else:
@@ -387,11 +387,11 @@ class PagedAttention(Part):
         win = int(s.window) if s.window else 0
         if cache.v_transposed and ctx.tuned:
             # the matrix-core kernel; requests with more than one token come first in the batch
-            k.zk_attention_bf16_step(qkv.ptr, width, cache.k.ptr, cache.v.ptr, g.block_table, g.max_blocks,
+            k.zk_attention_bf16_once(qkv.ptr, width, cache.k.ptr, cache.v.ptr, g.block_table, g.max_blocks,
                                      ctx.q_start, ctx.ctx_len, o.ptr, ctx.R, ctx.n_multi, ctx.max_q_len,
                                      ctx.max_ctx, nh, nkv, hd, g.page_size, s.scale, cap, win,
                                      self.decode_chunk, ctx.workspace.ptr, ctx.workspace.nbytes, 0, 0, 0, 0, hd, 0,
-                                     None, None, 0, getattr(ctx, "portion_ctx", 0), ctx.stream)
+                                     None, None, 0, getattr(ctx, "portion_ctx", 0), values_once(ctx, cache), ctx.stream)
         else:
             k.zk_attention_plain(qkv.ptr, width, cache.k.ptr, cache.v.ptr, g.block_table,
                                  g.max_blocks, ctx.req_of_token, ctx.positions, o.ptr, T, nh, nkv,

@@ -5,6 +5,7 @@ import ctypes
 
 from ..runtime.device import BF16, F32, Tensor
 
+MEMORY_SIDE_CACHE = 256 << 20       # bytes
 
 EPILOGUES = {None: 0, "softcap": 1, "gelu_tanh": 2, "silu": 3, "relu": 5, "clamped_swiglu": 6, "relu2": 7, "gelu": 8}
 GATED = ("gelu_tanh", "silu", "relu", "clamped_swiglu")
@@ -22,6 +23,16 @@ def strip_flag(ctx, w: Tensor) -> int:
     if w.layout != "strip":
         return 0
     return 3 if getattr(ctx, "weights_read_once", False) else 1
+
+
+def values_once(ctx, cache) -> int:
+    """1 where decoded tokens' values of ``cache`` may be read past the caches: nothing reads them again before they have left those.
+    That is so for a layer whose keys and values are its own, in a step that passes through more than the cache on the memory's side
+    holds, by the weights alone or by what its requests have cached (an upper bound)."""
+    if getattr(cache, "shared", False) or getattr(cache, "lent", False):
+        return 0
+    return int(getattr(ctx, "weights_read_once", False) or
+               ctx.R * ctx.max_ctx * getattr(ctx, "cache_token_bytes", 0) > MEMORY_SIDE_CACHE)
 
 
 class PendingNorm:

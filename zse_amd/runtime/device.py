@@ -267,6 +267,8 @@ BF16_KERNEL_SIGNATURES = {
                                 _F, _F, _I, _I, _VP, _SZ, _I, _I, _I, _I, _I, _I, _VP, _VP, _I, _VP],
     "zk_attention_bf16_step": [_VP, _I, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I,
                                 _F, _F, _I, _I, _VP, _SZ, _I, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _VP],
+    "zk_attention_bf16_once": [_VP, _I, _VP, _VP, _VP, _I, _VP, _VP, _VP, _I, _I, _I, _I, _I, _I, _I, _I,
+                               _F, _F, _I, _I, _VP, _SZ, _I, _I, _I, _I, _I, _I, _VP, _VP, _I, _I, _I, _VP],
     "zk_moe_experts_grouped_identity": [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I, _I, _I, _I, _I, _F, _I, _I, _I, _VP,
                                         _VP, _I, _VP],
     "zk_gdelta_chunked": [_VP, _I, _I, _I, _VP, _I, _VP, _VP, _VP, _VP, _I, _I, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _I, _I, _I, _I,
