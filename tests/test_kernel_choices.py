@@ -87,3 +87,14 @@ def test_steps_that_pass_through_more_than_the_cache():
     assert values_once(step(weights_read_once=True), own) == 1
     for other in (S(shared=True, lent=False), S(shared=False, lent=True)):      # the same values are read again within the step
         assert values_once(step(weights_read_once=True), other) == 0
+
+
+# 32-bit products: tiles of 64 x 32 and 80 x 64 only where K is in whole steps of 32 (else they go through scratch memory), and not for the shortest K
+@pytest.mark.parametrize("M,N,K,tile", [(303, 8192, 1024, (80, 64)), (303, 8192, 1000, (64, 64)), (303, 8192, 1023, (64, 64)), (64, 8192, 1024, (64, 32)),
+                                        (64, 8192, 1000, (32, 32)), (128, 18432, 520, (32, 32)), (160, 2048, 512, (48, 32)), (150, 18432, 512, (32, 32))])
+def test_tiles_of_32_bit_products(M, N, K, tile):
+    """128 x 18,432 columns of K 520 took 36.8 us by 32 x 32 and 58.4 by 64 x 32, 160 x 2,048 of 512 10.0 by 48 x 32 and 11.5 by 64 x 32."""
+    rows, columns = C.c_int(), C.c_int()
+    assert library("kernels_f32").zk_gemm_plain_tile(M, N, K, C.byref(rows), C.byref(columns)) == 1
+    assert (rows.value, columns.value) == tile
+    assert K % 32 == 0 or tile not in ((64, 32), (80, 64))

@@ -227,14 +227,16 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_f32_kernel(const float* __res
   }
 }
 
-// LONG: K of 512 or more only.
-template <int MF, int NF, int H, int AHEAD, bool LONG = false>
+// LONG: K of 512 or more only.  STEPS: K in whole steps of 32 only.
+template <int MF, int NF, int H, int AHEAD, bool LONG = false, bool STEPS = false>
 static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc, int M, int N, int K,
                       hipStream_t s) {
   const int tiles_m = (M + 16 * MF - 1) / (16 * MF);
-  auto kernel = K % 4    ? gemm_f32_kernel<MF, NF, H, AHEAD, 1, 8>
-                : K % 32 ? gemm_f32_kernel<MF, NF, H, AHEAD, 2, 8>
-                         : gemm_f32_kernel<MF, NF, H, AHEAD, 3, 8>;
+  auto kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 3, 8>;
+  if constexpr (!STEPS) {
+    if (K % 4) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 1, 8>;
+    else if (K % 32) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 2, 8>;
+  }
   if constexpr (!LONG) {
     if (K < 4) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 0, 1>;
     else if (K <= 32) kernel = gemm_f32_kernel<MF, NF, H, AHEAD, 1, 1>;
@@ -253,34 +255,49 @@ static int launch_f32(const float* A, int lda, const float* W, float* C, int ldc
 // More than sixteen rows, K of 512 or more: the tile with the least price.  A launch takes as many rounds as the CU
 // with the most blocks has, whatever a block's registers would allow (303 x 1024 x 4096: 320 blocks of 32 x 32 61 us, 224 of
 // 48 x 32 41): a block alone already takes what its CU gets from its L2.  Microseconds, fitted to 17 to 2,048
-// rows by thirteen weights (512 to 18,432 columns, K of 1,024 to 9,216; the last two to 64 to 303 rows, K of 1,024 and 4,096): a round's start, and for every 1,024 of K
-// one round's time and that of several.  The tile it names takes 1.009 times the best one's time in the mean and
-// 0.81 of that of 32 x 32 and 64 x 64 alone, 0.98 times the old rule's speed at the least.  The last two fill rounds that the others leave
-// half empty (us, without and with them: 303 x 8192 x 1024, 640 blocks of 64 x 64 or 512 of 80 x 64, 77.6 and 66.9; 150 rows 45 and 36;
-// 64 x 8192 x 1024, 256 blocks of 64 x 32, 20.8 and 18.3; 303 x 1536 x 1024 19.6 and 17.2).  The sums are the same bits.
-struct F32Tile { int mf, nf; double start, lone, several; };
+// rows by thirteen weights (512 to 18,432 columns, K of 1,024 to 9,216; the last two to 17 to 2,048 rows of 512 to
+// 32,768 columns, K of 512 to 9,216): a round's start, and for every 1,024 of K one round's time and that of several.  The
+// tile it names takes 1.009 times the best one's time in the mean and 0.81 of that of 32 x 32 and 64 x 64 alone, 0.98
+// times the old rule's speed at the least.  The last two fill rounds that the others leave half empty (us, without and with
+// them: 303 x 8192 x 1024, 640 blocks of 64 x 64 or 512 of 80 x 64, 77.6 and 66.9; 150 rows 45 and 36;
+// 64 x 8192 x 1024, 256 blocks of 64 x 32, 20.8 and 18.3; 303 x 1536 x 1024 19.6 and 17.2), but for K in whole steps of
+// 32 only: else they keep a part of what they work on in scratch memory (128 x 18432 x 520 36.8 and 58.4, 64 x 8192 x 1000 17.3 and
+// 22.3, 303 x 18432 x 514 122 and 137).  64 x 32 up to K = 2,560 (256 x 2048 x 4096 62.9 by 32 x 32 and 66.4), the price of 80 x 64 with
+// 3 % on top: over some 450 shapes at which the choice then differs from the other tiles' it is 1.02 times their best at the most, 0.89 in the mean.
+// The sums are the same bits.  (``longest``: 0, or the longest K, in whole steps.)
+struct F32Tile { int mf, nf; double start, lone, several; int longest; };
 static const F32Tile f32_tiles[] = {
-    {1, 1, 0.88, 3.65, 3.47},
-    {1, 2, 1.39, 5.45, 5.16},
-    {2, 2, 0.74, 8.06, 7.45},
-    {3, 2, 2.54, 8.66, 8.68},
-    {2, 3, 2.71, 8.94, 8.55},
-    {3, 4, 0.00, 22.29, 21.65},
-    {4, 4, 2.23, 23.23, 22.63},
-    {4, 2, -1.5, 16.1, 16.9},
-    {5, 4, 0.0, 32.7, 32.0}};
+    {1, 1, 0.88, 3.65, 3.47, 0},
+    {1, 2, 1.39, 5.45, 5.16, 0},
+    {2, 2, 0.74, 8.06, 7.45, 0},
+    {3, 2, 2.54, 8.66, 8.68, 0},
+    {2, 3, 2.71, 8.94, 8.55, 0},
+    {3, 4, 0.00, 22.29, 21.65, 0},
+    {4, 4, 2.23, 23.23, 22.63, 0},
+    {4, 2, 2.28, 11.92, 14.20, 2560},
+    {5, 4, 7.54, 25.33, 25.27, 1 << 30}};
 static int f32_tile(int M, int N, int K) {
   int best = 0;
   double best_time = 1e30;
   const double t_mem = ((double)N * K + (double)M * K + (double)M * N) * 4e-6 / 5.0;
   for (int i = 0; i < (int)(sizeof(f32_tiles) / sizeof(f32_tiles[0])); i++) {
     const F32Tile& t = f32_tiles[i];
+    if (t.longest && (K % 32 || K > t.longest)) continue;
     const long blocks = (long)((M + 16 * t.mf - 1) / (16 * t.mf)) * ((N + 16 * t.nf - 1) / (16 * t.nf)), rounds = (blocks + 255) / 256;
     const double work = rounds * (t.start + (rounds == 1 ? t.lone : t.several) * K / 1024.0);
     const double time = sqrt(sqrt(work * work * work * work + t_mem * t_mem * t_mem * t_mem));
     if (time < best_time) best = i, best_time = time;
   }
   return best;
+}
+
+// The tile's rows and columns; for tests.
+extern "C" int zk_gemm_plain_tile(int M, int N, int K, int* rows, int* columns) {
+  if (M <= 16 || N <= 0 || K < 512) return 0;
+  const F32Tile& t = f32_tiles[f32_tile(M, N, K)];
+  *rows = 16 * t.mf;
+  *columns = 16 * t.nf;
+  return 1;
 }
 #endif  // ZSE_ACT_BF16
 
@@ -317,8 +334,8 @@ extern "C" int zk_gemm_plain(const void* A, int lda, const void* W, void* C, int
       case 4: return launch_f32<2, 3, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
       case 5: return launch_f32<3, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
       case 6: return launch_f32<4, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
-      case 7: return launch_f32<4, 2, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
-      default: return launch_f32<5, 4, 2, 2, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      case 7: return launch_f32<4, 2, 2, 2, true, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
+      default: return launch_f32<5, 4, 2, 2, true, true>(a, lda, w, (float*)C, ldc, M, N, K, s);
     }
   }
   if (M > 16 && blocks(4, 4) >= 1024) return launch_f32<4, 4, 1, 3>(a, lda, w, (float*)C, ldc, M, N, K, s);
