@@ -323,10 +323,8 @@ __global__ __launch_bounds__(256) void norm_add_norm_fast_kernel(
 // ask for all planes of partial sums at once, eight a turn.  With so few rows the kernel's time is
 // its trips to memory and its two block sums, not its bytes: 8 rows of 4,608 values that come as
 // eight planes (27B shapes) 2.9 us less a launch, a decode step at batch 8 of 2B shapes 2.46 -> 2.42
-// ms, of 9B shapes (14 layers) 2.47 -> 2.40 ms, 2B shapes at batch 32 4.51 -> 4.40 ms.  us, 256 threads and 1,024, rows as activations: of
-// 2,304 values 65 rows 3.6 and 3.0, 256 4.4 and 3.9, 512 5.4 and 5.3, 768 6.1 and 7.2, 2,048 12.4 and 16.6 (9 waves of 16 have values);
-// of 3,584 (14 of 16) 441 to 512 7.3 and 6.6, 768 8.3 and 8.8, 1,024 12.1 and 10.5, 2,048 26.9 and 21.8; of 4,608 512 8.5 and 8.5, 2,048 39.3 and 34.1; of 2,048
-// 256 3.5 and 3.5, 384 4.4 and 4.6.  The sums of the planes are the same bits; the two row sums are added up in another
+// ms, of 9B shapes (14 layers) 2.47 -> 2.40 ms, 2B shapes at batch 32 4.51 -> 4.40 ms.  norm_wide says where the line lies.
+// The sums of the planes are the same bits; the two row sums are added up in another
 // order than by 256 threads, so which of the two kernels serves a launch depends on the rows and
 // the width alone, never on whether planes come.
 template <int MAXV>
@@ -884,6 +882,25 @@ int zk_round_rows(const float* x, void* out, size_t n, void* stream) {
   return zk_launch_status("zk_round_rows");
 }
 
+// Whether rows of up to 8,192 values go by 1,024 threads each instead of 256: few rows (a block a CU or two), and many of widths whose
+// vectors fill most of the threads.  1,024 threads' share of the time of 256, rows as activations (as four planes):
+//   H        257 rows     384          512          768          1,024        2,048        4,096
+//   2,048    -            1.05         -            -            -            -            -
+//   2,560    0.94 (0.89)  0.96 (0.90)  1.00 (0.98)  1.18 (0.99)  1.19 (0.97)  1.31 (0.90)  1.26 (0.88)
+//   3,072    0.92 (0.92)  1.00 (0.95)  1.03 (0.92)  1.17 (0.95)  1.16 (0.97)  1.27 (0.88)  1.09 (0.89)
+//   3,584    0.80 (0.96)  0.87 (0.90)  0.91 (0.90)  1.06 (0.93)  0.86 (0.86)  0.90 (0.90)  0.76 (0.93)
+//   4,608    0.95 (1.09)  0.96 (0.98)  1.00 (0.99)  0.88 (0.95)  0.88 (0.99)  0.85 (0.97)  0.82 (0.98)
+//   6,144    0.63 (0.69)  0.65 (0.70)  0.68 (0.79)  0.63 (0.78)  0.61 (0.77)  0.57 (0.75)  0.54 (0.73)
+// 3,328 and 4,096 as 3,584, 4,352 and 5,120 as 4,608, 5,376 and 8,192 as 6,144; up to 256 rows 0.6 to 1.0 at each.  The 32-bit library
+// keeps to one kernel whatever the rows, so that its results stay the same bits however a request's tokens are cut into steps.
+static bool norm_wide(int T, int H) {
+  if (!ZSE_ACT_BF16 || H % 4 || H < 2048 || H > 8192) return false;
+  const int few = H <= 2048 ? 256 : H <= 2560 ? 512 : H <= 3072 ? 384 : H <= 4096 ? 512 : H <= 5120 ? 256 : 512;
+  return T <= few || (T >= 1024 && H > 3072);
+}
+
+int zk_norm_wide(int T, int H) { return norm_wide(T, H); }
+
 // sub_parts > 0: sub holds that many float planes of [T, H] partial sums instead of [T, H]
 // values of the activation type (see sub_value).  An output without w_next receives the new stream
 // itself, rounded to the activation type.
@@ -893,10 +910,7 @@ int zk_norm_add_norm(const void* sub, int sub_parts, const float* w_post, float 
   ZK_REQUIRE(T >= 0 && H > 0 && sub_parts >= 0, "zk_norm_add_norm: bad sizes");
   ZK_REQUIRE(w_next == nullptr || out != nullptr, "zk_norm_add_norm: next norm without output");
   if (T == 0) return 0;
-  if (ZSE_ACT_BF16 && H % 4 == 0 && H >= 2048 && H <= 8192 && (T <= 256 || (H > 2048 && T <= 512) || (H > 2560 && T >= 1024))) {
-    // few rows of at least 2,048 values, and many that fill the threads (see the kernel).  The 32-bit
-    // library keeps to one kernel whatever the rows, so that its results stay the same bits
-    // however a request's tokens are cut into steps.
+  if (norm_wide(T, H)) {
     hipStream_t st = (hipStream_t)stream;
     if (H <= 4096)
       norm_add_norm_wide_kernel<1><<<T, 1024, 0, st>>>(sub, sub_parts, w_post, eps_post, uo_post, h, w_next, eps_next,
