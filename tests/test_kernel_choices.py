@@ -108,3 +108,16 @@ def test_norms_by_1024_threads(T, H, wide):
     """2,048 rows of 3,072 values took 12.1 us by 256 threads and 15.3 by 1,024, 1,024 of 2,816 7.9 and 9.3, 320 of 5,120 as three planes 10.0 and 10.5."""
     assert library().zk_norm_wide(T, H) == wide
     assert library("kernels_f32").zk_norm_wide(T, H) == 0
+
+
+# strips of gate (and as many of up), rows; strips a block, waves a strip, steps a chunk
+@pytest.mark.parametrize("strips,M,cut", [(1, 17, (1, 8, 8)), (256, 64, (1, 8, 8)), (257, 17, (2, 4, 8)), (512, 64, (2, 4, 8)), (513, 1, (3, 4, 4)),
+                                          (768, 16, (3, 4, 4)), (769, 1, (4, 2, 4)), (1025, 64, (3, 4, 4)), (1152, 64, (3, 4, 4)), (1280, 17, (3, 4, 4)),
+                                          (1537, 64, (4, 2, 4)), (1792, 64, (4, 2, 4)), (2304, 64, (3, 4, 4)), (2560, 33, (2, 4, 8))])
+def test_blocks_of_gated_products(strips, M, cut):
+    """1,152 strips of K 3,072 at 64 rows took 54.9 us by two waves a strip, 68.6 by one strip a block and 48.8 by three; 1,792 71.8, 102.1 and, by four, 61.1."""
+    out = (C.c_int * 4)()
+    mid_cut = library().zk_gemm_bf16_mid_cut
+    mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
+    assert mid_cut(2, 0, M, 16 * strips, 3072, 4096, 320 << 20, out) == 1
+    assert tuple(out) == cut + (1,)

@@ -1372,15 +1372,17 @@ static int mid_ranges(int cblocks, int ksteps, int ch) {
 static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
   const int nstrips = (N + 15) / 16, ksteps = K / 32;
   if (gated) {
-    // Few long strips (a lone block would fetch 0.8 MB and more): in ranges, with a join (2,048 columns of K 8,192 at 24 and 64 rows 20.1 and 22.0 us, whole
-    // 22.2 and 30.8; 512 of 4,096 at 64 14.4 and 16.5, at 24 not: 11.9 and 11.5).  Else whole, as many strips a block as give the fullest CU the
-    // least, of equals the more: 256 strips one a block, 512 two, 576 three, 896 four, 2,304 three.
+    // Few long strips (a lone block would fetch 0.8 MB and more): in ranges, with a join (2,048 columns of K 8,192 at 24 and 64
+    // rows 20.1 and 22.0 us, whole 22.2 and 30.8; 512 of 4,096 at 64 14.4 and 16.5, at 24 not: 11.9 and 11.5).  Else whole: a strip a
+    // block up to 256 of them, and then as many of two to four as give the fullest CU the least, of equals the more: 512 strips
+    // two a block, 576 three, 896 four, 1,152 three, 1,792 four, 2,304 three.  (One a block has every strip fetch all of the
+    // activations: us, 32 and 64 rows, one and three a block, 1,152 strips of K 3,072 44 and 69, 43 and 49; 1,792, one and four 65 and
+    // 102, 57 and 61.)
     if (split_ok && M > 16 && nstrips <= 192 && (64.0 + 2 * M) * K > 780e3) return {4, 2, 8, mid_ranges((nstrips + 3) / 4, ksteps, 8)};
-    int spb = 1;
+    int spb = nstrips <= 256 ? 1 : 2;
     auto most = [&](int b) { return (long)(((nstrips + b - 1) / b + 255) / 256) * b; };
-    for (int b = 2; b <= 4; b++)
-      if (most(b) <= most(spb)) spb = b;
-    if (nstrips <= 256) spb = 1;
+    for (int b = 3; b <= 4; b++)
+      if (nstrips > 256 && most(b) <= most(spb)) spb = b;
     return spb == 1 ? MidCut{1, 8, 8, 1} : spb == 2 ? MidCut{2, 4, 8, 1} : spb == 3 ? MidCut{3, 4, 4, 1} : MidCut{4, 2, 4, 1};
   }
   // Thousands of strips (a head): two strips a block up to 16 rows, eight beyond, where the activations weigh more
