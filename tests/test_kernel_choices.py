@@ -121,3 +121,18 @@ def test_blocks_of_gated_products(strips, M, cut):
     mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
     assert mid_cut(2, 0, M, 16 * strips, 3072, 4096, 320 << 20, out) == 1
     assert tuple(out) == cut + (1,)
+
+
+def test_cuts_of_up_to_16_rows():
+    """Every product of up to 16 rows that the blocks of gemm_mid_kernel take has one of the four cuts that are built for so few."""
+    out = (C.c_int * 4)()
+    mid_cut = library().zk_gemm_bf16_mid_cut
+    mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
+    seen = set()
+    for epi, by_reader in ((0, 0), (0, 1), (1, 0), (4, 0), (2, 0)):
+        for strips in [*range(1, 1100), 1536, 2304, 4095, 4096, 16000]:
+            for K in (32, 96, 1024, 2048, 2304, 4096, 8192, 14336):
+                for M in (1, 16):
+                    if mid_cut(epi, by_reader, M, 16 * strips, K, 4096, 320 << 20, out):
+                        seen.add((epi == 2,) + tuple(out)[:3])
+    assert seen == {(True, 3, 4, 4), (True, 4, 2, 4), (False, 2, 8, 16), (False, 3, 4, 8)}

@@ -1444,14 +1444,23 @@ static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, i
     if (reads_once(w_strip)) ZK_MID_(MT_, SPB_, KW_, CH_, true);                         \
     else ZK_MID_(MT_, SPB_, KW_, CH_, false);                                            \
   } while (0)
+// 17 to 64 rows
 #define ZK_MID_ROWS(SPB_, KW_, CH_)                   \
   do {                                                \
-    if (mt == 1) ZK_MID(1, SPB_, KW_, CH_);           \
-    else if (mt == 2) ZK_MID(2, SPB_, KW_, CH_);      \
+    if (mt == 2) ZK_MID(2, SPB_, KW_, CH_);           \
     else if (mt == 3) ZK_MID(3, SPB_, KW_, CH_);      \
     else ZK_MID(4, SPB_, KW_, CH_);                   \
   } while (0)
-  if (cut.spb == 4 && cut.ch == 8) ZK_MID_ROWS(4, 2, 8);
+  if (mt == 1) {
+    // the cuts of mid_for_few
+    if constexpr (GATED) {
+      if (cut.spb == 3) ZK_MID(1, 3, 4, 4);
+      else ZK_MID(1, 4, 2, 4);
+    } else {
+      if (cut.spb == 2) ZK_MID(1, 2, 8, 16);
+      else ZK_MID(1, 3, 4, 8);
+    }
+  } else if (cut.spb == 4 && cut.ch == 8) ZK_MID_ROWS(4, 2, 8);
   else if constexpr (GATED) {
     if (cut.spb == 1) ZK_MID_ROWS(1, 8, 8);
     else if (cut.spb == 2) ZK_MID_ROWS(2, 4, 8);
@@ -1459,8 +1468,6 @@ static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, i
     else ZK_MID_ROWS(4, 2, 4);
   } else {
     if (cut.spb == 8) ZK_MID_ROWS(8, 1, 4);
-    else if (cut.spb == 2) ZK_MID(1, 2, 8, 16);
-    else if (cut.spb == 3) ZK_MID(1, 3, 4, 8);
     else ZK_MID_ROWS(4, 4, 4);
   }
 #undef ZK_MID_ROWS
