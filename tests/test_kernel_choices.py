@@ -136,3 +136,15 @@ def test_cuts_of_up_to_16_rows():
                     if mid_cut(epi, by_reader, M, 16 * strips, K, 4096, 320 << 20, out):
                         seen.add((epi == 2,) + tuple(out)[:3])
     assert seen == {(True, 3, 4, 4), (True, 4, 2, 4), (False, 2, 8, 16), (False, 3, 4, 8)}
+
+
+@pytest.mark.parametrize("strips,M,cut", [(1023, 17, (4, 2, 8)), (1024, 17, (4, 4, 4)), (1025, 17, (3, 4, 4)), (1536, 64, (3, 4, 4)), (1537, 48, (4, 2, 8)),
+                                          (1537, 49, (4, 4, 4)), (4095, 17, (4, 2, 8)), (4096, 17, (8, 1, 4)), (1024, 16, (2, 8, 16)), (16000, 1, (2, 8, 16))])
+def test_blocks_of_wide_products(strips, M, cut):
+    """1,152 strips of K 4,096 took 34.5 us at 32 rows by two waves a strip, 36.9 by four of four strips and 29.7 of three; 2,560 at 17 rows 69.0, 73.8 and, by
+    two waves a strip, 62.1."""
+    out = (C.c_int * 4)()
+    mid_cut = library().zk_gemm_bf16_mid_cut
+    mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
+    assert mid_cut(0, 0, M, 16 * strips, 4096, 4096, 320 << 20, out) == 1
+    assert tuple(out)[:3] == cut

@@ -1385,11 +1385,16 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
       if (nstrips > 256 && most(b) <= most(spb)) spb = b;
     return spb == 1 ? MidCut{1, 8, 8, 1} : spb == 2 ? MidCut{2, 4, 8, 1} : spb == 3 ? MidCut{3, 4, 4, 1} : MidCut{4, 2, 4, 1};
   }
-  // Thousands of strips (a head): two strips a block up to 16 rows, eight beyond, where the activations weigh more
-  // (256,000 columns of K 2,304, four strips and eight, 24 rows 195 and 192 us, 48 228 and 214, 64 253 and 224); where those would be one block a
-  // CU, four with sixteen waves (32,768 of 2,048, eight and four: 24 rows 32.0 and 24.7, 64 36.1 and 27.3).
+  // Thousands of strips (a head, wide layers): two strips a block up to 16 rows, eight beyond, where the activations weigh more
+  // (256,000 columns of K 2,304, four strips and eight, 24 rows 195 and 192 us, 48 228 and 214, 64 253 and 224).  Where those would be few
+  // blocks a CU, three strips of four waves each up to 1,536 (17 and 64 rows of K 4,096, eight strips, four of four waves, three: 1,088 strips
+  // 29.8 and 35.3, 33.3 and 43.1, 26.7 and 39.1; before the blocks had shapes 31.8 and 42.6), beyond them four with two waves each up to 48
+  // rows and with four from there on (2,560 strips of K 4,096 64 rows, 16 waves a block 72.9, eight 74.3; 17 rows 73.8 and 62.1; before
+  // 82.8 and 69.0).  The three rounds of 2,049 to 2,304 strips stay 2 to 8 % behind K of 4,096 and more at 17 to 32 rows.
   if (M <= 16 && nstrips >= 1024) return {2, 8, 16, 1};
   if (nstrips >= 4096) return {8, 1, 4, 1};
+  if (nstrips > 1024 && nstrips <= 1536) return {3, 4, 4, 1};
+  if (nstrips > 1536 && M <= 48) return {4, 2, 8, 1};
   if (nstrips >= 1024) return {4, 4, 4, 1};
   if (M <= 16) return {3, 4, 8, split_ok ? mid_ranges((nstrips + 2) / 3, ksteps, 8) : 1};
   const int cblocks = (nstrips + 3) / 4;
@@ -1468,6 +1473,7 @@ static int launch_mid(const void* A, int lda, const void* W, void* C, int ldc, i
     else ZK_MID_ROWS(4, 2, 4);
   } else {
     if (cut.spb == 8) ZK_MID_ROWS(8, 1, 4);
+    else if (cut.spb == 3) ZK_MID_ROWS(3, 4, 4);
     else ZK_MID_ROWS(4, 4, 4);
   }
 #undef ZK_MID_ROWS
