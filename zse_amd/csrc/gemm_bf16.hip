@@ -1406,16 +1406,22 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
   return {4, 2, 8, ks};
 }
 
-// Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us, straight
-// and so, 1, 8 and 16 rows.  Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3, 33.1, 33.4;
-// not 8,192 of 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.  Heads: 256,000 of 2,304
-// 170, 186, 249 and 174, 179, 206; not 32,768 of 1,024 12.2, 13.1, 15.8 and 14.1, 14.5, 15.1.  Long ones with the partial sums left to the reader:
-// 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of 36,864 53, 54, 69 and 53, 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1,
-// 9.3, 9.5.
+// Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us, straight and so, 1, 8 and
+// 16 rows.
+// Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3, 33.1, 33.4; not 8,192 of
+// 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.
+// Heads: 256,000 of 2,304 170, 186, 249 and 174, 179, 206; not 32,768 of 1,024 12.2, 13.1, 15.8 and 14.1, 14.5, 15.1.
+// Long ones with the partial sums left to the reader: 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of 36,864 53, 54, 69 and 53,
+// 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1, 9.3, 9.5.  Their share of the time straight, 1 and 8 rows, by strips of K 8,192, 11,008,
+// 14,336: 193 to 384 0.82 to 1.01; 400, where K stays whole below 12,288, 1.10 and 1.08, 1.09 and 1.05, 0.93 and 0.89; 512, whose 342 blocks
+// fill a third of a second round, 0.99 and 1.00, 1.04 and 1.05, 1.02 and 1.04; 544 to 768 0.87 to 1.00; 832 1.18 and 1.11, 1.17 and 1.14, 1.16
+// and 1.16; 896 to 1,023 0.99 to 1.09.
 static bool mid_for_few(bool gated, int N, int K, bool by_reader) {
   const int nstrips = (N + 15) / 16;
   if (gated) return nstrips > 512 && nstrips <= 1024;
-  return (nstrips >= 1024 && K >= 2048) || (by_reader && K >= 8192 && nstrips > 192);
+  if (nstrips >= 1024) return K >= 2048;
+  if (!by_reader || K < 8192 || nstrips <= 192) return false;
+  return nstrips <= 384 || (nstrips > 512 && nstrips <= 768) || (nstrips < 512 && mid_ranges((nstrips + 2) / 3, K / 32, 8) > 1);
 }
 
 // Bytes of the partial sums of one range.
