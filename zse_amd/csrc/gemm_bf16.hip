@@ -1409,7 +1409,10 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
 // Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us, straight and so, 1, 8 and
 // 16 rows.
 // Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3, 33.1, 33.4; not 8,192 of
-// 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.
+// 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.  Their share of the time straight, 1 and 8
+// rows, K of 1,024, 2,048, 3,072, 4,096: 513 to 768 strips 0.86 to 1.03 and 0.84 to 0.99; 800 0.96, 0.94, 0.89, 0.97 and 0.91, 0.89, 0.85, 0.96; 896
+// 1.01, 1.00, 0.96, 1.06 and 0.94, 0.96, 0.91, 1.01; 960 1.00, 1.01, 0.95, 1.02 and 0.95, 0.98, 0.93, 1.01; 1,024 1.03, 1.04, 0.99, 1.02 and 0.99, 1.03,
+// 0.95, 1.00.
 // Heads: 256,000 of 2,304 170, 186, 249 and 174, 179, 206; not 32,768 of 1,024 12.2, 13.1, 15.8 and 14.1, 14.5, 15.1.
 // Long ones with the partial sums left to the reader: 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of 36,864 53, 54, 69 and 53,
 // 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1, 9.3, 9.5.  Their share of the time straight, 1 and 8 rows, by strips of K 8,192, 11,008,
@@ -1418,7 +1421,7 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
 // and 1.16; 896 to 1,023 0.99 to 1.09.
 static bool mid_for_few(bool gated, int N, int K, bool by_reader) {
   const int nstrips = (N + 15) / 16;
-  if (gated) return nstrips > 512 && nstrips <= 1024;
+  if (gated) return nstrips > 512 && nstrips <= (K % 4096 ? 960 : 800);
   if (nstrips >= 1024) return K >= 2048;
   if (!by_reader || K < 8192 || nstrips <= 192) return false;
   return nstrips <= 384 || (nstrips > 512 && nstrips <= 768) || (nstrips < 512 && mid_ranges((nstrips + 2) / 3, K / 32, 8) > 1);
