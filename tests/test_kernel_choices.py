@@ -171,3 +171,16 @@ def test_few_rows_of_gated_products(strips, K, blocks):
     mid_cut.argtypes = [C.c_int] * 5 + [C.c_void_p, C.c_size_t, C.POINTER(C.c_int)]
     for M in (1, 16):
         assert mid_cut(2, 0, M, 16 * strips, K, None, 0, out) == blocks
+
+
+# strips, K, planes of partial sums; whether the gated, the rotating product makes the row in front of it
+@pytest.mark.parametrize("strips,K,planes,gated,rotating", [
+    (256, 2304, 6, 1, 1), (288, 2304, 4, 1, 1), (288, 2304, 5, 0, 0), (511, 4096, 4, 1, 1), (512, 4096, 6, 1, 1), (576, 2304, 0, 1, 1), (576, 2304, 1, 1, 0),
+    (576, 3072, 0, 0, 1), (576, 3584, 0, 1, 1), (576, 3840, 0, 0, 1), (640, 2048, 1, 1, 0), (896, 2048, 0, 1, 1), (896, 3584, 0, 0, 1), (896, 4096, 1, 0, 0),
+    (896, 4096, 0, 1, 1), (1152, 3584, 0, 1, 1), (1152, 3584, 2, 0, 0), (1152, 1024, 6, 1, 1), (576, 1024, 0, 0, 1), (256, 4352, 0, 0, 0),
+    (256, 2048 + 32, 0, 0, 0), (256, 2304, 7, 0, 0)])
+def test_norms_inside_products(strips, K, planes, gated, rotating):
+    """Gated 896 strips of K 3,584 took 36.0 us as two launches and 38.8 as one, 640 rotating ones of K 2,304 with four planes 13.7 and 15.4."""
+    lib = library()
+    assert bool(lib.zk_norm_product_supports(16 * strips, K, planes)) == gated
+    assert bool(lib.zk_norm_rope_product_supports(16 * strips, K, planes)) == rotating

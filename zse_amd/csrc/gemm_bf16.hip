@@ -1686,10 +1686,26 @@ static int row_norm_of(RowNorm& p, const void* sub, int sub_parts, const float* 
   return 0;
 }
 
-// N: the gated product's columns (0: the rotating product)
-extern "C" int zk_norm_product_supports(int N, int K, int sub_parts) {
-  return K > 0 && K % 256 == 0 && K <= 4096 && sub_parts <= 6 && (N == 0 || K >= 2048 || !mid_for_few(true, N, K, false));
+// Where that is no slower than the two launches (a chain of either, one row, K of 2,048 to 4,096; its share of their time by planes of
+// partial sums).  Below K of 2,048 0.7 to 0.96 everywhere.  Rotating: up to 256 strips 0.81 to 0.94; 288 to 448 0.76 to 0.92 with up to four
+// planes and 1.02 to 1.07 with six, whose loads no longer fit beside the weights'; 512 0.86 to 0.95; 576 to 896 0.81 to 1.00 without planes and
+// 0.97 to 1.17 with them (eight waves' rows by four).  Gated straight from memory likewise: 256 and 512 strips 0.85 to 0.95; 1,024 to 2,304
+// 0.94 to 1.01 without planes, 0.93 to 1.05 with them.  Gated by blocks: of three strips K 2,048 0.92 to 0.99, 2,304 to 2,816 0.95 to 1.03, 3,072
+// 1.01 to 1.07, 3,328 and 3,584 0.97 to 1.02, 3,840 and 4,096 1.01 to 1.05; of four 2,048 0.97 to 1.00, beyond 1.00 to 1.11.
+static bool norm_product_pays(bool gated, int N, int K, int sub_parts) {
+  if (K <= 0 || K % 256 || K > 4096 || sub_parts > 6) return false;
+  const int nstrips = N / 16;
+  if (gated && mid_for_few(true, N, K, false)) {
+    if (K < 2048) return false;
+    return mid_cut(true, 1, N, K, false).spb == 3 ? K <= 2816 || (K > 3072 && K <= 3584) : K <= 2048;
+  }
+  if (K < 2048) return true;
+  return nstrips < 512 ? sub_parts <= 4 || nstrips <= 256 : nstrips == 512 || sub_parts == 0;
 }
+
+// Whether zk_norm_gated_bf16 (N columns), or zk_norm_qkv_rope_bf16 (N columns of q, k and v), is to take a row of so many planes.
+extern "C" int zk_norm_product_supports(int N, int K, int sub_parts) { return norm_product_pays(true, N, K, sub_parts); }
+extern "C" int zk_norm_rope_product_supports(int N, int K, int sub_parts) { return norm_product_pays(false, N, K, sub_parts); }
 
 #define ZK_NORM_MODES(NW_, SLOTS_, WIDE_)                                                          \
   do {                                                                                             \

@@ -333,11 +333,12 @@ class PagedAttention(Part):
     def takes_pending_norm(self, ctx, size: int, planes: int) -> bool:
         """Whether the product of one row that rotates and stores its results serves this mixer (and then makes its own norm)."""
         s, tables = self.spec, self.position.rotary_tables()
+        width = (s.num_heads + 2 * (0 if self.shared_kv else s.num_kv_heads)) * s.head_dim
         return bool(not self.general and type(self).forward is PagedAttention.forward and size == s.hidden_size and
                     type(self).between_product_and_rotation is PagedAttention.between_product_and_rotation and
                     tables is not None and tuned_gemm(ctx, s.hidden_size) and self.w_qkv.layout == "strip" and
                     ctx.k.zk_qkv_rope_bf16_supports(1, s.hidden_size, s.head_dim, tables[1]) and
-                    ctx.k.zk_norm_product_supports(0, size, planes))
+                    ctx.k.zk_norm_rope_product_supports(width, size, planes))
 
     def forward(self, ctx, x: Tensor, cache) -> Tensor:
         if self.general:

@@ -385,9 +385,10 @@ class KernelLibrary:
             self._dll.zk_qkv_rope_rows_bf16_supports.restype = C.c_int
             self._dll.zk_qkv_rope_rows_bf16_supports.argtypes = [_I, _I, _I, _I]
             self.zk_qkv_rope_rows_bf16_supports = self._dll.zk_qkv_rope_rows_bf16_supports
-            self._dll.zk_norm_product_supports.restype = C.c_int
-            self._dll.zk_norm_product_supports.argtypes = [_I, _I, _I]
-            self.zk_norm_product_supports = self._dll.zk_norm_product_supports
+            for name in ("zk_norm_product_supports", "zk_norm_rope_product_supports"):
+                fn = getattr(self._dll, name)
+                fn.restype, fn.argtypes = C.c_int, [_I, _I, _I]
+                setattr(self, name, fn)
             self._dll.zk_head_pick_bf16_workspace.restype = C.c_size_t
             self._dll.zk_head_pick_bf16_workspace.argtypes = [_I, _I]
             self.zk_head_pick_bf16_workspace = self._dll.zk_head_pick_bf16_workspace
