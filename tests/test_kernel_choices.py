@@ -184,3 +184,15 @@ def test_norms_inside_products(strips, K, planes, gated, rotating):
     lib = library()
     assert bool(lib.zk_norm_product_supports(16 * strips, K, planes)) == gated
     assert bool(lib.zk_norm_rope_product_supports(16 * strips, K, planes)) == rotating
+
+
+# rows, columns, K, channels of a head
+@pytest.mark.parametrize("M,N,K,hd,pays", [(17, 1536, 2560, 128, 1), (17, 1536, 3072, 128, 0), (64, 4096, 2304, 256, 1), (64, 4096, 3584, 256, 1),
+                                           (64, 4096, 4096, 256, 0), (64, 6144, 4096, 128, 1), (17, 6144, 4608, 128, 0), (64, 8192, 3584, 256, 1),
+                                           (64, 8192, 4608, 128, 1), (64, 8192, 5120, 128, 0), (32, 10240, 2304, 128, 1), (33, 10240, 512, 128, 0),
+                                           (17, 10240, 4096, 256, 0)])
+def test_rotating_products_of_17_to_64_rows(M, N, K, hd, pays):
+    """1,536 columns of K 4,096 took 11.1 and 13.7 us at 17 and 64 rows as two launches, 12.7 and 17.4 as one; 10,240 of 4,096 at 64 26.8 and 35.6."""
+    lib = library()
+    assert lib.zk_qkv_rope_rows_bf16_pays(M, N, K, hd) == pays
+    assert lib.zk_qkv_rope_rows_bf16_supports(M, K, hd, hd) == 1        # what it can do is another matter

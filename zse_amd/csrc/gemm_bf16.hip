@@ -1639,6 +1639,15 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
 // with K in ranges and the rotation that adds them up it is a launch less (us, 24, 40 and 64 rows, two launches and this: 4,096 columns of K
 // 2,304 11.3, 12.5, 13.8 and 9.8, 11.2, 12.4; 8,192 of 3,584 16.7, 18.0, 20.3 and 14.3, 16.1, 18.9; 1,536 of 1,024 9.8, 10.4, 11.8 and 5.8, 6.7, 7.3).  Rounds
 // to 16 bits in front of the rotation, as those do.
+// K whole has an end where the ranges fill the chip better (this one's share of the two launches' time, 17 to 64 rows, heads of 64 and 128
+// channels, of 256 in brackets): 96 to 320 strips K 2,304 0.82 to 1.03 (0.59 to 0.90), 3,072 0.93 to 1.11 (0.74 to 0.98), 3,584 0.99 to 1.17
+// (0.73 to 1.02), 4,096 0.98 to 1.24 (0.85 to 1.08), 5,120 1.10 to 1.40 (0.92 to 1.25); 384 and 448 4,096 0.90 to 0.98 (0.85 to 0.95), 4,608 0.98 to
+// 1.09; 512 4,608 0.95 to 1.02, 5,120 0.97 to 1.05; 640 up to 32 rows 768 to 2,304 0.79 to 1.01, 3,072 0.95 to 1.05, from 33 rows 1.03 to 1.40.
+extern "C" int zk_qkv_rope_rows_bf16_pays(int M, int N, int K, int hd) {
+  const int strips = N / 16;
+  return K <= (strips > 512 ? (M <= 32 ? 2304 : 0) : strips >= 480 ? 4608 : strips >= 384 ? 4096 : hd >= 256 ? 3584 : 2560);
+}
+
 extern "C" int zk_qkv_rope_rows_bf16_supports(int M, int K, int hd, int rotary_dim) {
   return M > 16 && M <= 64 && K > 0 && K % 32 == 0 && hd % 16 == 0 && rotary_dim == hd;
 }

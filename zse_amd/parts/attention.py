@@ -326,7 +326,8 @@ class PagedAttention(Part):
             return None
         if k.zk_qkv_rope_bf16_supports(T, s.hidden_size, s.head_dim, rotary_dim):
             return k.zk_qkv_rope_bf16
-        if self.w_qkv.layout == "strip" and k.zk_qkv_rope_rows_bf16_supports(T, s.hidden_size, s.head_dim, rotary_dim):
+        if (self.w_qkv.layout == "strip" and k.zk_qkv_rope_rows_bf16_supports(T, s.hidden_size, s.head_dim, rotary_dim) and
+                k.zk_qkv_rope_rows_bf16_pays(T, self.w_qkv.shape[0], s.hidden_size, s.head_dim)):
             return k.zk_qkv_rope_rows_bf16
         return None
 

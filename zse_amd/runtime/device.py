@@ -385,6 +385,9 @@ class KernelLibrary:
             self._dll.zk_qkv_rope_rows_bf16_supports.restype = C.c_int
             self._dll.zk_qkv_rope_rows_bf16_supports.argtypes = [_I, _I, _I, _I]
             self.zk_qkv_rope_rows_bf16_supports = self._dll.zk_qkv_rope_rows_bf16_supports
+            self._dll.zk_qkv_rope_rows_bf16_pays.restype = C.c_int
+            self._dll.zk_qkv_rope_rows_bf16_pays.argtypes = [_I, _I, _I, _I]
+            self.zk_qkv_rope_rows_bf16_pays = self._dll.zk_qkv_rope_rows_bf16_pays
             for name in ("zk_norm_product_supports", "zk_norm_rope_product_supports"):
                 fn = getattr(self._dll, name)
                 fn.restype, fn.argtypes = C.c_int, [_I, _I, _I]
