@@ -587,7 +587,7 @@ int zk_attention_bf16_once(const void* q, int q_stride, const void* kcache, cons
   p.q_start = q_start; p.ctx_len = ctx_len; p.out = (__bf16*)out;
   p.nh = nh; p.nkv = nkv; p.hd = hd; p.vd = vd; p.bs = bs; p.keep = keep;
   p.scale = scale; p.softcap = softcap; p.window = window;
-  p.from_window = 0; p.once = 0;
+  p.from_window = 0;
   p.mask_chunk = mask_chunk; p.sink = sink ? 1 : 0; p.wide_weights = wide_weights ? 1 : 0;
   p.sinks = sinks; p.gate = (const __bf16*)gate; p.gate_ld = gate_ld;
   p.bs_shift = 0;
@@ -642,7 +642,6 @@ int zk_attention_bf16_once(const void* q, int q_stride, const void* kcache, cons
     if (decode_on_narrow_tiles(nh, nkv, hd)) {
       // a block joins its four waves: one partial result per block of keys
       const bool long_blocks = decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk);
-      p.once = values_past_caches(once, bs, v_shift, long_blocks) ? 1 : 0;
       p.chunk = ATT_CHUNK;
       span = long_blocks ? 4 * p.chunk : ATT_DECODE_SPAN;
       grid.x = (max_ctx + span - 1) / span;
@@ -655,7 +654,8 @@ int zk_attention_bf16_once(const void* q, int q_stride, const void* kcache, cons
         grid.x = window_blocks;
       }
       p.part_ml = (float*)workspace + (size_t)n_dec * nh * p.nchunks * vd;
-      rc = launch_attn(long_blocks ? ATT_DECODE_LONG : ATT_DECODE, p, grid, s);
+      const bool past = values_past_caches(once, bs, v_shift, long_blocks);
+      rc = launch_attn(long_blocks ? (past ? ATT_DECODE_LONG_ONCE : ATT_DECODE_LONG) : past ? ATT_DECODE_ONCE : ATT_DECODE, p, grid, s);
     } else {
       rc = launch_attn(ATT_DECODE_WIDE, p, grid, s);
     }

@@ -55,7 +55,6 @@ struct AttnParams {
   const float* sinks;     // [nh] (may be null): exp(sinks[h]) joins head h's denominator, with no key and no value
   const __bf16* gate;     // (may be null) row t's numbers per head at gate + t * gate_ld; head h's output is
   int gate_ld;            // multiplied by the sigmoid of the h-th
-  int once;               // decoded tokens: values by loads that leave no trace in the caches (values_past_caches)
   int wide_weights;       // 1: a weight meets the values as two bf16 numbers, its rounded value and what the
                           // rounding left (16 bits of mantissa instead of 8; one more product a tile)
 };
@@ -1687,7 +1686,9 @@ __global__ __launch_bounds__(256, 2) void attn_decode_long_kernel(AttnParams p) 
 // One pair of sizes.  what: 0 decoded tokens on 32-wide tiles, 1 pairs of groups a block, 2 a group a block,
 // 3 shared tiles with four waves, 4 with eight, 5 with four and the keys in ranges, 6 decoded tokens
 // on 16-wide tiles (keys in whole 32s), 7 the same in blocks of 256 keys.
-enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE, ATT_DECODE_LONG, ATT_SHORT };
+enum AttnWhat { ATT_DECODE_WIDE, ATT_PAIRS, ATT_GROUPS, ATT_SHARED4, ATT_SHARED8, ATT_RANGES, ATT_DECODE, ATT_DECODE_LONG, ATT_SHORT,
+                // values past the caches (values_past_caches)
+                ATT_DECODE_ONCE, ATT_DECODE_LONG_ONCE };
 
 template <int HD16, int VD16, int NW, bool SPLIT>
 static int launch_shared_one(const AttnParams& p, dim3 grid, hipStream_t s) {
@@ -1761,6 +1762,7 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
         return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
       }
     case ATT_DECODE:
+    case ATT_DECODE_ONCE:
       if constexpr (HD16 % 2 == 0) {
         const size_t lds = (size_t)4 * (p.nh / p.nkv) * p.vd * sizeof(float) + (size_t)4 * (HD16 / 2) * 64 * sizeof(bf16x8);
         static std::atomic<bool> prepared{false};
@@ -1772,15 +1774,16 @@ static int launch_sizes(int what, const AttnParams& p, dim3 grid, hipStream_t s)
             return zk_fail("zk_attention_bf16: the decode kernel's LDS was refused");
           prepared = true;
         }
-        if (p.once) attn_decode_kernel<HD16 / 2, VD16, true><<<grid, 256, lds, s>>>(p);
+        if (what == ATT_DECODE_ONCE) attn_decode_kernel<HD16 / 2, VD16, true><<<grid, 256, lds, s>>>(p);
         else attn_decode_kernel<HD16 / 2, VD16, false><<<grid, 256, lds, s>>>(p);
         break;
       } else {
         return zk_fail("zk_attention_bf16: the narrow tiles take keys in whole 32s");
       }
     case ATT_DECODE_LONG:
+    case ATT_DECODE_LONG_ONCE:
       if constexpr (HD16 % 2 == 0) {
-        if (p.once) attn_decode_long_kernel<HD16 / 2, VD16, true><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
+        if (what == ATT_DECODE_LONG_ONCE) attn_decode_long_kernel<HD16 / 2, VD16, true><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
         else attn_decode_long_kernel<HD16 / 2, VD16, false><<<grid, 256, decode_long_lds(p.nh / p.nkv, p.vd), s>>>(p);
         break;
       } else {

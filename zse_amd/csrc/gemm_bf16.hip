@@ -135,6 +135,13 @@ __device__ __forceinline__ bf16x8 load_weights(const void* p) {
   return load_maybe_once<ONCE>((const bf16x8*)p);
 }
 
+// An argument of those forms of a kernel that read it: what a kernel is launched with is written and fetched whether it looks at it or
+// not, and the launch's own numbers, which the compiler reads behind the arguments, move into another line (a norm's 64 bytes on every
+// product of up to 16 rows: steps of 2, 8 and 16 decoded tokens, six layers of width 1,024, 207, 231 and 302 us and 212, 238 and 304).
+struct Nothing {};
+template <bool READ, typename T>
+using ArgumentIf = std::conditional_t<READ, T, Nothing>;
+
 // ------------------------------------------------------------------ the norm in front of a product of one row
 // h_out = h + post(sub) and the row next(h_out), as zk_norm_add_norm makes them, to the bit: sub as activations or ``parts`` planes of
 // float sums.  Every block of the product works the row out for itself, while its first weights are on their way, and the first
@@ -345,7 +352,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const __bf16* __re
                                                           int M, int N, int K, int epi, float cap,
                                                           int w_strip, RopeStore rs,
                                                           float* __restrict__ partials = nullptr, int ksplit = 1,
-                                                          RowNorm norm = RowNorm{}) {
+                                                          ArgumentIf<NORM != 0, RowNorm> norm = {}) {
   static_assert(!NORM || (WHOLE && !SPLIT), "a row made here is multiplied whole");
   __shared__ __align__(16) __bf16 own_row[NORM ? 4096 : 8];
   __shared__ float own_sums[NORM ? 32 : 1];
@@ -1088,7 +1095,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
                                                                  const __bf16* __restrict__ W,
                                                                  void* __restrict__ C, int ldc, int c_is_f32,
                                                                  int M, int N, int K, int epi, float cap,
-                                                                 float* __restrict__ partials, int ksplit, RopeStore rs = RopeStore{}) {
+                                                                 float* __restrict__ partials, int ksplit, ArgumentIf<ROPE, RopeStore> rs = {}) {
   static_assert(!ROPE || (!GATED && KW >= MT), "a wave finishes sixteen rows");
   constexpr int NS = GATED ? 2 : 1;
   constexpr int T = SPB * KW * 64, WSTEPS = CH / KW;     // threads; steps of a chunk a wave multiplies
@@ -1115,7 +1122,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   // (ROPE) the strip's rows are eight places of a head's first half and their partners, as in the kernel above
   int head = 0, hpos = 0, slot = -1;
   float sn[4], cs[4];
-  if (ROPE) {
+  if constexpr (ROPE) {
     const int per_head = rs.hd / 16;
     head = strip_read / per_head;
     hpos = (strip_read % per_head) * 8;
