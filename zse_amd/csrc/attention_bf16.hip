@@ -508,18 +508,22 @@ static bool decode_in_long_blocks(int nh, int nkv, int hd, int vd, int bs, int m
          decode_long_lds(nh / nkv, vd) + (size_t)hd / 32 * 4 * 64 * 16 <= 64 * 1024;
 }
 
-// Whether decoded tokens' values go past the caches (common.h's load_once) where the caller says that nothing reads them again before
-// they have left those anyway: only where a wave's loads take whole lines of a channel's page and one block alone reads them.  Pages of up to
-// 32 keys (a wave of the long blocks: 16), no value head under several key heads.  us, 64 requests of 4,000 keys, plain loads and these, 8
-// heads over 4 of 256 channels, pages of 8, 16, 32, 64, 128 keys: 201, 198, 198, 206, 231 and 189, 188, 185, 239, 279; 32 over 16 of 128: 393,
-// 392, 388, 397, 400 and 370, 365, 359, 441, 532; 1 request of 8,000 in long blocks, 8 over 4 of 256, pages of 16, 32, 64: 18.4, 17.5, 21.7 and 17.7, 17.9,
-// 22.9; 16 of 64 over 8 whose pairs share values of 128, 64 of 4,000, pages of 16: 113 and 128.
+// Whether decoded tokens' values go past the caches (common.h's load_once) where the caller says that nothing reads
+// them again before they have left those anyway: only where a wave's loads take whole lines of a channel's page and
+// one block alone reads them.  Pages of up to 32 keys (a wave of the long blocks: 16), no value head under several
+// key heads.  us, 64 requests of 4,000 keys, plain loads and these, 8 heads over 4 of 256 channels, pages of 8, 16,
+// 32, 64, 128 keys: 201, 198, 198, 206, 231 and 189, 188, 185, 239, 279; 32 over 16 of 128: 393, 392, 388, 397, 400
+// and 370, 365, 359, 441, 532; 1 request of 8,000 in long blocks, 8 over 4 of 256, pages of 16, 32, 64: 18.4, 17.5,
+// 21.7 and 17.7, 17.9, 22.9; 16 of 64 over 8 whose pairs share values of 128, 64 of 4,000, pages of 16: 113 and 128.
 static bool values_past_caches(int once, int bs, int v_shift, bool long_blocks) {
   return once && v_shift == 0 && bs <= (long_blocks ? 16 : 32);
 }
 
-extern "C" int zk_attention_bf16_values_past_caches(int once, int nh, int nkv, int hd, int vd, int bs, int max_blocks, int decode_chunk, int v_shift) {
-  return decode_on_narrow_tiles(nh, nkv, hd) && values_past_caches(once, bs, v_shift, decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk));
+// For tests.
+extern "C" int zk_attention_bf16_values_past_caches(int once, int nh, int nkv, int hd, int vd, int bs, int max_blocks,
+                                                    int decode_chunk, int v_shift) {
+  const bool long_blocks = decode_in_long_blocks(nh, nkv, hd, vd, bs, max_blocks, decode_chunk);
+  return decode_on_narrow_tiles(nh, nkv, hd) && values_past_caches(once, bs, v_shift, long_blocks);
 }
 
 // The longest context the split variant takes for decoded tokens (the joining kernel keeps one

@@ -31,11 +31,14 @@ template <>
 __device__ __forceinline__ __bf16 from_f32<__bf16>(float x) { return (__bf16)x; }
 
 // A load of 8 or 16 bytes that one block reads once in a launch (a weight, a cached value), marked non-temporal: the
-// caches do not make room for it.  A streaming read reaches 6.5 to 6.8 TB/s so, 6.0 to 6.1 without (blocks of 4 or 8 waves, 100 MB to 1.6 GB);
-// a step of 8 decoded tokens of 27B shapes 10,830 -> 9,760 us, of 8 and 1 of 2B shapes 2,228 -> 2,160 and 1,655 -> 1,595.  Only for
-// memory that no later launch finds in the memory side's cache of 256 MB anyway (six layers of width 1,024, 250 MB in all, one decoded token 200 -> 204
-// us), and for whole 128-byte lines a load (weights in strips, transposed values): where a wave asks for a line's halves one after the other (rows of
-// cached keys), the second half comes from further away again (64 requests of 200 to 3,840 keys with the keys so too: 4,880 -> 5,010 us).
+// caches do not make room for it.  A streaming read reaches 6.5 to 6.8 TB/s so, 6.0 to 6.1 without (blocks of 4 or 8
+// waves, 100 MB to 1.6 GB); a step of 8 decoded tokens of 27B shapes 10,830 -> 9,760 us, of 8 and 1 of 2B shapes 2,228
+// -> 2,160 and 1,655 -> 1,595.
+// Only for memory that no later launch finds in the memory side's cache of 256 MB anyway (six layers of width 1,024,
+// 250 MB in all, one decoded token 200 -> 204 us; 8 requests of 500 keys in the cache 11.2 -> 11.4), which the runner
+// says, and for whole 128-byte lines a load, which the launch looks at: where a wave asks for a line's halves one after
+// the other (rows of cached keys, values in pages of 64 keys and more), the second half comes from further away again
+// (64 requests of 200 to 3,840 keys with the keys so too 4,880 -> 5,010 us; 64 of 4,000 keys in pages of 128 231 -> 279).
 template <typename T>
 __device__ __forceinline__ T load_once(const T* p) {
   typedef unsigned words __attribute__((ext_vector_type(sizeof(T) / 4)));

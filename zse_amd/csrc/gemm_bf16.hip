@@ -172,11 +172,14 @@ __device__ __forceinline__ f32x4 load4_act(const __bf16* p) {
   return f32x4{(float)x[0], (float)x[1], (float)x[2], (float)x[3]};
 }
 
-// The sums run as in norm_add_norm_wide_kernel (WIDE, H >= 2,048: 16 waves, a vector of four a thread) or norm_add_norm_fast_kernel (4
-// waves, up to two vectors a thread), whose waves this block's NW waves take in turn, SLOTS each.  H a multiple of 256.  PL: 0, or as many planes asked for (parts <= PL).
-// Two halves, because loads come back in the order in which they were asked for: what the row is made of first, then (by the caller) the first
-// weights, then the sums, which wait for the former alone (weights first: a step of the 2B shapes 1,550 us, so 1,514).  All that forks is fixed at compile time: with branches on the planes and the width the compiler
-// waits for every load and keeps rows in scratch memory (4,096 columns of K 2,304 8.0 and 9.1 us in a trace of a step).
+// The sums run as in norm_add_norm_wide_kernel (WIDE, H >= 2,048: 16 waves, a vector of four a thread) or
+// norm_add_norm_fast_kernel (4 waves, up to two vectors a thread), whose waves this block's NW waves take in turn,
+// SLOTS each.  H a multiple of 256.  PL: 0, or as many planes asked for (parts <= PL).
+// Two halves, because loads come back in the order in which they were asked for: what the row is made of first, then
+// (by the caller) the first weights, then the sums, which wait for the former alone (weights first: a step of the 2B
+// shapes 1,550 us, so 1,514).  All that forks is fixed at compile time: with branches on the planes and the width the
+// compiler waits for every load and keeps rows in scratch memory (4,096 columns of K 2,304 8.0 and 9.1 us in a trace
+// of a step).
 template <int NW, int SLOTS, bool WIDE, int PL>
 struct RowInWork {
   static_assert(WIDE ? NW * SLOTS <= 16 || SLOTS <= 2 : NW == 4 && SLOTS <= 2, "every wave of the kernels above has a place");
@@ -1413,19 +1416,21 @@ static MidCut mid_cut(bool gated, int M, int N, int K, bool split_ok) {
   return {4, 2, 8, ks};
 }
 
-// Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us, straight and so, 1, 8 and
-// 16 rows.
-// Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3, 33.1, 33.4; not 8,192 of
-// 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105, 100, 101.  Their share of the time straight, 1 and 8
-// rows, K of 1,024, 2,048, 3,072, 4,096: 513 to 768 strips 0.86 to 1.03 and 0.84 to 0.99; 800 0.96, 0.94, 0.89, 0.97 and 0.91, 0.89, 0.85, 0.96; 896
-// 1.01, 1.00, 0.96, 1.06 and 0.94, 0.96, 0.91, 1.01; 960 1.00, 1.01, 0.95, 1.02 and 0.95, 0.98, 0.93, 1.01; 1,024 1.03, 1.04, 0.99, 1.02 and 0.99, 1.03,
-// 0.95, 1.00.
+// Which products of up to 16 rows take the blocks above; the others feed every wave straight from memory.  us,
+// straight and so, 1, 8 and 16 rows.
+// Gated: 9,216 columns of K 2,304 16.9, 17.4, 18.9 and 15.7, 15.7, 16.5, 14,336 of 3,584 33.9, 33.2, 37.2 and 33.3,
+// 33.1, 33.4; not 8,192 of 2,048 12.6, 12.8, 13.7 and 13.1, 13.1, 13.2, nor 36,864 of 4,608 102, 98, 104 and 105,
+// 100, 101.  Their share of the time straight, 1 and 8 rows, K of 1,024, 2,048, 3,072, 4,096: 513 to 768 strips 0.86
+// to 1.03 and 0.84 to 0.99; 800 0.96, 0.94, 0.89, 0.97 and 0.91, 0.89, 0.85, 0.96; 896 1.01, 1.00, 0.96, 1.06 and
+// 0.94, 0.96, 0.91, 1.01; 960 1.00, 1.01, 0.95, 1.02 and 0.95, 0.98, 0.93, 1.01; 1,024 1.03, 1.04, 0.99, 1.02 and
+// 0.99, 1.03, 0.95, 1.00.
 // Heads: 256,000 of 2,304 170, 186, 249 and 174, 179, 206; not 32,768 of 1,024 12.2, 13.1, 15.8 and 14.1, 14.5, 15.1.
-// Long ones with the partial sums left to the reader: 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of 36,864 53, 54, 69 and 53,
-// 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1, 9.3, 9.5.  Their share of the time straight, 1 and 8 rows, by strips of K 8,192, 11,008,
-// 14,336: 193 to 384 0.82 to 1.01; 400, where K stays whole below 12,288, 1.10 and 1.08, 1.09 and 1.05, 0.93 and 0.89; 512, whose 342 blocks
-// fill a third of a second round, 0.99 and 1.00, 1.04 and 1.05, 1.02 and 1.04; 544 to 768 0.87 to 1.00; 832 1.18 and 1.11, 1.17 and 1.14, 1.16
-// and 1.16; 896 to 1,023 0.99 to 1.09.
+// Long ones with the partial sums left to the reader: 3,584 of 14,336 17.7, 19.2, 23.5 and 17.2, 17.5, 18.2, 4,608 of
+// 36,864 53, 54, 69 and 53, 51, 52; not 2,304 of 9,216 in five ranges 8.6, 9.2, 11.0 and 9.1, 9.3, 9.5.  Their share
+// of the time straight, 1 and 8 rows, by strips of K 8,192, 11,008, 14,336: 193 to 384 0.82 to 1.01; 400, where K
+// stays whole below 12,288, 1.10 and 1.08, 1.09 and 1.05, 0.93 and 0.89; 512, whose 342 blocks fill a third of a
+// second round, 0.99 and 1.00, 1.04 and 1.05, 1.02 and 1.04; 544 to 768 0.87 to 1.00; 832 1.18 and 1.11, 1.17 and
+// 1.14, 1.16 and 1.16; 896 to 1,023 0.99 to 1.09.
 static bool mid_for_few(bool gated, int N, int K, bool by_reader) {
   const int nstrips = (N + 15) / 16;
   if (gated) return nstrips > 512 && nstrips <= (K % 4096 ? 960 : 800);
@@ -1642,14 +1647,16 @@ extern "C" int zk_qkv_rope_bf16(const void* A, int lda, const void* W, void* Q, 
   return zk_launch_status("zk_qkv_rope_bf16");
 }
 
-// The same for 17 to 64 rows (weights in strips): a strip of a head's places and their partners a block, or two, K whole.  Against the product
-// with K in ranges and the rotation that adds them up it is a launch less (us, 24, 40 and 64 rows, two launches and this: 4,096 columns of K
-// 2,304 11.3, 12.5, 13.8 and 9.8, 11.2, 12.4; 8,192 of 3,584 16.7, 18.0, 20.3 and 14.3, 16.1, 18.9; 1,536 of 1,024 9.8, 10.4, 11.8 and 5.8, 6.7, 7.3).  Rounds
-// to 16 bits in front of the rotation, as those do.
-// K whole has an end where the ranges fill the chip better (this one's share of the two launches' time, 17 to 64 rows, heads of 64 and 128
-// channels, of 256 in brackets): 96 to 320 strips K 2,304 0.82 to 1.03 (0.59 to 0.90), 3,072 0.93 to 1.11 (0.74 to 0.98), 3,584 0.99 to 1.17
-// (0.73 to 1.02), 4,096 0.98 to 1.24 (0.85 to 1.08), 5,120 1.10 to 1.40 (0.92 to 1.25); 384 and 448 4,096 0.90 to 0.98 (0.85 to 0.95), 4,608 0.98 to
-// 1.09; 512 4,608 0.95 to 1.02, 5,120 0.97 to 1.05; 640 up to 32 rows 768 to 2,304 0.79 to 1.01, 3,072 0.95 to 1.05, from 33 rows 1.03 to 1.40.
+// The same for 17 to 64 rows (weights in strips): a strip of a head's places and their partners a block, or two, K
+// whole.  Against the product with K in ranges and the rotation that adds them up it is a launch less (us, 24, 40 and
+// 64 rows, two launches and this: 4,096 columns of K 2,304 11.3, 12.5, 13.8 and 9.8, 11.2, 12.4; 8,192 of 3,584 16.7,
+// 18.0, 20.3 and 14.3, 16.1, 18.9; 1,536 of 1,024 9.8, 10.4, 11.8 and 5.8, 6.7, 7.3).  Rounds to 16 bits in front of
+// the rotation, as those do.
+// K whole has an end where the ranges fill the chip better (this one's share of the two launches' time, 17 to 64
+// rows, heads of 64 and 128 channels, of 256 in brackets): 96 to 320 strips K 2,304 0.82 to 1.03 (0.59 to 0.90),
+// 3,072 0.93 to 1.11 (0.74 to 0.98), 3,584 0.99 to 1.17 (0.73 to 1.02), 4,096 0.98 to 1.24 (0.85 to 1.08), 5,120 1.10
+// to 1.40 (0.92 to 1.25); 384 and 448 4,096 0.90 to 0.98 (0.85 to 0.95), 4,608 0.98 to 1.09; 512 4,608 0.95 to 1.02,
+// 5,120 0.97 to 1.05; 640 up to 32 rows 768 to 2,304 0.79 to 1.01, 3,072 0.95 to 1.05, from 33 rows 1.03 to 1.40.
 extern "C" int zk_qkv_rope_rows_bf16_pays(int M, int N, int K, int hd) {
   const int strips = N / 16;
   return K <= (strips > 512 ? (M <= 32 ? 2304 : 0) : strips >= 480 ? 4608 : strips >= 384 ? 4096 : hd >= 256 ? 3584 : 2560);
@@ -1689,8 +1696,10 @@ extern "C" int zk_qkv_rope_rows_bf16(const void* A, int lda, const void* W, void
   return zk_launch_status("zk_qkv_rope_rows_bf16");
 }
 
-// The two products behind a norm, for one row that the product makes itself: what zk_norm_add_norm (sub, up to 6 planes, w_post, h, w_next) followed by zk_qkv_rope_bf16, or by zk_gemm_bf16 with a gated epilogue, gives, to the bit.  h_out: the new stream,
-// elsewhere than h.  sub must not lie where the product writes.  Weights in strips, K a multiple of 256 up to 4,096.
+// The two products behind a norm, for one row that the product makes itself: what zk_norm_add_norm (sub, up to 6
+// planes, w_post, h, w_next) followed by zk_qkv_rope_bf16, or by zk_gemm_bf16 with a gated epilogue, gives, to the
+// bit.  h_out: the new stream, elsewhere than h.  sub must not lie where the product writes.  Weights in strips, K a
+// multiple of 256 up to 4,096.
 static int row_norm_of(RowNorm& p, const void* sub, int sub_parts, const float* w_post, float eps_post, int uo_post, const float* h, float* h_out,
                        const float* w_next, float eps_next, int uo_next, int K) {
   ZK_REQUIRE(K > 0 && K % 256 == 0 && K <= 4096, "zk_norm product: K must be a multiple of 256 up to 4096");
@@ -2025,9 +2034,10 @@ static int gemm_bf16_run(const void* A, int lda, const void* W, void* C, int ldc
 #undef ZK_TILE_
 }
 
-// Which tile (its number in tile_shapes) and how many ranges of K, of the last round's tiles alone, a product
-// of more than 64 rows by weights in strips, K a multiple of 64, takes with the standard workspace
-// (``by_reader``: the caller passes ``parts``), and which tile the columns behind the whole rounds take (-1: the same).  For tests that mean to reach each of them.
+// Which tile (its number in tile_shapes) and how many ranges of K, of the last round's tiles alone, a product of more
+// than 64 rows by weights in strips, K a multiple of 64, takes with the standard workspace (``by_reader``: the caller
+// passes ``parts``), and which tile the columns behind the whole rounds take (-1: the same).  For tests that mean to
+// reach each of them.
 extern "C" int zk_gemm_bf16_tile_cut(int gated, int by_reader, int M, int N, int K, int* shape, int* ks,
                                      int* tail_ks, int* rest) {
   ZK_REQUIRE(M > 64 && N > 0 && K > 0 && K % 64 == 0, "zk_gemm_bf16_tile_cut: no tile product of this size");
