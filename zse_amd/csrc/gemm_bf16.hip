@@ -1093,6 +1093,29 @@ __device__ __forceinline__ void mid_store(const f32x4& v, const f32x4& up, int m
   }
 }
 
+// Chains of products that a wave adds up side by side, by its steps of a chunk and by the turns of the loop: where
+// fewer waves walk K than before the blocks had shapes, or ranges of it are gone, no sum has longer chains than then.
+// The relative error against 64 bits, before, with one chain a wave and so: a head of 256,000 columns of K 2,304 at 17
+// to 64 rows 2.0e-7, 2.9e-7 and 2.0e-7; 4,608 columns of K 8,192 at one row, sums left to the reader, 1.1e-7, 1.9e-7
+// and 1.05e-7; gated 14,336 of 2,048 at up to 16 rows 1.87e-7, 2.64e-7 and 1.88e-7; gated 2,048 of 4,096 at 17 rows
+// 1.5e-7, 1.9e-7 and 1.3e-7.  The times are the same.
+template <int MT, int SPB, int KW, int CH>
+struct MidChains {
+  static constexpr int by_step = KW == 1 || (MT == 1 && CH == 2 * KW && SPB > 2) ? 2 : 1;
+  static constexpr int by_turn = KW == 8 && CH == 8 ? 3 : MT == 1 && SPB == 3 && KW == 4 && CH == 8 ? 2 : 1;
+  static constexpr int all = by_step * by_turn;
+};
+
+// t[0] + ... + t[N - 1], neighbours first
+template <int N>
+__device__ __forceinline__ f32x4 neighbours_sum(f32x4 (&t)[N]) {
+#pragma unroll
+  for (int w = 1; w < N; w *= 2)
+#pragma unroll
+    for (int k = 0; k + w < N; k += 2 * w) t[k] += t[k + w];
+  return t[0];
+}
+
 template <int MT, bool GATED, int SPB, int KW, int CH, bool ONCE, bool ROPE = false>
 __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* __restrict__ A, int lda,
                                                                  const __bf16* __restrict__ W,
@@ -1132,11 +1155,14 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
     const int row = head * rs.hd + hpos + (r < 8 ? r : rs.hd / 2 + r - 8);
     wp[0] = W + (size_t)(row / 16) * ksteps * 512 + (16 * kq + row % 16) * 8;
   }
-  f32x4 acc[NS][MT];
+  using Chains = MidChains<MT, SPB, KW, CH>;
+  f32x4 acc[NS][MT][Chains::all];
 #pragma unroll
   for (int g = 0; g < NS; g++)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[g][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int c = 0; c < Chains::all; c++) acc[g][mt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // Every load is issued, none under a condition: a step past the range reads the range's last
   // step again, a row past M row M - 1; activations outside are set to zero afterwards, which
@@ -1165,7 +1191,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
       for (int g = 0; g < NS; g++)
         wf[g][s] = load_weights<ONCE>(wp[g] + (size_t)min(s0 + kpart * WSTEPS + s, s_end - 1) * 512);
   };
-  auto multiply = [&](int buf, const bf16x8 (&wf)[NS][WSTEPS]) {
+  auto multiply = [&](int buf, auto turn, const bf16x8 (&wf)[NS][WSTEPS]) {
 #pragma unroll
     for (int s = 0; s < WSTEPS; s++)
 #pragma unroll
@@ -1173,7 +1199,8 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
         const bf16x8 af = *(const bf16x8*)(&sA[buf][mt * 16 + r][(kpart * WSTEPS + s) * 32 + kq * 8]);
 #pragma unroll
         for (int g = 0; g < NS; g++)
-          acc[g][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af, acc[g][mt], 0, 0, 0);
+          acc[g][mt][turn % Chains::by_turn * Chains::by_step + s % Chains::by_step] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[g][s], af, acc[g][mt][turn % Chains::by_turn * Chains::by_step + s % Chains::by_step], 0, 0, 0);
       }
   };
 
@@ -1199,31 +1226,31 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   }
   stash_a(0, ra0);
   __syncthreads();
-#define ZK_MID_TURN(BUF, WCUR, WNEXT2, RA_NEXT2, RA_NEXT1)    \
+#define ZK_MID_TURN(TURN, WCUR, WNEXT2, RA_NEXT2, RA_NEXT1)   \
   fetch_a(s0 + 2 * CH, RA_NEXT2);                             \
   fetch_w(s0 + 2 * CH, WNEXT2);                               \
-  multiply(BUF, WCUR);                                        \
+  multiply(TURN % 3, std::integral_constant<int, TURN>{}, WCUR); \
   s0 += CH;                                                   \
   if (s0 >= s_end) break;                                     \
-  stash_a((BUF + 1) % 3, RA_NEXT1);                           \
+  stash_a((TURN + 1) % 3, RA_NEXT1);                          \
   __syncthreads();
   for (int s0 = s_begin;;) {
     ZK_MID_TURN(0, w0, w2, ra0, ra1)
     ZK_MID_TURN(1, w1, w0, ra1, ra0)
     ZK_MID_TURN(2, w2, w1, ra0, ra1)
-    ZK_MID_TURN(0, w0, w2, ra1, ra0)
-    ZK_MID_TURN(1, w1, w0, ra0, ra1)
-    ZK_MID_TURN(2, w2, w1, ra1, ra0)
+    ZK_MID_TURN(3, w0, w2, ra1, ra0)
+    ZK_MID_TURN(4, w1, w0, ra0, ra1)
+    ZK_MID_TURN(5, w2, w1, ra1, ra0)
   }
 #undef ZK_MID_TURN
   // The waves of a strip lay their sums down (the activation buffers are free once every wave has left the
-  // loop) and share the rows out among themselves: sixteen rows a wave, the sums in the order of the chunk's parts.
+  // loop) and share the rows out among themselves: sixteen rows a wave, neighbouring parts of the chunks first.
   __syncthreads();
   f32x4* sums = (f32x4*)lds + ((size_t)place * KW * NS * MT) * 64 + lane;
 #pragma unroll
   for (int g = 0; g < NS; g++)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) sums[((kpart * NS + g) * MT + mt) * 64] = acc[g][mt];
+    for (int mt = 0; mt < MT; mt++) sums[((kpart * NS + g) * MT + mt) * 64] = neighbours_sum(acc[g][mt]);
   __syncthreads();
   if (!strip_ok) return;
   const size_t npad = (size_t)nstrips * 16;
@@ -1234,9 +1261,10 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
     f32x4 v[NS];
 #pragma unroll
     for (int g = 0; g < NS; g++) {
-      v[g] = sums[(g * MT + mt) * 64];
+      f32x4 part[KW];
 #pragma unroll
-      for (int k = 1; k < KW; k++) v[g] += sums[((k * NS + g) * MT + mt) * 64];
+      for (int k = 0; k < KW; k++) part[k] = sums[((k * NS + g) * MT + mt) * 64];
+      v[g] = neighbours_sum(part);
     }
     if constexpr (ROPE) {
       rope_store(rs, v[0], m, M, lane, head, hpos, slot, sn, cs, (__bf16*)C, ldc);
@@ -1268,7 +1296,13 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf
   const int ksteps = K / 32, nstrips = N / 16;
   const int strip = blockIdx.x * SPB + place, strip_read = min(strip, nstrips - 1);
   const __bf16* wp[2] = {W + (size_t)strip_read * ksteps * 512 + lane * 8, W + (size_t)(nstrips + strip_read) * ksteps * 512 + lane * 8};
-  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  using Chains = MidChains<1, SPB, KW, CH>;
+  static_assert(Chains::by_turn == 1, "the loop's turns are not told apart here");
+  f32x4 acc[2][Chains::all];
+#pragma unroll
+  for (int g = 0; g < 2; g++)
+#pragma unroll
+    for (int c = 0; c < Chains::all; c++) acc[g][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   bf16x8 w[DEPTH][2][WSTEPS];
   // (steps past the end read the last one again; the row is zero there)
   auto fetch = [&](int s0, bf16x8 (&wf)[2][WSTEPS]) {
@@ -1282,7 +1316,8 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf
     for (int s = 0; s < WSTEPS; s++) {
       const bf16x8 af = *(const bf16x8*)(row + (s0 + kpart * WSTEPS + s) * 32 + kq * 8);
 #pragma unroll
-      for (int g = 0; g < 2; g++) acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af, acc[g], 0, 0, 0);
+      for (int g = 0; g < 2; g++)
+        acc[g][s % Chains::by_step] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[g][s], af, acc[g][s % Chains::by_step], 0, 0, 0);
     }
   };
   RowOf<NW, NORM> own;
@@ -1303,15 +1338,16 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf
     }
   }
 #pragma unroll
-  for (int g = 0; g < 2; g++) sums[place * KW + kpart][g][lane] = acc[g];
+  for (int g = 0; g < 2; g++) sums[place * KW + kpart][g][lane] = neighbours_sum(acc[g]);
   __syncthreads();
   if (kpart > 0 || strip >= nstrips) return;
   f32x4 v[2];
 #pragma unroll
   for (int g = 0; g < 2; g++) {
-    v[g] = sums[place * KW][g][lane];
+    f32x4 part[KW];
 #pragma unroll
-    for (int k = 1; k < KW; k++) v[g] += sums[place * KW + k][g][lane];
+    for (int k = 0; k < KW; k++) part[k] = sums[place * KW + k][g][lane];
+    v[g] = neighbours_sum(part);
   }
   mid_store<true>(v[0], v[1], lane & 15, C, N, 0, 1, N, strip, lane, epi, 0.f, nullptr, nstrips);
 }
