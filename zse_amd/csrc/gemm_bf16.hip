@@ -1098,21 +1098,28 @@ __device__ __forceinline__ void mid_store(const f32x4& v, const f32x4& up, int m
 // The relative error against 64 bits, before, with one chain a wave and so: a head of 256,000 columns of K 2,304 at 17
 // to 64 rows 2.0e-7, 2.9e-7 and 2.0e-7; 4,608 columns of K 8,192 at one row, sums left to the reader, 1.1e-7, 1.9e-7
 // and 1.05e-7; gated 14,336 of 2,048 at up to 16 rows 1.87e-7, 2.64e-7 and 1.88e-7; gated 2,048 of 4,096 at 17 rows
-// 1.5e-7, 1.9e-7 and 1.3e-7.  The times are the same.
-template <int MT, int SPB, int KW, int CH>
+// 1.5e-7, 1.9e-7 and 1.3e-7.  The times are the same.  One chain where it is no longer than then: blocks of four waves a
+// strip and chunks of four steps, heads of up to 16 rows, and the rotating products (4,096 columns of K 2,304: nine steps a
+// wave in eight waves, as in two waves and four ranges).
+template <int MT, int SPB, int KW, int CH, bool ROPE = false>
 struct MidChains {
   static constexpr int by_step = KW == 1 || (MT == 1 && CH == 2 * KW && SPB > 2) ? 2 : 1;
-  static constexpr int by_turn = KW == 8 && CH == 8 ? 3 : MT == 1 && SPB == 3 && KW == 4 && CH == 8 ? 2 : 1;
+  static constexpr int by_turn = KW == 8 && CH == 8 && !ROPE ? 3 : MT == 1 && SPB == 3 && KW == 4 && CH == 8 ? 2 : 1;
   static constexpr int all = by_step * by_turn;
 };
 
-// t[0] + ... + t[N - 1], neighbours first
-template <int N>
-__device__ __forceinline__ f32x4 neighbours_sum(f32x4 (&t)[N]) {
+// t[0] + ... + t[N - 1]: neighbours first (PAIRS), or one after the other
+template <bool PAIRS, int N>
+__device__ __forceinline__ f32x4 sum_of(f32x4 (&t)[N]) {
+  if constexpr (PAIRS) {
 #pragma unroll
-  for (int w = 1; w < N; w *= 2)
+    for (int w = 1; w < N; w *= 2)
 #pragma unroll
-    for (int k = 0; k + w < N; k += 2 * w) t[k] += t[k + w];
+      for (int k = 0; k + w < N; k += 2 * w) t[k] += t[k + w];
+  } else {
+#pragma unroll
+    for (int k = 1; k < N; k++) t[0] += t[k];
+  }
   return t[0];
 }
 
@@ -1155,7 +1162,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
     const int row = head * rs.hd + hpos + (r < 8 ? r : rs.hd / 2 + r - 8);
     wp[0] = W + (size_t)(row / 16) * ksteps * 512 + (16 * kq + row % 16) * 8;
   }
-  using Chains = MidChains<MT, SPB, KW, CH>;
+  using Chains = MidChains<MT, SPB, KW, CH, ROPE>;
   f32x4 acc[NS][MT][Chains::all];
 #pragma unroll
   for (int g = 0; g < NS; g++)
@@ -1244,13 +1251,14 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
   }
 #undef ZK_MID_TURN
   // The waves of a strip lay their sums down (the activation buffers are free once every wave has left the
-  // loop) and share the rows out among themselves: sixteen rows a wave, neighbouring parts of the chunks first.
+  // loop) and share the rows out among themselves: sixteen rows a wave, the sums in the order of the
+  // chunk's parts, or neighbours first where a wave has several.
   __syncthreads();
   f32x4* sums = (f32x4*)lds + ((size_t)place * KW * NS * MT) * 64 + lane;
 #pragma unroll
   for (int g = 0; g < NS; g++)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) sums[((kpart * NS + g) * MT + mt) * 64] = neighbours_sum(acc[g][mt]);
+    for (int mt = 0; mt < MT; mt++) sums[((kpart * NS + g) * MT + mt) * 64] = sum_of<true>(acc[g][mt]);
   __syncthreads();
   if (!strip_ok) return;
   const size_t npad = (size_t)nstrips * 16;
@@ -1264,7 +1272,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_kernel(const __bf16* _
       f32x4 part[KW];
 #pragma unroll
       for (int k = 0; k < KW; k++) part[k] = sums[((k * NS + g) * MT + mt) * 64];
-      v[g] = neighbours_sum(part);
+      v[g] = sum_of<(Chains::all > 1)>(part);
     }
     if constexpr (ROPE) {
       rope_store(rs, v[0], m, M, lane, head, hpos, slot, sn, cs, (__bf16*)C, ldc);
@@ -1338,7 +1346,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf
     }
   }
 #pragma unroll
-  for (int g = 0; g < 2; g++) sums[place * KW + kpart][g][lane] = neighbours_sum(acc[g]);
+  for (int g = 0; g < 2; g++) sums[place * KW + kpart][g][lane] = sum_of<true>(acc[g]);
   __syncthreads();
   if (kpart > 0 || strip >= nstrips) return;
   f32x4 v[2];
@@ -1347,7 +1355,7 @@ __global__ __launch_bounds__(SPB * KW * 64) void gemm_mid_norm_kernel(const __bf
     f32x4 part[KW];
 #pragma unroll
     for (int k = 0; k < KW; k++) part[k] = sums[place * KW + k][g][lane];
-    v[g] = neighbours_sum(part);
+    v[g] = sum_of<(Chains::all > 1)>(part);
   }
   mid_store<true>(v[0], v[1], lane & 15, C, N, 0, 1, N, strip, lane, epi, 0.f, nullptr, nstrips);
 }
